@@ -1,6 +1,7 @@
 // Library-wide pieces of the artk C-ABI: error string and version.
 #include "common.hpp"
 
+#include <atomic>
 #include <mutex>
 #include <vector>
 
@@ -12,6 +13,16 @@ void set_error(const char* fmt, ...) {
   va_start(ap, fmt);
   vsnprintf(g_err, sizeof(g_err), fmt, ap);
   va_end(ap);
+}
+
+int num_cus() {
+  static std::atomic<int> known[64];   // 0: not asked yet
+  int dev = 0, v = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  if (dev >= 0 && dev < 64 && (v = known[dev].load(std::memory_order_relaxed)) > 0) return v;
+  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) return 256;
+  if (dev >= 0 && dev < 64) known[dev].store(v, std::memory_order_relaxed);
+  return v;
 }
 
 // ---- profiling -------------------------------------------------------------

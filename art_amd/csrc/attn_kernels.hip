@@ -1194,10 +1194,7 @@ int32_t artk_attn_bwd(const void* q, const void* k, const void* v, const void* o
   p.scale = scale;
   p.scale_log2e = scale * LOG2E;
   {
-    int cus = 0, dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-      cus = 256;
+    const int cus = num_cus();
     p.light_max = pl.nKb2 * Hkv >= cus ? ATT_LIGHT_MAX : 0;
     if (g_light_max_override >= 0) p.light_max = g_light_max_override;  // artk_attn_bwd_tuning
   }

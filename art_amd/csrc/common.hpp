@@ -39,6 +39,9 @@ void set_error(const char* fmt, ...);
     }                                                                               \
   } while (0)
 
+// Compute units of the current device (asked once per device).
+int num_cus();
+
 static inline bool aligned16(const void* p) { return (((uintptr_t)p) & 15) == 0; }
 static inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 

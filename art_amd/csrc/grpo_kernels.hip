@@ -925,19 +925,6 @@ __global__ __launch_bounds__(nthreads<GEMM_NI>()) void gemm_nt_kernel(GemmParams
 // ----------------------------------------------------------------------------
 // Host side
 // ----------------------------------------------------------------------------
-static int num_cus() {
-  static int n = 0;
-  if (n == 0) {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-      n = v;
-    else
-      n = 256;
-  }
-  return n;
-}
-
 // Split count for the d_hidden GEMM: fill whole rounds of CUs, keep every split
 // at least 32 K-steps long, prefer fewer splits on ties.
 static int choose_nsplit(int tiles, int ksteps) {

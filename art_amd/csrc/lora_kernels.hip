@@ -340,10 +340,7 @@ static int32_t launch_lora_gemm(const void* P, const void* Q, const uint16_t* Pe
   p.NT = (int)((N + TILE - 1) / TILE);
   prof_begin(PROF_LORA_GEMM, st);
   {
-    int cus = 0, dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-      cus = 256;
+    const int cus = num_cus();
     const int n_tiles = p.MT * p.NT;
     lora_gemm_kernel<<<(unsigned)(n_tiles < cus ? n_tiles : cus), nthreads<LORA_NI>(), 0, st>>>(p);
   }
@@ -491,17 +488,9 @@ static int32_t check_multi(const artk_lora_proj_t* proj, int32_t n, int64_t T, i
   return ARTK_OK;
 }
 
-static int lora_num_cus() {
-  int cus = 0, dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    cus = 256;
-  return cus;
-}
-
 static int32_t launch_lora_multi(const LoraMultiParams& p, hipStream_t st) {
   prof_begin(PROF_LORA_GEMM, st);
-  const int cus = lora_num_cus();
+  const int cus = num_cus();
   lora_multi_gemm_kernel<<<(unsigned)(p.n_tiles < cus ? p.n_tiles : cus), nthreads<LORA_NI>(), 0, st>>>(p);
   prof_end(PROF_LORA_GEMM, st);
   ARTK_CHECK_LAUNCH();

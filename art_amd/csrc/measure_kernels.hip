@@ -463,10 +463,7 @@ int32_t artk_gemm_loop_probe(const void* P, const void* Q, void* out, int64_t M,
   p.group = group;
   p.same_tile = same_tile != 0;
   p.cycles = cycles;
-  int cus = 0, dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    cus = 256;
+  const int cus = num_cus();
   const int64_t tiles = (int64_t)p.MT * p.NT;
   const unsigned grid = (unsigned)(tiles < cus ? tiles : cus);
   hipStream_t st = (hipStream_t)stream;

@@ -453,10 +453,7 @@ static int32_t launch_moe_gemm(const void* W, const void* X, const int* gather, 
   prof_begin(PROF_MOE_GEMM, st);
   {
     // persistent: one work-group per CU walks the device-side work list
-    int cus = 0, dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-      cus = 256;
+    const int cus = num_cus();
     const int64_t upper = (int64_t)max_row_tiles * p.MT;
     moe_gemm_kernel<<<(unsigned)(upper < cus ? upper : cus), nthreads<MOE_NI>(), 0, st>>>(p);
   }

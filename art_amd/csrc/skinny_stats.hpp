@@ -413,13 +413,6 @@ __global__ __launch_bounds__(256) static void stats_reduce_kernel(StatsReduceJob
 struct StatsGeom {
   int cc, rows_per_slab, n_slabs, n_chunks;
 };
-static inline int stats_num_cus() {
-  int cus = 0, dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    cus = 256;
-  return cus;
-}
 // Chunk width by rank (the factor and the accumulators of a chunk live in LDS / registers);
 // slab height so that the grid is one round of work-groups (one fits per CU) when the matrix
 // is large enough: a second, partly filled round would cost as much as the first.
@@ -427,7 +420,7 @@ static inline int stats_num_cus() {
 // (a row tile of cct column tiles also writes its ROW partial, about half a tile time) plus
 // about two tile times of set-up (factor load, filling the ring, flushing the accumulators).
 static inline int64_t stats_grid_cost(int64_t blocks, int64_t row_tiles_per_block, int cct) {
-  const int64_t cus = stats_num_cus();
+  const int64_t cus = num_cus();
   return ((blocks + cus - 1) / cus) * (row_tiles_per_block * (2 * cct + 1) + 4);
 }
 
@@ -440,7 +433,7 @@ static inline StatsGeom stats_geom(int64_t T, int64_t C, int r) {
   int64_t best_cost = -1;
   for (int cct = max_cct; cct >= 1; --cct) {
     const int64_t n_chunks = (col_tiles + cct - 1) / cct;
-    int64_t want = stats_num_cus() / n_chunks;
+    int64_t want = num_cus() / n_chunks;
     want = want < 1 ? 1 : (want > row_tiles ? row_tiles : want);
     for (int64_t w = want; w <= want + 1 && w <= row_tiles; ++w) {
       int64_t slab_tiles = (row_tiles + w - 1) / w;

@@ -96,3 +96,40 @@ def test_adamw8bit_matches_oracle(artk_lib, gpu):
         c1, c2, a1, a2, p = got1, got2, opt.absmax1.cpu().numpy(), opt.absmax2.cpu().numpy(), got_p
     assert torch.equal(flat.shadow, flat.master.to(torch.bfloat16))
     assert opt.exp_avg().shape == (n,) and opt.exp_avg_sq().min().item() >= 0.0
+
+
+@pytest.mark.parametrize("n", [5, 256 * 3 + 17, 256 * 16 * 512 + 300])
+@pytest.mark.parametrize("book", ["dynamic", "linear", "clustered"])
+def test_adamw8bit_any_code_book(artk_lib, gpu, n, book):
+    """One step from a given state at the edges of the grid (less than one block, a last partial block, more
+    blocks than waves) and for code books whose entries crowd a bin of the start table or leave most of them
+    empty.  Same bounds as test_adamw8bit_matches_oracle, for the same reason."""
+    import numpy as np
+
+    from art_amd.optim import dynamic_code_book
+
+    print("adamw 8-bit", n, book, flush=True)
+    rng = np.random.default_rng(n)
+    if book == "dynamic":
+        b1, b2 = dynamic_code_book(True).numpy(), dynamic_code_book(False).numpy()
+    elif book == "linear":
+        b1, b2 = np.linspace(-1, 1, 256, dtype=np.float32), np.linspace(0, 1, 256, dtype=np.float32)
+    else:
+        b1 = np.sort(np.concatenate([[-1, 0, 1], 0.5 + 1e-3 * rng.random(253)])).astype(np.float32)
+        b2 = np.sort(np.concatenate([[0, 1], 1e-8 * rng.random(100), 0.7 + 1e-2 * rng.random(154)])).astype(np.float32)
+    nb = (n + 255) // 256
+    p = (0.05 * rng.standard_normal(n)).astype(np.float32)
+    g = (0.01 * rng.standard_normal(n)).astype(np.float32)
+    c1, c2 = rng.integers(0, 256, n).astype(np.uint8), rng.integers(0, 256, n).astype(np.uint8)
+    a1, a2 = (1e-3 * rng.random(nb)).astype(np.float32), (1e-6 * rng.random(nb)).astype(np.float32)
+    want = optim_oracle.adamw8bit_step(p, g, c1, c2, a1, a2, b1, b2, 1e-3, (0.9, 0.99), 1e-8, 0.1, 3, 0.0)
+    t = [torch.from_numpy(x.copy()).to(gpu) for x in (p, g, c1, c2, a1, a2, b1, b2)]
+    shadow = torch.zeros(n, dtype=torch.bfloat16, device=gpu)
+    ops.adamw8bit_step(*t, shadow, 1e-3, 0.9, 0.99, 1e-8, 0.1, 3)
+    for got, ref in ((t[2], want[1]), (t[3], want[2])):
+        d = np.abs(got.cpu().numpy().astype(int) - ref.astype(int))
+        assert (d == 0).mean() >= 0.999 and d.max() <= 1
+    assert np.allclose(t[4].cpu().numpy(), want[3], rtol=2e-6, atol=0)
+    assert np.allclose(t[5].cpu().numpy(), want[4], rtol=2e-6, atol=0)
+    assert np.abs(t[0].cpu().numpy() - want[0]).max() <= 1e-6 * np.abs(want[0]).max()
+    assert torch.equal(shadow, t[0].to(torch.bfloat16))
