@@ -96,7 +96,22 @@ class Nf4Struct(C.Structure):
                 ("offset", _f32), ("blocksize", _i32)]
 
 
+class MoeExpertsStruct(C.Structure):
+    """artk_moe_experts_t of include/artk.h."""
+    _fields_ = ([(n, _p) for n in ("x", "router_logits", "W_gu", "W_d", "Wt_gu", "Wt_d", "gate_A", "gate_B", "up_A",
+                                   "up_B", "down_A", "down_B", "topk_idx", "topk_w", "perm", "inv_perm", "row_token",
+                                   "offsets", "tile_prefix", "blk_prefix", "saved")] + [("saved_bytes", _sz)]
+                + [(n, _p) for n in ("y", "g", "dx", "dgate_A", "dgate_B", "dup_A", "dup_B", "ddown_A", "ddown_B")]
+                + [(n, _i64) for n in ("T", "H", "I")] + [(n, _i32) for n in ("E", "k", "r", "adapters_bf16")]
+                + [("scale", _f32)])
+
+
 SIGNATURES.update({
+    "artk_moe_experts_saved_bytes": (_sz, [C.POINTER(MoeExpertsStruct)]),
+    "artk_moe_experts_fwd_workspace_bytes": (_sz, [C.POINTER(MoeExpertsStruct)]),
+    "artk_moe_experts_fwd": (_i32, [C.POINTER(MoeExpertsStruct), _p, _sz, _p]),
+    "artk_moe_experts_bwd_workspace_bytes": (_sz, [C.POINTER(MoeExpertsStruct)]),
+    "artk_moe_experts_bwd": (_i32, [C.POINTER(MoeExpertsStruct), _p, _sz, _p]),
     "artk_adamw8bit_step": (_i32, [_p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _f32, _f32, _f32, _f32, _f32, _i32,
                                    _p, _f32, _p]),
     "artk_nf4_dequant_t": (_i32, [_p, _p, _p, _p, _p, _f32, _i64, _i64, _i32, _p, _p]),

@@ -362,10 +362,12 @@ __global__ __launch_bounds__(nthreads<MOE_NI>()) void moe_gemm_kernel(MoeGemmPar
 
 // Grouped row products: 16-row blocks never straddle experts.
 //   out[i, j] = sum_k X[row(i), k] Mt_e[j, k],  Mt [E,R,K]
+// (the f32 output also times row_w[row_idx[i]], when given)
 __global__ __launch_bounds__(256) void moe_rowdot16_kernel(
     const uint16_t* __restrict__ X, const int* __restrict__ gather, const uint16_t* __restrict__ Mt,
     const int* __restrict__ offsets, const int* __restrict__ blk_prefix, int E, int64_t K, int R,
-    int RP, float scale, float* __restrict__ out_f32, uint16_t* __restrict__ out_bf16) {
+    int RP, float scale, const float* __restrict__ row_w, const int* __restrict__ row_idx,
+    float* __restrict__ out_f32, uint16_t* __restrict__ out_bf16) {
   __shared__ floatx4 red[3][64];
   const int b = blockIdx.x;
   if (b >= blk_prefix[E]) return;
@@ -387,11 +389,148 @@ __global__ __launch_bounds__(256) void moe_rowdot16_kernel(
     for (int q = 0; q < 4; ++q) {
       const int64_t i = row0 + (lane >> 4) * 4 + q;
       if (i < row_end) {
-        if (jm < R) out_f32[i * R + jm] = acc[q];
+        if (jm < R) out_f32[i * R + jm] = row_w ? acc[q] * row_w[row_idx[i]] : acc[q];
         out_bf16[i * RP + jm] = f32_to_bf16(acc[q] * scale);
       }
     }
   }
+}
+
+// ----------------------------------------------------------------------------
+// The expert block around its grouped products (artk_moe_experts_fwd / _bwd).  As torch element-wise and
+// gather calls these steps were 2.9 of the 4.8 ms of a block of 8192 tokens (top-8 of 128 experts, hidden
+// 2048, intermediate 768): the routing weights in fp32 copies of [T, k, H], the gating through four fp32
+// arrays, an index backward with a sort.  Here each is one pass with 16-byte accesses, and the routing
+// weight of a row never meets a [rows, H] array: the backward of the down projection reads the rows of the
+// token gradient through the gather, and the weight multiplies the rank-r products and the gated gradient.
+// ----------------------------------------------------------------------------
+
+// bf16 adapters of one block from its six parameters (f32 or bf16): gate and up share their input, so their
+// A are stacked ([E, 2r, H]) and their B form a block-diagonal [E, 2I, 2r]; down's are copied.
+struct MoePack {
+  const void *gate_A, *gate_B, *up_A, *up_B, *down_A, *down_B;
+  uint16_t *A_gu, *B_gu, *A_d, *B_d;
+  int64_t H, I;
+  int E, r, bf16;
+};
+
+__device__ __forceinline__ uint4 load8_bf16(const void* src, int64_t i, int is_bf16) {
+  if (is_bf16) return *(const uint4*)((const uint16_t*)src + i);
+  const float4 a = *(const float4*)((const float*)src + i), b = *(const float4*)((const float*)src + i + 4);
+  return make_uint4(pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w), pack_bf16x2(b.x, b.y), pack_bf16x2(b.z, b.w));
+}
+
+__global__ __launch_bounds__(256) void moe_pack_kernel(MoePack p) {
+  // every dimension is a multiple of 8: a thread writes 8 consecutive values of one output row
+  const int64_t nA = (int64_t)p.E * p.r * p.H / 8, nB = (int64_t)p.E * p.I * p.r / 8;   // per projection
+  const int64_t nAd = (int64_t)p.E * p.r * p.I / 8, nBd = (int64_t)p.E * p.H * p.r / 8;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < 2 * nA) {
+    const int up = i >= nA;
+    i = (i - up * nA) * 8;
+    const int64_t per = (int64_t)p.r * p.H, e = i / per;
+    *(uint4*)(p.A_gu + (2 * e + up) * per + (i - e * per)) = load8_bf16(up ? p.up_A : p.gate_A, i, p.bf16);
+    return;
+  }
+  i -= 2 * nA;
+  if (i < 2 * nB) {
+    const int up = i >= nB;
+    i = (i - up * nB) * 8;
+    const int64_t row = i / p.r, c = i - row * p.r, e = row / p.I;   // row of [E, I]
+    uint16_t* dst = p.B_gu + ((2 * e + up) * p.I + (row - e * p.I)) * 2 * p.r + c;
+    *(uint4*)(dst + up * p.r) = load8_bf16(up ? p.up_B : p.gate_B, i, p.bf16);
+    *(uint4*)(dst + (1 - up) * p.r) = make_uint4(0, 0, 0, 0);
+    return;
+  }
+  i -= 2 * nB;
+  if (i < nAd) {
+    *(uint4*)(p.A_d + i * 8) = load8_bf16(p.down_A, i * 8, p.bf16);
+    return;
+  }
+  i -= nAd;
+  if (i < nBd) *(uint4*)(p.B_d + i * 8) = load8_bf16(p.down_B, i * 8, p.bf16);
+}
+
+__device__ __forceinline__ void unpack8(const uint4& v, float (&f)[8]) {
+  unpack2(v.x, f[0], f[1]);
+  unpack2(v.y, f[2], f[3]);
+  unpack2(v.z, f[4], f[5]);
+  unpack2(v.w, f[6], f[7]);
+}
+__device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
+  return make_uint4(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7]));
+}
+
+// h[i, c] = silu(gu[i, c]) gu[i, I + c]; 6 B per element of h, HBM-bound.
+__global__ __launch_bounds__(256) void moe_silu_mul_kernel(const uint16_t* __restrict__ gu, int64_t n8, int I8,
+                                                           uint16_t* __restrict__ h) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n8) return;
+  const int64_t row = i / I8;
+  const int c = (int)(i - row * I8);
+  const uint4* src = (const uint4*)gu + row * 2 * I8 + c;
+  float g[8], u[8];
+  unpack8(src[0], g);
+  unpack8(src[I8], u);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) g[j] = g[j] / (1.f + expf(-g[j])) * u[j];
+  ((uint4*)h)[i] = pack8(g);
+}
+
+// Gradient of the gating for dh = w_i * dhr[i, :] (w_i: routing weight of sorted row i), written over gu's
+// layout: g_gu[i, c] = dh u silu'(g), g_gu[i, I + c] = dh silu(g).
+__global__ __launch_bounds__(256) void moe_silu_bwd_kernel(const uint16_t* __restrict__ gu,
+                                                           const uint16_t* __restrict__ dhr,
+                                                           const float* __restrict__ topk_w,
+                                                           const int* __restrict__ perm, int64_t n8, int I8,
+                                                           uint16_t* __restrict__ g_gu) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n8) return;
+  const int64_t row = i / I8;
+  const int c = (int)(i - row * I8);
+  const uint4* src = (const uint4*)gu + row * 2 * I8 + c;
+  uint4* dst = (uint4*)g_gu + row * 2 * I8 + c;
+  float g[8], u[8], d[8];
+  unpack8(src[0], g);
+  unpack8(src[I8], u);
+  unpack8(((const uint4*)dhr)[i], d);
+  const float w = topk_w[perm[row]];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float s = 1.f / (1.f + expf(-g[j])), dh = d[j] * w;
+    d[j] = dh * u[j] * (s * (1.f + g[j] * (1.f - s)));
+    u[j] = dh * (g[j] * s);
+  }
+  dst[0] = pack8(d);
+  dst[I8] = pack8(u);
+}
+
+// out[t, :] = sum_j w[t, j] rows[inv_perm[t k + j], :] in slot order (w == nullptr: plain sum); the k
+// sorted rows of a token are read once, 8 columns per thread, eight loads in flight.
+__global__ __launch_bounds__(256) void moe_combine_kernel(const uint16_t* __restrict__ rows,
+                                                          const int* __restrict__ inv_perm,
+                                                          const float* __restrict__ w, int64_t n8, int H8, int k,
+                                                          uint16_t* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n8) return;
+  const int64_t t = i / H8;
+  const int c = (int)(i - t * H8);
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int j0 = 0; j0 < k; j0 += 8) {
+    uint4 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      v[j] = j0 + j < k ? ((const uint4*)rows)[(int64_t)inv_perm[t * k + j0 + j] * H8 + c] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float wj = j0 + j >= k ? 0.f : (w ? w[t * k + j0 + j] : 1.f);
+      float f[8];
+      unpack8(v[j], f);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc[q] += wj * f[q];
+    }
+  }
+  ((uint4*)out)[i] = pack8(acc);
 }
 
 __global__ __launch_bounds__(256) void transpose_bf16_batched_kernel(const uint16_t* __restrict__ in,
@@ -465,10 +604,11 @@ static int32_t launch_moe_gemm(const void* W, const void* X, const int* gather, 
 static int32_t launch_moe_rowdot(const void* X, const int* gather, const uint16_t* Mt,
                                  const int* offsets, const int* blk_prefix, int64_t n_rows, int E,
                                  int64_t K, int R, int RP, float scale, float* out_f32,
-                                 uint16_t* out_bf16, hipStream_t st) {
+                                 uint16_t* out_bf16, hipStream_t st, const float* row_w = nullptr,
+                                 const int* row_idx = nullptr) {
   dim3 grid((unsigned)((n_rows + 15) / 16 + E), (unsigned)(RP / 16));
   moe_rowdot16_kernel<<<grid, 256, 0, st>>>((const uint16_t*)X, gather, Mt, offsets, blk_prefix, E, K,
-                                            R, RP, scale, out_f32, out_bf16);
+                                            R, RP, scale, row_w, row_idx, out_f32, out_bf16);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }
@@ -631,6 +771,231 @@ int32_t artk_moe_lora_grouped_bwd(const void* g, const void* x, const int32_t* g
   // one pass over x (through the row gather when there is one): dA_e [r,in] = s (g B_e)^T x
   return launch_stats_grouped(x, gather ? (int64_t)0x3fffffff / in : n_rows, gather, n_rows, in, nullptr, c.gb, r,
                               E, expert_offsets, nullptr, dA, scale, 1, c.dummy, st);
+}
+
+// ---- the whole expert block ---------------------------------------------------------------------------
+// What the forward leaves for the backward, carved in the same order by the size query and both calls.
+struct MoeSaved {
+  uint16_t *A_gu, *B_gu, *A_d, *B_d;  // bf16 adapters [E,2r,H], [E,2I,2r], [E,r,I], [E,H,r]
+  float *xa_gu, *xaw_d;               // x A^T [n,2r]; routing weight times h A_d^T [n,r]
+  uint16_t *gu, *h;                   // gate|up [n,2I], silu(gate) up [n,I]
+};
+static void carve_moe_saved(Workspace& ws, const artk_moe_experts_t& a, MoeSaved& c) {
+  const size_t n = (size_t)(a.T * a.k), E = (size_t)a.E, r = (size_t)a.r, H = (size_t)a.H, I = (size_t)a.I;
+  c.A_gu = ws.take<uint16_t>(E * 2 * r * H);
+  c.B_gu = ws.take<uint16_t>(E * 2 * I * 2 * r);
+  c.A_d = ws.take<uint16_t>(E * r * I);
+  c.B_d = ws.take<uint16_t>(E * H * r);
+  c.xa_gu = ws.take<float>(n * 2 * r);
+  c.xaw_d = ws.take<float>(n * r);
+  c.gu = ws.take<uint16_t>(n * 2 * I);
+  c.h = ws.take<uint16_t>(n * I);
+}
+struct MoeFwdScratch {
+  char* route;
+  size_t route_bytes;
+  uint16_t *xa16_gu, *xa16_d, *down;
+};
+static void carve_moe_fwd(Workspace& ws, const artk_moe_experts_t& a, MoeFwdScratch& c) {
+  const size_t n = (size_t)(a.T * a.k);
+  c.route_bytes = artk_moe_route_workspace_bytes(a.T, a.E, a.k);
+  c.route = ws.take<char>(c.route_bytes);
+  c.xa16_gu = ws.take<uint16_t>(n * round16(2 * a.r));
+  c.xa16_d = ws.take<uint16_t>(n * round16(a.r));
+  c.down = ws.take<uint16_t>(n * a.H);
+}
+struct MoeBlockBwdScratch {
+  uint16_t *Bt_gu, *At_gu, *Bt_d, *At_d;  // [E,2r,2I], [E,H,2r], [E,r,H], [E,I,r]
+  float *gb, *rowp, *dummy;
+  uint16_t *gb16, *dhr, *g_gu, *dx_rows;
+};
+static void carve_moe_block_bwd(Workspace& ws, const artk_moe_experts_t& a, MoeBlockBwdScratch& c) {
+  const size_t n = (size_t)(a.T * a.k), E = (size_t)a.E, r = (size_t)a.r, H = (size_t)a.H, I = (size_t)a.I;
+  c.Bt_gu = ws.take<uint16_t>(E * 2 * r * 2 * I);
+  c.At_gu = ws.take<uint16_t>(E * H * 2 * r);
+  c.Bt_d = ws.take<uint16_t>(E * r * H);
+  c.At_d = ws.take<uint16_t>(E * I * r);
+  const size_t p_d = (size_t)stats_grouped_chunks(a.H, a.r, a.E) * r;
+  const size_t p_gu = (size_t)stats_grouped_chunks(2 * a.I, 2 * a.r, a.E) * 2 * r;
+  c.rowp = ws.take<float>((p_d > p_gu ? p_d : p_gu) * n);
+  c.gb = ws.take<float>(n * 2 * r);
+  c.gb16 = ws.take<uint16_t>(n * round16(2 * a.r));
+  c.dummy = ws.take<float>(1024);
+  c.dhr = ws.take<uint16_t>(n * I);
+  c.g_gu = ws.take<uint16_t>(n * 2 * I);
+  c.dx_rows = ws.take<uint16_t>(n * H);
+}
+
+static int32_t check_moe_experts(const artk_moe_experts_t* a, bool backward) {
+  ARTK_CHECK_ARG(a != nullptr, "null argument");
+  ARTK_CHECK_ARG(a->T > 0 && a->k > 0 && a->E > 0 && a->k <= a->E, "T, E, k must be positive and k <= E");
+  if (a->E > MOE_MAX_E || a->k > MOE_MAX_K || a->T * a->k >= (1ll << 30)) {
+    set_error("supported: experts <= %d, top-k <= %d", MOE_MAX_E, MOE_MAX_K);
+    return ARTK_ERR_UNSUPPORTED_SHAPE;
+  }
+  const int64_t n = a->T * a->k;
+  int32_t rc = check_moe(n, a->H, 2 * a->I, a->E, 2 * a->r);
+  if (rc == 0) rc = check_moe(n, a->I, a->H, a->E, a->r);
+  if (rc) return rc;
+  const int64_t widest = backward && 2 * a->I > a->H ? 2 * a->I : a->H;
+  if (n * widest * 2 >= (1ll << 31)) {
+    set_error("T * k * %lld * 2 bytes (%lld) must stay below 2 GiB (31-bit row offsets)", (long long)widest,
+              (long long)(n * widest * 2));
+    return ARTK_ERR_UNSUPPORTED_SHAPE;
+  }
+  ARTK_CHECK_ARG(a->x && a->topk_idx && a->topk_w && a->perm && a->inv_perm && a->row_token && a->offsets &&
+                     a->tile_prefix && a->blk_prefix && a->saved,
+                 "null pointer argument");
+  ARTK_CHECK_ARG(aligned16(a->x) && aligned16(a->saved), "pointers must be 16-byte aligned");
+  return ARTK_OK;
+}
+
+size_t artk_moe_experts_saved_bytes(const artk_moe_experts_t* a) {
+  Workspace ws(nullptr, 0);
+  MoeSaved c;
+  carve_moe_saved(ws, *a, c);
+  return ws.used + 256;
+}
+size_t artk_moe_experts_fwd_workspace_bytes(const artk_moe_experts_t* a) {
+  Workspace ws(nullptr, 0);
+  MoeFwdScratch c;
+  carve_moe_fwd(ws, *a, c);
+  return ws.used + 256;
+}
+size_t artk_moe_experts_bwd_workspace_bytes(const artk_moe_experts_t* a) {
+  Workspace ws(nullptr, 0);
+  MoeBlockBwdScratch c;
+  carve_moe_block_bwd(ws, *a, c);
+  return ws.used + 256;
+}
+
+static unsigned blocks256(int64_t n) { return (unsigned)((n + 255) / 256); }
+
+int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,
+                             artk_stream_t stream) {
+  int32_t rc = check_moe_experts(a, false);
+  if (rc) return rc;
+  ARTK_CHECK_ARG(a->router_logits && a->W_gu && a->W_d && a->gate_A && a->gate_B && a->up_A && a->up_B && a->down_A &&
+                     a->down_B && a->y,
+                 "null pointer argument");
+  ARTK_CHECK_ARG(aligned16(a->W_gu) && aligned16(a->W_d) && aligned16(a->gate_A) && aligned16(a->gate_B) &&
+                     aligned16(a->up_A) && aligned16(a->up_B) && aligned16(a->down_A) && aligned16(a->down_B) &&
+                     aligned16(a->y),
+                 "pointers must be 16-byte aligned");
+  Workspace ws(workspace, workspace_bytes), sv(a->saved, a->saved_bytes);
+  MoeFwdScratch c;
+  MoeSaved s;
+  carve_moe_fwd(ws, *a, c);
+  carve_moe_saved(sv, *a, s);
+  if (!ws.ok() || !sv.ok()) {
+    set_error("workspace too small: need %zu and %zu bytes, got %zu and %zu", ws.used, sv.used, workspace_bytes,
+              a->saved_bytes);
+    return ARTK_ERR_WORKSPACE_TOO_SMALL;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  const int64_t n = a->T * a->k, H = a->H, I = a->I;
+  const int E = a->E, r = a->r;
+  if ((rc = artk_moe_route(a->router_logits, a->T, E, a->k, a->topk_idx, a->topk_w, a->perm, a->inv_perm, a->row_token,
+                           a->offsets, a->tile_prefix, a->blk_prefix, c.route, c.route_bytes, stream)))
+    return rc;
+  {
+    MoePack p{a->gate_A, a->gate_B, a->up_A, a->up_B, a->down_A, a->down_B, s.A_gu, s.B_gu, s.A_d, s.B_d,
+              H,         I,         E,       r,       a->adapters_bf16};
+    moe_pack_kernel<<<blocks256((int64_t)E * r * (3 * H + 3 * I) / 8), 256, 0, st>>>(p);
+    ARTK_CHECK_LAUNCH();
+  }
+  if ((rc = launch_moe_rowdot(a->x, a->row_token, s.A_gu, a->offsets, a->blk_prefix, n, E, H, 2 * r, round16(2 * r),
+                              a->scale, s.xa_gu, c.xa16_gu, st)))
+    return rc;
+  if ((rc = launch_moe_gemm(a->W_gu, a->x, a->row_token, s.B_gu, c.xa16_gu, s.gu, a->offsets, a->tile_prefix, n, 2 * I,
+                            H, E, 2 * r, round16(2 * r), st)))
+    return rc;
+  moe_silu_mul_kernel<<<blocks256(n * I / 8), 256, 0, st>>>(s.gu, n * I / 8, (int)(I / 8), s.h);
+  ARTK_CHECK_LAUNCH();
+  if ((rc = launch_moe_rowdot(s.h, nullptr, s.A_d, a->offsets, a->blk_prefix, n, E, I, r, round16(r), a->scale,
+                              s.xaw_d, c.xa16_d, st, a->topk_w, a->perm)))
+    return rc;
+  if ((rc = launch_moe_gemm(a->W_d, s.h, nullptr, s.B_d, c.xa16_d, c.down, a->offsets, a->tile_prefix, n, H, I, E, r,
+                            round16(r), st)))
+    return rc;
+  moe_combine_kernel<<<blocks256(a->T * H / 8), 256, 0, st>>>(c.down, a->inv_perm, a->topk_w, a->T * H / 8,
+                                                              (int)(H / 8), a->k, (uint16_t*)a->y);
+  ARTK_CHECK_LAUNCH();
+  return ARTK_OK;
+}
+
+int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,
+                             artk_stream_t stream) {
+  int32_t rc = check_moe_experts(a, true);
+  if (rc) return rc;
+  ARTK_CHECK_ARG(a->g && a->Wt_gu && a->Wt_d && a->dx && a->dgate_A && a->dgate_B && a->dup_A && a->dup_B &&
+                     a->ddown_A && a->ddown_B,
+                 "null pointer argument");
+  ARTK_CHECK_ARG(aligned16(a->g) && aligned16(a->Wt_gu) && aligned16(a->Wt_d) && aligned16(a->dx) &&
+                     aligned16(a->dgate_A) && aligned16(a->dgate_B) && aligned16(a->dup_A) && aligned16(a->dup_B) &&
+                     aligned16(a->ddown_A) && aligned16(a->ddown_B),
+                 "pointers must be 16-byte aligned");
+  Workspace ws(workspace, workspace_bytes), sv(a->saved, a->saved_bytes);
+  MoeBlockBwdScratch c;
+  MoeSaved s;
+  carve_moe_block_bwd(ws, *a, c);
+  carve_moe_saved(sv, *a, s);
+  if (!ws.ok() || !sv.ok()) {
+    set_error("workspace too small: need %zu and %zu bytes, got %zu and %zu", ws.used, sv.used, workspace_bytes,
+              a->saved_bytes);
+    return ARTK_ERR_WORKSPACE_TOO_SMALL;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  const int64_t n = a->T * a->k, H = a->H, I = a->I;
+  const int E = a->E, r = a->r;
+  {
+    SmallTransposeMulti m;
+    m.n = 4;
+    m.t[0] = {s.B_gu, c.Bt_gu, E, 2 * I, 2 * r};
+    m.t[1] = {s.A_gu, c.At_gu, E, 2 * r, H};
+    m.t[2] = {s.B_d, c.Bt_d, E, H, r};
+    m.t[3] = {s.A_d, c.At_d, E, r, I};
+    if ((rc = launch_small_transpose_multi(m, st))) return rc;
+  }
+  const StatsReduceJob none{nullptr, 0, 0, 0.f, nullptr, 0, nullptr, 0, 0.f};
+  // down, on the unweighted rows g[token]: g B_d per row and dB_d = s g^T (w h A_d^T) in one pass
+  if ((rc = launch_stats_grouped(a->g, a->T, a->row_token, n, H, c.Bt_d, s.xaw_d, r, E, a->offsets, c.rowp, a->ddown_B,
+                                 a->scale, 0, c.dummy, st)))
+    return rc;
+  {
+    StatsReduceJob ja{c.rowp, stats_grouped_chunks(H, r, E), n, 1.f, c.gb, 0, c.gb16, round16(r), a->scale};
+    ja.row_w = a->topk_w;
+    ja.row_idx = a->perm;
+    if ((rc = launch_stats_reduce(ja, none, r, st))) return rc;
+  }
+  if ((rc = launch_moe_gemm(a->Wt_d, a->g, a->row_token, c.At_d, c.gb16, c.dhr, a->offsets, a->tile_prefix, n, I, H, E,
+                            r, round16(r), st)))
+    return rc;
+  if ((rc = launch_stats_grouped(s.h, n, nullptr, n, I, nullptr, c.gb, r, E, a->offsets, nullptr, a->ddown_A, a->scale,
+                                 1, c.dummy, st)))
+    return rc;
+  moe_silu_bwd_kernel<<<blocks256(n * I / 8), 256, 0, st>>>(s.gu, c.dhr, a->topk_w, a->perm, n * I / 8, (int)(I / 8),
+                                                            c.g_gu);
+  ARTK_CHECK_LAUNCH();
+  // gate|up
+  if ((rc = launch_stats_grouped(c.g_gu, n, nullptr, n, 2 * I, c.Bt_gu, s.xa_gu, 2 * r, E, a->offsets, c.rowp,
+                                 a->dgate_B, a->scale, 0, c.dummy, st, a->dup_B, r, I)))
+    return rc;
+  {
+    StatsReduceJob ja{c.rowp, stats_grouped_chunks(2 * I, 2 * r, E), n,       1.f, c.gb, 0, c.gb16, round16(2 * r),
+                      a->scale};
+    if ((rc = launch_stats_reduce(ja, none, 2 * r, st))) return rc;
+  }
+  if ((rc = launch_moe_gemm(a->Wt_gu, c.g_gu, nullptr, c.At_gu, c.gb16, c.dx_rows, a->offsets, a->tile_prefix, n, H,
+                            2 * I, E, 2 * r, round16(2 * r), st)))
+    return rc;
+  if ((rc = launch_stats_grouped(a->x, a->T, a->row_token, n, H, nullptr, c.gb, 2 * r, E, a->offsets, nullptr,
+                                 a->dgate_A, a->scale, 1, c.dummy, st, a->dup_A, r, 0)))
+    return rc;
+  moe_combine_kernel<<<blocks256(a->T * H / 8), 256, 0, st>>>(c.dx_rows, a->inv_perm, nullptr, a->T * H / 8,
+                                                              (int)(H / 8), a->k, (uint16_t*)a->dx);
+  ARTK_CHECK_LAUNCH();
+  return ARTK_OK;
 }
 
 int32_t artk_transpose_bf16_batched(const void* in, void* out, int64_t n, int64_t R, int64_t C,

@@ -48,6 +48,12 @@ struct StatsParams {
   float col_scale;
   int col_transposed;
   int64_t x_rows;     // rows of X (grouped form: bound of the descriptor)
+  // Grouped form, two projections stacked along the rank (e < r_split: the first one) and, in the
+  // plain layout, along the columns (c < c_split): each gets its own array and the blocks that mix
+  // them, which belong to nobody, are not stored.  r_split == 0: one array.
+  float* col_out2 = nullptr;
+  int r_split = 0;
+  int64_t c_split = 0;
 };
 
 // XOR of the 16-byte chunk index of a 256-byte tile row: row-fragment reads (one chunk of
@@ -312,10 +318,21 @@ __device__ __forceinline__ void lora_stats_body(const StatsParams& p, const int 
           if (!grouped) {
             *(floatx4*)(p.col_part + ((int64_t)slab * p.C + c) * R + e0) = v;
           } else if (!p.col_transposed) {
-            *(floatx4*)(p.col_out + ((int64_t)slab * p.C + c) * R + e0) = v * p.col_scale;
+            if (p.r_split == 0) {
+              *(floatx4*)(p.col_out + ((int64_t)slab * p.C + c) * R + e0) = v * p.col_scale;
+            } else if (c < p.c_split) {
+              if (e0 < p.r_split)
+                *(floatx4*)(p.col_out + ((int64_t)slab * p.c_split + c) * p.r_split + e0) = v * p.col_scale;
+            } else if (e0 >= p.r_split) {
+              *(floatx4*)(p.col_out2 + ((int64_t)slab * (p.C - p.c_split) + c - p.c_split) * (R - p.r_split) + e0 -
+                          p.r_split) = v * p.col_scale;
+            }
           } else {
+            float* dst = p.col_out + ((int64_t)slab * (p.r_split ? p.r_split : R) + e0) * p.C + c;
+            if (p.r_split && e0 >= p.r_split)
+              dst = p.col_out2 + ((int64_t)slab * (R - p.r_split) + e0 - p.r_split) * p.C + c;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) p.col_out[((int64_t)slab * R + e0 + k) * p.C + c] = v[k] * p.col_scale;
+            for (int k = 0; k < 4; ++k) dst[k * p.C] = v[k] * p.col_scale;
           }
         }
     }
@@ -354,6 +371,9 @@ struct StatsReduceJob {
   uint16_t* out_bf16;
   int RP;
   float bf16_scale;
+  // plain f32 output: row i is also multiplied by row_w[row_idx[i]] (nullptr: not); the bf16 copy is not
+  const float* row_w = nullptr;
+  const int* row_idx = nullptr;
   // plain (not transposed) output: row pitch and first column of the R results inside a wider
   // [n][out_ld] array (0: dense [n][R])
   int out_ld = 0, out_off = 0;
@@ -398,7 +418,7 @@ __device__ __forceinline__ void stats_reduce_one(const StatsReduceJob& j, int R,
         j.out[(int64_t)e * j.n + row] = s;
       }
     } else {
-      j.out[row * (j.out_ld ? j.out_ld : R) + j.out_off + e] = s;
+      j.out[row * (j.out_ld ? j.out_ld : R) + j.out_off + e] = j.row_w ? s * j.row_w[j.row_idx[row]] : s;
     }
   }
   if (j.out_bf16) j.out_bf16[row * j.RP + e] = f32_to_bf16(s * j.bf16_scale);
@@ -532,8 +552,12 @@ static inline int32_t launch_stats_grouped(const void* X, int64_t x_rows, const 
                                            int64_t C, const uint16_t* F, const float* Y, int r, int E,
                                            const int* offsets, float* row_part, float* col_out,
                                            float col_scale, int col_transposed, float* row_dummy,
-                                           hipStream_t st) {
+                                           hipStream_t st, float* col_out2 = nullptr, int r_split = 0,
+                                           int64_t c_split = 0) {
   StatsParams p;
+  p.col_out2 = col_out2;
+  p.r_split = r_split;
+  p.c_split = c_split;
   p.X = (const uint16_t*)X;
   p.T = n_rows;
   p.C = C;

@@ -1,10 +1,9 @@
 """MoE expert block with per-expert LoRA on the MI355X kernels.
 
-Routing (top-k on the router logits, stable expert-contiguous permutation) and
-the three per-expert projections (gate, up, down; each W_e x + scale B_e A_e x)
-run in the artk library; the SiLU gating between them and the weighted
-recombination of a token's k expert outputs are elementwise / gather steps done
-with torch index ops in a fixed order.  The reference has no MoE code at this
+Routing (top-k on the router logits, stable expert-contiguous permutation), the
+three per-expert projections (gate, up, down; each W_e x + scale B_e A_e x), the
+SiLU gating between them and the weighted recombination of a token's k expert
+outputs run in the artk library, one call each way.  The reference has no MoE code at this
 commit; the shapes follow the Qwen3-30B-A3B-style benchmark configuration."""
 from __future__ import annotations
 
@@ -46,16 +45,26 @@ def grouped_lora_linear(x, W, W_t, A, B, scale, routing, use_gather: bool):
     return _GroupedLoRAFn.apply(x, W, W_t, A, B, float(scale), routing, use_gather)
 
 
-def _fuse_adapters(A1, B1, A2, B2):
-    """Adapters of two projections of the same input as one of rank r1 + r2:
-    A stacked, B block-diagonal (autograd routes the gradients back to the four
-    parameters; the off-diagonal blocks of dB belong to no adapter)."""
-    A = torch.cat([A1, A2], 1)                                       # [E, r1 + r2, in]
-    E, o1, r1 = B1.shape
-    o2, r2 = B2.shape[1], B2.shape[2]
-    top = torch.cat([B1, B1.new_zeros(E, o1, r2)], 2)
-    bot = torch.cat([B2.new_zeros(E, o2, r1), B2], 2)
-    return A, torch.cat([top, bot], 1)                               # [E, o1 + o2, r1 + r2]
+class _MoEExpertsFn(torch.autograd.Function):
+    """The whole block (routing, three projections, gating, recombination) as one library call each way."""
+
+    @staticmethod
+    def forward(ctx, x, logits, top_k, W_gu, W_d, Wt_gu, Wt_d, scale, *params):
+        dtype = params[0].dtype
+        if dtype not in (torch.float32, torch.bfloat16) or any(p.dtype != dtype for p in params):
+            dtype = torch.float32
+        adapters = {n: p.detach().to(dtype).contiguous() for n, p in zip(ops._MOE_PARAMS, params)}
+        y, routing, saved = ops.moe_experts_fwd(x, logits, top_k, W_gu, W_d, adapters, scale)
+        ctx.save_for_backward(x, saved, Wt_gu, Wt_d, *params)
+        ctx.routing, ctx.scale = routing, scale
+        return y, routing
+
+    @staticmethod
+    def backward(ctx, g, _g_routing):
+        x, saved, Wt_gu, Wt_d, *params = ctx.saved_tensors
+        dx, grads = ops.moe_experts_bwd(g.contiguous(), x, ctx.routing, saved, Wt_gu, Wt_d,
+                                        dict(zip(ops._MOE_PARAMS, params)), ctx.scale)
+        return (dx,) + (None,) * 7 + tuple(grads[n].to(p.dtype) for n, p in zip(ops._MOE_PARAMS, params))
 
 
 class MoELoRAExperts(nn.Module):
@@ -99,21 +108,10 @@ class MoELoRAExperts(nn.Module):
             self._wt[name] = (w._version, w.data_ptr(), ops.transpose_batched(w))
         return self._wt[name][2]
 
-    def _proj(self, name, x, routing, use_gather):
-        return grouped_lora_linear(x, getattr(self, f"{name}_weight"), self._transposed(name),
-                                   getattr(self, f"{name}_lora_A"), getattr(self, f"{name}_lora_B"),
-                                   self.scaling, routing, use_gather)
-
     def forward(self, x: torch.Tensor, router_logits: torch.Tensor):
         """x bf16 [T,H], router_logits f32 [T,E] -> (y bf16 [T,H], routing)."""
-        routing = ops.moe_route(router_logits.float().contiguous(), self.top_k)
-        x = x.to(torch.bfloat16).contiguous()
-        A_gu, B_gu = _fuse_adapters(self.gate_lora_A, self.gate_lora_B, self.up_lora_A, self.up_lora_B)
-        gate_up = grouped_lora_linear(x, self.gate_up_weight, self._transposed("gate_up"), A_gu, B_gu,
-                                      self.scaling, routing, True)
-        gate, up = gate_up[:, :self.intermediate], gate_up[:, self.intermediate:]
-        h = (torch.nn.functional.silu(gate.float()) * up.float()).to(torch.bfloat16)
-        down = self._proj("down", h, routing, False)  # [T*k, H] in sorted order
-        per_slot = down[routing.inv_perm.long()].view(x.shape[0], self.top_k, -1).float()
-        y = (per_slot * routing.topk_w.unsqueeze(-1)).sum(1).to(torch.bfloat16)
-        return y, routing
+        params = (self.gate_lora_A, self.gate_lora_B, self.up_lora_A, self.up_lora_B, self.down_lora_A, self.down_lora_B)
+        return _MoEExpertsFn.apply(
+            x.to(torch.bfloat16).contiguous(), router_logits.detach().float().contiguous(), self.top_k,
+            self.gate_up_weight, self.down_weight, self._transposed("gate_up"), self._transposed("down"),
+            float(self.scaling), *params)

@@ -410,6 +410,83 @@ def moe_lora_grouped_bwd(g, x, gather, W_t, A, B, xa, scale: float, routing: Rou
     return dx, dA, dB
 
 
+_MOE_PARAMS = ("gate_A", "gate_B", "up_A", "up_B", "down_A", "down_B")
+
+
+def _moe_experts_struct(x, routing: Routing, adapters, saved, scale: float):
+    """artk_moe_experts_t with the fields that both directions use (and its two sizes n, r)."""
+    import ctypes as C
+
+    T, H = x.shape
+    _, r, I = adapters["down_A"].shape
+    st = _lib.MoeExpertsStruct()
+    st.x = x.data_ptr()
+    for f in ("topk_idx", "topk_w", "perm", "inv_perm", "row_token", "offsets", "tile_prefix", "blk_prefix"):
+        setattr(st, f, getattr(routing, f).data_ptr())
+    st.T, st.H, st.I, st.E, st.k, st.r, st.scale = T, H, I, routing.n_experts, routing.k, r, scale
+    if saved is not None:
+        st.saved, st.saved_bytes = saved.data_ptr(), saved.numel()
+    return st, C.byref(st)
+
+
+def moe_experts_fwd(x, router_logits, k: int, W_gu, W_d, adapters: dict, scale: float):
+    """A block of gated-MLP experts (see artk_moe_experts_fwd): (y bf16 [T,H], routing, saved), where `saved`
+    is what moe_experts_bwd needs.  adapters: gate_A, gate_B, up_A, up_B, down_A, down_B, all f32 or all bf16."""
+    T, H = x.shape
+    E, _, I = W_d.shape
+    r = adapters["down_A"].shape[1]
+    dtype = adapters["down_A"].dtype
+    _need(x, "x", torch.bfloat16)
+    _need(router_logits, "router_logits", torch.float32, (T, E))
+    _need(W_gu, "W_gu", torch.bfloat16, (E, 2 * I, H))
+    _need(W_d, "W_d", torch.bfloat16, (E, H, I))
+    shapes = {"gate_A": (E, r, H), "up_A": (E, r, H), "gate_B": (E, I, r), "up_B": (E, I, r), "down_A": (E, r, I),
+              "down_B": (E, H, r)}
+    if dtype not in (torch.float32, torch.bfloat16):
+        raise TypeError(f"adapters must be float32 or bfloat16, got {dtype}")
+    for name in _MOE_PARAMS:
+        _need(adapters[name], name, dtype, shapes[name])
+    lib = _lib.load()
+    dev = x.device
+    n = T * k
+    i32 = lambda *shape: torch.empty(shape, dtype=torch.int32, device=dev)
+    rt = Routing()
+    rt.topk_idx, rt.topk_w = i32(T, k), torch.empty((T, k), dtype=torch.float32, device=dev)
+    rt.perm, rt.inv_perm, rt.row_token = i32(n), i32(n), i32(n)
+    rt.offsets, rt.tile_prefix, rt.blk_prefix = i32(E + 1), i32(E + 1), i32(E + 1)
+    rt.n_rows, rt.n_experts, rt.k = n, E, k
+    st, ref = _moe_experts_struct(x, rt, adapters, None, scale)
+    saved = _workspace(lib.artk_moe_experts_saved_bytes(ref), dev)
+    ws = _workspace(lib.artk_moe_experts_fwd_workspace_bytes(ref), dev)
+    y = torch.empty_like(x)
+    st.saved, st.saved_bytes = saved.data_ptr(), saved.numel()
+    st.router_logits, st.W_gu, st.W_d, st.y = (t.data_ptr() for t in (router_logits, W_gu, W_d, y))
+    for name in _MOE_PARAMS:
+        setattr(st, name, adapters[name].data_ptr())
+    st.adapters_bf16 = int(dtype == torch.bfloat16)
+    _lib.check(lib.artk_moe_experts_fwd(ref, ws.data_ptr(), ws.numel(), _stream(dev)))
+    return y, rt, saved
+
+
+def moe_experts_bwd(g, x, routing: Routing, saved, Wt_gu, Wt_d, adapters: dict, scale: float):
+    """(dx bf16 [T,H], dict of f32 adapter gradients) for upstream gradient g bf16 [T,H] of moe_experts_fwd's y."""
+    _need(g, "g", torch.bfloat16, tuple(x.shape))
+    E, I, H = Wt_d.shape
+    _need(Wt_d, "Wt_d", torch.bfloat16)
+    _need(Wt_gu, "Wt_gu", torch.bfloat16, (E, H, 2 * I))
+    lib = _lib.load()
+    dev = x.device
+    st, ref = _moe_experts_struct(x, routing, adapters, saved, scale)
+    dx = torch.empty_like(x)
+    grads = {name: torch.empty(adapters[name].shape, dtype=torch.float32, device=dev) for name in _MOE_PARAMS}
+    st.g, st.Wt_gu, st.Wt_d, st.dx = g.data_ptr(), Wt_gu.data_ptr(), Wt_d.data_ptr(), dx.data_ptr()
+    for name, t in grads.items():
+        setattr(st, "d" + name, t.data_ptr())
+    ws = _workspace(lib.artk_moe_experts_bwd_workspace_bytes(ref), dev)
+    _lib.check(lib.artk_moe_experts_bwd(ref, ws.data_ptr(), ws.numel(), _stream(dev)))
+    return dx, grads
+
+
 # -----------------------------------------------------------------------------
 # Packed-row attention
 # -----------------------------------------------------------------------------

@@ -247,6 +247,45 @@ int32_t artk_moe_lora_grouped_bwd(const void* g, const void* x, const int32_t* g
                                   int32_t E, int32_t r, void* dx, float* dA, float* dB,
                                   void* workspace, size_t workspace_bytes, artk_stream_t stream);
 
+/* A block of E experts, each a gated MLP with per-expert LoRA on its three projections:
+ *   rt = route(router_logits);  gu = [gate | up](x[token]);  h = silu(gate) up;
+ *   y[t] = sum_j topk_w[t,j] down(h)[row of (t, slot j)]
+ * One call runs routing, the three projections (gate and up as one grouped product), the gating and the
+ * weighted recombination; the backward gives dx and the six adapter gradients (the routing weights and
+ * the base weights have none).  The forward fills `saved`, which the backward of the same block reads.
+ *   x bf16 [T,H]; W_gu bf16 [E,2I,H] (gate rows first), W_d bf16 [E,H,I]; Wt_gu [E,H,2I], Wt_d [E,I,H]
+ *   gate_A, up_A [E,r,H], gate_B, up_B [E,I,r], down_A [E,r,I], down_B [E,H,r]: f32, or bf16 with
+ *   adapters_bf16; they are rounded to bf16 for the products
+ *   topk_idx .. blk_prefix: as in artk_moe_route, written by the forward, read by the backward
+ *   y bf16 [T,H] out; g bf16 [T,H] in; dx bf16 [T,H] out; d* f32 out, shaped as their parameters
+ *   H, I multiples of 64, r a multiple of 8 up to 32, E <= 256, k <= 16; T * k * H * 2 bytes (backward:
+ *   T * k * max(H, 2 I) * 2) below 2 GiB. */
+typedef struct {
+  const void* x;
+  const float* router_logits;
+  const void *W_gu, *W_d, *Wt_gu, *Wt_d;
+  const void *gate_A, *gate_B, *up_A, *up_B, *down_A, *down_B;
+  int32_t* topk_idx;
+  float* topk_w;
+  int32_t *perm, *inv_perm, *row_token, *offsets, *tile_prefix, *blk_prefix;
+  void* saved;
+  size_t saved_bytes;
+  void* y;
+  const void* g;
+  void* dx;
+  float *dgate_A, *dgate_B, *dup_A, *dup_B, *ddown_A, *ddown_B;
+  int64_t T, H, I;
+  int32_t E, k, r, adapters_bf16;
+  float scale;
+} artk_moe_experts_t;
+size_t artk_moe_experts_saved_bytes(const artk_moe_experts_t* a);
+size_t artk_moe_experts_fwd_workspace_bytes(const artk_moe_experts_t* a);
+int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,
+                             artk_stream_t stream);
+size_t artk_moe_experts_bwd_workspace_bytes(const artk_moe_experts_t* a);
+int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,
+                             artk_stream_t stream);
+
 /* out[b,c,r] = in[b,r,c] for n bf16 [R,C] matrices. */
 int32_t artk_transpose_bf16_batched(const void* in, void* out, int64_t n, int64_t R, int64_t C,
                                     artk_stream_t stream);

@@ -295,3 +295,39 @@ def test_moe_block_autograd(artk_lib, gpu):
     assert rel_l2(x.grad.cpu().float(), xr.grad) <= 2e-2
     for n in ("gate_lora_A", "gate_lora_B", "up_lora_A", "up_lora_B", "down_lora_A", "down_lora_B"):
         assert rel_l2(getattr(mod, n).grad.cpu(), P[n].grad) <= 2e-2, n
+
+
+@pytest.mark.parametrize("T,H,I,E,k,r,dtype", [
+    (1, 64, 64, 4, 1, 8, torch.float32),        # one row: every other expert empty
+    (37, 192, 320, 5, 3, 24, torch.float32),    # nothing divides a tile; odd k
+    (300, 128, 64, 3, 3, 32, torch.bfloat16),   # every expert gets every token; bf16 adapters, largest rank
+    (70, 128, 128, 24, 12, 8, torch.float32),   # more slots than one round of the recombination
+])
+def test_moe_experts_entry_points(artk_lib, gpu, T, H, I, E, k, r, dtype):
+    """artk_moe_experts_fwd / _bwd against the fp32 oracle on the same bf16-valued inputs.  2e-2 as in
+    test_moe_block_autograd: three bf16-rounded products (4e-3 relative each way) in a row."""
+    print("moe experts", T, H, I, E, k, r, dtype, flush=True)
+    g = torch.Generator().manual_seed(T + H)
+    rnd = lambda *s, std=1.0: (std * torch.randn(*s, generator=g)).to(torch.bfloat16)
+    x, up, logits = rnd(T, H), rnd(T, H), torch.randn(T, E, generator=g)
+    Wgu, Wd = rnd(E, 2 * I, H, std=H ** -0.5), rnd(E, H, I, std=I ** -0.5)
+    P = {"gate_A": rnd(E, r, H, std=H ** -0.5), "gate_B": rnd(E, I, r, std=0.1), "up_A": rnd(E, r, H, std=H ** -0.5),
+         "up_B": rnd(E, I, r, std=0.1), "down_A": rnd(E, r, I, std=I ** -0.5), "down_B": rnd(E, H, r, std=0.1)}
+    ref = moe_oracle.route(logits, k)
+    xr = x.float().requires_grad_(True)
+    Pr = {n: p.float().requires_grad_(True) for n, p in P.items()}
+    off, rows = ref["offsets"], xr[ref["row_token"]]
+    gate = moe_oracle.grouped_lora(rows, Wgu[:, :I].float(), Pr["gate_A"], Pr["gate_B"], 0.5, off)
+    u = moe_oracle.grouped_lora(rows, Wgu[:, I:].float(), Pr["up_A"], Pr["up_B"], 0.5, off)
+    down = moe_oracle.grouped_lora(torch.nn.functional.silu(gate) * u, Wd.float(), Pr["down_A"], Pr["down_B"], 0.5, off)
+    y0 = (down[ref["inv_perm"]].view(T, k, H) * ref["topk_w"].unsqueeze(-1)).sum(1)
+    y0.backward(up.float())
+    ad = {n: p.to(dtype).to(gpu) for n, p in P.items()}
+    y, rt, saved = ops.moe_experts_fwd(x.to(gpu), logits.to(gpu), k, Wgu.to(gpu), Wd.to(gpu), ad, 0.5)
+    dx, grads = ops.moe_experts_bwd(up.to(gpu), x.to(gpu), rt, saved, ops.transpose_batched(Wgu.to(gpu)),
+                                    ops.transpose_batched(Wd.to(gpu)), ad, 0.5)
+    assert torch.equal(rt.topk_idx.cpu().long(), ref["topk_idx"].long())
+    assert rel_l2(y.cpu().float(), y0.detach()) <= 2e-2
+    assert rel_l2(dx.cpu().float(), xr.grad) <= 2e-2
+    for n in P:
+        assert grads[n].shape == P[n].shape and rel_l2(grads[n].cpu(), Pr[n].grad) <= 2e-2, n
