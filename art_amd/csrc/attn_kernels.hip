@@ -10,14 +10,20 @@
 // the attention kernels walk only the visible blocks and evaluate the rule per
 // element only in the partly visible ones.
 //
-// Forward work-group: 256 queries x one head, 8 wavefronts of 32 queries, key
-// tiles of 64.  Scores are computed transposed (S^T = K Q^T, MFMA 32x32x16), so
-// that a lane owns one query: the row maximum and sum are in-lane reductions
-// plus one exchange between the two half-waves, the accumulator of S^T is
-// already in the B-operand layout of the second product O^T = V^T P^T, and the
-// running rescale of O^T is a per-lane scalar.  K tiles ([key][d]) and V^T
-// tiles ([d][key], from a transposed copy of V made once per call) are brought
-// into a 3-stage LDS ring by buffer_load ... lds.
+// Forward work-group: 128 queries x one head, 4 wavefronts of 32 queries, key
+// tiles of 64, two work-groups per CU (three at a head dimension of 64).  Scores
+// are computed transposed (S^T = K Q^T, MFMA 32x32x16), so that a lane owns one
+// query: the row maximum and sum are in-lane reductions plus one exchange between
+// the two half-waves, the accumulator of S^T is already in the B-operand layout of
+// the second product O^T = V^T P^T, and the running rescale of O^T is a per-lane
+// scalar.  K and V tiles are brought into a 2-stage LDS ring by buffer_load ... lds.
+// Bound: MFMA plus the softmax's vector work, and for packed rows (lists of a few
+// tiles) the set-up of a work-group.  Two independent work-groups per CU hide the
+// one's set-up and store behind the other's tiles, and a list is made for 128
+// queries instead of 256.  Against one work-group of 8 waves per CU with three
+// stages, 16384 positions of 8 prompts of 137 + 4 x 461, 28 / 4 heads of 128:
+// forward 214 -> 174 us, dQ 291 -> 241 us, dK/dV with its sums 470 -> 330 us;
+// a dense causal row (1.1 PFLOP/s) is level.
 #include <stdlib.h>
 
 #include "common.hpp"
@@ -25,17 +31,14 @@
 
 namespace artk {
 
-constexpr int ATT_BM = 256;    // queries per work-group
+constexpr int ATT_ROW = 256;   // row lengths are multiples of this
+constexpr int ATT_BM = 128;    // queries per work-group
 constexpr int ATT_BN = 64;     // keys per tile
-constexpr int ATT_STAGES = 3;
+constexpr int ATT_STAGES = 2;
 constexpr float ATT_LAZY = 8.f;   // forward: how far a score may exceed the exponentials' reference (log2 units)
 constexpr int ATT_MAX_KB = 1024;  // key blocks per row the list in LDS can hold
 constexpr int ATT_BQ2 = 64;    // dK/dV kernel: queries per tile
-constexpr int ATT_BK2 = 128;   // dK/dV kernel: keys per work-group (4 key groups x 32)
-// dK/dV with grouped-query heads: a key block seen by at most this many (query
-// tile, head) pairs is handled by ONE work-group for all heads of its group (no
-// partial sums); busier blocks get one work-group per head.
-constexpr int ATT_LIGHT_MAX = 64;
+constexpr int ATT_BK2 = 64;    // dK/dV kernel: keys per work-group (2 key groups x 32)
 
 // ----------------------------------------------------------------------------
 // Plan
@@ -78,12 +81,12 @@ __device__ __forceinline__ bool attn_visible(int i, int j, int gi, int pi, int g
 // Visibility of one (owner block, tile) pair, per wavefront of the kernel that
 // will process it:
 //   bits 14-15  1 = some pairs visible, 2 = all
-//   bits 16-23  wave w has at least one visible pair in its part of the tile
-//   bits 24-31  every pair of wave w's part is visible (no per-element test needed)
+//   bits 16-19  wave w has at least one visible pair in its part of the tile
+//   bits 24-27  every pair of wave w's part is visible (no per-element test needed)
 // 0 when nothing is visible.
-// MODE 0 (forward, dQ): owner = 256 queries, tile = 64 keys, wave w = queries 32w..32w+31.
-// MODE 1 (dK/dV):      owner = 128 keys, tile = 64 queries, wave w = keys 32(w&3).. x
-//                      queries 32(w>>2)..
+// MODE 0 (forward, dQ): owner = 128 queries, tile = 64 keys, wave w (of 4) = queries 32w..32w+31.
+// MODE 1 (dK/dV):      owner = 64 keys, tile = 64 queries, wave w (of 4) = keys 32(w&1).. x
+//                      queries 32(w>>1)..
 // One wavefront evaluates the rule on every pair of its (owner, tile).
 template <int MODE>
 __global__ __launch_bounds__(256) void attn_classify_kernel(const int* __restrict__ gc,
@@ -98,7 +101,7 @@ __global__ __launch_bounds__(256) void attn_classify_kernel(const int* __restric
     const int q0 = owner * ATT_BM, j = tile * ATT_BN + lane;
     if (tile * ATT_BN <= q0 + ATT_BM - 1) {
       const int gj = gc[j];
-      for (int g = 0; g < 8; ++g) {
+      for (int g = 0; g < ATT_BM / 32; ++g) {
         int cnt = 0;
         for (int ii = 0; ii < 32; ++ii) {
           const int i = q0 + 32 * g + ii;
@@ -111,27 +114,25 @@ __global__ __launch_bounds__(256) void attn_classify_kernel(const int* __restric
   } else {
     const int k0 = owner * ATT_BK2, q0 = tile * ATT_BQ2;
     if (k0 <= q0 + ATT_BQ2 - 1) {
-      for (int iter = 0; iter < 2; ++iter) {
-        const int j = k0 + 64 * iter + lane;
-        const int gj = gc[j];
-        for (int qh = 0; qh < 2; ++qh) {
-          int cnt = 0;
-          for (int ii = 0; ii < 32; ++ii) {
-            const int i = q0 + 32 * qh + ii;
-            cnt += attn_visible(i, j, gc[i], pc[i], gj) ? 1 : 0;
-          }
-          const unsigned long long ab = __ballot(cnt > 0), fb = __ballot(cnt == 32);
-          for (int hh = 0; hh < 2; ++hh) {
-            const int bit = 2 * iter + hh + 4 * qh;
-            any |= (uint32_t)((uint32_t)(ab >> (32 * hh)) != 0u) << bit;
-            all |= (uint32_t)((uint32_t)(fb >> (32 * hh)) == 0xffffffffu) << bit;
-          }
+      const int j = k0 + lane;
+      const int gj = gc[j];
+      for (int qh = 0; qh < 2; ++qh) {
+        int cnt = 0;
+        for (int ii = 0; ii < 32; ++ii) {
+          const int i = q0 + 32 * qh + ii;
+          cnt += attn_visible(i, j, gc[i], pc[i], gj) ? 1 : 0;
+        }
+        const unsigned long long ab = __ballot(cnt > 0), fb = __ballot(cnt == 32);
+        for (int kg = 0; kg < 2; ++kg) {
+          const int bit = kg + 2 * qh;
+          any |= (uint32_t)((uint32_t)(ab >> (32 * kg)) != 0u) << bit;
+          all |= (uint32_t)((uint32_t)(fb >> (32 * kg)) == 0xffffffffu) << bit;
         }
       }
     }
   }
   if (lane == 0) {
-    const uint32_t cls = all == 0xffu ? 2u : 1u;
+    const uint32_t cls = all == 0xfu ? 2u : 1u;
     info[(int64_t)owner * n_tile + tile] = any ? (cls << 14) | (any << 16) | (all << 24) : 0u;
   }
 }
@@ -161,18 +162,41 @@ __global__ __launch_bounds__(256) void attn_compact_kernel(const uint32_t* __res
   if (threadIdx.x == 0) cnt[row] = base;
 }
 
+// order[r] = the block with the r-th largest count (ties: the later block first): work-groups are dispatched
+// in this order, so the long ones do not end up alone at the end of a launch.  Work-group 0 sorts the query
+// blocks, 1 the key blocks (and adds up their counts); at most 1024 counts each, by rank.
+__global__ __launch_bounds__(1024) void attn_order_kernel(const int* __restrict__ cnt, int n, int* __restrict__ order,
+                                                          const int* __restrict__ cnt2, int n2,
+                                                          int* __restrict__ order2, int* __restrict__ total2) {
+  __shared__ int c[ATT_MAX_KB];
+  const bool second = blockIdx.x == 1;
+  const int m = second ? n2 : n;
+  const int t = threadIdx.x;
+  if (t < m) c[t] = (second ? cnt2 : cnt)[t];
+  __syncthreads();
+  if (t >= m) return;
+  int rank = 0, sum = 0;
+  for (int i = 0; i < m; ++i) sum += c[i];
+  if (second && t == 0) *total2 = sum;
+  for (int i = 0; i < m; ++i) rank += (c[i] > c[t] || (c[i] == c[t] && i > t)) ? 1 : 0;
+  (second ? order2 : order)[rank] = t;
+}
+
 // Device-memory layout of a plan for a row of S positions (S % 256 == 0).
 struct AttnPlan {
   int* gc;
   int* pc;
-  int nQb, nKb;        // forward / dQ: query blocks of 256, key tiles of 64
+  int nQb, nKb;        // forward / dQ: query blocks of 128, key tiles of 64
   uint32_t* info;      // [nQb][nKb]
   uint32_t* list;      // [nQb][nKb]
   int* cnt;            // [nQb]
-  int nQb2, nKb2;      // dK/dV: key blocks of 128, query tiles of 64
+  int* order;          // [nQb] query blocks by falling number of visible tiles
+  int nQb2, nKb2;      // dK/dV: key blocks of 64, query tiles of 64
   uint32_t* info2;     // [nKb2][nQb2]
   uint32_t* list2;     // [nKb2][nQb2]
   int* cnt2;           // [nKb2]
+  int* order2;         // [nKb2]
+  int* total2;         // sum of cnt2
 };
 
 static size_t attn_plan_layout(void* base, size_t bytes, int64_t S, AttnPlan& pl) {
@@ -186,9 +210,12 @@ static size_t attn_plan_layout(void* base, size_t bytes, int64_t S, AttnPlan& pl
   pl.info = ws.take<uint32_t>((size_t)pl.nQb * pl.nKb);
   pl.list = ws.take<uint32_t>((size_t)pl.nQb * pl.nKb);
   pl.cnt = ws.take<int>((size_t)pl.nQb);
+  pl.order = ws.take<int>((size_t)pl.nQb);
   pl.info2 = ws.take<uint32_t>((size_t)pl.nQb2 * pl.nKb2);
   pl.list2 = ws.take<uint32_t>((size_t)pl.nQb2 * pl.nKb2);
   pl.cnt2 = ws.take<int>((size_t)pl.nKb2);
+  pl.order2 = ws.take<int>((size_t)pl.nKb2);
+  pl.total2 = ws.take<int>(1);
   return ws.ok() || base == nullptr ? ws.used : (size_t)-1;
 }
 
@@ -208,8 +235,7 @@ struct AttnTile {
   static constexpr int CHK = D / 8;                    // 16-byte chunks of a row
   static constexpr int ROW = D * 2;                    // bytes
   static constexpr int BYTES = 64 * ROW;
-  static constexpr int N8 = BYTES / 1024 / 8;          // DMA instructions per wave, 8 waves
-  static constexpr int N4 = BYTES / 1024 / 4;          // 4 waves
+  static constexpr int N4 = BYTES / 1024 / 4;          // DMA instructions per wave
   // XOR applied to the chunk index of a row.  Two access patterns must be free of
   // bank conflicts (256 bytes = 16 chunk slots per bank line; with D = 64 two rows
   // share a line): a row-fragment read takes one chunk of 16 consecutive rows, a
@@ -293,6 +319,25 @@ __device__ __forceinline__ dma_rsrc_t attn_rsrc(const void* p) { return dma_make
 // ----------------------------------------------------------------------------
 // Forward
 // ----------------------------------------------------------------------------
+constexpr int ATT_THREADS = 2 * ATT_BM;  // forward and dQ: a wave per 32 queries
+
+// (query head, query block) of a work-group of the forward and dQ kernels.  A unit is the work-groups of
+// the heads that share one key/value head and query block: they read the same K and V tiles, so a unit
+// runs on one XCD (block b is placed on XCD b % 8), its heads one after the other; long blocks first.
+__device__ __forceinline__ bool attn_block(int Hq, int Hkv, int nQb, const int* order, int& hq, int& qb) {
+  const int rep = Hq / Hkv;
+  const int x = blockIdx.x & 7, loc = blockIdx.x >> 3;
+  const int unit = (loc / rep) * 8 + x;
+  const int hkv = unit % Hkv;
+  hq = hkv * rep + loc % rep;
+  if (unit / Hkv >= nQb) return false;
+  qb = order[unit / Hkv];
+  return true;
+}
+static unsigned attn_grid(int Hq, int Hkv, int nQb) {
+  return (unsigned)((nQb * Hkv + 7) / 8 * 8 * (Hq / Hkv));
+}
+
 struct AttnFwdParams {
   const uint16_t* Q;   // element (s, h, d) at s * q_ss + h * q_hs + d
   const uint16_t* K;
@@ -304,6 +349,7 @@ struct AttnFwdParams {
   const int* pc;
   const uint32_t* list;
   const int* cnt;
+  const int* order;
   int S, Hq, Hkv, nQb, nKb;
   float scale_log2e;
 };
@@ -315,7 +361,6 @@ struct AttnKvStage {
   static constexpr int V_OFF = T::BYTES;
   static constexpr int CODE_OFF = 2 * T::BYTES;
   static constexpr int STAGE = CODE_OFF + 1024;
-  static constexpr int N_PER = 2 * T::N8 + 1;
 };
 
 // DMA of key block kb into one stage: this wave's share of the K and V tiles,
@@ -331,16 +376,16 @@ __device__ __forceinline__ void attn_issue_kv(char* st, int kb, dma_rsrc_t rsrc_
   using G = AttnKvStage<D>;
   const int k0 = kb * ATT_BN;
 #pragma unroll
-  for (int i = 0; i < T::N8; ++i)
-    dma_load16(rsrc_k, voff_k[i], (int)(k0 * k_ss * 2), lds_addr_of(st + (wave * T::N8 + i) * 1024));
+  for (int i = 0; i < T::N4; ++i)
+    dma_load16(rsrc_k, voff_k[i], (int)(k0 * k_ss * 2), lds_addr_of(st + (wave * T::N4 + i) * 1024));
 #pragma unroll
-  for (int i = 0; i < T::N8; ++i)
-    dma_load16(rsrc_v, voff_v[i], (int)(k0 * v_ss * 2), lds_addr_of(st + G::V_OFF + (wave * T::N8 + i) * 1024));
+  for (int i = 0; i < T::N4; ++i)
+    dma_load16(rsrc_v, voff_v[i], (int)(k0 * v_ss * 2), lds_addr_of(st + G::V_OFF + (wave * T::N4 + i) * 1024));
   dma_load4(rsrc_c, lane * 4, k0 * 4, lds_addr_of(st + G::CODE_OFF));
 }
 
 template <int D>
-__global__ __launch_bounds__(512) void attn_fwd_kernel(AttnFwdParams p) {
+__global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_fwd_kernel(AttnFwdParams p) {
   using T = AttnTile<D>;
   using G = AttnKvStage<D>;
   // one LDS object for the stages and the tile list (see attn_smem_note)
@@ -349,13 +394,13 @@ __global__ __launch_bounds__(512) void attn_fwd_kernel(AttnFwdParams p) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5;
   const TrLane tr(lane);
-  const int hq = blockIdx.x % p.Hq;
-  const int qb = p.nQb - 1 - (int)(blockIdx.x / p.Hq);  // long rows first
+  int hq, qb;
+  if (!attn_block(p.Hq, p.Hkv, p.nQb, p.order, hq, qb)) return;
   const int hkv = hq / (p.Hq / p.Hkv);
   const int q = qb * ATT_BM + wave * 32 + n;
   const int cnt = p.cnt[qb];
 
-  for (int i = threadIdx.x; i < cnt; i += 512) s_list[i] = p.list[(int64_t)qb * p.nKb + i];
+  for (int i = threadIdx.x; i < cnt; i += ATT_THREADS) s_list[i] = p.list[(int64_t)qb * p.nKb + i];
 
   // this lane's query as B-operand fragments of S^T = K Q^T
   bf16x8 qf[D / 16];
@@ -369,11 +414,11 @@ __global__ __launch_bounds__(512) void attn_fwd_kernel(AttnFwdParams p) {
   const dma_rsrc_t rsrc_k = attn_rsrc(p.K + (int64_t)hkv * p.k_hs);
   const dma_rsrc_t rsrc_v = attn_rsrc(p.V + (int64_t)hkv * p.v_hs);
   const dma_rsrc_t rsrc_c = attn_rsrc(p.gc);
-  int voff_k[T::N8], voff_v[T::N8];
+  int voff_k[T::N4], voff_v[T::N4];
 #pragma unroll
-  for (int i = 0; i < T::N8; ++i) {
-    voff_k[i] = T::voff(wave * T::N8 + i, lane, p.k_ss);
-    voff_v[i] = T::voff(wave * T::N8 + i, lane, p.v_ss);
+  for (int i = 0; i < T::N4; ++i) {
+    voff_k[i] = T::voff(wave * T::N4 + i, lane, p.k_ss);
+    voff_v[i] = T::voff(wave * T::N4 + i, lane, p.v_ss);
   }
   __syncthreads();  // s_list
   auto* list_lds = s_list;
@@ -393,21 +438,15 @@ __global__ __launch_bounds__(512) void attn_fwd_kernel(AttnFwdParams p) {
   pin_loaded(gi);
   pin_loaded(pi);
   if (cnt > 0) ATTN_ISSUE(0, 0);
-  if (cnt > 1) ATTN_ISSUE(1, 1);
-  int stage = 0;
   for (int it = 0; it < cnt; ++it) {
-    if (it + 1 < cnt)
-      wait_vmcnt<G::N_PER>();
-    else
-      wait_vmcnt<0>();
+    wait_vmcnt<0>();
     barrier_lds_only();
-    if (it + 2 < cnt) ATTN_ISSUE(it + 2, stage >= 1 ? stage - 1 : ATT_STAGES - 1);
+    if (it + 1 < cnt) ATTN_ISSUE(it + 1, (it + 1) & 1);
     const int entry = __builtin_amdgcn_readfirstlane(s_list[it]);
     const int kb = entry & 0x3fff;
     const bool active = (entry >> (16 + wave)) & 1;        // this wave's 32 queries see part of the tile
     const bool partial = !((entry >> (24 + wave)) & 1);     // ... but not all of it
-    const char* st = smem + stage * G::STAGE;
-    stage = stage + 1 == ATT_STAGES ? 0 : stage + 1;
+    const char* st = smem + (it & 1) * G::STAGE;
     if (!active) continue;  // nothing of this tile is visible to this wave's queries
 
     // S^T tiles: keys 0..31 and 32..63 of the block x this wave's 32 queries
@@ -459,7 +498,10 @@ __global__ __launch_bounds__(512) void attn_fwd_kernel(AttnFwdParams p) {
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
       for (int j = 0; j < 16; ++j) mloc = fmaxf(mloc, sc[kt][j]);
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64)) * p.scale_log2e;
+    {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mloc), __float_as_uint(mloc), false, false);
+      mloc = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * p.scale_log2e;  // both halves of a query
+    }
     // The reference of the exponentials follows the running maximum lazily: it moves only when
     // some query of the wave has a score more than ATT_LAZY (in units of log2) above it, so the
     // 64 output accumulators are rescaled on few tiles instead of on most early ones.  Until
@@ -502,16 +544,13 @@ __global__ __launch_bounds__(512) void attn_fwd_kernel(AttnFwdParams p) {
 
   const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  uint16_t* op = p.O + (int64_t)q * p.o_ss + (int64_t)hq * p.o_hs + 4 * h;
+  uint16_t* op = p.O + (int64_t)q * p.o_ss + (int64_t)hq * p.o_hs;
 #pragma unroll
-  for (int dt = 0; dt < D / 32; ++dt)
+  for (int dt = 0; dt < D / 32; ++dt) {
 #pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      bf16x4 v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = (__bf16)(o[dt][4 * g4 + e] * inv);
-      *(bf16x4*)(op + 32 * dt + 8 * g4) = v;
-    }
+    for (int j = 0; j < 16; ++j) o[dt][j] *= inv;
+    store_block_bf16(op + 32 * dt, o[dt], h);
+  }
   if (h == 0) p.lse[(int64_t)hq * p.S + q] = (m_run + __builtin_amdgcn_logf(l_tot)) * LN2;
 }
 
@@ -525,6 +564,30 @@ __global__ __launch_bounds__(512) void attn_fwd_kernel(AttnFwdParams p) {
 // a block of queries and accumulates dQ over its visible key tiles.  Each
 // recomputes P from lse.
 // ----------------------------------------------------------------------------
+// How many heads of a group one dK/dV work-group takes for a key block with cnt query tiles.
+// A step is one (query tile, head); a work-group that takes all heads of a group writes dK and dV directly,
+// shares write fp32 partial sums.  So shares are as large as still lets the launch fill the GPU evenly: a
+// quarter of the steps that a resident work-group gets on average, two thirds where the key blocks alone
+// are at least two rounds of work-groups.  Backward in us by the divisor of that average (tenths):
+//   16384 positions, 8 prompts of 137 + 4 x 461, 28 / 4 heads of 128 (two rounds):  6: 629, 15: 595, 40: 623, 100: 707
+//   the same with 16 / 2 heads (one round):                                         15: 497, 30: 423, 40: 409, 100: 425
+//   8192 positions, 28 / 4 heads (one round):                                       15: 319, 30: 337, 40: 350, 100: 376
+//   16384 positions, one prompt of 900 + 2 x 7700, 16 / 2 heads (one round):        15: 2994, 30: 2483, 40: 2368, 100: 2273
+struct AttnKvSplit {
+  const int* total;  // steps of one head, from the plan
+  int heads_all;     // query heads
+  int div;           // steps of a share = total * heads_all / div
+  int light_max;     // >= 0 (artk_attn_bwd_tuning): all heads where they make at most this many steps, else one
+  __device__ __forceinline__ int heads(int cnt, int rep) const {
+    if (light_max >= 0) return cnt * rep <= light_max ? rep : 1;
+    const int steps = (int)((int64_t)*total * heads_all / div);
+    int g = cnt > 0 ? steps / cnt : rep;
+    g = g < 1 ? 1 : (g > rep ? rep : g);
+    const int groups = (rep + g - 1) / g;
+    return (rep + groups - 1) / groups;   // even shares
+  }
+};
+
 struct AttnBwdParams {
   const uint16_t *Q, *K, *V, *dO;
   const float* lse2;                // [Hq][S]  lse * log2(e)
@@ -534,12 +597,14 @@ struct AttnBwdParams {
   int64_t q_ss, q_hs, k_ss, k_hs, v_ss, v_hs, do_ss, do_hs, dq_ss, dq_hs, dk_ss, dk_hs, dv_ss, dv_hs;
   const int* gc;
   const int* pc;
-  const uint32_t* list;    // per query block of 256: key tiles of 64
+  const uint32_t* list;    // per query block of 128: key tiles of 64
   const int* cnt;
-  const uint32_t* listT;   // per key block of 128: query tiles of 64
+  const int* order;
+  const uint32_t* listT;   // per key block of 64: query tiles of 64
   const int* cntT;
+  const int* orderT;
   int S, Hq, Hkv, nQb, nKb, nQb2, nKb2;
-  int light_max;           // see ATT_LIGHT_MAX; 0 when there are too few key blocks to fill the GPU that way
+  AttnKvSplit split;
   float scale, scale_log2e;
 };
 
@@ -574,7 +639,7 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const uint16_t* __restr
 
 // ---- dQ: 256 queries x one head per work-group, lane = query ----------------
 template <int D>
-__global__ __launch_bounds__(512) void attn_bwd_dq_kernel(AttnBwdParams p) {
+__global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kernel(AttnBwdParams p) {
   using T = AttnTile<D>;
   using G = AttnKvStage<D>;
   // one LDS object for the stages and the tile list (see attn_smem_note)
@@ -583,12 +648,12 @@ __global__ __launch_bounds__(512) void attn_bwd_dq_kernel(AttnBwdParams p) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5;
   const TrLane tr(lane);
-  const int hq = blockIdx.x % p.Hq;
-  const int qb = p.nQb - 1 - (int)(blockIdx.x / p.Hq);
+  int hq, qb;
+  if (!attn_block(p.Hq, p.Hkv, p.nQb, p.order, hq, qb)) return;
   const int hkv = hq / (p.Hq / p.Hkv);
   const int q = qb * ATT_BM + wave * 32 + n;
   const int cnt = p.cnt[qb];
-  for (int i = threadIdx.x; i < cnt; i += 512) s_list[i] = p.list[(int64_t)qb * p.nKb + i];
+  for (int i = threadIdx.x; i < cnt; i += ATT_THREADS) s_list[i] = p.list[(int64_t)qb * p.nKb + i];
 
   bf16x8 qf[D / 16], dof[D / 16];
   {
@@ -607,11 +672,11 @@ __global__ __launch_bounds__(512) void attn_bwd_dq_kernel(AttnBwdParams p) {
   const dma_rsrc_t rsrc_k = attn_rsrc(p.K + (int64_t)hkv * p.k_hs);
   const dma_rsrc_t rsrc_v = attn_rsrc(p.V + (int64_t)hkv * p.v_hs);
   const dma_rsrc_t rsrc_c = attn_rsrc(p.gc);
-  int voff_k[T::N8], voff_v[T::N8];
+  int voff_k[T::N4], voff_v[T::N4];
 #pragma unroll
-  for (int i = 0; i < T::N8; ++i) {
-    voff_k[i] = T::voff(wave * T::N8 + i, lane, p.k_ss);
-    voff_v[i] = T::voff(wave * T::N8 + i, lane, p.v_ss);
+  for (int i = 0; i < T::N4; ++i) {
+    voff_k[i] = T::voff(wave * T::N4 + i, lane, p.k_ss);
+    voff_v[i] = T::voff(wave * T::N4 + i, lane, p.v_ss);
   }
   __syncthreads();
   auto* list_lds = s_list;
@@ -635,22 +700,16 @@ __global__ __launch_bounds__(512) void attn_bwd_dq_kernel(AttnBwdParams p) {
   pin_loaded(nlse2);
   pin_loaded(delta);
   if (cnt > 0) ATTN_ISSUE(0, 0);
-  if (cnt > 1) ATTN_ISSUE(1, 1);
-  int stage = 0;
   for (int it = 0; it < cnt; ++it) {
-    if (it + 1 < cnt)
-      wait_vmcnt<G::N_PER>();
-    else
-      wait_vmcnt<0>();
+    wait_vmcnt<0>();
     barrier_lds_only();
-    if (it + 2 < cnt) ATTN_ISSUE(it + 2, stage >= 1 ? stage - 1 : ATT_STAGES - 1);
+    if (it + 1 < cnt) ATTN_ISSUE(it + 1, (it + 1) & 1);
     const int entry = __builtin_amdgcn_readfirstlane(s_list[it]);
     const int kb = entry & 0x3fff;
     const bool active = (entry >> (16 + wave)) & 1;        // this wave's 32 queries see part of the tile
     const bool partial = !((entry >> (24 + wave)) & 1);     // ... but not all of it
-    const char* st = smem + stage * G::STAGE;
+    const char* st = smem + (it & 1) * G::STAGE;
     const int* codes = (const int*)(st + G::CODE_OFF);
-    stage = stage + 1 == ATT_STAGES ? 0 : stage + 1;
     if (!active) continue;
 
     bf16x8 dsf[4];
@@ -693,43 +752,38 @@ __global__ __launch_bounds__(512) void attn_bwd_dq_kernel(AttnBwdParams p) {
     }
   }
 #undef ATTN_ISSUE
-  uint16_t* op = p.dQ + (int64_t)q * p.dq_ss + (int64_t)hq * p.dq_hs + 4 * h;
+  uint16_t* op = p.dQ + (int64_t)q * p.dq_ss + (int64_t)hq * p.dq_hs;
 #pragma unroll
-  for (int dt = 0; dt < D / 32; ++dt)
+  for (int dt = 0; dt < D / 32; ++dt) {
 #pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      bf16x4 v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = (__bf16)(dq[dt][4 * g4 + e] * p.scale);
-      *(bf16x4*)(op + 32 * dt + 8 * g4) = v;
-    }
+    for (int j = 0; j < 16; ++j) dq[dt][j] *= p.scale;
+    store_block_bf16(op + 32 * dt, dq[dt], h);
+  }
 }
 
-// ---- dK, dV: 128 keys x one query head per work-group, lane = key ------------
-// 8 wavefronts = 4 key groups of 32 x 2 halves of each 64-query tile, so every
-// SIMD holds two waves and the exp2 / convert work of one overlaps the MFMAs of
-// the other.  The two waves of a key group keep separate accumulators, added
-// through LDS at the end.  The K and V rows of the block stay in LDS for the
-// whole kernel (their fragments are re-read per tile: keeping them in
-// registers would push a wave past 256 registers).
-// With grouped-query heads the work-groups of the heads that share a key/value
-// head write fp32 partial sums, which attn_kv_reduce_kernel adds in a fixed order.
+// ---- dK, dV: 64 keys x some query heads of a group per work-group, lane = key ------------
+// 4 wavefronts = 2 key groups of 32 x 2 halves of each 64-query tile; two work-groups per CU (D = 64:
+// three), so that the exp2 / convert work, the DMA latency and the set-up of one overlap the MFMAs of the
+// other.  The two waves of a key group keep separate accumulators, added through LDS at the end.  The K
+// and V rows of the block stay in LDS for the whole kernel (their fragments are re-read per tile: keeping
+// them in registers would push a wave past 256 registers).
+// A work-group that does not take all heads of its group writes fp32 partial sums, which
+// attn_kv_reduce_kernel adds in a fixed order.
 // LDS stage: Q tile, dO tile (64 queries), and lse2 / delta / group / parent codes
-// of those queries.
+// of those queries.  D = 128 has room for one stage per work-group only.
 template <int D>
 struct AttnQStage {
   using T = AttnTile<D>;
   static constexpr int DO_OFF = T::BYTES;
   static constexpr int ROW_OFF = 2 * T::BYTES;
   static constexpr int STAGE = ROW_OFF + 1024;
-  static constexpr int NSTAGE = 2;
-  static constexpr int KV_OFF = NSTAGE * STAGE;          // K block (2 tiles), then V block
-  static constexpr int LDS = KV_OFF + 4 * T::BYTES;
+  static constexpr int NSTAGE = 1;
+  static constexpr int KV_OFF = NSTAGE * STAGE;          // K block, then V block
+  static constexpr int LDS = KV_OFF + 2 * T::BYTES;
 };
 
 // DMA of one query tile into a stage: this wave's share of the Q and dO tiles and
-// one of the four per-query arrays (wave & 3 = 0: lse2, 1: delta, 2: group codes,
-// 3: parent codes; the upper four waves write the same bytes again).
+// one of the four per-query arrays (wave 0: lse2, 1: delta, 2: group codes, 3: parent codes).
 template <int D>
 __device__ __forceinline__ void attn_issue_q(char* st, int hq, int q0, dma_rsrc_t rsrc_q,
                                              dma_rsrc_t rsrc_do,
@@ -741,15 +795,15 @@ __device__ __forceinline__ void attn_issue_q(char* st, int hq, int q0, dma_rsrc_
   const int so_q = (int)((q0 * p.q_ss + hq * p.q_hs) * 2);
   const int so_do = (int)((q0 * p.do_ss + hq * p.do_hs) * 2);
 #pragma unroll
-  for (int i = 0; i < T::N8; ++i) {
-    dma_load16(rsrc_q, voff_q[i], so_q, lds_addr_of(st + (wave * T::N8 + i) * 1024));
-    dma_load16(rsrc_do, voff_do[i], so_do, lds_addr_of(st + G::DO_OFF + (wave * T::N8 + i) * 1024));
+  for (int i = 0; i < T::N4; ++i) {
+    dma_load16(rsrc_q, voff_q[i], so_q, lds_addr_of(st + (wave * T::N4 + i) * 1024));
+    dma_load16(rsrc_do, voff_do[i], so_do, lds_addr_of(st + G::DO_OFF + (wave * T::N4 + i) * 1024));
   }
-  const int arr = wave & 3;
+  const int arr = wave;
   dma_load4(rsrc_row, lane * 4, (int)(((arr < 2 ? (int64_t)hq * p.S : 0) + q0) * 4), lds_addr_of(st + G::ROW_OFF + arr * 256));
 }
 
-// The block's K and V rows (128 each = two 64-row tiles per operand).
+// The block's K and V rows (64 each).
 template <int D>
 __device__ __forceinline__ void attn_issue_kv_block(char* dst, int key0, dma_rsrc_t rsrc_k,
                                                     dma_rsrc_t rsrc_v, const int* voff_k,
@@ -757,16 +811,14 @@ __device__ __forceinline__ void attn_issue_kv_block(char* dst, int key0, dma_rsr
                                                     int wave) {
   using T = AttnTile<D>;
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int i = 0; i < T::N8; ++i) {
-      dma_load16(rsrc_k, voff_k[i], (int)((key0 + 64 * t) * k_ss * 2), lds_addr_of(dst + t * T::BYTES + (wave * T::N8 + i) * 1024));
-      dma_load16(rsrc_v, voff_v[i], (int)((key0 + 64 * t) * v_ss * 2), lds_addr_of(dst + (2 + t) * T::BYTES + (wave * T::N8 + i) * 1024));
-    }
+  for (int i = 0; i < T::N4; ++i) {
+    dma_load16(rsrc_k, voff_k[i], (int)(key0 * k_ss * 2), lds_addr_of(dst + (wave * T::N4 + i) * 1024));
+    dma_load16(rsrc_v, voff_v[i], (int)(key0 * v_ss * 2), lds_addr_of(dst + T::BYTES + (wave * T::N4 + i) * 1024));
+  }
 }
 
 template <int D>
-__global__ __launch_bounds__(512) void attn_bwd_kv_kernel(AttnBwdParams p) {
+__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnBwdParams p) {
   using T = AttnTile<D>;
   using G = AttnQStage<D>;
   // one LDS object for the stages and the tile list (see attn_smem_note)
@@ -774,35 +826,36 @@ __global__ __launch_bounds__(512) void attn_bwd_kv_kernel(AttnBwdParams p) {
   uint32_t* const s_list = (uint32_t*)(smem + G::LDS);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5;
-  const int kg = wave & 3, qh = wave >> 2;
+  const int kg = wave & 1, qh = wave >> 1;
   const TrLane tr(lane);
-  const int hq = blockIdx.x % p.Hq;
-  const int kb = (int)(blockIdx.x / p.Hq);  // early key blocks are seen by the most queries
+  int hq, kb;
+  if (!attn_block(p.Hq, p.Hkv, p.nKb2, p.orderT, hq, kb)) return;
   const int rep = p.Hq / p.Hkv;
-  const int hkv = hq / rep;
+  const int hkv = hq / rep, share = hq - hkv * rep;
   const int key = kb * ATT_BK2 + kg * 32 + n;
   const int cnt = p.cntT[kb];
-  const bool light = rep > 1 && cnt * rep <= p.light_max;
-  if (light && hq != hkv * rep) return;  // the group's first head does all of them
-  const int nheads = light ? rep : 1;
-  for (int i = threadIdx.x; i < cnt; i += 512) s_list[i] = p.listT[(int64_t)kb * p.nQb2 + i];
+  const int per = p.split.heads(cnt, rep);
+  if (share * per >= rep) return;
+  hq = hkv * rep + share * per;  // first head of this work-group's share
+  const int nheads = rep - share * per < per ? rep - share * per : per;
+  for (int i = threadIdx.x; i < cnt; i += 256) s_list[i] = p.listT[(int64_t)kb * p.nQb2 + i];
   int gk = p.gc[key];
 
   const dma_rsrc_t rsrc_q = attn_rsrc(p.Q);
   const dma_rsrc_t rsrc_do = attn_rsrc(p.dO);
-  const int arr = wave & 3;
+  const int arr = wave;
   const void* row_src = arr == 0 ? (const void*)p.lse2 : arr == 1 ? (const void*)p.delta
                         : arr == 2 ? (const void*)p.gc : (const void*)p.pc;
   const dma_rsrc_t rsrc_row = attn_rsrc(row_src);
-  int voff_q[T::N8], voff_do[T::N8];
+  int voff_q[T::N4], voff_do[T::N4];
   {
-    int voff_k[T::N8], voff_v[T::N8];
+    int voff_k[T::N4], voff_v[T::N4];
 #pragma unroll
-    for (int i = 0; i < T::N8; ++i) {
-      voff_q[i] = T::voff(wave * T::N8 + i, lane, p.q_ss);
-      voff_do[i] = T::voff(wave * T::N8 + i, lane, p.do_ss);
-      voff_k[i] = T::voff(wave * T::N8 + i, lane, p.k_ss);
-      voff_v[i] = T::voff(wave * T::N8 + i, lane, p.v_ss);
+    for (int i = 0; i < T::N4; ++i) {
+      voff_q[i] = T::voff(wave * T::N4 + i, lane, p.q_ss);
+      voff_do[i] = T::voff(wave * T::N4 + i, lane, p.do_ss);
+      voff_k[i] = T::voff(wave * T::N4 + i, lane, p.k_ss);
+      voff_v[i] = T::voff(wave * T::N4 + i, lane, p.v_ss);
     }
     attn_issue_kv_block<D>(smem + G::KV_OFF, kb * ATT_BK2, attn_rsrc(p.K + (int64_t)hkv * p.k_hs),
                            attn_rsrc(p.V + (int64_t)hkv * p.v_hs), voff_k, voff_v, p.k_ss, p.v_ss, wave);
@@ -825,24 +878,28 @@ __global__ __launch_bounds__(512) void attn_bwd_kv_kernel(AttnBwdParams p) {
     for (int j = 0; j < 16; ++j) dk[dt][j] = dv[dt][j] = 0.f;
 
   // this wave's keys inside the resident K / V blocks
-  const char* kblk = smem + G::KV_OFF + (kg >> 1) * T::BYTES;
-  const char* vblk = kblk + 2 * T::BYTES;
-  const int krow = 32 * (kg & 1) + n;
+  const char* kblk = smem + G::KV_OFF;
+  const char* vblk = kblk + T::BYTES;
+  const int krow = 32 * kg + n;
 
   const int total = cnt * nheads;
   pin_loaded(gk);
   if (total > 0) ATTN_ISSUE(0, 0);
   int ti = 0;
   for (int it = 0; it < total; ++it) {
+    if (G::NSTAGE == 1 && it > 0) {
+      barrier_lds_only();  // every wave is done with the tile before
+      ATTN_ISSUE(it, 0);
+    }
     wait_vmcnt<0>();
     barrier_lds_only();
-    if (it + 1 < total) ATTN_ISSUE(it + 1, (it + 1) & 1);
+    if (G::NSTAGE > 1 && it + 1 < total) ATTN_ISSUE(it + 1, (it + 1) & 1);
     const int entry = __builtin_amdgcn_readfirstlane(s_list[ti]);
     ti = ti + 1 == cnt ? 0 : ti + 1;
     const int q0 = (entry & 0x3fff) * ATT_BQ2;
     const bool active = (entry >> (16 + wave)) & 1;        // this wave's keys x query half
     const bool partial = !((entry >> (24 + wave)) & 1);
-    const char* st = smem + (it & 1) * G::STAGE;
+    const char* st = smem + (G::NSTAGE > 1 ? it & 1 : 0) * G::STAGE;
     const char* dot = st + G::DO_OFF;
     const float* r_lse2 = (const float*)(st + G::ROW_OFF);
     const float* r_delta = r_lse2 + 64;
@@ -923,8 +980,8 @@ __global__ __launch_bounds__(512) void attn_bwd_kv_kernel(AttnBwdParams p) {
   }
   if (qh == 1) return;
 
-  if (rep > 1 && !light) {
-    const int64_t o = ((((int64_t)(hq - hkv * rep) * p.S + key) * p.Hkv + hkv) * D) + 4 * h;
+  if (per < rep) {
+    const int64_t o = ((((int64_t)share * p.S + key) * p.Hkv + hkv) * D) + 4 * h;
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
@@ -957,12 +1014,12 @@ __global__ __launch_bounds__(512) void attn_bwd_kv_kernel(AttnBwdParams p) {
     }
 }
 
-// dK = scale * sum_r pK[r], dV = sum_r pV[r] over the query heads r of a group, in
+// dK = scale * sum_r pK[r], dV = sum_r pV[r] over the shares r of a group's heads, in
 // index order; 4 elements per thread.
 __global__ __launch_bounds__(256) void attn_kv_reduce_kernel(const float* __restrict__ pK,
                                                              const float* __restrict__ pV,
                                                              const int* __restrict__ cntT,
-                                                             int light_max, int rep,
+                                                             AttnKvSplit split, int rep,
                                                              int64_t S, int Hkv, int D, float scale,
                                                              uint16_t* __restrict__ dK, int64_t dk_ss,
                                                              int64_t dk_hs, uint16_t* __restrict__ dV,
@@ -974,9 +1031,10 @@ __global__ __launch_bounds__(256) void attn_kv_reduce_kernel(const float* __rest
   const int c = (int)(i % d4);
   const int hh = (int)((i / d4) % Hkv);
   const int64_t s = i / ((int64_t)d4 * Hkv);
-  if (cntT[s / ATT_BK2] * rep <= light_max) return;  // written directly by the dK/dV kernel
+  const int per = split.heads(cntT[s / ATT_BK2], rep);
+  if (per == rep) return;  // written directly by the dK/dV kernel
   floatx4 a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
-  for (int r = 0; r < rep; ++r) {
+  for (int r = 0; r * per < rep; ++r) {
     a += ((const floatx4*)pK)[(int64_t)r * n + i];
     b += ((const floatx4*)pV)[(int64_t)r * n + i];
   }
@@ -1008,8 +1066,8 @@ int32_t artk_attn_plan(const int64_t* group_ids, const int64_t* parent_ids, int6
                        size_t plan_bytes, artk_stream_t stream) {
   ARTK_CHECK_ARG(group_ids && parent_ids && plan, "null pointer argument");
   ARTK_CHECK_ARG(S > 0, "S must be positive");
-  if (S % ATT_BM != 0 || S / ATT_BN > ATT_MAX_KB) {
-    set_error("row length %lld must be a multiple of %d and at most %d", (long long)S, ATT_BM,
+  if (S % ATT_ROW != 0 || S / ATT_BN > ATT_MAX_KB) {
+    set_error("row length %lld must be a multiple of %d and at most %d", (long long)S, ATT_ROW,
               ATT_MAX_KB * ATT_BN);
     return ARTK_ERR_UNSUPPORTED_SHAPE;
   }
@@ -1031,14 +1089,16 @@ int32_t artk_attn_plan(const int64_t* group_ids, const int64_t* parent_ids, int6
   ARTK_CHECK_LAUNCH();
   attn_compact_kernel<<<(unsigned)pl.nKb2, 256, 0, st>>>(pl.info2, pl.nQb2, pl.list2, pl.cnt2);
   ARTK_CHECK_LAUNCH();
+  attn_order_kernel<<<2, 1024, 0, st>>>(pl.cnt, pl.nQb, pl.order, pl.cnt2, pl.nKb2, pl.order2, pl.total2);
+  ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }
 
 static int32_t attn_check(int64_t S, int32_t Hq, int32_t Hkv, int32_t D, const int64_t* strides,
                           int nstrides) {
   ARTK_CHECK_ARG(S > 0 && Hq > 0 && Hkv > 0, "S, Hq, Hkv must be positive");
-  if (S % ATT_BM != 0 || S / ATT_BN > ATT_MAX_KB) {
-    set_error("row length %lld must be a multiple of %d and at most %d", (long long)S, ATT_BM,
+  if (S % ATT_ROW != 0 || S / ATT_BN > ATT_MAX_KB) {
+    set_error("row length %lld must be a multiple of %d and at most %d", (long long)S, ATT_ROW,
               ATT_MAX_KB * ATT_BN);
     return ARTK_ERR_UNSUPPORTED_SHAPE;
   }
@@ -1097,18 +1157,19 @@ int32_t artk_attn_fwd(const void* q, const void* k, const void* v, const void* p
   p.pc = pl.pc;
   p.list = pl.list;
   p.cnt = pl.cnt;
+  p.order = pl.order;
   p.S = (int)S;
   p.Hq = Hq;
   p.Hkv = Hkv;
   p.nQb = pl.nQb;
   p.nKb = pl.nKb;
   p.scale_log2e = scale * LOG2E;
-  const unsigned grid = (unsigned)(pl.nQb * Hq);
+  const unsigned grid = attn_grid(Hq, Hkv, pl.nQb);
   prof_begin(PROF_ATTN_FWD, st);
   if (D == 128)
-    attn_fwd_kernel<128><<<grid, 512, 0, st>>>(p);
+    attn_fwd_kernel<128><<<grid, ATT_THREADS, 0, st>>>(p);
   else
-    attn_fwd_kernel<64><<<grid, 512, 0, st>>>(p);
+    attn_fwd_kernel<64><<<grid, ATT_THREADS, 0, st>>>(p);
   prof_end(PROF_ATTN_FWD, st);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
@@ -1182,8 +1243,10 @@ int32_t artk_attn_bwd(const void* q, const void* k, const void* v, const void* o
   p.pc = pl.pc;
   p.list = pl.list;
   p.cnt = pl.cnt;
+  p.order = pl.order;
   p.listT = pl.list2;
   p.cntT = pl.cnt2;
+  p.orderT = pl.order2;
   p.S = (int)S;
   p.Hq = Hq;
   p.Hkv = Hkv;
@@ -1194,29 +1257,31 @@ int32_t artk_attn_bwd(const void* q, const void* k, const void* v, const void* o
   p.scale = scale;
   p.scale_log2e = scale * LOG2E;
   {
-    const int cus = num_cus();
-    p.light_max = pl.nKb2 * Hkv >= cus ? ATT_LIGHT_MAX : 0;
-    if (g_light_max_override >= 0) p.light_max = g_light_max_override;  // artk_attn_bwd_tuning
+    const int slots = num_cus() * (D == 64 ? 3 : 2);  // resident work-groups
+    p.split.total = pl.total2;
+    p.split.heads_all = Hq;
+    p.split.div = pl.nKb2 * Hkv >= 2 * slots ? slots * 3 / 2 : slots * 4;
   }
+  p.split.light_max = g_light_max_override;  // artk_attn_bwd_tuning
   prof_begin(PROF_ATTN_BWD_KV, st);
   if (D == 128)
-    attn_bwd_kv_kernel<128><<<(unsigned)(pl.nKb2 * Hq), 512, 0, st>>>(p);
+    attn_bwd_kv_kernel<128><<<attn_grid(Hq, Hkv, pl.nKb2), 256, 0, st>>>(p);
   else
-    attn_bwd_kv_kernel<64><<<(unsigned)(pl.nKb2 * Hq), 512, 0, st>>>(p);
+    attn_bwd_kv_kernel<64><<<attn_grid(Hq, Hkv, pl.nKb2), 256, 0, st>>>(p);
   prof_end(PROF_ATTN_BWD_KV, st);
   ARTK_CHECK_LAUNCH();
   if (Hq != Hkv) {
     const int64_t n4 = S * Hkv * (D / 4);
     attn_kv_reduce_kernel<<<(unsigned)((n4 + 255) / 256), 256, 0, st>>>(
-        pk, pv, pl.cnt2, p.light_max, Hq / Hkv, S, Hkv, D, scale, (uint16_t*)dk, strides[12], strides[13], (uint16_t*)dv,
+        pk, pv, pl.cnt2, p.split, Hq / Hkv, S, Hkv, D, scale, (uint16_t*)dk, strides[12], strides[13], (uint16_t*)dv,
         strides[14], strides[15]);
     ARTK_CHECK_LAUNCH();
   }
   prof_begin(PROF_ATTN_BWD_Q, st);
   if (D == 128)
-    attn_bwd_dq_kernel<128><<<(unsigned)(pl.nQb * Hq), 512, 0, st>>>(p);
+    attn_bwd_dq_kernel<128><<<attn_grid(Hq, Hkv, pl.nQb), ATT_THREADS, 0, st>>>(p);
   else
-    attn_bwd_dq_kernel<64><<<(unsigned)(pl.nQb * Hq), 512, 0, st>>>(p);
+    attn_bwd_dq_kernel<64><<<attn_grid(Hq, Hkv, pl.nQb), ATT_THREADS, 0, st>>>(p);
   prof_end(PROF_ATTN_BWD_Q, st);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
