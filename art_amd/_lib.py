@@ -68,6 +68,15 @@ SIGNATURES = {
         _i32, [_p, _p, _p, _p, _p, _p, _p, _i64, _i32, _i32, _i32, C.POINTER(_i64), _f32, _p, _p, _p, _p,
                _sz, _p]),
     "artk_attn_bwd_tuning": (_i32, [_i32]),
+    "artk_attn_plan_rows_bytes": (_sz, [_i64, _i64]),
+    "artk_attn_plan_row_stride": (_sz, [_i64]),
+    "artk_attn_plan_rows": (_i32, [_p, _p, _i64, _i64, _p, _sz, _p]),
+    "artk_attn_fwd_rows": (
+        _i32, [_p, _p, _p, _p, _i64, _i64, _i32, _i32, _i32, C.POINTER(_i64), _f32, _p, _p, _p]),
+    "artk_attn_bwd_rows_workspace_bytes": (_sz, [_i64, _i64, _i32, _i32, _i32]),
+    "artk_attn_bwd_rows": (
+        _i32, [_p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _i32, _i32, C.POINTER(_i64), _f32, _p, _p, _p, _p,
+               _sz, _p]),
     "artk_sumsq_f32_workspace_bytes": (_sz, []),
     "artk_sumsq_f32": (_i32, [_p, _i64, _p, _p, _sz, _p]),
     "artk_adamw_step": (_i32, [_p, _p, _p, _p, _p, _i64, _f32, _f32, _f32, _f32, _f32, _i32, _p, _f32, _p]),

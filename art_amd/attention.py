@@ -12,11 +12,9 @@ from typing import List, Optional
 
 import torch
 
-import torch.nn.functional as F
-
 from . import ops
 
-ROW_MULTIPLE = 256  # the kernels take rows whose length is a multiple of this
+ROW_MULTIPLE = 256  # plans cover rows of this granularity; positions past the end see, and are seen by, nothing
 
 
 def attention_plans(group_ids: torch.Tensor, parent_ids: torch.Tensor) -> List[ops.AttnPlan]:
@@ -25,33 +23,24 @@ def attention_plans(group_ids: torch.Tensor, parent_ids: torch.Tensor) -> List[o
     batch; every layer and head reuses them."""
     if group_ids.dim() == 1:
         group_ids, parent_ids = group_ids.unsqueeze(0), parent_ids.unsqueeze(0)
-    S = group_ids.shape[1]
-    extra = -S % ROW_MULTIPLE
-    if extra:
-        # Rows of any length: append positions whose ids no real position carries (as group
-        # or as parent), so they see and are seen by nothing but themselves; packed_attention
-        # pads q, k, v to match and drops their outputs.
-        fill = (torch.minimum(group_ids.amin(), parent_ids.amin()) - 1).reshape(1, 1)
-        fill = fill.expand(group_ids.shape[0], extra)
-        group_ids = torch.cat([group_ids, fill], 1)
-        parent_ids = torch.cat([parent_ids, fill], 1)
-    return [ops.attn_plan(g.contiguous(), p.contiguous()) for g, p in zip(group_ids, parent_ids)]
+    return ops.attn_plan_rows(group_ids.contiguous(), parent_ids.contiguous())
 
 
 class _PackedAttentionFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, plan, scale):
-        out, lse = ops.attn_fwd(q, k, v, plan, scale)
-        ctx.save_for_backward(q, k, v, out, lse)
-        ctx.plan, ctx.scale = plan, scale
+        out, lse = ops.attn_fwd_rows(q, k, v, plan, scale)
+        ctx.save_for_backward(q, k, v, out, lse, plan)
+        ctx.scale = scale
         return out
 
     @staticmethod
     def backward(ctx, d_out):
-        q, k, v, out, lse = ctx.saved_tensors
-        if d_out.stride(2) != 1:
+        q, k, v, out, lse, plan = ctx.saved_tensors
+        d_out = d_out.to(torch.bfloat16)
+        if d_out.stride(3) != 1 or 0 in d_out.stride() or d_out.data_ptr() % 16 or any(st % 8 for st in d_out.stride()[:3]):
             d_out = d_out.contiguous()
-        dq, dk, dv = ops.attn_bwd(q, k, v, out, lse, d_out.to(torch.bfloat16), ctx.plan, ctx.scale)
+        dq, dk, dv = ops.attn_bwd_rows(q, k, v, out, lse, d_out, plan, ctx.scale)
         return dq, dk, dv, None, None
 
 
@@ -63,20 +52,14 @@ def packed_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plans: L
     a [B, H, S, D] tensor goes in as ``t.transpose(1, 2)``).  Returns [B, S, Hq, D] bf16.
     Differentiable w.r.t. q, k, v."""
     if q.dim() == 3:
-        return _row(q, k, v, plans[0], scale)
-    outs = [_row(q[b], k[b], v[b], plans[b], scale) for b in range(q.shape[0])]
-    return torch.stack(outs, 0)
-
-
-def _row(q, k, v, plan, scale):
-    S = q.shape[0]
-    extra = plan.S - S
-    if extra == 0:
-        return _PackedAttentionFn.apply(q, k, v, plan, scale)
-    if not 0 < extra < ROW_MULTIPLE:
-        raise ValueError(f"plan made for a row of {plan.S} positions, tensors have {S}")
-    if scale is None:
-        scale = float(q.shape[-1]) ** -0.5
-    pad = (0, 0, 0, 0, 0, extra)  # zero rows at the end of the sequence dimension
-    out = _PackedAttentionFn.apply(F.pad(q, pad), F.pad(k, pad), F.pad(v, pad), plan, scale)
-    return out[:S]
+        return packed_attention(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), plans[:1], scale)[0]
+    B, S = q.shape[:2]
+    for plan in plans[:B]:
+        if not 0 <= plan.S - S < ROW_MULTIPLE:
+            raise ValueError(f"plan made for a row of {plan.S} positions, tensors have {S}")
+    first = plans[0]
+    if first.rows == B and all(p.batch is first.batch and p.index == b for b, p in enumerate(plans[:B])):
+        return _PackedAttentionFn.apply(q, k, v, first.batch, scale)
+    # plans that were made one by one: a call per row
+    outs = [_PackedAttentionFn.apply(q[b:b + 1], k[b:b + 1], v[b:b + 1], plans[b].buf, scale) for b in range(B)]
+    return torch.cat(outs, 0)

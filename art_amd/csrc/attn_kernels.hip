@@ -44,34 +44,99 @@ constexpr int ATT_BK2 = 64;    // dK/dV kernel: keys per work-group (2 key group
 // Plan
 // ----------------------------------------------------------------------------
 
+// Every kernel of the plan takes a batch of rows: blockIdx.y (attn_heads_kernel: blockIdx.x) is the row, whose
+// plan lies `stride` bytes behind the one before.  Positions S .. Sp - 1 fill up the last block: they get codes
+// nothing else carries, so they see, and are seen by, themselves only.
+template <class T>
+__device__ __forceinline__ T* attn_row(T* p, int64_t stride, int row) {
+  return (T*)((char*)p + stride * row);
+}
+
+// heads = the positions whose group id differs from the one before, ascending: the first position of a group
+// is always one of them, so the equality codes need S x (runs) comparisons instead of S^2 (a packed row has a
+// run per prompt and completion).  One work-group per row, each thread a contiguous piece.
+__global__ __launch_bounds__(1024) void attn_heads_kernel(const int64_t* __restrict__ group_ids, int S,
+                                                          int64_t stride, int* __restrict__ heads,
+                                                          int* __restrict__ n_heads) {
+  __shared__ int wtot[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t* g = group_ids + (int64_t)blockIdx.x * S;
+  heads = attn_row(heads, stride, blockIdx.x);
+  const int per = (S + 1023) / 1024;
+  const int t0 = (int)threadIdx.x * per, t1 = t0 + per < S ? t0 + per : S;
+  int n = 0;
+  int64_t prev = t0 > 0 && t0 < S ? g[t0 - 1] : 0;
+  for (int t = t0; t < t1; ++t) {
+    const int64_t id = g[t];
+    n += t == 0 || id != prev;
+    prev = id;
+  }
+  int run = n;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int v = __shfl_up(run, d, 64);
+    if (lane >= d) run += v;
+  }
+  if (lane == 63) wtot[wave] = run;
+  __syncthreads();
+  int off = run - n;
+  for (int w = 0; w < wave; ++w) off += wtot[w];
+  prev = t0 > 0 && t0 < S ? g[t0 - 1] : 0;
+  for (int t = t0; t < t1; ++t) {
+    const int64_t id = g[t];
+    if (t == 0 || id != prev) heads[off++] = t;
+    prev = id;
+  }
+  if (threadIdx.x == 1023) *attn_row(n_heads, stride, blockIdx.x) = off;
+}
+
 // gc[t] = first position whose group id equals group_ids[t];
 // pc[t] = first position whose group id equals parent_ids[t], or -2 if none.
 // Then group[i] == group[j] <=> gc[i] == gc[j] and parent[i] == group[j] <=>
-// pc[i] == gc[j].  Brute force over all pairs (integer work, once per row).
+// pc[i] == gc[j].  uni[c] = {gc, pc} of positions 32 c .. 32 c + 31 where they all agree,
+// else ATT_MIXED in that component.
+constexpr int ATT_MIXED = (int)0x80000000;
 __global__ __launch_bounds__(256) void attn_codes_kernel(const int64_t* __restrict__ group_ids,
                                                          const int64_t* __restrict__ parent_ids,
-                                                         int S, int* __restrict__ gc,
-                                                         int* __restrict__ pc) {
-  __shared__ int64_t tile[256];
+                                                         int S, int64_t stride, const int* __restrict__ heads,
+                                                         const int* __restrict__ n_heads, int* __restrict__ gc,
+                                                         int* __restrict__ pc, int2* __restrict__ uni) {
+  __shared__ int64_t hid[256];
+  __shared__ int hpos[256];
+  const int row = blockIdx.y;
+  group_ids += (int64_t)row * S;
+  parent_ids += (int64_t)row * S;
+  heads = attn_row(heads, stride, row);
+  const int nh = *attn_row(n_heads, stride, row);
   const int t = blockIdx.x * 256 + threadIdx.x;
-  const int64_t g = t < S ? group_ids[t] : 0;
-  const int64_t pa = t < S ? parent_ids[t] : 0;
-  int first_g = 0x7fffffff, first_p = 0x7fffffff;
-  for (int j0 = 0; j0 < S; j0 += 256) {
+  const bool in = t < S;
+  const int64_t g = in ? group_ids[t] : 0;
+  const int64_t pa = in ? parent_ids[t] : 0;
+  int first_g = -1, first_p = -2;
+  for (int h0 = 0; h0 < nh; h0 += 256) {
+    const int lim = nh - h0 < 256 ? nh - h0 : 256;
     __syncthreads();
-    tile[threadIdx.x] = j0 + (int)threadIdx.x < S ? group_ids[j0 + threadIdx.x] : 0;
+    if ((int)threadIdx.x < lim) {
+      const int pos = heads[h0 + threadIdx.x];
+      hpos[threadIdx.x] = pos;
+      hid[threadIdx.x] = group_ids[pos];
+    }
     __syncthreads();
-    const int lim = S - j0 < 256 ? S - j0 : 256;
-    for (int jj = 0; jj < lim; ++jj) {
-      const int64_t id = tile[jj];
-      if (id == g && j0 + jj < first_g) first_g = j0 + jj;
-      if (id == pa && j0 + jj < first_p) first_p = j0 + jj;
+    for (int j = lim - 1; j >= 0; --j) {   // descending, so the first match wins within this piece
+      const int64_t id = hid[j];
+      const int pos = hpos[j];
+      if (id == g && (first_g < 0 || first_g >= hpos[0])) first_g = pos;
+      if (id == pa && (first_p < 0 || first_p >= hpos[0])) first_p = pos;
     }
   }
-  if (t < S) {
-    gc[t] = first_g;
-    pc[t] = first_p == 0x7fffffff ? -2 : first_p;
-  }
+  const int gcv = in ? first_g : -3 - t, pcv = in ? first_p : -2;
+  attn_row(gc, stride, row)[t] = gcv;
+  attn_row(pc, stride, row)[t] = pcv;
+  const int lane = threadIdx.x & 63, base = lane & 32;
+  const unsigned long long mine = 0xffffffffull << base;
+  const bool ug = (__ballot(gcv == __shfl(gcv, base, 64)) & mine) == mine;
+  const bool up = (__ballot(pcv == __shfl(pcv, base, 64)) & mine) == mine;
+  if ((lane & 31) == 0) attn_row(uni, stride, row)[t / 32] = make_int2(ug ? gcv : ATT_MIXED, up ? pcv : ATT_MIXED);
 }
 
 __device__ __forceinline__ bool attn_visible(int i, int j, int gi, int pi, int gj) {
@@ -84,71 +149,82 @@ __device__ __forceinline__ bool attn_visible(int i, int j, int gi, int pi, int g
 //   bits 16-19  wave w has at least one visible pair in its part of the tile
 //   bits 24-27  every pair of wave w's part is visible (no per-element test needed)
 // 0 when nothing is visible.
-// MODE 0 (forward, dQ): owner = 128 queries, tile = 64 keys, wave w (of 4) = queries 32w..32w+31.
-// MODE 1 (dK/dV):      owner = 64 keys, tile = 64 queries, wave w (of 4) = keys 32(w&1).. x
-//                      queries 32(w>>1)..
-// One wavefront evaluates the rule on every pair of its (owner, tile).
-template <int MODE>
-__global__ __launch_bounds__(256) void attn_classify_kernel(const int* __restrict__ gc,
-                                                            const int* __restrict__ pc, int n_tile,
-                                                            uint32_t* __restrict__ info) {
+//   info  (forward, dQ): owner = 128 queries, tile = 64 keys, wave w (of 4) = queries 32w..32w+31.
+//   info2 (dK/dV):       owner = 64 keys, tile = 64 queries, wave w (of 4) = keys 32(w&1).. x
+//                        queries 32(w>>1)..
+// One wavefront takes 128 queries x 64 keys = 8 cells of 32 x 32 and writes the entry of info and both
+// entries of info2.  A cell whose queries share their codes and whose keys share theirs is decided from
+// uni; only the others are evaluated pair by pair (64 lanes = 32 keys x 2 halves of the queries).
+__device__ __forceinline__ uint32_t attn_entry(uint32_t any, uint32_t all) {
+  return any ? ((all == 0xfu ? 2u : 1u) << 14) | (any << 16) | (all << 24) : 0u;
+}
+__global__ __launch_bounds__(256) void attn_classify_kernel(const int* __restrict__ gc, const int* __restrict__ pc,
+                                                            const int2* __restrict__ uni, int64_t stride, int nKb,
+                                                            int nQb2, uint32_t* __restrict__ info,
+                                                            uint32_t* __restrict__ info2) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int tile = blockIdx.x * 4 + wave;
-  const int owner = blockIdx.y;
-  if (tile >= n_tile) return;
-  uint32_t any = 0, all = 0;
-  if (MODE == 0) {
-    const int q0 = owner * ATT_BM, j = tile * ATT_BN + lane;
-    if (tile * ATT_BN <= q0 + ATT_BM - 1) {
+  const int row = blockIdx.z, owner = blockIdx.y, kb = blockIdx.x * 4 + wave;
+  if (kb >= nKb) return;
+  gc = attn_row(gc, stride, row);
+  pc = attn_row(pc, stride, row);
+  uni = attn_row(uni, stride, row);
+  info = attn_row(info, stride, row);
+  info2 = attn_row(info2, stride, row);
+  uint32_t any = 0, all = 0;   // bit 2 w + kg: cell of queries 32 w.., keys 32 kg..
+  if (kb * ATT_BN <= owner * ATT_BM + ATT_BM - 1) {
+    const int qc = owner * (ATT_BM / 32) + ((lane & 7) >> 1), kc = kb * 2 + (lane & 1);  // lanes 0..7: one cell each
+    const int2 uq = uni[qc];
+    const int gk = uni[kc].x;
+    const bool live = kc <= qc;
+    const bool known = !live || (uq.x != ATT_MIXED && uq.y != ATT_MIXED && gk != ATT_MIXED);
+    const bool eq = live && known && (gk == uq.x || gk == uq.y);
+    any = (uint32_t)__ballot(eq) & 0xffu;
+    all = (uint32_t)__ballot(eq && kc < qc) & 0xffu;
+    for (uint32_t left = (uint32_t)__ballot(!known) & 0xffu; left; left &= left - 1) {
+      const int cell = __builtin_ctz(left);
+      const int q0 = (owner * (ATT_BM / 32) + (cell >> 1)) * 32 + 16 * (lane >> 5);
+      const int j = (kb * 2 + (cell & 1)) * 32 + (lane & 31);
       const int gj = gc[j];
-      for (int g = 0; g < ATT_BM / 32; ++g) {
-        int cnt = 0;
-        for (int ii = 0; ii < 32; ++ii) {
-          const int i = q0 + 32 * g + ii;
-          cnt += attn_visible(i, j, gc[i], pc[i], gj) ? 1 : 0;
-        }
-        any |= (uint32_t)(__ballot(cnt > 0) != 0ull) << g;
-        all |= (uint32_t)(__ballot(cnt == 32) == ~0ull) << g;
-      }
-    }
-  } else {
-    const int k0 = owner * ATT_BK2, q0 = tile * ATT_BQ2;
-    if (k0 <= q0 + ATT_BQ2 - 1) {
-      const int j = k0 + lane;
-      const int gj = gc[j];
-      for (int qh = 0; qh < 2; ++qh) {
-        int cnt = 0;
-        for (int ii = 0; ii < 32; ++ii) {
-          const int i = q0 + 32 * qh + ii;
-          cnt += attn_visible(i, j, gc[i], pc[i], gj) ? 1 : 0;
-        }
-        const unsigned long long ab = __ballot(cnt > 0), fb = __ballot(cnt == 32);
-        for (int kg = 0; kg < 2; ++kg) {
-          const int bit = kg + 2 * qh;
-          any |= (uint32_t)((uint32_t)(ab >> (32 * kg)) != 0u) << bit;
-          all |= (uint32_t)((uint32_t)(fb >> (32 * kg)) == 0xffffffffu) << bit;
-        }
-      }
+      int cnt = 0;
+#pragma unroll
+      for (int ii = 0; ii < 16; ++ii) cnt += attn_visible(q0 + ii, j, gc[q0 + ii], pc[q0 + ii], gj) ? 1 : 0;
+      any |= (uint32_t)(__ballot(cnt > 0) != 0ull) << cell;
+      all |= (uint32_t)(__ballot(cnt == 16) == ~0ull) << cell;
     }
   }
   if (lane == 0) {
-    const uint32_t cls = all == 0xfu ? 2u : 1u;
-    info[(int64_t)owner * n_tile + tile] = any ? (cls << 14) | (any << 16) | (all << 24) : 0u;
+    uint32_t a4 = 0, l4 = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      a4 |= (uint32_t)((any >> (2 * w) & 3u) != 0u) << w;
+      l4 |= (uint32_t)((all >> (2 * w) & 3u) == 3u) << w;
+    }
+    info[(int64_t)owner * nKb + kb] = attn_entry(a4, l4);
+    info2[(int64_t)kb * nQb2 + 2 * owner] = attn_entry(any & 0xfu, all & 0xfu);
+    info2[(int64_t)kb * nQb2 + 2 * owner + 1] = attn_entry(any >> 4, all >> 4);
   }
 }
 
 // list[row][0..cnt[row]) = tile index | info for the tiles of info[row][*] that
-// are not 0, ascending.  One work-group per row.
-__global__ __launch_bounds__(256) void attn_compact_kernel(const uint32_t* __restrict__ info, int ncol,
-                                                           uint32_t* __restrict__ list,
-                                                           int* __restrict__ cnt) {
+// are not 0, ascending.  One work-group per row of either table (the key blocks after the query blocks).
+struct AttnTable {
+  const uint32_t* info;
+  uint32_t* list;
+  int* cnt;
+  int nrow, ncol;
+};
+__global__ __launch_bounds__(256) void attn_compact_kernel(AttnTable a, AttnTable b, int64_t stride) {
   __shared__ int wtot[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = blockIdx.x;
+  const bool second = (int)blockIdx.x >= a.nrow;
+  const int row = second ? (int)blockIdx.x - a.nrow : (int)blockIdx.x;
+  const int ncol = second ? b.ncol : a.ncol;
+  const uint32_t* info = attn_row(second ? b.info : a.info, stride, blockIdx.y) + (int64_t)row * ncol;
+  uint32_t* list = attn_row(second ? b.list : a.list, stride, blockIdx.y) + (int64_t)row * ncol;
   int base = 0;
   for (int c0 = 0; c0 < ncol; c0 += 256) {
     const int c = c0 + threadIdx.x;
-    const uint32_t v = c < ncol ? info[(int64_t)row * ncol + c] : 0u;
+    const uint32_t v = c < ncol ? info[c] : 0u;
     const unsigned long long m = __ballot(v != 0);
     const int rank = __popcll(m & ((1ull << lane) - 1ull));
     __syncthreads();
@@ -156,33 +232,36 @@ __global__ __launch_bounds__(256) void attn_compact_kernel(const uint32_t* __res
     __syncthreads();
     int off = base;
     for (int w = 0; w < wave; ++w) off += wtot[w];
-    if (v) list[(int64_t)row * ncol + off + rank] = (uint32_t)c | v;
+    if (v) list[off + rank] = (uint32_t)c | v;
     base += wtot[0] + wtot[1] + wtot[2] + wtot[3];
   }
-  if (threadIdx.x == 0) cnt[row] = base;
+  if (threadIdx.x == 0) attn_row(second ? b.cnt : a.cnt, stride, blockIdx.y)[row] = base;
 }
 
 // order[r] = the block with the r-th largest count (ties: the later block first): work-groups are dispatched
-// in this order, so the long ones do not end up alone at the end of a launch.  Work-group 0 sorts the query
-// blocks, 1 the key blocks (and adds up their counts); at most 1024 counts each, by rank.
+// in this order, so the long ones do not end up alone at the end of a launch.  Work-group x = 0 sorts the
+// query blocks, 1 the key blocks (and adds up their counts); at most 1024 counts each, by rank.
 __global__ __launch_bounds__(1024) void attn_order_kernel(const int* __restrict__ cnt, int n, int* __restrict__ order,
                                                           const int* __restrict__ cnt2, int n2,
-                                                          int* __restrict__ order2, int* __restrict__ total2) {
+                                                          int* __restrict__ order2, int* __restrict__ total2,
+                                                          int64_t stride) {
   __shared__ int c[ATT_MAX_KB];
   const bool second = blockIdx.x == 1;
   const int m = second ? n2 : n;
   const int t = threadIdx.x;
-  if (t < m) c[t] = (second ? cnt2 : cnt)[t];
+  if (t < m) c[t] = attn_row(second ? cnt2 : cnt, stride, blockIdx.y)[t];
   __syncthreads();
   if (t >= m) return;
   int rank = 0, sum = 0;
-  for (int i = 0; i < m; ++i) sum += c[i];
-  if (second && t == 0) *total2 = sum;
-  for (int i = 0; i < m; ++i) rank += (c[i] > c[t] || (c[i] == c[t] && i > t)) ? 1 : 0;
-  (second ? order2 : order)[rank] = t;
+  for (int i = 0; i < m; ++i) {
+    sum += c[i];
+    rank += (c[i] > c[t] || (c[i] == c[t] && i > t)) ? 1 : 0;
+  }
+  if (second && t == 0) *attn_row(total2, stride, blockIdx.y) = sum;
+  attn_row(second ? order2 : order, stride, blockIdx.y)[rank] = t;
 }
 
-// Device-memory layout of a plan for a row of S positions (S % 256 == 0).
+// Device-memory layout of the plan of one row of S positions (a multiple of 256).
 struct AttnPlan {
   int* gc;
   int* pc;
@@ -197,6 +276,10 @@ struct AttnPlan {
   int* cnt2;           // [nKb2]
   int* order2;         // [nKb2]
   int* total2;         // sum of cnt2
+  int2* uni;           // [S / 32]
+  int* heads;          // [S]
+  int* n_heads;
+  int64_t stride;      // bytes from one row's plan to the next
 };
 
 static size_t attn_plan_layout(void* base, size_t bytes, int64_t S, AttnPlan& pl) {
@@ -216,6 +299,10 @@ static size_t attn_plan_layout(void* base, size_t bytes, int64_t S, AttnPlan& pl
   pl.cnt2 = ws.take<int>((size_t)pl.nKb2);
   pl.order2 = ws.take<int>((size_t)pl.nKb2);
   pl.total2 = ws.take<int>(1);
+  pl.uni = ws.take<int2>((size_t)S / 32);
+  pl.heads = ws.take<int>((size_t)S);
+  pl.n_heads = ws.take<int>(1);
+  pl.stride = (int64_t)align_up(ws.used, 256);
   return ws.ok() || base == nullptr ? ws.used : (size_t)-1;
 }
 
@@ -314,6 +401,12 @@ __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// Descriptor of one head's rows 0 .. S-1 (`stride` elements apart): rows past the end, which fill up the last
+// tile of a row whose length is no multiple of the tile's, arrive in LDS as zeros.
+template <int D>
+__device__ __forceinline__ dma_rsrc_t attn_head_rsrc(const uint16_t* head, int64_t stride, int S) {
+  return dma_make_rsrc(head, (uint32_t)(((int64_t)(S - 1) * stride + D) * 2));
+}
 __device__ __forceinline__ dma_rsrc_t attn_rsrc(const void* p) { return dma_make_rsrc(p, 0x7fffffffu); }
 
 // ----------------------------------------------------------------------------
@@ -350,6 +443,7 @@ struct AttnFwdParams {
   const uint32_t* list;
   const int* cnt;
   const int* order;
+  int64_t plan_stride, q_bs, k_bs, v_bs, o_bs;   // per row of the batch (blockIdx.y)
   int S, Hq, Hkv, nQb, nKb;
   float scale_log2e;
 };
@@ -394,37 +488,40 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_fwd_kernel(
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5;
   const TrLane tr(lane);
+  const int row = blockIdx.y;
   int hq, qb;
-  if (!attn_block(p.Hq, p.Hkv, p.nQb, p.order, hq, qb)) return;
+  if (!attn_block(p.Hq, p.Hkv, p.nQb, attn_row(p.order, p.plan_stride, row), hq, qb)) return;
   const int hkv = hq / (p.Hq / p.Hkv);
   const int q = qb * ATT_BM + wave * 32 + n;
-  const int cnt = p.cnt[qb];
+  const int qc = q < p.S ? q : p.S - 1;  // queries past the end compute something that is not stored
+  const int* const gc = attn_row(p.gc, p.plan_stride, row);
+  const uint32_t* const list = attn_row(p.list, p.plan_stride, row) + (int64_t)qb * p.nKb;
+  const int cnt = attn_row(p.cnt, p.plan_stride, row)[qb];
 
-  for (int i = threadIdx.x; i < cnt; i += ATT_THREADS) s_list[i] = p.list[(int64_t)qb * p.nKb + i];
-
-  // this lane's query as B-operand fragments of S^T = K Q^T
-  bf16x8 qf[D / 16];
-  {
-    const uint16_t* qp = p.Q + (int64_t)q * p.q_ss + (int64_t)hq * p.q_hs + 8 * h;
-#pragma unroll
-    for (int s = 0; s < D / 16; ++s) qf[s] = *(const bf16x8*)(qp + 16 * s);
-  }
-  int gi = p.gc[q], pi = p.pc[q];
-
-  const dma_rsrc_t rsrc_k = attn_rsrc(p.K + (int64_t)hkv * p.k_hs);
-  const dma_rsrc_t rsrc_v = attn_rsrc(p.V + (int64_t)hkv * p.v_hs);
-  const dma_rsrc_t rsrc_c = attn_rsrc(p.gc);
+  const dma_rsrc_t rsrc_k = attn_head_rsrc<D>(p.K + row * p.k_bs + (int64_t)hkv * p.k_hs, p.k_ss, p.S);
+  const dma_rsrc_t rsrc_v = attn_head_rsrc<D>(p.V + row * p.v_bs + (int64_t)hkv * p.v_hs, p.v_ss, p.S);
+  const dma_rsrc_t rsrc_c = attn_rsrc(gc);
   int voff_k[T::N4], voff_v[T::N4];
 #pragma unroll
   for (int i = 0; i < T::N4; ++i) {
     voff_k[i] = T::voff(wave * T::N4 + i, lane, p.k_ss);
     voff_v[i] = T::voff(wave * T::N4 + i, lane, p.v_ss);
   }
-  __syncthreads();  // s_list
-  auto* list_lds = s_list;
-#define ATTN_ISSUE(IT, STG)                                                                          \
-  attn_issue_kv<D>(smem + (STG) * G::STAGE, __builtin_amdgcn_readfirstlane(list_lds[IT] & 0x3fff),    \
-                   rsrc_k, rsrc_v, rsrc_c, voff_k, voff_v, p.k_ss, p.v_ss, wave, lane)
+#define ATTN_ISSUE(ENTRY, STG)                                                                        \
+  attn_issue_kv<D>(smem + (STG) * G::STAGE, __builtin_amdgcn_readfirstlane((ENTRY) & 0x3fff), rsrc_k,  \
+                   rsrc_v, rsrc_c, voff_k, voff_v, p.k_ss, p.v_ss, wave, lane)
+  // the first tile is on its way before anything else is read
+  if (cnt > 0) ATTN_ISSUE(list[0], 0);
+  for (int i = threadIdx.x; i < cnt; i += ATT_THREADS) s_list[i] = list[i];
+
+  // this lane's query as B-operand fragments of S^T = K Q^T
+  bf16x8 qf[D / 16];
+  {
+    const uint16_t* qp = p.Q + row * p.q_bs + (int64_t)qc * p.q_ss + (int64_t)hq * p.q_hs + 8 * h;
+#pragma unroll
+    for (int s = 0; s < D / 16; ++s) qf[s] = *(const bf16x8*)(qp + 16 * s);
+  }
+  int gi = gc[q], pi = attn_row(p.pc, p.plan_stride, row)[q];
 
   floatx16 o[D / 32];
 #pragma unroll
@@ -437,11 +534,10 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_fwd_kernel(
   for (int s = 0; s < D / 16; ++s) pin_loaded(qf[s]);
   pin_loaded(gi);
   pin_loaded(pi);
-  if (cnt > 0) ATTN_ISSUE(0, 0);
   for (int it = 0; it < cnt; ++it) {
     wait_vmcnt<0>();
     barrier_lds_only();
-    if (it + 1 < cnt) ATTN_ISSUE(it + 1, (it + 1) & 1);
+    if (it + 1 < cnt) ATTN_ISSUE(s_list[it + 1], (it + 1) & 1);
     const int entry = __builtin_amdgcn_readfirstlane(s_list[it]);
     const int kb = entry & 0x3fff;
     const bool active = (entry >> (16 + wave)) & 1;        // this wave's 32 queries see part of the tile
@@ -544,14 +640,15 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_fwd_kernel(
 
   const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  uint16_t* op = p.O + (int64_t)q * p.o_ss + (int64_t)hq * p.o_hs;
+  if (q >= p.S) return;  // (both lanes of a query)
+  uint16_t* op = p.O + row * p.o_bs + (int64_t)q * p.o_ss + (int64_t)hq * p.o_hs;
 #pragma unroll
   for (int dt = 0; dt < D / 32; ++dt) {
 #pragma unroll
     for (int j = 0; j < 16; ++j) o[dt][j] *= inv;
     store_block_bf16(op + 32 * dt, o[dt], h);
   }
-  if (h == 0) p.lse[(int64_t)hq * p.S + q] = (m_run + __builtin_amdgcn_logf(l_tot)) * LN2;
+  if (h == 0) p.lse[((int64_t)row * p.Hq + hq) * p.S + q] = (m_run + __builtin_amdgcn_logf(l_tot)) * LN2;
 }
 
 // ----------------------------------------------------------------------------
@@ -578,9 +675,9 @@ struct AttnKvSplit {
   int heads_all;     // query heads
   int div;           // steps of a share = total * heads_all / div
   int light_max;     // >= 0 (artk_attn_bwd_tuning): all heads where they make at most this many steps, else one
-  __device__ __forceinline__ int heads(int cnt, int rep) const {
+  __device__ __forceinline__ int heads(int cnt, int rep, int64_t stride, int row) const {
     if (light_max >= 0) return cnt * rep <= light_max ? rep : 1;
-    const int steps = (int)((int64_t)*total * heads_all / div);
+    const int steps = (int)((int64_t)*attn_row(total, stride, row) * heads_all / div);
     int g = cnt > 0 ? steps / cnt : rep;
     g = g < 1 ? 1 : (g > rep ? rep : g);
     const int groups = (rep + g - 1) / g;
@@ -590,10 +687,14 @@ struct AttnKvSplit {
 
 struct AttnBwdParams {
   const uint16_t *Q, *K, *V, *dO;
-  const float* lse2;                // [Hq][S]  lse * log2(e)
-  const float* delta;               // [Hq][S]
+  const uint16_t* O;
+  const float* lse;                 // [Hq][S]
+  float* lse2;                      // [Hq][Sp]  lse * log2(e), Sp = S rounded up to a multiple of 256
+  float* delta;                     // [Hq][Sp]
   uint16_t *dQ, *dK, *dV;
-  float *pK, *pV;                   // [Hq/Hkv][S][Hkv][D] per-head partial sums (grouped-query heads only)
+  float *pK, *pV;                   // [Hq/Hkv][Sp][Hkv][D] partial sums per share (grouped-query heads only)
+  int64_t plan_stride, q_bs, k_bs, v_bs, o_bs, do_bs, dq_bs, dk_bs, dv_bs;  // per row of the batch (blockIdx.y)
+  int64_t o_ss, o_hs;
   int64_t q_ss, q_hs, k_ss, k_hs, v_ss, v_hs, do_ss, do_hs, dq_ss, dq_hs, dk_ss, dk_hs, dv_ss, dv_hs;
   const int* gc;
   const int* pc;
@@ -603,41 +704,14 @@ struct AttnBwdParams {
   const uint32_t* listT;   // per key block of 64: query tiles of 64
   const int* cntT;
   const int* orderT;
-  int S, Hq, Hkv, nQb, nKb, nQb2, nKb2;
+  int S, Sp, Hq, Hkv, nQb, nKb, nQb2, nKb2;
   AttnKvSplit split;
   float scale, scale_log2e;
 };
 
-// delta[h][s] = sum_d dO[s,h,d] * O[s,h,d] and lse2 = lse * log2(e); 16 lanes per (s, h).
-__global__ __launch_bounds__(256) void attn_delta_kernel(const uint16_t* __restrict__ O, int64_t o_ss,
-                                                         int64_t o_hs,
-                                                         const uint16_t* __restrict__ dO,
-                                                         int64_t do_ss, int64_t do_hs,
-                                                         const float* __restrict__ lse, int S, int H,
-                                                         int D, float* __restrict__ delta,
-                                                         float* __restrict__ lse2) {
-  const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-  const int sub = threadIdx.x & 15;
-  if (row >= (int64_t)S * H) return;
-  const int s = (int)(row / H), hh = (int)(row - (int64_t)s * H);
-  const uint16_t* op = O + (int64_t)s * o_ss + (int64_t)hh * o_hs;
-  const uint16_t* gp = dO + (int64_t)s * do_ss + (int64_t)hh * do_hs;
-  float acc = 0.f;
-  for (int d = sub * 8; d < D; d += 128) {
-    const bf16x8 a = *(const bf16x8*)(op + d);
-    const bf16x8 b = *(const bf16x8*)(gp + d);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc += (float)a[e] * (float)b[e];
-  }
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-  if (sub == 0) {
-    delta[(int64_t)hh * S + s] = acc;
-    lse2[(int64_t)hh * S + s] = lse[(int64_t)hh * S + s] * LOG2E;
-  }
-}
-
-// ---- dQ: 256 queries x one head per work-group, lane = query ----------------
+// ---- dQ: 128 queries x one head per work-group, lane = query ----------------
+// Runs first and leaves delta and lse2 of its queries for the dK/dV kernel: it holds their dO anyway, so a
+// pass of its own over O and dO (47 us for 16384 positions, 28 heads of 128) became a read of O.
 template <int D>
 __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kernel(AttnBwdParams p) {
   using T = AttnTile<D>;
@@ -648,41 +722,56 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kern
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5;
   const TrLane tr(lane);
+  const int row = blockIdx.y;
   int hq, qb;
-  if (!attn_block(p.Hq, p.Hkv, p.nQb, p.order, hq, qb)) return;
+  if (!attn_block(p.Hq, p.Hkv, p.nQb, attn_row(p.order, p.plan_stride, row), hq, qb)) return;
   const int hkv = hq / (p.Hq / p.Hkv);
   const int q = qb * ATT_BM + wave * 32 + n;
-  const int cnt = p.cnt[qb];
-  for (int i = threadIdx.x; i < cnt; i += ATT_THREADS) s_list[i] = p.list[(int64_t)qb * p.nKb + i];
+  const int qc = q < p.S ? q : p.S - 1;  // queries past the end compute something that is not stored
+  const int* const gc = attn_row(p.gc, p.plan_stride, row);
+  const uint32_t* const list = attn_row(p.list, p.plan_stride, row) + (int64_t)qb * p.nKb;
+  const int cnt = attn_row(p.cnt, p.plan_stride, row)[qb];
 
-  bf16x8 qf[D / 16], dof[D / 16];
-  {
-    const uint16_t* qp = p.Q + (int64_t)q * p.q_ss + (int64_t)hq * p.q_hs + 8 * h;
-    const uint16_t* gp = p.dO + (int64_t)q * p.do_ss + (int64_t)hq * p.do_hs + 8 * h;
-#pragma unroll
-    for (int s = 0; s < D / 16; ++s) {
-      qf[s] = *(const bf16x8*)(qp + 16 * s);
-      dof[s] = *(const bf16x8*)(gp + 16 * s);
-    }
-  }
-  int gi = p.gc[q], pi = p.pc[q];
-  float nlse2 = -p.lse2[(int64_t)hq * p.S + q];
-  float delta = p.delta[(int64_t)hq * p.S + q];
-
-  const dma_rsrc_t rsrc_k = attn_rsrc(p.K + (int64_t)hkv * p.k_hs);
-  const dma_rsrc_t rsrc_v = attn_rsrc(p.V + (int64_t)hkv * p.v_hs);
-  const dma_rsrc_t rsrc_c = attn_rsrc(p.gc);
+  const dma_rsrc_t rsrc_k = attn_head_rsrc<D>(p.K + row * p.k_bs + (int64_t)hkv * p.k_hs, p.k_ss, p.S);
+  const dma_rsrc_t rsrc_v = attn_head_rsrc<D>(p.V + row * p.v_bs + (int64_t)hkv * p.v_hs, p.v_ss, p.S);
+  const dma_rsrc_t rsrc_c = attn_rsrc(gc);
   int voff_k[T::N4], voff_v[T::N4];
 #pragma unroll
   for (int i = 0; i < T::N4; ++i) {
     voff_k[i] = T::voff(wave * T::N4 + i, lane, p.k_ss);
     voff_v[i] = T::voff(wave * T::N4 + i, lane, p.v_ss);
   }
-  __syncthreads();
-  auto* list_lds = s_list;
-#define ATTN_ISSUE(IT, STG)                                                                          \
-  attn_issue_kv<D>(smem + (STG) * G::STAGE, __builtin_amdgcn_readfirstlane(list_lds[IT] & 0x3fff),    \
-                   rsrc_k, rsrc_v, rsrc_c, voff_k, voff_v, p.k_ss, p.v_ss, wave, lane)
+#define ATTN_ISSUE(ENTRY, STG)                                                                        \
+  attn_issue_kv<D>(smem + (STG) * G::STAGE, __builtin_amdgcn_readfirstlane((ENTRY) & 0x3fff), rsrc_k,  \
+                   rsrc_v, rsrc_c, voff_k, voff_v, p.k_ss, p.v_ss, wave, lane)
+  if (cnt > 0) ATTN_ISSUE(list[0], 0);
+  for (int i = threadIdx.x; i < cnt; i += ATT_THREADS) s_list[i] = list[i];
+
+  bf16x8 qf[D / 16], dof[D / 16];
+  float delta = 0.f;
+  {
+    const uint16_t* qp = p.Q + row * p.q_bs + (int64_t)qc * p.q_ss + (int64_t)hq * p.q_hs + 8 * h;
+    const uint16_t* gp = p.dO + row * p.do_bs + (int64_t)qc * p.do_ss + (int64_t)hq * p.do_hs + 8 * h;
+    const uint16_t* op = p.O + row * p.o_bs + (int64_t)qc * p.o_ss + (int64_t)hq * p.o_hs + 8 * h;
+#pragma unroll
+    for (int s = 0; s < D / 16; ++s) dof[s] = *(const bf16x8*)(gp + 16 * s);
+#pragma unroll
+    for (int s = 0; s < D / 16; ++s) {
+      const bf16x8 of = *(const bf16x8*)(op + 16 * s);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) delta += (float)of[e] * (float)dof[s][e];
+    }
+#pragma unroll
+    for (int s = 0; s < D / 16; ++s) qf[s] = *(const bf16x8*)(qp + 16 * s);
+  }
+  delta += __shfl_xor(delta, 32, 64);
+  int gi = gc[q], pi = attn_row(p.pc, p.plan_stride, row)[q];
+  float nlse2 = -LOG2E * p.lse[((int64_t)row * p.Hq + hq) * p.S + qc];
+  if (h == 0) {
+    const int64_t o = ((int64_t)row * p.Hq + hq) * p.Sp + q;
+    p.lse2[o] = -nlse2;
+    p.delta[o] = q < p.S ? delta : 0.f;
+  }
 
   floatx16 dq[D / 32];
 #pragma unroll
@@ -699,11 +788,10 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kern
   pin_loaded(pi);
   pin_loaded(nlse2);
   pin_loaded(delta);
-  if (cnt > 0) ATTN_ISSUE(0, 0);
   for (int it = 0; it < cnt; ++it) {
     wait_vmcnt<0>();
     barrier_lds_only();
-    if (it + 1 < cnt) ATTN_ISSUE(it + 1, (it + 1) & 1);
+    if (it + 1 < cnt) ATTN_ISSUE(s_list[it + 1], (it + 1) & 1);
     const int entry = __builtin_amdgcn_readfirstlane(s_list[it]);
     const int kb = entry & 0x3fff;
     const bool active = (entry >> (16 + wave)) & 1;        // this wave's 32 queries see part of the tile
@@ -752,7 +840,8 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kern
     }
   }
 #undef ATTN_ISSUE
-  uint16_t* op = p.dQ + (int64_t)q * p.dq_ss + (int64_t)hq * p.dq_hs;
+  if (q >= p.S) return;
+  uint16_t* op = p.dQ + row * p.dq_bs + (int64_t)q * p.dq_ss + (int64_t)hq * p.dq_hs;
 #pragma unroll
   for (int dt = 0; dt < D / 32; ++dt) {
 #pragma unroll
@@ -785,22 +874,23 @@ struct AttnQStage {
 // DMA of one query tile into a stage: this wave's share of the Q and dO tiles and
 // one of the four per-query arrays (wave 0: lse2, 1: delta, 2: group codes, 3: parent codes).
 template <int D>
-__device__ __forceinline__ void attn_issue_q(char* st, int hq, int q0, dma_rsrc_t rsrc_q,
-                                             dma_rsrc_t rsrc_do,
+__device__ __forceinline__ void attn_issue_q(char* st, int hq, int q0, const uint16_t* q_row, const uint16_t* do_row,
                                              dma_rsrc_t rsrc_row, const int* voff_q,
                                              const int* voff_do, const AttnBwdParams& p, int wave,
                                              int lane) {
   using T = AttnTile<D>;
   using G = AttnQStage<D>;
-  const int so_q = (int)((q0 * p.q_ss + hq * p.q_hs) * 2);
-  const int so_do = (int)((q0 * p.do_ss + hq * p.do_hs) * 2);
+  const dma_rsrc_t rsrc_q = attn_head_rsrc<D>(q_row + hq * p.q_hs, p.q_ss, p.S);
+  const dma_rsrc_t rsrc_do = attn_head_rsrc<D>(do_row + hq * p.do_hs, p.do_ss, p.S);
+  const int so_q = (int)(q0 * p.q_ss * 2);
+  const int so_do = (int)(q0 * p.do_ss * 2);
 #pragma unroll
   for (int i = 0; i < T::N4; ++i) {
     dma_load16(rsrc_q, voff_q[i], so_q, lds_addr_of(st + (wave * T::N4 + i) * 1024));
     dma_load16(rsrc_do, voff_do[i], so_do, lds_addr_of(st + G::DO_OFF + (wave * T::N4 + i) * 1024));
   }
   const int arr = wave;
-  dma_load4(rsrc_row, lane * 4, (int)(((arr < 2 ? (int64_t)hq * p.S : 0) + q0) * 4), lds_addr_of(st + G::ROW_OFF + arr * 256));
+  dma_load4(rsrc_row, lane * 4, (int)(((arr < 2 ? (int64_t)hq * p.Sp : 0) + q0) * 4), lds_addr_of(st + G::ROW_OFF + arr * 256));
 }
 
 // The block's K and V rows (64 each).
@@ -828,24 +918,28 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
   const int n = lane & 31, h = lane >> 5;
   const int kg = wave & 1, qh = wave >> 1;
   const TrLane tr(lane);
+  const int brow = blockIdx.y;
   int hq, kb;
-  if (!attn_block(p.Hq, p.Hkv, p.nKb2, p.orderT, hq, kb)) return;
+  if (!attn_block(p.Hq, p.Hkv, p.nKb2, attn_row(p.orderT, p.plan_stride, brow), hq, kb)) return;
   const int rep = p.Hq / p.Hkv;
   const int hkv = hq / rep, share = hq - hkv * rep;
   const int key = kb * ATT_BK2 + kg * 32 + n;
-  const int cnt = p.cntT[kb];
-  const int per = p.split.heads(cnt, rep);
+  const int cnt = attn_row(p.cntT, p.plan_stride, brow)[kb];
+  const int per = p.split.heads(cnt, rep, p.plan_stride, brow);
   if (share * per >= rep) return;
   hq = hkv * rep + share * per;  // first head of this work-group's share
   const int nheads = rep - share * per < per ? rep - share * per : per;
-  for (int i = threadIdx.x; i < cnt; i += 256) s_list[i] = p.listT[(int64_t)kb * p.nQb2 + i];
-  int gk = p.gc[key];
+  const int* const gc = attn_row(p.gc, p.plan_stride, brow);
+  const uint32_t* const list = attn_row(p.listT, p.plan_stride, brow) + (int64_t)kb * p.nQb2;
+  for (int i = threadIdx.x; i < cnt; i += 256) s_list[i] = list[i];
+  int gk = gc[key];
 
-  const dma_rsrc_t rsrc_q = attn_rsrc(p.Q);
-  const dma_rsrc_t rsrc_do = attn_rsrc(p.dO);
+  const uint16_t* const q_row = p.Q + brow * p.q_bs;
+  const uint16_t* const do_row = p.dO + brow * p.do_bs;
   const int arr = wave;
-  const void* row_src = arr == 0 ? (const void*)p.lse2 : arr == 1 ? (const void*)p.delta
-                        : arr == 2 ? (const void*)p.gc : (const void*)p.pc;
+  const int64_t stat_row = (int64_t)brow * p.Hq * p.Sp;
+  const void* row_src = arr == 0 ? (const void*)(p.lse2 + stat_row) : arr == 1 ? (const void*)(p.delta + stat_row)
+                        : arr == 2 ? (const void*)gc : (const void*)attn_row(p.pc, p.plan_stride, brow);
   const dma_rsrc_t rsrc_row = attn_rsrc(row_src);
   int voff_q[T::N4], voff_do[T::N4];
   {
@@ -857,8 +951,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
       voff_k[i] = T::voff(wave * T::N4 + i, lane, p.k_ss);
       voff_v[i] = T::voff(wave * T::N4 + i, lane, p.v_ss);
     }
-    attn_issue_kv_block<D>(smem + G::KV_OFF, kb * ATT_BK2, attn_rsrc(p.K + (int64_t)hkv * p.k_hs),
-                           attn_rsrc(p.V + (int64_t)hkv * p.v_hs), voff_k, voff_v, p.k_ss, p.v_ss, wave);
+    attn_issue_kv_block<D>(smem + G::KV_OFF, kb * ATT_BK2, attn_head_rsrc<D>(p.K + brow * p.k_bs + (int64_t)hkv * p.k_hs, p.k_ss, p.S),
+                           attn_head_rsrc<D>(p.V + brow * p.v_bs + (int64_t)hkv * p.v_hs, p.v_ss, p.S), voff_k, voff_v, p.k_ss, p.v_ss, wave);
   }
   __syncthreads();  // s_list
   auto* list_lds = s_list;
@@ -867,7 +961,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
   do {                                                                                               \
     const int hi_ = (IT) / cnt, ti_ = (IT) - hi_ * cnt;                                               \
     attn_issue_q<D>(smem + (STG) * G::STAGE, hq + hi_,                                                \
-                    __builtin_amdgcn_readfirstlane(list_lds[ti_] & 0x3fff) * ATT_BQ2, rsrc_q, rsrc_do, \
+                    __builtin_amdgcn_readfirstlane(list_lds[ti_] & 0x3fff) * ATT_BQ2, q_row, do_row, \
                     rsrc_row, voff_q, voff_do, p, wave, lane);                                        \
   } while (0)
 
@@ -978,10 +1072,10 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
         }
     }
   }
-  if (qh == 1) return;
+  if (qh == 1 || key >= p.S) return;
 
   if (per < rep) {
-    const int64_t o = ((((int64_t)share * p.S + key) * p.Hkv + hkv) * D) + 4 * h;
+    const int64_t o = (((((int64_t)brow * rep + share) * p.Sp + key) * p.Hkv + hkv) * D) + 4 * h;
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
@@ -997,8 +1091,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
       }
     return;
   }
-  uint16_t* kp = p.dK + (int64_t)key * p.dk_ss + (int64_t)hkv * p.dk_hs + 4 * h;
-  uint16_t* vp = p.dV + (int64_t)key * p.dv_ss + (int64_t)hkv * p.dv_hs + 4 * h;
+  uint16_t* kp = p.dK + brow * p.dk_bs + (int64_t)key * p.dk_ss + (int64_t)hkv * p.dk_hs + 4 * h;
+  uint16_t* vp = p.dV + brow * p.dv_bs + (int64_t)key * p.dv_ss + (int64_t)hkv * p.dv_hs + 4 * h;
 #pragma unroll
   for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
@@ -1016,36 +1110,31 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
 
 // dK = scale * sum_r pK[r], dV = sum_r pV[r] over the shares r of a group's heads, in
 // index order; 4 elements per thread.
-__global__ __launch_bounds__(256) void attn_kv_reduce_kernel(const float* __restrict__ pK,
-                                                             const float* __restrict__ pV,
-                                                             const int* __restrict__ cntT,
-                                                             AttnKvSplit split, int rep,
-                                                             int64_t S, int Hkv, int D, float scale,
-                                                             uint16_t* __restrict__ dK, int64_t dk_ss,
-                                                             int64_t dk_hs, uint16_t* __restrict__ dV,
-                                                             int64_t dv_ss, int64_t dv_hs) {
+__global__ __launch_bounds__(256) void attn_kv_reduce_kernel(AttnBwdParams p, int D) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int d4 = D / 4;
-  const int64_t n = S * Hkv * d4;
-  if (i >= n) return;
+  const int d4 = D / 4, brow = blockIdx.y, rep = p.Hq / p.Hkv;
+  const int64_t n = (int64_t)p.Sp * p.Hkv * d4;
   const int c = (int)(i % d4);
-  const int hh = (int)((i / d4) % Hkv);
-  const int64_t s = i / ((int64_t)d4 * Hkv);
-  const int per = split.heads(cntT[s / ATT_BK2], rep);
+  const int hh = (int)((i / d4) % p.Hkv);
+  const int64_t s = i / ((int64_t)d4 * p.Hkv);
+  if (s >= p.S) return;
+  const int per = p.split.heads(attn_row(p.cntT, p.plan_stride, brow)[s / ATT_BK2], rep, p.plan_stride, brow);
   if (per == rep) return;  // written directly by the dK/dV kernel
+  const floatx4* pk = (const floatx4*)p.pK + (int64_t)brow * rep * n + i;
+  const floatx4* pv = (const floatx4*)p.pV + (int64_t)brow * rep * n + i;
   floatx4 a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
   for (int r = 0; r * per < rep; ++r) {
-    a += ((const floatx4*)pK)[(int64_t)r * n + i];
-    b += ((const floatx4*)pV)[(int64_t)r * n + i];
+    a += pk[(int64_t)r * n];
+    b += pv[(int64_t)r * n];
   }
   bf16x4 oa, ob;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    oa[e] = (__bf16)(a[e] * scale);
+    oa[e] = (__bf16)(a[e] * p.scale);
     ob[e] = (__bf16)b[e];
   }
-  *(bf16x4*)(dK + s * dk_ss + (int64_t)hh * dk_hs + 4 * c) = oa;
-  *(bf16x4*)(dV + s * dv_ss + (int64_t)hh * dv_hs + 4 * c) = ob;
+  *(bf16x4*)(p.dK + brow * p.dk_bs + s * p.dk_ss + (int64_t)hh * p.dk_hs + 4 * c) = oa;
+  *(bf16x4*)(p.dV + brow * p.dv_bs + s * p.dv_ss + (int64_t)hh * p.dv_hs + 4 * c) = ob;
 }
 
 }  // namespace artk
@@ -1057,51 +1146,82 @@ using namespace artk;
 
 extern "C" {
 
-size_t artk_attn_plan_bytes(int64_t S) {
+static int64_t attn_padded(int64_t S) { return (S + ATT_ROW - 1) / ATT_ROW * ATT_ROW; }
+
+size_t artk_attn_plan_rows_bytes(int64_t B, int64_t S) {
   AttnPlan pl;
-  return attn_plan_layout(nullptr, 0, S, pl) + 256;
+  attn_plan_layout(nullptr, 0, attn_padded(S), pl);
+  return (size_t)(B * pl.stride) + 256;
+}
+size_t artk_attn_plan_row_stride(int64_t S) {
+  AttnPlan pl;
+  attn_plan_layout(nullptr, 0, attn_padded(S), pl);
+  return (size_t)pl.stride;
+}
+size_t artk_attn_plan_bytes(int64_t S) { return artk_attn_plan_rows_bytes(1, S); }
+
+static int32_t attn_check_len(int64_t B, int64_t S) {
+  ARTK_CHECK_ARG(B > 0 && S > 0, "B and S must be positive");
+  if (attn_padded(S) / ATT_BN > ATT_MAX_KB || B > 65535) {
+    set_error("row length %lld must be at most %d (and the batch at most 65535 rows)", (long long)S, ATT_MAX_KB * ATT_BN);
+    return ARTK_ERR_UNSUPPORTED_SHAPE;
+  }
+  return ARTK_OK;
+}
+static int32_t attn_check_multiple(int64_t S) {
+  if (S % ATT_ROW != 0 || S / ATT_BN > ATT_MAX_KB) {
+    set_error("row length %lld must be a multiple of %d and at most %d", (long long)S, ATT_ROW,
+              ATT_MAX_KB * ATT_BN);
+    return ARTK_ERR_UNSUPPORTED_SHAPE;
+  }
+  return ARTK_OK;
+}
+
+int32_t artk_attn_plan_rows(const int64_t* group_ids, const int64_t* parent_ids, int64_t B, int64_t S, void* plan,
+                            size_t plan_bytes, artk_stream_t stream) {
+  ARTK_CHECK_ARG(group_ids && parent_ids && plan, "null pointer argument");
+  int32_t rc = attn_check_len(B, S);
+  if (rc) return rc;
+  AttnPlan pl;
+  if (plan_bytes < artk_attn_plan_rows_bytes(B, S) ||
+      attn_plan_layout(plan, plan_bytes, attn_padded(S), pl) == (size_t)-1) {
+    set_error("plan buffer too small: need %zu bytes, got %zu", artk_attn_plan_rows_bytes(B, S), plan_bytes);
+    return ARTK_ERR_WORKSPACE_TOO_SMALL;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  const unsigned b = (unsigned)B;
+  attn_heads_kernel<<<b, 1024, 0, st>>>(group_ids, (int)S, pl.stride, pl.heads, pl.n_heads);
+  ARTK_CHECK_LAUNCH();
+  attn_codes_kernel<<<dim3((unsigned)(attn_padded(S) / 256), b), 256, 0, st>>>(group_ids, parent_ids, (int)S, pl.stride,
+                                                                              pl.heads, pl.n_heads, pl.gc, pl.pc,
+                                                                              pl.uni);
+  ARTK_CHECK_LAUNCH();
+  attn_classify_kernel<<<dim3((unsigned)((pl.nKb + 3) / 4), (unsigned)pl.nQb, b), 256, 0, st>>>(
+      pl.gc, pl.pc, pl.uni, pl.stride, pl.nKb, pl.nQb2, pl.info, pl.info2);
+  ARTK_CHECK_LAUNCH();
+  const AttnTable t1{pl.info, pl.list, pl.cnt, pl.nQb, pl.nKb}, t2{pl.info2, pl.list2, pl.cnt2, pl.nKb2, pl.nQb2};
+  attn_compact_kernel<<<dim3((unsigned)(pl.nQb + pl.nKb2), b), 256, 0, st>>>(t1, t2, pl.stride);
+  ARTK_CHECK_LAUNCH();
+  attn_order_kernel<<<dim3(2, b), 1024, 0, st>>>(pl.cnt, pl.nQb, pl.order, pl.cnt2, pl.nKb2, pl.order2, pl.total2,
+                                                 pl.stride);
+  ARTK_CHECK_LAUNCH();
+  return ARTK_OK;
 }
 
 int32_t artk_attn_plan(const int64_t* group_ids, const int64_t* parent_ids, int64_t S, void* plan,
                        size_t plan_bytes, artk_stream_t stream) {
   ARTK_CHECK_ARG(group_ids && parent_ids && plan, "null pointer argument");
   ARTK_CHECK_ARG(S > 0, "S must be positive");
-  if (S % ATT_ROW != 0 || S / ATT_BN > ATT_MAX_KB) {
-    set_error("row length %lld must be a multiple of %d and at most %d", (long long)S, ATT_ROW,
-              ATT_MAX_KB * ATT_BN);
-    return ARTK_ERR_UNSUPPORTED_SHAPE;
-  }
-  AttnPlan pl;
-  if (attn_plan_layout(plan, plan_bytes, S, pl) == (size_t)-1) {
-    set_error("plan buffer too small: need %zu bytes, got %zu", artk_attn_plan_bytes(S), plan_bytes);
-    return ARTK_ERR_WORKSPACE_TOO_SMALL;
-  }
-  hipStream_t st = (hipStream_t)stream;
-  attn_codes_kernel<<<(unsigned)(S / 256), 256, 0, st>>>(group_ids, parent_ids, (int)S, pl.gc, pl.pc);
-  ARTK_CHECK_LAUNCH();
-  attn_classify_kernel<0><<<dim3((unsigned)((pl.nKb + 3) / 4), (unsigned)pl.nQb), 256, 0, st>>>(
-      pl.gc, pl.pc, pl.nKb, pl.info);
-  ARTK_CHECK_LAUNCH();
-  attn_compact_kernel<<<(unsigned)pl.nQb, 256, 0, st>>>(pl.info, pl.nKb, pl.list, pl.cnt);
-  ARTK_CHECK_LAUNCH();
-  attn_classify_kernel<1><<<dim3((unsigned)((pl.nQb2 + 3) / 4), (unsigned)pl.nKb2), 256, 0, st>>>(
-      pl.gc, pl.pc, pl.nQb2, pl.info2);
-  ARTK_CHECK_LAUNCH();
-  attn_compact_kernel<<<(unsigned)pl.nKb2, 256, 0, st>>>(pl.info2, pl.nQb2, pl.list2, pl.cnt2);
-  ARTK_CHECK_LAUNCH();
-  attn_order_kernel<<<2, 1024, 0, st>>>(pl.cnt, pl.nQb, pl.order, pl.cnt2, pl.nKb2, pl.order2, pl.total2);
-  ARTK_CHECK_LAUNCH();
-  return ARTK_OK;
+  int32_t rc = attn_check_multiple(S);
+  if (rc) return rc;
+  return artk_attn_plan_rows(group_ids, parent_ids, 1, S, plan, plan_bytes, stream);
 }
 
-static int32_t attn_check(int64_t S, int32_t Hq, int32_t Hkv, int32_t D, const int64_t* strides,
-                          int nstrides) {
-  ARTK_CHECK_ARG(S > 0 && Hq > 0 && Hkv > 0, "S, Hq, Hkv must be positive");
-  if (S % ATT_ROW != 0 || S / ATT_BN > ATT_MAX_KB) {
-    set_error("row length %lld must be a multiple of %d and at most %d", (long long)S, ATT_ROW,
-              ATT_MAX_KB * ATT_BN);
-    return ARTK_ERR_UNSUPPORTED_SHAPE;
-  }
+// strides: (batch, position, head) of nt tensors, in elements.
+static int32_t attn_check(int64_t B, int64_t S, int32_t Hq, int32_t Hkv, int32_t D, const int64_t* strides, int nt) {
+  ARTK_CHECK_ARG(Hq > 0 && Hkv > 0, "S, Hq, Hkv must be positive");
+  int32_t rc = attn_check_len(B, S);
+  if (rc) return rc;
   if (D != 64 && D != 128) {
     set_error("head dimension %d is not supported (64 or 128)", D);
     return ARTK_ERR_UNSUPPORTED_SHAPE;
@@ -1110,9 +1230,11 @@ static int32_t attn_check(int64_t S, int32_t Hq, int32_t Hkv, int32_t D, const i
     set_error("query heads (%d) must be a multiple of key/value heads (%d)", Hq, Hkv);
     return ARTK_ERR_UNSUPPORTED_SHAPE;
   }
-  for (int i = 0; i < nstrides; ++i) {
-    ARTK_CHECK_ARG(strides[i] > 0 && strides[i] % 8 == 0, "strides must be positive multiples of 8 elements");
-    ARTK_CHECK_ARG(i % 2 != 0 || S * strides[i] * 2 < (1ll << 31), "operand spans 2 GiB or more");
+  for (int i = 0; i < nt; ++i) {
+    const int64_t *s = strides + 3 * i;
+    ARTK_CHECK_ARG(s[1] > 0 && s[1] % 8 == 0 && s[2] > 0 && s[2] % 8 == 0 && s[0] >= 0 && s[0] % 8 == 0,
+                   "strides must be positive multiples of 8 elements");
+    ARTK_CHECK_ARG(attn_padded(S) * s[1] * 2 < (1ll << 31), "operand spans 2 GiB or more");
   }
   return ARTK_OK;
 }
@@ -1122,22 +1244,17 @@ size_t artk_attn_fwd_workspace_bytes(int64_t S, int32_t Hkv, int32_t D) {
   return 256;  // the forward needs no scratch; kept so that every op has the same calling pattern
 }
 
-int32_t artk_attn_fwd(const void* q, const void* k, const void* v, const void* plan, int64_t S,
-                      int32_t Hq, int32_t Hkv, int32_t D, int64_t q_stride_s, int64_t q_stride_h,
-                      int64_t k_stride_s, int64_t k_stride_h, int64_t v_stride_s, int64_t v_stride_h,
-                      int64_t o_stride_s, int64_t o_stride_h, float scale, void* out, float* lse,
-                      void* workspace, size_t workspace_bytes, artk_stream_t stream) {
-  ARTK_CHECK_ARG(q && k && v && plan && out && lse, "null pointer argument");
+int32_t artk_attn_fwd_rows(const void* q, const void* k, const void* v, const void* plan, int64_t B, int64_t S,
+                           int32_t Hq, int32_t Hkv, int32_t D, const int64_t* strides, float scale, void* out,
+                           float* lse, artk_stream_t stream) {
+  ARTK_CHECK_ARG(q && k && v && plan && out && lse && strides, "null pointer argument");
   ARTK_CHECK_ARG(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out),
                  "q, k, v, out must be 16-byte aligned");
-  const int64_t strides[8] = {q_stride_s, q_stride_h, k_stride_s, k_stride_h,
-                              v_stride_s, v_stride_h, o_stride_s, o_stride_h};
-  int32_t rc = attn_check(S, Hq, Hkv, D, strides, 8);
+  int32_t rc = attn_check(B, S, Hq, Hkv, D, strides, 4);
   if (rc) return rc;
   ARTK_CHECK_ARG(scale > 0.f && scale < INFINITY, "scale must be positive and finite");
-  (void)workspace; (void)workspace_bytes;
   AttnPlan pl;
-  attn_plan_layout(const_cast<void*>(plan), (size_t)1 << 40, S, pl);
+  attn_plan_layout(const_cast<void*>(plan), (size_t)1 << 40, attn_padded(S), pl);
   hipStream_t st = (hipStream_t)stream;
   AttnFwdParams p;
   p.Q = (const uint16_t*)q;
@@ -1145,26 +1262,23 @@ int32_t artk_attn_fwd(const void* q, const void* k, const void* v, const void* p
   p.V = (const uint16_t*)v;
   p.O = (uint16_t*)out;
   p.lse = lse;
-  p.q_ss = q_stride_s;
-  p.q_hs = q_stride_h;
-  p.k_ss = k_stride_s;
-  p.k_hs = k_stride_h;
-  p.v_ss = v_stride_s;
-  p.v_hs = v_stride_h;
-  p.o_ss = o_stride_s;
-  p.o_hs = o_stride_h;
+  p.q_bs = strides[0];  p.q_ss = strides[1];   p.q_hs = strides[2];
+  p.k_bs = strides[3];  p.k_ss = strides[4];   p.k_hs = strides[5];
+  p.v_bs = strides[6];  p.v_ss = strides[7];   p.v_hs = strides[8];
+  p.o_bs = strides[9];  p.o_ss = strides[10];  p.o_hs = strides[11];
   p.gc = pl.gc;
   p.pc = pl.pc;
   p.list = pl.list;
   p.cnt = pl.cnt;
   p.order = pl.order;
+  p.plan_stride = pl.stride;
   p.S = (int)S;
   p.Hq = Hq;
   p.Hkv = Hkv;
   p.nQb = pl.nQb;
   p.nKb = pl.nKb;
   p.scale_log2e = scale * LOG2E;
-  const unsigned grid = attn_grid(Hq, Hkv, pl.nQb);
+  const dim3 grid(attn_grid(Hq, Hkv, pl.nQb), (unsigned)B);
   prof_begin(PROF_ATTN_FWD, st);
   if (D == 128)
     attn_fwd_kernel<128><<<grid, ATT_THREADS, 0, st>>>(p);
@@ -1175,70 +1289,85 @@ int32_t artk_attn_fwd(const void* q, const void* k, const void* v, const void* p
   return ARTK_OK;
 }
 
-size_t artk_attn_bwd_workspace_bytes(int64_t S, int32_t Hq, int32_t Hkv, int32_t D) {
-  Workspace ws(nullptr, 0);
-  ws.take<float>((size_t)S * Hq);
-  ws.take<float>((size_t)S * Hq);
-  if (Hq != Hkv) {
-    ws.take<float>((size_t)S * Hq * D);
-    ws.take<float>((size_t)S * Hq * D);
-  }
-  return ws.used + 256;
+int32_t artk_attn_fwd(const void* q, const void* k, const void* v, const void* plan, int64_t S,
+                      int32_t Hq, int32_t Hkv, int32_t D, int64_t q_stride_s, int64_t q_stride_h,
+                      int64_t k_stride_s, int64_t k_stride_h, int64_t v_stride_s, int64_t v_stride_h,
+                      int64_t o_stride_s, int64_t o_stride_h, float scale, void* out, float* lse,
+                      void* workspace, size_t workspace_bytes, artk_stream_t stream) {
+  (void)workspace; (void)workspace_bytes;
+  ARTK_CHECK_ARG(S > 0, "S, Hq, Hkv must be positive");
+  int32_t rc = attn_check_multiple(S);
+  if (rc) return rc;
+  const int64_t strides[12] = {0, q_stride_s, q_stride_h, 0, k_stride_s, k_stride_h,
+                               0, v_stride_s, v_stride_h, 0, o_stride_s, o_stride_h};
+  return artk_attn_fwd_rows(q, k, v, plan, 1, S, Hq, Hkv, D, strides, scale, out, lse, stream);
 }
 
-int32_t artk_attn_bwd(const void* q, const void* k, const void* v, const void* out, const float* lse,
-                      const void* d_out, const void* plan, int64_t S, int32_t Hq, int32_t Hkv,
-                      int32_t D, const int64_t* strides, float scale, void* dq, void* dk, void* dv,
-                      void* workspace, size_t workspace_bytes, artk_stream_t stream) {
+struct AttnBwdScratch {
+  float *delta, *lse2, *pk, *pv;
+};
+static void carve_attn_bwd(Workspace& ws, int64_t B, int64_t S, int Hq, int Hkv, int D, AttnBwdScratch& c) {
+  const size_t n = (size_t)(B * attn_padded(S) * Hq);
+  c.delta = ws.take<float>(n);
+  c.lse2 = ws.take<float>(n);
+  c.pk = Hq != Hkv ? ws.take<float>(n * D) : nullptr;
+  c.pv = Hq != Hkv ? ws.take<float>(n * D) : nullptr;
+}
+size_t artk_attn_bwd_rows_workspace_bytes(int64_t B, int64_t S, int32_t Hq, int32_t Hkv, int32_t D) {
+  Workspace ws(nullptr, 0);
+  AttnBwdScratch c;
+  carve_attn_bwd(ws, B, S, Hq, Hkv, D, c);
+  return ws.used + 256;
+}
+size_t artk_attn_bwd_workspace_bytes(int64_t S, int32_t Hq, int32_t Hkv, int32_t D) {
+  return artk_attn_bwd_rows_workspace_bytes(1, S, Hq, Hkv, D);
+}
+
+int32_t artk_attn_bwd_rows(const void* q, const void* k, const void* v, const void* out, const float* lse,
+                           const void* d_out, const void* plan, int64_t B, int64_t S, int32_t Hq, int32_t Hkv,
+                           int32_t D, const int64_t* strides, float scale, void* dq, void* dk, void* dv,
+                           void* workspace, size_t workspace_bytes, artk_stream_t stream) {
   ARTK_CHECK_ARG(q && k && v && out && lse && d_out && plan && strides && dq && dk && dv,
                  "null pointer argument");
   ARTK_CHECK_ARG(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out) && aligned16(d_out) &&
                      aligned16(dq) && aligned16(dk) && aligned16(dv),
                  "tensors must be 16-byte aligned");
-  int32_t rc = attn_check(S, Hq, Hkv, D, strides, 16);
+  int32_t rc = attn_check(B, S, Hq, Hkv, D, strides, 8);
   if (rc) return rc;
-  // the dK/dV kernel addresses q and d_out by head through 31-bit offsets
-  ARTK_CHECK_ARG((S * strides[0] + Hq * strides[1]) * 2 < (1ll << 31) &&
-                     (S * strides[8] + Hq * strides[9]) * 2 < (1ll << 31) && (int64_t)S * Hq * 4 < (1ll << 31),
-                 "q / d_out span 2 GiB or more");
+  // the dK/dV kernel addresses lse2 and delta by head through 31-bit offsets
+  ARTK_CHECK_ARG(attn_padded(S) * Hq * 4 < (1ll << 31), "S * Hq is too large");
   Workspace ws(workspace, workspace_bytes);
-  float* delta = ws.take<float>((size_t)S * Hq);
-  float* lse2 = ws.take<float>((size_t)S * Hq);
-  float *pk = nullptr, *pv = nullptr;
-  if (Hq != Hkv) {
-    pk = ws.take<float>((size_t)S * Hq * D);
-    pv = ws.take<float>((size_t)S * Hq * D);
-  }
+  AttnBwdScratch c;
+  carve_attn_bwd(ws, B, S, Hq, Hkv, D, c);
   if (!ws.ok()) {
     set_error("workspace too small: need %zu bytes, got %zu", ws.used, workspace_bytes);
     return ARTK_ERR_WORKSPACE_TOO_SMALL;
   }
   AttnPlan pl;
-  attn_plan_layout(const_cast<void*>(plan), (size_t)1 << 40, S, pl);
+  attn_plan_layout(const_cast<void*>(plan), (size_t)1 << 40, attn_padded(S), pl);
   hipStream_t st = (hipStream_t)stream;
-  attn_delta_kernel<<<(unsigned)((S * Hq + 15) / 16), 256, 0, st>>>(
-      (const uint16_t*)out, strides[6], strides[7], (const uint16_t*)d_out, strides[8], strides[9], lse,
-      (int)S, Hq, D, delta, lse2);
-  ARTK_CHECK_LAUNCH();
   AttnBwdParams p;
   p.Q = (const uint16_t*)q;
   p.K = (const uint16_t*)k;
   p.V = (const uint16_t*)v;
+  p.O = (const uint16_t*)out;
   p.dO = (const uint16_t*)d_out;
-  p.lse2 = lse2;
-  p.delta = delta;
+  p.lse = lse;
+  p.lse2 = c.lse2;
+  p.delta = c.delta;
   p.dQ = (uint16_t*)dq;
   p.dK = (uint16_t*)dk;
   p.dV = (uint16_t*)dv;
-  p.pK = pk;
-  p.pV = pv;
-  p.q_ss = strides[0];  p.q_hs = strides[1];
-  p.k_ss = strides[2];  p.k_hs = strides[3];
-  p.v_ss = strides[4];  p.v_hs = strides[5];
-  p.do_ss = strides[8]; p.do_hs = strides[9];
-  p.dq_ss = strides[10]; p.dq_hs = strides[11];
-  p.dk_ss = strides[12]; p.dk_hs = strides[13];
-  p.dv_ss = strides[14]; p.dv_hs = strides[15];
+  p.pK = c.pk;
+  p.pV = c.pv;
+  p.q_bs = strides[0];   p.q_ss = strides[1];   p.q_hs = strides[2];
+  p.k_bs = strides[3];   p.k_ss = strides[4];   p.k_hs = strides[5];
+  p.v_bs = strides[6];   p.v_ss = strides[7];   p.v_hs = strides[8];
+  p.o_bs = strides[9];   p.o_ss = strides[10];  p.o_hs = strides[11];
+  p.do_bs = strides[12]; p.do_ss = strides[13]; p.do_hs = strides[14];
+  p.dq_bs = strides[15]; p.dq_ss = strides[16]; p.dq_hs = strides[17];
+  p.dk_bs = strides[18]; p.dk_ss = strides[19]; p.dk_hs = strides[20];
+  p.dv_bs = strides[21]; p.dv_ss = strides[22]; p.dv_hs = strides[23];
   p.gc = pl.gc;
   p.pc = pl.pc;
   p.list = pl.list;
@@ -1247,7 +1376,9 @@ int32_t artk_attn_bwd(const void* q, const void* k, const void* v, const void* o
   p.listT = pl.list2;
   p.cntT = pl.cnt2;
   p.orderT = pl.order2;
+  p.plan_stride = pl.stride;
   p.S = (int)S;
+  p.Sp = (int)attn_padded(S);
   p.Hq = Hq;
   p.Hkv = Hkv;
   p.nQb = pl.nQb;
@@ -1259,32 +1390,48 @@ int32_t artk_attn_bwd(const void* q, const void* k, const void* v, const void* o
   {
     const int slots = num_cus() * (D == 64 ? 3 : 2);  // resident work-groups
     p.split.total = pl.total2;
-    p.split.heads_all = Hq;
-    p.split.div = pl.nKb2 * Hkv >= 2 * slots ? slots * 3 / 2 : slots * 4;
+    p.split.heads_all = (int)(B * Hq);   // (rows of a batch are taken to be alike)
+    p.split.div = B * pl.nKb2 * Hkv >= 2 * slots ? slots * 3 / 2 : slots * 4;
+    p.split.light_max = g_light_max_override;  // artk_attn_bwd_tuning
   }
-  p.split.light_max = g_light_max_override;  // artk_attn_bwd_tuning
+  const dim3 grid_q(attn_grid(Hq, Hkv, pl.nQb), (unsigned)B), grid_kv(attn_grid(Hq, Hkv, pl.nKb2), (unsigned)B);
+  prof_begin(PROF_ATTN_BWD_Q, st);
+  if (D == 128)
+    attn_bwd_dq_kernel<128><<<grid_q, ATT_THREADS, 0, st>>>(p);
+  else
+    attn_bwd_dq_kernel<64><<<grid_q, ATT_THREADS, 0, st>>>(p);
+  prof_end(PROF_ATTN_BWD_Q, st);
+  ARTK_CHECK_LAUNCH();
   prof_begin(PROF_ATTN_BWD_KV, st);
   if (D == 128)
-    attn_bwd_kv_kernel<128><<<attn_grid(Hq, Hkv, pl.nKb2), 256, 0, st>>>(p);
+    attn_bwd_kv_kernel<128><<<grid_kv, 256, 0, st>>>(p);
   else
-    attn_bwd_kv_kernel<64><<<attn_grid(Hq, Hkv, pl.nKb2), 256, 0, st>>>(p);
+    attn_bwd_kv_kernel<64><<<grid_kv, 256, 0, st>>>(p);
   prof_end(PROF_ATTN_BWD_KV, st);
   ARTK_CHECK_LAUNCH();
   if (Hq != Hkv) {
-    const int64_t n4 = S * Hkv * (D / 4);
-    attn_kv_reduce_kernel<<<(unsigned)((n4 + 255) / 256), 256, 0, st>>>(
-        pk, pv, pl.cnt2, p.split, Hq / Hkv, S, Hkv, D, scale, (uint16_t*)dk, strides[12], strides[13], (uint16_t*)dv,
-        strides[14], strides[15]);
+    const int64_t n4 = (int64_t)p.Sp * Hkv * (D / 4);
+    attn_kv_reduce_kernel<<<dim3((unsigned)((n4 + 255) / 256), (unsigned)B), 256, 0, st>>>(p, D);
     ARTK_CHECK_LAUNCH();
   }
-  prof_begin(PROF_ATTN_BWD_Q, st);
-  if (D == 128)
-    attn_bwd_dq_kernel<128><<<attn_grid(Hq, Hkv, pl.nQb), ATT_THREADS, 0, st>>>(p);
-  else
-    attn_bwd_dq_kernel<64><<<attn_grid(Hq, Hkv, pl.nQb), ATT_THREADS, 0, st>>>(p);
-  prof_end(PROF_ATTN_BWD_Q, st);
-  ARTK_CHECK_LAUNCH();
   return ARTK_OK;
+}
+
+int32_t artk_attn_bwd(const void* q, const void* k, const void* v, const void* out, const float* lse,
+                      const void* d_out, const void* plan, int64_t S, int32_t Hq, int32_t Hkv,
+                      int32_t D, const int64_t* strides, float scale, void* dq, void* dk, void* dv,
+                      void* workspace, size_t workspace_bytes, artk_stream_t stream) {
+  ARTK_CHECK_ARG(S > 0 && strides, "S, Hq, Hkv must be positive");
+  int32_t rc = attn_check_multiple(S);
+  if (rc) return rc;
+  int64_t s3[24];
+  for (int i = 0; i < 8; ++i) {
+    s3[3 * i] = 0;
+    s3[3 * i + 1] = strides[2 * i];
+    s3[3 * i + 2] = strides[2 * i + 1];
+  }
+  return artk_attn_bwd_rows(q, k, v, out, lse, d_out, plan, 1, S, Hq, Hkv, D, s3, scale, dq, dk, dv, workspace,
+                            workspace_bytes, stream);
 }
 
 int32_t artk_attn_bwd_tuning(int32_t light_max) {

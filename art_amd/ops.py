@@ -491,9 +491,11 @@ def moe_experts_bwd(g, x, routing: Routing, saved, Wt_gu, Wt_d, adapters: dict, 
 # Packed-row attention
 # -----------------------------------------------------------------------------
 class AttnPlan:
-    """Device-side description of one packed row's visibility (see artk_attn_plan)."""
+    """Device-side description of one packed row's visibility (see artk_attn_plan).  ``S``: the
+    row's length rounded up to a multiple of 256.  Plans made together (attn_plan_rows) keep the
+    buffer of all of them in ``batch`` and their place in it in ``index``."""
 
-    __slots__ = ("buf", "S")
+    __slots__ = ("buf", "S", "batch", "index", "rows")
 
 
 def attn_plan(group_ids: torch.Tensor, parent_ids: torch.Tensor) -> AttnPlan:
@@ -505,10 +507,78 @@ def attn_plan(group_ids: torch.Tensor, parent_ids: torch.Tensor) -> AttnPlan:
     dev = group_ids.device
     plan = AttnPlan()
     plan.S = S
-    plan.buf = torch.empty(lib.artk_attn_plan_bytes(S), dtype=torch.uint8, device=dev)
+    plan.buf = plan.batch = torch.empty(lib.artk_attn_plan_bytes(S), dtype=torch.uint8, device=dev)
+    plan.index, plan.rows = 0, 1
     _lib.check(lib.artk_attn_plan(group_ids.data_ptr(), parent_ids.data_ptr(), S, plan.buf.data_ptr(),
                                   plan.buf.numel(), _stream(dev)))
     return plan
+
+
+def attn_plan_rows(group_ids: torch.Tensor, parent_ids: torch.Tensor) -> "list[AttnPlan]":
+    """One plan per row of int64 [B, S] ids, of any length S, made in one call."""
+    B, S = group_ids.shape
+    _need(group_ids, "group_ids", torch.int64, (B, S))
+    _need(parent_ids, "parent_ids", torch.int64, (B, S))
+    lib = _lib.load()
+    dev = group_ids.device
+    buf = torch.empty(lib.artk_attn_plan_rows_bytes(B, S), dtype=torch.uint8, device=dev)
+    _lib.check(lib.artk_attn_plan_rows(group_ids.data_ptr(), parent_ids.data_ptr(), B, S, buf.data_ptr(),
+                                       buf.numel(), _stream(dev)))
+    step = lib.artk_attn_plan_row_stride(S) if B > 1 else 0
+    plans = []
+    for b in range(B):
+        plan = AttnPlan()
+        plan.S, plan.batch, plan.index, plan.rows = (S + 255) // 256 * 256, buf, b, B
+        plan.buf = buf[b * step:] if b else buf
+        plans.append(plan)
+    return plans
+
+
+def _strides3(t: torch.Tensor, name: str):
+    """(batch, position, head) strides of a bf16 [B, S, H, D] view whose last dimension is contiguous."""
+    if t.dtype != torch.bfloat16 or t.dim() != 4 or t.stride(3) != 1 or not t.is_cuda:
+        raise ValueError(f"{name}: expected a bf16 device tensor [B, S, H, D] with contiguous D")
+    return (t.stride(0) if t.shape[0] > 1 else 0, t.stride(1), t.stride(2))
+
+
+def attn_fwd_rows(q, k, v, plan: torch.Tensor, scale: Optional[float] = None):
+    """(out bf16 [B, S, Hq, D], lse f32 [B, Hq, S]) for q [B, S, Hq, D], k/v [B, S, Hkv, D] (any strides over
+    B, S, H) and the plan buffer of B rows (AttnPlan.batch, or AttnPlan.buf for one row)."""
+    B, S, Hq, D = q.shape
+    Hkv = k.shape[2]
+    if k.shape != (B, S, Hkv, D) or v.shape != (B, S, Hkv, D):
+        raise ValueError("attention: inconsistent shapes")
+    lib = _lib.load()
+    dev = q.device
+    out = torch.empty((B, S, Hq, D), dtype=torch.bfloat16, device=dev)
+    lse = torch.empty((B, Hq, S), dtype=torch.float32, device=dev)
+    strides = (_lib._i64 * 12)(*_strides3(q, "q"), *_strides3(k, "k"), *_strides3(v, "v"), S * Hq * D, Hq * D, D)
+    scale = float(D) ** -0.5 if scale is None else float(scale)
+    _lib.check(lib.artk_attn_fwd_rows(q.data_ptr(), k.data_ptr(), v.data_ptr(), plan.data_ptr(), B, S, Hq, Hkv, D,
+                                      strides, scale, out.data_ptr(), lse.data_ptr(), _stream(dev)))
+    return out, lse
+
+
+def attn_bwd_rows(q, k, v, out, lse, d_out, plan: torch.Tensor, scale: Optional[float] = None):
+    """(dq, dk, dv) bf16, contiguous [B, S, H, D], for the upstream gradient d_out of attn_fwd_rows' out."""
+    B, S, Hq, D = q.shape
+    Hkv = k.shape[2]
+    lib = _lib.load()
+    dev = q.device
+    dq = torch.empty((B, S, Hq, D), dtype=torch.bfloat16, device=dev)
+    dk = torch.empty((B, S, Hkv, D), dtype=torch.bfloat16, device=dev)
+    dv = torch.empty((B, S, Hkv, D), dtype=torch.bfloat16, device=dev)
+    _need(lse, "lse", torch.float32, (B, Hq, S))
+    kv = (S * Hkv * D, Hkv * D, D)
+    strides = (_lib._i64 * 24)(*_strides3(q, "q"), *_strides3(k, "k"), *_strides3(v, "v"), *_strides3(out, "out"),
+                               *_strides3(d_out, "d_out"), S * Hq * D, Hq * D, D, *kv, *kv)
+    ws = _workspace(lib.artk_attn_bwd_rows_workspace_bytes(B, S, Hq, Hkv, D), dev)
+    scale = float(D) ** -0.5 if scale is None else float(scale)
+    _lib.check(lib.artk_attn_bwd_rows(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
+                                      d_out.data_ptr(), plan.data_ptr(), B, S, Hq, Hkv, D, strides, scale,
+                                      dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), ws.numel(),
+                                      _stream(dev)))
+    return dq, dk, dv
 
 
 def _shd(t: torch.Tensor, name: str):

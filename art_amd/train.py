@@ -275,8 +275,7 @@ def get_compute_loss_fn(trainer) -> Callable[..., torch.Tensor]:
             # opt-in (no counterpart in the reference): the model's attention layers call
             # art_amd.attention.packed_attention and take, as `causal_mask`, one plan per packed row
             # made from the ids; the dense [B, S, S] bias (2 S^2 bytes per row) is never built
-            attn_bias = [ops.attn_plan(inputs["group_ids"][b].contiguous(), inputs["parent_ids"][b].contiguous())
-                         for b in range(batch_size)]
+            attn_bias = ops.attn_plan_rows(inputs["group_ids"].contiguous(), inputs["parent_ids"].contiguous())
         else:
             attn_bias = calculate_attn_bias(batch_size, seq_len, device, inputs["group_ids"],
                                             inputs["parent_ids"], autocast_dtype)

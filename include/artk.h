@@ -327,12 +327,29 @@ int32_t artk_attn_bwd(const void* q, const void* k, const void* v, const void* o
                       int32_t D, const int64_t* strides, float scale, void* dq, void* dk, void* dv,
                       void* workspace, size_t workspace_bytes, artk_stream_t stream);
 
-/* Tuning aid of artk_attn_bwd (no counterpart in the reference).  With grouped-query heads a
- * key block seen by at most `light_max` (query tile, head) pairs is handled by one work-group
- * for all heads of its group; busier blocks get one work-group per head and a fixed-order
- * reduction.  The library picks the threshold by itself (64 for rows long enough to fill the
- * GPU that way, else 0); this call overrides it for later artk_attn_bwd calls made on the
- * calling thread, light_max < 0 restores the automatic choice.  Results agree to rounding. */
+/* The same for a batch of B rows of any length S in one call each (what art_amd.attention uses): ids
+ * [B,S]; a plan of artk_attn_plan_rows_bytes(B, S) bytes, in which row b's plan lies
+ * artk_attn_plan_row_stride(S) bytes behind row b-1's and can be used on its own; strides: (batch,
+ * position, head) of q, k, v, out (12 values), then d_out, dq, dk, dv (24); lse f32 [B,Hq,S]. */
+size_t artk_attn_plan_rows_bytes(int64_t B, int64_t S);
+size_t artk_attn_plan_row_stride(int64_t S);
+int32_t artk_attn_plan_rows(const int64_t* group_ids, const int64_t* parent_ids, int64_t B, int64_t S, void* plan,
+                            size_t plan_bytes, artk_stream_t stream);
+int32_t artk_attn_fwd_rows(const void* q, const void* k, const void* v, const void* plan, int64_t B, int64_t S,
+                           int32_t Hq, int32_t Hkv, int32_t D, const int64_t* strides, float scale, void* out,
+                           float* lse, artk_stream_t stream);
+size_t artk_attn_bwd_rows_workspace_bytes(int64_t B, int64_t S, int32_t Hq, int32_t Hkv, int32_t D);
+int32_t artk_attn_bwd_rows(const void* q, const void* k, const void* v, const void* out, const float* lse,
+                           const void* d_out, const void* plan, int64_t B, int64_t S, int32_t Hq, int32_t Hkv,
+                           int32_t D, const int64_t* strides, float scale, void* dq, void* dk, void* dv,
+                           void* workspace, size_t workspace_bytes, artk_stream_t stream);
+
+/* Tuning aid of artk_attn_bwd (no counterpart in the reference).  With grouped-query heads the heads
+ * of a group are shared out over work-groups, with a fixed-order reduction where they are more than
+ * one; the library picks the share from the load of the launch.  This call overrides it for later
+ * artk_attn_bwd calls made on the calling thread: all heads in one work-group for a key block seen by
+ * at most `light_max` (query tile, head) pairs, one head per work-group otherwise; light_max < 0
+ * restores the automatic choice.  Results agree to rounding. */
 int32_t artk_attn_bwd_tuning(int32_t light_max);
 
 /* ------------------------------------------------------------------------- *

@@ -296,3 +296,42 @@ def test_attn_bwd_mixed_light_and_heavy_key_blocks(artk_lib, gpu):
         assert rel_l2(dv.float().cpu(), ref_dv) <= 1e-2
         results[knob] = (dk, dv)
     assert rel_l2(results[64][0].float(), results[0][0].float()) <= 4e-3
+
+
+@pytest.mark.parametrize("B,S,Hq,Hkv,D,head_major", [
+    (3, 5, 2, 1, 64, False),       # a handful of positions (one alone has a zero gradient, no relative error)
+    (2, 65, 4, 4, 128, True),      # one head per group; one position in the second key tile
+    (3, 257, 6, 2, 64, True),      # one position in the second padded block
+    (2, 700, 7, 1, 128, False),
+])
+def test_packed_attention_ragged_batch(artk_lib, gpu, B, S, Hq, Hkv, D, head_major):
+    """A batch of rows whose length is no multiple of a tile, in one call: nothing outside a head's S rows may
+    be read (the tensors are embedded in NaN) and every row equals the oracle.  Plans made together and plans
+    made one by one (a call per row) agree bit for bit."""
+    from art_amd.attention import attention_plans, packed_attention
+    print("ragged batch", B, S, Hq, Hkv, D, head_major, flush=True)
+    g = torch.Generator().manual_seed(B * 1000 + S)
+    data = [torch.randn(B, S, H, D, generator=g).to(torch.bfloat16) for H in (Hq, Hkv, Hkv, Hq)]
+
+    def embed(t):   # the same values inside a larger tensor of NaN
+        b, s, h, d = t.shape
+        big = torch.full((b, h + 1, s + 9, d) if head_major else (b, s + 9, h + 1, d), float("nan"),
+                         dtype=torch.bfloat16, device=gpu)
+        view = big[:, :h, :s].transpose(1, 2) if head_major else big[:, :s, :h]
+        view.copy_(t)
+        return view
+
+    ids = [synthetic.packed_row_ids(60 + b, S, 1, max(S // 5, 1), 2, S // 4) for b in range(B)]
+    group, parent = torch.stack([i[0] for i in ids]), torch.stack([i[1] for i in ids])
+    q, k, v, up = (embed(t) for t in data)
+    leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+    plans = attention_plans(group.to(gpu), parent.to(gpu))
+    out = packed_attention(*leaves, plans)
+    grads = torch.autograd.grad(out, leaves, up)
+    single = [attention_plans(group[b].to(gpu), parent[b].to(gpu))[0] for b in range(B)]
+    out1 = packed_attention(*leaves, single)
+    assert torch.equal(out1, out)
+    for b in range(B):
+        ref = attn_oracle.attention_grads(*(t[b] for t in data[:3]), group[b], parent[b], data[3][b])
+        for got, want in zip((out, *grads), ref):
+            assert torch.isfinite(got[b]).all() and rel_l2(got[b].float().cpu(), want) <= 1e-2
