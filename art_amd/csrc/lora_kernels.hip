@@ -17,6 +17,7 @@
 #include "common.hpp"
 #include "gemm_nt.hpp"
 #include "gemm_plain8.hpp"
+#include "gemm_small.hpp"
 #include "lora_common.hpp"
 #include "skinny_stats.hpp"
 
@@ -250,6 +251,126 @@ __global__ __launch_bounds__(nthreads<LORA_NI>()) void lora_multi_gemm_kernel(Lo
 }
 
 // ----------------------------------------------------------------------------
+// The same jobs on 128 x 128 tiles with the K range split over `split` work-groups (gemm_small.hpp), for products
+// whose 256 x 256 tiles do not fill the GPU.  Tiles are numbered through the jobs (job[].tile0 and MT count 128-row
+// tiles here), unit = tile * split + part.  The parts of a tile are equal shares of the K steps of all segments
+// together; with split > 1 each leaves its fp32 accumulators in `part` as [unit][wave][block][4][lane][4] and
+// lora_small_reduce_kernel adds them in order.
+// ----------------------------------------------------------------------------
+struct LoraSmallParams {
+  LoraMultiParams m;
+  float* part;
+  int split, ksteps[LORA_MAX_SEG];   // K steps of all segments of a job
+};
+
+__device__ __forceinline__ void lora_small_locate(const LoraSmallParams& p, int tile, int& j, int& mt, int& nt) {
+  j = 0;
+  while (j + 1 < p.m.n_jobs && tile >= p.m.job[j + 1].tile0) ++j;
+  tile_coords(tile - p.m.job[j].tile0, p.m.job[j].MT, p.m.NT, mt, nt);
+}
+
+// Bias and bf16 store of the 32 x 32 block whose first output feature is m0 and whose lane's column is col.
+__device__ __forceinline__ void lora_block_store(floatx16& c, const uint16_t* bias, uint16_t* out, int64_t M,
+                                                 int64_t N, int64_t m0, int64_t col, int half) {
+  if (m0 >= M) return;  // wave-uniform; M is a multiple of 64, so blocks are whole
+  if (bias != nullptr) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const bf16x4 bv = *(const bf16x4*)(bias + m0 + q * 8 + half * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) c[q * 4 + e] += (float)bv[e];
+    }
+  }
+  if (col < N) store_block_bf16(out + col * M + m0, c, half);
+}
+
+__global__ __launch_bounds__(ST2_THREADS, 2) void lora_small_gemm_kernel(LoraSmallParams p) {
+  __shared__ __attribute__((aligned(1024))) char smem[ST2_LDS_BYTES];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int unit = xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = unit / p.split, part = unit - tile * p.split;
+  int j, mt, nt;
+  lora_small_locate(p, tile, j, mt, nt);
+  const LoraJob& job = p.m.job[j];
+  const int total = p.ksteps[j];
+  int b = (int)((int64_t)total * part / p.split), e = (int)((int64_t)total * (part + 1) / p.split);
+  SmallAcc acc;
+  acc.zero();
+  const int wm = wave >> 1, wn = wave & 1, half = lane >> 5;
+  for (int s = 0; s < job.nseg; ++s) {
+    const LoraSeg& sg = p.m.seg[job.seg0 + s];
+    const int ks = (int)(sg.K / BK);
+    const int lo = b < 0 ? 0 : b, hi = e < ks ? e : ks;
+    if (lo < hi) {
+      SmallPanel lp, lq;
+      lp.init(sg.P, sg.K, (int64_t)mt * ST2, job.M, lane);
+      lq.init(sg.Q, sg.K, (int64_t)nt * ST2, p.m.N, lane);
+      small_tile_run(acc, smem, lp, lq, lo * BK, hi - lo);
+    }
+    b -= ks;
+    e -= ks;
+    if (part == 0 && sg.Pe != nullptr) {
+      // rank-r steps (see lowrank_steps), by the first part
+      for (int e0 = 0; e0 < sg.RP; e0 += 16) {
+        const int c = e0 + half * 8;
+        const bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
+        bf16x8 pf[2], qf[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          int64_t pr = (int64_t)mt * ST2 + wm * 64 + i * 32 + (lane & 31), qr = (int64_t)nt * ST2 + wn * 64 + i * 32 + (lane & 31);
+          pr = pr < job.M ? pr : job.M - 1;
+          qr = qr < p.m.N ? qr : p.m.N - 1;
+          pf[i] = *(const bf16x8*)(sg.Pe + pr * sg.r + (c < sg.r ? c : 0));
+          qf[i] = *(const bf16x8*)(sg.Qe + qr * sg.RP + c);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) pf[i] = c < sg.r ? pf[i] : z;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc.c[i >> 1][i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pf[i >> 1], qf[i & 1], acc.c[i >> 1][i & 1], 0, 0, 0);
+      }
+    }
+  }
+  if (p.split > 1) {
+    float* dst = p.part + (((int64_t)unit * 4 + wave) * 4) * 1024 + lane * 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *(floatx4*)(dst + i * 1024 + 256 * q) = floatx4{acc.c[i >> 1][i & 1][4 * q], acc.c[i >> 1][i & 1][4 * q + 1],
+                                                     acc.c[i >> 1][i & 1][4 * q + 2], acc.c[i >> 1][i & 1][4 * q + 3]};
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    lora_block_store(acc.c[i >> 1][i & 1], job.bias, job.out, job.M, p.m.N, (int64_t)mt * ST2 + wm * 64 + (i >> 1) * 32,
+                     (int64_t)nt * ST2 + wn * 64 + (i & 1) * 32 + (lane & 31), half);
+}
+
+// One work-group per tile and wave of the product kernel, one wave per 32 x 32 block.
+__global__ __launch_bounds__(256) void lora_small_reduce_kernel(LoraSmallParams p) {
+  const int lane = threadIdx.x & 63, i = threadIdx.x >> 6;
+  const int tile = blockIdx.x >> 2, wave = blockIdx.x & 3;
+  int j, mt, nt;
+  lora_small_locate(p, tile, j, mt, nt);
+  const LoraJob& job = p.m.job[j];
+  floatx16 c;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) c[k] = 0.f;
+  const float* src = p.part + (((int64_t)tile * p.split * 4 + wave) * 4 + i) * 1024 + lane * 4;
+#pragma unroll 4
+  for (int s = 0; s < p.split; ++s)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const floatx4 v = *(const floatx4*)(src + (int64_t)s * 16384 + 256 * q);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) c[4 * q + k] += v[k];
+    }
+  lora_block_store(c, job.bias, job.out, job.M, p.m.N, (int64_t)mt * ST2 + (wave >> 1) * 64 + (i >> 1) * 32,
+                   (int64_t)nt * ST2 + (wave & 1) * 64 + (i & 1) * 32 + (lane & 31), lane >> 5);
+}
+
+// ----------------------------------------------------------------------------
 // Row products: out[t, j] = sum_k X[t,k] Mt[j,k], Mt [R,K].  A block owns 16 rows
 // of X and 16 rows j0..j0+15 of Mt (rows >= R read as zero); its 4 waves split K.
 // Writes f32 [T,R] (unscaled) and bf16 [T,RP] (scaled, zero padded to RP).
@@ -321,32 +442,125 @@ static int32_t check_lora(int64_t T, int64_t in, int64_t out, int r) {
   return ARTK_OK;
 }
 
-static int32_t launch_lora_gemm(const void* P, const void* Q, const uint16_t* Pe, const uint16_t* Qe,
-                                const uint16_t* bias, void* out, int64_t M, int64_t N, int64_t K, int r,
-                                int RP, hipStream_t st) {
-  LoraGemmParams p;
-  p.P = P;
-  p.Q = Q;
-  p.Pe = Pe;
-  p.Qe = Qe;
-  p.bias = bias;
-  p.out = (uint16_t*)out;
-  p.M = M;
-  p.N = N;
-  p.K = K;
-  p.r = r;
-  p.RP = RP;
-  p.MT = (int)((M + TILE - 1) / TILE);
-  p.NT = (int)((N + TILE - 1) / TILE);
+// How the products of one call run: 256 x 256 tiles (split == 0) or 128 x 128 tiles with the K range in `split` parts.
+struct LoraTiling {
+  int split;
+  int tiles;  // 128 x 128 tiles of all jobs
+  size_t part_floats() const { return split > 1 ? (size_t)tiles * split * ST2 * ST2 : 0; }
+};
+// M and K steps of the n jobs over N columns.
+// The estimate, in us, was fitted to both paths over 200 to 8192 rows and in / out sizes of 896 to 44032 (168
+// products; the choice is within 2 % of the best measured one on average):
+//   256 x 256: 1 us per K step and round of work-groups while few CUs run, 1.45 at the power limit of a full chip;
+//   128 x 128: 0.58 us per K step alone on a CU, 1.0 for two side by side;
+//   a split adds the reduction's launch and a write and a read of 64 KiB per unit.
+// Both sides at some of them (us, 256 x 256 / best 128 x 128): 333 rows, 896 -> 896: 22 / 14 (no split); 333 rows,
+// 22016 -> 2048: 331 / 66 (split 8); 2531 rows, 11008 -> 2048: 182 / 132; 8192 rows, 2048 -> 2048: 61 / 72;
+// 2531 rows, 2048 -> 22016: 209 / 235.
+static LoraTiling lora_tiling(const int64_t* M, const int64_t* ksteps, int n, int64_t N) {
+  const int64_t cus = num_cus();
+  const int64_t nt2 = (N + TILE - 1) / TILE, nt1 = (N + ST2 - 1) / ST2;
+  int64_t tiles2 = 0, tiles1 = 0, k = 0;
+  for (int i = 0; i < n; ++i) {
+    tiles2 += (M[i] + TILE - 1) / TILE * nt2;
+    tiles1 += (M[i] + ST2 - 1) / ST2 * nt1;
+    k = ksteps[i] > k ? ksteps[i] : k;
+  }
+  LoraTiling best{0, (int)tiles1};
+  const double fill = tiles2 < cus ? (double)tiles2 / (double)cus : 1.0;
+  double cost = 0.93 * (8.0 + (double)((tiles2 + cus - 1) / cus * k) * (1.0 + 0.45 * fill));
+  if (tiles1 > (1 << 24)) return best;
+  for (int split = 1; split <= 16 && split <= k; ++split) {
+    const double per_cu = (double)(tiles1 * split) / (double)cus;
+    const double full = (double)(tiles1 * split / (2 * cus)), rest = per_cu - 2.0 * full;
+    const double conc = full + (rest <= 0.0 ? 0.0 : rest <= 1.0 ? 0.58 : 0.58 + 0.42 * (rest - 1.0));
+    const double c = 8.0 + (double)((k + split - 1) / split) * conc +
+                     (split > 1 ? 5.0 + 0.3 * split + 0.02 * (double)(tiles1 * split) : 0.0);
+    if (c < cost) {
+      cost = c;
+      best.split = split;
+    }
+  }
+  return best;
+}
+// The tiling of a call with one job per projection (forward) or one job over all of them (input gradient).
+static LoraTiling lora_tiling_fwd(const artk_lora_proj_t* proj, int n, int64_t T, int64_t in) {
+  int64_t M[LORA_MAX_SEG], ks[LORA_MAX_SEG];
+  for (int i = 0; i < n; ++i) {
+    M[i] = proj[i].out;
+    ks[i] = in / BK;
+  }
+  return lora_tiling(M, ks, n, T);
+}
+static LoraTiling lora_tiling_bwd(const artk_lora_proj_t* proj, int n, int64_t T, int64_t in) {
+  int64_t ks = 0;
+  for (int i = 0; i < n; ++i) ks += proj[i].out / BK;
+  return lora_tiling(&in, &ks, 1, T);
+}
+
+// Runs the jobs of m (256-row tile numbering) as `t` says; part: t.part_floats() floats.
+static int32_t launch_lora_jobs(const LoraMultiParams& m, const LoraTiling& t, float* part, hipStream_t st) {
+  const int cus = num_cus();
   prof_begin(PROF_LORA_GEMM, st);
-  {
-    const int cus = num_cus();
-    const int n_tiles = p.MT * p.NT;
-    lora_gemm_kernel<<<(unsigned)(n_tiles < cus ? n_tiles : cus), nthreads<LORA_NI>(), 0, st>>>(p);
+  if (t.split == 0) {
+    if (m.n_jobs == 1 && m.job[0].nseg == 1) {
+      const LoraJob& j = m.job[0];
+      const LoraSeg& g = m.seg[j.seg0];
+      LoraGemmParams p;
+      p.P = g.P;
+      p.Q = g.Q;
+      p.Pe = g.Pe;
+      p.Qe = g.Qe;
+      p.bias = j.bias;
+      p.out = j.out;
+      p.M = j.M;
+      p.N = m.N;
+      p.K = g.K;
+      p.r = g.r;
+      p.RP = g.RP;
+      p.MT = j.MT;
+      p.NT = m.NT;
+      lora_gemm_kernel<<<(unsigned)(m.n_tiles < cus ? m.n_tiles : cus), nthreads<LORA_NI>(), 0, st>>>(p);
+    } else {
+      lora_multi_gemm_kernel<<<(unsigned)(m.n_tiles < cus ? m.n_tiles : cus), nthreads<LORA_NI>(), 0, st>>>(m);
+    }
+  } else {
+    LoraSmallParams p;
+    p.m = m;
+    p.part = part;
+    p.split = t.split;
+    p.m.NT = (int)((m.N + ST2 - 1) / ST2);
+    int tile = 0;
+    for (int i = 0; i < m.n_jobs; ++i) {
+      LoraJob& j = p.m.job[i];
+      j.MT = (int)((j.M + ST2 - 1) / ST2);
+      j.tile0 = tile;
+      tile += j.MT * p.m.NT;
+      p.ksteps[i] = 0;
+      for (int g = 0; g < j.nseg; ++g) p.ksteps[i] += (int)(m.seg[j.seg0 + g].K / BK);
+    }
+    lora_small_gemm_kernel<<<(unsigned)(tile * t.split), ST2_THREADS, 0, st>>>(p);
+    if (t.split > 1) {
+      ARTK_CHECK_LAUNCH();
+      lora_small_reduce_kernel<<<(unsigned)(tile * 4), 256, 0, st>>>(p);
+    }
   }
   prof_end(PROF_LORA_GEMM, st);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
+}
+
+static int32_t launch_lora_gemm(const void* P, const void* Q, const uint16_t* Pe, const uint16_t* Qe,
+                                const uint16_t* bias, void* out, int64_t M, int64_t N, int64_t K, int r,
+                                int RP, const LoraTiling& t, float* part, hipStream_t st) {
+  LoraMultiParams m;
+  m.N = N;
+  m.NT = (int)((N + TILE - 1) / TILE);
+  m.n_jobs = 1;
+  m.seg[0] = LoraSeg{P, Q, Pe, Qe, K, r, RP};
+  m.job[0] = LoraJob{(uint16_t*)out, bias, M, (int)((M + TILE - 1) / TILE), 0, 0, 1};
+  m.n_tiles = m.job[0].MT * m.NT;
+  return launch_lora_jobs(m, t, part, st);
 }
 
 // out_f32 [T,R] = X Mt^T (unscaled), out_bf16 [T,RP] = scale * that, zero padded.
@@ -365,11 +579,15 @@ using namespace artk;
 
 extern "C" {
 
+static LoraTiling lora_tiling_one(int64_t T, int64_t K, int64_t M) {
+  const int64_t ks = K / BK;
+  return lora_tiling(&M, &ks, 1, T);
+}
+
 size_t artk_lora_linear_fwd_workspace_bytes(int64_t T, int64_t in, int64_t out, int32_t r) {
-  (void)in;
-  (void)out;
   Workspace ws(nullptr, 0);
   ws.take<uint16_t>((size_t)T * round16(r));  // s * x A^T, bf16 [T,RP]
+  ws.take<float>(lora_tiling_one(T, in, out).part_floats());
   return ws.used + 256;
 }
 
@@ -385,20 +603,23 @@ int32_t artk_lora_linear_fwd(const void* x, const void* W, const void* A, const 
   const int RP = round16(r);
   Workspace ws(workspace, workspace_bytes);
   uint16_t* xa16 = ws.take<uint16_t>((size_t)T * RP);
+  const LoraTiling tiling = lora_tiling_one(T, in, out);
+  float* part = ws.take<float>(tiling.part_floats());
   if (!ws.ok()) {
     set_error("workspace too small: need %zu bytes, got %zu", ws.used, workspace_bytes);
     return ARTK_ERR_WORKSPACE_TOO_SMALL;
   }
   hipStream_t st = (hipStream_t)stream;
   if ((rc = launch_rowdot(x, A, T, in, r, RP, scale, xa, xa16, st))) return rc;
-  return launch_lora_gemm(W, x, (const uint16_t*)B, xa16, (const uint16_t*)bias, y, out, T, in, r, RP, st);
+  return launch_lora_gemm(W, x, (const uint16_t*)B, xa16, (const uint16_t*)bias, y, out, T, in, r, RP, tiling, part, st);
 }
 
 // Scratch of the backward, carved in the same order by the size query and the call.
 struct LoraBwdScratch {
   uint16_t *Bt, *At, *gb16;
-  float *gb, *rowp_g, *colp_g, *colp_x, *dummy;
+  float *gb, *rowp_g, *colp_g, *colp_x, *dummy, *part;
   StatsGeom gg, gx;
+  LoraTiling tiling;  // of the input gradient
 };
 static void carve_lora_bwd(Workspace& ws, int64_t T, int64_t in, int64_t out, int r, LoraBwdScratch& c) {
   const int RP = round16(r);
@@ -412,6 +633,8 @@ static void carve_lora_bwd(Workspace& ws, int64_t T, int64_t in, int64_t out, in
   c.colp_g = ws.take<float>((size_t)c.gg.n_slabs * out * r);
   c.colp_x = ws.take<float>((size_t)c.gx.n_slabs * in * r);
   c.dummy = ws.take<float>(1024);
+  c.tiling = lora_tiling_one(T, out, in);
+  c.part = ws.take<float>(c.tiling.part_floats());
 }
 
 size_t artk_lora_linear_bwd_workspace_bytes(int64_t T, int64_t in, int64_t out, int32_t r) {
@@ -449,7 +672,7 @@ int32_t artk_lora_linear_bwd(const void* g, const void* x, const void* W_t, cons
     if ((rc = launch_stats_reduce(ja, jb, r, st))) return rc;
   }
   // dx = g W + (s g B) A
-  if ((rc = launch_lora_gemm(W_t, g, c.At, c.gb16, nullptr, dx, in, T, out, r, RP, st))) return rc;
+  if ((rc = launch_lora_gemm(W_t, g, c.At, c.gb16, nullptr, dx, in, T, out, r, RP, c.tiling, c.part, st))) return rc;
   // one pass over x: dA [r,in] = s (g B)^T x
   if ((rc = launch_stats(x, T, in, nullptr, c.gb, r, c.gx, nullptr, c.colp_x, c.dummy, st))) return rc;
   {
@@ -488,21 +711,12 @@ static int32_t check_multi(const artk_lora_proj_t* proj, int32_t n, int64_t T, i
   return ARTK_OK;
 }
 
-static int32_t launch_lora_multi(const LoraMultiParams& p, hipStream_t st) {
-  prof_begin(PROF_LORA_GEMM, st);
-  const int cus = num_cus();
-  lora_multi_gemm_kernel<<<(unsigned)(p.n_tiles < cus ? p.n_tiles : cus), nthreads<LORA_NI>(), 0, st>>>(p);
-  prof_end(PROF_LORA_GEMM, st);
-  ARTK_CHECK_LAUNCH();
-  return ARTK_OK;
-}
-
 size_t artk_lora_linear_multi_fwd_workspace_bytes(int64_t T, int64_t in, const artk_lora_proj_t* proj,
                                                   int32_t n) {
-  (void)in;
+  if (proj == nullptr || n < 1 || n > ARTK_LORA_MULTI_MAX) return 256;
   Workspace ws(nullptr, 0);
-  for (int i = 0; proj != nullptr && i < n && i < ARTK_LORA_MULTI_MAX; ++i)
-    ws.take<uint16_t>((size_t)T * round16(proj[i].r));
+  for (int i = 0; i < n; ++i) ws.take<uint16_t>((size_t)T * round16(proj[i].r));
+  ws.take<float>(lora_tiling_fwd(proj, n, T, in).part_floats());
   return ws.used + 256;
 }
 
@@ -515,6 +729,8 @@ int32_t artk_lora_linear_multi_fwd(const void* x, const artk_lora_proj_t* proj, 
   Workspace ws(workspace, workspace_bytes);
   uint16_t* xa16[ARTK_LORA_MULTI_MAX];
   for (int i = 0; i < n; ++i) xa16[i] = ws.take<uint16_t>((size_t)T * round16(proj[i].r));
+  const LoraTiling tiling = lora_tiling_fwd(proj, n, T, in);
+  float* part = ws.take<float>(tiling.part_floats());
   if (!ws.ok()) {
     set_error("workspace too small: need %zu bytes, got %zu", ws.used, workspace_bytes);
     return ARTK_ERR_WORKSPACE_TOO_SMALL;
@@ -547,7 +763,7 @@ int32_t artk_lora_linear_multi_fwd(const void* x, const artk_lora_proj_t* proj, 
   dim3 grid((unsigned)((T + 15) / 16), (unsigned)y);
   rowdot16_multi_kernel<<<grid, 256, 0, st>>>((const uint16_t*)x, m, T, in, scale);
   ARTK_CHECK_LAUNCH();
-  return launch_lora_multi(p, st);
+  return launch_lora_jobs(p, tiling, part, st);
 }
 
 struct LoraMultiBwdScratch {
@@ -555,7 +771,9 @@ struct LoraMultiBwdScratch {
   float* gb_cat;   // [T, r_total]: g_i B_i side by side, the Y of the pass over x
   float* colp_x;   // [n_slabs][in][r_total]
   float* dummy;
+  float* part;
   StatsGeom gx;
+  LoraTiling tiling;
   int r_total;
 };
 static void carve_lora_multi_bwd(Workspace& ws, int64_t T, int64_t in, const artk_lora_proj_t* proj, int n,
@@ -577,6 +795,8 @@ static void carve_lora_multi_bwd(Workspace& ws, int64_t T, int64_t in, const art
   c.gb_cat = ws.take<float>((size_t)T * c.r_total);
   c.colp_x = ws.take<float>((size_t)c.gx.n_slabs * in * c.r_total);
   c.dummy = ws.take<float>(1024);
+  c.tiling = lora_tiling_bwd(proj, n, T, in);
+  c.part = ws.take<float>(c.tiling.part_floats());
 }
 
 size_t artk_lora_linear_multi_bwd_workspace_bytes(int64_t T, int64_t in, const artk_lora_proj_t* proj,
@@ -656,7 +876,7 @@ int32_t artk_lora_linear_multi_bwd(const void* x, const artk_lora_proj_t* proj, 
   }
   if ((rc = launch_stats_reduce_multi(rm, st))) return rc;
   // dx = sum_i ( g_i W_i + (s g_i B_i) A_i ): one launch, the projections as K segments
-  if ((rc = launch_lora_multi(p, st))) return rc;
+  if ((rc = launch_lora_jobs(p, c.tiling, c.part, st))) return rc;
   // one pass over x: [dA_0; dA_1; ...] = s [g_0 B_0 | g_1 B_1 | ...]^T x
   if ((rc = launch_stats(x, T, in, nullptr, c.gb_cat, c.r_total, c.gx, nullptr, c.colp_x, c.dummy, st))) return rc;
   StatsReduceJob none{nullptr, 0, 0, 0.f, nullptr, 0, nullptr, 0, 0.f};

@@ -280,3 +280,36 @@ def test_concatenated_projections_config2_full_size(artk_lib, gpu, T, n_in, outs
     xa0 = x.double() @ A.double().t()
     dB_full = scale * (up.double().t() @ xa0)
     assert rel_l2(dB.cpu(), dB_full) <= TOL
+
+
+@pytest.mark.parametrize("T,n_in,outs,r", [
+    (1, 64, (64,), 8),                  # one row, one K step
+    (129, 320, (192, 64), 16),          # one row and half a tile past an edge, two jobs
+    (130, 4864, (896,), 8),             # long K, few tiles: split in the forward
+    (200, 128, (4864, 64), 24),         # input gradient over two segments of very different length, split
+    (200, 64, (64, 8192, 128), 8),      # split boundaries inside the middle segment
+])
+def test_small_products(artk_lib, gpu, T, n_in, outs, r):
+    """Sizes that run on 128 x 128 tiles with the K range split: forward with bias and backward of all
+    projections against fp32 (1e-2: bf16 outputs and bf16 low-rank products, as for the large tiles)."""
+    print("small products", T, n_in, outs, r, flush=True)
+    g = torch.Generator().manual_seed(T + n_in)
+    rnd = lambda *s, std=1.0: (std * torch.randn(*s, generator=g)).to(torch.bfloat16)
+    x = rnd(T, n_in)
+    W, A, B = ([rnd(o, n_in, std=0.02) for o in outs], [rnd(r, n_in, std=n_in ** -0.5) for _ in outs],
+               [rnd(o, r, std=0.05) for o in outs])
+    bias, up = [rnd(o) for o in outs], [rnd(T, o) for o in outs]
+    dev = lambda ts: [t.to(gpu) for t in ts]
+    ys, xas = ops.lora_linear_multi_fwd(x.to(gpu), dev(W), dev(A), dev(B), 0.5, dev(bias))
+    dx, dAs, dBs = ops.lora_linear_multi_bwd(dev(up), x.to(gpu), [ops.transpose(w.to(gpu)) for w in W], dev(A), dev(B),
+                                             xas, 0.5)
+    rel = lambda a, b: ((a.float().cpu() - b).norm() / b.norm()).item()
+    xf, dx0 = x.float(), 0
+    for i in range(len(outs)):
+        Wf, Af, Bf, gf = (t.float() for t in (W[i], A[i], B[i], up[i]))
+        assert rel(ys[i], xf @ Wf.T + bias[i].float() + 0.5 * (xf @ Af.T) @ Bf.T) <= 1e-2
+        assert rel(dAs[i], 0.5 * (gf @ Bf).T @ xf) <= 1e-2 and rel(dBs[i], 0.5 * gf.T @ (xf @ Af.T)) <= 1e-2
+        dx0 = dx0 + gf @ Wf + 0.5 * (gf @ Bf) @ Af
+        y1, _ = ops.lora_linear_fwd(x.to(gpu), W[i].to(gpu), A[i].to(gpu), B[i].to(gpu), 0.5, bias[i].to(gpu))
+        assert rel(y1, ys[i].float().cpu()) <= 4e-3   # one rounding to bf16; the K range may be split elsewhere
+    assert rel(dx, dx0) <= 1e-2
