@@ -76,7 +76,7 @@ struct FwdParams {
   int64_t S, V, H;
   int shift;
   float2* part;         // [2*VT][Tc]  (max, sumexp)
-  float* sel;           // [Tc]        selected logit (pre-filled with NaN)
+  float* sel;           // [Tc]        selected logit (written for rows whose target is a vocabulary id)
   uint16_t* stash;      // [Tc,V] bf16 or nullptr: exp(logit - ref[row]) of the rows the backward reads
   const float* ref;     // [Tc] reference logit of each row (stash only): the target's own logit
   const uint8_t* need;  // [Tc] rows of the stash that the backward will read; nullptr: all
@@ -340,15 +340,185 @@ __global__ __launch_bounds__(nthreads<FWD_NI>()) void lmhead_fwd_kernel(FwdParam
   }
 }
 
+// Which rows of a chunk the backward will read: those whose upstream gradient is not zero (grad, by chunk row),
+// or, in the fused step, the positions that can have a non-zero loss coefficient: the (shifted) mask is set and
+// weight and advantage are non-zero (the advantage does not matter with a KL term).  Neither given: all rows.
+struct NeedSource {
+  const float* grad;
+  const uint8_t* mask;
+  const float *weights, *adv, *ref_lp;
+  __device__ __forceinline__ bool position(int64_t t, int64_t S, int shift) const {
+    int64_t src;
+    return shifted_index(t, S, shift, src) && mask[src] != 0 && weights[src] != 0.f &&
+           (adv[src] != 0.f || ref_lp != nullptr);
+  }
+};
+
+// Number of positions of the batch whose shifted mask is set: every set byte counts but the first of a row.
+// All threads of the work-group call it (16 bytes per load); the result is valid in thread 0.
+__device__ int count_shifted_mask(const uint8_t* mask, int64_t T, int64_t S, int shift, int* red) {
+  int c = 0;
+  const bool vec = ((uintptr_t)mask & 15) == 0;
+  for (int64_t t = (int64_t)threadIdx.x * 16; t < T; t += (int64_t)blockDim.x * 16) {
+    if (vec && t + 16 <= T) {
+      const uint4 v = *(const uint4*)(mask + t);
+      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) c += (w[k] >> (8 * b) & 0xffu) != 0u;
+    } else {
+      for (int64_t i = t; i < t + 16 && i < T; ++i) c += mask[i] != 0;
+    }
+    if (shift) {
+      const int64_t first = (t + S - 1) / S * S;  // row starts among these 16
+      for (int64_t i = first; i < t + 16 && i < T; i += S) c -= mask[i] != 0;
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = c;
+  __syncthreads();
+  int s = 0;
+  if (threadIdx.x == 0)
+    for (int i = 0; i < (int)(blockDim.x >> 6); ++i) s += red[i];
+  return s;
+}
+
+// Positions of the whole batch that can have a non-zero loss coefficient (see NeedSource), ascending, and
+// their number; also the mask count, and the counter of dropped rows set to zero.  One block.
+__global__ __launch_bounds__(1024) void compact_eval_kernel(NeedSource need, int64_t T, int64_t S, int shift,
+                                                            int* __restrict__ eval_idx, int* __restrict__ n_eval,
+                                                            int* __restrict__ count, float* __restrict__ dropped) {
+  __shared__ int wave_tot[16], red[16];
+  const int64_t per = (T + 1023) / 1024;
+  const int64_t r0 = threadIdx.x * per;
+  auto wanted = [&](int64_t t) { return need.position(t, S, shift); };
+  const int masked = count_shifted_mask(need.mask, T, S, shift, red);
+  if (threadIdx.x == 0) {
+    *count = masked;
+    *dropped = 0.f;
+  }
+  int cnt = 0;
+  for (int64_t i = 0; i < per; ++i)
+    if (r0 + i < T && wanted(r0 + i)) ++cnt;
+  int incl = cnt;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    int v = __shfl_up(incl, o, 64);
+    if ((threadIdx.x & 63) >= o) incl += v;
+  }
+  if ((threadIdx.x & 63) == 63) wave_tot[threadIdx.x >> 6] = incl;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int run = 0;
+    for (int w = 0; w < 16; ++w) {
+      int v = wave_tot[w];
+      wave_tot[w] = run;
+      run += v;
+    }
+    *n_eval = run;
+  }
+  __syncthreads();
+  int at = wave_tot[threadIdx.x >> 6] + incl - cnt;
+  for (int64_t i = 0; i < per; ++i)
+    if (r0 + i < T && wanted(r0 + i)) eval_idx[at++] = (int)(r0 + i);
+}
+
+// What positions that are not evaluated keep: logprob NaN, zero loss terms, a zero d_hidden row.
+__global__ __launch_bounds__(256) void skip_fill_kernel(float* __restrict__ logprob, float* __restrict__ pl,
+                                                        float* __restrict__ kl, int64_t T, uint4* __restrict__ d_hidden,
+                                                        int64_t n16) {
+  const int64_t step = (int64_t)gridDim.x * 256;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += step) d_hidden[i] = make_uint4(0, 0, 0, 0);
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < T; i += step) {
+    logprob[i] = NAN;
+    pl[i] = 0.f;
+    kl[i] = 0.f;
+  }
+}
+
+// ----------------------------------------------------------------------------
+// Loss kernels
+// ----------------------------------------------------------------------------
+
+// *count = number of positions whose (shifted) assistant mask is set.  One block.
+__global__ __launch_bounds__(1024) void mask_count_kernel(const uint8_t* __restrict__ mask,
+                                                          int64_t T, int64_t S, int shift,
+                                                          int* __restrict__ count) {
+  __shared__ int red[16];
+  const int c = count_shifted_mask(mask, T, S, shift, red);
+  if (threadIdx.x == 0) *count = c;
+}
+
+struct LossParams {
+  const float* new_lp;   // [T] by position (whole batch)
+  const float* old_lp;   // [T] whole batch (frame given by shift)
+  const float* adv;      // [T]
+  const uint8_t* mask;   // [T]
+  const float* weights;  // [T]
+  const float* ref_lp;   // [T] by position, or nullptr
+  const int* count;      // mask count of the whole batch
+  ChunkRows rows;
+  int64_t S;
+  int shift;
+  float clip_lo, clip_hi, beta;
+  float* pl_tok;         // [T] by position: weighted policy-loss term
+  float* kl_tok;         // [T] by position: weighted KL term
+  float* coef;           // [rows.cap] by chunk row: d loss / d new_lp, or nullptr
+};
+
+// Loss terms and gradient coefficient of chunk row i, whose logprob is nw.
+__device__ __forceinline__ void grpo_loss_row(const LossParams& p, int i, float nw) {
+  const int64_t t = p.rows.token(i);
+  int64_t src;
+  const bool in = shifted_index(t, p.S, p.shift, src);
+  float oldv = in ? p.old_lp[src] : 0.f;
+  const float adv = in ? p.adv[src] : 0.f;
+  const float w = in ? p.weights[src] : 0.f;
+  const float m = (in && p.mask[src] != 0) ? 1.f : 0.f;
+  if (isnan(oldv)) oldv = nw;  // missing old logprob: sampled under the current policy
+  const float ratio = expf(nw - oldv);
+  const float a = ratio * adv;
+  const float clipped = fminf(fmaxf(ratio, p.clip_lo), p.clip_hi);
+  const float b = clipped * adv;
+  const float pl = -fminf(a, b);
+  // Gradient of -min(a, b) w.r.t. new_lp. Inside the clip range a and b are the
+  // same number and both pass the gradient; outside only a does, when it is the min.
+  const bool inside = ratio >= p.clip_lo && ratio <= p.clip_hi;
+  float g = (inside || a < b) ? -a : 0.f;
+  float kl = 0.f;
+  if (p.ref_lp != nullptr) {
+    const float d = p.ref_lp[t] - nw;
+    const float e = expf(d);
+    kl = e - d - 1.f;
+    g += p.beta * (1.f - e);
+  }
+  const float denom = (float)(*p.count) + 1e-6f;
+  const float wm = w * m;
+  p.pl_tok[t] = pl * wm;
+  p.kl_tok[t] = kl * wm;
+  if (p.coef) p.coef[i] = (wm != 0.f) ? g * wm / denom : 0.f;
+}
+
+__global__ __launch_bounds__(256) void grpo_loss_tok_kernel(LossParams p) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= p.rows.n()) return;
+  grpo_loss_row(p, (int)i, p.new_lp[p.rows.token((int)i)]);
+}
+
 // K2: merge the per-tile (max, sumexp) partials of each position.  A block
 // handles 16 positions; 16 threads per position each merge a strided share of
 // the partials online, then the 16 shares are merged through LDS.
-// logprob is indexed by position (whole batch), lse by chunk row.
+// logprob is indexed by position (whole batch), lse by chunk row.  A target that is no vocabulary id gives NaN.
+// LOSS: the loss terms of the row follow at once (the fused step; a launch of its own otherwise).
+template <bool LOSS>
 __global__ __launch_bounds__(256) void lse_finalize_kernel(const float2* __restrict__ part,
                                                            int nparts, int64_t Tc, ChunkRows rows,
                                                            const float* __restrict__ sel,
-                                                           float* __restrict__ logprob,
-                                                           float* __restrict__ lse) {
+                                                           const int64_t* __restrict__ ids, int64_t S, int shift,
+                                                           int64_t V, float* __restrict__ logprob,
+                                                           float* __restrict__ lse, LossParams loss) {
   __shared__ float2 red[16][17];
   const int tl = threadIdx.x & 15, sl = threadIdx.x >> 4;
   const int64_t t = (int64_t)blockIdx.x * 16 + tl;
@@ -387,171 +557,21 @@ __global__ __launch_bounds__(256) void lse_finalize_kernel(const float2* __restr
     }
     const float z = M + logf(L);
     lse[t] = z;
-    if (logprob) logprob[rows.token((int)t)] = sel[t] - z;
-  }
-}
-
-// need[i] = 1 when position t0+i can have a non-zero loss coefficient: its
-// (shifted) mask is set and weight and advantage are non-zero.
-__global__ __launch_bounds__(256) void need_from_inputs_kernel(const uint8_t* __restrict__ mask,
-                                                               const float* __restrict__ weights,
-                                                               const float* __restrict__ adv,
-                                                               const float* __restrict__ ref_lp,
-                                                               int64_t t0, int64_t n, int64_t S,
-                                                               int shift, uint8_t* __restrict__ need) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  int64_t src;
-  uint8_t v = 0;
-  if (shifted_index(t0 + i, S, shift, src))
-    v = mask[src] != 0 && weights[src] != 0.f && (adv[src] != 0.f || ref_lp != nullptr);
-  need[i] = v;
-}
-
-__global__ __launch_bounds__(256) void need_from_grad_kernel(const float* __restrict__ g, int64_t n,
-                                                             uint8_t* __restrict__ need) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) need[i] = g[i] != 0.f;
-}
-
-// Positions of the whole batch that can have a non-zero loss coefficient (same
-// test as need_from_inputs_kernel), ascending, and their number.  One block.
-__global__ __launch_bounds__(1024) void compact_eval_kernel(const uint8_t* __restrict__ mask,
-                                                            const float* __restrict__ weights,
-                                                            const float* __restrict__ adv,
-                                                            const float* __restrict__ ref_lp, int64_t T,
-                                                            int64_t S, int shift,
-                                                            int* __restrict__ eval_idx,
-                                                            int* __restrict__ n_eval) {
-  __shared__ int wave_tot[16];
-  const int64_t per = (T + 1023) / 1024;
-  const int64_t r0 = threadIdx.x * per;
-  auto wanted = [&](int64_t t) {
-    int64_t src;
-    return shifted_index(t, S, shift, src) && mask[src] != 0 && weights[src] != 0.f &&
-           (adv[src] != 0.f || ref_lp != nullptr);
-  };
-  int cnt = 0;
-  for (int64_t i = 0; i < per; ++i)
-    if (r0 + i < T && wanted(r0 + i)) ++cnt;
-  int incl = cnt;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    int v = __shfl_up(incl, o, 64);
-    if ((threadIdx.x & 63) >= o) incl += v;
-  }
-  if ((threadIdx.x & 63) == 63) wave_tot[threadIdx.x >> 6] = incl;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int run = 0;
-    for (int w = 0; w < 16; ++w) {
-      int v = wave_tot[w];
-      wave_tot[w] = run;
-      run += v;
+    if (logprob) {
+      const int64_t y = target_id(ids, rows.token((int)t), S, shift);
+      const float lp = y >= 0 && y < V ? sel[t] - z : NAN;
+      logprob[rows.token((int)t)] = lp;
+      if (LOSS) grpo_loss_row(loss, (int)t, lp);
     }
-    *n_eval = run;
-  }
-  __syncthreads();
-  int at = wave_tot[threadIdx.x >> 6] + incl - cnt;
-  for (int64_t i = 0; i < per; ++i)
-    if (r0 + i < T && wanted(r0 + i)) eval_idx[at++] = (int)(r0 + i);
-}
-
-__global__ void fill_f32_kernel(float* p, int64_t n, float v) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-
-// ----------------------------------------------------------------------------
-// Loss kernels
-// ----------------------------------------------------------------------------
-
-// count[0] = number of positions whose (shifted) assistant mask is set; count[1] = 0. One block.
-__global__ __launch_bounds__(1024) void mask_count_kernel(const uint8_t* __restrict__ mask,
-                                                          int64_t T, int64_t S, int shift,
-                                                          int* __restrict__ count) {
-  __shared__ int red[16];
-  int c = 0;
-  for (int64_t t = threadIdx.x; t < T; t += 1024) {
-    int64_t src;
-    if (shifted_index(t, S, shift, src)) c += mask[src] != 0;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = c;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int s = 0;
-    for (int i = 0; i < 16; ++i) s += red[i];
-    count[0] = s;
-    count[1] = 0;  // rows dropped by splitk_reduce_kernel (fused step only)
   }
 }
 
-struct LossParams {
-  const float* new_lp;   // [T] by position (whole batch)
-  const float* old_lp;   // [T] whole batch (frame given by shift)
-  const float* adv;      // [T]
-  const uint8_t* mask;   // [T]
-  const float* weights;  // [T]
-  const float* ref_lp;   // [T] by position, or nullptr
-  const int* count;      // mask count of the whole batch
-  ChunkRows rows;
-  int64_t S;
-  int shift;
-  float clip_lo, clip_hi, beta;
-  float* pl_tok;         // [T] by position: weighted policy-loss term
-  float* kl_tok;         // [T] by position: weighted KL term
-  float* coef;           // [rows.cap] by chunk row: d loss / d new_lp, or nullptr
-};
-
-__global__ __launch_bounds__(256) void grpo_loss_tok_kernel(LossParams p) {
-  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= p.rows.n()) return;
-  const int64_t t = p.rows.token((int)i);
-  int64_t src;
-  const bool in = shifted_index(t, p.S, p.shift, src);
-  float oldv = in ? p.old_lp[src] : 0.f;
-  const float adv = in ? p.adv[src] : 0.f;
-  const float w = in ? p.weights[src] : 0.f;
-  const float m = (in && p.mask[src] != 0) ? 1.f : 0.f;
-  const float nw = p.new_lp[t];
-  if (isnan(oldv)) oldv = nw;  // missing old logprob: sampled under the current policy
-  const float ratio = expf(nw - oldv);
-  const float a = ratio * adv;
-  const float clipped = fminf(fmaxf(ratio, p.clip_lo), p.clip_hi);
-  const float b = clipped * adv;
-  const float pl = -fminf(a, b);
-  // Gradient of -min(a, b) w.r.t. new_lp. Inside the clip range a and b are the
-  // same number and both pass the gradient; outside only a does, when it is the min.
-  const bool inside = ratio >= p.clip_lo && ratio <= p.clip_hi;
-  float g = (inside || a < b) ? -a : 0.f;
-  float kl = 0.f;
-  if (p.ref_lp != nullptr) {
-    const float d = p.ref_lp[t] - nw;
-    const float e = expf(d);
-    kl = e - d - 1.f;
-    g += p.beta * (1.f - e);
-  }
-  const float denom = (float)(*p.count) + 1e-6f;
-  const float wm = w * m;
-  p.pl_tok[t] = pl * wm;
-  p.kl_tok[t] = kl * wm;
-  if (p.coef) p.coef[i] = (wm != 0.f) ? g * wm / denom : 0.f;
-}
-
-// scalars = {loss, mean_policy_loss, mean_kl, mask_count} and, with `with_dropped` (the fused
-// step), scalars[4] = count[1], the rows whose gradient was dropped.  One block; fixed
+// scalars[0..3] = {loss, mean_policy_loss, mean_kl, mask_count}.  All threads of one work-group; fixed
 // summation order, so the result is bit-reproducible run to run.
-__global__ __launch_bounds__(1024) void grpo_loss_reduce_kernel(const float* __restrict__ pl_tok,
-                                                                const float* __restrict__ kl_tok,
-                                                                int64_t T,
-                                                                const int* __restrict__ count,
-                                                                float beta, int with_dropped,
-                                                                float* __restrict__ scalars) {
-  __shared__ double red[2][16];
+__device__ void grpo_loss_reduce(const float* pl_tok, const float* kl_tok, int64_t T, const int* count, float beta,
+                                 float* scalars, double (*red)[16]) {
   double a = 0.0, b = 0.0;
-  for (int64_t t = threadIdx.x; t < T; t += 1024) {
+  for (int64_t t = threadIdx.x; t < T; t += blockDim.x) {
     a += (double)pl_tok[t];
     b += (double)kl_tok[t];
   }
@@ -564,7 +584,7 @@ __global__ __launch_bounds__(1024) void grpo_loss_reduce_kernel(const float* __r
   __syncthreads();
   if (threadIdx.x == 0) {
     double sa = 0.0, sb = 0.0;
-    for (int i = 0; i < 16; ++i) {
+    for (int i = 0; i < (int)(blockDim.x >> 6); ++i) {
       sa += red[0][i];
       sb += red[1][i];
     }
@@ -575,8 +595,21 @@ __global__ __launch_bounds__(1024) void grpo_loss_reduce_kernel(const float* __r
     scalars[1] = mpl;
     scalars[2] = mkl;
     scalars[3] = (float)(*count);
-    if (with_dropped) scalars[4] = (float)count[1];
   }
+}
+__global__ __launch_bounds__(1024) void grpo_loss_reduce_kernel(const float* __restrict__ pl_tok,
+                                                                const float* __restrict__ kl_tok, int64_t T,
+                                                                const int* __restrict__ count, float beta,
+                                                                float* __restrict__ scalars) {
+  __shared__ double red[2][16];
+  grpo_loss_reduce(pl_tok, kl_tok, T, count, beta, scalars, red);
+}
+
+// Most K splits of the d_hidden GEMM that are considered: 16, or as many as give every CU one work-group when
+// there are few tiles.  (184 active rows at a hidden size of 896 are 4 tiles: 16 splits left 192 CUs idle, 221 us.)
+__host__ __device__ static inline int max_splits(int tiles, int cus) {
+  const int fill = (cus + tiles - 1) / tiles;
+  return fill > 16 ? fill : 16;
 }
 
 // ----------------------------------------------------------------------------
@@ -638,7 +671,7 @@ __global__ __launch_bounds__(1024) void compact_rows_kernel(const float* __restr
     const int tiles = HT * tta;
     int best = 1;
     float best_eff = 0.f;
-    for (int ns = 1; ns <= 16 && tiles > 0; ++ns) {
+    for (int ns = 1; tiles > 0 && ns <= max_splits(tiles, num_cus); ++ns) {
       if (ns > 1 && (ksteps / ns < 32 || ns * tta * TILE > part_rows)) break;
       int blocks = tiles * ns;
       int rounds = (blocks + num_cus - 1) / num_cus;
@@ -667,22 +700,35 @@ __global__ __launch_bounds__(1024) void compact_rows_kernel(const float* __restr
 // pass of its own: d_hidden[t] = coef_t (W[y_t] - exp(ref_t - lse_t) sum_v e[t,v] W[v]),
 // the sum being the GEMM K4 and the rest the epilogue of K5.  (A stash of logits needed a
 // 2 x [Tc_active, V] read-modify-write between K2 and K4 to turn them into gradients.)
-// One wave per row.
+// One wave per row, which also decides whether the row is needed (need_out, when given).  With `count` the
+// work-group past the last row counts the batch's mask (first chunk of the fused step).
 __global__ __launch_bounds__(256) void target_ref_kernel(const uint16_t* __restrict__ hidden,
                                                          const uint16_t* __restrict__ W,
                                                          const int64_t* __restrict__ ids, ChunkRows rows,
-                                                         const uint8_t* __restrict__ need, int64_t S,
+                                                         NeedSource need, uint8_t* __restrict__ need_out, int64_t S,
                                                          int shift, int64_t V, int64_t H,
-                                                         float* __restrict__ ref) {
+                                                         float* __restrict__ ref, int64_t T, int* __restrict__ count,
+                                                         float* __restrict__ dropped) {
+  __shared__ int red[4];
+  if (count != nullptr && blockIdx.x == 0) {
+    const int c = count_shifted_mask(need.mask, T, S, shift, red);
+    if (threadIdx.x == 0) {
+      *count = c;
+      *dropped = 0.f;
+    }
+    return;
+  }
   const int lane = threadIdx.x & 63;
-  const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int r = (blockIdx.x - (count != nullptr ? 1 : 0)) * 4 + (threadIdx.x >> 6);
   if (r >= rows.n()) return;
   float s = 0.f;
-  const int64_t y = target_id(ids, rows.token(r), S, shift);
-  if ((need == nullptr || need[r] != 0) && y >= 0 && y < V) {
+  const int64_t t = rows.token(r);
+  const bool needed = need.grad ? need.grad[r] != 0.f : need.mask ? need.position(t, S, shift) : true;
+  const int64_t y = target_id(ids, t, S, shift);
+  if (needed && y >= 0 && y < V) {
     // `hidden` starts at the chunk's first row when the rows are dense, at position 0 when they
     // are gathered
-    const uint16_t* h = hidden + (int64_t)(rows.row_token ? rows.token(r) : r) * H;
+    const uint16_t* h = hidden + (int64_t)(rows.row_token ? t : r) * H;
     const uint16_t* w = W + y * H;
     for (int64_t k = lane * 8; k < H; k += 512) {
       const uint4 a = *(const uint4*)(h + k), b = *(const uint4*)(w + k);
@@ -696,7 +742,10 @@ __global__ __launch_bounds__(256) void target_ref_kernel(const uint16_t* __restr
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
   }
-  if (lane == 0) ref[r] = s;
+  if (lane == 0) {
+    ref[r] = s;
+    if (need_out) need_out[r] = needed;
+  }
 }
 
 // ----------------------------------------------------------------------------
@@ -767,7 +816,15 @@ constexpr float STASH_MAX_NATS = 80.f;
 // exponential and, times max |W|, every element of G, so up to the limit all of them are finite
 // in bf16 / fp32, and beyond it they may be inf or NaN.  Such a row gets a zero gradient (what
 // the reference would compute for it is cf * (W[y] - p W) with p ~ one-hot elsewhere: a finite
-// row; dropping it keeps the step finite) and is counted in *dropped (may be null).
+// row; dropping it keeps the step finite) and is counted in *dropped (may be null; a float, exact up to 2^24).
+// With `loss_scalars` (the last chunk of the fused step) work-group 0 adds up the batch's loss terms.
+struct LossReduce {
+  const float *pl, *kl;
+  int64_t T;
+  const int* count;
+  float beta;
+  float* scalars;
+};
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ partial,
                                                             const int* __restrict__ pos,
                                                             const int* __restrict__ sched,
@@ -778,8 +835,13 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
                                                             const int64_t* __restrict__ ids, int64_t S,
                                                             int shift, const uint16_t* __restrict__ W,
                                                             uint16_t* __restrict__ out,
-                                                            int* __restrict__ dropped) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+                                                            float* __restrict__ dropped, LossReduce loss) {
+  __shared__ double red[2][16];
+  if (loss.scalars != nullptr && blockIdx.x == 0) {
+    grpo_loss_reduce(loss.pl, loss.kl, loss.T, loss.count, loss.beta, loss.scalars, red);
+    return;
+  }
+  const int64_t i = (int64_t)(blockIdx.x - (loss.scalars != nullptr ? 1 : 0)) * 256 + threadIdx.x;
   const int64_t h4 = H / 4;
   if (i >= (int64_t)rows.n() * h4) return;
   const int64_t r = i / h4, c = i - r * h4;
@@ -787,7 +849,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   floatx4 s = {0.f, 0.f, 0.f, 0.f};
   const bool over = pr >= 0 && !(lse[r] - ref[r] <= STASH_MAX_NATS);  // also true for NaN
   if (over) {
-    if (c == 0 && dropped != nullptr) atomicAdd(dropped, 1);
+    if (c == 0 && dropped != nullptr) atomicAdd(dropped, 1.f);
   } else if (pr >= 0) {
     const int nsplit = sched[2];
     const int64_t rows_per_split = (int64_t)sched[1] * TILE;
@@ -811,6 +873,23 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 #pragma unroll
   for (int e = 0; e < 4; ++e) o[e] = (__bf16)s[e];
   ((bf16x4*)out)[rows.token((int)r) * h4 + c] = o;
+}
+
+// out = in * *factor (the upstream gradient of the loss times the d_hidden of the fused step), 4 B per element,
+// HBM-bound: 117 MB at 16384 x 3584 took 194 us as a torch element-wise product with a 0-dim tensor, 50 us here.
+__global__ __launch_bounds__(256) void scale_bf16_kernel(const uint4* __restrict__ in, const float* __restrict__ factor,
+                                                         uint4* __restrict__ out, int64_t n16) {
+  const float f = *factor;
+  const int64_t step = (int64_t)gridDim.x * 256;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += step) {
+    const uint4 v = in[i];
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      o[k] = pack_bf16x2(__uint_as_float(w[k] << 16) * f, __uint_as_float(w[k] & 0xffff0000u) * f);
+    out[i] = make_uint4(o[0], o[1], o[2], o[3]);
+  }
 }
 
 // ----------------------------------------------------------------------------
@@ -931,7 +1010,7 @@ static int choose_nsplit(int tiles, int ksteps) {
   const int cus = num_cus();
   int best = 1;
   double best_eff = 0.0;
-  for (int ns = 1; ns <= 16; ++ns) {
+  for (int ns = 1; ns <= max_splits(tiles, cus); ++ns) {
     if (ksteps / ns < 32 && ns > 1) break;
     int blocks = tiles * ns;
     int rounds = (blocks + cus - 1) / cus;
@@ -976,18 +1055,28 @@ static ChunkRows dense_rows(int64_t t0, int64_t n) {
   return r;
 }
 
-// Launch K0 (when the chunk is stashed), K1 (+ NaN pre-fill of sel) and K2 for the rows of one chunk.  `logprob`
-// (may be null) is the whole batch's array; `lse_chunk` is indexed by chunk row.
+// Launch K0 (when the chunk is stashed), K1 and K2 for the rows of one chunk.  `logprob` (may be null) is the
+// whole batch's array; `lse_chunk` is indexed by chunk row.  `need_out`: flags of the rows the backward will read
+// (null: all of them); loss (with `count` for the first chunk): see target_ref_kernel and lse_finalize_kernel.
+struct FwdFused {
+  LossParams loss;
+  int64_t T;
+  int* count;      // nullptr: already counted
+  float* dropped;
+};
 static int32_t launch_fwd_chunk(const void* hidden, const void* lm_head, const int64_t* ids,
                                 int shift, const ChunkRows& rows, int64_t S, int64_t V, int64_t H,
-                                float2* part, float* sel, uint16_t* stash, float* ref, const uint8_t* need,
-                                float* logprob, float* lse_chunk, hipStream_t st) {
+                                float2* part, float* sel, uint16_t* stash, float* ref, const NeedSource& source,
+                                uint8_t* need, float* logprob, float* lse_chunk, const FwdFused* fused,
+                                hipStream_t st) {
   const int64_t Tc = rows.cap;
   if (stash) {
+    int* count = fused ? fused->count : nullptr;
     prof_begin(PROF_TARGET_REF, st);
-    target_ref_kernel<<<(unsigned)((Tc + 3) / 4), 256, 0, st>>>(
+    target_ref_kernel<<<(unsigned)((Tc + 3) / 4 + (count ? 1 : 0)), 256, 0, st>>>(
         (const uint16_t*)(rows.row_token ? hidden : (const void*)((const char*)hidden + rows.t0 * H * 2)),
-        (const uint16_t*)lm_head, ids, rows, need, S, shift, V, H, ref);
+        (const uint16_t*)lm_head, ids, rows, source, need, S, shift, V, H, ref, fused ? fused->T : 0, count,
+        fused ? fused->dropped : nullptr);
     prof_end(PROF_TARGET_REF, st);
     ARTK_CHECK_LAUNCH();
   }
@@ -1008,8 +1097,6 @@ static int32_t launch_fwd_chunk(const void* hidden, const void* lm_head, const i
   p.need = need;
   p.VT = (int)((V + TILE - 1) / TILE);
   p.TT = (int)((Tc + TILE - 1) / TILE);
-  fill_f32_kernel<<<(unsigned)((Tc + 255) / 256), 256, 0, st>>>(sel, Tc, NAN);
-  ARTK_CHECK_LAUNCH();
   const int n_tiles = p.VT * p.TT;
   const unsigned grid = (unsigned)(n_tiles < num_cus() ? n_tiles : num_cus());
   prof_begin(PROF_LMHEAD_FWD, st);
@@ -1024,8 +1111,13 @@ static int32_t launch_fwd_chunk(const void* hidden, const void* lm_head, const i
     lmhead_fwd_kernel<false, false><<<grid, nthreads<FWD_NI>(), 0, st>>>(p);
   prof_end(PROF_LMHEAD_FWD, st);
   ARTK_CHECK_LAUNCH();
-  lse_finalize_kernel<<<(unsigned)((Tc + 15) / 16), 256, 0, st>>>(part, 2 * p.VT, Tc, rows, sel, logprob,
-                                                                    lse_chunk);
+  const unsigned fin = (unsigned)((Tc + 15) / 16);
+  if (fused)
+    lse_finalize_kernel<true><<<fin, 256, 0, st>>>(part, 2 * p.VT, Tc, rows, sel, ids, S, shift, V, logprob, lse_chunk,
+                                                   fused->loss);
+  else
+    lse_finalize_kernel<false><<<fin, 256, 0, st>>>(part, 2 * p.VT, Tc, rows, sel, ids, S, shift, V, logprob,
+                                                    lse_chunk, LossParams{});
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }
@@ -1051,7 +1143,8 @@ struct BwdScratch {
 static int32_t launch_bwd_chunk(uint16_t* stash, const void* lm_head, const void* lm_head_t, const int64_t* ids,
                                 int shift, const ChunkRows& rows, int64_t S, int64_t V, int64_t H,
                                 const float* lse_chunk, const float* coef_chunk, const float* ref_chunk,
-                                const BwdScratch& sc, uint16_t* d_hidden, int* dropped, hipStream_t st) {
+                                const BwdScratch& sc, uint16_t* d_hidden, float* dropped, const LossReduce& loss,
+                                hipStream_t st) {
   const int64_t Tc = rows.cap;
   const int HT = (int)((H + TILE - 1) / TILE);
   const int TT = (int)((Tc + TILE - 1) / TILE);
@@ -1068,16 +1161,16 @@ static int32_t launch_bwd_chunk(uint16_t* stash, const void* lm_head, const void
   b.sched = sc.sched;
   b.partial = sc.partial;
   const int64_t max_blocks = sc.part_rows / TILE * HT;  // tiles * splits can never exceed this
-  const int64_t dense_cap = (int64_t)HT * TT * 16;
+  const int64_t dense_cap = (int64_t)HT * TT * max_splits(HT, num_cus());
   const unsigned grid = (unsigned)(max_blocks < dense_cap ? max_blocks : dense_cap);
   prof_begin(PROF_DHIDDEN_GEMM, st);
   dhidden_gemm_kernel<<<grid, nthreads<BWD_NI>(), 0, st>>>(b);
   prof_end(PROF_DHIDDEN_GEMM, st);
   ARTK_CHECK_LAUNCH();
   const int64_t n4 = Tc * H / 4;
-  splitk_reduce_kernel<<<(unsigned)((n4 + 255) / 256), 256, 0, st>>>(
+  splitk_reduce_kernel<<<(unsigned)((n4 + 255) / 256 + (loss.scalars ? 1 : 0)), 256, 0, st>>>(
       sc.partial, sc.pos, sc.sched, rows, H, V, coef_chunk, lse_chunk, ref_chunk, ids, S, shift,
-      (const uint16_t*)lm_head, d_hidden, dropped);
+      (const uint16_t*)lm_head, d_hidden, dropped, loss);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }
@@ -1149,7 +1242,7 @@ int32_t artk_logprob_fwd(const void* hidden, const void* lm_head, const int64_t*
     return ARTK_ERR_WORKSPACE_TOO_SMALL;
   }
   return launch_fwd_chunk(hidden, lm_head, ids, shift, dense_rows(0, T), S, V, H, part, sel, nullptr, nullptr,
-                          nullptr, logprob, lse, (hipStream_t)stream);
+                          NeedSource{}, nullptr, logprob, lse, nullptr, (hipStream_t)stream);
 }
 
 // Scratch of one chunk of Tc positions carved out of the caller's workspace.
@@ -1260,14 +1353,14 @@ int32_t artk_logprob_bwd(const void* hidden, const void* lm_head, const void* lm
     step = steps.step(ci);
     const int64_t n = (T - t0 < step) ? (T - t0) : step;
     // The scratch row pitch is V, so a shorter chunk simply uses fewer rows.
-    need_from_grad_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(grad_logprob + t0, n, c.need);
-    ARTK_CHECK_LAUNCH();
+    NeedSource source{};
+    source.grad = grad_logprob + t0;
     const ChunkRows rows = dense_rows(t0, n);
-    rc = launch_fwd_chunk(hidden, lm_head, ids, shift, rows, S, V, H, c.part, c.sel, c.stash, c.ref, c.need,
-                          nullptr, c.lse_tmp, st);
+    rc = launch_fwd_chunk(hidden, lm_head, ids, shift, rows, S, V, H, c.part, c.sel, c.stash, c.ref, source,
+                          c.need, nullptr, c.lse_tmp, nullptr, st);
     if (rc) return rc;
     rc = launch_bwd_chunk(c.stash, lm_head, lm_head_t, ids, shift, rows, S, V, H, lse + t0, grad_logprob + t0,
-                          c.ref, c.bwd, (uint16_t*)d_hidden, nullptr, st);
+                          c.ref, c.bwd, (uint16_t*)d_hidden, nullptr, LossReduce{}, st);
     if (rc) return rc;
   }
   return ARTK_OK;
@@ -1320,7 +1413,7 @@ static int32_t grpo_loss_run(const float* new_logprob, const float* old_logprob,
   p.coef = coef;
   grpo_loss_tok_kernel<<<(unsigned)((T + 255) / 256), 256, 0, st>>>(p);
   ARTK_CHECK_LAUNCH();
-  grpo_loss_reduce_kernel<<<1, 1024, 0, st>>>(pl, kl, T, count, p.ref_lp ? beta : 0.f, 0, scalars);
+  grpo_loss_reduce_kernel<<<1, 1024, 0, st>>>(pl, kl, T, count, p.ref_lp ? beta : 0.f, scalars);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }
@@ -1391,22 +1484,14 @@ int32_t artk_grpo_fused(const void* hidden, const void* lm_head, const void* lm_
   }
   hipStream_t st = (hipStream_t)stream;
   const float* ref = (beta > 0.f) ? ref_logprob : nullptr;
-  mask_count_kernel<<<1, 1024, 0, st>>>(mask, T, S, 1, c.count);
-  ARTK_CHECK_LAUNCH();
+  const NeedSource source{nullptr, mask, weights, advantages, ref};
   if (skip) {
-    // Positions that are not evaluated keep: logprob NaN, zero loss terms, zero d_hidden.
-    compact_eval_kernel<<<1, 1024, 0, st>>>(mask, weights, advantages, ref, T, S, 1, c.eval_idx,
-                                            c.n_eval);
+    compact_eval_kernel<<<1, 1024, 0, st>>>(source, T, S, 1, c.eval_idx, c.n_eval, c.count, scalars + 4);
     ARTK_CHECK_LAUNCH();
-    const unsigned gT = (unsigned)((T + 255) / 256);
-    fill_f32_kernel<<<gT, 256, 0, st>>>(logprob, T, NAN);
-    ARTK_CHECK_LAUNCH();
-    fill_f32_kernel<<<gT, 256, 0, st>>>(c.pl, T, 0.f);
-    ARTK_CHECK_LAUNCH();
-    fill_f32_kernel<<<gT, 256, 0, st>>>(c.kl, T, 0.f);
-    ARTK_CHECK_LAUNCH();
-    const int64_t nd = T * H / 2;  // bf16 pairs
-    fill_f32_kernel<<<(unsigned)((nd + 255) / 256), 256, 0, st>>>((float*)d_hidden, nd, 0.f);
+    const int64_t n16 = T * H / 8;
+    const int64_t blocks = (n16 + 1023) / 1024;
+    skip_fill_kernel<<<(unsigned)(blocks < 8 * num_cus() ? blocks : 8 * num_cus()), 256, 0, st>>>(
+        logprob, c.pl, c.kl, T, (uint4*)d_hidden, n16);
     ARTK_CHECK_LAUNCH();
   }
   // In skip mode the number of evaluated rows is known only on the device: every
@@ -1425,14 +1510,9 @@ int32_t artk_grpo_fused(const void* hidden, const void* lm_head, const void* lm_
     } else {
       const int64_t n = (T - t0 < step) ? (T - t0) : step;
       rows = dense_rows(t0, n);
-      need_from_inputs_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(mask, weights, advantages,
-                                                                           ref, t0, n, S, 1, c.need);
-      ARTK_CHECK_LAUNCH();
     }
-    rc = launch_fwd_chunk(hidden, lm_head, tokens, 1, rows, S, V, H, c.part, c.sel, c.stash, c.ref,
-                          skip ? nullptr : c.need, logprob, c.lse, st);
-    if (rc) return rc;
-    LossParams p;
+    FwdFused f;
+    LossParams& p = f.loss;
     p.new_lp = logprob;
     p.old_lp = old_logprob;
     p.adv = advantages;
@@ -1449,13 +1529,29 @@ int32_t artk_grpo_fused(const void* hidden, const void* lm_head, const void* lm_
     p.pl_tok = c.pl;
     p.kl_tok = c.kl;
     p.coef = c.coef;
-    grpo_loss_tok_kernel<<<(unsigned)((rows.cap + 255) / 256), 256, 0, st>>>(p);
-    ARTK_CHECK_LAUNCH();
+    f.T = T;
+    f.count = t0 == 0 && !skip ? c.count : nullptr;
+    f.dropped = scalars + 4;
+    // (compact rows are all needed)
+    rc = launch_fwd_chunk(hidden, lm_head, tokens, 1, rows, S, V, H, c.part, c.sel, c.stash, c.ref,
+                          skip ? NeedSource{} : source, skip ? nullptr : c.need, logprob, c.lse, &f, st);
+    if (rc) return rc;
+    LossReduce sum{};
+    if (t0 + step >= T) sum = LossReduce{c.pl, c.kl, T, c.count, ref ? beta : 0.f, scalars};
     rc = launch_bwd_chunk(c.stash, lm_head, lm_head_t, tokens, 1, rows, S, V, H, c.lse, c.coef, c.ref, c.bwd,
-                          (uint16_t*)d_hidden, c.count + 1, st);
+                          (uint16_t*)d_hidden, scalars + 4, sum, st);
     if (rc) return rc;
   }
-  grpo_loss_reduce_kernel<<<1, 1024, 0, st>>>(c.pl, c.kl, T, c.count, ref ? beta : 0.f, 1, scalars);
+  return ARTK_OK;
+}
+
+int32_t artk_scale_bf16(const void* in, const float* factor, void* out, int64_t n, artk_stream_t stream) {
+  ARTK_CHECK_ARG(in && factor && out, "null pointer argument");
+  ARTK_CHECK_ARG(n > 0 && n % 8 == 0 && aligned16(in) && aligned16(out),
+                 "n must be a positive multiple of 8, pointers 16-byte aligned");
+  const int64_t n16 = n / 8, blocks = (n16 + 1023) / 1024;
+  scale_bf16_kernel<<<(unsigned)(blocks < 8 * num_cus() ? blocks : 8 * num_cus()), 256, 0, (hipStream_t)stream>>>(
+      (const uint4*)in, factor, (uint4*)out, n16);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }

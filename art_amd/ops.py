@@ -260,6 +260,16 @@ def grpo_fused(hidden, lm_head, lm_head_t, tokens, old_logprob, advantages, mask
     return scalars, logprob, d_hidden
 
 
+def scale_bf16(x: torch.Tensor, factor: torch.Tensor) -> torch.Tensor:
+    """x * factor for a bf16 tensor and an f32 scalar on the device."""
+    _need(x, "x", torch.bfloat16)
+    _need(factor, "factor", torch.float32, ())
+    out = torch.empty_like(x)
+    _lib.check(_lib.load().artk_scale_bf16(x.data_ptr(), factor.data_ptr(), out.data_ptr(), x.numel(),
+                                           _stream(x.device)))
+    return out
+
+
 def grpo_fused_workspace_bytes(T: int, V: int, H: int, chunk_tokens: int = DEFAULT_CHUNK_TOKENS) -> int:
     return int(_lib.load().artk_grpo_fused_workspace_bytes(T, V, H, chunk_tokens))
 

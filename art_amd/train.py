@@ -180,13 +180,15 @@ class _FusedGRPOLossFn(torch.autograd.Function):
         ctx.shape = (B, S, H)
         logprob = logprob.view(B, S)
         ctx.mark_non_differentiable(scalars, logprob)
+        ctx.set_materialize_grads(False)  # no zero tensors for the outputs without a gradient
         return scalars[0], scalars, logprob
 
     @staticmethod
     def backward(ctx, g_loss, _g_scalars, _g_logprob):
         (d_hidden,) = ctx.saved_tensors
-        g = (d_hidden * g_loss).to(d_hidden.dtype).view(ctx.shape)
-        return (g,) + (None,) * 12
+        if g_loss is None:
+            return (None,) * 13
+        return (ops.scale_bf16(d_hidden, g_loss.to(torch.float32)).view(ctx.shape),) + (None,) * 12
 
 
 def fused_grpo_loss(hidden_states, lm_head, tokens, logprobs, advantages, assistant_mask, weights,
