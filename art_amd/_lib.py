@@ -132,6 +132,8 @@ SIGNATURES.update({
     "artk_lora_linear_multi_fwd_workspace_bytes": (_sz, [_i64, _i64, C.POINTER(LoraProjStruct), _i32]),
     "artk_lora_linear_multi_fwd": (_i32, [_p, C.POINTER(LoraProjStruct), _i32, _f32, _i64, _i64, _p, _sz, _p]),
     "artk_lora_linear_multi_bwd_workspace_bytes": (_sz, [_i64, _i64, C.POINTER(LoraProjStruct), _i32]),
+    "artk_lora_linear_multi_bwd_typed": (
+        _i32, [_p, C.POINTER(LoraProjStruct), _i32, _f32, _i64, _i64, _i32, _p, _p, _sz, _p]),
     "artk_lora_linear_multi_bwd": (_i32, [_p, C.POINTER(LoraProjStruct), _i32, _f32, _i64, _i64, _p, _p, _sz, _p]),
     "artk_lora_linear_bwd_nf4": (
         _i32, [_p, _p, C.POINTER(Nf4Struct), _p, _p, _p, _f32, _i64, _i64, _i64, _i32, _p, _p, _p, _p, _sz, _p]),
@@ -157,6 +159,18 @@ def load() -> C.CDLL:
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+def native():
+    """The autograd functions over the C-ABI (art_amd/_native.so, built with libartk.so from
+    ``csrc/native_ops.cpp``); there is no fallback."""
+    load()
+    try:
+        from . import _native
+    except ImportError as e:
+        raise ImportError(f"art_amd/_native.so is not built for this Python and torch ({e}). Build it with "
+                          f"`make -C {os.path.dirname(LIB_PATH)}`.") from e
+    return _native
 
 
 class ArtkError(RuntimeError):

@@ -12,7 +12,9 @@ from typing import List, Optional
 
 import torch
 
-from . import ops
+from . import _lib, ops
+
+_native = _lib.native()
 
 ROW_MULTIPLE = 256  # plans cover rows of this granularity; positions past the end see, and are seen by, nothing
 
@@ -24,24 +26,6 @@ def attention_plans(group_ids: torch.Tensor, parent_ids: torch.Tensor) -> List[o
     if group_ids.dim() == 1:
         group_ids, parent_ids = group_ids.unsqueeze(0), parent_ids.unsqueeze(0)
     return ops.attn_plan_rows(group_ids.contiguous(), parent_ids.contiguous())
-
-
-class _PackedAttentionFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, q, k, v, plan, scale):
-        out, lse = ops.attn_fwd_rows(q, k, v, plan, scale)
-        ctx.save_for_backward(q, k, v, out, lse, plan)
-        ctx.scale = scale
-        return out
-
-    @staticmethod
-    def backward(ctx, d_out):
-        q, k, v, out, lse, plan = ctx.saved_tensors
-        d_out = d_out.to(torch.bfloat16)
-        if d_out.stride(3) != 1 or 0 in d_out.stride() or d_out.data_ptr() % 16 or any(st % 8 for st in d_out.stride()[:3]):
-            d_out = d_out.contiguous()
-        dq, dk, dv = ops.attn_bwd_rows(q, k, v, out, lse, d_out, plan, ctx.scale)
-        return dq, dk, dv, None, None
 
 
 def packed_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plans: List[ops.AttnPlan],
@@ -59,7 +43,7 @@ def packed_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plans: L
             raise ValueError(f"plan made for a row of {plan.S} positions, tensors have {S}")
     first = plans[0]
     if first.rows == B and all(p.batch is first.batch and p.index == b for b, p in enumerate(plans[:B])):
-        return _PackedAttentionFn.apply(q, k, v, first.batch, scale)
+        return _native.attention(q, k, v, first.batch, scale)
     # plans that were made one by one: a call per row
-    outs = [_PackedAttentionFn.apply(q[b:b + 1], k[b:b + 1], v[b:b + 1], plans[b].buf, scale) for b in range(B)]
+    outs = [_native.attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], plans[b].buf, scale) for b in range(B)]
     return torch.cat(outs, 0)

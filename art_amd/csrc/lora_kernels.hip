@@ -811,6 +811,12 @@ size_t artk_lora_linear_multi_bwd_workspace_bytes(int64_t T, int64_t in, const a
 int32_t artk_lora_linear_multi_bwd(const void* x, const artk_lora_proj_t* proj, int32_t n, float scale,
                                    int64_t T, int64_t in, void* dx, void* workspace, size_t workspace_bytes,
                                    artk_stream_t stream) {
+  return artk_lora_linear_multi_bwd_typed(x, proj, n, scale, T, in, 0, dx, workspace, workspace_bytes, stream);
+}
+
+int32_t artk_lora_linear_multi_bwd_typed(const void* x, const artk_lora_proj_t* proj, int32_t n, float scale,
+                                         int64_t T, int64_t in, int32_t grad_bf16, void* dx, void* workspace,
+                                         size_t workspace_bytes, artk_stream_t stream) {
   int32_t rc = check_multi(proj, n, T, in, true);
   if (rc) return rc;
   ARTK_CHECK_ARG(x != nullptr && dx != nullptr && aligned16(x) && aligned16(dx),
@@ -832,6 +838,7 @@ int32_t artk_lora_linear_multi_bwd(const void* x, const artk_lora_proj_t* proj, 
   p.n_tiles = MT * p.NT;
   StatsReduceJob jx{c.colp_x, c.gx.n_slabs, in, scale, nullptr, 1, nullptr, 0, 0.f};
   jx.n_split = n;
+  jx.to_bf16 = grad_bf16 != 0;
   SmallTransposeMulti tr;
   StatsMulti sm;
   StatsReduceMulti rm;
@@ -854,6 +861,7 @@ int32_t artk_lora_linear_multi_bwd(const void* x, const artk_lora_proj_t* proj, 
     ja.out_off = r0;
     rm.job[2 * i] = ja;
     rm.job[2 * i + 1] = StatsReduceJob{o.colp_g, o.gg.n_slabs, q.out, scale, q.dB, 0, nullptr, 0, 0.f};
+    rm.job[2 * i + 1].to_bf16 = grad_bf16 != 0;
     rm.R[2 * i] = rm.R[2 * i + 1] = q.r;
     p.seg[i] = LoraSeg{q.W_t, q.g, o.At, o.gb16, q.out, q.r, RP};
     jx.outs[i] = q.dA;

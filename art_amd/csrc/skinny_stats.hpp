@@ -382,7 +382,13 @@ struct StatsReduceJob {
   int n_split = 0;
   float* outs[4] = {nullptr, nullptr, nullptr, nullptr};
   int e_start[5] = {0, 0, 0, 0, 0};
+  // out / outs are bf16 arrays of the same shapes (gradients of bf16 parameters)
+  int to_bf16 = 0;
 };
+__device__ __forceinline__ void stats_put(float* base, int64_t i, float v, int to_bf16) {
+  if (to_bf16) ((uint16_t*)base)[i] = f32_to_bf16(v);
+  else base[i] = v;
+}
 
 __device__ __forceinline__ void stats_reduce_one(const StatsReduceJob& j, int R, int64_t i) {
   const int width = j.out_bf16 ? j.RP : R;
@@ -413,12 +419,13 @@ __device__ __forceinline__ void stats_reduce_one(const StatsReduceJob& j, int R,
             dst = j.outs[k];
             e0 = j.e_start[k];
           }
-        dst[(int64_t)(e - e0) * j.n + row] = s;
+        stats_put(dst, (int64_t)(e - e0) * j.n + row, s, j.to_bf16);
       } else {
-        j.out[(int64_t)e * j.n + row] = s;
+        stats_put(j.out, (int64_t)e * j.n + row, s, j.to_bf16);
       }
     } else {
-      j.out[row * (j.out_ld ? j.out_ld : R) + j.out_off + e] = j.row_w ? s * j.row_w[j.row_idx[row]] : s;
+      stats_put(j.out, row * (j.out_ld ? j.out_ld : R) + j.out_off + e, j.row_w ? s * j.row_w[j.row_idx[row]] : s,
+                j.to_bf16);
     }
   }
   if (j.out_bf16) j.out_bf16[row * j.RP + e] = f32_to_bf16(s * j.bf16_scale);

@@ -14,67 +14,36 @@ import math
 import torch
 from torch import nn
 
-from . import ops
+from . import _lib, ops
+
+_native = _lib.native()
 
 
-class _LoRALinearFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, weight, lora_A, lora_B, scale, bias=None):
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, x.shape[-1]).to(torch.bfloat16).contiguous()
-        A = lora_A.detach().to(torch.bfloat16).contiguous()
-        B = lora_B.detach().to(torch.bfloat16).contiguous()
-        y, xa = ops.lora_linear_fwd(x2, weight, A, B, scale, bias)
-        ctx.save_for_backward(x2, weight, A, B, xa)
-        ctx.scale = scale
-        ctx.lead = lead
-        ctx.param_dtypes = (lora_A.dtype, lora_B.dtype, x.dtype)
-        return y.view(*lead, weight.shape[0])
-
-    @staticmethod
-    def backward(ctx, g):
-        x2, weight, A, B, xa = ctx.saved_tensors
-        g2 = g.reshape(-1, g.shape[-1]).to(torch.bfloat16).contiguous()
-        dx, dA, dB = ops.lora_linear_bwd(g2, x2, ops.transposed_weight(weight), A, B, xa, ctx.scale)
-        a_dtype, b_dtype, x_dtype = ctx.param_dtypes
-        return (dx.view(*ctx.lead, x2.shape[-1]).to(x_dtype), None, dA.to(a_dtype), dB.to(b_dtype), None, None)
+def _frozen_bias(bias):
+    if bias is None:
+        return None
+    if bias.requires_grad:
+        raise ValueError("the bias of a LoRA-wrapped linear is frozen (peft bias='none'); got requires_grad=True")
+    return bias.detach().to(torch.bfloat16).contiguous()
 
 
-class _LoRALinearNF4Fn(torch.autograd.Function):
-    """The same linear with the frozen weight kept as NF4 codes (art_amd.quant.NF4Weight)."""
-
-    @staticmethod
-    def forward(ctx, x, w_nf4, lora_A, lora_B, scale, bias=None):
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, x.shape[-1]).to(torch.bfloat16).contiguous()
-        A = lora_A.detach().to(torch.bfloat16).contiguous()
-        B = lora_B.detach().to(torch.bfloat16).contiguous()
-        y, xa = ops.lora_linear_fwd_nf4(x2, w_nf4, A, B, scale, bias)
-        ctx.save_for_backward(x2, A, B, xa)
-        ctx.w_nf4 = w_nf4
-        ctx.scale = scale
-        ctx.lead = lead
-        ctx.param_dtypes = (lora_A.dtype, lora_B.dtype, x.dtype)
-        return y.view(*lead, w_nf4.shape[0])
-
-    @staticmethod
-    def backward(ctx, g):
-        x2, A, B, xa = ctx.saved_tensors
-        g2 = g.reshape(-1, g.shape[-1]).to(torch.bfloat16).contiguous()
-        dx, dA, dB = ops.lora_linear_bwd_nf4(g2, x2, ctx.w_nf4, A, B, xa, ctx.scale)
-        a_dtype, b_dtype, x_dtype = ctx.param_dtypes
-        return (dx.view(*ctx.lead, x2.shape[-1]).to(x_dtype), None, dA.to(a_dtype), dB.to(b_dtype), None, None)
+def _lora_projections(x, weights, lora_As, lora_Bs, scale: float, biases):
+    """Projections of the same x through the native autograd function (art_amd/csrc/native_ops.cpp): one call
+    each way, nothing concatenated.  The transposed copies of the frozen weights are only looked up when there
+    can be a backward."""
+    graph = torch.is_grad_enabled() and any(t.requires_grad for t in (x, *lora_As, *lora_Bs))
+    wts = [ops.transposed_weight(w) for w in weights] if graph else []
+    return _native.lora_multi(x, weights, wts, lora_As, lora_Bs, biases, scale)
 
 
 def lora_linear(x, weight, lora_A, lora_B, scale: float, bias=None):
     """y = x W^T + bias + scale * (x A^T) B^T with gradients for x, A and B (W and bias frozen)."""
-    if bias is not None:
-        if bias.requires_grad:
-            raise ValueError("the bias of a LoRA-wrapped linear is frozen (peft bias='none'); got requires_grad=True")
-        bias = bias.detach().to(torch.bfloat16).contiguous()
-    if not isinstance(weight, torch.Tensor):   # an NF4Weight
-        return _LoRALinearNF4Fn.apply(x, weight, lora_A, lora_B, float(scale), bias)
-    return _LoRALinearFn.apply(x, weight, lora_A, lora_B, float(scale), bias)
+    bias = _frozen_bias(bias)
+    if not isinstance(weight, torch.Tensor):   # an NF4Weight: the bf16 weight lives inside each call only
+        w = weight
+        return _native.lora_nf4(x, w.packed, w.absmax, w.absmax_q, w.code2, w.absmax2, float(w.offset), w.blocksize,
+                                *w.shape, lora_A, lora_B, bias, float(scale))
+    return _lora_projections(x, [weight], [lora_A], [lora_B], float(scale), [bias])[0]
 
 
 class LoRALinear(nn.Module):
@@ -133,48 +102,6 @@ class LoRALinear(nn.Module):
         return lora_linear(x, weight, self.lora_A, self.lora_B, self.scaling, self.bias)
 
 
-class _FusedLoRAFn(torch.autograd.Function):
-    """Several projections of the same input through the library's multi-projection entry
-    points: one launch walks the tiles of all of them over one x, the input gradient is one
-    accumulation over all of them.  Weights, adapters, outputs and upstream gradients stay
-    separate tensors: nothing is concatenated and no block-diagonal factor is built."""
-
-    @staticmethod
-    def forward(ctx, x, scale, n, *rest):
-        weights, biases = rest[:n], rest[n:2 * n]
-        As, Bs = rest[2 * n:3 * n], rest[3 * n:4 * n]
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, x.shape[-1]).to(torch.bfloat16).contiguous()
-        A16 = [a.detach().to(torch.bfloat16).contiguous() for a in As]
-        B16 = [b.detach().to(torch.bfloat16).contiguous() for b in Bs]
-        ys, xas = ops.lora_linear_multi_fwd(x2, list(weights), A16, B16, scale, list(biases))
-        ctx.save_for_backward(x2, *weights, *A16, *B16, *xas)
-        ctx.meta = (scale, n, lead, [a.dtype for a in As], [b.dtype for b in Bs], x.dtype)
-        return tuple(y.view(*lead, y.shape[-1]) for y in ys)
-
-    @staticmethod
-    def backward(ctx, *gs):
-        scale, n, lead, a_dt, b_dt, x_dt = ctx.meta
-        saved = ctx.saved_tensors
-        x2 = saved[0]
-        weights, A16, B16, xas = (saved[1 + k * n:1 + (k + 1) * n] for k in range(4))
-        g2 = []
-        for g, w in zip(gs, weights):   # an output nobody used has no gradient: zeros
-            g2.append(torch.zeros((x2.shape[0], w.shape[0]), dtype=torch.bfloat16, device=x2.device) if g is None
-                      else g.reshape(-1, g.shape[-1]).to(torch.bfloat16).contiguous())
-        dx, dAs, dBs = ops.lora_linear_multi_bwd(g2, x2, [ops.transposed_weight(w) for w in weights], list(A16),
-                                                 list(B16), list(xas), scale)
-        # gradients in the parameters' dtypes: one multi-tensor copy instead of a cast per tensor
-        grads, want = list(dAs) + list(dBs), list(a_dt) + list(b_dt)
-        cast = [i for i, (g_, t) in enumerate(zip(grads, want)) if g_.dtype != t]
-        if cast:
-            dst = [torch.empty_like(grads[i], dtype=want[i]) for i in cast]
-            torch._foreach_copy_(dst, [grads[i] for i in cast])
-            for i, d in zip(cast, dst):
-                grads[i] = d
-        return (dx.view(*lead, x2.shape[-1]).to(x_dt), None, None, *([None] * (2 * n)), *grads)
-
-
 class FusedLoRALinear(nn.Module):
     """Projections that read the same activations (q/k/v, or gate/up) in one call each way:
     one persistent launch over the tiles of all of them (the narrow projections, k and v with
@@ -201,9 +128,5 @@ class FusedLoRALinear(nn.Module):
 
     def forward(self, x: torch.Tensor):
         ls = self.layers
-        for l in ls:
-            if l.bias is not None and l.bias.requires_grad:
-                raise ValueError("the bias of a LoRA-wrapped linear is frozen (peft bias='none')")
-        biases = [None if l.bias is None else l.bias.detach().to(torch.bfloat16).contiguous() for l in ls]
-        return _FusedLoRAFn.apply(x, float(self.scaling), len(ls), *[l.weight for l in ls], *biases,
-                                  *[l.lora_A for l in ls], *[l.lora_B for l in ls])
+        return tuple(_lora_projections(x, [l.weight for l in ls], [l.lora_A for l in ls], [l.lora_B for l in ls],
+                                       float(self.scaling), [_frozen_bias(l.bias) for l in ls]))

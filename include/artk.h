@@ -485,6 +485,10 @@ size_t artk_lora_linear_multi_bwd_workspace_bytes(int64_t T, int64_t in, const a
 int32_t artk_lora_linear_multi_bwd(const void* x, const artk_lora_proj_t* proj, int32_t n, float scale,
                                    int64_t T, int64_t in, void* dx, void* workspace, size_t workspace_bytes,
                                    artk_stream_t stream);
+/* The same with dA and dB written as bf16 when grad_bf16 is set (their pointers then address bf16 arrays). */
+int32_t artk_lora_linear_multi_bwd_typed(const void* x, const artk_lora_proj_t* proj, int32_t n, float scale,
+                                         int64_t T, int64_t in, int32_t grad_bf16, void* dx, void* workspace,
+                                         size_t workspace_bytes, artk_stream_t stream);
 
 /* ------------------------------------------------------------------------- *
  * Per-kernel timing (measurement aid; no counterpart in the reference).

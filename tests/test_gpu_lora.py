@@ -313,3 +313,42 @@ def test_small_products(artk_lib, gpu, T, n_in, outs, r):
         y1, _ = ops.lora_linear_fwd(x.to(gpu), W[i].to(gpu), A[i].to(gpu), B[i].to(gpu), 0.5, bias[i].to(gpu))
         assert rel(y1, ys[i].float().cpu()) <= 4e-3   # one rounding to bf16; the K range may be split elsewhere
     assert rel(dx, dx0) <= 1e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_native_autograd_function(artk_lib, gpu, dtype):
+    """The native autograd function around the projections: leading dimensions, an fp32 input, adapters in either
+    dtype (gradients come back in it), an output nobody uses, no graph under no_grad, and an in-place change of
+    the frozen weight between forward and backward, which is an error.  1e-2: bf16 products; the gradients of
+    bf16 adapters are the fp32 sums rounded once (4e-3)."""
+    from art_amd.lora import FusedLoRALinear, LoRALinear
+
+    torch.manual_seed(5)
+    T, n_in, outs, r = 70, 128, (192, 64), 8
+    layers = [LoRALinear(n_in, o, r=r, lora_alpha=16, device=gpu, dtype=dtype) for o in outs]
+    with torch.no_grad():
+        for l in layers:
+            l.lora_B.normal_(std=0.05)
+    mod = FusedLoRALinear(layers)
+    x = torch.randn(2, T // 2, n_in, device=gpu, requires_grad=True)
+    up = torch.randn(2, T // 2, outs[0], device=gpu)
+    y, _ = mod(x)
+    assert y.shape == (2, T // 2, outs[0]) and y.dtype == torch.bfloat16
+    y.backward(up.to(torch.bfloat16))
+    f = lambda t: t.detach().to(torch.bfloat16).float().cpu()
+    xf, gf, W, A, B = f(x).view(T, n_in), f(up).view(T, outs[0]), f(layers[0].weight), f(layers[0].lora_A), f(layers[0].lora_B)
+    rel = lambda a, b: ((a.float().cpu() - b).norm() / b.norm()).item()
+    assert x.grad.dtype == torch.float32 and rel(x.grad.view(T, n_in), gf @ W + 2.0 * (gf @ B) @ A) <= 1e-2
+    assert layers[0].lora_A.grad.dtype == dtype and rel(layers[0].lora_A.grad, 2.0 * (gf @ B).T @ xf) <= 1e-2
+    assert layers[0].lora_B.grad.dtype == dtype and rel(layers[0].lora_B.grad, 2.0 * gf.T @ (xf @ A.T)) <= 1e-2
+    assert layers[1].lora_A.grad.abs().max().item() == 0.0 and layers[1].lora_B.grad.abs().max().item() == 0.0
+    with torch.no_grad():
+        y2, _ = mod(x)
+    assert not y2.requires_grad and torch.equal(y2, y)
+    y3, _ = mod(x)
+    with torch.no_grad():
+        layers[0].weight.mul_(2.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y3.sum().backward()
+    with pytest.raises(ValueError):
+        mod(x.cpu())
