@@ -131,13 +131,15 @@ struct LoraFunction : torch::autograd::Function<LoraFunction> {
     saved.insert(saved.end(), A16.begin(), A16.end());
     saved.insert(saved.end(), B16.begin(), B16.end());
     saved.insert(saved.end(), xa.begin(), xa.end());
+    // Frozen storage that outlives the call (codes, transposed copies) rides on the node itself: as saved tensors,
+    // hooks that move activations to the host would copy it for every projection.
     if (a.nf4) {
-      for (const Tensor& t : {a.nf4->packed, a.nf4->absmax, a.nf4->absmax_q, a.nf4->code2, a.nf4->absmax2})
-        saved.push_back(t);
+      ctx->saved_data["frozen"] =
+          variable_list{a.nf4->packed, a.nf4->absmax, a.nf4->absmax_q, a.nf4->code2, a.nf4->absmax2};
       ctx->saved_data["offset"] = a.nf4->offset;
       ctx->saved_data["blocksize"] = a.nf4->blocksize;
     } else {
-      saved.insert(saved.end(), a.W_t.begin(), a.W_t.end());
+      ctx->saved_data["frozen"] = a.W_t;
       saved.insert(saved.end(), a.W.begin(), a.W.end());  // (their versions are checked with the rest)
     }
     ctx->save_for_backward(saved);
@@ -161,15 +163,15 @@ struct LoraFunction : torch::autograd::Function<LoraFunction> {
     const Tensor& x2 = saved[0];
     c10::OptionalDeviceGuard guard(x2.device());
     const int64_t T = x2.size(0), in = x2.size(1);
+    const auto t = ctx->saved_data["frozen"].toTensorVector();
     Tensor W_t;
     if (on_codes) {
-      const Tensor* t = &saved[1 + 3 * n];
       const Nf4 w{t[0], t[1], t[2], t[3], t[4], ctx->saved_data["offset"].toDouble(),
                   ctx->saved_data["blocksize"].toInt(), saved[1 + n].size(0), in};
       W_t = make(x2, {in, w.out}, at::kBFloat16);
       w.dequantise(true, W_t);
     } else {
-      TORCH_CHECK((int)saved.size() == 1 + 5 * n, "the projections were called without a graph");
+      TORCH_CHECK((int)t.size() == n, "the projections were called without a graph");
     }
     artk_lora_proj_t proj[ARTK_LORA_MULTI_MAX] = {};
     std::vector<Tensor> g2, dA, dB;
@@ -178,7 +180,7 @@ struct LoraFunction : torch::autograd::Function<LoraFunction> {
     const at::ScalarType gt = all_bf16 ? at::kBFloat16 : at::kFloat;
     for (int i = 0; i < n; ++i) {
       const Tensor &A = saved[1 + i], &B = saved[1 + n + i], &xa = saved[1 + 2 * n + i];
-      const Tensor& Wt = on_codes ? W_t : saved[1 + 3 * n + i];
+      const Tensor& Wt = on_codes ? W_t : t[i];
       const int64_t out = B.size(0), r = B.size(1);
       g2.push_back(rows_bf16(grads[i]));
       need(Wt, "W_t", at::kBFloat16, {in, out});
@@ -223,6 +225,7 @@ Tensor lora_nf4(const Tensor& x, const Tensor& packed, std::optional<Tensor> abs
                 int64_t out, int64_t in, const Tensor& A, const Tensor& B, std::optional<Tensor> bias, double scale) {
   auto w = std::make_shared<Nf4>();
   auto set = [](std::optional<Tensor>& t) { return t ? *t : Tensor(); };
+  TORCH_CHECK_VALUE(blocksize >= 32, "the quantisation block size must be at least 32, got ", blocksize);
   need(packed, "packed", at::kByte, {out * in / 2});
   const int64_t blocks = out * in / blocksize;
   if (absmax) {
@@ -268,14 +271,16 @@ struct AttentionFunction : torch::autograd::Function<AttentionFunction> {
     strides_of(out, "out", st + 9);
     check(artk_attn_fwd_rows(q.data_ptr(), k.data_ptr(), v.data_ptr(), plan.data_ptr(), B, S, (int32_t)Hq, (int32_t)Hkv,
                              (int32_t)D, st, (float)scale, out.data_ptr(), lse.data_ptr<float>(), stream_of(q)));
-    ctx->save_for_backward({q, k, v, out, lse, plan});
+    ctx->save_for_backward({q, k, v, out, lse});
+    ctx->saved_data["plan"] = plan;  // shared by all layers: hooks on saved tensors need not see it
     ctx->saved_data["scale"] = scale;
     return out;
   }
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list saved = ctx->get_saved_variables();
-    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4], &plan = saved[5];
+    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4];
+    const Tensor plan = ctx->saved_data["plan"].toTensor();
     c10::OptionalDeviceGuard guard(q.device());
     const int64_t B = q.size(0), S = q.size(1), Hq = q.size(2), D = q.size(3), Hkv = k.size(2);
     Tensor g = grads[0].to(at::kBFloat16);

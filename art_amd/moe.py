@@ -55,16 +55,17 @@ class _MoEExpertsFn(torch.autograd.Function):
             dtype = torch.float32
         adapters = {n: p.detach().to(dtype).contiguous() for n, p in zip(ops._MOE_PARAMS, params)}
         y, routing, saved = ops.moe_experts_fwd(x, logits, top_k, W_gu, W_d, adapters, scale)
-        ctx.save_for_backward(x, saved, Wt_gu, Wt_d, *params)
+        ctx.save_for_backward(x, saved, Wt_gu, Wt_d)
         ctx.routing, ctx.scale = routing, scale
+        ctx.rank, ctx.dtypes = params[0].shape[1], [p.dtype for p in params]   # (their values are in `saved`)
         return y, routing
 
     @staticmethod
     def backward(ctx, g, _g_routing):
-        x, saved, Wt_gu, Wt_d, *params = ctx.saved_tensors
-        dx, grads = ops.moe_experts_bwd(g.contiguous(), x, ctx.routing, saved, Wt_gu, Wt_d,
-                                        dict(zip(ops._MOE_PARAMS, params)), ctx.scale)
-        return (dx,) + (None,) * 7 + tuple(grads[n].to(p.dtype) for n, p in zip(ops._MOE_PARAMS, params))
+        x, saved, Wt_gu, Wt_d = ctx.saved_tensors
+        dx, grads = ops.moe_experts_bwd(g.contiguous(), x, ctx.routing, saved, Wt_gu, Wt_d, ctx.rank,
+                                        ctx.scale)
+        return (dx,) + (None,) * 7 + tuple(grads[n].to(t) for n, t in zip(ops._MOE_PARAMS, ctx.dtypes))
 
 
 class MoELoRAExperts(nn.Module):
@@ -110,7 +111,8 @@ class MoELoRAExperts(nn.Module):
 
     def forward(self, x: torch.Tensor, router_logits: torch.Tensor):
         """x bf16 [T,H], router_logits f32 [T,E] -> (y bf16 [T,H], routing)."""
-        params = (self.gate_lora_A, self.gate_lora_B, self.up_lora_A, self.up_lora_B, self.down_lora_A, self.down_lora_B)
+        params = (self.gate_lora_A, self.gate_lora_B, self.up_lora_A, self.up_lora_B, self.down_lora_A,
+                  self.down_lora_B)
         return _MoEExpertsFn.apply(
             x.to(torch.bfloat16).contiguous(), router_logits.detach().float().contiguous(), self.top_k,
             self.gate_up_weight, self.down_weight, self._transposed("gate_up"), self._transposed("down"),

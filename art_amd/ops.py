@@ -423,12 +423,16 @@ def moe_lora_grouped_bwd(g, x, gather, W_t, A, B, xa, scale: float, routing: Rou
 _MOE_PARAMS = ("gate_A", "gate_B", "up_A", "up_B", "down_A", "down_B")
 
 
-def _moe_experts_struct(x, routing: Routing, adapters, saved, scale: float):
-    """artk_moe_experts_t with the fields that both directions use (and its two sizes n, r)."""
+def _moe_param_shapes(E: int, H: int, I: int, r: int) -> dict:
+    return {"gate_A": (E, r, H), "up_A": (E, r, H), "gate_B": (E, I, r), "up_B": (E, I, r), "down_A": (E, r, I),
+            "down_B": (E, H, r)}
+
+
+def _moe_experts_struct(x, routing: Routing, I: int, r: int, saved, scale: float):
+    """artk_moe_experts_t with the fields that both directions use."""
     import ctypes as C
 
     T, H = x.shape
-    _, r, I = adapters["down_A"].shape
     st = _lib.MoeExpertsStruct()
     st.x = x.data_ptr()
     for f in ("topk_idx", "topk_w", "perm", "inv_perm", "row_token", "offsets", "tile_prefix", "blk_prefix"):
@@ -450,8 +454,7 @@ def moe_experts_fwd(x, router_logits, k: int, W_gu, W_d, adapters: dict, scale: 
     _need(router_logits, "router_logits", torch.float32, (T, E))
     _need(W_gu, "W_gu", torch.bfloat16, (E, 2 * I, H))
     _need(W_d, "W_d", torch.bfloat16, (E, H, I))
-    shapes = {"gate_A": (E, r, H), "up_A": (E, r, H), "gate_B": (E, I, r), "up_B": (E, I, r), "down_A": (E, r, I),
-              "down_B": (E, H, r)}
+    shapes = _moe_param_shapes(E, H, I, r)
     if dtype not in (torch.float32, torch.bfloat16):
         raise TypeError(f"adapters must be float32 or bfloat16, got {dtype}")
     for name in _MOE_PARAMS:
@@ -465,7 +468,7 @@ def moe_experts_fwd(x, router_logits, k: int, W_gu, W_d, adapters: dict, scale: 
     rt.perm, rt.inv_perm, rt.row_token = i32(n), i32(n), i32(n)
     rt.offsets, rt.tile_prefix, rt.blk_prefix = i32(E + 1), i32(E + 1), i32(E + 1)
     rt.n_rows, rt.n_experts, rt.k = n, E, k
-    st, ref = _moe_experts_struct(x, rt, adapters, None, scale)
+    st, ref = _moe_experts_struct(x, rt, I, r, None, scale)
     saved = _workspace(lib.artk_moe_experts_saved_bytes(ref), dev)
     ws = _workspace(lib.artk_moe_experts_fwd_workspace_bytes(ref), dev)
     y = torch.empty_like(x)
@@ -478,17 +481,18 @@ def moe_experts_fwd(x, router_logits, k: int, W_gu, W_d, adapters: dict, scale: 
     return y, rt, saved
 
 
-def moe_experts_bwd(g, x, routing: Routing, saved, Wt_gu, Wt_d, adapters: dict, scale: float):
-    """(dx bf16 [T,H], dict of f32 adapter gradients) for upstream gradient g bf16 [T,H] of moe_experts_fwd's y."""
+def moe_experts_bwd(g, x, routing: Routing, saved, Wt_gu, Wt_d, r: int, scale: float):
+    """(dx bf16 [T,H], dict of f32 adapter gradients) for upstream gradient g bf16 [T,H] of moe_experts_fwd's y.
+    The rank-r adapters themselves are in `saved`, as the forward used them."""
     _need(g, "g", torch.bfloat16, tuple(x.shape))
     E, I, H = Wt_d.shape
     _need(Wt_d, "Wt_d", torch.bfloat16)
     _need(Wt_gu, "Wt_gu", torch.bfloat16, (E, H, 2 * I))
     lib = _lib.load()
     dev = x.device
-    st, ref = _moe_experts_struct(x, routing, adapters, saved, scale)
+    st, ref = _moe_experts_struct(x, routing, I, r, saved, scale)
     dx = torch.empty_like(x)
-    grads = {name: torch.empty(adapters[name].shape, dtype=torch.float32, device=dev) for name in _MOE_PARAMS}
+    grads = {name: torch.empty(s, dtype=torch.float32, device=dev) for name, s in _moe_param_shapes(E, H, I, r).items()}
     st.g, st.Wt_gu, st.Wt_d, st.dx = g.data_ptr(), Wt_gu.data_ptr(), Wt_d.data_ptr(), dx.data_ptr()
     for name, t in grads.items():
         setattr(st, "d" + name, t.data_ptr())

@@ -352,3 +352,37 @@ def test_native_autograd_function(artk_lib, gpu, dtype):
         y3.sum().backward()
     with pytest.raises(ValueError):
         mod(x.cpu())
+
+
+def test_saved_tensor_hooks_see_activations_only(artk_lib, gpu):
+    """Hooks that move saved tensors to the host (torch.autograd.graph.save_on_cpu) see the activations, adapters
+    and frozen bf16 weights, not the 4-bit codes, the transposed weights or the attention plan, which outlive the
+    call anyway; the gradients are the same bits."""
+    from art_amd import attention, quant
+    from art_amd.lora import LoRALinear
+
+    torch.manual_seed(6)
+    dense = LoRALinear(128, 192, device=gpu)
+    nf4 = LoRALinear.from_nf4(quant.NF4Weight.from_float(torch.randn(64, 192, device=gpu).to(torch.bfloat16)))
+    ids = torch.zeros(1, 70, dtype=torch.int64, device=gpu)
+    plans = attention.attention_plans(ids, ids)
+    x = torch.randn(1, 70, 128, device=gpu, dtype=torch.bfloat16, requires_grad=True)
+
+    def step():
+        h = dense(x)
+        q = h.view(1, 70, 3, 64)
+        y = nf4(attention.packed_attention(q, q[:, :, :1], q[:, :, 1:2], plans).reshape(1, 70, 192))
+        return torch.autograd.grad(y.float().sum(), [x, dense.lora_A, nf4.lora_B])
+
+    want = step()
+    seen = []
+
+    def pack(t):
+        seen.append((t.dtype, tuple(t.shape)))
+        return t.cpu()
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.to(gpu)):
+        got = step()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert (torch.bfloat16, (192, 128)) in seen and (torch.bfloat16, (128, 192)) not in seen
+    assert not any(dtype == torch.uint8 for dtype, _ in seen)

@@ -325,9 +325,31 @@ def test_moe_experts_entry_points(artk_lib, gpu, T, H, I, E, k, r, dtype):
     ad = {n: p.to(dtype).to(gpu) for n, p in P.items()}
     y, rt, saved = ops.moe_experts_fwd(x.to(gpu), logits.to(gpu), k, Wgu.to(gpu), Wd.to(gpu), ad, 0.5)
     dx, grads = ops.moe_experts_bwd(up.to(gpu), x.to(gpu), rt, saved, ops.transpose_batched(Wgu.to(gpu)),
-                                    ops.transpose_batched(Wd.to(gpu)), ad, 0.5)
+                                    ops.transpose_batched(Wd.to(gpu)), r, 0.5)
     assert torch.equal(rt.topk_idx.cpu().long(), ref["topk_idx"].long())
     assert rel_l2(y.cpu().float(), y0.detach()) <= 2e-2
     assert rel_l2(dx.cpu().float(), xr.grad) <= 2e-2
     for n in P:
         assert grads[n].shape == P[n].shape and rel_l2(grads[n].cpu(), Pr[n].grad) <= 2e-2, n
+
+
+def test_moe_parameters_changed_between_forward_and_backward(artk_lib, gpu):
+    """fp32 adapters may change between forward and backward (the gradients are those of the values that the
+    forward used), as long as the inputs stay."""
+    from art_amd.moe import MoELoRAExperts
+
+    torch.manual_seed(11)
+    m = MoELoRAExperts(64, 64, 4, 2, r=8, lora_alpha=16, device=gpu)
+    params = [p for p in m.parameters() if p.requires_grad]
+    with torch.no_grad():
+        for p in params:
+            p.normal_(std=0.05)
+    x, logits = torch.randn(9, 64, device=gpu, dtype=torch.bfloat16), torch.randn(9, 4, device=gpu)
+    up = torch.randn(9, 64, device=gpu, dtype=torch.bfloat16)
+    want = torch.autograd.grad(m(x, logits)[0], params, up)
+    y, _ = m(x, logits)
+    with torch.no_grad():
+        for p in params:
+            p.add_(1.0)
+    for got, ref in zip(torch.autograd.grad(y, params, up), want):
+        assert torch.equal(got, ref)
