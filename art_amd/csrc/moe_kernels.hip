@@ -98,16 +98,18 @@ __global__ __launch_bounds__(PERM_CHUNK) void moe_hist_kernel(const int* __restr
 // position of chunk b's entries of expert e; tile_prefix / blk_prefix: prefix
 // sums of ceil(rows_e / 256) and ceil(rows_e / 16) (work lists of the grouped
 // kernels).  One block of 1024 threads: thread (part, e) walks a quarter of the
-// chunks of expert e, eight independent loads at a time.
+// chunks of expert e, eight independent loads at a time.  order (or nullptr): the
+// experts by falling number of rows, ties by index.
 constexpr int SCAN_PARTS = 4;
 __global__ __launch_bounds__(SCAN_PARTS * MOE_MAX_E) void moe_scan_kernel(const int* __restrict__ cnt, int nb, int E,
                                                                           int* __restrict__ offsets,
                                                                           int* __restrict__ base,
                                                                           int* __restrict__ tile_prefix,
-                                                                          int* __restrict__ blk_prefix) {
+                                                                          int* __restrict__ blk_prefix,
+                                                                          int* __restrict__ order) {
   __shared__ int part[SCAN_PARTS][MOE_MAX_E];
   __shared__ int wsum[3][MOE_MAX_E / 64];
-  __shared__ int off[MOE_MAX_E];
+  __shared__ int off[MOE_MAX_E], rows[MOE_MAX_E], rank[MOE_MAX_E];
   const int e = threadIdx.x % MOE_MAX_E, pt = threadIdx.x / MOE_MAX_E;
   const int per = (nb + SCAN_PARTS - 1) / SCAN_PARTS;
   const int b0 = pt * per, b1 = b0 + per < nb ? b0 + per : nb;
@@ -161,6 +163,8 @@ __global__ __launch_bounds__(SCAN_PARTS * MOE_MAX_E) void moe_scan_kernel(const 
       tile_prefix[e + 1] = tp;
       blk_prefix[e + 1] = bp;
       off[e] = run - tot;
+      rows[e] = tot;
+      rank[e] = 0;
     }
     if (e == 0) {
       offsets[0] = 0;
@@ -182,6 +186,18 @@ __global__ __launch_bounds__(SCAN_PARTS * MOE_MAX_E) void moe_scan_kernel(const 
         pos += v[u];
       }
     }
+  }
+  if (order != nullptr) {
+    const int j0 = pt * (MOE_MAX_E / SCAN_PARTS), j1 = j0 + MOE_MAX_E / SCAN_PARTS;
+    if (e < E) {
+      const int c = rows[e];
+      int before = 0;
+#pragma unroll 8
+      for (int j = j0; j < (j1 < E ? j1 : E); ++j) before += (rows[j] > c || (rows[j] == c && j < e)) ? 1 : 0;
+      atomicAdd(&rank[e], before);
+    }
+    __syncthreads();
+    if (pt == 0 && e < E) order[rank[e]] = e;
   }
 }
 
@@ -628,10 +644,10 @@ size_t artk_moe_route_workspace_bytes(int64_t T, int32_t E, int32_t k) {
   return ws.used + 256;
 }
 
-int32_t artk_moe_route(const float* router_logits, int64_t T, int32_t E, int32_t k, int32_t* topk_idx,
-                       float* topk_w, int32_t* perm, int32_t* inv_perm, int32_t* row_token,
-                       int32_t* expert_offsets, int32_t* tile_prefix, int32_t* blk_prefix,
-                       void* workspace, size_t workspace_bytes, artk_stream_t stream) {
+static int32_t moe_route(const float* router_logits, int64_t T, int32_t E, int32_t k, int32_t* topk_idx,
+                         float* topk_w, int32_t* perm, int32_t* inv_perm, int32_t* row_token,
+                         int32_t* expert_offsets, int32_t* tile_prefix, int32_t* blk_prefix, int32_t* order,
+                         void* workspace, size_t workspace_bytes, artk_stream_t stream) {
   ARTK_CHECK_ARG(router_logits && topk_idx && topk_w && perm && inv_perm && row_token &&
                      expert_offsets && tile_prefix && blk_prefix,
                  "null pointer argument");
@@ -654,11 +670,20 @@ int32_t artk_moe_route(const float* router_logits, int64_t T, int32_t E, int32_t
   ARTK_CHECK_LAUNCH();
   moe_hist_kernel<<<nb, PERM_CHUNK, 0, st>>>(topk_idx, n, E, cnt);
   ARTK_CHECK_LAUNCH();
-  moe_scan_kernel<<<1, SCAN_PARTS * MOE_MAX_E, 0, st>>>(cnt, nb, E, expert_offsets, base, tile_prefix, blk_prefix);
+  moe_scan_kernel<<<1, SCAN_PARTS * MOE_MAX_E, 0, st>>>(cnt, nb, E, expert_offsets, base, tile_prefix, blk_prefix,
+                                                          order);
   ARTK_CHECK_LAUNCH();
   moe_scatter_kernel<<<nb, PERM_CHUNK, 0, st>>>(topk_idx, n, E, k, base, perm, inv_perm, row_token);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
+}
+
+int32_t artk_moe_route(const float* router_logits, int64_t T, int32_t E, int32_t k, int32_t* topk_idx,
+                       float* topk_w, int32_t* perm, int32_t* inv_perm, int32_t* row_token,
+                       int32_t* expert_offsets, int32_t* tile_prefix, int32_t* blk_prefix,
+                       void* workspace, size_t workspace_bytes, artk_stream_t stream) {
+  return moe_route(router_logits, T, E, k, topk_idx, topk_w, perm, inv_perm, row_token, expert_offsets, tile_prefix,
+                   blk_prefix, nullptr, workspace, workspace_bytes, stream);
 }
 
 size_t artk_moe_lora_grouped_fwd_workspace_bytes(int64_t n_rows, int64_t in, int64_t out, int32_t E,
@@ -715,7 +740,7 @@ static void carve_moe_bwd(Workspace& ws, int64_t n_rows, int64_t in, int64_t out
   c.At = ws.take<uint16_t>((size_t)E * in * r);   // [E,in,r]
   c.gb = ws.take<float>((size_t)n_rows * r);
   c.gb16 = ws.take<uint16_t>((size_t)n_rows * RP);
-  c.rowp = ws.take<float>((size_t)stats_grouped_chunks(out, r, E) * n_rows * r);
+  c.rowp = ws.take<float>((size_t)stats_grouped_chunks(n_rows, out, r, E) * n_rows * r);
   c.dummy = ws.take<float>(1024);
 }
 
@@ -761,7 +786,7 @@ int32_t artk_moe_lora_grouped_bwd(const void* g, const void* x, const int32_t* g
                                  scale, 0, c.dummy, st)))
     return rc;
   {
-    StatsReduceJob ja{c.rowp, stats_grouped_chunks(out, r, E), n_rows, 1.f, c.gb, 0, c.gb16, RP, scale};
+    StatsReduceJob ja{c.rowp, stats_grouped_chunks(n_rows, out, r, E), n_rows, 1.f, c.gb, 0, c.gb16, RP, scale};
     StatsReduceJob jb{nullptr, 0, 0, 0.f, nullptr, 0, nullptr, 0, 0.f};
     if ((rc = launch_stats_reduce(ja, jb, r, st))) return rc;
   }
@@ -779,6 +804,7 @@ struct MoeSaved {
   uint16_t *A_gu, *B_gu, *A_d, *B_d;  // bf16 adapters [E,2r,H], [E,2I,2r], [E,r,I], [E,H,r]
   float *xa_gu, *xaw_d;               // x A^T [n,2r]; routing weight times h A_d^T [n,r]
   uint16_t *gu, *h;                   // gate|up [n,2I], silu(gate) up [n,I]
+  int* order;                         // experts by falling number of rows
 };
 static void carve_moe_saved(Workspace& ws, const artk_moe_experts_t& a, MoeSaved& c) {
   const size_t n = (size_t)(a.T * a.k), E = (size_t)a.E, r = (size_t)a.r, H = (size_t)a.H, I = (size_t)a.I;
@@ -790,6 +816,7 @@ static void carve_moe_saved(Workspace& ws, const artk_moe_experts_t& a, MoeSaved
   c.xaw_d = ws.take<float>(n * r);
   c.gu = ws.take<uint16_t>(n * 2 * I);
   c.h = ws.take<uint16_t>(n * I);
+  c.order = ws.take<int>(E);
 }
 struct MoeFwdScratch {
   char* route;
@@ -815,8 +842,8 @@ static void carve_moe_block_bwd(Workspace& ws, const artk_moe_experts_t& a, MoeB
   c.At_gu = ws.take<uint16_t>(E * H * 2 * r);
   c.Bt_d = ws.take<uint16_t>(E * r * H);
   c.At_d = ws.take<uint16_t>(E * I * r);
-  const size_t p_d = (size_t)stats_grouped_chunks(a.H, a.r, a.E) * r;
-  const size_t p_gu = (size_t)stats_grouped_chunks(2 * a.I, 2 * a.r, a.E) * 2 * r;
+  const size_t p_d = (size_t)stats_grouped_chunks(a.T * a.k, a.H, a.r, a.E) * r;
+  const size_t p_gu = (size_t)stats_grouped_chunks(a.T * a.k, 2 * a.I, 2 * a.r, a.E) * 2 * r;
   c.rowp = ws.take<float>((p_d > p_gu ? p_d : p_gu) * n);
   c.gb = ws.take<float>(n * 2 * r);
   c.gb16 = ws.take<uint16_t>(n * round16(2 * a.r));
@@ -869,6 +896,12 @@ size_t artk_moe_experts_bwd_workspace_bytes(const artk_moe_experts_t* a) {
   return ws.used + 256;
 }
 
+// Experts of a row tile or less are all alike to the skinny passes: no order for them (and no look-up, 1 to 4 us of
+// a 20 us launch).
+static int* moe_order(const artk_moe_experts_t* a, const MoeSaved& s) {
+  return a->T * a->k > (int64_t)a->E * ST_TILE ? s.order : nullptr;
+}
+
 static unsigned blocks256(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,
@@ -895,8 +928,8 @@ int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_
   hipStream_t st = (hipStream_t)stream;
   const int64_t n = a->T * a->k, H = a->H, I = a->I;
   const int E = a->E, r = a->r;
-  if ((rc = artk_moe_route(a->router_logits, a->T, E, a->k, a->topk_idx, a->topk_w, a->perm, a->inv_perm, a->row_token,
-                           a->offsets, a->tile_prefix, a->blk_prefix, c.route, c.route_bytes, stream)))
+  if ((rc = moe_route(a->router_logits, a->T, E, a->k, a->topk_idx, a->topk_w, a->perm, a->inv_perm, a->row_token,
+                      a->offsets, a->tile_prefix, a->blk_prefix, moe_order(a, s), c.route, c.route_bytes, stream)))
     return rc;
   {
     MoePack p{a->gate_A, a->gate_B, a->up_A, a->up_B, a->down_A, a->down_B, s.A_gu, s.B_gu, s.A_d, s.B_d,
@@ -948,6 +981,7 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
   hipStream_t st = (hipStream_t)stream;
   const int64_t n = a->T * a->k, H = a->H, I = a->I;
   const int E = a->E, r = a->r;
+  const int* order = moe_order(a, s);
   {
     SmallTransposeMulti m;
     m.n = 4;
@@ -960,10 +994,10 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
   const StatsReduceJob none{nullptr, 0, 0, 0.f, nullptr, 0, nullptr, 0, 0.f};
   // down, on the unweighted rows g[token]: g B_d per row and dB_d = s g^T (w h A_d^T) in one pass
   if ((rc = launch_stats_grouped(a->g, a->T, a->row_token, n, H, c.Bt_d, s.xaw_d, r, E, a->offsets, c.rowp, a->ddown_B,
-                                 a->scale, 0, c.dummy, st)))
+                                 a->scale, 0, c.dummy, st, order)))
     return rc;
   {
-    StatsReduceJob ja{c.rowp, stats_grouped_chunks(H, r, E), n, 1.f, c.gb, 0, c.gb16, round16(r), a->scale};
+    StatsReduceJob ja{c.rowp, stats_grouped_chunks(n, H, r, E), n, 1.f, c.gb, 0, c.gb16, round16(r), a->scale};
     ja.row_w = a->topk_w;
     ja.row_idx = a->perm;
     if ((rc = launch_stats_reduce(ja, none, r, st))) return rc;
@@ -972,17 +1006,17 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
                             r, round16(r), st)))
     return rc;
   if ((rc = launch_stats_grouped(s.h, n, nullptr, n, I, nullptr, c.gb, r, E, a->offsets, nullptr, a->ddown_A, a->scale,
-                                 1, c.dummy, st)))
+                                 1, c.dummy, st, order)))
     return rc;
   moe_silu_bwd_kernel<<<blocks256(n * I / 8), 256, 0, st>>>(s.gu, c.dhr, a->topk_w, a->perm, n * I / 8, (int)(I / 8),
                                                             c.g_gu);
   ARTK_CHECK_LAUNCH();
   // gate|up
   if ((rc = launch_stats_grouped(c.g_gu, n, nullptr, n, 2 * I, c.Bt_gu, s.xa_gu, 2 * r, E, a->offsets, c.rowp,
-                                 a->dgate_B, a->scale, 0, c.dummy, st, a->dup_B, r, I)))
+                                 a->dgate_B, a->scale, 0, c.dummy, st, order, a->dup_B, r, I)))
     return rc;
   {
-    StatsReduceJob ja{c.rowp, stats_grouped_chunks(2 * I, 2 * r, E), n,       1.f, c.gb, 0, c.gb16, round16(2 * r),
+    StatsReduceJob ja{c.rowp, stats_grouped_chunks(n, 2 * I, 2 * r, E), n, 1.f, c.gb, 0, c.gb16, round16(2 * r),
                       a->scale};
     if ((rc = launch_stats_reduce(ja, none, 2 * r, st))) return rc;
   }
@@ -990,7 +1024,7 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
                             2 * I, E, 2 * r, round16(2 * r), st)))
     return rc;
   if ((rc = launch_stats_grouped(a->x, a->T, a->row_token, n, H, nullptr, c.gb, 2 * r, E, a->offsets, nullptr,
-                                 a->dgate_A, a->scale, 1, c.dummy, st, a->dup_A, r, 0)))
+                                 a->dgate_A, a->scale, 1, c.dummy, st, order, a->dup_A, r, 0)))
     return rc;
   moe_combine_kernel<<<blocks256(a->T * H / 8), 256, 0, st>>>(c.dx_rows, a->inv_perm, nullptr, a->T * H / 8,
                                                               (int)(H / 8), a->k, (uint16_t*)a->dx);

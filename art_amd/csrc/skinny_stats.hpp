@@ -54,6 +54,7 @@ struct StatsParams {
   float* col_out2 = nullptr;
   int r_split = 0;
   int64_t c_split = 0;
+  const int* order = nullptr;  // grouped form: slab numbers in the order in which they are dispatched
 };
 
 // XOR of the 16-byte chunk index of a 256-byte tile row: row-fragment reads (one chunk of
@@ -103,8 +104,10 @@ __device__ __forceinline__ void lora_stats_body(const StatsParams& p, const int 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 31, half = lane >> 5;
-  const int slab = block / p.n_chunks, chunk = block - slab * p.n_chunks;
+  int slab = block / p.n_chunks;
+  const int chunk = block - slab * p.n_chunks;
   const bool grouped = p.offsets != nullptr;
+  if (grouped && p.order != nullptr) slab = p.order[slab];
   const int64_t t0 = grouped ? (int64_t)p.offsets[slab] : (int64_t)slab * p.rows_per_slab;
   const int64_t c0 = (int64_t)chunk * p.cc;
   const int rows_here = grouped ? p.offsets[slab + 1] - p.offsets[slab]
@@ -536,32 +539,45 @@ static inline int32_t launch_stats_multi(StatsMulti& m, bool wide_rank, hipStrea
 
 // Grouped form: slab = expert.  ROW partials go to row_part [n_chunks][n_rows][r]; the COL
 // product of each expert is written to col_out, scaled.
-static inline int stats_grouped_cc(int64_t C, int r, int E) {
+// Chunk width: the launch lasts as long as its work divided by the CUs, or as its longest expert, whichever is
+// more (half tile times as in stats_grid_cost, with twice the set-up: an expert's factor and results are its own).
+// Routing is uneven (of 8192 tokens, top-8 of 128 experts, the fullest expert gets 3 to 5 times the average), so
+// with one wide chunk per expert most CUs wait for the fullest one, unless it is dispatched first (`order`) and is
+// not too long; the estimate takes 2.5 times the average.  Measured at that size, us with the experts by index /
+// by falling length: rows of 2048 through the gather with the ROW product 112 / 71 (chunks of 512; 256: 79),
+// without it 89 / 57, 1536 columns 100 / 62 (chunks of 384; 512: 71), 768 columns 46 / 38 (chunks of 256; 384: 46).
+static inline int stats_grouped_cc(int64_t n_rows, int64_t C, int r, int E) {
   const int max_cct = r > 32 ? 2 : 4;
   const int64_t col_tiles = (C + ST_TILE - 1) / ST_TILE;
+  const double avg = (double)n_rows / E / ST_TILE, tiles = avg > 1.0 ? avg + 0.5 : 1.0;
   int best = max_cct;
-  int64_t best_cost = -1;
+  double best_cost = -1.0;
   for (int cct = max_cct; cct >= 1; --cct) {
     const int64_t n_chunks = (col_tiles + cct - 1) / cct;
-    const int64_t cost = stats_grid_cost((int64_t)E * n_chunks, 2, cct);  // a couple of row tiles per expert
-    if (best_cost < 0 || cost < best_cost) {
+    double rounds = (double)(E * n_chunks) / num_cus();
+    if (avg <= 1.0) rounds = ceil(rounds);  // (all alike: whole rounds)
+    const double total = (rounds > 1.0 ? rounds : 1.0) * (tiles * (2 * cct + 1) + 8.0);
+    const double longest = (avg > 1.0 ? 2.5 : 1.0) * tiles * (2 * cct + 1) + 8.0;
+    const double cost = total > longest ? total : longest;
+    if (best_cost < 0.0 || cost < best_cost) {
       best_cost = cost;
       best = cct;
     }
   }
   return best * ST_TILE;
 }
-static inline int stats_grouped_chunks(int64_t C, int r, int E) {
-  const int cc = stats_grouped_cc(C, r, E);
+static inline int stats_grouped_chunks(int64_t n_rows, int64_t C, int r, int E) {
+  const int cc = stats_grouped_cc(n_rows, C, r, E);
   return (int)((C + cc - 1) / cc);
 }
 static inline int32_t launch_stats_grouped(const void* X, int64_t x_rows, const int* gather, int64_t n_rows,
                                            int64_t C, const uint16_t* F, const float* Y, int r, int E,
                                            const int* offsets, float* row_part, float* col_out,
                                            float col_scale, int col_transposed, float* row_dummy,
-                                           hipStream_t st, float* col_out2 = nullptr, int r_split = 0,
-                                           int64_t c_split = 0) {
+                                           hipStream_t st, const int* order = nullptr,
+                                           float* col_out2 = nullptr, int r_split = 0, int64_t c_split = 0) {
   StatsParams p;
+  p.order = order;
   p.col_out2 = col_out2;
   p.r_split = r_split;
   p.c_split = c_split;
@@ -582,8 +598,8 @@ static inline int32_t launch_stats_grouped(const void* X, int64_t x_rows, const 
   p.R = r;
   p.rows_per_slab = 0;
   p.n_slabs = E;
-  p.cc = stats_grouped_cc(C, r, E);
-  p.n_chunks = stats_grouped_chunks(C, r, E);
+  p.cc = stats_grouped_cc(n_rows, C, r, E);
+  p.n_chunks = stats_grouped_chunks(n_rows, C, r, E);
   const unsigned grid = (unsigned)(E * p.n_chunks);
   if (gather) {
     if (r > 32)

@@ -353,3 +353,38 @@ def test_moe_parameters_changed_between_forward_and_backward(artk_lib, gpu):
             p.add_(1.0)
     for got, ref in zip(torch.autograd.grad(y, params, up), want):
         assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("E,hot", [(3, 700), (24, 4000)])
+def test_moe_experts_uneven_load(artk_lib, gpu, E, hot):
+    """More than a row tile per expert on average, so the skinny passes go by falling expert size: one expert with
+    most of the rows, one without any, the rest of equal or nearly equal size.  Gradients against the fp32 oracle,
+    2e-2 as in test_moe_experts_entry_points."""
+    T, H, I, k, r = hot, 128, 64, 2, 8
+    print("moe uneven", E, hot, flush=True)
+    g = torch.Generator().manual_seed(E)
+    rnd = lambda *s, std=1.0: (std * torch.randn(*s, generator=g)).to(torch.bfloat16)
+    x, up, logits = rnd(T, H), rnd(T, H), torch.randn(T, E, generator=g)
+    logits[:, 1] += 8.0
+    logits[:, 0] -= 50.0
+    Wgu, Wd = rnd(E, 2 * I, H, std=H ** -0.5), rnd(E, H, I, std=I ** -0.5)
+    P = {"gate_A": rnd(E, r, H, std=H ** -0.5), "gate_B": rnd(E, I, r, std=0.1), "up_A": rnd(E, r, H, std=H ** -0.5),
+         "up_B": rnd(E, I, r, std=0.1), "down_A": rnd(E, r, I, std=I ** -0.5), "down_B": rnd(E, H, r, std=0.1)}
+    ref = moe_oracle.route(logits, k)
+    off = ref["offsets"]
+    assert T * k > E * 128 and int(off[1]) == 0 and int(off[2]) == T
+    Pr = {n: p.float().requires_grad_(True) for n, p in P.items()}
+    rows = x.float()[ref["row_token"]]
+    gate = moe_oracle.grouped_lora(rows, Wgu[:, :I].float(), Pr["gate_A"], Pr["gate_B"], 0.5, off)
+    u = moe_oracle.grouped_lora(rows, Wgu[:, I:].float(), Pr["up_A"], Pr["up_B"], 0.5, off)
+    down = moe_oracle.grouped_lora(torch.nn.functional.silu(gate) * u, Wd.float(), Pr["down_A"], Pr["down_B"], 0.5, off)
+    y0 = (down[ref["inv_perm"]].view(T, k, H) * ref["topk_w"].unsqueeze(-1)).sum(1)
+    y0.backward(up.float())
+    ad = {n: p.to(gpu) for n, p in P.items()}
+    y, rt, saved = ops.moe_experts_fwd(x.to(gpu), logits.to(gpu), k, Wgu.to(gpu), Wd.to(gpu), ad, 0.5)
+    _, grads = ops.moe_experts_bwd(up.to(gpu), x.to(gpu), rt, saved, ops.transpose_batched(Wgu.to(gpu)),
+                                   ops.transpose_batched(Wd.to(gpu)), r, 0.5)
+    assert rel_l2(y.cpu().float(), y0.detach()) <= 2e-2
+    for n in P:
+        assert rel_l2(grads[n].cpu(), Pr[n].grad) <= 2e-2, n
+        assert not grads[n][0].any()   # the expert without rows
