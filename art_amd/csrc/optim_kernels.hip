@@ -143,6 +143,7 @@ struct AdamW8Params {
 constexpr int LUT_E0 = 104;                      // exponents 104 .. 127: [2^-23, 1]; smaller values share bin 0
 constexpr int LUT_HALF = (128 - LUT_E0) * 128;   // bins of one sign
 constexpr int LUT_BINS = 2 * LUT_HALF;           // ascending: negative bins first
+// (in LDS by sign bit, then magnitude, so that an index is one multiply-add)
 
 // Lower end of bin j (ascending order), -inf for the first one.
 __device__ __forceinline__ float lut_edge(int j) {
@@ -162,7 +163,7 @@ __device__ void build_lut(uint8_t* lut, const float* map, int tid, int nthreads)
   for (int j = tid * per; j < (tid + 1) * per; ++j) {
     const float e = lut_edge(j);
     while (lo < 254 && map[lo + 1] <= e) ++lo;
-    lut[j] = (uint8_t)lo;
+    lut[j < LUT_HALF ? LUT_BINS - 1 - j : j - LUT_HALF] = (uint8_t)lo;
   }
 }
 
@@ -170,7 +171,7 @@ __device__ __forceinline__ int nearest_code(const float* map, const uint8_t* lut
   const uint32_t u = __float_as_uint(x);
   int k = (int)(u >> 16 & 0x7fff) - LUT_E0 * 128;
   k = k < 0 ? 0 : (k > LUT_HALF - 1 ? LUT_HALF - 1 : k);
-  int lo = lut[(int)u < 0 ? LUT_HALF - 1 - k : LUT_HALF + k];
+  int lo = lut[k + (int)(u >> 31) * LUT_HALF];
   float cur = map[lo], next = map[lo + 1];
   while (lo < 254 && next <= x) {
     ++lo;
@@ -181,12 +182,34 @@ __device__ __forceinline__ int nearest_code(const float* map, const uint8_t* lut
   return (x - cur <= next - x) ? lo : lo + 1;
 }
 
+// x / max for the elements of a block (|x| <= max).  With max scaled to [0.5, 1) and x by the same power of two, one
+// correction of x times the correctly rounded reciprocal gives the correctly rounded quotient (Markstein): 4
+// instructions per element for the 10 of a division and no branch (one on the range of max cost 25 spilled registers
+// and twice the time).  An element that the scaling takes below the normal range is nearest to the smallest code
+// either way.  max == 0: all elements are 0; infinite: finite elements give 0, infinite ones NaN.
+struct BlockMax {
+  float d, y;
+  int e;
+  __device__ __forceinline__ explicit BlockMax(float max) {
+    const bool plain = max > 0.f && max < INFINITY;
+    e = plain ? -__builtin_amdgcn_frexp_expf(max) : 0;
+    d = plain ? __builtin_amdgcn_frexp_mantf(max) : 1.f;
+    y = plain ? 1.f / d : 0.f;
+  }
+  __device__ __forceinline__ float quotient(float x) const {
+    x = __builtin_amdgcn_ldexpf(x, e);
+    const float q = x * y;
+    return fmaf(fmaf(-q, d, x), y, q);
+  }
+};
+
 // One wave = one block of 256 elements, 4 consecutive elements per lane: 16-byte loads of parameters and
-// gradients, 4-byte loads of the codes, block maxima by wave reduction without a barrier.  Bound: HBM
-// (18 B per element; the gradient's second read after the norm comes from the Infinity Cache).  The grid
+// gradients, 4-byte loads of the codes, block maxima by wave reduction without a barrier.  18 B per
+// element, of which the gradient's second read after the norm comes from the Infinity Cache.  The grid
 // is two work-groups of 16 waves per CU that walk the blocks, so the two tables are built once per
 // work-group and not once per 256 elements.  20.2 M elements: 182 us as one work-group per block with a
-// bisection, 104 us now (2.0 -> 3.5 TB/s).
+// bisection, 104 us with the start table; the vector instructions bound it then, and quotients without divisions
+// and fewer spilled registers took another 16 us off the step (123 -> 107 us with the norm).
 constexpr int ADAM8_THREADS = 1024;
 
 __global__ __launch_bounds__(ADAM8_THREADS, 8) void adamw8bit_kernel(AdamW8Params a, int64_t n_blocks, int vec) {
@@ -240,33 +263,45 @@ __global__ __launch_bounds__(ADAM8_THREADS, 8) void adamw8bit_kernel(AdamW8Param
       mx1 = fmaxf(mx1, fabsf(m[j]));
       mx2 = fmaxf(mx2, fabsf(v[j]));
     }
-    mx1 = wave_max(mx1);
-    mx2 = wave_max(mx2);
+    mx1 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(wave_max(mx1))));
+    mx2 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(wave_max(mx2))));
+    const BlockMax q1(mx1), q2(mx2);
     if (lane == 0) {
       a.absmax1[b] = mx1;
       a.absmax2[b] = mx2;
     }
-    c1 = c2 = 0;
+    // parameters leave before the codes are searched: their registers are needed there
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       pv[j] = pv[j] + a.step_size * (m[j] / (sqrtf(v[j]) + a.eps_scaled));
       if (a.weight_decay > 0.f) pv[j] = pv[j] * (1.f - a.lr * a.weight_decay);
-      c1 |= (uint32_t)nearest_code(map1, lut1, mx1 > 0.f ? m[j] / mx1 : 0.f) << (8 * j);
-      c2 |= (uint32_t)nearest_code(map2, lut2, mx2 > 0.f ? v[j] / mx2 : 0.f) << (8 * j);
     }
     if (full) {
       *(float4*)(a.p + i) = *(float4*)pv;
       if (a.p_bf16)
         *(uint2*)(a.p_bf16 + i) = make_uint2((uint32_t)f32_to_bf16(pv[0]) | ((uint32_t)f32_to_bf16(pv[1]) << 16),
                                              (uint32_t)f32_to_bf16(pv[2]) | ((uint32_t)f32_to_bf16(pv[3]) << 16));
-      *(uint32_t*)(a.c1 + i) = c1;
-      *(uint32_t*)(a.c2 + i) = c2;
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (i + j < a.n) {
           a.p[i + j] = pv[j];
           if (a.p_bf16) a.p_bf16[i + j] = f32_to_bf16(pv[j]);
+        }
+    }
+    c1 = c2 = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      c1 |= (uint32_t)nearest_code(map1, lut1, q1.quotient(m[j])) << (8 * j);
+      c2 |= (uint32_t)nearest_code(map2, lut2, q2.quotient(v[j])) << (8 * j);
+    }
+    if (full) {
+      *(uint32_t*)(a.c1 + i) = c1;
+      *(uint32_t*)(a.c2 + i) = c2;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (i + j < a.n) {
           a.c1[i + j] = (uint8_t)(c1 >> (8 * j));
           a.c2[i + j] = (uint8_t)(c2 >> (8 * j));
         }

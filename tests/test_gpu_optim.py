@@ -133,3 +133,32 @@ def test_adamw8bit_any_code_book(artk_lib, gpu, n, book):
     assert np.allclose(t[5].cpu().numpy(), want[4], rtol=2e-6, atol=0)
     assert np.abs(t[0].cpu().numpy() - want[0]).max() <= 1e-6 * np.abs(want[0]).max()
     assert torch.equal(shadow, t[0].to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("exponents", [(-140, -100), (-66, -54), (54, 90)])
+def test_adamw8bit_block_maxima_of_any_size(artk_lib, gpu, exponents):
+    """Re-quantisation of moments whose block maxima are zero, subnormal, small or large: the quotient by the
+    maximum is taken with a scaled reciprocal.  The gradients are zero, so that the moments stay what the codes and block maxima say, times beta;
+    same bounds as test_adamw8bit_any_code_book."""
+    import numpy as np
+
+    from art_amd.optim import dynamic_code_book
+
+    print("adamw 8-bit maxima", exponents, flush=True)
+    n = 256 * 64 + 9
+    rng = np.random.default_rng(7)
+    nb = (n + 255) // 256
+    b1, b2 = dynamic_code_book(True).numpy(), dynamic_code_book(False).numpy()
+    p, g = np.zeros(n, np.float32), np.zeros(n, np.float32)
+    c1, c2 = rng.integers(0, 256, n).astype(np.uint8), rng.integers(0, 256, n).astype(np.uint8)
+    a1, a2 = (np.exp2(rng.uniform(*exponents, nb)).astype(np.float32) for _ in range(2))
+    a1[3] = a2[5] = 0.0
+    want = optim_oracle.adamw8bit_step(p, g, c1, c2, a1, a2, b1, b2, 0.0, (0.9, 0.99), 1e-8, 0.0, 3, 0.0)
+    t = [torch.from_numpy(x.copy()).to(gpu) for x in (p, g, c1, c2, a1, a2, b1, b2)]
+    shadow = torch.zeros(n, dtype=torch.bfloat16, device=gpu)
+    ops.adamw8bit_step(*t, shadow, 0.0, 0.9, 0.99, 1e-8, 0.0, 3)
+    for got, ref in ((t[2], want[1]), (t[3], want[2])):
+        d = np.abs(got.cpu().numpy().astype(int) - ref.astype(int))
+        assert (d == 0).mean() >= 0.999 and d.max() <= 1
+    assert np.allclose(t[4].cpu().numpy(), want[3], rtol=2e-6, atol=0)
+    assert np.allclose(t[5].cpu().numpy(), want[4], rtol=2e-6, atol=0)
