@@ -246,27 +246,47 @@ Tensor lora_nf4(const Tensor& x, const Tensor& packed, std::optional<Tensor> abs
 }
 
 // ---- attention over packed rows -------------------------------------------------------------------------------
-// (batch, position, head) strides of a bf16 [B, S, H, D] view whose last dimension is contiguous.
+void need_heads(const Tensor& t, const char* name) {
+  TORCH_CHECK_VALUE(t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.dim() == 4, name,
+                    ": expected a bf16 device tensor [B, S, H, D]");
+}
+
+// (batch, position, head) strides of a [B, S, H, D] view whose last dimension is contiguous.
 void strides_of(const Tensor& t, const char* name, int64_t* out) {
-  TORCH_CHECK_VALUE(t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.dim() == 4 && t.stride(3) == 1, name,
-                    ": expected a bf16 device tensor [B, S, H, D] with contiguous D");
+  TORCH_CHECK_VALUE(t.stride(3) == 1, name, ": expected a bf16 device tensor [B, S, H, D] with contiguous D");
   out[0] = t.size(0) > 1 ? t.stride(0) : 0;
   out[1] = t.stride(1);
   out[2] = t.stride(2);
 }
 
+// `t` [B, S, H, D], or a copy of it where its layout is none that the kernels address.
+Tensor addressable(const Tensor& t) {
+  const int64_t rows = (t.size(1) + 255) / 256 * 256;  // a row's tiles cover this many positions
+  bool ok = t.stride(3) == 1 && ((uintptr_t)t.data_ptr() & 15) == 0 && rows * t.stride(1) * 2 < (1ll << 31);
+  for (int i = t.size(0) > 1 ? 0 : 1; i < 3; ++i) ok = ok && t.stride(i) > 0 && t.stride(i) % 8 == 0;
+  // (not contiguous(): it returns t itself where only a pointer or the stride of a dimension of size 1 is odd)
+  return ok ? t : t.clone(at::MemoryFormat::Contiguous);
+}
+
 struct AttentionFunction : torch::autograd::Function<AttentionFunction> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& plan,
-                        double scale) {
-    int64_t st[12];
-    strides_of(q, "q", st);
-    strides_of(k, "k", st + 3);
-    strides_of(v, "v", st + 6);
+  static Tensor forward(AutogradContext* ctx, Tensor q, Tensor k, Tensor v, const Tensor& plan, double scale) {
+    need_heads(q, "q");
+    need_heads(k, "k");
+    need_heads(v, "v");
     const int64_t B = q.size(0), S = q.size(1), Hq = q.size(2), D = q.size(3), Hkv = k.size(2);
     TORCH_CHECK_VALUE(k.sizes() == at::IntArrayRef({B, S, Hkv, D}) && v.sizes() == k.sizes(),
                       "attention: inconsistent shapes");
     TORCH_CHECK_VALUE((size_t)plan.numel() >= (size_t)B * artk_attn_plan_row_stride(S), "the plan is for other rows");
     c10::OptionalDeviceGuard guard(q.device());
+    if (S % 256 != 0) {  // rows that end inside a block may have any layout; whole blocks are taken as they are
+      q = addressable(q);
+      k = addressable(k);
+      v = addressable(v);
+    }
+    int64_t st[12];
+    strides_of(q, "q", st);
+    strides_of(k, "k", st + 3);
+    strides_of(v, "v", st + 6);
     const Tensor out = make(q, {B, S, Hq, D}, at::kBFloat16), lse = make(q, {B, Hq, S}, at::kFloat);
     strides_of(out, "out", st + 9);
     check(artk_attn_fwd_rows(q.data_ptr(), k.data_ptr(), v.data_ptr(), plan.data_ptr(), B, S, (int32_t)Hq, (int32_t)Hkv,
@@ -283,15 +303,12 @@ struct AttentionFunction : torch::autograd::Function<AttentionFunction> {
     const Tensor plan = ctx->saved_data["plan"].toTensor();
     c10::OptionalDeviceGuard guard(q.device());
     const int64_t B = q.size(0), S = q.size(1), Hq = q.size(2), D = q.size(3), Hkv = k.size(2);
-    Tensor g = grads[0].to(at::kBFloat16);
-    bool plain = g.stride(3) == 1 && ((uintptr_t)g.data_ptr() & 15) == 0;
-    for (int i = 0; i < 3; ++i) plain = plain && g.stride(i) > 0 && g.stride(i) % 8 == 0;
-    if (!plain) g = g.contiguous();
+    const Tensor g = addressable(grads[0].to(at::kBFloat16));
     const Tensor dq = make(q, {B, S, Hq, D}, at::kBFloat16), dk = make(q, {B, S, Hkv, D}, at::kBFloat16),
                  dv = make(q, {B, S, Hkv, D}, at::kBFloat16);
     int64_t st[24];
     int i = 0;
-    for (const Tensor* t : {&q, &k, &v, &out, (const Tensor*)&g, &dq, &dk, &dv}) strides_of(*t, "attention", st + 3 * i++);
+    for (const Tensor* t : {&q, &k, &v, &out, &g, &dq, &dk, &dv}) strides_of(*t, "attention", st + 3 * i++);
     const Tensor ws = workspace(q, artk_attn_bwd_rows_workspace_bytes(B, S, (int32_t)Hq, (int32_t)Hkv, (int32_t)D));
     check(artk_attn_bwd_rows(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(),
                              g.data_ptr(), plan.data_ptr(), B, S, (int32_t)Hq, (int32_t)Hkv, (int32_t)D, st,
@@ -302,7 +319,7 @@ struct AttentionFunction : torch::autograd::Function<AttentionFunction> {
 };
 
 Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& plan, std::optional<double> scale) {
-  TORCH_CHECK_VALUE(q.dim() == 4, "q: expected a bf16 device tensor [B, S, H, D] with contiguous D");
+  need_heads(q, "q");
   return AttentionFunction::apply(q, k, v, plan, scale ? *scale : 1.0 / std::sqrt((double)q.size(3)));
 }
 

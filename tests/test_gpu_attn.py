@@ -335,3 +335,44 @@ def test_packed_attention_ragged_batch(artk_lib, gpu, B, S, Hq, Hkv, D, head_maj
         ref = attn_oracle.attention_grads(*(t[b] for t in data[:3]), group[b], parent[b], data[3][b])
         for got, want in zip((out, *grads), ref):
             assert torch.isfinite(got[b]).all() and rel_l2(got[b].float().cpu(), want) <= 1e-2
+
+
+LAYOUT_VIEWS = {
+    # views whose values, [2, S, H, 64], the kernels cannot address as they lie
+    "every_other_d": lambda t: torch.stack([t, t], -1).flatten(-2)[..., ::2],
+    "odd_stride": lambda t: torch.nn.functional.pad(t, (0, 3))[..., :-3],
+    "odd_pointer": lambda t: torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape),
+    "one_head_for_all": lambda t: t[:, :, :1].expand(t.shape),
+}
+
+
+@pytest.mark.parametrize("view", list(LAYOUT_VIEWS))
+@pytest.mark.parametrize("S", [1, 300])
+def test_packed_attention_any_layout(artk_lib, gpu, S, view):
+    """Rows that are no multiple of 256 may have any strides and alignment, and the upstream gradient may at any
+    length: the same bits as contiguous copies give.  Whole blocks with such strides are refused."""
+    from art_amd.attention import attention_plans, packed_attention
+    print("attention layout", S, view, flush=True)
+    make = LAYOUT_VIEWS[view]
+    g = torch.Generator().manual_seed(S)
+    data = [torch.randn(2, S, H, 64, generator=g).to(torch.bfloat16).to(gpu) for H in (4, 2, 2, 4)]
+    odd = [make(t) for t in data]
+    plain = [t.clone(memory_format=torch.contiguous_format) for t in odd]
+    ids = torch.zeros(2, S, dtype=torch.int64, device=gpu)
+    plans = attention_plans(ids, ids)
+
+    def run(q, k, v, up):
+        leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        out = packed_attention(*leaves, plans)
+        return [out.detach(), *torch.autograd.grad(out, leaves, up)]
+
+    want = run(*plain)
+    for got, ref in zip(run(*odd), want):
+        assert torch.equal(got, ref)
+    whole = [torch.randn(2, 256, H, 64, generator=g).to(torch.bfloat16).to(gpu) for H in (4, 2, 2, 4)]
+    ids = torch.zeros(2, 256, dtype=torch.int64, device=gpu)
+    plans = attention_plans(ids, ids)
+    for got, ref in zip(run(*whole[:3], make(whole[3])), run(*whole[:3], make(whole[3]).clone())):
+        assert torch.equal(got, ref)
+    with pytest.raises(ValueError):
+        packed_attention(make(whole[0]), *whole[1:3], plans)
