@@ -5,6 +5,7 @@
 // kernels take 60.  Here it is a few microseconds of C++ each way, without the interpreter lock.
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/extension.h>
 
 #include "../../include/artk.h"
@@ -15,10 +16,18 @@ using at::Tensor;
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
+// ValueError for an argument error, art_amd._lib.ArtkError for a hipError_t, as art_amd._lib.check raises them.
 void check(int32_t rc) {
   if (rc == 0) return;
-  TORCH_CHECK_VALUE(rc > 0, "artk error ", rc, ": ", artk_last_error());
-  TORCH_CHECK(false, "artk error ", rc, ": ", artk_last_error());
+  const std::string text = artk_last_error();  // (of this thread)
+  TORCH_CHECK_VALUE(rc > 0, "artk error ", rc, ": ", text);
+  py::gil_scoped_acquire gil;
+  const py::object type = py::module_::import("art_amd._lib").attr("ArtkError");
+  const py::object error = type(rc, py::bytes(text).attr("decode")("utf-8", "replace"));
+  PyErr_SetObject(type.ptr(), error.ptr());
+  python_error e;
+  e.persist();
+  throw e;
 }
 
 void need(const Tensor& t, const char* name, at::ScalarType dtype, at::IntArrayRef shape) {
@@ -326,11 +335,13 @@ Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  const auto nogil = py::call_guard<py::gil_scoped_release>();
-  m.def("lora_multi", &lora_multi, nogil, py::arg("x"), py::arg("W"), py::arg("W_t"), py::arg("A"), py::arg("B"),
-        py::arg("bias"), py::arg("scale"));
-  m.def("lora_nf4", &lora_nf4, nogil, py::arg("x"), py::arg("packed"), py::arg("absmax"), py::arg("absmax_q"),
-        py::arg("code2"), py::arg("absmax2"), py::arg("offset"), py::arg("blocksize"), py::arg("out"), py::arg("in_"),
+  // (the wrapper hands Python exceptions on as they are and releases the interpreter lock)
+  m.def("lora_multi", torch::wrap_pybind_function_no_gil(&lora_multi), py::arg("x"), py::arg("W"), py::arg("W_t"),
         py::arg("A"), py::arg("B"), py::arg("bias"), py::arg("scale"));
-  m.def("attention", &attention, nogil, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("plan"), py::arg("scale"));
+  m.def("lora_nf4", torch::wrap_pybind_function_no_gil(&lora_nf4), py::arg("x"), py::arg("packed"), py::arg("absmax"),
+        py::arg("absmax_q"), py::arg("code2"), py::arg("absmax2"), py::arg("offset"), py::arg("blocksize"),
+        py::arg("out"), py::arg("in_"), py::arg("A"), py::arg("B"), py::arg("bias"), py::arg("scale"));
+  m.def("attention", torch::wrap_pybind_function_no_gil(&attention), py::arg("q"), py::arg("k"), py::arg("v"),
+        py::arg("plan"), py::arg("scale"));
+  m.def("_check", torch::wrap_pybind_function_no_gil(&check), py::arg("rc"));
 }

@@ -100,3 +100,17 @@ def test_header_is_plain_c(tmp_path):
     r = subprocess.run([gcc, "-std=c99", "-Wall", "-Wextra", "-pedantic", "-Werror", "-I", inc, "-fsyntax-only",
                         str(src)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+def test_native_functions_raise_the_package_errors(artk_lib):
+    """A status code means the same exception whether the call went through ctypes or through the native autograd
+    functions: ValueError for an argument error, ArtkError with its code for a hipError_t."""
+    from art_amd import _lib
+
+    native = _lib.native()
+    native._check(0)
+    with pytest.raises(_lib.ArtkError, match="artk error 719") as e:
+        native._check(719)
+    assert e.value.code == 719
+    with pytest.raises(ValueError, match="artk error -1"):
+        native._check(_lib.ERR_INVALID_ARGUMENT)
