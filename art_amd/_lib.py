@@ -140,6 +140,7 @@ SIGNATURES.update({
 })
 
 _lib = None
+_native = None
 
 
 def load() -> C.CDLL:
@@ -163,14 +164,18 @@ def load() -> C.CDLL:
 
 def native():
     """The autograd functions over the C-ABI (art_amd/_native.so, built with libartk.so from
-    ``csrc/native_ops.cpp``); there is no fallback."""
+    ``csrc/native_ops.cpp``), loaded on first use; there is no fallback."""
+    global _native
+    if _native is not None:
+        return _native
     load()
     try:
-        from . import _native
+        from . import _native as module
     except ImportError as e:
         raise ImportError(f"art_amd/_native.so is not built for this Python and torch ({e}). Build it with "
                           f"`make -C {os.path.dirname(LIB_PATH)}`.") from e
-    return _native
+    _native = module
+    return module
 
 
 class ArtkError(RuntimeError):

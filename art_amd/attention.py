@@ -14,8 +14,6 @@ import torch
 
 from . import _lib, ops
 
-_native = _lib.native()
-
 ROW_MULTIPLE = 256  # plans cover rows of this granularity; positions past the end see, and are seen by, nothing
 
 
@@ -43,7 +41,7 @@ def packed_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plans: L
             raise ValueError(f"plan made for a row of {plan.S} positions, tensors have {S}")
     first = plans[0]
     if first.rows == B and all(p.batch is first.batch and p.index == b for b, p in enumerate(plans[:B])):
-        return _native.attention(q, k, v, first.batch, scale)
+        return _lib.native().attention(q, k, v, first.batch, scale)
     # plans that were made one by one: a call per row
-    outs = [_native.attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], plans[b].buf, scale) for b in range(B)]
+    outs = [_lib.native().attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], plans[b].buf, scale) for b in range(B)]
     return torch.cat(outs, 0)

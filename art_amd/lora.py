@@ -16,8 +16,6 @@ from torch import nn
 
 from . import _lib, ops
 
-_native = _lib.native()
-
 
 def _frozen_bias(bias):
     if bias is None:
@@ -33,7 +31,7 @@ def _lora_projections(x, weights, lora_As, lora_Bs, scale: float, biases):
     can be a backward."""
     graph = torch.is_grad_enabled() and any(t.requires_grad for t in (x, *lora_As, *lora_Bs))
     wts = [ops.transposed_weight(w) for w in weights] if graph else []
-    return _native.lora_multi(x, weights, wts, lora_As, lora_Bs, biases, scale)
+    return _lib.native().lora_multi(x, weights, wts, lora_As, lora_Bs, biases, scale)
 
 
 def lora_linear(x, weight, lora_A, lora_B, scale: float, bias=None):
@@ -41,8 +39,8 @@ def lora_linear(x, weight, lora_A, lora_B, scale: float, bias=None):
     bias = _frozen_bias(bias)
     if not isinstance(weight, torch.Tensor):   # an NF4Weight: the bf16 weight lives inside each call only
         w = weight
-        return _native.lora_nf4(x, w.packed, w.absmax, w.absmax_q, w.code2, w.absmax2, float(w.offset), w.blocksize,
-                                *w.shape, lora_A, lora_B, bias, float(scale))
+        return _lib.native().lora_nf4(x, w.packed, w.absmax, w.absmax_q, w.code2, w.absmax2, float(w.offset),
+                                      w.blocksize, *w.shape, lora_A, lora_B, bias, float(scale))
     return _lora_projections(x, [weight], [lora_A], [lora_B], float(scale), [bias])[0]
 
 

@@ -14,10 +14,10 @@ def pytest_configure(config):
 
 @pytest.fixture(scope="session")
 def artk_lib():
-    """The built C-ABI library; tests never build it (build() does, on the CPU box)."""
+    """The built C-ABI library; tests build only if it, or the native functions over it, are not there."""
     from art_amd import _lib
 
-    if not os.path.exists(_lib.LIB_PATH):
+    if not os.path.exists(_lib.LIB_PATH) or not os.path.exists(os.path.join(ROOT, "art_amd", "_native.so")):
         import __graft_entry__
 
         __graft_entry__.build()

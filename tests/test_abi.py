@@ -114,3 +114,26 @@ def test_native_functions_raise_the_package_errors(artk_lib):
     assert e.value.code == 719
     with pytest.raises(ValueError, match="artk error -1"):
         native._check(_lib.ERR_INVALID_ARGUMENT)
+
+
+def test_modules_import_without_the_built_libraries(tmp_path):
+    """Importing any module needs no built library (a packer or a data loader on another machine has none); the
+    first use says what is missing."""
+    import shutil
+    import subprocess
+    import sys
+
+    shutil.copytree(os.path.join(ROOT, "art_amd"), tmp_path / "art_amd", ignore=shutil.ignore_patterns("*.so", "csrc"))
+    code = """
+import art_amd, torch
+from art_amd import advantage, attention, lora, moe, optim, pack, quant, synthetic, train
+m = lora.LoRALinear(64, 64)
+try:
+    with torch.no_grad():
+        m(torch.zeros(1, 64))
+except ImportError as e:
+    assert "not built" in str(e)
+else:
+    raise SystemExit("no error")
+"""
+    subprocess.run([sys.executable, "-c", code], cwd=tmp_path, check=True, env={**os.environ, "PYTHONPATH": str(tmp_path)})
