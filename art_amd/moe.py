@@ -45,6 +45,13 @@ def grouped_lora_linear(x, W, W_t, A, B, scale, routing, use_gather: bool):
     return _GroupedLoRAFn.apply(x, W, W_t, A, B, float(scale), routing, use_gather)
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """``t``, contiguous and on the 16 bytes that the library's vector loads need (a view into a flat buffer of
+    parameters or gradients may lie anywhere)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 class _MoEExpertsFn(torch.autograd.Function):
     """The whole block (routing, three projections, gating, recombination) as one library call each way."""
 
@@ -53,7 +60,7 @@ class _MoEExpertsFn(torch.autograd.Function):
         dtype = params[0].dtype
         if dtype not in (torch.float32, torch.bfloat16) or any(p.dtype != dtype for p in params):
             dtype = torch.float32
-        adapters = {n: p.detach().to(dtype).contiguous() for n, p in zip(ops._MOE_PARAMS, params)}
+        adapters = {n: _aligned(p.detach().to(dtype)) for n, p in zip(ops._MOE_PARAMS, params)}
         y, routing, saved = ops.moe_experts_fwd(x, logits, top_k, W_gu, W_d, adapters, scale)
         ctx.save_for_backward(x, saved, Wt_gu, Wt_d)
         ctx.routing, ctx.scale = routing, scale
@@ -63,8 +70,7 @@ class _MoEExpertsFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g, _g_routing):
         x, saved, Wt_gu, Wt_d = ctx.saved_tensors
-        dx, grads = ops.moe_experts_bwd(g.contiguous(), x, ctx.routing, saved, Wt_gu, Wt_d, ctx.rank,
-                                        ctx.scale)
+        dx, grads = ops.moe_experts_bwd(_aligned(g), x, ctx.routing, saved, Wt_gu, Wt_d, ctx.rank, ctx.scale)
         return (dx,) + (None,) * 7 + tuple(grads[n].to(t) for n, t in zip(ops._MOE_PARAMS, ctx.dtypes))
 
 

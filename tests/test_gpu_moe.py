@@ -388,3 +388,31 @@ def test_moe_experts_uneven_load(artk_lib, gpu, E, hot):
     for n in P:
         assert rel_l2(grads[n].cpu(), Pr[n].grad) <= 2e-2, n
         assert not grads[n][0].any()   # the expert without rows
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_moe_block_takes_views_of_flat_buffers(artk_lib, gpu, dtype):
+    """Adapters that are views into one buffer, and an upstream gradient that is one, at any alignment: the bits of
+    the aligned call."""
+    torch.manual_seed(12)
+    mod = MoELoRAExperts(64, 64, 4, 2, r=8, lora_alpha=16, device=gpu)
+    params = [p for p in mod.parameters() if p.requires_grad]
+    with torch.no_grad():
+        for p in params:
+            p.data = p.normal_(std=0.05).to(dtype)
+    x = torch.randn(9, 64, device=gpu, dtype=torch.bfloat16, requires_grad=True)
+    logits, up = torch.randn(9, 4, device=gpu), torch.randn(9, 64, device=gpu, dtype=torch.bfloat16)
+
+    def odd(t):
+        return torch.cat([t.new_zeros(1), t.detach().flatten()])[1:].view(t.shape)
+
+    def step(up):
+        y, _ = mod(x, logits)
+        return [y.detach(), *torch.autograd.grad(y, [x] + params, up)]
+
+    want = step(up)
+    for p in params:
+        p.data = odd(p)
+    assert all(p.data_ptr() % 16 for p in params) and odd(up).data_ptr() % 16
+    for got, ref in zip(step(odd(up)), want):
+        assert torch.equal(got, ref)
