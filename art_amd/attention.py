@@ -36,6 +36,8 @@ def packed_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plans: L
     if q.dim() == 3:
         return packed_attention(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), plans[:1], scale)[0]
     B, S = q.shape[:2]
+    if len(plans) < B:
+        raise IndexError(f"{len(plans)} plans for {B} rows")
     for plan in plans[:B]:
         if not 0 <= plan.S - S < ROW_MULTIPLE:
             raise ValueError(f"plan made for a row of {plan.S} positions, tensors have {S}")

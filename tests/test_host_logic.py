@@ -119,3 +119,19 @@ def test_frozen_weight_view_is_stable_until_the_weight_changes():
     assert d is _as_vh(w32.t()) and d.dtype == torch.bfloat16
     plain = torch.randn(4, 12).to(torch.bfloat16)      # an [H, V] tensor that is not such a view
     assert torch.equal(_as_vh(plain), plain.t())
+
+
+def test_packed_attention_wants_a_plan_per_row():
+    """Fewer plans than rows are refused, also when those given were made for a batch of as many rows."""
+    from art_amd.attention import packed_attention
+
+    plans = []
+    for index in range(2):
+        plan = ops.AttnPlan()
+        plan.S, plan.index, plan.rows = 256, index, 2
+        plan.batch = plan.buf = plans[0].batch if plans else torch.empty(1 << 20, dtype=torch.uint8)
+        plans.append(plan)
+    q, kv = torch.zeros(2, 256, 2, 64, dtype=torch.bfloat16), torch.zeros(2, 256, 1, 64, dtype=torch.bfloat16)
+    for short in ([], plans[:1]):
+        with pytest.raises(IndexError):
+            packed_attention(q, kv, kv, short)
