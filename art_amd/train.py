@@ -188,6 +188,11 @@ class _FusedGRPOLossFn(torch.autograd.Function):
         (d_hidden,) = ctx.saved_tensors
         if g_loss is None:
             return (None,) * 13
+        if (torch.is_grad_enabled() or torch._C._functorch.is_legacy_batchedtensor(g_loss)
+                or torch._C._functorch.is_functorch_wrapped_tensor(g_loss)):
+            # a graph of this gradient is wanted (create_graph), or there is a batch of upstream gradients
+            # (is_grads_batched): both see torch operations only
+            return ((d_hidden * g_loss).to(d_hidden.dtype).view(ctx.shape),) + (None,) * 12
         return (ops.scale_bf16(d_hidden, g_loss.to(torch.float32)).view(ctx.shape),) + (None,) * 12
 
 

@@ -135,3 +135,23 @@ def test_packed_attention_wants_a_plan_per_row():
     for short in ([], plans[:1]):
         with pytest.raises(IndexError):
             packed_attention(q, kv, kv, short)
+
+
+def test_fused_loss_gradient_has_a_graph_and_takes_batched_upstream(monkeypatch):
+    """create_graph=True gives a gradient that depends on the upstream gradient, is_grads_batched=True takes several
+    upstream gradients in one call: both see torch operations, not the library's scaling kernel."""
+    from art_amd import train
+
+    d_hidden = torch.arange(16, dtype=torch.float32).view(2, 8).to(torch.bfloat16)
+    monkeypatch.setattr(ops, "transposed_weight", lambda w: w)
+    monkeypatch.setattr(ops, "grpo_fused", lambda *a, **k: (torch.arange(5.0), torch.zeros(2), d_hidden.clone()))
+    hidden = torch.zeros(1, 2, 8, dtype=torch.bfloat16, requires_grad=True)
+    row = torch.zeros(1, 2)
+    loss = train._FusedGRPOLossFn.apply(hidden, d_hidden, row, row, row, row, row, None, 0.2, 0.2, 0.0, 64, False)[0]
+    up = torch.tensor(2.0, requires_grad=True)
+    (g,) = torch.autograd.grad(loss, hidden, up, create_graph=True, retain_graph=True)
+    assert torch.equal(g, 2 * d_hidden.view(1, 2, 8))
+    (gg,) = torch.autograd.grad(g, up, torch.ones_like(g))
+    assert gg.item() == d_hidden.float().sum().item()
+    (batch,) = torch.autograd.grad(loss, hidden, torch.tensor([1.0, 2.0, 4.0]), is_grads_batched=True)
+    assert torch.equal(batch, torch.stack([k * d_hidden.view(1, 2, 8) for k in (1, 2, 4)]))
