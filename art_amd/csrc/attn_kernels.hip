@@ -22,8 +22,12 @@
 // one's set-up and store behind the other's tiles, and a list is made for 128
 // queries instead of 256.  Against one work-group of 8 waves per CU with three
 // stages, 16384 positions of 8 prompts of 137 + 4 x 461, 28 / 4 heads of 128:
-// forward 214 -> 174 us, dQ 291 -> 241 us, dK/dV with its sums 470 -> 330 us;
-// a dense causal row (1.1 PFLOP/s) is level.
+// forward 205 -> 154 us, dQ 279 -> 244 us, dK/dV 433 -> 297 us.  On dense causal
+// rows, where every tile comes into LDS twice as often, forward + backward are
+// 14 % faster to 5 % slower (us, 8 waves / now):
+//   heads of 128, 28 / 4: 4096 positions 617 / 619, 8192 2201 / 2103, 16384 8158 / 8281
+//   16 / 2: 8192 1216 / 1277, 12288 2701 / 2674;  16 / 16: 8192 1188 / 1230
+//   heads of 64, 14 / 2: 2048 173 / 148, 8192 724 / 684, 16384 2641 / 2308
 #include <stdlib.h>
 
 #include "common.hpp"
@@ -382,6 +386,36 @@ __device__ __forceinline__ bf16x8 tr_frag(const char* tile, const TrLane& t, int
   return __builtin_bit_cast(bf16x8, v);
 }
 
+// The same reads from byte offsets that the caller prepares once.  A row is a power of two of bytes long, so the chunk
+// of step s (row fragments) or of the 32 columns dt (transposed ones) can be XORed into the offset of chunk 0, and
+// rows 16 apart have the same swizzle.  One register per row instead of one per address: where those are short.
+template <int D>
+__device__ __forceinline__ int frag_base(int row, int h) {
+  return row * AttnTile<D>::ROW + ((h ^ AttnTile<D>::swz(row)) << 4);
+}
+__device__ __forceinline__ bf16x8 frag_at(const char* tile, int base, int s) {
+  return *(const bf16x8*)(tile + (base ^ (s << 5)));
+}
+struct TrBase {
+  int lo, hi;  // rows k0 + 4h + {0..3} and 8 below
+};
+template <int D>
+__device__ __forceinline__ TrBase tr_base(const TrLane& t, int k0) {
+  using T = AttnTile<D>;
+  const int r0 = k0 + t.row_off, r1 = r0 + 8, c = (t.dcol & 4) * 2;
+  return {r0 * T::ROW + (((t.dcol >> 3) ^ T::swz(r0)) << 4) + c, r1 * T::ROW + (((t.dcol >> 3) ^ T::swz(r1)) << 4) + c};
+}
+// Slab u (16 rows each) below k0, columns 32 dt ..
+template <int D>
+__device__ __forceinline__ bf16x8 tr_at(const char* tile, const TrBase& b, int u, int dt) {
+  const char* slab = tile + u * 16 * AttnTile<D>::ROW;
+  const shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_ptr)(slab + (b.lo ^ (dt << 6))));
+  const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_ptr)(slab + (b.hi ^ (dt << 6))));
+  typedef __attribute__((__vector_size__(8 * sizeof(short)))) short shortx8;
+  const shortx8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_bit_cast(bf16x8, v);
+}
+
 // attn_smem_note: the kernels below track the completion of their LDS DMA by hand (wait_vmcnt
 // before the barrier that publishes a stage).  Two things would make the compiler drain every
 // outstanding DMA instead, serialising the ring: a second LDS variable in the kernel (it then
@@ -417,9 +451,15 @@ constexpr int ATT_THREADS = 2 * ATT_BM;  // forward and dQ: a wave per 32 querie
 // (query head, query block) of a work-group of the forward and dQ kernels.  A unit is the work-groups of
 // the heads that share one key/value head and query block: they read the same K and V tiles, so a unit
 // runs on one XCD (block b is placed on XCD b % 8), its heads one after the other; long blocks first.
-__device__ __forceinline__ bool attn_block(int Hq, int Hkv, int nQb, const int* order, int& hq, int& qb) {
+// There are 8 / Hkv XCDs to a key/value head.  With `turn` they are dealt the blocks forwards and backwards by
+// turns, or the first of them would get the longest block of every turn (of 64 blocks of a dense causal row and 2
+// key/value heads: 5 % more work than the average; forward 281 -> 270 us at 8192 positions, 16 / 2 heads of 128).
+// The dK/dV kernel, whose work-groups are not ordered by their work alone, did not gain.
+__device__ __forceinline__ bool attn_block(int Hq, int Hkv, int nQb, const int* order, bool turn, int& hq, int& qb) {
   const int rep = Hq / Hkv;
-  const int x = blockIdx.x & 7, loc = blockIdx.x >> 3;
+  const int loc = blockIdx.x >> 3;
+  int x = blockIdx.x & 7;
+  if (turn && 8 % Hkv == 0 && (loc / rep & 1)) x = (8 / Hkv - 1 - x / Hkv) * Hkv + x % Hkv;
   const int unit = (loc / rep) * 8 + x;
   const int hkv = unit % Hkv;
   hq = hkv * rep + loc % rep;
@@ -490,7 +530,7 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_fwd_kernel(
   const TrLane tr(lane);
   const int row = blockIdx.y;
   int hq, qb;
-  if (!attn_block(p.Hq, p.Hkv, p.nQb, attn_row(p.order, p.plan_stride, row), hq, qb)) return;
+  if (!attn_block(p.Hq, p.Hkv, p.nQb, attn_row(p.order, p.plan_stride, row), true, hq, qb)) return;
   const int hkv = hq / (p.Hq / p.Hkv);
   const int q = qb * ATT_BM + wave * 32 + n;
   const int qc = q < p.S ? q : p.S - 1;  // queries past the end compute something that is not stored
@@ -670,14 +710,24 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_fwd_kernel(
 //   the same with 16 / 2 heads (one round):                                         15: 497, 30: 423, 40: 409, 100: 425
 //   8192 positions, 28 / 4 heads (one round):                                       15: 319, 30: 337, 40: 350, 100: 376
 //   16384 positions, one prompt of 900 + 2 x 7700, 16 / 2 heads (one round):        15: 2994, 30: 2483, 40: 2368, 100: 2273
+// A share also costs evenness: its steps come in pieces that the dispatch order (longest list first) does not rank.
+// Where the lists are long on average the set-up is small against one head's steps, and every work-group takes one
+// head: from 16 tiles on where the key blocks are less than two rounds, from 100 on where they are more (there the
+// partial sums of all heads weigh more).  Backward and forward in us, shares / one head each, by the average list:
+//   one round:  8: 427 / 460 (8192 positions, 28 / 4 heads), 12: 315 / 316 (16384, 14 / 2 of 64), 19: 423 / 407 (4096,
+//     28 / 4), 24: 540 / 529 (16384, 14 / 2 of 64), 39: 1375 / 1342 (8192, 28 / 4), 64: 1326 / 1267 (8192, 16 / 2)
+//   two rounds (16384, 28 / 4): 19: 1416 / 1590, 30: 2055 / 2230, 72: 4700 / 4820, 128: 8207 / 8139
 struct AttnKvSplit {
   const int* total;  // steps of one head, from the plan
+  int long_total;    // total from which lists are long
   int heads_all;     // query heads
   int div;           // steps of a share = total * heads_all / div
   int light_max;     // >= 0 (artk_attn_bwd_tuning): all heads where they make at most this many steps, else one
   __device__ __forceinline__ int heads(int cnt, int rep, int64_t stride, int row) const {
     if (light_max >= 0) return cnt * rep <= light_max ? rep : 1;
-    const int steps = (int)((int64_t)*attn_row(total, stride, row) * heads_all / div);
+    const int all = *attn_row(total, stride, row);
+    if (all >= long_total) return 1;
+    const int steps = (int)((int64_t)all * heads_all / div);
     int g = cnt > 0 ? steps / cnt : rep;
     g = g < 1 ? 1 : (g > rep ? rep : g);
     const int groups = (rep + g - 1) / g;
@@ -724,7 +774,7 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kern
   const TrLane tr(lane);
   const int row = blockIdx.y;
   int hq, qb;
-  if (!attn_block(p.Hq, p.Hkv, p.nQb, attn_row(p.order, p.plan_stride, row), hq, qb)) return;
+  if (!attn_block(p.Hq, p.Hkv, p.nQb, attn_row(p.order, p.plan_stride, row), true, hq, qb)) return;
   const int hkv = hq / (p.Hq / p.Hkv);
   const int q = qb * ATT_BM + wave * 32 + n;
   const int qc = q < p.S ? q : p.S - 1;  // queries past the end compute something that is not stored
@@ -853,21 +903,22 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kern
 // ---- dK, dV: 64 keys x some query heads of a group per work-group, lane = key ------------
 // 4 wavefronts = 2 key groups of 32 x 2 halves of each 64-query tile; two work-groups per CU (D = 64:
 // three), so that the exp2 / convert work, the DMA latency and the set-up of one overlap the MFMAs of the
-// other.  The two waves of a key group keep separate accumulators, added through LDS at the end.  The K
-// and V rows of the block stay in LDS for the whole kernel (their fragments are re-read per tile: keeping
-// them in registers would push a wave past 256 registers).
+// other.  The two waves of a key group keep separate accumulators, added through LDS at the end.
+// Bound: LDS.  A wave's step of 32 MFMAs reads 48 KiB of fragments and its share of the DMA writes 8, about 90 bytes per
+// clock and CU.  So the wave's K rows stay in registers for the whole kernel (40 KiB to read; the V rows, which do
+// not fit beside them, are re-read from LDS), with one register per fragment row instead of one per address to make
+// the room.  Dense causal rows, dK/dV in us before / after: 16384 positions, 28 / 4 heads of 128: 4225 / 4010; 8192,
+// 16 / 2: 665 / 633; the row of the header's figures: 314 / 297.  (The next tile's DMA issued in two halves, each as
+// soon as its tile is free, measured level.)
 // A work-group that does not take all heads of its group writes fp32 partial sums, which
 // attn_kv_reduce_kernel adds in a fixed order.
-// LDS stage: Q tile, dO tile (64 queries), and lse2 / delta / group / parent codes
-// of those queries.  D = 128 has room for one stage per work-group only.
+// LDS: Q tile, dO tile (64 queries), lse2 / delta / group / parent codes of those queries, and the block's K and V rows.
 template <int D>
 struct AttnQStage {
   using T = AttnTile<D>;
   static constexpr int DO_OFF = T::BYTES;
   static constexpr int ROW_OFF = 2 * T::BYTES;
-  static constexpr int STAGE = ROW_OFF + 1024;
-  static constexpr int NSTAGE = 1;
-  static constexpr int KV_OFF = NSTAGE * STAGE;          // K block, then V block
+  static constexpr int KV_OFF = ROW_OFF + 1024;          // K block, then V block
   static constexpr int LDS = KV_OFF + 2 * T::BYTES;
 };
 
@@ -920,7 +971,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
   const TrLane tr(lane);
   const int brow = blockIdx.y;
   int hq, kb;
-  if (!attn_block(p.Hq, p.Hkv, p.nKb2, attn_row(p.orderT, p.plan_stride, brow), hq, kb)) return;
+  if (!attn_block(p.Hq, p.Hkv, p.nKb2, attn_row(p.orderT, p.plan_stride, brow), false, hq, kb)) return;
   const int rep = p.Hq / p.Hkv;
   const int hkv = hq / rep, share = hq - hkv * rep;
   const int key = kb * ATT_BK2 + kg * 32 + n;
@@ -954,16 +1005,10 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
     attn_issue_kv_block<D>(smem + G::KV_OFF, kb * ATT_BK2, attn_head_rsrc<D>(p.K + brow * p.k_bs + (int64_t)hkv * p.k_hs, p.k_ss, p.S),
                            attn_head_rsrc<D>(p.V + brow * p.v_bs + (int64_t)hkv * p.v_hs, p.v_ss, p.S), voff_k, voff_v, p.k_ss, p.v_ss, wave);
   }
-  __syncthreads();  // s_list
-  auto* list_lds = s_list;
-  // step IT of the flattened (head, visible query tile) sequence
-#define ATTN_ISSUE(IT, STG)                                                                          \
-  do {                                                                                               \
-    const int hi_ = (IT) / cnt, ti_ = (IT) - hi_ * cnt;                                               \
-    attn_issue_q<D>(smem + (STG) * G::STAGE, hq + hi_,                                                \
-                    __builtin_amdgcn_readfirstlane(list_lds[ti_] & 0x3fff) * ATT_BQ2, q_row, do_row, \
-                    rsrc_row, voff_q, voff_do, p, wave, lane);                                        \
-  } while (0)
+  const int total = cnt * nheads;
+  if (total > 0)  // the first tile of the flattened (head, visible query tile) sequence
+    attn_issue_q<D>(smem, hq, __builtin_amdgcn_readfirstlane(list[0] & 0x3fff) * ATT_BQ2, q_row, do_row, rsrc_row,
+                    voff_q, voff_do, p, wave, lane);
 
   floatx16 dk[D / 32], dv[D / 32];
 #pragma unroll
@@ -971,45 +1016,73 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
 #pragma unroll
     for (int j = 0; j < 16; ++j) dk[dt][j] = dv[dt][j] = 0.f;
 
-  // this wave's keys inside the resident K / V blocks
-  const char* kblk = smem + G::KV_OFF;
-  const char* vblk = kblk + T::BYTES;
-  const int krow = 32 * kg + n;
-
-  const int total = cnt * nheads;
   pin_loaded(gk);
-  if (total > 0) ATTN_ISSUE(0, 0);
-  int ti = 0;
+  wait_vmcnt<0>();
+  barrier_lds_only();  // the list, the block's K and V rows and the first tile are there
+  const char* const vblk = smem + G::KV_OFF + T::BYTES;
+  const int krow = 32 * kg + n;  // this wave's keys inside the block
+  bf16x8 kf[D / 16];
+#pragma unroll
+  for (int s = 0; s < D / 16; ++s) kf[s] = T::row_frag(smem + G::KV_OFF, krow, s, h);
+#pragma unroll
+  for (int s = 0; s < D / 16; ++s) pin_loaded(kf[s]);
+  int bq = frag_base<D>(32 * qh + n, h), bv = frag_base<D>(krow, h);
+  TrBase bt = tr_base<D>(tr, 32 * qh);
+  int ti = 0, head = hq;
   for (int it = 0; it < total; ++it) {
-    if (G::NSTAGE == 1 && it > 0) {
+    if (it > 0) {
       barrier_lds_only();  // every wave is done with the tile before
-      ATTN_ISSUE(it, 0);
+      attn_issue_q<D>(smem, head, __builtin_amdgcn_readfirstlane(s_list[ti] & 0x3fff) * ATT_BQ2, q_row, do_row, rsrc_row,
+                      voff_q, voff_do, p, wave, lane);
+      wait_vmcnt<0>();
+      barrier_lds_only();
     }
-    wait_vmcnt<0>();
-    barrier_lds_only();
-    if (G::NSTAGE > 1 && it + 1 < total) ATTN_ISSUE(it + 1, (it + 1) & 1);
     const int entry = __builtin_amdgcn_readfirstlane(s_list[ti]);
-    ti = ti + 1 == cnt ? 0 : ti + 1;
+    if (++ti == cnt) {
+      ti = 0;
+      ++head;
+    }
     const int q0 = (entry & 0x3fff) * ATT_BQ2;
     const bool active = (entry >> (16 + wave)) & 1;        // this wave's keys x query half
     const bool partial = !((entry >> (24 + wave)) & 1);
-    const char* st = smem + (G::NSTAGE > 1 ? it & 1 : 0) * G::STAGE;
-    const char* dot = st + G::DO_OFF;
-    const float* r_lse2 = (const float*)(st + G::ROW_OFF);
+    const char* dot = smem + G::DO_OFF;
+    const float* r_lse2 = (const float*)(smem + G::ROW_OFF);
     const float* r_delta = r_lse2 + 64;
     const int* r_gc = (const int*)(r_lse2 + 128);
     const int* r_pc = r_gc + 64;
     if (!active) continue;
+    // (or the addresses of all reads are kept in registers of their own)
+    pin_loaded(bq);
+    pin_loaded(bv);
+    pin_loaded(bt.lo);
+    pin_loaded(bt.hi);
 
     floatx16 sc, dp;
 #pragma unroll
     for (int j = 0; j < 16; ++j) sc[j] = dp[j] = 0.f;
+    {
+      // fragments two steps ahead of the MFMAs that use them (LDS latency; more would not fit the registers)
+      constexpr int NS = D / 16, PF = 2;
+      bf16x8 qf[NS], of[NS], vf[NS];
 #pragma unroll
-    for (int s = 0; s < D / 16; ++s) {
-      sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(T::row_frag(st, 32 * qh + n, s, h),
-                                                   T::row_frag(kblk, krow, s, h), sc, 0, 0, 0);
-      dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(T::row_frag(dot, 32 * qh + n, s, h),
-                                                   T::row_frag(vblk, krow, s, h), dp, 0, 0, 0);
+      for (int s = 0; s < PF; ++s) {
+        qf[s] = frag_at(smem, bq, s);
+        of[s] = frag_at(dot, bq, s);
+        vf[s] = frag_at(vblk, bv, s);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x100, 3 * PF, 0);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        if (s + PF < NS) {
+          qf[s + PF] = frag_at(smem, bq, s + PF);
+          of[s + PF] = frag_at(dot, bq, s + PF);
+          vf[s + PF] = frag_at(vblk, bv, s + PF);
+        }
+        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[s], kf[s], sc, 0, 0, 0);
+        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(of[s], vf[s], dp, 0, 0, 0);
+        if (s + PF < NS) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+      }
     }
     bf16x8 pf[2], dsf[2];
 #pragma unroll
@@ -1039,14 +1112,11 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
     for (int u = 0; u < 2; ++u) {
 #pragma unroll
       for (int dt = 0; dt < D / 32; ++dt) {
-        dv[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag<D>(dot, tr, 32 * qh + 16 * u, 32 * dt), pf[u],
-                                                         dv[dt], 0, 0, 0);
-        dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag<D>(st, tr, 32 * qh + 16 * u, 32 * dt), dsf[u],
-                                                         dk[dt], 0, 0, 0);
+        dv[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_at<D>(dot, bt, u, dt), pf[u], dv[dt], 0, 0, 0);
+        dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_at<D>(smem, bt, u, dt), dsf[u], dk[dt], 0, 0, 0);
       }
     }
   }
-#undef ATTN_ISSUE
 
   // add the accumulators of the two query halves: the upper waves park theirs in
   // LDS ([key group][register][lane], conflict-free), the lower waves add and store
@@ -1391,7 +1461,9 @@ int32_t artk_attn_bwd_rows(const void* q, const void* k, const void* v, const vo
     const int slots = num_cus() * (D == 64 ? 3 : 2);  // resident work-groups
     p.split.total = pl.total2;
     p.split.heads_all = (int)(B * Hq);   // (rows of a batch are taken to be alike)
-    p.split.div = B * pl.nKb2 * Hkv >= 2 * slots ? slots * 3 / 2 : slots * 4;
+    const bool two_rounds = B * pl.nKb2 * Hkv >= 2 * slots;
+    p.split.div = two_rounds ? slots * 3 / 2 : slots * 4;
+    p.split.long_total = (two_rounds ? 100 : 16) * pl.nKb2;
     p.split.light_max = g_light_max_override;  // artk_attn_bwd_tuning
   }
   const dim3 grid_q(attn_grid(Hq, Hkv, pl.nQb), (unsigned)B), grid_kv(attn_grid(Hq, Hkv, pl.nKb2), (unsigned)B);

@@ -298,6 +298,22 @@ def test_attn_bwd_mixed_light_and_heavy_key_blocks(artk_lib, gpu):
     assert rel_l2(results[64][0].float(), results[0][0].float()) <= 4e-3
 
 
+@pytest.mark.parametrize("S,Hq,Hkv,D", [(1792, 7, 1, 64), (2304, 7, 1, 64), (2304, 4, 2, 128), (2304, 2, 2, 128)])
+def test_attn_dense_causal_row(artk_lib, gpu, S, Hq, Hkv, D):
+    """One conversation: the lists of 28 key blocks average 14.5 query tiles (several heads per work-group of dK/dV), those
+    of 36 average 18.5 (one); 18 query blocks do not divide by the XCDs that share a key/value head."""
+    print("attention dense row", S, Hq, Hkv, D, flush=True)
+    q, k, v = make_qkv(S + Hq, S, Hq, Hkv, D)
+    d_out = torch.randn(S, Hq, D, generator=torch.Generator().manual_seed(S)).to(torch.bfloat16)
+    ids = torch.zeros(S, dtype=torch.int64)
+    ref = attn_oracle.attention_grads(q, k, v, ids, ids, d_out)
+    plan = ops.attn_plan(ids.to(gpu), ids.to(gpu))
+    qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
+    out, lse = ops.attn_fwd(qd, kd, vd, plan)
+    for got, want in zip((out, *ops.attn_bwd(qd, kd, vd, out, lse, d_out.to(gpu), plan)), ref):
+        assert rel_l2(got.float().cpu(), want) <= 1e-2
+
+
 @pytest.mark.parametrize("B,S,Hq,Hkv,D,head_major", [
     (3, 5, 2, 1, 64, False),       # a handful of positions (one alone has a zero gradient, no relative error)
     (2, 65, 4, 4, 128, True),      # one head per group; one position in the second key tile
