@@ -742,7 +742,9 @@ struct AttnBwdParams {
   float* lse2;                      // [Hq][Sp]  lse * log2(e), Sp = S rounded up to a multiple of 256
   float* delta;                     // [Hq][Sp]
   uint16_t *dQ, *dK, *dV;
-  float *pK, *pV;                   // [Hq/Hkv][Sp][Hkv][D] partial sums per share (grouped-query heads only)
+  float *pK, *pV;                   // [rows of the launch][Hq/Hkv][Sp][Hkv][D] partial sums per share (grouped-query
+                                    // heads only)
+  int row0;                         // dK/dV kernel and its reduction: first row of the launch
   int64_t plan_stride, q_bs, k_bs, v_bs, o_bs, do_bs, dq_bs, dk_bs, dv_bs;  // per row of the batch (blockIdx.y)
   int64_t o_ss, o_hs;
   int64_t q_ss, q_hs, k_ss, k_hs, v_ss, v_hs, do_ss, do_hs, dq_ss, dq_hs, dk_ss, dk_hs, dv_ss, dv_hs;
@@ -969,7 +971,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
   const int n = lane & 31, h = lane >> 5;
   const int kg = wave & 1, qh = wave >> 1;
   const TrLane tr(lane);
-  const int brow = blockIdx.y;
+  const int brow = p.row0 + blockIdx.y;
   int hq, kb;
   if (!attn_block(p.Hq, p.Hkv, p.nKb2, attn_row(p.orderT, p.plan_stride, brow), false, hq, kb)) return;
   const int rep = p.Hq / p.Hkv;
@@ -1145,7 +1147,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
   if (qh == 1 || key >= p.S) return;
 
   if (per < rep) {
-    const int64_t o = (((((int64_t)brow * rep + share) * p.Sp + key) * p.Hkv + hkv) * D) + 4 * h;
+    const int64_t o = (((((int64_t)blockIdx.y * rep + share) * p.Sp + key) * p.Hkv + hkv) * D) + 4 * h;
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
@@ -1182,7 +1184,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
 // index order; 4 elements per thread.
 __global__ __launch_bounds__(256) void attn_kv_reduce_kernel(AttnBwdParams p, int D) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int d4 = D / 4, brow = blockIdx.y, rep = p.Hq / p.Hkv;
+  const int d4 = D / 4, brow = p.row0 + blockIdx.y, rep = p.Hq / p.Hkv;
   const int64_t n = (int64_t)p.Sp * p.Hkv * d4;
   const int c = (int)(i % d4);
   const int hh = (int)((i / d4) % p.Hkv);
@@ -1190,8 +1192,8 @@ __global__ __launch_bounds__(256) void attn_kv_reduce_kernel(AttnBwdParams p, in
   if (s >= p.S) return;
   const int per = p.split.heads(attn_row(p.cntT, p.plan_stride, brow)[s / ATT_BK2], rep, p.plan_stride, brow);
   if (per == rep) return;  // written directly by the dK/dV kernel
-  const floatx4* pk = (const floatx4*)p.pK + (int64_t)brow * rep * n + i;
-  const floatx4* pv = (const floatx4*)p.pV + (int64_t)brow * rep * n + i;
+  const floatx4* pk = (const floatx4*)p.pK + (int64_t)blockIdx.y * rep * n + i;
+  const floatx4* pv = (const floatx4*)p.pV + (int64_t)blockIdx.y * rep * n + i;
   floatx4 a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
   for (int r = 0; r * per < rep; ++r) {
     a += pk[(int64_t)r * n];
@@ -1375,13 +1377,25 @@ int32_t artk_attn_fwd(const void* q, const void* k, const void* v, const void* p
 
 struct AttnBwdScratch {
   float *delta, *lse2, *pk, *pv;
+  int64_t kv_rows;
 };
+// Rows of a batch whose dK and dV are computed by one launch.  The partial sums of grouped-query heads are two fp32 arrays
+// of q's shape, so the rows of a batch share 448 MiB of them (what 16384 positions of 28 heads of 128 need), or what one
+// row needs.  Half of that costs 5 % of the backward of 8 rows of 2048 (663 -> 695 us), whose launches no longer fill
+// the GPU.
+static int64_t attn_kv_rows(int64_t B, int64_t S, int Hq, int Hkv, int D) {
+  if (Hq == Hkv || B <= 0 || S <= 0 || Hq <= 0 || D <= 0) return B;
+  const int64_t most = (448ll << 20) / (attn_padded(S) * Hq * D * 8);
+  const int64_t launches = most > 0 ? (B + most - 1) / most : B;
+  return (B + launches - 1) / launches;
+}
 static void carve_attn_bwd(Workspace& ws, int64_t B, int64_t S, int Hq, int Hkv, int D, AttnBwdScratch& c) {
-  const size_t n = (size_t)(B * attn_padded(S) * Hq);
-  c.delta = ws.take<float>(n);
-  c.lse2 = ws.take<float>(n);
-  c.pk = Hq != Hkv ? ws.take<float>(n * D) : nullptr;
-  c.pv = Hq != Hkv ? ws.take<float>(n * D) : nullptr;
+  const size_t row = (size_t)(attn_padded(S) * Hq);
+  c.delta = ws.take<float>(B * row);
+  c.lse2 = ws.take<float>(B * row);
+  c.kv_rows = attn_kv_rows(B, S, Hq, Hkv, D);
+  c.pk = Hq != Hkv ? ws.take<float>(c.kv_rows * row * D) : nullptr;
+  c.pv = Hq != Hkv ? ws.take<float>(c.kv_rows * row * D) : nullptr;
 }
 size_t artk_attn_bwd_rows_workspace_bytes(int64_t B, int64_t S, int32_t Hq, int32_t Hkv, int32_t D) {
   Workspace ws(nullptr, 0);
@@ -1457,16 +1471,7 @@ int32_t artk_attn_bwd_rows(const void* q, const void* k, const void* v, const vo
   p.nKb2 = pl.nKb2;
   p.scale = scale;
   p.scale_log2e = scale * LOG2E;
-  {
-    const int slots = num_cus() * (D == 64 ? 3 : 2);  // resident work-groups
-    p.split.total = pl.total2;
-    p.split.heads_all = (int)(B * Hq);   // (rows of a batch are taken to be alike)
-    const bool two_rounds = B * pl.nKb2 * Hkv >= 2 * slots;
-    p.split.div = two_rounds ? slots * 3 / 2 : slots * 4;
-    p.split.long_total = (two_rounds ? 100 : 16) * pl.nKb2;
-    p.split.light_max = g_light_max_override;  // artk_attn_bwd_tuning
-  }
-  const dim3 grid_q(attn_grid(Hq, Hkv, pl.nQb), (unsigned)B), grid_kv(attn_grid(Hq, Hkv, pl.nKb2), (unsigned)B);
+  const dim3 grid_q(attn_grid(Hq, Hkv, pl.nQb), (unsigned)B);
   prof_begin(PROF_ATTN_BWD_Q, st);
   if (D == 128)
     attn_bwd_dq_kernel<128><<<grid_q, ATT_THREADS, 0, st>>>(p);
@@ -1474,17 +1479,29 @@ int32_t artk_attn_bwd_rows(const void* q, const void* k, const void* v, const vo
     attn_bwd_dq_kernel<64><<<grid_q, ATT_THREADS, 0, st>>>(p);
   prof_end(PROF_ATTN_BWD_Q, st);
   ARTK_CHECK_LAUNCH();
-  prof_begin(PROF_ATTN_BWD_KV, st);
-  if (D == 128)
-    attn_bwd_kv_kernel<128><<<grid_kv, 256, 0, st>>>(p);
-  else
-    attn_bwd_kv_kernel<64><<<grid_kv, 256, 0, st>>>(p);
-  prof_end(PROF_ATTN_BWD_KV, st);
-  ARTK_CHECK_LAUNCH();
-  if (Hq != Hkv) {
-    const int64_t n4 = (int64_t)p.Sp * Hkv * (D / 4);
-    attn_kv_reduce_kernel<<<dim3((unsigned)((n4 + 255) / 256), (unsigned)B), 256, 0, st>>>(p, D);
+  for (int64_t row0 = 0; row0 < B; row0 += c.kv_rows) {
+    const int64_t rows = B - row0 < c.kv_rows ? B - row0 : c.kv_rows;
+    const int slots = num_cus() * (D == 64 ? 3 : 2);  // resident work-groups
+    const bool two_rounds = rows * pl.nKb2 * Hkv >= 2 * slots;
+    p.row0 = (int)row0;
+    p.split.total = pl.total2;
+    p.split.long_total = (two_rounds ? 100 : 16) * pl.nKb2;
+    p.split.heads_all = (int)(rows * Hq);   // (rows of a batch are taken to be alike)
+    p.split.div = two_rounds ? slots * 3 / 2 : slots * 4;
+    p.split.light_max = g_light_max_override;  // artk_attn_bwd_tuning
+    const dim3 grid_kv(attn_grid(Hq, Hkv, pl.nKb2), (unsigned)rows);
+    prof_begin(PROF_ATTN_BWD_KV, st);
+    if (D == 128)
+      attn_bwd_kv_kernel<128><<<grid_kv, 256, 0, st>>>(p);
+    else
+      attn_bwd_kv_kernel<64><<<grid_kv, 256, 0, st>>>(p);
+    prof_end(PROF_ATTN_BWD_KV, st);
     ARTK_CHECK_LAUNCH();
+    if (Hq != Hkv) {
+      const int64_t n4 = (int64_t)p.Sp * Hkv * (D / 4);
+      attn_kv_reduce_kernel<<<dim3((unsigned)((n4 + 255) / 256), (unsigned)rows), 256, 0, st>>>(p, D);
+      ARTK_CHECK_LAUNCH();
+    }
   }
   return ARTK_OK;
 }

@@ -137,3 +137,16 @@ else:
     raise SystemExit("no error")
 """
     subprocess.run([sys.executable, "-c", code], cwd=tmp_path, check=True, env={**os.environ, "PYTHONPATH": str(tmp_path)})
+
+
+def test_attention_workspace_does_not_grow_with_the_batch(artk_lib):
+    """The fp32 partial sums of dK and dV (two arrays of q's shape) are not carved for all rows of a batch at once:
+    448 MiB are shared, or what one row needs.  The two statistics per query and head are."""
+    size = artk_lib.artk_attn_bwd_rows_workspace_bytes
+    S, Hq, Hkv, D = 16384, 28, 4, 128
+    stats, sums = 2 * 4 * S * Hq, 2 * 4 * S * Hq * D
+    assert size(1, S, Hq, Hkv, D) - stats - sums < 4096
+    assert size(16, S, Hq, Hkv, D) - 16 * stats - sums < 4096
+    short = 1024
+    assert size(64, short, Hq, Hkv, D) - 64 * 2 * 4 * short * Hq < (448 << 20) + 4096
+    assert size(0, 0, Hq, Hkv, D) > 0 and size(1, 0, Hq, Hkv, D) > 0   # (refused by the call itself)

@@ -353,6 +353,29 @@ def test_packed_attention_ragged_batch(artk_lib, gpu, B, S, Hq, Hkv, D, head_maj
             assert torch.isfinite(got[b]).all() and rel_l2(got[b].float().cpu(), want) <= 1e-2
 
 
+def test_attn_batch_backward_in_several_launches(artk_lib, gpu):
+    """Three rows whose partial sums of dK and dV do not fit the shared scratch together: two launches, of two rows and
+    of one, and each row's gradients are those of a call of its own (to the rounding of another order of heads)."""
+    from art_amd.attention import attention_plans, packed_attention
+    B, S, Hq, Hkv, D = 3, 8000, 28, 4, 128
+    assert 2 * 2 * 4 * 8192 * Hq * D <= 448 << 20 < 3 * 2 * 4 * 8192 * Hq * D
+    print("attention batch", B, S, Hq, Hkv, D, flush=True)
+    g = torch.Generator(device=gpu).manual_seed(5)
+    data = [torch.randn(B, S, H, D, generator=g, device=gpu).to(torch.bfloat16) for H in (Hq, Hkv, Hkv, Hq)]
+    ids = [synthetic.packed_row_ids(70 + b, S, 1 + b, 100, 2, 600) for b in range(B)]
+    group, parent = (torch.stack([i[j] for i in ids]).to(gpu) for j in (0, 1))
+
+    def grads(rows):
+        leaves = [t[rows].detach().requires_grad_(True) for t in data[:3]]
+        return torch.autograd.grad(packed_attention(*leaves, attention_plans(group[rows], parent[rows])), leaves,
+                                   data[3][rows])
+
+    batch = grads(slice(None))
+    for b in range(B):
+        for got, want in zip(batch, grads(slice(b, b + 1))):
+            assert rel_l2(got[b].float(), want[0].float()) <= 4e-3
+
+
 LAYOUT_VIEWS = {
     # views whose values, [2, S, H, 64], the kernels cannot address as they lie
     "every_other_d": lambda t: torch.stack([t, t], -1).flatten(-2)[..., ::2],
