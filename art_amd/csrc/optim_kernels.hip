@@ -186,7 +186,7 @@ __device__ __forceinline__ int nearest_code(const float* map, const uint8_t* lut
 // correction of x times the correctly rounded reciprocal gives the correctly rounded quotient (Markstein): 4
 // instructions per element for the 10 of a division and no branch (one on the range of max cost 25 spilled registers
 // and twice the time).  An element that the scaling takes below the normal range is nearest to the smallest code
-// either way.  max == 0: all elements are 0; infinite: finite elements give 0, infinite ones NaN.
+// either way.  Infinite max: finite elements give 0, infinite ones NaN.  Zero or NaN: see the kernel.
 struct BlockMax {
   float d, y;
   int e;
@@ -249,7 +249,7 @@ __global__ __launch_bounds__(ADAM8_THREADS, 8) void adamw8bit_kernel(AdamW8Param
         }
     }
     const float s1 = a.absmax1[b], s2 = a.absmax2[b];
-    float m[4], v[4], mx1 = 0.f, mx2 = 0.f;
+    float m[4], v[4], mx1, mx2;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       m[j] = v[j] = 0.f;
@@ -260,8 +260,9 @@ __global__ __launch_bounds__(ADAM8_THREADS, 8) void adamw8bit_kernel(AdamW8Param
         m[j] = m[j] * a.beta1 + (1.f - a.beta1) * gc;
         v[j] = v[j] * a.beta2 + (1.f - a.beta2) * gc * gc;
       }
-      mx1 = fmaxf(mx1, fabsf(m[j]));
-      mx2 = fmaxf(mx2, fabsf(v[j]));
+      // (fmaxf passes over NaN: the maximum is NaN only where the whole block is)
+      mx1 = j == 0 ? fabsf(m[j]) : fmaxf(mx1, fabsf(m[j]));
+      mx2 = j == 0 ? fabsf(v[j]) : fmaxf(mx2, fabsf(v[j]));
     }
     mx1 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(wave_max(mx1))));
     mx2 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(wave_max(mx2))));
@@ -289,6 +290,9 @@ __global__ __launch_bounds__(ADAM8_THREADS, 8) void adamw8bit_kernel(AdamW8Param
           if (a.p_bf16) a.p_bf16[i + j] = f32_to_bf16(pv[j]);
         }
     }
+    // a block without a positive maximum holds the code of 0, also for NaN
+    if (!(mx1 > 0.f)) m[0] = m[1] = m[2] = m[3] = 0.f;
+    if (!(mx2 > 0.f)) v[0] = v[1] = v[2] = v[3] = 0.f;
     c1 = c2 = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {

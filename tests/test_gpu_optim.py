@@ -162,3 +162,34 @@ def test_adamw8bit_block_maxima_of_any_size(artk_lib, gpu, exponents):
         assert (d == 0).mean() >= 0.999 and d.max() <= 1
     assert np.allclose(t[4].cpu().numpy(), want[3], rtol=2e-6, atol=0)
     assert np.allclose(t[5].cpu().numpy(), want[4], rtol=2e-6, atol=0)
+
+
+def test_adamw8bit_non_finite_gradients(artk_lib, gpu):
+    """Codes and block maxima where gradients are not finite (fresh moments): a block of NaN keeps NaN as its maximum and
+    the code of 0; NaN among zeros leaves a maximum of 0 and codes of 0; NaN and infinities among numbers get code 1, and
+    next to an infinity a finite element is 0."""
+    import numpy as np
+
+    from art_amd.optim import dynamic_code_book
+
+    print("adamw 8-bit non-finite", flush=True)
+    books = [dynamic_code_book(s).numpy() for s in (True, False)]
+    zero = [int(optim_oracle.nearest_code(b, np.zeros(1, np.float32))[0]) for b in books]
+    n = 4 * 256 + 17
+    g = np.zeros(n, np.float32)
+    g[:256] = g[4 * 256:] = np.nan      # a whole block, and a last block that is not full
+    g[[256 + 3, 256 + 70, 511]] = np.nan
+    g[512:1024] = 0.01
+    g[512 + 5] = np.inf
+    g[768 + 7] = np.nan
+    t = [torch.zeros(n, device=gpu), torch.from_numpy(g).to(gpu)]
+    t += [torch.full((n,), z, dtype=torch.uint8, device=gpu) for z in zero] + [torch.zeros(5, device=gpu) for _ in range(2)]
+    t += [torch.from_numpy(b).to(gpu) for b in books]
+    ops.adamw8bit_step(*t, torch.zeros(n, dtype=torch.bfloat16, device=gpu), 1e-3, 0.9, 0.99, 1e-8, 0.0, 1)
+    for codes, maxima, z, one in zip(t[2:4], t[4:6], zero, (np.float32(1e-3), np.float32(1e-6))):
+        c, a = codes.cpu().numpy(), maxima.cpu().numpy()
+        want = np.full(n, z)
+        want[768:1024] = 255
+        want[[512 + 5, 768 + 7]] = 1
+        assert (c == want).all()
+        assert np.isnan(a[0]) and a[1] == 0 and np.isinf(a[2]) and np.isclose(a[3], one, rtol=1e-5) and a[4] == 0
