@@ -740,7 +740,7 @@ static void carve_moe_bwd(Workspace& ws, int64_t n_rows, int64_t in, int64_t out
   c.At = ws.take<uint16_t>((size_t)E * in * r);   // [E,in,r]
   c.gb = ws.take<float>((size_t)n_rows * r);
   c.gb16 = ws.take<uint16_t>((size_t)n_rows * RP);
-  c.rowp = ws.take<float>((size_t)stats_grouped_chunks(n_rows, out, r, E) * n_rows * r);
+  c.rowp = ws.take<float>((size_t)stats_grouped_chunks(n_rows, out, r, E, false) * n_rows * r);
   c.dummy = ws.take<float>(1024);
 }
 
@@ -786,7 +786,7 @@ int32_t artk_moe_lora_grouped_bwd(const void* g, const void* x, const int32_t* g
                                  scale, 0, c.dummy, st)))
     return rc;
   {
-    StatsReduceJob ja{c.rowp, stats_grouped_chunks(n_rows, out, r, E), n_rows, 1.f, c.gb, 0, c.gb16, RP, scale};
+    StatsReduceJob ja{c.rowp, stats_grouped_chunks(n_rows, out, r, E, false), n_rows, 1.f, c.gb, 0, c.gb16, RP, scale};
     StatsReduceJob jb{nullptr, 0, 0, 0.f, nullptr, 0, nullptr, 0, 0.f};
     if ((rc = launch_stats_reduce(ja, jb, r, st))) return rc;
   }
@@ -842,8 +842,8 @@ static void carve_moe_block_bwd(Workspace& ws, const artk_moe_experts_t& a, MoeB
   c.At_gu = ws.take<uint16_t>(E * H * 2 * r);
   c.Bt_d = ws.take<uint16_t>(E * r * H);
   c.At_d = ws.take<uint16_t>(E * I * r);
-  const size_t p_d = (size_t)stats_grouped_chunks(a.T * a.k, a.H, a.r, a.E) * r;
-  const size_t p_gu = (size_t)stats_grouped_chunks(a.T * a.k, 2 * a.I, 2 * a.r, a.E) * 2 * r;
+  const size_t p_d = (size_t)stats_grouped_chunks(a.T * a.k, a.H, a.r, a.E, true) * r;
+  const size_t p_gu = (size_t)stats_grouped_chunks(a.T * a.k, 2 * a.I, 2 * a.r, a.E, true) * 2 * r;
   c.rowp = ws.take<float>((p_d > p_gu ? p_d : p_gu) * n);
   c.gb = ws.take<float>(n * 2 * r);
   c.gb16 = ws.take<uint16_t>(n * round16(2 * a.r));
@@ -982,6 +982,7 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
   const int64_t n = a->T * a->k, H = a->H, I = a->I;
   const int E = a->E, r = a->r;
   const int* order = moe_order(a, s);
+  const StatsBlock down{order}, gate_up_B{order, a->dup_B, r, I}, gate_up_A{order, a->dup_A, r, 0};
   {
     SmallTransposeMulti m;
     m.n = 4;
@@ -994,10 +995,10 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
   const StatsReduceJob none{nullptr, 0, 0, 0.f, nullptr, 0, nullptr, 0, 0.f};
   // down, on the unweighted rows g[token]: g B_d per row and dB_d = s g^T (w h A_d^T) in one pass
   if ((rc = launch_stats_grouped(a->g, a->T, a->row_token, n, H, c.Bt_d, s.xaw_d, r, E, a->offsets, c.rowp, a->ddown_B,
-                                 a->scale, 0, c.dummy, st, order)))
+                                 a->scale, 0, c.dummy, st, &down)))
     return rc;
   {
-    StatsReduceJob ja{c.rowp, stats_grouped_chunks(n, H, r, E), n, 1.f, c.gb, 0, c.gb16, round16(r), a->scale};
+    StatsReduceJob ja{c.rowp, stats_grouped_chunks(n, H, r, E, true), n, 1.f, c.gb, 0, c.gb16, round16(r), a->scale};
     ja.row_w = a->topk_w;
     ja.row_idx = a->perm;
     if ((rc = launch_stats_reduce(ja, none, r, st))) return rc;
@@ -1006,17 +1007,17 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
                             r, round16(r), st)))
     return rc;
   if ((rc = launch_stats_grouped(s.h, n, nullptr, n, I, nullptr, c.gb, r, E, a->offsets, nullptr, a->ddown_A, a->scale,
-                                 1, c.dummy, st, order)))
+                                 1, c.dummy, st, &down)))
     return rc;
   moe_silu_bwd_kernel<<<blocks256(n * I / 8), 256, 0, st>>>(s.gu, c.dhr, a->topk_w, a->perm, n * I / 8, (int)(I / 8),
                                                             c.g_gu);
   ARTK_CHECK_LAUNCH();
   // gate|up
   if ((rc = launch_stats_grouped(c.g_gu, n, nullptr, n, 2 * I, c.Bt_gu, s.xa_gu, 2 * r, E, a->offsets, c.rowp,
-                                 a->dgate_B, a->scale, 0, c.dummy, st, order, a->dup_B, r, I)))
+                                 a->dgate_B, a->scale, 0, c.dummy, st, &gate_up_B)))
     return rc;
   {
-    StatsReduceJob ja{c.rowp, stats_grouped_chunks(n, 2 * I, 2 * r, E), n, 1.f, c.gb, 0, c.gb16, round16(2 * r),
+    StatsReduceJob ja{c.rowp, stats_grouped_chunks(n, 2 * I, 2 * r, E, true), n, 1.f, c.gb, 0, c.gb16, round16(2 * r),
                       a->scale};
     if ((rc = launch_stats_reduce(ja, none, 2 * r, st))) return rc;
   }
@@ -1024,7 +1025,7 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
                             2 * I, E, 2 * r, round16(2 * r), st)))
     return rc;
   if ((rc = launch_stats_grouped(a->x, a->T, a->row_token, n, H, nullptr, c.gb, 2 * r, E, a->offsets, nullptr,
-                                 a->dgate_A, a->scale, 1, c.dummy, st, order, a->dup_A, r, 0)))
+                                 a->dgate_A, a->scale, 1, c.dummy, st, &gate_up_A)))
     return rc;
   moe_combine_kernel<<<blocks256(a->T * H / 8), 256, 0, st>>>(c.dx_rows, a->inv_perm, nullptr, a->T * H / 8,
                                                               (int)(H / 8), a->k, (uint16_t*)a->dx);

@@ -28,6 +28,15 @@ constexpr int ST_ROW_BYTES = ST_TILE * 2;             // 256
 constexpr int ST_TILE_BYTES = ST_TILE * ST_ROW_BYTES;  // 32 KiB
 constexpr int ST_STAGES = 3;
 
+// What the passes of a whole expert block add to the grouped form.  Two projections may be stacked along the rank
+// (e < r_split: the first one) and, in the plain layout, along the columns (c < c_split): each gets its own array and
+// the blocks that mix them, which belong to nobody, are not stored.  r_split == 0: one array.
+struct StatsBlock {
+  const int* order = nullptr;  // slab numbers in the order in which they are dispatched (nullptr: by number)
+  float* col_out2 = nullptr;
+  int r_split = 0;
+  int64_t c_split = 0;
+};
 struct StatsParams {
   const uint16_t* X;
   int64_t T, C;
@@ -48,13 +57,7 @@ struct StatsParams {
   float col_scale;
   int col_transposed;
   int64_t x_rows;     // rows of X (grouped form: bound of the descriptor)
-  // Grouped form, two projections stacked along the rank (e < r_split: the first one) and, in the
-  // plain layout, along the columns (c < c_split): each gets its own array and the blocks that mix
-  // them, which belong to nobody, are not stored.  r_split == 0: one array.
-  float* col_out2 = nullptr;
-  int r_split = 0;
-  int64_t c_split = 0;
-  const int* order = nullptr;  // grouped form: slab numbers in the order in which they are dispatched
+  StatsBlock block = {};  // BLOCK only
 };
 
 // XOR of the 16-byte chunk index of a 256-byte tile row: row-fragment reads (one chunk of
@@ -90,7 +93,9 @@ __device__ __forceinline__ bf16x8 st_tr_frag(const char* tile, int lane, int k0,
 // operation, the ring included): each wave fetches the 32 indices of its own rows of row tile
 // q into a private slot, NST row tiles ahead of the first tile that needs them, ordered
 // (p % 8) 4 + p / 8 so that a lane reads the 8 it needs as two 16-byte LDS loads.
-template <int NTE, int NCT, int NST, bool GATHER>
+// (BLOCK is a form of its own: its tests and index products cost the other callers 2 to 6 us a launch, 17 -> 21 us for
+// 300 tokens)
+template <int NTE, int NCT, int NST, bool GATHER, bool BLOCK = false>
 __device__ __forceinline__ void lora_stats_body(const StatsParams& p, const int block) {
   constexpr int CC = NCT * ST_TILE;
   constexpr int FPITCH = CC + 8;  // halfwords; +16 bytes: rows e land in different banks
@@ -107,7 +112,8 @@ __device__ __forceinline__ void lora_stats_body(const StatsParams& p, const int 
   int slab = block / p.n_chunks;
   const int chunk = block - slab * p.n_chunks;
   const bool grouped = p.offsets != nullptr;
-  if (grouped && p.order != nullptr) slab = p.order[slab];
+  if constexpr (BLOCK)
+    if (p.block.order != nullptr) slab = p.block.order[slab];
   const int64_t t0 = grouped ? (int64_t)p.offsets[slab] : (int64_t)slab * p.rows_per_slab;
   const int64_t c0 = (int64_t)chunk * p.cc;
   const int rows_here = grouped ? p.offsets[slab + 1] - p.offsets[slab]
@@ -320,31 +326,36 @@ __device__ __forceinline__ void lora_stats_body(const StatsParams& p, const int 
                               acc_col[ct][et][4 * q + 3]};
           if (!grouped) {
             *(floatx4*)(p.col_part + ((int64_t)slab * p.C + c) * R + e0) = v;
-          } else if (!p.col_transposed) {
-            if (p.r_split == 0) {
+          } else if (!BLOCK || p.block.r_split == 0) {
+            if (!p.col_transposed) {
               *(floatx4*)(p.col_out + ((int64_t)slab * p.C + c) * R + e0) = v * p.col_scale;
-            } else if (c < p.c_split) {
-              if (e0 < p.r_split)
-                *(floatx4*)(p.col_out + ((int64_t)slab * p.c_split + c) * p.r_split + e0) = v * p.col_scale;
-            } else if (e0 >= p.r_split) {
-              *(floatx4*)(p.col_out2 + ((int64_t)slab * (p.C - p.c_split) + c - p.c_split) * (R - p.r_split) + e0 -
-                          p.r_split) = v * p.col_scale;
-            }
-          } else {
-            float* dst = p.col_out + ((int64_t)slab * (p.r_split ? p.r_split : R) + e0) * p.C + c;
-            if (p.r_split && e0 >= p.r_split)
-              dst = p.col_out2 + ((int64_t)slab * (R - p.r_split) + e0 - p.r_split) * p.C + c;
+            } else {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) dst[k * p.C] = v[k] * p.col_scale;
+              for (int k = 0; k < 4; ++k) p.col_out[((int64_t)slab * R + e0 + k) * p.C + c] = v[k] * p.col_scale;
+            }
+          } else if constexpr (BLOCK) {
+            const StatsBlock& two = p.block;
+            if (p.col_transposed) {
+              float* dst = e0 < two.r_split ? p.col_out + ((int64_t)slab * two.r_split + e0) * p.C + c
+                                            : two.col_out2 + ((int64_t)slab * (R - two.r_split) + e0 - two.r_split) * p.C + c;
+#pragma unroll
+              for (int k = 0; k < 4; ++k) dst[k * p.C] = v[k] * p.col_scale;
+            } else if (c < two.c_split) {
+              if (e0 < two.r_split)
+                *(floatx4*)(p.col_out + ((int64_t)slab * two.c_split + c) * two.r_split + e0) = v * p.col_scale;
+            } else if (e0 >= two.r_split) {
+              *(floatx4*)(two.col_out2 + ((int64_t)slab * (p.C - two.c_split) + c - two.c_split) * (R - two.r_split) + e0 -
+                          two.r_split) = v * p.col_scale;
+            }
           }
         }
     }
   }
 }
 
-template <int NTE, int NCT, int NST, bool GATHER>
+template <int NTE, int NCT, int NST, bool GATHER, bool BLOCK = false>
 __global__ __launch_bounds__(256) void lora_stats_kernel(StatsParams p) {
-  lora_stats_body<NTE, NCT, NST, GATHER>(p, (int)blockIdx.x);
+  lora_stats_body<NTE, NCT, NST, GATHER, BLOCK>(p, (int)blockIdx.x);
 }
 
 // Several independent passes (the upstream gradients of projections that share an input) in one
@@ -546,7 +557,8 @@ static inline int32_t launch_stats_multi(StatsMulti& m, bool wide_rank, hipStrea
 // not too long; the estimate takes 2.5 times the average.  Measured at that size, us with the experts by index /
 // by falling length: rows of 2048 through the gather with the ROW product 112 / 71 (chunks of 512; 256: 79),
 // without it 89 / 57, 1536 columns 100 / 62 (chunks of 384; 512: 71), 768 columns 46 / 38 (chunks of 256; 384: 46).
-static inline int stats_grouped_cc(int64_t n_rows, int64_t C, int r, int E) {
+// A caller without an order for the experts (`block` false) assumes a couple of row tiles for each.
+static inline int stats_grouped_cc(int64_t n_rows, int64_t C, int r, int E, bool block) {
   const int max_cct = r > 32 ? 2 : 4;
   const int64_t col_tiles = (C + ST_TILE - 1) / ST_TILE;
   const double avg = (double)n_rows / E / ST_TILE, tiles = avg > 1.0 ? avg + 0.5 : 1.0;
@@ -554,11 +566,16 @@ static inline int stats_grouped_cc(int64_t n_rows, int64_t C, int r, int E) {
   double best_cost = -1.0;
   for (int cct = max_cct; cct >= 1; --cct) {
     const int64_t n_chunks = (col_tiles + cct - 1) / cct;
-    double rounds = (double)(E * n_chunks) / num_cus();
-    if (avg <= 1.0) rounds = ceil(rounds);  // (all alike: whole rounds)
-    const double total = (rounds > 1.0 ? rounds : 1.0) * (tiles * (2 * cct + 1) + 8.0);
-    const double longest = (avg > 1.0 ? 2.5 : 1.0) * tiles * (2 * cct + 1) + 8.0;
-    const double cost = total > longest ? total : longest;
+    double cost;
+    if (block) {
+      double rounds = (double)(E * n_chunks) / num_cus();
+      if (avg <= 1.0) rounds = ceil(rounds);  // (all alike: whole rounds)
+      const double total = (rounds > 1.0 ? rounds : 1.0) * (tiles * (2 * cct + 1) + 8.0);
+      const double longest = (avg > 1.0 ? 2.5 : 1.0) * tiles * (2 * cct + 1) + 8.0;
+      cost = total > longest ? total : longest;
+    } else {
+      cost = (double)stats_grid_cost((int64_t)E * n_chunks, 2, cct);
+    }
     if (best_cost < 0.0 || cost < best_cost) {
       best_cost = cost;
       best = cct;
@@ -566,21 +583,17 @@ static inline int stats_grouped_cc(int64_t n_rows, int64_t C, int r, int E) {
   }
   return best * ST_TILE;
 }
-static inline int stats_grouped_chunks(int64_t n_rows, int64_t C, int r, int E) {
-  const int cc = stats_grouped_cc(n_rows, C, r, E);
+static inline int stats_grouped_chunks(int64_t n_rows, int64_t C, int r, int E, bool block) {
+  const int cc = stats_grouped_cc(n_rows, C, r, E, block);
   return (int)((C + cc - 1) / cc);
 }
 static inline int32_t launch_stats_grouped(const void* X, int64_t x_rows, const int* gather, int64_t n_rows,
                                            int64_t C, const uint16_t* F, const float* Y, int r, int E,
                                            const int* offsets, float* row_part, float* col_out,
                                            float col_scale, int col_transposed, float* row_dummy,
-                                           hipStream_t st, const int* order = nullptr,
-                                           float* col_out2 = nullptr, int r_split = 0, int64_t c_split = 0) {
+                                           hipStream_t st, const StatsBlock* block = nullptr) {
   StatsParams p;
-  p.order = order;
-  p.col_out2 = col_out2;
-  p.r_split = r_split;
-  p.c_split = c_split;
+  if (block) p.block = *block;
   p.X = (const uint16_t*)X;
   p.T = n_rows;
   p.C = C;
@@ -598,20 +611,27 @@ static inline int32_t launch_stats_grouped(const void* X, int64_t x_rows, const 
   p.R = r;
   p.rows_per_slab = 0;
   p.n_slabs = E;
-  p.cc = stats_grouped_cc(n_rows, C, r, E);
-  p.n_chunks = stats_grouped_chunks(n_rows, C, r, E);
+  p.cc = stats_grouped_cc(n_rows, C, r, E, block != nullptr);
+  p.n_chunks = stats_grouped_chunks(n_rows, C, r, E, block != nullptr);
   const unsigned grid = (unsigned)(E * p.n_chunks);
-  if (gather) {
-    if (r > 32)
-      lora_stats_kernel<2, 2, 2, true><<<grid, 256, 0, st>>>(p);
-    else
-      lora_stats_kernel<1, 4, 3, true><<<grid, 256, 0, st>>>(p);
-  } else {
-    if (r > 32)
-      lora_stats_kernel<2, 2, 2, false><<<grid, 256, 0, st>>>(p);
-    else
-      lora_stats_kernel<1, 4, 3, false><<<grid, 256, 0, st>>>(p);
-  }
+  auto launch = [&](auto is_block) {
+    constexpr bool BLOCK = decltype(is_block)::value;
+    if (gather) {
+      if (r > 32)
+        lora_stats_kernel<2, 2, 2, true, BLOCK><<<grid, 256, 0, st>>>(p);
+      else
+        lora_stats_kernel<1, 4, 3, true, BLOCK><<<grid, 256, 0, st>>>(p);
+    } else {
+      if (r > 32)
+        lora_stats_kernel<2, 2, 2, false, BLOCK><<<grid, 256, 0, st>>>(p);
+      else
+        lora_stats_kernel<1, 4, 3, false, BLOCK><<<grid, 256, 0, st>>>(p);
+    }
+  };
+  if (block)
+    launch(std::true_type{});
+  else
+    launch(std::false_type{});
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }
