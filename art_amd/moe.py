@@ -62,15 +62,17 @@ class _MoEExpertsFn(torch.autograd.Function):
             dtype = torch.float32
         adapters = {n: _aligned(p.detach().to(dtype)) for n, p in zip(ops._MOE_PARAMS, params)}
         y, routing, saved = ops.moe_experts_fwd(x, logits, top_k, W_gu, W_d, adapters, scale)
-        ctx.save_for_backward(x, saved, Wt_gu, Wt_d)
-        ctx.routing, ctx.scale = routing, scale
+        ctx.save_for_backward(x, saved)
+        # the module's transposed weights outlive the call: as saved tensors, hooks that move activations to the host
+        # would copy them for every block
+        ctx.routing, ctx.scale, ctx.frozen = routing, scale, (Wt_gu, Wt_d)
         ctx.rank, ctx.dtypes = params[0].shape[1], [p.dtype for p in params]   # (their values are in `saved`)
         return y, routing
 
     @staticmethod
     def backward(ctx, g, _g_routing):
-        x, saved, Wt_gu, Wt_d = ctx.saved_tensors
-        dx, grads = ops.moe_experts_bwd(_aligned(g), x, ctx.routing, saved, Wt_gu, Wt_d, ctx.rank, ctx.scale)
+        x, saved = ctx.saved_tensors
+        dx, grads = ops.moe_experts_bwd(_aligned(g), x, ctx.routing, saved, *ctx.frozen, ctx.rank, ctx.scale)
         return (dx,) + (None,) * 7 + tuple(grads[n].to(t) for n, t in zip(ops._MOE_PARAMS, ctx.dtypes))
 
 

@@ -416,3 +416,32 @@ def test_moe_block_takes_views_of_flat_buffers(artk_lib, gpu, dtype):
     assert all(p.data_ptr() % 16 for p in params) and odd(up).data_ptr() % 16
     for got, ref in zip(step(odd(up)), want):
         assert torch.equal(got, ref)
+
+
+def test_moe_block_hooks_see_no_frozen_weights(artk_lib, gpu):
+    """Hooks that move saved tensors to the host (torch.autograd.graph.save_on_cpu) see the expert block's activations, not
+    its weights or their transposed copies; the gradients are the same bits.  On a stream that is not the default one."""
+    torch.manual_seed(14)
+    mod = MoELoRAExperts(128, 64, 4, 2, r=8, lora_alpha=16, device=gpu)
+    params = [p for p in mod.parameters() if p.requires_grad]
+    x = torch.randn(9, 128, device=gpu, dtype=torch.bfloat16, requires_grad=True)
+    logits, up = torch.randn(9, 4, device=gpu), torch.randn(9, 128, device=gpu, dtype=torch.bfloat16)
+
+    def step():
+        y, _ = mod(x, logits)
+        return [y.detach(), *torch.autograd.grad(y, [x] + params, up)]
+
+    want = step()
+    seen = []
+
+    def pack(t):
+        seen.append(tuple(t.shape))
+        return t.cpu()
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side), torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.to(gpu)):
+        got = step()
+    side.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert (9, 128) in seen and not any(len(s) == 3 for s in seen)
