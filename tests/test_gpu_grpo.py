@@ -279,6 +279,37 @@ def test_fused_all_or_no_rows_active(artk_lib, gpu, density):
         assert metrics["mask_count"].item() == T - 1  # the last position's mask shifts out
 
 
+@pytest.mark.parametrize("skip", [False, True])
+@pytest.mark.parametrize("H,V", [(64, 40000), (320, 152064)])
+def test_fused_few_rows_many_k_splits(artk_lib, gpu, H, V, skip):
+    """One or two tiles of d_hidden over a vocabulary long enough for more than 16 K splits (19 and 74 of at least 32
+    steps), an odd number of positions in several rows, and an upstream gradient that is not 1."""
+    B, S, up = 3, 71, 1.75
+    assert V // 64 // 17 >= 32
+    print(f"fused few rows H={H} V={V} skip={skip}", flush=True)
+    case = synthetic.make_grpo_case("t", H, B * S, H, V, B, B, 0.5)
+    for name in ("hidden", "tokens", "assistant_mask", "advantages", "weights", "noise"):
+        t = getattr(case, name)
+        setattr(case, name, t.view(B, S, *t.shape[2:]))
+    new = grpo_oracle.calculate_logprobs(case.lm_head.float().t(), case.hidden.float(),
+                                         grpo_oracle.shift_tensor(case.tokens, 0), S)
+    case.logprobs = torch.full_like(new, float("nan"))
+    case.logprobs[:, 1:] = torch.where(case.assistant_mask[:, 1:], new[:, :-1] + case.noise[:, :-1], float("nan"))
+    ref = grpo_oracle.loss_and_grad(case.hidden, case.lm_head, case.tokens, case.logprobs, case.advantages,
+                                    case.assistant_mask, case.weights, chunk_size=S)
+    hidden = case.hidden.to(gpu).requires_grad_(True)
+    loss, metrics, logprob = fused_grpo_loss(
+        hidden, case.lm_head.to(gpu), case.tokens.to(gpu), case.logprobs.to(gpu), case.advantages.to(gpu),
+        case.assistant_mask.to(gpu), case.weights.to(gpu), skip_inactive=skip)
+    loss.backward(torch.tensor(up, device=gpu))
+    assert abs(loss.item() - ref["loss"].item()) <= LOSS_TOL * abs(ref["loss"].item())
+    assert metrics["mask_count"].item() == grpo_oracle.shift_tensor(case.assistant_mask, False).sum().item()
+    done = ~torch.isnan(logprob.cpu())
+    assert done.all() or skip
+    assert (logprob.cpu() - ref["logprobs"])[done].abs().max().item() <= LP_TOL
+    assert rel_l2(hidden.grad.float().cpu(), up * ref["d_hidden"]) <= GRAD_TOL
+
+
 @pytest.mark.parametrize("T,H,V,n_traj,chunk_tokens,density,beta",
                          [(512, 256, 8192, 4, 4096, 0.5, 0.0), (1024, 128, 4096, 8, 256, 0.3, 0.0),
                           (768, 192, 8000, 4, 256, 0.5, 0.05), (512, 128, 4096, 4, 256, 0.0, 0.0),

@@ -386,3 +386,37 @@ def test_saved_tensor_hooks_see_activations_only(artk_lib, gpu):
     assert all(torch.equal(a, b) for a, b in zip(got, want))
     assert (torch.bfloat16, (192, 128)) in seen and (torch.bfloat16, (128, 192)) not in seen
     assert not any(dtype == torch.uint8 for dtype, _ in seen)
+
+
+def test_native_functions_on_another_stream(artk_lib, gpu):
+    """The projections and packed attention, forward and backward, on a stream that is not the default one while the
+    default stream is busy: inputs made on that stream, the bits of the default stream's results."""
+    from art_amd import attention
+    from art_amd.lora import FusedLoRALinear, LoRALinear
+
+    torch.manual_seed(8)
+    layers = [LoRALinear(256, o, device=gpu) for o in (256, 64, 64)]
+    for m in layers:
+        m.lora_B.data.normal_(std=0.05)
+    fused = FusedLoRALinear(layers)
+    ids = torch.zeros(2, 300, dtype=torch.int64, device=gpu)
+    host = torch.randn(2, 300, 256, dtype=torch.bfloat16)
+    params = [p for m in layers for p in (m.lora_A, m.lora_B)]
+
+    def step(x):
+        x = x.detach().requires_grad_(True)
+        q, k, v = (t.view(2, 300, -1, 64) for t in fused(x))
+        out = attention.packed_attention(q, k, v, attention.attention_plans(ids, ids))
+        return [out.detach(), *torch.autograd.grad(out.float().square().sum(), [x] + params)]
+
+    want = step(host.to(gpu))
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    busy = torch.randn(4096, 4096, device=gpu)
+    for _ in range(20):
+        busy = busy @ busy * 1e-3
+    with torch.cuda.stream(side):
+        got = step(host.to(gpu, non_blocking=True))
+    side.synchronize()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
