@@ -13,38 +13,6 @@ from torch import nn
 from . import ops
 
 
-class _GroupedLoRAFn(torch.autograd.Function):
-    """y_rows = per-expert LoRA linear of the sorted (token, expert) rows."""
-
-    @staticmethod
-    def forward(ctx, x, W, W_t, A, B, scale, routing, use_gather):
-        gather = routing.row_token if use_gather else None
-        A16 = A.detach().to(torch.bfloat16).contiguous()
-        B16 = B.detach().to(torch.bfloat16).contiguous()
-        y, xa = ops.moe_lora_grouped_fwd(x, gather, W, A16, B16, scale, routing)
-        ctx.save_for_backward(x, W_t, A16, B16, xa)
-        ctx.routing, ctx.scale, ctx.use_gather = routing, scale, use_gather
-        ctx.dtypes = (A.dtype, B.dtype)
-        return y
-
-    @staticmethod
-    def backward(ctx, g):
-        x, W_t, A16, B16, xa = ctx.saved_tensors
-        r = ctx.routing
-        gather = r.row_token if ctx.use_gather else None
-        dx_rows, dA, dB = ops.moe_lora_grouped_bwd(g.contiguous(), x, gather, W_t, A16, B16, xa,
-                                                   ctx.scale, r)
-        if ctx.use_gather:  # sum the k sorted rows of each token, slot order
-            dx = dx_rows[r.inv_perm.long()].view(-1, r.k, dx_rows.shape[1]).float().sum(1).to(x.dtype)
-        else:
-            dx = dx_rows
-        return dx, None, None, dA.to(ctx.dtypes[0]), dB.to(ctx.dtypes[1]), None, None, None
-
-
-def grouped_lora_linear(x, W, W_t, A, B, scale, routing, use_gather: bool):
-    return _GroupedLoRAFn.apply(x, W, W_t, A, B, float(scale), routing, use_gather)
-
-
 def _aligned(t: torch.Tensor) -> torch.Tensor:
     """``t``, contiguous and on the 16 bytes that the library's vector loads need (a view into a flat buffer of
     parameters or gradients may lie anywhere)."""

@@ -548,53 +548,6 @@ def attn_plan_rows(group_ids: torch.Tensor, parent_ids: torch.Tensor) -> "list[A
     return plans
 
 
-def _strides3(t: torch.Tensor, name: str):
-    """(batch, position, head) strides of a bf16 [B, S, H, D] view whose last dimension is contiguous."""
-    if t.dtype != torch.bfloat16 or t.dim() != 4 or t.stride(3) != 1 or not t.is_cuda:
-        raise ValueError(f"{name}: expected a bf16 device tensor [B, S, H, D] with contiguous D")
-    return (t.stride(0) if t.shape[0] > 1 else 0, t.stride(1), t.stride(2))
-
-
-def attn_fwd_rows(q, k, v, plan: torch.Tensor, scale: Optional[float] = None):
-    """(out bf16 [B, S, Hq, D], lse f32 [B, Hq, S]) for q [B, S, Hq, D], k/v [B, S, Hkv, D] (any strides over
-    B, S, H) and the plan buffer of B rows (AttnPlan.batch, or AttnPlan.buf for one row)."""
-    B, S, Hq, D = q.shape
-    Hkv = k.shape[2]
-    if k.shape != (B, S, Hkv, D) or v.shape != (B, S, Hkv, D):
-        raise ValueError("attention: inconsistent shapes")
-    lib = _lib.load()
-    dev = q.device
-    out = torch.empty((B, S, Hq, D), dtype=torch.bfloat16, device=dev)
-    lse = torch.empty((B, Hq, S), dtype=torch.float32, device=dev)
-    strides = (_lib._i64 * 12)(*_strides3(q, "q"), *_strides3(k, "k"), *_strides3(v, "v"), S * Hq * D, Hq * D, D)
-    scale = float(D) ** -0.5 if scale is None else float(scale)
-    _lib.check(lib.artk_attn_fwd_rows(q.data_ptr(), k.data_ptr(), v.data_ptr(), plan.data_ptr(), B, S, Hq, Hkv, D,
-                                      strides, scale, out.data_ptr(), lse.data_ptr(), _stream(dev)))
-    return out, lse
-
-
-def attn_bwd_rows(q, k, v, out, lse, d_out, plan: torch.Tensor, scale: Optional[float] = None):
-    """(dq, dk, dv) bf16, contiguous [B, S, H, D], for the upstream gradient d_out of attn_fwd_rows' out."""
-    B, S, Hq, D = q.shape
-    Hkv = k.shape[2]
-    lib = _lib.load()
-    dev = q.device
-    dq = torch.empty((B, S, Hq, D), dtype=torch.bfloat16, device=dev)
-    dk = torch.empty((B, S, Hkv, D), dtype=torch.bfloat16, device=dev)
-    dv = torch.empty((B, S, Hkv, D), dtype=torch.bfloat16, device=dev)
-    _need(lse, "lse", torch.float32, (B, Hq, S))
-    kv = (S * Hkv * D, Hkv * D, D)
-    strides = (_lib._i64 * 24)(*_strides3(q, "q"), *_strides3(k, "k"), *_strides3(v, "v"), *_strides3(out, "out"),
-                               *_strides3(d_out, "d_out"), S * Hq * D, Hq * D, D, *kv, *kv)
-    ws = _workspace(lib.artk_attn_bwd_rows_workspace_bytes(B, S, Hq, Hkv, D), dev)
-    scale = float(D) ** -0.5 if scale is None else float(scale)
-    _lib.check(lib.artk_attn_bwd_rows(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
-                                      d_out.data_ptr(), plan.data_ptr(), B, S, Hq, Hkv, D, strides, scale,
-                                      dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), ws.numel(),
-                                      _stream(dev)))
-    return dq, dk, dv
-
-
 def _shd(t: torch.Tensor, name: str):
     """(stride_s, stride_h) of a bf16 [S, H, D] view whose last dimension is contiguous."""
     if t.dtype != torch.bfloat16 or t.dim() != 3 or t.stride(2) != 1 or not t.is_cuda:

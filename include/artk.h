@@ -154,11 +154,11 @@ int32_t artk_grpo_fused(const void* hidden, const void* lm_head, const void* lm_
                         float* logprob, void* d_hidden, void* workspace, size_t workspace_bytes,
                         artk_stream_t stream);
 
-/* out[c,r] = in[r,c] for a bf16 [R,C] matrix (R, C multiples of 8).  Used once
- * per frozen weight to build the K-contiguous operand of the backward GEMMs. */
 /* out = in * *factor for n bf16 values (factor: f32 on the device; n a multiple of 8). */
 int32_t artk_scale_bf16(const void* in, const float* factor, void* out, int64_t n, artk_stream_t stream);
 
+/* out[c,r] = in[r,c] for a bf16 [R,C] matrix (R, C multiples of 8).  Used once
+ * per frozen weight to build the K-contiguous operand of the backward GEMMs. */
 int32_t artk_transpose_bf16(const void* in, void* out, int64_t R, int64_t C, artk_stream_t stream);
 
 /* Plain NT GEMM out[n,m] (bf16 or f32) = sum_k Q[n,k] * P[m,k]; exposed for
