@@ -24,10 +24,10 @@
 // stages, 16384 positions of 8 prompts of 137 + 4 x 461, 28 / 4 heads of 128:
 // forward 205 -> 154 us, dQ 279 -> 244 us, dK/dV 433 -> 297 us.  On dense causal
 // rows, where every tile comes into LDS twice as often, forward + backward are
-// 14 % faster to 5 % slower (us, 8 waves / now):
-//   heads of 128, 28 / 4: 4096 positions 617 / 619, 8192 2201 / 2103, 16384 8158 / 8281
-//   16 / 2: 8192 1216 / 1277, 12288 2701 / 2674;  16 / 16: 8192 1188 / 1230
-//   heads of 64, 14 / 2: 2048 173 / 148, 8192 724 / 684, 16384 2641 / 2308
+// 15 % faster to 3 % slower (us, 8 waves / now):
+//   heads of 128, 28 / 4: 4096 positions 630 / 618, 8192 2248 / 2151, 16384 8268 / 8379
+//   16 / 2: 8192 1253 / 1284, 12288 2772 / 2731;  16 / 16: 8192 1232 / 1241
+//   heads of 64, 14 / 2: 2048 172 / 147, 8192 728 / 682, 16384 2671 / 2359
 #include <stdlib.h>
 
 #include "common.hpp"
@@ -451,15 +451,26 @@ constexpr int ATT_THREADS = 2 * ATT_BM;  // forward and dQ: a wave per 32 querie
 // (query head, query block) of a work-group of the forward and dQ kernels.  A unit is the work-groups of
 // the heads that share one key/value head and query block: they read the same K and V tiles, so a unit
 // runs on one XCD (block b is placed on XCD b % 8), its heads one after the other; long blocks first.
-// There are 8 / Hkv XCDs to a key/value head.  With `turn` they are dealt the blocks forwards and backwards by
-// turns, or the first of them would get the longest block of every turn (of 64 blocks of a dense causal row and 2
-// key/value heads: 5 % more work than the average; forward 281 -> 270 us at 8192 positions, 16 / 2 heads of 128).
-// The dK/dV kernel, whose work-groups are not ordered by their work alone, did not gain.
-__device__ __forceinline__ bool attn_block(int Hq, int Hkv, int nQb, const int* order, bool turn, int& hq, int& qb) {
+// With `even` (forward and dQ; the dK/dV kernel, whose work-groups are not ordered by their work alone, became slower):
+// - There are 8 / Hkv XCDs to a key/value head.  They are dealt the blocks forwards and backwards by turns, or the first
+//   of them would get the longest block of every turn (of 64 blocks of a dense causal row and 2 key/value heads: 5 %
+//   more work than the average).
+// - The first two work-groups of each of an XCD's 32 CUs start together, and share the CU's speed.  The second ones come
+//   shortest first, so that a CU with the longest block of the row has the shortest beside it.  Longest first throughout,
+//   one CU had 128 + 96 tiles of work to begin with and another 98 + 66, which was then free for the longest of the rest,
+//   twice (clock stamps at 8192 positions, 16 heads: CUs ended between 232 and 306 us).
+// Dense causal row of 8192 positions, heads of 128, forward / dQ in us: 16 / 2 heads 289 / 404 -> 271 / 390 (half of it
+// by either), 16 / 16 heads 287 / 403 -> 274 / 392.
+constexpr int ATT_XCD_CUS = 32;
+__device__ __forceinline__ bool attn_block(int Hq, int Hkv, int nQb, const int* order, bool even, int& hq, int& qb) {
   const int rep = Hq / Hkv;
-  const int loc = blockIdx.x >> 3;
+  int loc = blockIdx.x >> 3;
   int x = blockIdx.x & 7;
-  if (turn && 8 % Hkv == 0 && (loc / rep & 1)) x = (8 / Hkv - 1 - x / Hkv) * Hkv + x % Hkv;
+  if (even) {
+    const int n = (int)(gridDim.x >> 3), end = n < 2 * ATT_XCD_CUS ? n : 2 * ATT_XCD_CUS;
+    if (blockIdx.y == 0 && loc >= ATT_XCD_CUS && loc < end) loc = ATT_XCD_CUS + end - 1 - loc;
+    if (8 % Hkv == 0 && (loc / rep & 1)) x = (8 / Hkv - 1 - x / Hkv) * Hkv + x % Hkv;
+  }
   const int unit = (loc / rep) * 8 + x;
   const int hkv = unit % Hkv;
   hq = hkv * rep + loc % rep;
