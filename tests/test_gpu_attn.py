@@ -298,10 +298,12 @@ def test_attn_bwd_mixed_light_and_heavy_key_blocks(artk_lib, gpu):
     assert rel_l2(results[64][0].float(), results[0][0].float()) <= 4e-3
 
 
-@pytest.mark.parametrize("S,Hq,Hkv,D", [(1792, 7, 1, 64), (2304, 7, 1, 64), (2304, 4, 2, 128), (2304, 2, 2, 128)])
+@pytest.mark.parametrize("S,Hq,Hkv,D", [(1792, 7, 1, 64), (2304, 7, 1, 64), (2304, 4, 2, 128), (2304, 2, 2, 128),
+                                         (2304, 16, 2, 64)])
 def test_attn_dense_causal_row(artk_lib, gpu, S, Hq, Hkv, D):
     """One conversation: the lists of 28 key blocks average 14.5 query tiles (several heads per work-group of dK/dV), those
-    of 36 average 18.5 (one); 18 query blocks do not divide by the XCDs that share a key/value head."""
+    of 36 average 18.5 (one); 18 query blocks do not divide by the XCDs that share a key/value head; with 16 heads an XCD
+    has 40 work-groups, 8 of them second on their CU."""
     print("attention dense row", S, Hq, Hkv, D, flush=True)
     q, k, v = make_qkv(S + Hq, S, Hq, Hkv, D)
     d_out = torch.randn(S, Hq, D, generator=torch.Generator().manual_seed(S)).to(torch.bfloat16)
