@@ -77,9 +77,25 @@ struct Nf4 {
   }
 };
 
+// The transposed copies of frozen weights as art_amd.ops.transposed_weight keeps them (made there if need be).
+std::vector<Tensor> transposed_weights(const std::vector<Tensor>& W) {
+  py::gil_scoped_acquire gil;
+  std::vector<Tensor> out;
+  try {
+    const py::object find = py::module_::import("art_amd.ops").attr("transposed_weight");
+    for (const Tensor& w : W) out.push_back(find(w).cast<Tensor>());
+  } catch (py::error_already_set& e) {  // on to the caller as the Python exception that it is
+    e.restore();
+    python_error error;
+    error.persist();
+    throw error;
+  }
+  return out;
+}
+
 // What a call of n projections over one input brings besides the differentiable tensors.
 struct LoraArgs {
-  std::vector<Tensor> W, W_t;               // frozen weights and their transposed copies (W_t: empty without a graph)
+  std::vector<Tensor> W, W_t;               // frozen weights and their transposed copies (W_t: empty where not all exist)
   std::vector<std::optional<Tensor>> bias;  // frozen
   std::shared_ptr<Nf4> nf4;                 // one projection on 4-bit codes instead of W
   double scale = 1;
@@ -149,6 +165,7 @@ struct LoraFunction : torch::autograd::Function<LoraFunction> {
       ctx->saved_data["blocksize"] = a.nf4->blocksize;
     } else {
       ctx->saved_data["frozen"] = a.W_t;
+      if (a.W_t.empty()) ctx->saved_data["W"] = a.W;  // the backward asks for the copies
       saved.insert(saved.end(), a.W.begin(), a.W.end());  // (their versions are checked with the rest)
     }
     ctx->save_for_backward(saved);
@@ -172,7 +189,7 @@ struct LoraFunction : torch::autograd::Function<LoraFunction> {
     const Tensor& x2 = saved[0];
     c10::OptionalDeviceGuard guard(x2.device());
     const int64_t T = x2.size(0), in = x2.size(1);
-    const auto t = ctx->saved_data["frozen"].toTensorVector();
+    auto t = ctx->saved_data["frozen"].toTensorVector();
     Tensor W_t;
     if (on_codes) {
       const Nf4 w{t[0], t[1], t[2], t[3], t[4], ctx->saved_data["offset"].toDouble(),
@@ -180,7 +197,8 @@ struct LoraFunction : torch::autograd::Function<LoraFunction> {
       W_t = make(x2, {in, w.out}, at::kBFloat16);
       w.dequantise(true, W_t);
     } else {
-      TORCH_CHECK((int)t.size() == n, "the projections were called without a graph");
+      if (t.empty()) t = transposed_weights(ctx->saved_data["W"].toTensorVector());
+      TORCH_CHECK((int)t.size() == n, "a transposed copy for each weight is needed");
     }
     artk_lora_proj_t proj[ARTK_LORA_MULTI_MAX] = {};
     std::vector<Tensor> g2, dA, dB;

@@ -27,10 +27,12 @@ def _frozen_bias(bias):
 
 def _lora_projections(x, weights, lora_As, lora_Bs, scale: float, biases):
     """Projections of the same x through the native autograd function (art_amd/csrc/native_ops.cpp): one call
-    each way, nothing concatenated.  The transposed copies of the frozen weights are only looked up when there
-    can be a backward."""
+    each way, nothing concatenated.  The transposed copies of the frozen weights go along if there are any; the
+    backward makes them on its first use otherwise."""
     graph = torch.is_grad_enabled() and any(t.requires_grad for t in (x, *lora_As, *lora_Bs))
-    wts = [ops.transposed_weight(w) for w in weights] if graph else []
+    wts = [ops.known_transpose(w) for w in weights] if graph else []
+    if any(wt is None for wt in wts):
+        wts = []
     return _lib.native().lora_multi(x, weights, wts, lora_As, lora_Bs, biases, scale)
 
 

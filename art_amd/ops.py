@@ -69,16 +69,24 @@ def transpose(x: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def transposed_weight(w: torch.Tensor) -> torch.Tensor:
-    """Transposed copy of a (frozen) weight, cached until the weight is modified
-    in place or freed.  The backward GEMMs need the weight with its other
-    dimension contiguous; the copy is made once per weight version."""
-    key = id(w)
-    hit = _transpose_cache.get(key)
+def known_transpose(w: torch.Tensor) -> Optional[torch.Tensor]:
+    """The copy that transposed_weight keeps of ``w``, or None if there is none (yet, or of this version)."""
+    hit = _transpose_cache.get(id(w))
     if hit is not None:
         ref, version, ptr, wt = hit
         if ref() is w and version == w._version and ptr == w.data_ptr():
             return wt
+    return None
+
+
+def transposed_weight(w: torch.Tensor) -> torch.Tensor:
+    """Transposed copy of a (frozen) weight, cached until the weight is modified
+    in place or freed.  The backward GEMMs need the weight with its other
+    dimension contiguous; the copy is made once per weight version."""
+    wt = known_transpose(w)
+    if wt is not None:
+        return wt
+    key = id(w)
     wt = transpose(w)
     try:
         ref = weakref.ref(w, lambda _r, k=key: _transpose_cache.pop(k, None))

@@ -420,3 +420,34 @@ def test_native_functions_on_another_stream(artk_lib, gpu):
     side.synchronize()
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+def test_forward_makes_no_transposed_weight(artk_lib, gpu):
+    """A forward with a graph but without a backward keeps no second copy of a weight; the first backward makes it, of
+    the module's own weight also where saved-tensor hooks hand the node a copy, and the gradients are those of later
+    passes, in which the copy is there."""
+    from art_amd.lora import FusedLoRALinear, LoRALinear
+
+    torch.manual_seed(9)
+    layers = [LoRALinear(128, o, device=gpu) for o in (192, 64)]
+    for m in layers:
+        m.lora_B.data.normal_(std=0.05)
+    fused = FusedLoRALinear(layers)
+    x = torch.randn(1, 70, 128, device=gpu, dtype=torch.bfloat16, requires_grad=True)
+    params = [p for m in layers for p in (m.lora_A, m.lora_B)]
+
+    def grads():
+        return torch.autograd.grad(sum(y.float().square().sum() for y in fused(x)), [x] + params)
+
+    fused(x)
+    assert all(ops.known_transpose(m.weight) is None for m in layers)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(gpu)):
+        first = grads()
+    assert all(torch.equal(ops.known_transpose(m.weight), m.weight.t()) for m in layers)
+    for a, b in zip(first, grads()):
+        assert torch.equal(a, b)
+    with torch.no_grad():
+        layers[0].weight.mul_(2)
+    assert ops.known_transpose(layers[0].weight) is None
+    for a, b in zip(grads(), grads()):
+        assert torch.equal(a, b)
