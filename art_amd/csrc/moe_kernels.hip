@@ -259,6 +259,7 @@ struct MoeGemmParams {
   const int* tile_prefix;  // [E+1]
   int64_t M, K;
   int E, r, RP, MT;
+  const int* order;
 };
 
 // One tile of the grouped product: expert, rows and weight tile.
@@ -373,6 +374,183 @@ __global__ __launch_bounds__(nthreads<MOE_NI>()) void moe_gemm_kernel(MoeGemmPar
     if (!more) break;
     t = t2;
     cur = nxt;
+  }
+}
+
+// ----------------------------------------------------------------------------
+// The same grouped product where an expert has few rows: the launch reads every weight once for a handful of columns
+// and is as long as those reads.  A work-group streams 128 weight rows of one expert past up to 128 of its rows at a
+// time (4 waves, 32 weight rows each), two work-groups per CU.  The weights come from HBM and have a ring of three or
+// four stages of 64 K elements, the activations from L2 and have two; waves 0 and 1 issue the weights' DMA, waves 2 and
+// 3 the activations', because a wave's DMA completes in order and a wait for the younger activations would wait for
+// the weights behind them.  So up to 96 KiB of weights are on their way per CU where the 256 x 256 tile above has 32.
+// ----------------------------------------------------------------------------
+constexpr int SG_ROWS = 128;                      // weight rows of a work-group
+constexpr int SG_COLS = 128;                      // most columns in one pass over the weights
+constexpr int SG_P_BYTES = SG_ROWS * BK * 2;      // 16 KiB
+constexpr int SG_LDS_BYTES = 80 * 1024;           // two work-groups per CU
+template <int NQ> constexpr int sg_stages() { return NQ <= 2 ? 4 : 3; }
+
+// acc[i] += 32 weight rows of this wave x columns 32 i .. 32 i + 31 over nk K steps.  Every wave calls it together; LDS
+// may be reused when it returns.  ONCE: nobody reads the weights again, they pass the caches by (0.8 GB in 135 us instead of 150).
+template <int NQ, bool ONCE>
+__device__ __forceinline__ void moe_stream_run(floatx16 (&acc)[NQ], char* smem, dma_rsrc_t prsrc, const int (&pv)[2],
+                                               int pstep, dma_rsrc_t qrsrc, const int (&qv)[2 * NQ], int nk) {
+  constexpr int NST = sg_stages<NQ>(), Q_BYTES = NQ * 4096, Q_OFF = NST * SG_P_BYTES;
+  static_assert(Q_OFF + 2 * Q_BYTES <= SG_LDS_BYTES, "rings");
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t lds = lds_addr_of(smem);
+  auto issue_p = [&](int kt, int buf) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int g = wave * 8 + i;
+      dma_load16<ONCE>(prsrc, pv[i & 1], g * pstep + kt * (BK * 2), lds + buf * SG_P_BYTES + g * 1024);
+    }
+  };
+  auto issue_q = [&](int kt) {
+#pragma unroll
+    for (int i = 0; i < 2 * NQ; ++i)
+      dma_load16(qrsrc, qv[i], kt * (BK * 2), lds + Q_OFF + (kt & 1) * Q_BYTES + ((wave - 2) * 2 * NQ + i) * 1024);
+  };
+  int off[4];
+  {
+    const int rl = lane & 31, f = swz(rl);
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) off[kk] = rl * 128 + (((kk * 2 + (lane >> 5)) ^ f) << 4);
+  }
+  if (wave < 2) {
+#pragma unroll
+    for (int i = 0; i < NST - 1; ++i)
+      if (i < nk) issue_p(i, i);
+  } else {
+    issue_q(0);
+  }
+  int buf = 0, fill = NST - 1;  // weight stage of K step kt, and the one that is free after its barrier
+  for (int kt = 0; kt < nk; ++kt) {
+    // stage kt has landed: of the weights, only the stages after it may be on their way
+    if (wave >= 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else if (kt + NST - 1 <= nk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 2) * 8) : "memory");
+    else if (NST == 4 && kt + 2 == nk) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    barrier_lds_only();  // ... for every wave, and every wave is done with stage kt - 1
+    if (wave < 2) {
+      if (kt + NST - 1 < nk) issue_p(kt + NST - 1, fill);
+    } else {
+      if (kt + 1 < nk) issue_q(kt + 1);
+    }
+    const char* sp = smem + buf * SG_P_BYTES + wave * 4096;
+    const char* sq = smem + Q_OFF + (kt & 1) * Q_BYTES;
+    bf16x8 p[4], q[4][NQ];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      p[kk] = *(const bf16x8*)(sp + off[kk]);
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) q[kk][i] = *(const bf16x8*)(sq + off[kk] + i * 4096);
+    }
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p[kk], q[kk][i], acc[i], 0, 0, 0);
+    buf = buf + 1 == NST ? 0 : buf + 1;
+    fill = fill + 1 == NST ? 0 : fill + 1;
+  }
+  barrier_lds_only();
+}
+
+// n <= 32 NQ rows of expert e, from sorted row row0 on, against its weight rows m0 ..
+template <int NQ, bool ONCE>
+__device__ __forceinline__ void moe_stream_cols(const MoeGemmParams& p, char* smem, int e, int64_t m0, int64_t row0,
+                                                int n) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = lane >> 5;
+  const int r = lane >> 3, pc = lane & 7;
+  const int64_t wrows = p.M - m0 < SG_ROWS ? p.M - m0 : SG_ROWS;  // rows past the end arrive as zeros
+  const dma_rsrc_t prsrc =
+      dma_make_rsrc((const char*)p.W + ((int64_t)e * p.M + m0) * p.K * 2, (uint32_t)(wrows * p.K * 2));
+  const int pv[2] = {(int)(r * p.K * 2) + ((pc ^ r) << 4), (int)(r * p.K * 2) + ((pc ^ r ^ 1) << 4)};  // as PanelLoader
+  const dma_rsrc_t qrsrc = dma_make_rsrc((const char*)p.X + (p.gather ? 0 : row0 * p.K * 2), 0x7fffffffu);
+  int qv[2 * NQ];
+#pragma unroll
+  for (int i = 0; i < 2 * NQ; ++i) {
+    const int row = ((wave & 1) * 2 * NQ + i) * 8 + r;
+    int64_t src = row < n ? row : n - 1;
+    if (p.gather) src = p.gather[row0 + src];
+    qv[i] = (int)(src * p.K * 2) + ((pc ^ swz(row)) << 4);
+  }
+  floatx16 acc[NQ];
+#pragma unroll
+  for (int i = 0; i < NQ; ++i)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
+  moe_stream_run<NQ, ONCE>(acc, smem, prsrc, pv, (int)(8 * p.K * 2), qrsrc, qv, (int)(p.K / BK));
+
+  const int64_t mw = m0 + wave * 32;  // first weight row of this wave
+  if (mw >= p.M) return;              // (M is a multiple of 64: a wave's rows are all there or none)
+  if (p.Pe != nullptr) {
+    const uint16_t* Pe = p.Pe + ((int64_t)e * p.M + mw + (lane & 31)) * p.r;
+    for (int e0 = 0; e0 < p.RP; e0 += 16) {
+      const int c = e0 + half * 8;
+      const bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
+      bf16x8 pf = *(const bf16x8*)(Pe + (c < p.r ? c : 0));
+      bf16x8 qf[NQ];
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) {
+        const int col = i * 32 + (lane & 31);
+        qf[i] = *(const bf16x8*)(p.Qe + (row0 + (col < n ? col : n - 1)) * p.RP + c);
+      }
+      pf = c < p.r ? pf : z;
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pf, qf[i], acc[i], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    const int col = i * 32 + (lane & 31);
+    if (col < n) store_block_bf16(p.out + (row0 + col) * p.M + mw, acc[i], half);
+  }
+}
+
+template <bool ONCE>
+__device__ __forceinline__ void moe_stream_pass(const MoeGemmParams& p, char* smem, int e, int64_t m0, int64_t row0,
+                                                int n) {
+  if (n > 96) moe_stream_cols<4, ONCE>(p, smem, e, m0, row0, n < SG_COLS ? n : SG_COLS);
+  else if (n > 64) moe_stream_cols<3, ONCE>(p, smem, e, m0, row0, n);
+  else if (n > 32) moe_stream_cols<2, ONCE>(p, smem, e, m0, row0, n);
+  else moe_stream_cols<1, ONCE>(p, smem, e, m0, row0, n);
+}
+
+// Experts are dealt to the XCDs in falling order of their rows; an XCD's units are numbered expert by expert, weight
+// tile by weight tile, and the passes of an expert with more than SG_COLS rows (even shares of them, in whole 32) are
+// neighbours, so they read a weight tile together.  A wave finds the expert of unit `loc` from its lanes' counts.
+__global__ __launch_bounds__(256, 2) void moe_stream_gemm_kernel(MoeGemmParams p) {
+  __shared__ __attribute__((aligned(1024))) char smem[SG_LDS_BYTES];
+  const int lane = threadIdx.x & 63;
+  const int x = blockIdx.x & 7;
+  int ex = 8 * lane + ((lane & 1) ? 7 - x : x);  // this lane's expert
+  int first = 0, n_e = 0;
+  if (ex < p.E) {
+    if (p.order != nullptr) ex = p.order[ex];
+    first = p.offsets[ex];
+    n_e = p.offsets[ex + 1] - first;
+  }
+  const int passes = (n_e + SG_COLS - 1) / SG_COLS;
+  int end = passes * p.MT;  // units of the experts up to this one
+#pragma unroll
+  for (int d = 1; d < MOE_MAX_E / 8; d <<= 1) {
+    const int v = __shfl_up(end, d, 64);
+    if (lane >= d) end += v;
+  }
+  const int total = __builtin_amdgcn_readlane(end, MOE_MAX_E / 8 - 1);
+  for (int loc = blockIdx.x >> 3; loc < total; loc += gridDim.x >> 3) {
+    const int l = __popcll(__ballot(lane < MOE_MAX_E / 8 && end <= loc));
+    const int e = __builtin_amdgcn_readlane(ex, l), n = __builtin_amdgcn_readlane(n_e, l);
+    const int np = __builtin_amdgcn_readlane(passes, l), row0 = __builtin_amdgcn_readlane(first, l);
+    const int unit = loc - (__builtin_amdgcn_readlane(end, l) - np * p.MT);
+    const int per = ((n + np - 1) / np + 31) & ~31, c0 = (unit % np) * per;
+    const int64_t m0 = (int64_t)(unit / np) * SG_ROWS;
+    const int left = n - c0 < per ? n - c0 : per;
+    if (np == 1) moe_stream_pass<true>(p, smem, e, m0, row0, left);
+    else if (left > 0) moe_stream_pass<false>(p, smem, e, m0, row0 + c0, left);
   }
 }
 
@@ -588,7 +766,7 @@ static int32_t check_moe(int64_t n_rows, int64_t in, int64_t out, int E, int r) 
 static int32_t launch_moe_gemm(const void* W, const void* X, const int* gather, const uint16_t* Pe,
                                const uint16_t* Qe, void* out, const int* offsets,
                                const int* tile_prefix, int64_t n_rows, int64_t M, int64_t K, int E,
-                               int r, int RP, hipStream_t st) {
+                               int r, int RP, hipStream_t st, const int* order = nullptr) {
   MoeGemmParams p;
   p.W = W;
   p.X = X;
@@ -606,7 +784,17 @@ static int32_t launch_moe_gemm(const void* W, const void* X, const int* gather, 
   p.MT = (int)((M + TILE - 1) / TILE);
   const int64_t max_row_tiles = (n_rows + TILE - 1) / TILE + E;
   prof_begin(PROF_MOE_GEMM, st);
-  {
+  // Up to SG_COLS rows per expert the streaming kernel is the faster one.  Four products of a block, us, 256 x 256 tiles
+  // / streamed (hidden 2048, intermediate 768): 128 experts, 203 tokens (13 rows each) 517 / 423, 512 (32) 569 / 498,
+  // 1024 (64) 681 / 579, 2048 (128) 728 / 705, 3000 (188) 888 / 868; 64 experts, 400 tokens (50) 333 / 279,
+  // 1024 (128) 405 / 389, 1300 (163) 418 / 432.
+  if (n_rows <= (int64_t)E * SG_COLS) {
+    p.MT = (int)((M + SG_ROWS - 1) / SG_ROWS);
+    p.order = order;
+    // (as many as there are units if the XCDs' shares are even; the rest comes in a second turn)
+    const int64_t per_xcd = (E + 7) / 8 + (n_rows + 8 * SG_COLS - 1) / (8 * SG_COLS);
+    moe_stream_gemm_kernel<<<(unsigned)(8 * per_xcd * p.MT), 256, 0, st>>>(p);
+  } else {
     // persistent: one work-group per CU walks the device-side work list
     const int cus = num_cus();
     const int64_t upper = (int64_t)max_row_tiles * p.MT;
@@ -929,7 +1117,7 @@ int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_
   const int64_t n = a->T * a->k, H = a->H, I = a->I;
   const int E = a->E, r = a->r;
   if ((rc = moe_route(a->router_logits, a->T, E, a->k, a->topk_idx, a->topk_w, a->perm, a->inv_perm, a->row_token,
-                      a->offsets, a->tile_prefix, a->blk_prefix, moe_order(a, s), c.route, c.route_bytes, stream)))
+                      a->offsets, a->tile_prefix, a->blk_prefix, s.order, c.route, c.route_bytes, stream)))
     return rc;
   {
     MoePack p{a->gate_A, a->gate_B, a->up_A, a->up_B, a->down_A, a->down_B, s.A_gu, s.B_gu, s.A_d, s.B_d,
@@ -941,7 +1129,7 @@ int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_
                               a->scale, s.xa_gu, c.xa16_gu, st)))
     return rc;
   if ((rc = launch_moe_gemm(a->W_gu, a->x, a->row_token, s.B_gu, c.xa16_gu, s.gu, a->offsets, a->tile_prefix, n, 2 * I,
-                            H, E, 2 * r, round16(2 * r), st)))
+                            H, E, 2 * r, round16(2 * r), st, s.order)))
     return rc;
   moe_silu_mul_kernel<<<blocks256(n * I / 8), 256, 0, st>>>(s.gu, n * I / 8, (int)(I / 8), s.h);
   ARTK_CHECK_LAUNCH();
@@ -949,7 +1137,7 @@ int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_
                               s.xaw_d, c.xa16_d, st, a->topk_w, a->perm)))
     return rc;
   if ((rc = launch_moe_gemm(a->W_d, s.h, nullptr, s.B_d, c.xa16_d, c.down, a->offsets, a->tile_prefix, n, H, I, E, r,
-                            round16(r), st)))
+                            round16(r), st, s.order)))
     return rc;
   moe_combine_kernel<<<blocks256(a->T * H / 8), 256, 0, st>>>(c.down, a->inv_perm, a->topk_w, a->T * H / 8,
                                                               (int)(H / 8), a->k, (uint16_t*)a->y);
@@ -1004,7 +1192,7 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
     if ((rc = launch_stats_reduce(ja, none, r, st))) return rc;
   }
   if ((rc = launch_moe_gemm(a->Wt_d, a->g, a->row_token, c.At_d, c.gb16, c.dhr, a->offsets, a->tile_prefix, n, I, H, E,
-                            r, round16(r), st)))
+                            r, round16(r), st, s.order)))
     return rc;
   if ((rc = launch_stats_grouped(s.h, n, nullptr, n, I, nullptr, c.gb, r, E, a->offsets, nullptr, a->ddown_A, a->scale,
                                  1, c.dummy, st, &down)))
@@ -1022,7 +1210,7 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
     if ((rc = launch_stats_reduce(ja, none, 2 * r, st))) return rc;
   }
   if ((rc = launch_moe_gemm(a->Wt_gu, c.g_gu, nullptr, c.At_gu, c.gb16, c.dx_rows, a->offsets, a->tile_prefix, n, H,
-                            2 * I, E, 2 * r, round16(2 * r), st)))
+                            2 * I, E, 2 * r, round16(2 * r), st, s.order)))
     return rc;
   if ((rc = launch_stats_grouped(a->x, a->T, a->row_token, n, H, nullptr, c.gb, 2 * r, E, a->offsets, nullptr,
                                  a->dgate_A, a->scale, 1, c.dummy, st, &gate_up_A)))

@@ -137,6 +137,45 @@ def test_grouped_lora_ranks(artk_lib, gpu, r, use_gather):
     assert rel_l2(dB.cpu(), dB0) <= TOL
 
 
+@pytest.mark.parametrize("rows,H,I,r,use_gather", [
+    ([0, 1, 31, 32, 33, 64, 65, 0], 64, 64, 8, True),            # one K step, half a tile of weight rows
+    ([96, 97, 128, 5, 0, 17, 63, 2, 40], 192, 320, 24, False),   # fewer K steps than ring stages, a ragged weight tile
+    ([129, 0, 260, 3, 0, 0, 0, 0, 0, 77], 128, 448, 8, True),    # experts in two and three passes
+    ([3] * 255 + [200], 128, 128, 16, True),                     # the most experts
+    ([300, 1, 130], 128, 192, 8, True),                          # more than 128 rows per expert: 256 x 256 tiles
+    ([257, 384], 192, 320, 40, False),
+])
+def test_grouped_lora_rows_per_expert(artk_lib, gpu, rows, H, I, r, use_gather):
+    """Row counts around the column tiles of both grouped products (32, 64, 96, 128 columns of a streaming pass, 256 of
+    a tile) with K ranges shorter and longer than their rings.  TOL as above."""
+    print(f"moe grouped rows {rows[:10]} H={H} I={I} r={r} gather={use_gather}", flush=True)
+    E, T = len(rows), sum(rows)
+    g = torch.Generator().manual_seed(T + H)
+    owner = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))[torch.randperm(T, generator=g)]
+    logits = torch.zeros(T, E)
+    logits[torch.arange(T), owner] = 1.0
+    rt, ref = check_routing(logits, 1, gpu)
+    off = ref["offsets"]
+    assert [int(off[e + 1] - off[e]) for e in range(E)] == rows
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    W, A, B = make_experts(E, I, H, r, 21)
+    up = torch.randn(T, I, generator=g).to(torch.bfloat16)
+    y0, dx0, dA0, dB0 = moe_oracle.grouped_lora_grads(
+        x, ref["row_token"] if use_gather else None, W, A, B, 0.5, off, up)
+    gather = rt.row_token if use_gather else None
+    y, xa = ops.moe_lora_grouped_fwd(x.to(gpu), gather, W.to(gpu), A.to(gpu), B.to(gpu), 0.5, rt)
+    dx, dA, dB = ops.moe_lora_grouped_bwd(up.to(gpu), x.to(gpu), gather, ops.transpose_batched(W.to(gpu)),
+                                          A.to(gpu), B.to(gpu), xa, 0.5, rt)
+    if use_gather:
+        dx = dx[rt.inv_perm.long()]
+    for a, b in ((y, y0), (dx, dx0)):
+        assert rel_l2(a.cpu().float(), b) <= TOL
+    for e in range(E):  # no expert's rows are lost among the others'
+        if rows[e]:
+            assert rel_l2(y[off[e]:off[e + 1]].cpu().float(), y0[off[e]:off[e + 1]]) <= TOL
+    assert rel_l2(dA.cpu(), dA0) <= TOL and rel_l2(dB.cpu(), dB0) <= TOL
+
+
 @pytest.mark.parametrize("use_gather", [True, False])
 def test_grouped_lora_with_empty_experts(artk_lib, gpu, use_gather):
     """Experts that no token chose: their dA_e and dB_e are exactly zero, the others match the oracle
