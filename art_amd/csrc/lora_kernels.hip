@@ -623,8 +623,8 @@ struct LoraBwdScratch {
 };
 static void carve_lora_bwd(Workspace& ws, int64_t T, int64_t in, int64_t out, int r, LoraBwdScratch& c) {
   const int RP = round16(r);
-  c.gg = stats_geom(T, out, r);
-  c.gx = stats_geom(T, in, r);
+  c.gg = stats_geom(T, out, r, out);
+  c.gx = stats_geom(T, in, r, in);
   c.Bt = ws.take<uint16_t>((size_t)r * out);   // B^T [r,out]: factor of the g B product
   c.At = ws.take<uint16_t>((size_t)in * r);    // A^T [in,r]: low-rank factor of dx
   c.gb = ws.take<float>((size_t)T * r);        // g B, f32 [T,r]
@@ -779,19 +779,23 @@ struct LoraMultiBwdScratch {
 static void carve_lora_multi_bwd(Workspace& ws, int64_t T, int64_t in, const artk_lora_proj_t* proj, int n,
                                  LoraMultiBwdScratch& c) {
   c.r_total = 0;
-  for (int i = 0; i < n; ++i) c.r_total += proj[i].r;
+  int64_t out_all = 0;
+  for (int i = 0; i < n; ++i) {
+    c.r_total += proj[i].r;
+    out_all += proj[i].out;
+  }
   for (int i = 0; i < n; ++i) {
     const int64_t out = proj[i].out;
     const int r = proj[i].r, RP = round16(r);
     LoraBwdScratch& o = c.one[i];
-    o.gg = stats_geom(T, out, r);
+    o.gg = stats_geom(T, out, r, out_all);
     o.Bt = ws.take<uint16_t>((size_t)r * out);
     o.At = ws.take<uint16_t>((size_t)in * r);
     o.gb16 = ws.take<uint16_t>((size_t)T * RP);
     o.rowp_g = ws.take<float>((size_t)o.gg.n_chunks * T * r);
     o.colp_g = ws.take<float>((size_t)o.gg.n_slabs * out * r);
   }
-  c.gx = stats_geom(T, in, c.r_total);
+  c.gx = stats_geom(T, in, c.r_total, in);
   c.gb_cat = ws.take<float>((size_t)T * c.r_total);
   c.colp_x = ws.take<float>((size_t)c.gx.n_slabs * in * c.r_total);
   c.dummy = ws.take<float>(1024);
@@ -845,13 +849,13 @@ int32_t artk_lora_linear_multi_bwd_typed(const void* x, const artk_lora_proj_t* 
   tr.n = 2 * n;
   sm.n = n;
   rm.n = 2 * n;
-  bool any_wide = false, any_narrow = false;
+  bool one_shape = true;
   int r0 = 0;
   for (int i = 0; i < n; ++i) {
     const artk_lora_proj_t& q = proj[i];
     LoraBwdScratch& o = c.one[i];
     const int RP = round16(q.r);
-    (q.r > 32 ? any_wide : any_narrow) = true;
+    one_shape = one_shape && stats_shape(q.r) == stats_shape(proj[0].r);
     tr.t[2 * i] = SmallTranspose{(const uint16_t*)q.B, o.Bt, 1, q.out, q.r};
     tr.t[2 * i + 1] = SmallTranspose{(const uint16_t*)q.A, o.At, 1, q.r, in};
     // one pass over g_i: partials of g_i B_i (over column chunks) and of g_i^T (x A_i^T) (over row slabs)
@@ -870,16 +874,10 @@ int32_t artk_lora_linear_multi_bwd_typed(const void* x, const artk_lora_proj_t* 
   }
   jx.e_start[n] = r0;
   if ((rc = launch_small_transpose_multi(tr, st))) return rc;
-  if (any_wide && any_narrow) {  // the stats kernel has one shape per side of rank 32: one launch per projection
-    for (int i = 0; i < n; ++i) {
-      const StatsParams& sp = sm.p[i];
-      if (sp.R > 32)
-        lora_stats_kernel<2, 2, 2, false><<<(unsigned)(sp.n_slabs * sp.n_chunks), 256, 0, st>>>(sp);
-      else
-        lora_stats_kernel<1, 4, 3, false><<<(unsigned)(sp.n_slabs * sp.n_chunks), 256, 0, st>>>(sp);
-      ARTK_CHECK_LAUNCH();
-    }
-  } else if ((rc = launch_stats_multi(sm, any_wide, st))) {
+  if (!one_shape) {  // one launch per projection
+    for (int i = 0; i < n; ++i)
+      if ((rc = launch_stats_params(sm.p[i], st))) return rc;
+  } else if ((rc = launch_stats_multi(sm, stats_shape(proj[0].r), st))) {
     return rc;
   }
   if ((rc = launch_stats_reduce_multi(rm, st))) return rc;

@@ -700,7 +700,8 @@ __global__ __launch_bounds__(256) void moe_silu_bwd_kernel(const uint16_t* __res
 }
 
 // out[t, :] = sum_j w[t, j] rows[inv_perm[t k + j], :] in slot order (w == nullptr: plain sum); the k
-// sorted rows of a token are read once, 8 columns per thread, eight loads in flight.
+// sorted rows of a token are read once, 8 columns per thread, eight loads in flight.  Nobody reads
+// them again: non-temporal loads, 57 -> 51 us for 65536 rows of 2048, level up to 16384 rows.
 __global__ __launch_bounds__(256) void moe_combine_kernel(const uint16_t* __restrict__ rows,
                                                           const int* __restrict__ inv_perm,
                                                           const float* __restrict__ w, int64_t n8, int H8, int k,
@@ -713,8 +714,15 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const uint16_t* __rest
   for (int j0 = 0; j0 < k; j0 += 8) {
     uint4 v[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      v[j] = j0 + j < k ? ((const uint4*)rows)[(int64_t)inv_perm[t * k + j0 + j] * H8 + c] : make_uint4(0, 0, 0, 0);
+    for (int j = 0; j < 8; ++j) {
+      typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+      u32x4 x = {0, 0, 0, 0};
+      if (j0 + j < k) {
+        const u32x4* src = (const u32x4*)rows + (int64_t)inv_perm[t * k + j0 + j] * H8 + c;
+        x = __builtin_nontemporal_load(src);
+      }
+      v[j] = make_uint4(x[0], x[1], x[2], x[3]);
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const float wj = j0 + j >= k ? 0.f : (w ? w[t * k + j0 + j] : 1.f);
@@ -1092,6 +1100,13 @@ static int* moe_order(const artk_moe_experts_t* a, const MoeSaved& s) {
 
 static unsigned blocks256(int64_t n) { return (unsigned)((n + 255) / 256); }
 
+static int32_t launch_moe_combine(const uint16_t* rows, const artk_moe_experts_t* a, const float* w, void* out, hipStream_t st) {
+  const int64_t n8 = a->T * a->H / 8;
+  moe_combine_kernel<<<blocks256(n8), 256, 0, st>>>(rows, a->inv_perm, w, n8, (int)(a->H / 8), a->k, (uint16_t*)out);
+  ARTK_CHECK_LAUNCH();
+  return ARTK_OK;
+}
+
 int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,
                              artk_stream_t stream) {
   int32_t rc = check_moe_experts(a, false);
@@ -1139,10 +1154,7 @@ int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_
   if ((rc = launch_moe_gemm(a->W_d, s.h, nullptr, s.B_d, c.xa16_d, c.down, a->offsets, a->tile_prefix, n, H, I, E, r,
                             round16(r), st, s.order)))
     return rc;
-  moe_combine_kernel<<<blocks256(a->T * H / 8), 256, 0, st>>>(c.down, a->inv_perm, a->topk_w, a->T * H / 8,
-                                                              (int)(H / 8), a->k, (uint16_t*)a->y);
-  ARTK_CHECK_LAUNCH();
-  return ARTK_OK;
+  return launch_moe_combine(c.down, a, a->topk_w, a->y, st);
 }
 
 int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,
@@ -1215,10 +1227,7 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
   if ((rc = launch_stats_grouped(a->x, a->T, a->row_token, n, H, nullptr, c.gb, 2 * r, E, a->offsets, nullptr,
                                  a->dgate_A, a->scale, 1, c.dummy, st, &gate_up_A)))
     return rc;
-  moe_combine_kernel<<<blocks256(a->T * H / 8), 256, 0, st>>>(c.dx_rows, a->inv_perm, nullptr, a->T * H / 8,
-                                                              (int)(H / 8), a->k, (uint16_t*)a->dx);
-  ARTK_CHECK_LAUNCH();
-  return ARTK_OK;
+  return launch_moe_combine(c.dx_rows, a, nullptr, a->dx, st);
 }
 
 int32_t artk_transpose_bf16_batched(const void* in, void* out, int64_t n, int64_t R, int64_t C,

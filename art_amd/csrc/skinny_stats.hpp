@@ -84,6 +84,37 @@ __device__ __forceinline__ bf16x8 st_tr_frag(const char* tile, int lane, int k0,
   return __builtin_bit_cast(bf16x8, v);
 }
 
+// COL result of column c, ranks e0 .. e0 + 3, of a slab.
+template <bool BLOCK>
+__device__ __forceinline__ void stats_put_col(const StatsParams& p, int slab, bool grouped, int64_t c, int e0,
+                                              const floatx4& v) {
+  const int R = p.R;
+  if (!grouped) {
+    *(floatx4*)(p.col_part + ((int64_t)slab * p.C + c) * R + e0) = v;
+  } else if (!BLOCK || p.block.r_split == 0) {
+    if (!p.col_transposed) {
+      *(floatx4*)(p.col_out + ((int64_t)slab * p.C + c) * R + e0) = v * p.col_scale;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) p.col_out[((int64_t)slab * R + e0 + k) * p.C + c] = v[k] * p.col_scale;
+    }
+  } else if constexpr (BLOCK) {
+    const StatsBlock& two = p.block;
+    if (p.col_transposed) {
+      float* dst = e0 < two.r_split ? p.col_out + ((int64_t)slab * two.r_split + e0) * p.C + c
+                                    : two.col_out2 + ((int64_t)slab * (R - two.r_split) + e0 - two.r_split) * p.C + c;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) dst[k * p.C] = v[k] * p.col_scale;
+    } else if (c < two.c_split) {
+      if (e0 < two.r_split)
+        *(floatx4*)(p.col_out + ((int64_t)slab * two.c_split + c) * two.r_split + e0) = v * p.col_scale;
+    } else if (e0 >= two.r_split) {
+      *(floatx4*)(two.col_out2 + ((int64_t)slab * (p.C - two.c_split) + c - two.c_split) * (R - two.r_split) + e0 -
+                  two.r_split) = v * p.col_scale;
+    }
+  }
+}
+
 // NTE: 32-wide tiles of e (rank <= 32 NTE); NCT: 128-column tiles per chunk; NST: LDS stages.
 // All memory traffic of the main loop is LDS DMA, ordered by hand with s_waitcnt vmcnt(n)
 // (the compiler inserts no waits for it): per wave, a tile is 8 DMA instructions, the Y rows
@@ -322,35 +353,253 @@ __device__ __forceinline__ void lora_stats_body(const StatsParams& p, const int 
         for (int q = 0; q < 4; ++q) {
           const int e0 = 32 * et + 8 * q + 4 * half;
           if (e0 >= R) continue;
-          floatx4 v = floatx4{acc_col[ct][et][4 * q], acc_col[ct][et][4 * q + 1], acc_col[ct][et][4 * q + 2],
-                              acc_col[ct][et][4 * q + 3]};
-          if (!grouped) {
-            *(floatx4*)(p.col_part + ((int64_t)slab * p.C + c) * R + e0) = v;
-          } else if (!BLOCK || p.block.r_split == 0) {
-            if (!p.col_transposed) {
-              *(floatx4*)(p.col_out + ((int64_t)slab * p.C + c) * R + e0) = v * p.col_scale;
-            } else {
-#pragma unroll
-              for (int k = 0; k < 4; ++k) p.col_out[((int64_t)slab * R + e0 + k) * p.C + c] = v[k] * p.col_scale;
-            }
-          } else if constexpr (BLOCK) {
-            const StatsBlock& two = p.block;
-            if (p.col_transposed) {
-              float* dst = e0 < two.r_split ? p.col_out + ((int64_t)slab * two.r_split + e0) * p.C + c
-                                            : two.col_out2 + ((int64_t)slab * (R - two.r_split) + e0 - two.r_split) * p.C + c;
-#pragma unroll
-              for (int k = 0; k < 4; ++k) dst[k * p.C] = v[k] * p.col_scale;
-            } else if (c < two.c_split) {
-              if (e0 < two.r_split)
-                *(floatx4*)(p.col_out + ((int64_t)slab * two.c_split + c) * two.r_split + e0) = v * p.col_scale;
-            } else if (e0 >= two.r_split) {
-              *(floatx4*)(two.col_out2 + ((int64_t)slab * (p.C - two.c_split) + c - two.c_split) * (R - two.r_split) + e0 -
-                          two.r_split) = v * p.col_scale;
-            }
-          }
+          const floatx4 v = floatx4{acc_col[ct][et][4 * q], acc_col[ct][et][4 * q + 1], acc_col[ct][et][4 * q + 2],
+                                    acc_col[ct][et][4 * q + 3]};
+          stats_put_col<BLOCK>(p, slab, grouped, c, e0, v);
         }
     }
   }
+}
+
+// ----------------------------------------------------------------------------
+// The same two products for ranks up to 16 NTE, on MFMA 16x16x32 (at rank 8 or 16 half or more of a 32 x 32 tile of e
+// would be multiplied for nothing) and small enough for two work-groups per CU: tiles of 64 rows x 128 columns, three
+// stages of 16 KiB, the factor of the chunk in registers (NCT * NTE * 4 fragments a lane).  One work-group computes,
+// stores its results or fills its ring while the other's reads are on their way.  Wave w owns rows 16w.. of a tile for
+// ROW and columns 32w.. for COL.  Everything else as above.
+// ----------------------------------------------------------------------------
+constexpr int SN_ROWS = 64;
+constexpr int SN_TILE_BYTES = SN_ROWS * ST_ROW_BYTES;  // 16 KiB
+constexpr int SN_STAGES = 3;
+
+// Transposed fragment for MFMA 16x16x32: lane (n, s) gets column d0 + n of rows k0 + 8 s + {0..7} (see st_tr_frag).
+__device__ __forceinline__ bf16x8 sn_tr_frag(const char* tile, int lane, int k0, int d0) {
+  const int i = lane & 15;
+  const int col = d0 + 4 * (i & 3);
+  const int r0 = k0 + 8 * (lane >> 4) + (i >> 2), r1 = r0 + 4;
+  const st_shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (st_lds_shortx4_ptr)(tile + r0 * ST_ROW_BYTES + (((col >> 3) ^ st_swz(r0)) * 16) + (col & 4) * 2));
+  const st_shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (st_lds_shortx4_ptr)(tile + r1 * ST_ROW_BYTES + (((col >> 3) ^ st_swz(r1)) * 16) + (col & 4) * 2));
+  typedef __attribute__((__vector_size__(8 * sizeof(short)))) short shortx8;
+  const shortx8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_bit_cast(bf16x8, v);
+}
+
+template <int NTE, int NCT, bool GATHER, bool BLOCK = false, bool ONCE = false>
+__device__ __forceinline__ void lora_stats_narrow_body(const StatsParams& p, const int block) {
+  constexpr int NST = SN_STAGES;
+  constexpr int IDX_SLOTS = NST + 1;
+  constexpr int Y_BYTES = SN_ROWS * NTE * 16 * 4;  // Y rows of a row tile, [t][R] f32; two of them
+  constexpr int Y_OFF = NST * SN_TILE_BYTES, IDX_OFF = Y_OFF + 2 * Y_BYTES;
+  __shared__ __attribute__((aligned(1024))) char ring[IDX_OFF + (GATHER ? 4 * IDX_SLOTS * 256 : 0)];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n16 = lane & 15, sub = lane >> 4;
+  int slab = block / p.n_chunks;
+  const int chunk = block - slab * p.n_chunks;
+  const bool grouped = p.offsets != nullptr;
+  if constexpr (BLOCK)
+    if (p.block.order != nullptr) slab = p.block.order[slab];
+  const int64_t t0 = grouped ? (int64_t)p.offsets[slab] : (int64_t)slab * p.rows_per_slab;
+  const int64_t c0 = (int64_t)chunk * p.cc;
+  const int rows_here = grouped ? p.offsets[slab + 1] - p.offsets[slab]
+                                : (int)(p.T - t0 < p.rows_per_slab ? p.T - t0 : p.rows_per_slab);
+  const int n_rt = (rows_here + SN_ROWS - 1) / SN_ROWS;
+  const int cols_here = (int)(p.C - c0 < p.cc ? p.C - c0 : p.cc);
+  const int nct = (cols_here + ST_TILE - 1) / ST_TILE;
+  const int nt = n_rt * nct;
+  const bool do_row = p.F != nullptr, do_col = p.Y != nullptr;
+  const int R = p.R;
+
+  // fragments of the chunk's factor: fa[ct][ks][et] = F[16 et + n16][c0 + 128 ct + 32 ks + 8 sub ..], zero past R and C
+  bf16x8 fa[NCT][4][NTE];
+  if (do_row) {
+    const uint16_t* F = grouped ? p.F + (int64_t)slab * R * p.C : p.F;
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int et = 0; et < NTE; ++et) {
+          const int e = 16 * et + n16;
+          const int64_t c = c0 + ct * ST_TILE + ks * 32 + sub * 8;
+          const bool ok = e < R && c < p.C;
+          const bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
+          const bf16x8 v = *(const bf16x8*)(F + (ok ? (int64_t)e * p.C + c : 0));
+          fa[ct][ks][et] = ok ? v : z;
+        }
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int et = 0; et < NTE; ++et) asm volatile("" : "+v"(fa[ct][ks][et]));  // in registers before the ring starts
+  }
+
+  const int64_t xbase = grouped ? 0 : t0;
+  const int64_t left = ((grouped ? p.x_rows : p.T) - xbase) * p.C * 2;
+  const dma_rsrc_t rsrc = dma_make_rsrc(p.X + xbase * p.C, (uint32_t)(left < 0x7fffffff ? left : 0x7fffffff));
+  const int64_t yleft = do_col ? (grouped ? (int64_t)rows_here : p.T - t0) * R * 4 : 0;
+  const dma_rsrc_t yrsrc =
+      dma_make_rsrc(do_col ? p.Y + t0 * R : nullptr, (uint32_t)(yleft < 0x7fffffff ? yleft : 0x7fffffff));
+  const uint32_t ring_addr = lds_addr_of(ring);
+  const dma_rsrc_t irsrc = dma_make_rsrc(GATHER ? p.gather + t0 : nullptr, GATHER ? (uint32_t)rows_here * 4u : 0u);
+  // the 16 indices of the wave's own rows of row tile q, ordered so that a lane reads its four as one 16-byte LDS load
+  auto issue_idx = [&](int q) {
+    int rg = q * SN_ROWS + wave * 16 + (lane & 3) * 4 + (n16 >> 2);
+    rg = rg < rows_here ? rg : rows_here - 1;
+    dma_load4(irsrc, rg * 4, 0, ring_addr + IDX_OFF + (wave * IDX_SLOTS + q % IDX_SLOTS) * 256);
+  };
+  const int row_bytes = (int)(p.C * 2);
+  auto issue_tile = [&](int i) {
+    const int rt = i / nct, ct = i - rt * nct;
+    const uint32_t stage = ring_addr + (i % NST) * SN_TILE_BYTES;
+    int gidx[4];
+    if constexpr (GATHER) {
+      const int4 ip = *(const int4*)(ring + IDX_OFF + (wave * IDX_SLOTS + rt % IDX_SLOTS) * 256 + sub * 16);
+      gidx[0] = ip.x; gidx[1] = ip.y; gidx[2] = ip.z; gidx[3] = ip.w;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int instr = wave * 4 + k;
+      const int row = instr * 4 + sub;
+      int xrow = rt * SN_ROWS + row;
+      xrow = xrow < rows_here ? xrow : rows_here - 1;
+      if constexpr (GATHER) xrow = gidx[k];
+      else if (grouped) xrow += (int)t0;
+      // (columns past the end re-read the row's first chunk: see above)
+      int col = (int)c0 + ct * ST_TILE + (n16 ^ st_swz(row)) * 8;
+      col = col < (int)p.C ? col : 0;
+      dma_load16<ONCE>(rsrc, xrow * row_bytes + col * 2, 0, stage + instr * 1024);
+    }
+  };
+  // Y rows of row tile rt: 64 R floats, R / 4 instructions per wave
+  auto issue_y = [&](int rt) {
+    for (int k = 0; k < R / 4; ++k) {
+      const int instr = wave * (R / 4) + k;
+      dma_load4(yrsrc, rt * SN_ROWS * R * 4 + instr * 256 + lane * 4, 0, ring_addr + Y_OFF + (rt & 1) * Y_BYTES + instr * 256);
+    }
+  };
+  if (nt > 0) {
+    if constexpr (GATHER) {
+#pragma unroll
+      for (int q = 0; q < NST; ++q)
+        if (q < n_rt) issue_idx(q);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    if (do_col) issue_y(0);
+#pragma unroll
+    for (int i = 0; i < NST - 1; ++i)
+      if (i < nt) issue_tile(i);
+  }
+
+  floatx4 acc_row[NTE];
+  floatx4 acc_col[NCT][2][NTE];
+  bf16x8 ya[2][NTE];  // Y^T fragments of the current row tile
+#pragma unroll
+  for (int et = 0; et < NTE; ++et) {
+    acc_row[et] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) acc_col[ct][0][et] = acc_col[ct][1][et] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  bool stored = false;  // the previous tile ended with NTE stores, newer than the tile after it
+  auto do_tile = [&](int rt, auto ct_tag) {
+    constexpr int ct = decltype(ct_tag)::value;
+    const int i = rt * nct + ct;
+    // tile i, and the Y rows and indices requested before tile i + 1, have landed; tile i + 1 may be on its way
+    if (i + 1 < nt) {
+      if (stored) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 + NTE) : "memory");
+      else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    barrier_lds_only();  // ... for every wave, and every wave is done with tile i - 1 and, at ct == 0, the last row tile's Y
+    stored = false;
+    if (ct == 0) {
+      if (do_col) {
+        const float* yr = (const float*)(ring + Y_OFF + (rt & 1) * Y_BYTES);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+          for (int et = 0; et < NTE; ++et) {
+            const int e = 16 * et + n16;
+            const int ec = e < R ? e : 0;
+            bf16x8 v;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const float y = yr[(32 * ks + 8 * sub + j) * R + ec];
+              v[j] = (__bf16)(e < R ? y : 0.f);
+            }
+            ya[ks][et] = v;
+          }
+        if (rt + 1 < n_rt) issue_y(rt + 1);
+      }
+      if constexpr (GATHER)
+        if (rt + NST < n_rt) issue_idx(rt + NST);
+    }
+    if (i + NST - 1 < nt) issue_tile(i + NST - 1);
+    const char* tile = ring + (i % NST) * SN_TILE_BYTES;
+    if (do_row) {
+      const int row = 16 * wave + n16;
+      const int sw = st_swz(row);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const bf16x8 xb = *(const bf16x8*)(tile + row * ST_ROW_BYTES + (((4 * ks + sub) ^ sw) * 16));
+#pragma unroll
+        for (int et = 0; et < NTE; ++et)
+          acc_row[et] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[ct][ks][et], xb, acc_row[et], 0, 0, 0);
+      }
+    }
+    if (do_col) {
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+          const bf16x8 xb = sn_tr_frag(tile, lane, 32 * ks, 32 * wave + 16 * nb);
+#pragma unroll
+          for (int et = 0; et < NTE; ++et)
+            acc_col[ct][nb][et] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ya[ks][et], xb, acc_col[ct][nb][et], 0, 0, 0);
+        }
+    }
+    if (do_row && ct == nct - 1) {
+      const int lrow = rt * SN_ROWS + 16 * wave + n16;
+#pragma unroll
+      for (int et = 0; et < NTE; ++et) {
+        // every lane stores (the wait above counts NTE stores): out of range goes to a dummy slot
+        const int e0 = 16 * et + 4 * sub;
+        const bool ok = lrow < rows_here && e0 < R;
+        float* dst = ok ? p.row_part + ((int64_t)chunk * p.T + t0 + lrow) * R + e0 : p.row_dummy + (tid & 255) * 4;
+        *(floatx4*)dst = acc_row[et];
+        acc_row[et] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+      stored = true;
+    }
+  };
+  for (int rt = 0; rt < n_rt; ++rt) {
+    do_tile(rt, std::integral_constant<int, 0>{});
+    if constexpr (NCT > 1) if (nct > 1) do_tile(rt, std::integral_constant<int, 1>{});
+    if constexpr (NCT > 2) if (nct > 2) do_tile(rt, std::integral_constant<int, 2>{});
+    if constexpr (NCT > 3) if (nct > 3) do_tile(rt, std::integral_constant<int, 3>{});
+  }
+  if (do_col) {
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb) {
+        const int64_t c = c0 + ct * ST_TILE + 32 * wave + 16 * nb + n16;
+        if (ct >= nct || c >= p.C) continue;
+#pragma unroll
+        for (int et = 0; et < NTE; ++et)
+          if (16 * et + 4 * sub < R) stats_put_col<BLOCK>(p, slab, grouped, c, 16 * et + 4 * sub, acc_col[ct][nb][et]);
+      }
+  }
+}
+
+template <int NTE, int NCT, bool GATHER, bool BLOCK = false, bool ONCE = false>
+__global__ __launch_bounds__(256, 2) void lora_stats_narrow_kernel(StatsParams p) {
+  lora_stats_narrow_body<NTE, NCT, GATHER, BLOCK, ONCE>(p, (int)blockIdx.x);
 }
 
 template <int NTE, int NCT, int NST, bool GATHER, bool BLOCK = false>
@@ -371,6 +620,13 @@ __global__ __launch_bounds__(256) void lora_stats_multi_kernel(StatsMulti m) {
   int i = 0;
   while (i + 1 < m.n && (int)blockIdx.x >= m.block0[i + 1]) ++i;
   lora_stats_body<NTE, NCT, NST, false>(m.p[i], (int)blockIdx.x - m.block0[i]);
+}
+
+template <int NTE, int NCT, bool ONCE>
+__global__ __launch_bounds__(256, 2) void lora_stats_narrow_multi_kernel(StatsMulti m) {
+  int i = 0;
+  while (i + 1 < m.n && (int)blockIdx.x >= m.block0[i + 1]) ++i;
+  lora_stats_narrow_body<NTE, NCT, false, false, ONCE>(m.p[i], (int)blockIdx.x - m.block0[i]);
 }
 
 // out[i][e] = scale * sum over parts (fixed order) of part[k][i][e]; written as f32 [n][R] (or
@@ -460,32 +716,39 @@ struct StatsGeom {
 // Cost of a grid in half tile times: rounds of work-groups on the CUs, each as long as its tiles
 // (a row tile of cct column tiles also writes its ROW partial, about half a tile time) plus
 // about two tile times of set-up (factor load, filling the ring, flushing the accumulators).
-static inline int64_t stats_grid_cost(int64_t blocks, int64_t row_tiles_per_block, int cct) {
-  const int64_t cus = num_cus();
-  return ((blocks + cus - 1) / cus) * (row_tiles_per_block * (2 * cct + 1) + 4);
+static inline int64_t stats_grid_cost(int64_t blocks, int64_t row_tiles_per_block, int cct, int64_t slots, int64_t setup) {
+  return ((blocks + slots - 1) / slots) * (row_tiles_per_block * (2 * cct + 1) + setup);
 }
 
-static inline StatsGeom stats_geom(int64_t T, int64_t C, int r) {
+// c_all: columns of all passes of the launch (the work-group slots are shared by them).
+static inline StatsGeom stats_geom(int64_t T, int64_t C, int r, int64_t c_all) {
   const int max_cct = r > 32 ? 2 : 4;  // column tiles per chunk the kernel holds accumulators for
-  const int64_t row_tiles = (T + ST_TILE - 1) / ST_TILE, col_tiles = (C + ST_TILE - 1) / ST_TILE;
+  const int tile_rows = r > 16 ? ST_TILE : SN_ROWS;
+  const int64_t row_tiles = (T + tile_rows - 1) / tile_rows, col_tiles = (C + ST_TILE - 1) / ST_TILE;
+  int64_t slots = num_cus();
+  if (r <= 16) {
+    slots = 2 * slots * C / c_all;
+    slots = slots < 1 ? 1 : slots;
+  }
   // row offsets inside a slab are 31-bit byte offsets
-  const int64_t cap = ((1ll << 31) - 1) / (2 * C) / ST_TILE;
+  const int64_t cap = ((1ll << 31) - 1) / (2 * C) / tile_rows;
   StatsGeom best{};
   int64_t best_cost = -1;
   for (int cct = max_cct; cct >= 1; --cct) {
     const int64_t n_chunks = (col_tiles + cct - 1) / cct;
-    int64_t want = num_cus() / n_chunks;
+    int64_t want = slots / n_chunks;
     want = want < 1 ? 1 : (want > row_tiles ? row_tiles : want);
     for (int64_t w = want; w <= want + 1 && w <= row_tiles; ++w) {
       int64_t slab_tiles = (row_tiles + w - 1) / w;
       if (slab_tiles > cap) slab_tiles = cap < 1 ? 1 : cap;
       const int64_t n_slabs = (row_tiles + slab_tiles - 1) / slab_tiles;
-      const int64_t cost = stats_grid_cost(n_slabs * n_chunks, slab_tiles, cct);
+      // (narrow: the write and the read of a slab's COL partial are cct r / 8 half tiles)
+      const int64_t cost = stats_grid_cost(n_slabs * n_chunks, slab_tiles, cct, slots, r <= 16 ? 4 + cct * r / 8 : 4);
       if (best_cost < 0 || cost < best_cost) {
         best_cost = cost;
         best.cc = cct * ST_TILE;
         best.n_chunks = (int)n_chunks;
-        best.rows_per_slab = (int)(slab_tiles * ST_TILE);
+        best.rows_per_slab = (int)(slab_tiles * tile_rows);
         best.n_slabs = (int)n_slabs;
       }
     }
@@ -518,31 +781,51 @@ static inline StatsParams stats_params(const void* X, int64_t T, int64_t C, cons
   return p;
 }
 
-static inline int32_t launch_stats(const void* X, int64_t T, int64_t C, const uint16_t* F, const float* Y, int r,
-                            const StatsGeom& g, float* row_part, float* col_part, float* row_dummy,
-                            hipStream_t st) {
-  const StatsParams p = stats_params(X, T, C, F, Y, r, g, row_part, col_part, row_dummy);
-  const unsigned grid = (unsigned)(g.n_slabs * g.n_chunks);
-  if (r > 32)
-    lora_stats_kernel<2, 2, 2, false><<<grid, 256, 0, st>>>(p);
-  else
-    lora_stats_kernel<1, 4, 3, false><<<grid, 256, 0, st>>>(p);
+// X that the 256 MiB Infinity Cache cannot hold is read with non-temporal loads, which leave alone what is in it:
+// 361 MB of upstream gradients 102 -> 75 us.  (201 MB that the kernel before has just written: 67 -> 72 us.)
+static inline bool stats_once(int64_t bytes) { return bytes > (256ll << 20); }
+
+// Which kernel takes a rank; the passes of one launch are all of one shape (the caller checks).
+enum StatsShape { STATS_NARROW, STATS_32, STATS_WIDE };
+static inline StatsShape stats_shape(int r) { return r > 32 ? STATS_WIDE : r > 16 ? STATS_32 : STATS_NARROW; }
+
+static inline int32_t launch_stats_params(const StatsParams& p, hipStream_t st) {
+  const unsigned grid = (unsigned)(p.n_slabs * p.n_chunks);
+  switch (stats_shape(p.R)) {
+    case STATS_WIDE: lora_stats_kernel<2, 2, 2, false><<<grid, 256, 0, st>>>(p); break;
+    case STATS_32: lora_stats_kernel<1, 4, 3, false><<<grid, 256, 0, st>>>(p); break;
+    case STATS_NARROW:
+      if (stats_once(p.T * p.C * 2)) lora_stats_narrow_kernel<1, 4, false, false, true><<<grid, 256, 0, st>>>(p);
+      else lora_stats_narrow_kernel<1, 4, false><<<grid, 256, 0, st>>>(p);
+      break;
+  }
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }
+static inline int32_t launch_stats(const void* X, int64_t T, int64_t C, const uint16_t* F, const float* Y, int r,
+                                   const StatsGeom& g, float* row_part, float* col_part, float* row_dummy,
+                                   hipStream_t st) {
+  return launch_stats_params(stats_params(X, T, C, F, Y, r, g, row_part, col_part, row_dummy), st);
+}
 
-// The passes of m in one launch; all ranks on the same side of 32 (the caller checks).
-static inline int32_t launch_stats_multi(StatsMulti& m, bool wide_rank, hipStream_t st) {
+// The passes of m in one launch.
+static inline int32_t launch_stats_multi(StatsMulti& m, StatsShape shape, hipStream_t st) {
   int blocks = 0;
+  int64_t bytes = 0;
   for (int i = 0; i < m.n; ++i) {
     m.block0[i] = blocks;
     blocks += m.p[i].n_slabs * m.p[i].n_chunks;
+    bytes += m.p[i].T * m.p[i].C * 2;
   }
   m.block0[m.n] = blocks;
-  if (wide_rank)
+  if (shape == STATS_WIDE)
     lora_stats_multi_kernel<2, 2, 2><<<(unsigned)blocks, 256, 0, st>>>(m);
-  else
+  else if (shape == STATS_32)
     lora_stats_multi_kernel<1, 4, 3><<<(unsigned)blocks, 256, 0, st>>>(m);
+  else if (stats_once(bytes))
+    lora_stats_narrow_multi_kernel<1, 4, true><<<(unsigned)blocks, 256, 0, st>>>(m);
+  else
+    lora_stats_narrow_multi_kernel<1, 4, false><<<(unsigned)blocks, 256, 0, st>>>(m);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }
@@ -550,31 +833,34 @@ static inline int32_t launch_stats_multi(StatsMulti& m, bool wide_rank, hipStrea
 
 // Grouped form: slab = expert.  ROW partials go to row_part [n_chunks][n_rows][r]; the COL
 // product of each expert is written to col_out, scaled.
-// Chunk width: the launch lasts as long as its work divided by the CUs, or as its longest expert, whichever is
-// more (half tile times as in stats_grid_cost, with twice the set-up: an expert's factor and results are its own).
+// Chunk width: the launch lasts as long as its work divided by the work-group slots, or as its longest expert, whichever
+// is more (half tile times as in stats_grid_cost, with twice the set-up: an expert's factor and results are its own).
 // Routing is uneven (of 8192 tokens, top-8 of 128 experts, the fullest expert gets 3 to 5 times the average), so
 // with one wide chunk per expert most CUs wait for the fullest one, unless it is dispatched first (`order`) and is
-// not too long; the estimate takes 2.5 times the average.  Measured at that size, us with the experts by index /
-// by falling length: rows of 2048 through the gather with the ROW product 112 / 71 (chunks of 512; 256: 79),
-// without it 89 / 57, 1536 columns 100 / 62 (chunks of 384; 512: 71), 768 columns 46 / 38 (chunks of 256; 384: 46).
+// not too long; the estimate takes 2.5 times the average.  The ROW partials of a chunk are written and read back.
+// Measured at that size, us for chunks of 128 / 256 / 384 / 512 columns (ranks up to 16, with the order): rows of 2048
+// through the gather with the ROW product 58 / 48 / 59 / 70, without it 48 / 43 / 54 / 63, 1536 columns with the
+// reduction 70 / 64 / 73 / 83, 768 columns 32 / 41 / 50 / 60; 203 tokens: 23 / 15 / 16 / 11, 16 / 12 / 12 / 10,
+// 20 / 15 / 11 / 12 and 7 / 6 / 7 / 8 (without the reductions).
 // A caller without an order for the experts (`block` false) assumes a couple of row tiles for each.
 static inline int stats_grouped_cc(int64_t n_rows, int64_t C, int r, int E, bool block) {
   const int max_cct = r > 32 ? 2 : 4;
   const int64_t col_tiles = (C + ST_TILE - 1) / ST_TILE;
-  const double avg = (double)n_rows / E / ST_TILE, tiles = avg > 1.0 ? avg + 0.5 : 1.0;
+  const int64_t slots = r > 16 ? num_cus() : 2 * num_cus();
+  const double avg = (double)n_rows / E / (r > 16 ? ST_TILE : SN_ROWS), tiles = avg > 1.0 ? avg + 0.5 : 1.0;
   int best = max_cct;
   double best_cost = -1.0;
   for (int cct = max_cct; cct >= 1; --cct) {
     const int64_t n_chunks = (col_tiles + cct - 1) / cct;
     double cost;
     if (block) {
-      double rounds = (double)(E * n_chunks) / num_cus();
+      double rounds = (double)(E * n_chunks) / slots;
       if (avg <= 1.0) rounds = ceil(rounds);  // (all alike: whole rounds)
       const double total = (rounds > 1.0 ? rounds : 1.0) * (tiles * (2 * cct + 1) + 8.0);
       const double longest = (avg > 1.0 ? 2.5 : 1.0) * tiles * (2 * cct + 1) + 8.0;
-      cost = total > longest ? total : longest;
+      cost = (total > longest ? total : longest) + (double)(E * n_chunks) / slots * tiles * r / 10.0;
     } else {
-      cost = (double)stats_grid_cost((int64_t)E * n_chunks, 2, cct);
+      cost = (double)stats_grid_cost((int64_t)E * n_chunks, r > 16 ? 2 : 4, cct, slots, 4);
     }
     if (best_cost < 0.0 || cost < best_cost) {
       best_cost = cost;
@@ -619,11 +905,15 @@ static inline int32_t launch_stats_grouped(const void* X, int64_t x_rows, const 
     if (gather) {
       if (r > 32)
         lora_stats_kernel<2, 2, 2, true, BLOCK><<<grid, 256, 0, st>>>(p);
+      else if (r <= 16)
+        lora_stats_narrow_kernel<1, 4, true, BLOCK><<<grid, 256, 0, st>>>(p);
       else
         lora_stats_kernel<1, 4, 3, true, BLOCK><<<grid, 256, 0, st>>>(p);
     } else {
       if (r > 32)
         lora_stats_kernel<2, 2, 2, false, BLOCK><<<grid, 256, 0, st>>>(p);
+      else if (r <= 16)
+        lora_stats_narrow_kernel<1, 4, false, BLOCK><<<grid, 256, 0, st>>>(p);
       else
         lora_stats_kernel<1, 4, 3, false, BLOCK><<<grid, 256, 0, st>>>(p);
     }

@@ -451,3 +451,23 @@ def test_forward_makes_no_transposed_weight(artk_lib, gpu):
     assert ops.known_transpose(layers[0].weight) is None
     for a, b in zip(grads(), grads()):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T,n_in,n_out,r", [
+    (1, 64, 64, 8), (63, 128, 192, 16), (65, 640, 448, 8),        # one row, around a 64-row tile, ragged 128-column tiles
+    (257, 64, 576, 16),                                           # one column tile: the ring runs over row tiles alone
+    (129, 4160, 1088, 8),                                         # several chunks of columns
+    (8192, 64, 16448, 16)])                                       # more than 256 MiB of g: non-temporal loads
+def test_skinny_passes_of_small_ranks(artk_lib, gpu, T, n_in, n_out, r):
+    """dA, dB and, through dx, g B at the edges of the one-pass backward of ranks up to 16.  TOL as above: bf16 factors
+    on the way."""
+    print(f"skinny passes T={T} in={n_in} out={n_out} r={r}", flush=True)
+    x, W, A, B, up = (t.to(gpu) for t in make(T, n_in, n_out, r, T + n_out, b_std=0.3))
+    scale = 2.0
+    _, xa = ops.lora_linear_fwd(x, W, A, B, scale)
+    dx, dA, dB = ops.lora_linear_bwd(up, x, ops.transpose(W), A, B, xa, scale)
+    g, xf, Af, Bf = up.float(), x.float(), A.float(), B.float()
+    gb = g @ Bf
+    assert rel_l2(dA, scale * gb.t() @ xf) <= TOL
+    assert rel_l2(dB, scale * g.t() @ (xf @ Af.t())) <= TOL
+    assert rel_l2(dx, g @ W.float() + scale * gb @ Af) <= TOL
