@@ -371,62 +371,110 @@ __global__ __launch_bounds__(256) void lora_small_reduce_kernel(LoraSmallParams 
 }
 
 // ----------------------------------------------------------------------------
-// Row products: out[t, j] = sum_k X[t,k] Mt[j,k], Mt [R,K].  A block owns 16 rows
-// of X and 16 rows j0..j0+15 of Mt (rows >= R read as zero); its 4 waves split K.
-// Writes f32 [T,R] (unscaled) and bf16 [T,RP] (scaled, zero padded to RP).
+// Row products of one X with several factors: out_i[t, j] = sum_k X[t,k] Mt_i[j,k], Mt_i [R_i,K], on MFMA 16x16x32.
+// The factor rows of all i are numbered through (e0[i] ..); a work-group takes 16 NJ of them (blockIdx.y) and 16 rows of
+// X.  K is dealt to its NW waves in pieces of 64 (two MFMA steps; a lane takes 32 contiguous bytes of its row, so a wave
+// reads whole cache lines), U of them in flight at a time.  Writes f32 [T,R] (unscaled) and bf16 [T,RP] (scaled, zero
+// padded to RP).
+// Where there are rows enough the factors are packed (e0 by R: two ranks of 8 are one block) and X is read once for
+// ranks that add up to 64; else every factor starts a block of its own (e0 by RP) and there are more work-groups.  us, a
+// work-group per 16 rows and factor / packed: [8192, 2048] and 2 ranks of 8 21 / 14, [4096, 2048] and 3 of 8 14 / 9,
+// [8192, 896] and 2 of 8 9 / 7, [1000, 3584] and 2 of 8 11 / 13.
 // ----------------------------------------------------------------------------
-__device__ __forceinline__ void rowdot16_body(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Mt,
-                                              int64_t T, int64_t K, int R, int RP, float scale,
-                                              float* __restrict__ out_f32, uint16_t* __restrict__ out_bf16,
-                                              int j0, floatx4 (*red)[64]) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int64_t t0 = (int64_t)blockIdx.x * 16;
-  int64_t trow = t0 + (lane & 15);
-  if (trow >= T) trow = T - 1;
-  const int jm = j0 + (lane & 15);
-  const uint16_t* xp = X + trow * K + (lane >> 4) * 8;
-  const uint16_t* mp = Mt + (int64_t)(jm < R ? jm : 0) * K + (lane >> 4) * 8;
-  floatx4 acc = rowdot_accumulate(xp, mp, jm < R, K, wave);
-  acc = rowdot_block_sum(acc, red);
-  if (wave == 0) {
-    // lane holds column j = lane % 16 of rows (lane / 16) * 4 + e
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int64_t t = t0 + (lane >> 4) * 4 + e;
-      if (t < T) {
-        if (jm < R) out_f32[t * R + jm] = acc[e];
-        out_bf16[t * RP + jm] = f32_to_bf16(acc[e] * scale);
-      }
-    }
-  }
-}
-
-__global__ __launch_bounds__(256) void rowdot16_kernel(const uint16_t* __restrict__ X,
-                                                       const uint16_t* __restrict__ Mt, int64_t T,
-                                                       int64_t K, int R, int RP, float scale,
-                                                       float* __restrict__ out_f32,
-                                                       uint16_t* __restrict__ out_bf16) {
-  __shared__ floatx4 red[3][64];
-  rowdot16_body(X, Mt, T, K, R, RP, scale, out_f32, out_bf16, blockIdx.y * 16, red);
-}
-
-// The same for several factors over one X in one launch: blockIdx.y walks the 16-row groups of
-// factor 0, then of factor 1, ...; each factor has its own outputs.
 struct RowdotMulti {
   const uint16_t* Mt[LORA_MAX_SEG];
   float* out_f32[LORA_MAX_SEG];
   uint16_t* out_bf16[LORA_MAX_SEG];
-  int R[LORA_MAX_SEG], RP[LORA_MAX_SEG], y0[LORA_MAX_SEG + 1];
+  int R[LORA_MAX_SEG], RP[LORA_MAX_SEG], e0[LORA_MAX_SEG + 1];
   int n;
 };
-__global__ __launch_bounds__(256) void rowdot16_multi_kernel(const uint16_t* __restrict__ X, RowdotMulti m,
-                                                             int64_t T, int64_t K, float scale) {
-  __shared__ floatx4 red[3][64];
-  const int by = blockIdx.y;
-  int i = 0;
-  while (i + 1 < m.n && by >= m.y0[i + 1]) ++i;
-  rowdot16_body(X, m.Mt[i], T, K, m.R[i], m.RP[i], scale, m.out_f32[i], m.out_bf16[i], (by - m.y0[i]) * 16, red);
+template <int NJ, int NW>
+__global__ __launch_bounds__(64 * NW) void rowdot_multi_kernel(const uint16_t* __restrict__ X, RowdotMulti m, int64_t T,
+                                                               int64_t K, float scale) {
+  constexpr int STEP = NW * 64, U = NW == 8 && NJ <= 2 ? 4 : 2;
+  __shared__ floatx4 red[NJ][NW][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t t0 = (int64_t)blockIdx.x * 16;
+  const int64_t trow = t0 + (lane & 15) < T ? t0 + (lane & 15) : T - 1;
+  const uint16_t *xp = X + trow * K + (lane >> 4) * 16, *mp[NJ];
+  bool ok[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int e = (blockIdx.y * NJ + j) * 16 + (lane & 15);
+    const uint16_t* f = m.Mt[0];
+    int el = e, R = m.R[0];
+#pragma unroll
+    for (int i = 1; i < LORA_MAX_SEG; ++i)
+      if (i < m.n && e >= m.e0[i]) {
+        f = m.Mt[i];
+        el = e - m.e0[i];
+        R = m.R[i];
+      }
+    ok[j] = el < R;
+    mp[j] = f + (int64_t)(ok[j] ? el : 0) * K + (lane >> 4) * 16;
+  }
+  const bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
+  floatx4 acc[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = wave * 64; k0 < K; k0 += U * STEP) {
+    bf16x8 f[U][2][NJ], x[U][2];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + u * STEP < K ? k0 + u * STEP : k0;  // (wave-uniform)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        x[u][h] = *(const bf16x8*)(xp + k + 8 * h);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) f[u][h][j] = *(const bf16x8*)(mp[j] + k + 8 * h);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // (or the scheduler sinks the loads to their MFMAs to save registers)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // (past the end both operands are zero: the re-read row may hold infinities; a branch would take the loads with it)
+      const bool in = k0 + u * STEP < K;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        x[u][h] = in ? x[u][h] : z;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[u][h], in && ok[j] ? f[u][h][j] : z, acc[j], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) red[j][wave][lane] = acc[j];
+  __syncthreads();
+  // wave j adds up block j, in a fixed order; a lane holds factor row lane % 16 of rows (lane / 16) * 4 + q
+  for (int j = wave; j < NJ; j += NW) {
+    floatx4 s = red[j][0][lane];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) s += red[j][w][lane];
+    const int e = (blockIdx.y * NJ + j) * 16 + (lane & 15);
+    float* of = m.out_f32[0];
+    uint16_t* ob = m.out_bf16[0];
+    int el = e, R = m.R[0], RP = m.RP[0];
+    bool packed = m.e0[1] == m.R[0];
+#pragma unroll
+    for (int i = 1; i < LORA_MAX_SEG; ++i)
+      if (i < m.n && e >= m.e0[i]) {
+        of = m.out_f32[i];
+        ob = m.out_bf16[i];
+        el = e - m.e0[i];
+        R = m.R[i];
+        RP = m.RP[i];
+        packed = m.e0[i + 1] - m.e0[i] == R;
+      }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int64_t t = t0 + (lane >> 4) * 4 + q;
+      if (t >= T || el >= RP) continue;
+      if (el < R) of[t * R + el] = s[q];
+      ob[t * RP + el] = el < R ? f32_to_bf16(s[q] * scale) : (uint16_t)0;
+      if (packed && el < R && el + 8 >= R && RP > R) ob[t * RP + el + 8] = 0;  // (R is a multiple of 8, RP the next of 16)
+    }
+  }
 }
 
 static int32_t check_lora(int64_t T, int64_t in, int64_t out, int r) {
@@ -563,12 +611,50 @@ static int32_t launch_lora_gemm(const void* P, const void* Q, const uint16_t* Pe
   return launch_lora_jobs(m, t, part, st);
 }
 
-// out_f32 [T,R] = X Mt^T (unscaled), out_bf16 [T,RP] = scale * that, zero padded.
-static int32_t launch_rowdot(const void* X, const void* Mt, int64_t T, int64_t K, int R, int RP,
-                             float scale, float* out_f32, uint16_t* out_bf16, hipStream_t st) {
-  dim3 grid((unsigned)((T + 15) / 16), (unsigned)(RP / 16));
-  rowdot16_kernel<<<grid, 256, 0, st>>>((const uint16_t*)X, (const uint16_t*)Mt, T, K, R, RP, scale,
-                                        out_f32, out_bf16);
+// Row products of a long K over few rows: one work-group per 16 rows leaves most CUs idle (2531 rows of 11008: 159
+// work-groups, 23 us, however many waves they have), so they run as the ROW half of the one-pass kernel, a work-group
+// per chunk of columns and slab of rows, and a reduction.
+// (us, product / split: rows x K 333 x 4864 11 / 10, 333 x 11008 19 / 11, 1200 x 18944 31 / 16, 2531 x 11008 20 / 17, 4090 x 11008 22 / 22;
+// the split is one launch more)
+static bool rowdot_split(int64_t T, int64_t K, int n, int r) { return n == 1 && r <= 16 && K >= 8192 && T < 12 * num_cus(); }
+static size_t rowdot_split_floats(int64_t T, int64_t K, int n, int r) {
+  return rowdot_split(T, K, n, r) ? (size_t)stats_geom(T, K, r, K).n_chunks * T * r + 1024 : 0;
+}
+// (part: rowdot_split_floats(T, K, 1, r) floats)
+static int32_t launch_rowdot_split(const void* X, const void* Mt, int64_t T, int64_t K, int r, int RP, float scale,
+                                   float* out_f32, uint16_t* out_bf16, float* part, hipStream_t st) {
+  const StatsGeom g = stats_geom(T, K, r, K);
+  int32_t rc = launch_stats(X, T, K, (const uint16_t*)Mt, nullptr, r, g, part + 1024, nullptr, part, st);
+  if (rc) return rc;
+  return launch_stats_reduce(StatsReduceJob{part + 1024, g.n_chunks, T, 1.f, out_f32, 0, out_bf16, RP, scale},
+                             StatsReduceJob{nullptr, 0, 0, 0.f, nullptr, 0, nullptr, 0, 0.f}, r, st);
+}
+
+// Fills m.e0 and launches.
+static int32_t launch_rowdot(const void* X, RowdotMulti& m, int64_t T, int64_t K, float scale, hipStream_t st) {
+  const bool pack = m.n > 1 && T >= 16 * num_cus();
+  int e = 0;
+  for (int i = 0; i < m.n; ++i) {
+    m.e0[i] = e;
+    e += pack ? m.R[i] : m.RP[i];
+  }
+  for (int i = m.n; i <= LORA_MAX_SEG; ++i) m.e0[i] = e;
+  const int nj = (e + 15) / 16;
+  auto launch = [&](auto nj_tag, auto nw_tag) {
+    constexpr int NJ = decltype(nj_tag)::value, NW = decltype(nw_tag)::value;
+    rowdot_multi_kernel<NJ, NW><<<dim3((unsigned)((T + 15) / 16), (unsigned)((nj + NJ - 1) / NJ)), 64 * NW, 0, st>>>(
+        (const uint16_t*)X, m, T, K, scale);
+  };
+  using four = std::integral_constant<int, 4>;
+  using eight = std::integral_constant<int, 8>;
+  auto waves = [&](auto nj_tag) {
+    // (by the shape alone: a projection has the same sums alone and among others)
+    if (T >= 16 * num_cus() && K >= 1536 && K <= 2048) launch(nj_tag, eight{});
+    else launch(nj_tag, four{});
+  };
+  if (!pack || nj == 1) waves(std::integral_constant<int, 1>{});
+  else if (nj == 2) waves(std::integral_constant<int, 2>{});
+  else waves(four{});
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }
@@ -588,6 +674,7 @@ size_t artk_lora_linear_fwd_workspace_bytes(int64_t T, int64_t in, int64_t out, 
   Workspace ws(nullptr, 0);
   ws.take<uint16_t>((size_t)T * round16(r));  // s * x A^T, bf16 [T,RP]
   ws.take<float>(lora_tiling_one(T, in, out).part_floats());
+  ws.take<float>(rowdot_split_floats(T, in, 1, r));
   return ws.used + 256;
 }
 
@@ -605,12 +692,22 @@ int32_t artk_lora_linear_fwd(const void* x, const void* W, const void* A, const 
   uint16_t* xa16 = ws.take<uint16_t>((size_t)T * RP);
   const LoraTiling tiling = lora_tiling_one(T, in, out);
   float* part = ws.take<float>(tiling.part_floats());
+  float* rpart = ws.take<float>(rowdot_split_floats(T, in, 1, r));
   if (!ws.ok()) {
     set_error("workspace too small: need %zu bytes, got %zu", ws.used, workspace_bytes);
     return ARTK_ERR_WORKSPACE_TOO_SMALL;
   }
   hipStream_t st = (hipStream_t)stream;
-  if ((rc = launch_rowdot(x, A, T, in, r, RP, scale, xa, xa16, st))) return rc;
+  RowdotMulti m;
+  m.n = 1;
+  m.Mt[0] = (const uint16_t*)A;
+  m.out_f32[0] = xa;
+  m.out_bf16[0] = xa16;
+  m.R[0] = r;
+  m.RP[0] = RP;
+  if (rowdot_split(T, in, 1, r)) rc = launch_rowdot_split(x, A, T, in, r, RP, scale, xa, xa16, rpart, st);
+  else rc = launch_rowdot(x, m, T, in, scale, st);
+  if (rc) return rc;
   return launch_lora_gemm(W, x, (const uint16_t*)B, xa16, (const uint16_t*)bias, y, out, T, in, r, RP, tiling, part, st);
 }
 
@@ -717,6 +814,7 @@ size_t artk_lora_linear_multi_fwd_workspace_bytes(int64_t T, int64_t in, const a
   Workspace ws(nullptr, 0);
   for (int i = 0; i < n; ++i) ws.take<uint16_t>((size_t)T * round16(proj[i].r));
   ws.take<float>(lora_tiling_fwd(proj, n, T, in).part_floats());
+  ws.take<float>(rowdot_split_floats(T, in, n, proj[0].r));
   return ws.used + 256;
 }
 
@@ -731,6 +829,7 @@ int32_t artk_lora_linear_multi_fwd(const void* x, const artk_lora_proj_t* proj, 
   for (int i = 0; i < n; ++i) xa16[i] = ws.take<uint16_t>((size_t)T * round16(proj[i].r));
   const LoraTiling tiling = lora_tiling_fwd(proj, n, T, in);
   float* part = ws.take<float>(tiling.part_floats());
+  float* rpart = ws.take<float>(rowdot_split_floats(T, in, n, proj[0].r));
   if (!ws.ok()) {
     set_error("workspace too small: need %zu bytes, got %zu", ws.used, workspace_bytes);
     return ARTK_ERR_WORKSPACE_TOO_SMALL;
@@ -739,7 +838,7 @@ int32_t artk_lora_linear_multi_fwd(const void* x, const artk_lora_proj_t* proj, 
   RowdotMulti m;
   LoraMultiParams p;
   m.n = n;
-  int y = 0, tile = 0;
+  int tile = 0;
   p.N = T;
   p.NT = (int)((T + TILE - 1) / TILE);
   p.n_jobs = n;
@@ -751,18 +850,17 @@ int32_t artk_lora_linear_multi_fwd(const void* x, const artk_lora_proj_t* proj, 
     m.out_bf16[i] = xa16[i];
     m.R[i] = q.r;
     m.RP[i] = RP;
-    m.y0[i] = y;
-    y += RP / 16;
     p.seg[i] = LoraSeg{q.W, x, (const uint16_t*)q.B, xa16[i], in, q.r, RP};
     const int MT = (int)((q.out + TILE - 1) / TILE);
     p.job[i] = LoraJob{(uint16_t*)q.y, (const uint16_t*)q.bias, q.out, MT, tile, i, 1};
     tile += MT * p.NT;
   }
-  m.y0[n] = y;
   p.n_tiles = tile;
-  dim3 grid((unsigned)((T + 15) / 16), (unsigned)y);
-  rowdot16_multi_kernel<<<grid, 256, 0, st>>>((const uint16_t*)x, m, T, in, scale);
-  ARTK_CHECK_LAUNCH();
+  if (rowdot_split(T, in, n, proj[0].r))
+    rc = launch_rowdot_split(x, proj[0].A, T, in, proj[0].r, round16(proj[0].r), scale, proj[0].xa, xa16[0], rpart, st);
+  else
+    rc = launch_rowdot(x, m, T, in, scale, st);
+  if (rc) return rc;
   return launch_lora_jobs(p, tiling, part, st);
 }
 

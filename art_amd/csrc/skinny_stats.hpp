@@ -465,13 +465,13 @@ __device__ __forceinline__ void lora_stats_narrow_body(const StatsParams& p, con
       const int instr = wave * 4 + k;
       const int row = instr * 4 + sub;
       int xrow = rt * SN_ROWS + row;
-      xrow = xrow < rows_here ? xrow : rows_here - 1;
+      // What lies past the last row or column is read past the end of the descriptor and arrives as zeros (elements of the
+      // matrix in its place could be infinities, of which a zero in the other operand would make NaN).
+      const int col = (int)c0 + ct * ST_TILE + (n16 ^ st_swz(row)) * 8;
+      const bool in = xrow < rows_here && col < (int)p.C;
       if constexpr (GATHER) xrow = gidx[k];
       else if (grouped) xrow += (int)t0;
-      // (columns past the end re-read the row's first chunk: see above)
-      int col = (int)c0 + ct * ST_TILE + (n16 ^ st_swz(row)) * 8;
-      col = col < (int)p.C ? col : 0;
-      dma_load16<ONCE>(rsrc, xrow * row_bytes + col * 2, 0, stage + instr * 1024);
+      dma_load16<ONCE>(rsrc, in ? xrow * row_bytes + col * 2 : -16, 0, stage + instr * 1024);
     }
   };
   // Y rows of row tile rt: 64 R floats, R / 4 instructions per wave

@@ -466,8 +466,41 @@ def test_skinny_passes_of_small_ranks(artk_lib, gpu, T, n_in, n_out, r):
     scale = 2.0
     _, xa = ops.lora_linear_fwd(x, W, A, B, scale)
     dx, dA, dB = ops.lora_linear_bwd(up, x, ops.transpose(W), A, B, xa, scale)
+    # an infinity in the last row and column reaches its own sums only
+    up2, x2 = up.clone(), x.clone()
+    up2[-1, -1] = float("inf")
+    x2[-1, -1] = float("inf")
+    _, dA2, dB2 = ops.lora_linear_bwd(up2, x2, ops.transpose(W), A, B, xa.clamp(min=0.5), scale)
+    assert torch.isfinite(dB2[:-1]).all() and torch.isinf(dB2[-1]).all()
+    assert torch.isfinite(dA2[:, :-1]).sum() == 0
     g, xf, Af, Bf = up.float(), x.float(), A.float(), B.float()
     gb = g @ Bf
     assert rel_l2(dA, scale * gb.t() @ xf) <= TOL
     assert rel_l2(dB, scale * g.t() @ (xf @ Af.t())) <= TOL
     assert rel_l2(dx, g @ W.float() + scale * gb @ Af) <= TOL
+
+
+@pytest.mark.parametrize("T,n_in,ranks", [
+    (4097, 64, (8, 24, 16, 40)),      # packed: blocks of 16 factor rows over several ranks, 6 of them
+    (4100, 1600, (8, 8, 8)),          # packed, eight waves, the last pieces of K short
+    (5000, 192, (64, 64, 64, 64)),
+    (37, 448, (8, 16)),               # few rows: every factor starts its own block
+    (37, 8256, (16,)), (2000, 8192, (8,)),  # long K over few rows: split over the chunks of the one-pass kernel
+])
+def test_row_products(artk_lib, gpu, T, n_in, ranks):
+    """x A_i^T of every way the row products are dealt out, element by element: fp32 sums of bf16 products, in another
+    order than the reference's, are off by at most about sqrt(K) 2^-24 of sum |x a|; 2e-6 of it is eight times that here."""
+    print(f"row products T={T} in={n_in} ranks={ranks}", flush=True)
+    g = torch.Generator().manual_seed(T + n_in)
+    x = torch.randn(T, n_in, generator=g).to(torch.bfloat16).to(gpu)
+    x[0, :4] = float("inf")            # reaches its own row only
+    rand = lambda *s: (0.1 * torch.randn(*s, generator=g)).to(torch.bfloat16).to(gpu)
+    Ws, As, Bs = [rand(64, n_in) for _ in ranks], [rand(r, n_in) for r in ranks], [rand(64, r) for r in ranks]
+    for A in As:
+        A[:, :4] = A[:, :4].abs() + 0.1
+    _, xas = ops.lora_linear_multi_fwd(x, Ws, As, Bs, 2.0)
+    for A, xa in zip(As, xas):
+        assert torch.isinf(xa[0]).all()
+        ref = x[1:].double() @ A.double().t()
+        bound = x[1:].double().abs() @ A.double().abs().t()
+        assert ((xa[1:].double() - ref).abs() <= 2e-6 * bound).all()
