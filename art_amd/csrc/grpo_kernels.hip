@@ -508,12 +508,14 @@ __global__ __launch_bounds__(256) void grpo_loss_tok_kernel(LossParams p) {
 }
 
 // K2: merge the per-tile (max, sumexp) partials of each position.  A block
-// handles 16 positions; 16 threads per position each merge a strided share of
-// the partials online, then the 16 shares are merged through LDS.
+// handles 16 positions; 64 threads per position each merge a strided share of
+// the partials online (a chain of dependent merges: with 16 of them it was 16 us for
+// 317 positions), then the shares are merged, four within a wave and 16 through LDS.
 // logprob is indexed by position (whole batch), lse by chunk row.  A target that is no vocabulary id gives NaN.
 // LOSS: the loss terms of the row follow at once (the fused step; a launch of its own otherwise).
+constexpr int LSE_SHARES = 64;
 template <bool LOSS>
-__global__ __launch_bounds__(256) void lse_finalize_kernel(const float2* __restrict__ part,
+__global__ __launch_bounds__(16 * LSE_SHARES) void lse_finalize_kernel(const float2* __restrict__ part,
                                                            int nparts, int64_t Tc, ChunkRows rows,
                                                            const float* __restrict__ sel,
                                                            const int64_t* __restrict__ ids, int64_t S, int shift,
@@ -526,16 +528,16 @@ __global__ __launch_bounds__(256) void lse_finalize_kernel(const float2* __restr
   float m = -INFINITY, l = 0.f;
   if (t < n) {
     // eight loads in flight per thread (the merge itself is a dependent chain), same merge order
-    for (int i0 = sl; i0 < nparts; i0 += 16 * 8) {
+    for (int i0 = sl; i0 < nparts; i0 += LSE_SHARES * 8) {
       float2 v[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const int i = i0 + 16 * u;
+        const int i = i0 + LSE_SHARES * u;
         v[u] = i < nparts ? part[(int64_t)i * Tc + t] : make_float2(-INFINITY, 0.f);
       }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        if (i0 + 16 * u >= nparts) break;
+        if (i0 + LSE_SHARES * u >= nparts) break;
         const float mn = fmaxf(m, v[u].x);
         if (mn != -INFINITY)
           l = l * __builtin_amdgcn_exp2f((m - mn) * LOG2E) + v[u].y * __builtin_amdgcn_exp2f((v[u].x - mn) * LOG2E);
@@ -543,7 +545,13 @@ __global__ __launch_bounds__(256) void lse_finalize_kernel(const float2* __restr
       }
     }
   }
-  red[sl][tl] = make_float2(m, l);
+#pragma unroll
+  for (int d = 16; d < 64; d <<= 1) {
+    const float mo = __shfl_xor(m, d, 64), lo = __shfl_xor(l, d, 64), mn = fmaxf(m, mo);
+    if (mn != -INFINITY) l = l * __builtin_amdgcn_exp2f((m - mn) * LOG2E) + lo * __builtin_amdgcn_exp2f((mo - mn) * LOG2E);
+    m = mn;
+  }
+  if ((sl & 3) == 0) red[sl >> 2][tl] = make_float2(m, l);
   __syncthreads();
   if (sl == 0 && t < n) {
     float M = -INFINITY;
@@ -626,6 +634,7 @@ __global__ __launch_bounds__(1024) void compact_rows_kernel(const float* __restr
                                                             int* __restrict__ sched) {
   __shared__ int wave_tot[16];
   __shared__ int total;
+  __shared__ float split_eff[1024];
   const int Tc = rows.n();
   const int per = (rows.cap + 1023) / 1024;
   const int r0 = threadIdx.x * per;
@@ -665,17 +674,28 @@ __global__ __launch_bounds__(1024) void compact_rows_kernel(const float* __restr
       pos[r] = -1;
     }
   }
+  const int n = total;
+  const int tta = (n + TILE - 1) / TILE;
+  const int tiles = HT * tta;
+  {
+    // how full the rounds of ns = threadIdx.x + 1 splits are; negative: not allowed (and none after it)
+    const int ns = threadIdx.x + 1;
+    float eff = -1.f;
+    if (tiles > 0 && ns <= max_splits(tiles, num_cus) &&
+        (ns == 1 || (ksteps / ns >= 32 && ns * tta * TILE <= part_rows))) {
+      const int blocks = tiles * ns;
+      const int rounds = (blocks + num_cus - 1) / num_cus;
+      eff = (float)blocks / ((float)rounds * num_cus);
+    }
+    split_eff[threadIdx.x] = eff;
+  }
+  __syncthreads();
   if (threadIdx.x == 0) {
-    const int n = total;
-    const int tta = (n + TILE - 1) / TILE;
-    const int tiles = HT * tta;
     int best = 1;
     float best_eff = 0.f;
-    for (int ns = 1; tiles > 0 && ns <= max_splits(tiles, num_cus); ++ns) {
-      if (ns > 1 && (ksteps / ns < 32 || ns * tta * TILE > part_rows)) break;
-      int blocks = tiles * ns;
-      int rounds = (blocks + num_cus - 1) / num_cus;
-      float eff = (float)blocks / ((float)rounds * num_cus);
+    for (int ns = 1; ns <= 1024; ++ns) {
+      const float eff = split_eff[ns - 1];
+      if (eff < 0.f) break;
       if (eff > best_eff + 0.02f) {
         best_eff = eff;
         best = ns;
@@ -853,6 +873,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   } else if (pr >= 0) {
     const int nsplit = sched[2];
     const int64_t rows_per_split = (int64_t)sched[1] * TILE;
+#pragma unroll 8
     for (int k = 0; k < nsplit; ++k)
       s += ((const floatx4*)(partial + ((int64_t)k * rows_per_split + pr) * H))[c];
     const float cf = coef[r];
@@ -1113,10 +1134,10 @@ static int32_t launch_fwd_chunk(const void* hidden, const void* lm_head, const i
   ARTK_CHECK_LAUNCH();
   const unsigned fin = (unsigned)((Tc + 15) / 16);
   if (fused)
-    lse_finalize_kernel<true><<<fin, 256, 0, st>>>(part, 2 * p.VT, Tc, rows, sel, ids, S, shift, V, logprob, lse_chunk,
+    lse_finalize_kernel<true><<<fin, 16 * LSE_SHARES, 0, st>>>(part, 2 * p.VT, Tc, rows, sel, ids, S, shift, V, logprob, lse_chunk,
                                                    fused->loss);
   else
-    lse_finalize_kernel<false><<<fin, 256, 0, st>>>(part, 2 * p.VT, Tc, rows, sel, ids, S, shift, V, logprob,
+    lse_finalize_kernel<false><<<fin, 16 * LSE_SHARES, 0, st>>>(part, 2 * p.VT, Tc, rows, sel, ids, S, shift, V, logprob,
                                                     lse_chunk, LossParams{});
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
