@@ -18,6 +18,25 @@ namespace artk {
 
 constexpr int SUMSQ_BLOCKS = 1024;
 
+// Loads and stores of what a step touches once.  A step over more than the 256 MiB Infinity Cache holds finds nothing
+// of it there the next time, and reading and writing it past the cache leaves the gradients, which the norm has just
+// read, in it: 20.2 M elements with 8-bit moments 103 -> 94 us a step (loads or stores alone: no gain; the gradients
+// too: 110).
+// With fp32 moments a step of 449 MB still finds enough there (78 us, 80 past the cache); 605 MB: 117 -> 104 us.
+static inline bool step_once8(int64_t n) { return 18 * n > (256ll << 20); }
+static inline bool step_once32(int64_t n) { return 30 * n > (512ll << 20); }
+template <bool ONCE, class T>
+__device__ __forceinline__ T once_load(const T* p) {
+  if constexpr (ONCE) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+template <bool ONCE, class T>
+__device__ __forceinline__ void once_store(T v, T* p) {
+  if constexpr (ONCE) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+
 // part[b] = sum of x[i]^2 over the slice of block b, accumulated in double in a
 // fixed order; sumsq_final_kernel adds the partials in index order.
 __global__ __launch_bounds__(256) void sumsq_partial_kernel(const float* __restrict__ x, int64_t n,
@@ -74,6 +93,7 @@ __device__ __forceinline__ float adamw_one(float& p, float g, float& m, float& v
   return p;
 }
 
+template <bool ONCE>
 __global__ __launch_bounds__(256) void adamw_kernel(AdamWParams a) {
   float clip = 1.f;
   if (a.grad_sumsq != nullptr) {
@@ -84,18 +104,22 @@ __global__ __launch_bounds__(256) void adamw_kernel(AdamWParams a) {
   const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= a.n) return;
   if (i + 4 <= a.n) {
-    float4 p = *(float4*)(a.p + i), m = *(float4*)(a.m + i), v = *(float4*)(a.v + i);
-    const float4 g = *(const float4*)(a.g + i);
-    adamw_one(p.x, g.x, m.x, v.x, a, clip);
-    adamw_one(p.y, g.y, m.y, v.y, a, clip);
-    adamw_one(p.z, g.z, m.z, v.z, a, clip);
-    adamw_one(p.w, g.w, m.w, v.w, a, clip);
-    *(float4*)(a.p + i) = p;
-    *(float4*)(a.m + i) = m;
-    *(float4*)(a.v + i) = v;
+    const f32x4 p4 = once_load<ONCE>((const f32x4*)(a.p + i)), m4 = once_load<ONCE>((const f32x4*)(a.m + i));
+    const f32x4 v4 = once_load<ONCE>((const f32x4*)(a.v + i)), g4 = *(const f32x4*)(a.g + i);
+    float p[4], m[4], v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      p[j] = p4[j];
+      m[j] = m4[j];
+      v[j] = v4[j];
+      adamw_one(p[j], g4[j], m[j], v[j], a, clip);
+    }
+    once_store<ONCE>(f32x4{p[0], p[1], p[2], p[3]}, (f32x4*)(a.p + i));
+    once_store<ONCE>(f32x4{m[0], m[1], m[2], m[3]}, (f32x4*)(a.m + i));
+    once_store<ONCE>(f32x4{v[0], v[1], v[2], v[3]}, (f32x4*)(a.v + i));
     if (a.p_bf16) {
-      const uint32_t lo = (uint32_t)f32_to_bf16(p.x) | ((uint32_t)f32_to_bf16(p.y) << 16);
-      const uint32_t hi = (uint32_t)f32_to_bf16(p.z) | ((uint32_t)f32_to_bf16(p.w) << 16);
+      const uint32_t lo = (uint32_t)f32_to_bf16(p[0]) | ((uint32_t)f32_to_bf16(p[1]) << 16);
+      const uint32_t hi = (uint32_t)f32_to_bf16(p[2]) | ((uint32_t)f32_to_bf16(p[3]) << 16);
       *(uint2*)(a.p_bf16 + i) = make_uint2(lo, hi);
     }
   } else {
@@ -134,44 +158,78 @@ struct AdamW8Params {
   float eps_scaled;  // sqrt(1 - beta2^t) * eps
 };
 
-// Nearest entry of an ascending 256-entry code book (ties to the lower index).  A bisection is eight
-// dependent LDS gathers per value, 16 per element for the two moments, and was what this kernel waited
-// for (182 us for 20.2 M elements, 2.0 TB/s).  Instead the leading 16 bits of the fp32 value (sign,
-// exponent, 7 mantissa bits) select a byte: the last entry that is not above anything in that bin.  The
-// search walks up from there; the books in use have at most one or two entries per bin (the finest
-// octave, [0.5, 1), holds 71), any other ascending book only walks further.
+// Nearest entry of an ascending 256-entry code book (ties to the lower index): entry k up to thr[k], the largest value
+// that is not nearer to entry k + 1.  The leading 16 bits of the fp32 value (sign, exponent, 7 mantissa bits) select a
+// byte: the first entry whose threshold is not below everything in that bin.  In the books in use no bin holds two
+// thresholds (the finest octave, [0.5, 1), has 71 entries in 128 bins), so the code is that byte, or one more where the
+// value is above its threshold: two LDS gathers and no loop.  A book with a fuller bin walks up from there, over the
+// entries themselves.  (A bisection, eight dependent gathers per value, took 182 us for 20.2 M elements; a start byte and
+// a walk that compares with two neighbours 84 us, 137 vector instructions per element.)
 constexpr int LUT_E0 = 104;                      // exponents 104 .. 127: [2^-23, 1]; smaller values share bin 0
 constexpr int LUT_HALF = (128 - LUT_E0) * 128;   // bins of one sign
 constexpr int LUT_BINS = 2 * LUT_HALF;           // ascending: negative bins first
 // (in LDS by sign bit, then magnitude, so that an index is one multiply-add)
 
-// Lower end of bin j (ascending order), -inf for the first one.
+// Lower end of bin j (ascending order), -inf for the first one, inf past the last.
 __device__ __forceinline__ float lut_edge(int j) {
   if (j == LUT_HALF) return 0.f;
+  if (j >= LUT_BINS) return INFINITY;
   if (j > LUT_HALF) return __uint_as_float((uint32_t)(j - LUT_HALF + LUT_E0 * 128) << 16);
   return j == 0 ? -INFINITY : -__uint_as_float((uint32_t)(LUT_HALF - j + LUT_E0 * 128) << 16);
 }
 
-__device__ void build_lut(uint8_t* lut, const float* map, int tid, int nthreads) {
+// The largest float that the rule gives to entry `cur` rather than to the next one, and whether it was found (within 32
+// floats of the middle; always, in an ascending book).
+__device__ bool code_threshold(float cur, float next, float& thr) {
+  auto lower = [&](float x) { return x < next && x - cur <= next - x; };
+  auto key = [](float x) {  // floats in the order of integers, and back
+    const int i = (int)__float_as_uint(x);
+    return i < 0 ? (int)0x80000000 - i : i;
+  };
+  auto val = [](int k) { return __uint_as_float((uint32_t)(k < 0 ? (int)0x80000000 - k : k)); };
+  int k = key(0.5f * cur + 0.5f * next);
+  bool found = false;
+  for (int step = 0; step < 32 && !found; ++step) {
+    const bool here = lower(val(k)), above = lower(val(k + 1));
+    found = here && !above;
+    if (!found) k += here ? 1 : -1;
+  }
+  thr = val(k);
+  return found;
+}
+
+// Start bytes and whether two gathers do (thr[255] is infinite).
+__device__ bool build_lut(uint8_t* lut, const float* thr, int tid, int nthreads) {
   const int per = LUT_BINS / nthreads;
-  int lo = 0, hi = 255;
+  int lo = -1, hi = 255;  // thr[lo] < first <= thr[hi]
   const float first = lut_edge(tid * per);
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
-    if (map[mid] <= first) lo = mid; else hi = mid;
+    if (thr[mid] < first) lo = mid; else hi = mid;
   }
+  bool one = true;
   for (int j = tid * per; j < (tid + 1) * per; ++j) {
-    const float e = lut_edge(j);
-    while (lo < 254 && map[lo + 1] <= e) ++lo;
-    lut[j < LUT_HALF ? LUT_BINS - 1 - j : j - LUT_HALF] = (uint8_t)lo;
+    const float e = lut_edge(j), end = lut_edge(j + 1);
+    while (hi < 255 && thr[hi] < e) ++hi;
+    lut[j < LUT_HALF ? LUT_BINS - 1 - j : j - LUT_HALF] = (uint8_t)hi;
+    one = one && (hi >= 254 || thr[hi + 1] >= end);
   }
+  return one;
 }
 
-__device__ __forceinline__ int nearest_code(const float* map, const uint8_t* lut, float x) {
+template <bool ONE>
+__device__ __forceinline__ int nearest_code(const float* map, const float* thr, const uint8_t* lut, float x) {
   const uint32_t u = __float_as_uint(x);
   int k = (int)(u >> 16 & 0x7fff) - LUT_E0 * 128;
   k = k < 0 ? 0 : (k > LUT_HALF - 1 ? LUT_HALF - 1 : k);
   int lo = lut[k + (int)(u >> 31) * LUT_HALF];
+  if constexpr (ONE) {
+    lo += x > thr[lo] ? 1 : 0;
+    return x != x ? 1 : lo;
+  }
+  // (entries at or before the start byte's may be the nearest one of a book without thresholds)
+  lo = lo > 254 ? 254 : lo;
+  while (lo > 0 && map[lo] > x) --lo;
   float cur = map[lo], next = map[lo + 1];
   while (lo < 254 && next <= x) {
     ++lo;
@@ -206,14 +264,15 @@ struct BlockMax {
 // One wave = one block of 256 elements, 4 consecutive elements per lane: 16-byte loads of parameters and
 // gradients, 4-byte loads of the codes, block maxima by wave reduction without a barrier.  18 B per
 // element, of which the gradient's second read after the norm comes from the Infinity Cache.  The grid
-// is two work-groups of 16 waves per CU that walk the blocks, so the two tables are built once per
-// work-group and not once per 256 elements.  20.2 M elements: 182 us as one work-group per block with a
-// bisection, 104 us with the start table; the vector instructions bound it then, and quotients without divisions
-// and fewer spilled registers took another 16 us off the step (123 -> 107 us with the norm).
+// is two work-groups of 16 waves per CU that walk the blocks, so the tables are built once per
+// work-group and not once per 256 elements.  20.2 M elements, this kernel alone: 182 us as one work-group per block with a
+// bisection, 104 us with a start table, 84 us with quotients without divisions, 75 us with thresholds in place of
+// neighbours.
 constexpr int ADAM8_THREADS = 1024;
 
+template <bool ONCE>
 __global__ __launch_bounds__(ADAM8_THREADS, 8) void adamw8bit_kernel(AdamW8Params a, int64_t n_blocks, int vec) {
-  __shared__ float map1[256], map2[256];
+  __shared__ float map1[256], map2[256], thr1[256], thr2[256];
   __shared__ uint8_t lut1[LUT_BINS], lut2[LUT_BINS];
   const int tid = threadIdx.x, lane = tid & 63;
   if (tid < 256) map1[tid] = a.qmap1[tid];
@@ -224,9 +283,19 @@ __global__ __launch_bounds__(ADAM8_THREADS, 8) void adamw8bit_kernel(AdamW8Param
     clip = c < 1.f ? c : 1.f;
   }
   __syncthreads();
-  build_lut(lut1, map1, tid, ADAM8_THREADS);
-  build_lut(lut2, map2, tid, ADAM8_THREADS);
-  __syncthreads();
+  bool ok = true;
+  if (tid < 512) {
+    const float* map = tid < 256 ? map1 : map2;
+    float* thr = tid < 256 ? thr1 : thr2;
+    const int k = tid & 255;
+    float t = INFINITY;
+    if (k < 255) ok = code_threshold(map[k], map[k + 1], t);
+    thr[k] = t;
+  }
+  ok = __syncthreads_and(ok);
+  ok = build_lut(lut1, thr1, tid, ADAM8_THREADS) && ok;
+  ok = build_lut(lut2, thr2, tid, ADAM8_THREADS) && ok;
+  const bool one = __syncthreads_and(ok);  // (the same for the whole work-group)
   const int64_t stride = (int64_t)gridDim.x * (ADAM8_THREADS / 64);
   for (int64_t b = (int64_t)blockIdx.x * (ADAM8_THREADS / 64) + (tid >> 6); b < n_blocks; b += stride) {
     const int64_t i = b * 256 + lane * 4;
@@ -235,9 +304,9 @@ __global__ __launch_bounds__(ADAM8_THREADS, 8) void adamw8bit_kernel(AdamW8Param
     uint32_t c1 = 0, c2 = 0;
     if (full) {
       *(float4*)g = *(const float4*)(a.g + i);
-      *(float4*)pv = *(const float4*)(a.p + i);
-      c1 = *(const uint32_t*)(a.c1 + i);
-      c2 = *(const uint32_t*)(a.c2 + i);
+      *(f32x4*)pv = once_load<ONCE>((const f32x4*)(a.p + i));
+      c1 = once_load<ONCE>((const uint32_t*)(a.c1 + i));
+      c2 = once_load<ONCE>((const uint32_t*)(a.c2 + i));
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -278,7 +347,7 @@ __global__ __launch_bounds__(ADAM8_THREADS, 8) void adamw8bit_kernel(AdamW8Param
       if (a.weight_decay > 0.f) pv[j] = pv[j] * (1.f - a.lr * a.weight_decay);
     }
     if (full) {
-      *(float4*)(a.p + i) = *(float4*)pv;
+      once_store<ONCE>(*(f32x4*)pv, (f32x4*)(a.p + i));
       if (a.p_bf16)
         *(uint2*)(a.p_bf16 + i) = make_uint2((uint32_t)f32_to_bf16(pv[0]) | ((uint32_t)f32_to_bf16(pv[1]) << 16),
                                              (uint32_t)f32_to_bf16(pv[2]) | ((uint32_t)f32_to_bf16(pv[3]) << 16));
@@ -294,14 +363,21 @@ __global__ __launch_bounds__(ADAM8_THREADS, 8) void adamw8bit_kernel(AdamW8Param
     if (!(mx1 > 0.f)) m[0] = m[1] = m[2] = m[3] = 0.f;
     if (!(mx2 > 0.f)) v[0] = v[1] = v[2] = v[3] = 0.f;
     c1 = c2 = 0;
+    if (one) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      c1 |= (uint32_t)nearest_code(map1, lut1, q1.quotient(m[j])) << (8 * j);
-      c2 |= (uint32_t)nearest_code(map2, lut2, q2.quotient(v[j])) << (8 * j);
+      for (int j = 0; j < 4; ++j) {
+        c1 |= (uint32_t)nearest_code<true>(map1, thr1, lut1, q1.quotient(m[j])) << (8 * j);
+        c2 |= (uint32_t)nearest_code<true>(map2, thr2, lut2, q2.quotient(v[j])) << (8 * j);
+      }
+    } else {
+      for (int j = 0; j < 4; ++j) {
+        c1 |= (uint32_t)nearest_code<false>(map1, thr1, lut1, q1.quotient(m[j])) << (8 * j);
+        c2 |= (uint32_t)nearest_code<false>(map2, thr2, lut2, q2.quotient(v[j])) << (8 * j);
+      }
     }
     if (full) {
-      *(uint32_t*)(a.c1 + i) = c1;
-      *(uint32_t*)(a.c2 + i) = c2;
+      once_store<ONCE>(c1, (uint32_t*)(a.c1 + i));
+      once_store<ONCE>(c2, (uint32_t*)(a.c2 + i));
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -368,7 +444,8 @@ int32_t artk_adamw_step(float* params, const float* grads, float* exp_avg, float
   a.step_size = (float)((double)lr / bc1);
   a.inv_bc2_sqrt = (float)(1.0 / sqrt(bc2));
   const int64_t n4 = (n + 3) / 4;
-  adamw_kernel<<<(unsigned)((n4 + 255) / 256), 256, 0, (hipStream_t)stream>>>(a);
+  if (step_once32(n)) adamw_kernel<true><<<(unsigned)((n4 + 255) / 256), 256, 0, (hipStream_t)stream>>>(a);
+  else adamw_kernel<false><<<(unsigned)((n4 + 255) / 256), 256, 0, (hipStream_t)stream>>>(a);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }
@@ -410,7 +487,8 @@ int32_t artk_adamw8bit_step(float* params, const float* grads, void* state1, voi
   // 16-byte accesses where every buffer allows them (buffers of FlatParams do)
   const int vec = aligned16(params) && aligned16(grads) && (((uintptr_t)state1 | (uintptr_t)state2) & 3) == 0 &&
                   ((uintptr_t)params_bf16 & 7) == 0;
-  adamw8bit_kernel<<<(unsigned)grid, ADAM8_THREADS, 0, (hipStream_t)stream>>>(a, n_blocks, vec);
+  if (step_once8(n)) adamw8bit_kernel<true><<<(unsigned)grid, ADAM8_THREADS, 0, (hipStream_t)stream>>>(a, n_blocks, vec);
+  else adamw8bit_kernel<false><<<(unsigned)grid, ADAM8_THREADS, 0, (hipStream_t)stream>>>(a, n_blocks, vec);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }

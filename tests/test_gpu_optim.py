@@ -193,3 +193,36 @@ def test_adamw8bit_non_finite_gradients(artk_lib, gpu):
         want[[512 + 5, 768 + 7]] = 1
         assert (c == want).all()
         assert np.isnan(a[0]) and a[1] == 0 and np.isinf(a[2]) and np.isclose(a[3], one, rtol=1e-5) and a[4] == 0
+
+
+@pytest.mark.parametrize("moments", ["8 bit", "fp32"])
+def test_steps_past_the_cache_match_steps_of_parts(artk_lib, gpu, moments):
+    """A step over more than the caches hold reads and writes past them: bit for bit the steps of its parts."""
+    from art_amd.optim import dynamic_code_book
+
+    n = 256 * 74000  # 18.9 M: above both limits, the parts below
+    print("adamw past the cache", moments, n, flush=True)
+    gen = torch.Generator(device=gpu).manual_seed(3)
+    rand = lambda s: torch.randn(n, generator=gen, device=gpu) * s
+    p, g = rand(0.05), rand(0.01)
+    parts = [slice(0, 256 * 30000), slice(256 * 30000, n)]
+    if moments == "fp32":
+        m, v = rand(1e-3), rand(1e-3).abs()
+        state = [p, g, m, v, torch.zeros(n, dtype=torch.bfloat16, device=gpu)]
+        step = lambda t: ops.adamw_step(*t, 1e-3, 0.9, 0.99, 1e-8, 0.1, 3)
+        cut = lambda s: [t[s].clone() for t in state]
+    else:
+        c = [torch.randint(0, 256, (n,), generator=gen, device=gpu).to(torch.uint8) for _ in range(2)]
+        a = [torch.rand(n // 256, generator=gen, device=gpu) * x for x in (1e-3, 1e-6)]
+        books = [dynamic_code_book(True).to(gpu), dynamic_code_book(False).to(gpu)]
+        state = [p, g, *c, *a, *books, torch.zeros(n, dtype=torch.bfloat16, device=gpu)]
+        step = lambda t: ops.adamw8bit_step(*t, 1e-3, 0.9, 0.99, 1e-8, 0.1, 3)
+        at = lambda t, s: t if t.numel() == 256 else t[slice(s.start // 256, s.stop // 256)] if t.numel() < n else t[s]
+        cut = lambda s: [at(t, s).clone() for t in state]
+    small = [cut(s) for s in parts]
+    for t in small:
+        step(t)
+    step(state)
+    for i, t in enumerate(state):
+        if t.numel() != 256:
+            assert torch.equal(t, torch.cat([x[i] for x in small])), i
