@@ -162,18 +162,9 @@ __device__ __forceinline__ bool attn_visible(int i, int j, int gi, int pi, int g
 __device__ __forceinline__ uint32_t attn_entry(uint32_t any, uint32_t all) {
   return any ? ((all == 0xfu ? 2u : 1u) << 14) | (any << 16) | (all << 24) : 0u;
 }
-__global__ __launch_bounds__(256) void attn_classify_kernel(const int* __restrict__ gc, const int* __restrict__ pc,
-                                                            const int2* __restrict__ uni, int64_t stride, int nKb,
-                                                            int nQb2, uint32_t* __restrict__ info,
-                                                            uint32_t* __restrict__ info2) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = blockIdx.z, owner = blockIdx.y, kb = blockIdx.x * 4 + wave;
-  if (kb >= nKb) return;
-  gc = attn_row(gc, stride, row);
-  pc = attn_row(pc, stride, row);
-  uni = attn_row(uni, stride, row);
-  info = attn_row(info, stride, row);
-  info2 = attn_row(info2, stride, row);
+// info_row: the query block's row of info.
+__device__ __forceinline__ void attn_classify_pair(const int* gc, const int* pc, const int2* uni, int nQb2, int owner, int kb, uint32_t* info_row, uint32_t* info2) {
+  const int lane = threadIdx.x & 63;
   uint32_t any = 0, all = 0;   // bit 2 w + kg: cell of queries 32 w.., keys 32 kg..
   if (kb * ATT_BN <= owner * ATT_BM + ATT_BM - 1) {
     const int qc = owner * (ATT_BM / 32) + ((lane & 7) >> 1), kc = kb * 2 + (lane & 1);  // lanes 0..7: one cell each
@@ -203,10 +194,19 @@ __global__ __launch_bounds__(256) void attn_classify_kernel(const int* __restric
       a4 |= (uint32_t)((any >> (2 * w) & 3u) != 0u) << w;
       l4 |= (uint32_t)((all >> (2 * w) & 3u) == 3u) << w;
     }
-    info[(int64_t)owner * nKb + kb] = attn_entry(a4, l4);
+    info_row[kb] = attn_entry(a4, l4);
     info2[(int64_t)kb * nQb2 + 2 * owner] = attn_entry(any & 0xfu, all & 0xfu);
     info2[(int64_t)kb * nQb2 + 2 * owner + 1] = attn_entry(any >> 4, all >> 4);
   }
+}
+__global__ __launch_bounds__(256) void attn_classify_kernel(const int* __restrict__ gc, const int* __restrict__ pc,
+                                                            const int2* __restrict__ uni, int64_t stride, int nKb,
+                                                            int nQb2, uint32_t* __restrict__ info,
+                                                            uint32_t* __restrict__ info2) {
+  const int row = blockIdx.z, owner = blockIdx.y, kb = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (kb >= nKb) return;
+  attn_classify_pair(attn_row(gc, stride, row), attn_row(pc, stride, row), attn_row(uni, stride, row), nQb2, owner, kb,
+                     attn_row(info, stride, row) + (int64_t)owner * nKb, attn_row(info2, stride, row));
 }
 
 // list[row][0..cnt[row]) = tile index | info for the tiles of info[row][*] that
@@ -308,6 +308,108 @@ static size_t attn_plan_layout(void* base, size_t bytes, int64_t S, AttnPlan& pl
   pl.n_heads = ws.take<int>(1);
   pl.stride = (int64_t)align_up(ws.used, 256);
   return ws.ok() || base == nullptr ? ws.used : (size_t)-1;
+}
+
+// The plan of a short row in two launches instead of the chain of five above (18 us and the gaps between them in front of
+// a layer of 60 us at 1009 positions).  In the first, a work-group per query block finds the codes of the whole row for
+// itself, in LDS, and classifies and lists its own tiles, a wave per 64 keys; the second lists the tiles of the key blocks
+// and sorts.  Every array of the plan gets the values that the chain writes.  (In one launch with one work-group per row
+// the mixed cells of the whole row take 30 us on their one CU.)
+constexpr int ATT_SHORT = 1024;  // positions, padded
+__global__ __launch_bounds__(1024) void attn_plan_short_kernel(const int64_t* __restrict__ group_ids,
+                                                               const int64_t* __restrict__ parent_ids, int S, AttnPlan pl) {
+  static_assert(ATT_SHORT <= 1024 && ATT_SHORT / ATT_BN <= 16, "one position per thread, a key tile per wave");
+  __shared__ int64_t hid[ATT_SHORT];
+  __shared__ int hpos[ATT_SHORT], gc[ATT_SHORT], pc[ATT_SHORT];
+  __shared__ int2 uni[ATT_SHORT / 32];
+  __shared__ uint32_t info[16];
+  __shared__ int wtot[16];
+  const int row = blockIdx.y, owner = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int padded = pl.nKb * ATT_BN;
+  const bool in = t < S;
+  const int64_t g = in ? group_ids[(int64_t)row * S + t] : 0, pa = in ? parent_ids[(int64_t)row * S + t] : 0;
+
+  // positions where a run of equal group ids begins
+  const int64_t prev = in && t > 0 ? group_ids[(int64_t)row * S + t - 1] : 0;
+  const bool head = in && (t == 0 || g != prev);
+  const unsigned long long hm = __ballot(head);
+  if (lane == 0) wtot[wave] = __popcll(hm);
+  __syncthreads();
+  int at = __popcll(hm & ((1ull << lane) - 1ull)), nh = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    at += w < wave ? wtot[w] : 0;
+    nh += wtot[w];
+  }
+  if (head) {
+    hpos[at] = t;
+    hid[at] = g;
+    if (owner == 0) attn_row(pl.heads, pl.stride, row)[at] = t;
+  }
+  if (owner == 0 && t == 0) *attn_row(pl.n_heads, pl.stride, row) = nh;
+  __syncthreads();
+
+  // codes
+  int first_g = -1, first_p = -2;
+  for (int j = nh - 1; j >= 0; --j) {  // descending: the first match wins
+    const int64_t id = hid[j];
+    if (id == g) first_g = hpos[j];
+    if (id == pa) first_p = hpos[j];
+  }
+  const int gcv = in ? first_g : -3 - t, pcv = in ? first_p : -2;
+  gc[t] = gcv;
+  pc[t] = pcv;
+  const int base = lane & 32;
+  const unsigned long long mine = 0xffffffffull << base;
+  const bool ug = (__ballot(gcv == __shfl(gcv, base, 64)) & mine) == mine;
+  const bool up = (__ballot(pcv == __shfl(pcv, base, 64)) & mine) == mine;
+  if (owner == 0 && t < padded) {
+    attn_row(pl.gc, pl.stride, row)[t] = gcv;
+    attn_row(pl.pc, pl.stride, row)[t] = pcv;
+  }
+  if ((lane & 31) == 0) {
+    const int2 u = make_int2(ug ? gcv : ATT_MIXED, up ? pcv : ATT_MIXED);
+    uni[t / 32] = u;
+    if (owner == 0 && t < padded) attn_row(pl.uni, pl.stride, row)[t / 32] = u;
+  }
+  __syncthreads();
+
+  if (wave < pl.nKb)
+    attn_classify_pair(gc, pc, uni, pl.nQb2, owner, wave, info, attn_row(pl.info2, pl.stride, row));
+  __syncthreads();
+  if (wave == 0) {
+    const uint32_t v = lane < pl.nKb ? info[lane] : 0u;
+    const unsigned long long m = __ballot(v != 0);
+    if (v) attn_row(pl.list, pl.stride, row)[owner * pl.nKb + __popcll(m & ((1ull << lane) - 1ull))] = (uint32_t)lane | v;
+    if (lane < pl.nKb) attn_row(pl.info, pl.stride, row)[owner * pl.nKb + lane] = v;
+    if (lane == 0) attn_row(pl.cnt, pl.stride, row)[owner] = __popcll(m);
+  }
+}
+
+__global__ __launch_bounds__(1024) void attn_plan_short_order_kernel(AttnPlan pl) {
+  __shared__ int cnt2[16];
+  const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (wave < pl.nKb2) {
+    const uint32_t v = lane < pl.nQb2 ? attn_row(pl.info2, pl.stride, row)[wave * pl.nQb2 + lane] : 0u;
+    const unsigned long long m = __ballot(v != 0);
+    if (v) attn_row(pl.list2, pl.stride, row)[wave * pl.nQb2 + __popcll(m & ((1ull << lane) - 1ull))] = (uint32_t)lane | v;
+    if (lane == 0) attn_row(pl.cnt2, pl.stride, row)[wave] = cnt2[wave] = __popcll(m);
+  }
+  __syncthreads();
+  // order of dispatch, by rank: wave 0 the query blocks, wave 1 the key blocks
+  if (wave < 2) {
+    const bool second = wave == 1;
+    const int m = second ? pl.nKb2 : pl.nQb;
+    const int mine = lane < m ? (second ? cnt2[lane] : attn_row(pl.cnt, pl.stride, row)[lane]) : 0;
+    int rank = 0, sum = 0;
+    for (int i = 0; i < m; ++i) {
+      const int c = __shfl(mine, i, 64);
+      sum += c;
+      rank += (c > mine || (c == mine && i > lane)) ? 1 : 0;
+    }
+    if (second && lane == 0) *attn_row(pl.total2, pl.stride, row) = sum;
+    if (lane < m) attn_row(second ? pl.order2 : pl.order, pl.stride, row)[rank] = lane;
+  }
 }
 
 // ----------------------------------------------------------------------------
@@ -1273,6 +1375,13 @@ int32_t artk_attn_plan_rows(const int64_t* group_ids, const int64_t* parent_ids,
   }
   hipStream_t st = (hipStream_t)stream;
   const unsigned b = (unsigned)B;
+  if (attn_padded(S) <= ATT_SHORT) {
+    attn_plan_short_kernel<<<dim3((unsigned)pl.nQb, b), 1024, 0, st>>>(group_ids, parent_ids, (int)S, pl);
+    ARTK_CHECK_LAUNCH();
+    attn_plan_short_order_kernel<<<b, 1024, 0, st>>>(pl);
+    ARTK_CHECK_LAUNCH();
+    return ARTK_OK;
+  }
   attn_heads_kernel<<<b, 1024, 0, st>>>(group_ids, (int)S, pl.stride, pl.heads, pl.n_heads);
   ARTK_CHECK_LAUNCH();
   attn_codes_kernel<<<dim3((unsigned)(attn_padded(S) / 256), b), 256, 0, st>>>(group_ids, parent_ids, (int)S, pl.stride,

@@ -417,3 +417,57 @@ def test_packed_attention_any_layout(artk_lib, gpu, S, view):
         assert torch.equal(got, ref)
     with pytest.raises(ValueError):
         packed_attention(make(whole[0]), *whole[1:3], plans)
+
+
+def plan_arrays(plan, S):
+    """The arrays of a row's plan (S: padded) by name, from the layout the library documents by its allocator: in order,
+    each at the next multiple of 256 bytes."""
+    q, k = S // 128, S // 64
+    buf, off, out = plan.buf.cpu(), 0, {}
+    for name, n, shape in (("gc", S, (S,)), ("pc", S, (S,)), ("info", q * k, (q, k)), ("list", q * k, (q, k)), ("cnt", q, (q,)),
+                           ("order", q, (q,)), ("info2", k * k, (k, k)), ("list2", k * k, (k, k)), ("cnt2", k, (k,)),
+                           ("order2", k, (k,)), ("total2", 1, (1,)), ("uni", S // 16, (S // 32, 2)), ("heads", S, (S,)),
+                           ("n_heads", 1, (1,))):
+        off = (off + 255) // 256 * 256
+        out[name] = buf[off:off + 4 * n].view(torch.int32).view(*shape)
+        off += 4 * n
+    return out
+
+
+@pytest.mark.parametrize("S", [1, 31, 64, 130, 256, 257, 700, 1009, 1024])
+@pytest.mark.parametrize("ids", ["packed", "random", "one"])
+def test_plan_of_a_short_row_is_that_of_a_long_one(artk_lib, gpu, S, ids):
+    """Rows of up to 1024 positions have their plan from one work-group, longer ones from a chain of kernels.  Continued by
+    positions whose ids occur nowhere else, a short row becomes a long one with the same visibility."""
+    print(f"short plan S={S} ids={ids}", flush=True)
+    g = torch.Generator().manual_seed(S)
+    if ids == "packed" and S >= 130:
+        group, parent = synthetic.packed_row_ids(S, S, 2, S // 20 + 1, 3, S // 8)
+    elif ids == "one":
+        group, parent = torch.zeros(S, dtype=torch.int64), torch.zeros(S, dtype=torch.int64)
+    else:
+        group, parent = (torch.randint(-4, 5, (S,), generator=g) * (1 << 40) for _ in range(2))
+    pad, L = (S + 255) // 256 * 256, 2048
+    more = torch.arange(L - S) + (1 << 50)
+    rows = lambda a, b: ops.attn_plan_rows(torch.stack([a, a.flip(0)]).to(gpu), torch.stack([b, b.flip(0)]).to(gpu))
+    short = rows(group, parent)
+    long = rows(torch.cat([group, more]), torch.cat([parent, more + (1 << 51)]))
+    long_flip = ops.attn_plan_rows(torch.cat([group.flip(0), more]).unsqueeze(0).to(gpu),
+                                   torch.cat([parent.flip(0), more + (1 << 51)]).unsqueeze(0).to(gpu))
+    for plan, ref in ((short[0], long[0]), (short[1], long_flip[0])):
+        a, b = plan_arrays(plan, pad), plan_arrays(ref, L)
+        assert torch.equal(a["gc"][:S], b["gc"][:S]) and torch.equal(a["pc"], b["pc"][:pad])
+        for t, q in (("", pad // 128), ("2", pad // 64)):
+            k = pad // 64
+            assert torch.equal(a["info" + t], b["info" + t][:q, :k])
+            assert torch.equal(a["cnt" + t], b["cnt" + t][:q])
+            for i in range(q):
+                n = int(a["cnt" + t][i])
+                assert torch.equal(a["list" + t][i, :n], b["list" + t][i, :n])
+            cnt = a["cnt" + t].tolist()
+            assert a["order" + t].tolist() == sorted(range(q), key=lambda i: (-cnt[i], -i))
+        assert int(a["total2"]) == int(a["cnt2"].sum())
+        n = int(a["n_heads"])
+        assert n == int((b["heads"][:int(b["n_heads"])] < S).sum()) and torch.equal(a["heads"][:n], b["heads"][:n])
+        whole = S // 32
+        assert torch.equal(a["uni"][:whole], b["uni"][:whole])
