@@ -371,6 +371,94 @@ __global__ __launch_bounds__(256) void lora_small_reduce_kernel(LoraSmallParams 
 }
 
 // ----------------------------------------------------------------------------
+// The same jobs on 256 x 256 tiles with the K range of a tile in `split` parts, for long products of a few tiles: unit =
+// tile * split + part, one work-group each; every part leaves its fp32 accumulators in `part` as
+// [unit][wave][mi][ni][4][lane][4] and lora_split_reduce_kernel adds them in order.  Tiles are numbered as for the
+// persistent kernels (job[].tile0 and MT count 256-row tiles).  Bound by the main loop: half the bytes into LDS per product
+// of a 128 x 128 tile, for 0.25 MiB of partials a unit.
+// ----------------------------------------------------------------------------
+__global__ __launch_bounds__(nthreads<LORA_NI>()) void lora_split_gemm_kernel(LoraSmallParams p) {
+  __shared__ __attribute__((aligned(1024))) char smem[GEMM_LDS_BYTES];
+  // ids run through the tiles of a part first: the 32 work-groups of an XCD share panels of one K range
+  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  const int part = id / p.m.n_tiles, tile = id - part * p.m.n_tiles, unit = tile * p.split + part;
+  int j, mt, nt;
+  lora_small_locate(p, tile, j, mt, nt);
+  const LoraJob& job = p.m.job[j];
+  const int total = p.ksteps[j];
+  const int b = (int)((int64_t)total * part / p.split), e = (int)((int64_t)total * (part + 1) / p.split);
+  // the segments that the part's K steps b .. e - 1 fall into (no part is empty); off: first step of segment s0
+  int s0 = 0, off = 0;
+  while (b >= off + (int)(p.m.seg[job.seg0 + s0].K / BK)) off += (int)(p.m.seg[job.seg0 + s0++].K / BK);
+  TileAcc<LORA_NI> acc;
+  acc.zero();
+  // (one branch around all segments, and no segment skipped inside: see gemm_plain8.hpp)
+  if (plain8_leader()) {
+    int at = off, s = s0;
+    do {
+      const LoraSeg& sg = p.m.seg[job.seg0 + s];
+      const int ks = (int)(sg.K / BK), lo = b > at ? b - at : 0, hi = e - at < ks ? e - at : ks;
+      PlainTileLoaders cur;
+      cur.init(sg.P, sg.K, (int64_t)mt * TILE, job.M, sg.Q, sg.K, (int64_t)nt * TILE, p.m.N, lo * BK, hi * BK);
+      cur.issue_first_leader(smem);
+      gemm_tile_run<2, 2, false>(acc, smem, cur);
+      at += ks;
+      ++s;
+    } while (at < e);
+  } else {
+    int at = off, s = s0;
+    do {
+      const int ks = (int)(p.m.seg[job.seg0 + s].K / BK), lo = b > at ? b - at : 0, hi = e - at < ks ? e - at : ks;
+      const NoLoaders none{lo * BK, hi * BK};
+      gemm_tile_run<2, 2, false>(acc, smem, none);
+      at += ks;
+      ++s;
+    } while (at < e);
+  }
+  // rank-r steps, by the first part
+  for (int s = 0; s < (part == 0 ? job.nseg : 0); ++s) {
+    const LoraSeg& sg = p.m.seg[job.seg0 + s];
+    if (sg.Pe != nullptr) lora_tile_lowrank(acc, sg.Pe, sg.r, sg.Qe, sg.RP, job.M, p.m.N, mt, nt);
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float* dst = p.part + ((int64_t)unit * 8 + wave) * 8192 + lane * 4;
+#pragma unroll
+  for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < LORA_NI; ++ni)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *(floatx4*)(dst + (mi * LORA_NI + ni) * 1024 + 256 * q) =
+            floatx4{acc.c[mi][ni][4 * q], acc.c[mi][ni][4 * q + 1], acc.c[mi][ni][4 * q + 2], acc.c[mi][ni][4 * q + 3]};
+}
+
+// One wave per 32 x 32 block: 16 work-groups per tile.
+__global__ __launch_bounds__(256) void lora_split_reduce_kernel(LoraSmallParams p) {
+  const int lane = threadIdx.x & 63;
+  const int tile = blockIdx.x >> 4, blk = (blockIdx.x & 15) * 4 + (threadIdx.x >> 6);  // blk = wave * 8 + mi * 2 + ni
+  const int wave = blk >> 3, mi = (blk >> 1) & 3, ni = blk & 1;
+  int j, mt, nt;
+  lora_small_locate(p, tile, j, mt, nt);
+  const LoraJob& job = p.m.job[j];
+  const int64_t m0 = (int64_t)mt * TILE + wave_m<LORA_NI>(wave) * 128 + mi * 32;
+  const int64_t col = (int64_t)nt * TILE + acc_col<LORA_NI>(wave_n<LORA_NI>(wave), ni, lane);
+  if (m0 >= job.M || (int64_t)nt * TILE + wave_n<LORA_NI>(wave) * 64 + ni * 32 >= p.m.N) return;  // wave-uniform
+  floatx16 c;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) c[k] = 0.f;
+  const float* src = p.part + ((int64_t)tile * p.split * 64 + blk) * 1024 + lane * 4;
+#pragma unroll 4
+  for (int s = 0; s < p.split; ++s)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const floatx4 v = *(const floatx4*)(src + (int64_t)s * 65536 + 256 * q);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) c[4 * q + k] += v[k];
+    }
+  lora_block_store(c, job.bias, job.out, job.M, p.m.N, m0, col, lane >> 5);
+}
+
+// ----------------------------------------------------------------------------
 // Row products of one X with several factors: out_i[t, j] = sum_k X[t,k] Mt_i[j,k], Mt_i [R_i,K], on MFMA 16x16x32.
 // The factor rows of all i are numbered through (e0[i] ..); a work-group takes 16 NJ of them (blockIdx.y) and 16 rows of
 // X.  K is dealt to its NW waves in pieces of 64 (two MFMA steps; a lane takes 32 contiguous bytes of its row, so a wave
@@ -490,11 +578,15 @@ static int32_t check_lora(int64_t T, int64_t in, int64_t out, int r) {
   return ARTK_OK;
 }
 
-// How the products of one call run: 256 x 256 tiles (split == 0) or 128 x 128 tiles with the K range in `split` parts.
+// How the products of one call run: 256 x 256 tiles (split == 0), 128 x 128 tiles with the K range in `split` parts, or
+// 256 x 256 tiles in `split` parts (wide).
 struct LoraTiling {
   int split;
-  int tiles;  // 128 x 128 tiles of all jobs
-  size_t part_floats() const { return split > 1 ? (size_t)tiles * split * ST2 * ST2 : 0; }
+  int tiles;  // 128 x 128 tiles of all jobs; wide: 256 x 256
+  bool wide = false;
+  size_t part_floats() const {
+    return wide ? (size_t)tiles * split * TILE * TILE : split > 1 ? (size_t)tiles * split * ST2 * ST2 : 0;
+  }
 };
 // M and K steps of the n jobs over N columns.
 // The estimate, in us, was fitted to both paths over 200 to 8192 rows and in / out sizes of 896 to 44032 (168
@@ -527,6 +619,23 @@ static LoraTiling lora_tiling(const int64_t* M, const int64_t* ksteps, int n, in
     if (c < cost) {
       cost = c;
       best.split = split;
+    }
+  }
+  // 256 x 256 tiles in parts: a round of work-groups at the rate of its fill, then the partials' write and read.  Both
+  // sides, us with the reduction (best of the other two / in parts): rows x K -> M 2531 x 11008 -> 2048 139 / 114,
+  // 1500 x 11008 -> 2048 85 / 74, 4090 x 11008 -> 2048 182 / 169, 1200 x 18944 -> 3584 264 / 190, 2500 x 18944 -> 3584
+  // 449 / 399, 1300 x 22016 -> 2048 170 / 125, 2000 x 22016 -> 2048 200 / 172, 1300 x 37888 -> 3584 481 / 363.
+  for (int split = 2; split <= 8 && split * 16 <= k; ++split) {
+    const int64_t units = tiles2 * split;
+    if (units > 2 * cus) break;
+    const double f = units < cus ? (double)units / (double)cus : 1.0;
+    const double c = 0.93 * (8.0 + (double)((units + cus - 1) / cus * ((k + split - 1) / split)) * (1.0 + 0.45 * f)) + 7.0 +
+                     0.11 * (double)units;
+    if (c < cost) {
+      cost = c;
+      best.split = split;
+      best.tiles = (int)tiles2;
+      best.wide = true;
     }
   }
   return best;
@@ -572,6 +681,18 @@ static int32_t launch_lora_jobs(const LoraMultiParams& m, const LoraTiling& t, f
     } else {
       lora_multi_gemm_kernel<<<(unsigned)(m.n_tiles < cus ? m.n_tiles : cus), nthreads<LORA_NI>(), 0, st>>>(m);
     }
+  } else if (t.wide) {
+    LoraSmallParams p;
+    p.m = m;
+    p.part = part;
+    p.split = t.split;
+    for (int i = 0; i < m.n_jobs; ++i) {
+      p.ksteps[i] = 0;
+      for (int g = 0; g < m.job[i].nseg; ++g) p.ksteps[i] += (int)(m.seg[m.job[i].seg0 + g].K / BK);
+    }
+    lora_split_gemm_kernel<<<(unsigned)(m.n_tiles * t.split), nthreads<LORA_NI>(), 0, st>>>(p);
+    ARTK_CHECK_LAUNCH();
+    lora_split_reduce_kernel<<<(unsigned)(m.n_tiles * 16), 256, 0, st>>>(p);
   } else {
     LoraSmallParams p;
     p.m = m;

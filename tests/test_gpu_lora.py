@@ -504,3 +504,29 @@ def test_row_products(artk_lib, gpu, T, n_in, ranks):
         ref = x[1:].double() @ A.double().t()
         bound = x[1:].double().abs() @ A.double().abs().t()
         assert ((xa[1:].double() - ref).abs() <= 2e-6 * bound).all()
+
+
+@pytest.mark.parametrize("T,n_in,outs", [
+    (1500, 11008, (2048,)),          # forward in parts, rows that are no multiple of a tile
+    (1300, 2048, (11008, 11008)),    # input gradient in parts, of which some span both projections
+    (700, 9024, (960, 1088)),        # two jobs, ragged weight tiles
+])
+def test_long_products_of_few_tiles(artk_lib, gpu, T, n_in, outs):
+    """Products whose K range is split over work-groups on 256 x 256 tiles, block by block (bf16 output rounding: 2e-3
+    relative; a part that is missing or added twice is a third of the block or more)."""
+    print(f"long products T={T} in={n_in} outs={outs}", flush=True)
+    g = torch.Generator().manual_seed(T)
+    rand = lambda *s, std=1.0: (std * torch.randn(*s, generator=g)).to(torch.bfloat16).to(gpu)
+    x, r = rand(T, n_in), 8
+    Ws, As = [rand(o, n_in, std=0.02) for o in outs], [rand(r, n_in, std=0.02) for _ in outs]
+    Bs, ups, biases = [rand(o, r, std=0.2) for o in outs], [rand(T, o) for o in outs], [rand(o, std=0.5) for o in outs]
+    ys, xas = ops.lora_linear_multi_fwd(x, Ws, As, Bs, 2.0, biases)
+    dx, _, _ = ops.lora_linear_multi_bwd(ups, x, [ops.transpose(w) for w in Ws], As, Bs, xas, 2.0)
+    pairs = [(y, x.float() @ W.float().t() + 2.0 * (x.float() @ A.float().t()) @ B.float().t() + b.float())
+             for y, W, A, B, b in zip(ys, Ws, As, Bs, biases)]
+    pairs.append((dx, sum(u.float() @ W.float() + 2.0 * (u.float() @ B.float()) @ A.float()
+                          for u, W, A, B in zip(ups, Ws, As, Bs))))
+    for a, ref in pairs:
+        for i in range(0, a.shape[0], 32):
+            for j in range(0, a.shape[1], 512):
+                assert rel_l2(a[i:i + 32, j:j + 512].float(), ref[i:i + 32, j:j + 512]) <= TOL, (i, j)
