@@ -12,7 +12,7 @@
 // products ride along as extra K = 16 MFMA steps whose operands (the low-rank
 // factors) are read straight from global memory, so y and dx are each one GEMM
 // launch.  The skinny products are bandwidth-bound: x A^T in the forward is a row
-// product (rowdot16_kernel); in the backward g B and dB come from one pass over g
+// product (rowdot_multi_kernel); in the backward g B and dB come from one pass over g
 // and dA from one pass over x (lora_stats_kernel, skinny_stats.hpp).
 #include "common.hpp"
 #include "gemm_nt.hpp"
