@@ -14,7 +14,7 @@ namespace artk {
 //   ROW  rp[chunk][t][e] = sum_{c in chunk} X[t,c] F[e,c]      F bf16 [R,C]  (g B: F = B^T)
 //   COL  cp[slab][c][e]  = sum_{t in slab}  X[t,c] Y[t,e]      Y f32 [T,R]   (dB: Y = x A^T)
 // A work-group owns a slab of rows x a chunk of columns and streams it through LDS
-// in 128 x 128 tiles (buffer_load ... lds, three stages in flight), so X is read
+// in 128 x 128 tiles (buffer_load ... lds, a ring of NST stages), so X is read
 // from HBM once, fully coalesced, for both products.  Both run on MFMA 32x32x16
 // with the small dimension e as the M operand: ROW contracts over the columns
 // (row fragments of the tile, ds_read_b128), COL over the rows (transposed
@@ -26,7 +26,6 @@ namespace artk {
 constexpr int ST_TILE = 128;
 constexpr int ST_ROW_BYTES = ST_TILE * 2;             // 256
 constexpr int ST_TILE_BYTES = ST_TILE * ST_ROW_BYTES;  // 32 KiB
-constexpr int ST_STAGES = 3;
 
 // What the passes of a whole expert block add to the grouped form.  Two projections may be stacked along the rank
 // (e < r_split: the first one) and, in the plain layout, along the columns (c < c_split): each gets its own array and
@@ -115,10 +114,10 @@ __device__ __forceinline__ void stats_put_col(const StatsParams& p, int slab, bo
   }
 }
 
-// NTE: 32-wide tiles of e (rank <= 32 NTE); NCT: 128-column tiles per chunk; NST: LDS stages.
-// All memory traffic of the main loop is LDS DMA, ordered by hand with s_waitcnt vmcnt(n)
-// (the compiler inserts no waits for it): per wave, a tile is 8 DMA instructions, the Y rows
-// of a row tile R / 8, a flush of the ROW accumulators 4 NTE stores.
+// NTE: 32-wide tiles of e (rank <= 32 NTE); NCT: 128-column tiles per chunk; NST: LDS stages (two).  Ranks above 32;
+// the others have lora_stats_narrow_body below.
+// All memory traffic of the main loop is LDS DMA, ordered by hand with s_waitcnt vmcnt
+// (the compiler inserts no waits for it).
 // GATHER: the grouped form with a row gather.  The gather indices travel by DMA as well (an
 // ordinary global load in the issue path would make the compiler wait for every outstanding
 // operation, the ring included): each wave fetches the 32 indices of its own rows of row tile
@@ -190,18 +189,14 @@ __device__ __forceinline__ void lora_stats_body(const StatsParams& p, const int 
     for (int k = 0; k < 8; ++k) {
       const int instr = wave * 8 + k;
       const int row = instr * 4 + (lane >> 4);
-      int rg = rt * ST_TILE + row;
-      rg = rg < rows_here ? rg : rows_here - 1;
+      const int rg = rt * ST_TILE + row;
       int64_t xrow = rg;
       if constexpr (GATHER) xrow = gidx[k];
       else if (grouped) xrow = t0 + rg;
-      const int c = (lane & 15) ^ st_swz(row);
-      // columns past the end of a row (the ragged last column tile) re-read the row's first
-      // chunk instead: their ROW factor is zero and their COL results are never stored, and
-      // nothing is read outside the row, whatever follows it in memory
-      int64_t col = c0 + ct * ST_TILE + c * 8;
-      col = col < p.C ? col : 0;
-      const int voff = (int)(xrow * p.C * 2) + (int)(col * 2);
+      // What lies past the last row or column is read past the end of the descriptor and arrives as zeros (elements of the
+      // matrix in its place could be infinities, of which a zero in the other operand would make NaN).
+      const int64_t col = c0 + ct * ST_TILE + ((lane & 15) ^ st_swz(row)) * 8;
+      const int voff = rg < rows_here && col < p.C ? (int)(xrow * p.C * 2) + (int)(col * 2) : -16;
       dma_load16(rsrc, voff, 0, stage + instr * 1024);
     }
   };
@@ -250,20 +245,12 @@ __device__ __forceinline__ void lora_stats_body(const StatsParams& p, const int 
       for (int j = 0; j < 16; ++j) acc_col[ct][et][j] = 0.f;
   }
 
-  bool stored = false;  // the previous tile ended with a flush (its stores are newer than the DMA before them)
   // One tile; the column tile index is a compile-time constant so that its accumulators are too.
   auto do_tile = [&](int rt, auto ct_tag) {
     constexpr int ct = decltype(ct_tag)::value;
     const int i = rt * nct + ct;
-    // tile i has landed (with three stages tile i+1, and the stores of a flush, may still be on their way)
-    if (NST == 3 && i + 1 < nt && nct > 1) {
-      if (stored) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + 4 * NTE) : "memory");
-      else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // tile i has landed ...
     barrier_lds_only();  // ... for every wave, and every wave is done with tile i - 1
-    stored = false;
     if (ct == 0 && do_col) {
       // this lane's Y^T fragments: e = 32 et + m, rows 16 ks + 4 half + {0..3} and + 8
       const float* yr = (const float*)yraw;
@@ -323,17 +310,14 @@ __device__ __forceinline__ void lora_stats_body(const StatsParams& p, const int 
       for (int et = 0; et < NTE; ++et) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          // every lane stores (the wait above counts 4 NTE stores): out of range goes to a dummy slot
           const int e0 = 32 * et + 8 * q + 4 * half;
-          const bool ok = lrow < rows_here && e0 < R;
-          float* dst = ok ? p.row_part + ((int64_t)chunk * p.T + t) * R + e0 : p.row_dummy + (tid & 255) * 4;
-          *(floatx4*)dst =
-              floatx4{acc_row[et][4 * q], acc_row[et][4 * q + 1], acc_row[et][4 * q + 2], acc_row[et][4 * q + 3]};
+          if (lrow < rows_here && e0 < R)
+            *(floatx4*)(p.row_part + ((int64_t)chunk * p.T + t) * R + e0) =
+                floatx4{acc_row[et][4 * q], acc_row[et][4 * q + 1], acc_row[et][4 * q + 2], acc_row[et][4 * q + 3]};
         }
 #pragma unroll
         for (int j = 0; j < 16; ++j) acc_row[et][j] = 0.f;
       }
-      stored = true;
     }
   };
   for (int rt = 0; rt < n_rt; ++rt) {
@@ -362,11 +346,13 @@ __device__ __forceinline__ void lora_stats_body(const StatsParams& p, const int 
 }
 
 // ----------------------------------------------------------------------------
-// The same two products for ranks up to 16 NTE, on MFMA 16x16x32 (at rank 8 or 16 half or more of a 32 x 32 tile of e
-// would be multiplied for nothing) and small enough for two work-groups per CU: tiles of 64 rows x 128 columns, three
+// The same two products for ranks up to 16 NTE, NTE = 1 or 2, on MFMA 16x16x32 (at rank 8 or 16 half or more of a 32 x 32
+// tile of e would be multiplied for nothing) and small enough for two work-groups per CU: tiles of 64 rows x 128 columns, three
 // stages of 16 KiB, the factor of the chunk in registers (NCT * NTE * 4 fragments a lane).  One work-group computes,
-// stores its results or fills its ring while the other's reads are on their way.  Wave w owns rows 16w.. of a tile for
-// ROW and columns 32w.. for COL.  Everything else as above.
+// stores its results or fills its ring while the other's reads are on their way.  (On 32 x 32 tiles of e with 150 KiB of LDS,
+// one work-group per CU, us: ranks of 8 over 203 tokens of an expert block 21 + 9 + 20 + 20 -> 12 + 6 + 11 + 10, of 16 and 32
+// 24 + 10 + 26 + 23 -> 15 + 7 + 19 + 16; rank 32 over 8192 tokens 84 + 75 -> 88 + 69; rank 24 over [3000, 3584] 10 -> 9.)  Wave w owns
+// rows 16w.. of a tile for ROW and columns 32w.. for COL.  Everything else as above.
 // ----------------------------------------------------------------------------
 constexpr int SN_ROWS = 64;
 constexpr int SN_TILE_BYTES = SN_ROWS * ST_ROW_BYTES;  // 16 KiB
@@ -465,8 +451,7 @@ __device__ __forceinline__ void lora_stats_narrow_body(const StatsParams& p, con
       const int instr = wave * 4 + k;
       const int row = instr * 4 + sub;
       int xrow = rt * SN_ROWS + row;
-      // What lies past the last row or column is read past the end of the descriptor and arrives as zeros (elements of the
-      // matrix in its place could be infinities, of which a zero in the other operand would make NaN).
+      // (past the last row or column: zeros, see above)
       const int col = (int)c0 + ct * ST_TILE + (n16 ^ st_swz(row)) * 8;
       const bool in = xrow < rows_here && col < (int)p.C;
       if constexpr (GATHER) xrow = gidx[k];
@@ -722,11 +707,11 @@ static inline int64_t stats_grid_cost(int64_t blocks, int64_t row_tiles_per_bloc
 
 // c_all: columns of all passes of the launch (the work-group slots are shared by them).
 static inline StatsGeom stats_geom(int64_t T, int64_t C, int r, int64_t c_all) {
-  const int max_cct = r > 32 ? 2 : 4;  // column tiles per chunk the kernel holds accumulators for
-  const int tile_rows = r > 16 ? ST_TILE : SN_ROWS;
+  const int max_cct = r > 16 ? 2 : 4;  // column tiles per chunk the kernel holds accumulators for
+  const int tile_rows = r > 32 ? ST_TILE : SN_ROWS;
   const int64_t row_tiles = (T + tile_rows - 1) / tile_rows, col_tiles = (C + ST_TILE - 1) / ST_TILE;
   int64_t slots = num_cus();
-  if (r <= 16) {
+  if (r <= 32) {
     slots = 2 * slots * C / c_all;
     slots = slots < 1 ? 1 : slots;
   }
@@ -743,7 +728,7 @@ static inline StatsGeom stats_geom(int64_t T, int64_t C, int r, int64_t c_all) {
       if (slab_tiles > cap) slab_tiles = cap < 1 ? 1 : cap;
       const int64_t n_slabs = (row_tiles + slab_tiles - 1) / slab_tiles;
       // (narrow: the write and the read of a slab's COL partial are cct r / 8 half tiles)
-      const int64_t cost = stats_grid_cost(n_slabs * n_chunks, slab_tiles, cct, slots, r <= 16 ? 4 + cct * r / 8 : 4);
+      const int64_t cost = stats_grid_cost(n_slabs * n_chunks, slab_tiles, cct, slots, r <= 32 ? 4 + cct * r / 8 : 4);
       if (best_cost < 0 || cost < best_cost) {
         best_cost = cost;
         best.cc = cct * ST_TILE;
@@ -793,7 +778,10 @@ static inline int32_t launch_stats_params(const StatsParams& p, hipStream_t st) 
   const unsigned grid = (unsigned)(p.n_slabs * p.n_chunks);
   switch (stats_shape(p.R)) {
     case STATS_WIDE: lora_stats_kernel<2, 2, 2, false><<<grid, 256, 0, st>>>(p); break;
-    case STATS_32: lora_stats_kernel<1, 4, 3, false><<<grid, 256, 0, st>>>(p); break;
+    case STATS_32:
+      if (stats_once(p.T * p.C * 2)) lora_stats_narrow_kernel<2, 2, false, false, true><<<grid, 256, 0, st>>>(p);
+      else lora_stats_narrow_kernel<2, 2, false><<<grid, 256, 0, st>>>(p);
+      break;
     case STATS_NARROW:
       if (stats_once(p.T * p.C * 2)) lora_stats_narrow_kernel<1, 4, false, false, true><<<grid, 256, 0, st>>>(p);
       else lora_stats_narrow_kernel<1, 4, false><<<grid, 256, 0, st>>>(p);
@@ -820,8 +808,10 @@ static inline int32_t launch_stats_multi(StatsMulti& m, StatsShape shape, hipStr
   m.block0[m.n] = blocks;
   if (shape == STATS_WIDE)
     lora_stats_multi_kernel<2, 2, 2><<<(unsigned)blocks, 256, 0, st>>>(m);
+  else if (shape == STATS_32 && stats_once(bytes))
+    lora_stats_narrow_multi_kernel<2, 2, true><<<(unsigned)blocks, 256, 0, st>>>(m);
   else if (shape == STATS_32)
-    lora_stats_multi_kernel<1, 4, 3><<<(unsigned)blocks, 256, 0, st>>>(m);
+    lora_stats_narrow_multi_kernel<2, 2, false><<<(unsigned)blocks, 256, 0, st>>>(m);
   else if (stats_once(bytes))
     lora_stats_narrow_multi_kernel<1, 4, true><<<(unsigned)blocks, 256, 0, st>>>(m);
   else
@@ -844,10 +834,10 @@ static inline int32_t launch_stats_multi(StatsMulti& m, StatsShape shape, hipStr
 // 20 / 15 / 11 / 12 and 7 / 6 / 7 / 8 (without the reductions).
 // A caller without an order for the experts (`block` false) assumes a couple of row tiles for each.
 static inline int stats_grouped_cc(int64_t n_rows, int64_t C, int r, int E, bool block) {
-  const int max_cct = r > 32 ? 2 : 4;
+  const int max_cct = r > 16 ? 2 : 4;
   const int64_t col_tiles = (C + ST_TILE - 1) / ST_TILE;
-  const int64_t slots = r > 16 ? num_cus() : 2 * num_cus();
-  const double avg = (double)n_rows / E / (r > 16 ? ST_TILE : SN_ROWS), tiles = avg > 1.0 ? avg + 0.5 : 1.0;
+  const int64_t slots = r > 32 ? num_cus() : 2 * num_cus();
+  const double avg = (double)n_rows / E / (r > 32 ? ST_TILE : SN_ROWS), tiles = avg > 1.0 ? avg + 0.5 : 1.0;
   int best = max_cct;
   double best_cost = -1.0;
   for (int cct = max_cct; cct >= 1; --cct) {
@@ -860,7 +850,7 @@ static inline int stats_grouped_cc(int64_t n_rows, int64_t C, int r, int E, bool
       const double longest = (avg > 1.0 ? 2.5 : 1.0) * tiles * (2 * cct + 1) + 8.0;
       cost = (total > longest ? total : longest) + (double)(E * n_chunks) / slots * tiles * r / 10.0;
     } else {
-      cost = (double)stats_grid_cost((int64_t)E * n_chunks, r > 16 ? 2 : 4, cct, slots, 4);
+      cost = (double)stats_grid_cost((int64_t)E * n_chunks, r > 32 ? 2 : 4, cct, slots, 4);
     }
     if (best_cost < 0.0 || cost < best_cost) {
       best_cost = cost;
@@ -905,17 +895,17 @@ static inline int32_t launch_stats_grouped(const void* X, int64_t x_rows, const 
     if (gather) {
       if (r > 32)
         lora_stats_kernel<2, 2, 2, true, BLOCK><<<grid, 256, 0, st>>>(p);
-      else if (r <= 16)
-        lora_stats_narrow_kernel<1, 4, true, BLOCK><<<grid, 256, 0, st>>>(p);
+      else if (r > 16)
+        lora_stats_narrow_kernel<2, 2, true, BLOCK><<<grid, 256, 0, st>>>(p);
       else
-        lora_stats_kernel<1, 4, 3, true, BLOCK><<<grid, 256, 0, st>>>(p);
+        lora_stats_narrow_kernel<1, 4, true, BLOCK><<<grid, 256, 0, st>>>(p);
     } else {
       if (r > 32)
         lora_stats_kernel<2, 2, 2, false, BLOCK><<<grid, 256, 0, st>>>(p);
-      else if (r <= 16)
-        lora_stats_narrow_kernel<1, 4, false, BLOCK><<<grid, 256, 0, st>>>(p);
+      else if (r > 16)
+        lora_stats_narrow_kernel<2, 2, false, BLOCK><<<grid, 256, 0, st>>>(p);
       else
-        lora_stats_kernel<1, 4, 3, false, BLOCK><<<grid, 256, 0, st>>>(p);
+        lora_stats_narrow_kernel<1, 4, false, BLOCK><<<grid, 256, 0, st>>>(p);
     }
   };
   if (block)

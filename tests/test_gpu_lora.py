@@ -457,9 +457,11 @@ def test_forward_makes_no_transposed_weight(artk_lib, gpu):
     (1, 64, 64, 8), (63, 128, 192, 16), (65, 640, 448, 8),        # one row, around a 64-row tile, ragged 128-column tiles
     (257, 64, 576, 16),                                           # one column tile: the ring runs over row tiles alone
     (129, 4160, 1088, 8),                                         # several chunks of columns
-    (8192, 64, 16448, 16)])                                       # more than 256 MiB of g: non-temporal loads
+    (8192, 64, 16448, 16),                                        # more than 256 MiB of g: non-temporal loads
+    (65, 640, 448, 24), (1, 128, 64, 32), (300, 64, 1088, 32),    # two blocks of 16 ranks
+    (130, 192, 448, 40)])                                         # the kernel of larger ranks
 def test_skinny_passes_of_small_ranks(artk_lib, gpu, T, n_in, n_out, r):
-    """dA, dB and, through dx, g B at the edges of the one-pass backward of ranks up to 16.  TOL as above: bf16 factors
+    """dA, dB and, through dx, g B at the edges of the one-pass backward.  TOL as above: bf16 factors
     on the way."""
     print(f"skinny passes T={T} in={n_in} out={n_out} r={r}", flush=True)
     x, W, A, B, up = (t.to(gpu) for t in make(T, n_in, n_out, r, T + n_out, b_std=0.3))
