@@ -98,9 +98,24 @@ __global__ __launch_bounds__(PERM_CHUNK) void moe_hist_kernel(const int* __restr
 // position of chunk b's entries of expert e; tile_prefix / blk_prefix: prefix
 // sums of ceil(rows_e / 256) and ceil(rows_e / 16) (work lists of the grouped
 // kernels).  One block of 1024 threads: thread (part, e) walks a quarter of the
-// chunks of expert e, eight independent loads at a time.  order (or nullptr): the
-// experts by falling number of rows, ties by index.
+// chunks of expert e, eight independent loads at a time.  order [E+1] (or nullptr): the
+// experts by falling number of rows, ties by index, then moe_split_rows.
 constexpr int SCAN_PARTS = 4;
+constexpr int SG_COLS = 128;  // rows of an expert in one pass of the streaming product over its weights
+
+// The streaming product deals whole experts to the XCDs, back and forth in falling order of their rows.
+__device__ __forceinline__ int moe_dealt_to(int rank) { return rank & 8 ? 7 - (rank & 7) : rank & 7; }
+// Experts with more rows than this are split between the XCDs instead: none if no XCD gets more than 5 / 4 of its share of
+// the passes (share[x]) that way, else those with more than 1 / 32 of all rows (there are fewer than 32).
+__device__ __forceinline__ int moe_split_rows(const int* share, int n_rows) {
+  int all = 0, most = 0;
+#pragma unroll
+  for (int x = 0; x < 8; ++x) {
+    all += share[x];
+    most = most > share[x] ? most : share[x];
+  }
+  return 4 * 8 * most > 5 * all ? n_rows / 32 : 0x7fffffff;
+}
 __global__ __launch_bounds__(SCAN_PARTS * MOE_MAX_E) void moe_scan_kernel(const int* __restrict__ cnt, int nb, int E,
                                                                           int* __restrict__ offsets,
                                                                           int* __restrict__ base,
@@ -109,7 +124,7 @@ __global__ __launch_bounds__(SCAN_PARTS * MOE_MAX_E) void moe_scan_kernel(const 
                                                                           int* __restrict__ order) {
   __shared__ int part[SCAN_PARTS][MOE_MAX_E];
   __shared__ int wsum[3][MOE_MAX_E / 64];
-  __shared__ int off[MOE_MAX_E], rows[MOE_MAX_E], rank[MOE_MAX_E];
+  __shared__ int off[MOE_MAX_E], rows[MOE_MAX_E], rank[MOE_MAX_E], share[8];
   const int e = threadIdx.x % MOE_MAX_E, pt = threadIdx.x / MOE_MAX_E;
   const int per = (nb + SCAN_PARTS - 1) / SCAN_PARTS;
   const int b0 = pt * per, b1 = b0 + per < nb ? b0 + per : nb;
@@ -171,6 +186,7 @@ __global__ __launch_bounds__(SCAN_PARTS * MOE_MAX_E) void moe_scan_kernel(const 
       tile_prefix[0] = 0;
       blk_prefix[0] = 0;
     }
+    if (e < 8) share[e] = 0;
   }
   __syncthreads();
   if (e < E) {
@@ -197,7 +213,12 @@ __global__ __launch_bounds__(SCAN_PARTS * MOE_MAX_E) void moe_scan_kernel(const 
       atomicAdd(&rank[e], before);
     }
     __syncthreads();
-    if (pt == 0 && e < E) order[rank[e]] = e;
+    if (pt == 0 && e < E) {
+      order[rank[e]] = e;
+      atomicAdd(&share[moe_dealt_to(rank[e])], (rows[e] + SG_COLS - 1) / SG_COLS);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) order[E] = moe_split_rows(share, off[E - 1] + rows[E - 1]);
   }
 }
 
@@ -259,7 +280,7 @@ struct MoeGemmParams {
   const int* tile_prefix;  // [E+1]
   int64_t M, K;
   int E, r, RP, MT;
-  const int* order;
+  const int* order;        // [E+1] experts by falling number of rows, then moe_split_rows
 };
 
 // One tile of the grouped product: expert, rows and weight tile.
@@ -386,7 +407,6 @@ __global__ __launch_bounds__(nthreads<MOE_NI>()) void moe_gemm_kernel(MoeGemmPar
 // the weights behind them.  So up to 96 KiB of weights are on their way per CU where the 256 x 256 tile above has 32.
 // ----------------------------------------------------------------------------
 constexpr int SG_ROWS = 128;                      // weight rows of a work-group
-constexpr int SG_COLS = 128;                      // most columns in one pass over the weights
 constexpr int SG_P_BYTES = SG_ROWS * BK * 2;      // 16 KiB
 constexpr int SG_LDS_BYTES = 80 * 1024;           // two work-groups per CU
 template <int NQ> constexpr int sg_stages() { return NQ <= 2 ? 4 : 3; }
@@ -519,39 +539,71 @@ __device__ __forceinline__ void moe_stream_pass(const MoeGemmParams& p, char* sm
   else moe_stream_cols<1, ONCE>(p, smem, e, m0, row0, n);
 }
 
-// Experts are dealt to the XCDs in falling order of their rows; an XCD's units are numbered expert by expert, weight
-// tile by weight tile, and the passes of an expert with more than SG_COLS rows (even shares of them, in whole 32) are
-// neighbours, so they read a weight tile together.  A wave finds the expert of unit `loc` from its lanes' counts.
+// An XCD has the experts that it is dealt (lanes 32 .. 63), whose rows are then in one L2, and an eighth of the units of every
+// expert that is split (lanes 0 .. 31; they come first in the order).  Without the split, XCDs have nothing to do where there are
+// fewer than eight experts, and one of them works alone where an expert has most of the rows: forward of a block (hidden
+// 2048, intermediate 768), us, 256 x 256 tiles / dealt only / with the split: 8000 rows on one of 128 experts
+// 160 / 688 / 198, 4000 rows on each of two 154 / 399 / 181, 4 experts of 125 rows and intermediate 5632 236 / 220 / 186.
+// An XCD's units are numbered expert by expert, weight tile by weight tile, and the passes of an expert with more than SG_COLS
+// rows (even shares of them, in whole 32) are neighbours, so they read a weight tile together.
 __global__ __launch_bounds__(256, 2) void moe_stream_gemm_kernel(MoeGemmParams p) {
+  static_assert(MOE_MAX_E <= 8 * 32, "a lane per expert of an XCD");
   __shared__ __attribute__((aligned(1024))) char smem[SG_LDS_BYTES];
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, l32 = lane & 31;
   const int x = blockIdx.x & 7;
-  int ex = 8 * lane + ((lane & 1) ? 7 - x : x);  // this lane's expert
-  int first = 0, n_e = 0;
-  if (ex < p.E) {
-    if (p.order != nullptr) ex = p.order[ex];
+  const bool parts = lane < 32;
+  const int pos = parts ? l32 : 8 * l32 + ((l32 & 1) ? 7 - x : x);  // of this lane's expert in the order (moe_dealt_to)
+  const int split_rows = p.order[p.E];
+  int ex = 0, first = 0, n_e = 0;
+  if (pos < p.E) {
+    ex = p.order[pos];
     first = p.offsets[ex];
     n_e = p.offsets[ex + 1] - first;
   }
   const int passes = (n_e + SG_COLS - 1) / SG_COLS;
-  int end = passes * p.MT;  // units of the experts up to this one
+  int from = 0, units = passes * p.MT;  // this XCD's units of the expert
+  if (parts) {
+    const int y = (x + l32) & 7;
+    from = units * y / 8;
+    units = units * (y + 1) / 8 - from;
+  }
+  if ((n_e > split_rows) != parts) units = 0;
+  int end = units;  // units of the experts up to this one
 #pragma unroll
-  for (int d = 1; d < MOE_MAX_E / 8; d <<= 1) {
+  for (int d = 1; d < 64; d <<= 1) {
     const int v = __shfl_up(end, d, 64);
     if (lane >= d) end += v;
   }
-  const int total = __builtin_amdgcn_readlane(end, MOE_MAX_E / 8 - 1);
+  const int shift = end - units - from;
+  const int total = __builtin_amdgcn_readlane(end, 63);
   for (int loc = blockIdx.x >> 3; loc < total; loc += gridDim.x >> 3) {
-    const int l = __popcll(__ballot(lane < MOE_MAX_E / 8 && end <= loc));
+    const int l = __popcll(__ballot(end <= loc));
     const int e = __builtin_amdgcn_readlane(ex, l), n = __builtin_amdgcn_readlane(n_e, l);
     const int np = __builtin_amdgcn_readlane(passes, l), row0 = __builtin_amdgcn_readlane(first, l);
-    const int unit = loc - (__builtin_amdgcn_readlane(end, l) - np * p.MT);
+    const int unit = loc - __builtin_amdgcn_readlane(shift, l);
     const int per = ((n + np - 1) / np + 31) & ~31, c0 = (unit % np) * per;
     const int64_t m0 = (int64_t)(unit / np) * SG_ROWS;
     const int left = n - c0 < per ? n - c0 : per;
     if (np == 1) moe_stream_pass<true>(p, smem, e, m0, row0, left);
     else if (left > 0) moe_stream_pass<false>(p, smem, e, m0, row0 + c0, left);
   }
+}
+
+// order [E+1] as moe_scan_kernel leaves it.
+__global__ __launch_bounds__(MOE_MAX_E) void moe_order_kernel(const int* __restrict__ offsets, int E, int* __restrict__ order) {
+  __shared__ int rows[MOE_MAX_E], share[8];
+  const int e = threadIdx.x, c = e < E ? offsets[e + 1] - offsets[e] : 0;
+  rows[e] = c;
+  if (e < 8) share[e] = 0;
+  __syncthreads();
+  if (e < E) {
+    int rank = 0;
+    for (int j = 0; j < E; ++j) rank += (rows[j] > c || (rows[j] == c && j < e)) ? 1 : 0;
+    order[rank] = e;
+    atomicAdd(&share[moe_dealt_to(rank)], (c + SG_COLS - 1) / SG_COLS);
+  }
+  __syncthreads();
+  if (e == 0) order[E] = moe_split_rows(share, offsets[E] - offsets[0]);
 }
 
 // Grouped row products: 16-row blocks never straddle experts.
@@ -771,10 +823,25 @@ static int32_t check_moe(int64_t n_rows, int64_t in, int64_t out, int E, int r) 
   return ARTK_OK;
 }
 
+// Up to SG_COLS rows per expert the streaming kernel is the faster one.  Four products of a block, us, 256 x 256 tiles
+// / streamed (hidden 2048, intermediate 768): 128 experts, 203 tokens (13 rows each) 517 / 423, 512 (32) 569 / 498,
+// 1024 (64) 681 / 579, 2048 (128) 728 / 705, 3000 (188) 888 / 868; 64 experts, 400 tokens (50) 333 / 279,
+// 1024 (128) 405 / 389, 1300 (163) 418 / 432.
+static bool moe_streams(int64_t n_rows, int E) { return n_rows <= (int64_t)E * SG_COLS; }
+
+// For a product whose routing did not leave the order (2 us).
+static int32_t launch_moe_order(const int* offsets, int64_t n_rows, int E, int* order, hipStream_t st) {
+  if (!moe_streams(n_rows, E)) return ARTK_OK;
+  moe_order_kernel<<<1, MOE_MAX_E, 0, st>>>(offsets, E, order);
+  ARTK_CHECK_LAUNCH();
+  return ARTK_OK;
+}
+
+// order: read by the streaming kernel only.
 static int32_t launch_moe_gemm(const void* W, const void* X, const int* gather, const uint16_t* Pe,
                                const uint16_t* Qe, void* out, const int* offsets,
                                const int* tile_prefix, int64_t n_rows, int64_t M, int64_t K, int E,
-                               int r, int RP, hipStream_t st, const int* order = nullptr) {
+                               int r, int RP, const int* order, hipStream_t st) {
   MoeGemmParams p;
   p.W = W;
   p.X = X;
@@ -792,11 +859,7 @@ static int32_t launch_moe_gemm(const void* W, const void* X, const int* gather, 
   p.MT = (int)((M + TILE - 1) / TILE);
   const int64_t max_row_tiles = (n_rows + TILE - 1) / TILE + E;
   prof_begin(PROF_MOE_GEMM, st);
-  // Up to SG_COLS rows per expert the streaming kernel is the faster one.  Four products of a block, us, 256 x 256 tiles
-  // / streamed (hidden 2048, intermediate 768): 128 experts, 203 tokens (13 rows each) 517 / 423, 512 (32) 569 / 498,
-  // 1024 (64) 681 / 579, 2048 (128) 728 / 705, 3000 (188) 888 / 868; 64 experts, 400 tokens (50) 333 / 279,
-  // 1024 (128) 405 / 389, 1300 (163) 418 / 432.
-  if (n_rows <= (int64_t)E * SG_COLS) {
+  if (moe_streams(n_rows, E)) {
     p.MT = (int)((M + SG_ROWS - 1) / SG_ROWS);
     p.order = order;
     // (as many as there are units if the XCDs' shares are even; the rest comes in a second turn)
@@ -886,9 +949,9 @@ size_t artk_moe_lora_grouped_fwd_workspace_bytes(int64_t n_rows, int64_t in, int
                                                  int32_t r) {
   (void)in;
   (void)out;
-  (void)E;
   Workspace ws(nullptr, 0);
   ws.take<uint16_t>((size_t)n_rows * round16(r));
+  ws.take<int>((size_t)E + 1);
   return ws.used + 256;
 }
 
@@ -913,6 +976,7 @@ int32_t artk_moe_lora_grouped_fwd(const void* x, const int32_t* gather, const vo
   const int RP = round16(r);
   Workspace ws(workspace, workspace_bytes);
   uint16_t* xa16 = ws.take<uint16_t>((size_t)n_rows * RP);
+  int* order = ws.take<int>((size_t)E + 1);
   if (!ws.ok()) {
     set_error("workspace too small: need %zu bytes, got %zu", ws.used, workspace_bytes);
     return ARTK_ERR_WORKSPACE_TOO_SMALL;
@@ -921,14 +985,16 @@ int32_t artk_moe_lora_grouped_fwd(const void* x, const int32_t* gather, const vo
   if ((rc = launch_moe_rowdot(x, gather, (const uint16_t*)A, expert_offsets, blk_prefix, n_rows, E, in,
                               r, RP, scale, xa, xa16, st)))
     return rc;
+  if ((rc = launch_moe_order(expert_offsets, n_rows, E, order, st))) return rc;
   return launch_moe_gemm(W, x, gather, (const uint16_t*)B, xa16, y, expert_offsets, tile_prefix, n_rows,
-                         out, in, E, r, RP, st);
+                         out, in, E, r, RP, order, st);
 }
 
 // Scratch of the grouped backward, carved in the same order by the size query and the call.
 struct MoeBwdScratch {
   uint16_t *Bt, *At, *gb16;
   float *gb, *rowp, *dummy;
+  int* order;
 };
 static void carve_moe_bwd(Workspace& ws, int64_t n_rows, int64_t in, int64_t out, int E, int r, MoeBwdScratch& c) {
   const int RP = round16(r);
@@ -938,6 +1004,7 @@ static void carve_moe_bwd(Workspace& ws, int64_t n_rows, int64_t in, int64_t out
   c.gb16 = ws.take<uint16_t>((size_t)n_rows * RP);
   c.rowp = ws.take<float>((size_t)stats_grouped_chunks(n_rows, out, r, E, false) * n_rows * r);
   c.dummy = ws.take<float>(1024);
+  c.order = ws.take<int>((size_t)E + 1);
 }
 
 size_t artk_moe_lora_grouped_bwd_workspace_bytes(int64_t n_rows, int64_t in, int64_t out, int32_t E,
@@ -986,8 +1053,9 @@ int32_t artk_moe_lora_grouped_bwd(const void* g, const void* x, const int32_t* g
     StatsReduceJob jb{nullptr, 0, 0, 0.f, nullptr, 0, nullptr, 0, 0.f};
     if ((rc = launch_stats_reduce(ja, jb, r, st))) return rc;
   }
+  if ((rc = launch_moe_order(expert_offsets, n_rows, E, c.order, st))) return rc;
   if ((rc = launch_moe_gemm(W_t, g, nullptr, c.At, c.gb16, dx, expert_offsets, tile_prefix, n_rows, in, out,
-                            E, r, RP, st)))
+                            E, r, RP, c.order, st)))
     return rc;
   // one pass over x (through the row gather when there is one): dA_e [r,in] = s (g B_e)^T x
   return launch_stats_grouped(x, gather ? (int64_t)0x3fffffff / in : n_rows, gather, n_rows, in, nullptr, c.gb, r,
@@ -1000,7 +1068,7 @@ struct MoeSaved {
   uint16_t *A_gu, *B_gu, *A_d, *B_d;  // bf16 adapters [E,2r,H], [E,2I,2r], [E,r,I], [E,H,r]
   float *xa_gu, *xaw_d;               // x A^T [n,2r]; routing weight times h A_d^T [n,r]
   uint16_t *gu, *h;                   // gate|up [n,2I], silu(gate) up [n,I]
-  int* order;                         // experts by falling number of rows
+  int* order;                         // [E+1] experts by falling number of rows, then moe_split_rows
 };
 static void carve_moe_saved(Workspace& ws, const artk_moe_experts_t& a, MoeSaved& c) {
   const size_t n = (size_t)(a.T * a.k), E = (size_t)a.E, r = (size_t)a.r, H = (size_t)a.H, I = (size_t)a.I;
@@ -1012,7 +1080,7 @@ static void carve_moe_saved(Workspace& ws, const artk_moe_experts_t& a, MoeSaved
   c.xaw_d = ws.take<float>(n * r);
   c.gu = ws.take<uint16_t>(n * 2 * I);
   c.h = ws.take<uint16_t>(n * I);
-  c.order = ws.take<int>(E);
+  c.order = ws.take<int>(E + 1);
 }
 struct MoeFwdScratch {
   char* route;
@@ -1144,7 +1212,7 @@ int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_
                               a->scale, s.xa_gu, c.xa16_gu, st)))
     return rc;
   if ((rc = launch_moe_gemm(a->W_gu, a->x, a->row_token, s.B_gu, c.xa16_gu, s.gu, a->offsets, a->tile_prefix, n, 2 * I,
-                            H, E, 2 * r, round16(2 * r), st, s.order)))
+                            H, E, 2 * r, round16(2 * r), s.order, st)))
     return rc;
   moe_silu_mul_kernel<<<blocks256(n * I / 8), 256, 0, st>>>(s.gu, n * I / 8, (int)(I / 8), s.h);
   ARTK_CHECK_LAUNCH();
@@ -1152,7 +1220,7 @@ int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_
                               s.xaw_d, c.xa16_d, st, a->topk_w, a->perm)))
     return rc;
   if ((rc = launch_moe_gemm(a->W_d, s.h, nullptr, s.B_d, c.xa16_d, c.down, a->offsets, a->tile_prefix, n, H, I, E, r,
-                            round16(r), st, s.order)))
+                            round16(r), s.order, st)))
     return rc;
   return launch_moe_combine(c.down, a, a->topk_w, a->y, st);
 }
@@ -1204,7 +1272,7 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
     if ((rc = launch_stats_reduce(ja, none, r, st))) return rc;
   }
   if ((rc = launch_moe_gemm(a->Wt_d, a->g, a->row_token, c.At_d, c.gb16, c.dhr, a->offsets, a->tile_prefix, n, I, H, E,
-                            r, round16(r), st, s.order)))
+                            r, round16(r), s.order, st)))
     return rc;
   if ((rc = launch_stats_grouped(s.h, n, nullptr, n, I, nullptr, c.gb, r, E, a->offsets, nullptr, a->ddown_A, a->scale,
                                  1, c.dummy, st, &down)))
@@ -1222,7 +1290,7 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
     if ((rc = launch_stats_reduce(ja, none, 2 * r, st))) return rc;
   }
   if ((rc = launch_moe_gemm(a->Wt_gu, c.g_gu, nullptr, c.At_gu, c.gb16, c.dx_rows, a->offsets, a->tile_prefix, n, H,
-                            2 * I, E, 2 * r, round16(2 * r), st, s.order)))
+                            2 * I, E, 2 * r, round16(2 * r), s.order, st)))
     return rc;
   if ((rc = launch_stats_grouped(a->x, a->T, a->row_token, n, H, nullptr, c.gb, 2 * r, E, a->offsets, nullptr,
                                  a->dgate_A, a->scale, 1, c.dummy, st, &gate_up_A)))

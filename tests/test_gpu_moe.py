@@ -142,6 +142,8 @@ def test_grouped_lora_ranks(artk_lib, gpu, r, use_gather):
     ([96, 97, 128, 5, 0, 17, 63, 2, 40], 192, 320, 24, False),   # fewer K steps than ring stages, a ragged weight tile
     ([129, 0, 260, 3, 0, 0, 0, 0, 0, 77], 128, 448, 8, True),    # experts in two and three passes
     ([3] * 255 + [200], 128, 128, 16, True),                     # the most experts
+    ([400, 90, 90] + [0, 1, 7] * 20, 1088, 64, 8, True),         # shares of full experts, nine weight tiles over eight XCDs
+    ([40], 192, 1152, 8, False),                                 # one expert
     ([300, 1, 130], 128, 192, 8, True),                          # more than 128 rows per expert: 256 x 256 tiles
     ([257, 384], 192, 320, 40, False),
 ])
@@ -174,6 +176,36 @@ def test_grouped_lora_rows_per_expert(artk_lib, gpu, rows, H, I, r, use_gather):
         if rows[e]:
             assert rel_l2(y[off[e]:off[e + 1]].cpu().float(), y0[off[e]:off[e + 1]]) <= TOL
     assert rel_l2(dA.cpu(), dA0) <= TOL and rel_l2(dB.cpu(), dB0) <= TOL
+
+
+def test_one_full_expert_among_many_takes_no_longer_than_alone(artk_lib, gpu):
+    """All tokens on one of 128 experts: its units are spread over the GPU (on one XCD the block took four times as long
+    as the same rows through a block of one expert; the streaming kernel may cost some of what the tiles of many rows
+    take)."""
+    T, H, I = 4000, 2048, 768
+    x = torch.randn(T, H, device=gpu).to(torch.bfloat16)
+    blocks = []
+    for E in (1, 128):
+        m = MoELoRAExperts(H, I, E, 1, r=8, lora_alpha=16, device=gpu)
+        logits = torch.zeros(T, E, device=gpu)
+        logits[:, 0] = 30.0
+        blocks.append((m, logits))
+
+    def median_us(m, logits):
+        times = []
+        for _ in range(15):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            with torch.no_grad():
+                m(x, logits)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b) * 1e3)
+        return sorted(times)[7]
+
+    alone, among = (median_us(*b) for b in blocks)
+    print(f"moe one expert: alone {alone:.0f} us, among 128 {among:.0f} us", flush=True)
+    assert among <= 2 * alone
 
 
 @pytest.mark.parametrize("use_gather", [True, False])
