@@ -1160,12 +1160,6 @@ size_t artk_moe_experts_bwd_workspace_bytes(const artk_moe_experts_t* a) {
   return ws.used + 256;
 }
 
-// Experts of a row tile or less are all alike to the skinny passes: no order for them (and no look-up, 1 to 4 us of
-// a 20 us launch).
-static int* moe_order(const artk_moe_experts_t* a, const MoeSaved& s) {
-  return a->T * a->k > (int64_t)a->E * ST_TILE ? s.order : nullptr;
-}
-
 static unsigned blocks256(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 static int32_t launch_moe_combine(const uint16_t* rows, const artk_moe_experts_t* a, const float* w, void* out, hipStream_t st) {
@@ -1249,8 +1243,7 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
   hipStream_t st = (hipStream_t)stream;
   const int64_t n = a->T * a->k, H = a->H, I = a->I;
   const int E = a->E, r = a->r;
-  const int* order = moe_order(a, s);
-  const StatsBlock down{order}, gate_up_B{order, a->dup_B, r, I}, gate_up_A{order, a->dup_A, r, 0};
+  const StatsBlock down{s.order}, gate_up_B{s.order, a->dup_B, r, I}, gate_up_A{s.order, a->dup_A, r, 0};
   {
     SmallTransposeMulti m;
     m.n = 4;

@@ -31,7 +31,7 @@ constexpr int ST_TILE_BYTES = ST_TILE * ST_ROW_BYTES;  // 32 KiB
 // (e < r_split: the first one) and, in the plain layout, along the columns (c < c_split): each gets its own array and
 // the blocks that mix them, which belong to nobody, are not stored.  r_split == 0: one array.
 struct StatsBlock {
-  const int* order = nullptr;  // slab numbers in the order in which they are dispatched (nullptr: by number)
+  const int* order;            // slab numbers in the order in which they are dispatched (nullptr, ranks above 32: by number)
   float* col_out2 = nullptr;
   int r_split = 0;
   int64_t c_split = 0;
@@ -385,8 +385,7 @@ __device__ __forceinline__ void lora_stats_narrow_body(const StatsParams& p, con
   int slab = block / p.n_chunks;
   const int chunk = block - slab * p.n_chunks;
   const bool grouped = p.offsets != nullptr;
-  if constexpr (BLOCK)
-    if (p.block.order != nullptr) slab = p.block.order[slab];
+  if constexpr (BLOCK) slab = p.block.order[slab];
   const int64_t t0 = grouped ? (int64_t)p.offsets[slab] : (int64_t)slab * p.rows_per_slab;
   const int64_t c0 = (int64_t)chunk * p.cc;
   const int rows_here = grouped ? p.offsets[slab + 1] - p.offsets[slab]
@@ -826,12 +825,15 @@ static inline int32_t launch_stats_multi(StatsMulti& m, StatsShape shape, hipStr
 // Chunk width: the launch lasts as long as its work divided by the work-group slots, or as its longest expert, whichever
 // is more (half tile times as in stats_grid_cost, with twice the set-up: an expert's factor and results are its own).
 // Routing is uneven (of 8192 tokens, top-8 of 128 experts, the fullest expert gets 3 to 5 times the average), so
-// with one wide chunk per expert most CUs wait for the fullest one, unless it is dispatched first (`order`) and is
+// with one wide chunk per expert most CUs wait for the fullest one, unless it is dispatched first (a block's `order`) and is
 // not too long; the estimate takes 2.5 times the average.  The ROW partials of a chunk are written and read back.
 // Measured at that size, us for chunks of 128 / 256 / 384 / 512 columns (ranks up to 16, with the order): rows of 2048
 // through the gather with the ROW product 58 / 48 / 59 / 70, without it 48 / 43 / 54 / 63, 1536 columns with the
 // reduction 70 / 64 / 73 / 83, 768 columns 32 / 41 / 50 / 60; 203 tokens: 23 / 15 / 16 / 11, 16 / 12 / 12 / 10,
 // 20 / 15 / 11 / 12 and 7 / 6 / 7 / 8 (without the reductions).
+// (In the middle of the range, the four passes of a block with their reductions, rank 8: 512 tokens 84 / 69 / 65 / 68, as chosen here 62;
+// 1024 95 / 81 / 83 / 93, 85; 1500 93 / 74 / 75 / 81, 74; 2048 102 / 83 / 87 / 99, 80; 4096 155 / 189 / 233 / 279, 179;
+// 64 experts, 700 tokens 62 / 61 / 71 / 81, 62; 1500 84 / 105 / 126 / 150, 84.)
 // A caller without an order for the experts (`block` false) assumes a couple of row tiles for each.
 static inline int stats_grouped_cc(int64_t n_rows, int64_t C, int r, int E, bool block) {
   const int max_cct = r > 16 ? 2 : 4;
@@ -870,6 +872,12 @@ static inline int32_t launch_stats_grouped(const void* X, int64_t x_rows, const 
                                            hipStream_t st, const StatsBlock* block = nullptr) {
   StatsParams p;
   if (block) p.block = *block;
+  // The look-up of the order costs ranks above 32, one work-group per CU, about 4 us a launch, and its gain begins at 20 rows per
+  // expert; the narrow kernel has it for nothing.  Passes and reductions of a block, by number / in the order, us: 128
+  // experts, rank 24 (48 in two of the four passes) 203 tokens (13 rows) 116 / 124, 300 (19) 119 / 127, 400 (25) 128 / 127,
+  // 512 137 / 129, 1024 157 / 147; rank 16 203 tokens 66 / 63, 1024 110 / 96, 2048 134 / 108; rank 8 203 tokens 49 / 48,
+  // 1024 85 / 86, 1500 85 / 74.
+  if (r > 32 && n_rows < 24 * (int64_t)E) p.block.order = nullptr;
   p.X = (const uint16_t*)X;
   p.T = n_rows;
   p.C = C;
