@@ -461,13 +461,16 @@ __global__ __launch_bounds__(256) void lora_split_reduce_kernel(LoraSmallParams 
 // ----------------------------------------------------------------------------
 // Row products of one X with several factors: out_i[t, j] = sum_k X[t,k] Mt_i[j,k], Mt_i [R_i,K], on MFMA 16x16x32.
 // The factor rows of all i are numbered through (e0[i] ..); a work-group takes 16 NJ of them (blockIdx.y) and 16 rows of
-// X.  K is dealt to its NW waves in pieces of 64 (two MFMA steps; a lane takes 32 contiguous bytes of its row, so a wave
-// reads whole cache lines), U of them in flight at a time.  Writes f32 [T,R] (unscaled) and bf16 [T,RP] (scaled, zero
+// X.  K is dealt to its four waves in pieces of 64 (two MFMA steps; a lane takes 32 contiguous bytes of its row, so a wave
+// reads whole cache lines), two of them in flight at a time.  Writes f32 [T,R] (unscaled) and bf16 [T,RP] (scaled, zero
 // padded to RP).
 // Where there are rows enough the factors are packed (e0 by R: two ranks of 8 are one block) and X is read once for
 // ranks that add up to 64; else every factor starts a block of its own (e0 by RP) and there are more work-groups.  us, a
 // work-group per 16 rows and factor / packed: [8192, 2048] and 2 ranks of 8 21 / 14, [4096, 2048] and 3 of 8 14 / 9,
 // [8192, 896] and 2 of 8 9 / 7, [1000, 3584] and 2 of 8 11 / 13.
+// (Eight waves and twice the pieces in flight: one factor of rank 8 over 8192 rows, K = 896 6.1 / 10.4, 1536 7.9 / 10.3,
+// 2048 11.8 / 9.4, 2560 10.5 / 14.8, 4096 15.3 / 15.5, 8192 31.7 / 30.3; two factors at 2048 11.6 / 12.4.  Not kept for one
+// width.)
 // ----------------------------------------------------------------------------
 struct RowdotMulti {
   const uint16_t* Mt[LORA_MAX_SEG];
@@ -476,10 +479,10 @@ struct RowdotMulti {
   int R[LORA_MAX_SEG], RP[LORA_MAX_SEG], e0[LORA_MAX_SEG + 1];
   int n;
 };
-template <int NJ, int NW>
-__global__ __launch_bounds__(64 * NW) void rowdot_multi_kernel(const uint16_t* __restrict__ X, RowdotMulti m, int64_t T,
-                                                               int64_t K, float scale) {
-  constexpr int STEP = NW * 64, U = NW == 8 && NJ <= 2 ? 4 : 2;
+template <int NJ>
+__global__ __launch_bounds__(256) void rowdot_multi_kernel(const uint16_t* __restrict__ X, RowdotMulti m, int64_t T,
+                                                           int64_t K, float scale) {
+  constexpr int NW = 4, STEP = NW * 64, U = 2;
   __shared__ floatx4 red[NJ][NW][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t t0 = (int64_t)blockIdx.x * 16;
@@ -736,7 +739,7 @@ static int32_t launch_lora_gemm(const void* P, const void* Q, const uint16_t* Pe
 // work-groups, 23 us, however many waves they have), so they run as the ROW half of the one-pass kernel, a work-group
 // per chunk of columns and slab of rows, and a reduction.
 // (us, product / split: rows x K 333 x 4864 11 / 10, 333 x 11008 19 / 11, 1200 x 18944 31 / 16, 2531 x 11008 20 / 17, 4090 x 11008 22 / 22;
-// the split is one launch more)
+// the split is one launch more.  The only case where a projection has other sums alone than among others.)
 static bool rowdot_split(int64_t T, int64_t K, int n, int r) { return n == 1 && r <= 16 && K >= 8192 && T < 12 * num_cus(); }
 static size_t rowdot_split_floats(int64_t T, int64_t K, int n, int r) {
   return rowdot_split(T, K, n, r) ? (size_t)stats_geom(T, K, r, K).n_chunks * T * r + 1024 : 0;
@@ -761,21 +764,14 @@ static int32_t launch_rowdot(const void* X, RowdotMulti& m, int64_t T, int64_t K
   }
   for (int i = m.n; i <= LORA_MAX_SEG; ++i) m.e0[i] = e;
   const int nj = (e + 15) / 16;
-  auto launch = [&](auto nj_tag, auto nw_tag) {
-    constexpr int NJ = decltype(nj_tag)::value, NW = decltype(nw_tag)::value;
-    rowdot_multi_kernel<NJ, NW><<<dim3((unsigned)((T + 15) / 16), (unsigned)((nj + NJ - 1) / NJ)), 64 * NW, 0, st>>>(
+  auto launch = [&](auto nj_tag) {
+    constexpr int NJ = decltype(nj_tag)::value;
+    rowdot_multi_kernel<NJ><<<dim3((unsigned)((T + 15) / 16), (unsigned)((nj + NJ - 1) / NJ)), 256, 0, st>>>(
         (const uint16_t*)X, m, T, K, scale);
   };
-  using four = std::integral_constant<int, 4>;
-  using eight = std::integral_constant<int, 8>;
-  auto waves = [&](auto nj_tag) {
-    // (by the shape alone: a projection has the same sums alone and among others)
-    if (T >= 16 * num_cus() && K >= 1536 && K <= 2048) launch(nj_tag, eight{});
-    else launch(nj_tag, four{});
-  };
-  if (!pack || nj == 1) waves(std::integral_constant<int, 1>{});
-  else if (nj == 2) waves(std::integral_constant<int, 2>{});
-  else waves(four{});
+  if (!pack || nj == 1) launch(std::integral_constant<int, 1>{});
+  else if (nj == 2) launch(std::integral_constant<int, 2>{});
+  else launch(std::integral_constant<int, 4>{});
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }

@@ -484,14 +484,15 @@ def test_skinny_passes_of_small_ranks(artk_lib, gpu, T, n_in, n_out, r):
 
 @pytest.mark.parametrize("T,n_in,ranks", [
     (4097, 64, (8, 24, 16, 40)),      # packed: blocks of 16 factor rows over several ranks, 6 of them
-    (4100, 1600, (8, 8, 8)),          # packed, eight waves, the last pieces of K short
+    (4100, 1600, (8, 8, 8)),          # packed, the last pieces of K short
     (5000, 192, (64, 64, 64, 64)),
     (37, 448, (8, 16)),               # few rows: every factor starts its own block
     (37, 8256, (16,)), (2000, 8192, (8,)),  # long K over few rows: split over the chunks of the one-pass kernel
 ])
 def test_row_products(artk_lib, gpu, T, n_in, ranks):
-    """x A_i^T of every way the row products are dealt out, element by element: fp32 sums of bf16 products, in another
-    order than the reference's, are off by at most about sqrt(K) 2^-24 of sum |x a|; 2e-6 of it is eight times that here."""
+    """x A_i^T of every way the row products are dealt out, element by element: fp32 sums of bf16 products, of which none
+    here has more than 34 MFMA steps and additions of partial sums (K / 128 steps and four waves; 16 steps and the chunks
+    of the split form), each off by at most 2^-24 of sum |x a|: 2e-6 of it."""
     print(f"row products T={T} in={n_in} ranks={ranks}", flush=True)
     g = torch.Generator().manual_seed(T + n_in)
     x = torch.randn(T, n_in, generator=g).to(torch.bfloat16).to(gpu)
