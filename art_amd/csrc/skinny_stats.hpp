@@ -14,7 +14,7 @@ namespace artk {
 //   ROW  rp[chunk][t][e] = sum_{c in chunk} X[t,c] F[e,c]      F bf16 [R,C]  (g B: F = B^T)
 //   COL  cp[slab][c][e]  = sum_{t in slab}  X[t,c] Y[t,e]      Y f32 [T,R]   (dB: Y = x A^T)
 // A work-group owns a slab of rows x a chunk of columns and streams it through LDS
-// in 128 x 128 tiles (buffer_load ... lds, a ring of NST stages), so X is read
+// in 128 x 128 tiles (buffer_load ... lds, two stages), so X is read
 // from HBM once, fully coalesced, for both products.  Both run on MFMA 32x32x16
 // with the small dimension e as the M operand: ROW contracts over the columns
 // (row fragments of the tile, ds_read_b128), COL over the rows (transposed
@@ -114,8 +114,7 @@ __device__ __forceinline__ void stats_put_col(const StatsParams& p, int slab, bo
   }
 }
 
-// NTE: 32-wide tiles of e (rank <= 32 NTE); NCT: 128-column tiles per chunk; NST: LDS stages (two).  Ranks above 32;
-// the others have lora_stats_narrow_body below.
+// Ranks above 32 (two 32-wide tiles of e); the others have lora_stats_narrow_body below.
 // All memory traffic of the main loop is LDS DMA, ordered by hand with s_waitcnt vmcnt
 // (the compiler inserts no waits for it).
 // GATHER: the grouped form with a row gather.  The gather indices travel by DMA as well (an
@@ -125,8 +124,9 @@ __device__ __forceinline__ void stats_put_col(const StatsParams& p, int slab, bo
 // (p % 8) 4 + p / 8 so that a lane reads the 8 it needs as two 16-byte LDS loads.
 // (BLOCK is a form of its own: its tests and index products cost the other callers 2 to 6 us a launch, 17 -> 21 us for
 // 300 tokens)
-template <int NTE, int NCT, int NST, bool GATHER, bool BLOCK = false>
+template <bool GATHER, bool BLOCK = false>
 __device__ __forceinline__ void lora_stats_body(const StatsParams& p, const int block) {
+  constexpr int NTE = 2, NCT = 2, NST = 2;  // tiles of e, 128-column tiles per chunk, LDS stages
   constexpr int CC = NCT * ST_TILE;
   constexpr int FPITCH = CC + 8;  // halfwords; +16 bytes: rows e land in different banks
   constexpr int YRAW_BYTES = ST_TILE * NTE * 32 * 4;
@@ -322,9 +322,7 @@ __device__ __forceinline__ void lora_stats_body(const StatsParams& p, const int 
   };
   for (int rt = 0; rt < n_rt; ++rt) {
     do_tile(rt, std::integral_constant<int, 0>{});
-    if constexpr (NCT > 1) if (nct > 1) do_tile(rt, std::integral_constant<int, 1>{});
-    if constexpr (NCT > 2) if (nct > 2) do_tile(rt, std::integral_constant<int, 2>{});
-    if constexpr (NCT > 3) if (nct > 3) do_tile(rt, std::integral_constant<int, 3>{});
+    if (nct > 1) do_tile(rt, std::integral_constant<int, 1>{});
   }
   if (do_col) {
 #pragma unroll
@@ -586,9 +584,9 @@ __global__ __launch_bounds__(256, 2) void lora_stats_narrow_kernel(StatsParams p
   lora_stats_narrow_body<NTE, NCT, GATHER, BLOCK, ONCE>(p, (int)blockIdx.x);
 }
 
-template <int NTE, int NCT, int NST, bool GATHER, bool BLOCK = false>
+template <bool GATHER, bool BLOCK = false>
 __global__ __launch_bounds__(256) void lora_stats_kernel(StatsParams p) {
-  lora_stats_body<NTE, NCT, NST, GATHER, BLOCK>(p, (int)blockIdx.x);
+  lora_stats_body<GATHER, BLOCK>(p, (int)blockIdx.x);
 }
 
 // Several independent passes (the upstream gradients of projections that share an input) in one
@@ -599,11 +597,10 @@ struct StatsMulti {
   int block0[STATS_MULTI_MAX + 1];
   int n;
 };
-template <int NTE, int NCT, int NST>
-__global__ __launch_bounds__(256) void lora_stats_multi_kernel(StatsMulti m) {
+__global__ __launch_bounds__(256) static void lora_stats_multi_kernel(StatsMulti m) {
   int i = 0;
   while (i + 1 < m.n && (int)blockIdx.x >= m.block0[i + 1]) ++i;
-  lora_stats_body<NTE, NCT, NST, false>(m.p[i], (int)blockIdx.x - m.block0[i]);
+  lora_stats_body<false>(m.p[i], (int)blockIdx.x - m.block0[i]);
 }
 
 template <int NTE, int NCT, bool ONCE>
@@ -769,19 +766,20 @@ static inline StatsParams stats_params(const void* X, int64_t T, int64_t C, cons
 // 361 MB of upstream gradients 102 -> 75 us.  (201 MB that the kernel before has just written: 67 -> 72 us.)
 static inline bool stats_once(int64_t bytes) { return bytes > (256ll << 20); }
 
-// Which kernel takes a rank; the passes of one launch are all of one shape (the caller checks).
-enum StatsShape { STATS_NARROW, STATS_32, STATS_WIDE };
-static inline StatsShape stats_shape(int r) { return r > 32 ? STATS_WIDE : r > 16 ? STATS_32 : STATS_NARROW; }
+// Which kernel takes a rank, by the largest: the narrow one with one or two blocks of 16, or the one above.  The passes of one
+// launch are all of one shape (the caller checks).
+enum StatsShape { STATS_16, STATS_32, STATS_64 };
+static inline StatsShape stats_shape(int r) { return r > 32 ? STATS_64 : r > 16 ? STATS_32 : STATS_16; }
 
 static inline int32_t launch_stats_params(const StatsParams& p, hipStream_t st) {
   const unsigned grid = (unsigned)(p.n_slabs * p.n_chunks);
   switch (stats_shape(p.R)) {
-    case STATS_WIDE: lora_stats_kernel<2, 2, 2, false><<<grid, 256, 0, st>>>(p); break;
+    case STATS_64: lora_stats_kernel<false><<<grid, 256, 0, st>>>(p); break;
     case STATS_32:
       if (stats_once(p.T * p.C * 2)) lora_stats_narrow_kernel<2, 2, false, false, true><<<grid, 256, 0, st>>>(p);
       else lora_stats_narrow_kernel<2, 2, false><<<grid, 256, 0, st>>>(p);
       break;
-    case STATS_NARROW:
+    case STATS_16:
       if (stats_once(p.T * p.C * 2)) lora_stats_narrow_kernel<1, 4, false, false, true><<<grid, 256, 0, st>>>(p);
       else lora_stats_narrow_kernel<1, 4, false><<<grid, 256, 0, st>>>(p);
       break;
@@ -805,8 +803,8 @@ static inline int32_t launch_stats_multi(StatsMulti& m, StatsShape shape, hipStr
     bytes += m.p[i].T * m.p[i].C * 2;
   }
   m.block0[m.n] = blocks;
-  if (shape == STATS_WIDE)
-    lora_stats_multi_kernel<2, 2, 2><<<(unsigned)blocks, 256, 0, st>>>(m);
+  if (shape == STATS_64)
+    lora_stats_multi_kernel<<<(unsigned)blocks, 256, 0, st>>>(m);
   else if (shape == STATS_32 && stats_once(bytes))
     lora_stats_narrow_multi_kernel<2, 2, true><<<(unsigned)blocks, 256, 0, st>>>(m);
   else if (shape == STATS_32)
@@ -902,14 +900,14 @@ static inline int32_t launch_stats_grouped(const void* X, int64_t x_rows, const 
     constexpr bool BLOCK = decltype(is_block)::value;
     if (gather) {
       if (r > 32)
-        lora_stats_kernel<2, 2, 2, true, BLOCK><<<grid, 256, 0, st>>>(p);
+        lora_stats_kernel<true, BLOCK><<<grid, 256, 0, st>>>(p);
       else if (r > 16)
         lora_stats_narrow_kernel<2, 2, true, BLOCK><<<grid, 256, 0, st>>>(p);
       else
         lora_stats_narrow_kernel<1, 4, true, BLOCK><<<grid, 256, 0, st>>>(p);
     } else {
       if (r > 32)
-        lora_stats_kernel<2, 2, 2, false, BLOCK><<<grid, 256, 0, st>>>(p);
+        lora_stats_kernel<false, BLOCK><<<grid, 256, 0, st>>>(p);
       else if (r > 16)
         lora_stats_narrow_kernel<2, 2, false, BLOCK><<<grid, 256, 0, st>>>(p);
       else
