@@ -23,6 +23,10 @@ constexpr int SUMSQ_BLOCKS = 1024;
 // read, in it: 20.2 M elements with 8-bit moments 103 -> 94 us a step (loads or stores alone: no gain; the gradients
 // too: 110).
 // With fp32 moments a step of 449 MB still finds enough there (78 us, 80 past the cache); 605 MB: 117 -> 104 us.
+// The kernels of a step in a trace, through the caches / past them, step after step; and each after 1 GiB of other writes,
+// as behind a backward pass: 8-bit moments 11.6 M elements 62 / 62; 76 / 73, 15.0 M 73 / 75; 93 / 92, 20.2 M 95 / 92;
+// 115 / 110, 40.4 M 192 / 171; 211 / 203; fp32 11.6 M 63 / 65; 83 / 79, 15.0 M 80 / 80; 103 / 98, 20.2 M 120 / 106;
+// 140 / 130, 40.4 M 269 / 218; 280 / 267.
 static inline bool step_once8(int64_t n) { return 18 * n > (256ll << 20); }
 static inline bool step_once32(int64_t n) { return 30 * n > (512ll << 20); }
 template <bool ONCE, class T>
@@ -162,8 +166,8 @@ struct AdamW8Params {
 // that is not nearer to entry k + 1.  The leading 16 bits of the fp32 value (sign, exponent, 7 mantissa bits) select a
 // byte: the first entry whose threshold is not below everything in that bin.  In the books in use no bin holds two
 // thresholds (the finest octave, [0.5, 1), has 71 entries in 128 bins), so the code is that byte, or one more where the
-// value is above its threshold: two LDS gathers and no loop.  A book with a fuller bin walks up from there, over the
-// entries themselves.  (A bisection, eight dependent gathers per value, took 182 us for 20.2 M elements; a start byte and
+// value is above its threshold: two LDS gathers and no loop.  A book with a fuller bin, or without all its thresholds, walks
+// from there, over the entries themselves.  (A bisection, eight dependent gathers per value, took 182 us for 20.2 M elements; a start byte and
 // a walk that compares with two neighbours 84 us, 137 vector instructions per element.)
 constexpr int LUT_E0 = 104;                      // exponents 104 .. 127: [2^-23, 1]; smaller values share bin 0
 constexpr int LUT_HALF = (128 - LUT_E0) * 128;   // bins of one sign
@@ -178,8 +182,9 @@ __device__ __forceinline__ float lut_edge(int j) {
   return j == 0 ? -INFINITY : -__uint_as_float((uint32_t)(LUT_HALF - j + LUT_E0 * 128) << 16);
 }
 
-// The largest float that the rule gives to entry `cur` rather than to the next one, and whether it was found (within 32
-// floats of the middle; always, in an ascending book).
+// The largest float that the rule gives to entry `cur` rather than to the next one, and whether it was found within 32 floats
+// of the middle.  It is in the books in use; not between -a and a for instance, where everything near 0 is a tie once
+// the differences are rounded.  A book with such a gap takes the walk below.
 __device__ bool code_threshold(float cur, float next, float& thr) {
   auto lower = [&](float x) { return x < next && x - cur <= next - x; };
   auto key = [](float x) {  // floats in the order of integers, and back

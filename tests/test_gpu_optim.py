@@ -99,7 +99,7 @@ def test_adamw8bit_matches_oracle(artk_lib, gpu):
 
 
 @pytest.mark.parametrize("n", [5, 256 * 3 + 17, 256 * 16 * 512 + 300])
-@pytest.mark.parametrize("book", ["dynamic", "linear", "clustered"])
+@pytest.mark.parametrize("book", ["dynamic", "linear", "clustered", "gap"])
 def test_adamw8bit_any_code_book(artk_lib, gpu, n, book):
     """One step from a given state at the edges of the grid (less than one block, a last partial block, more
     blocks than waves) and for code books whose entries crowd a bin of the start table or leave most of them
@@ -114,6 +114,10 @@ def test_adamw8bit_any_code_book(artk_lib, gpu, n, book):
         b1, b2 = dynamic_code_book(True).numpy(), dynamic_code_book(False).numpy()
     elif book == "linear":
         b1, b2 = np.linspace(-1, 1, 256, dtype=np.float32), np.linspace(0, 1, 256, dtype=np.float32)
+    elif book == "gap":
+        b1 = np.linspace(-1, 1, 256, dtype=np.float32)
+        b1[:128], b1[128:] = -np.linspace(1, 0.25, 128), np.linspace(0.25, 1, 128)
+        b2 = np.linspace(0.25, 1, 256, dtype=np.float32)
     else:
         b1 = np.sort(np.concatenate([[-1, 0, 1], 0.5 + 1e-3 * rng.random(253)])).astype(np.float32)
         b2 = np.sort(np.concatenate([[0, 1], 1e-8 * rng.random(100), 0.7 + 1e-2 * rng.random(154)])).astype(np.float32)
