@@ -437,8 +437,9 @@ def plan_arrays(plan, S):
 @pytest.mark.parametrize("S", [1, 31, 64, 130, 256, 257, 700, 1009, 1024])
 @pytest.mark.parametrize("ids", ["packed", "random", "one"])
 def test_plan_of_a_short_row_is_that_of_a_long_one(artk_lib, gpu, S, ids):
-    """Rows of up to 1024 positions have their plan from one work-group, longer ones from a chain of kernels.  Continued by
-    positions whose ids occur nowhere else, a short row becomes a long one with the same visibility."""
+    """Rows of up to 1024 positions have their plan from two launches (a work-group per query block that finds the codes of
+    the row for itself, then one per row that orders the tiles), longer ones from a chain of five.  Continued by positions
+    whose ids occur nowhere else, a short row becomes a long one with the same visibility."""
     print(f"short plan S={S} ids={ids}", flush=True)
     g = torch.Generator().manual_seed(S)
     if ids == "packed" and S >= 130:

@@ -12,7 +12,7 @@ import torch
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oracle"))
 import lora_oracle  # noqa: E402
 
-from art_amd import ops  # noqa: E402
+from art_amd import _lib, ops  # noqa: E402
 from art_amd.lora import LoRALinear, lora_linear  # noqa: E402
 
 pytestmark = pytest.mark.gpu
@@ -509,14 +509,29 @@ def test_row_products(artk_lib, gpu, T, n_in, ranks):
         assert ((xa[1:].double() - ref).abs() <= 2e-6 * bound).all()
 
 
-@pytest.mark.parametrize("T,n_in,outs", [
-    (1500, 11008, (2048,)),          # forward in parts, rows that are no multiple of a tile
-    (1300, 2048, (11008, 11008)),    # input gradient in parts, of which some span both projections
-    (700, 9024, (960, 1088)),        # two jobs, ragged weight tiles
+def partial_units(T, K, Ms):
+    """Units of 256 x 256 fp32 partial sums in the workspace of products [M_i, K] x [T, K]^T (at rank 24, where nothing else
+    in it comes near one)."""
+    proj = (_lib.LoraProjStruct * len(Ms))()
+    for p, M in zip(proj, Ms):
+        p.out, p.r = M, 24
+    return _lib.load().artk_lora_linear_multi_fwd_workspace_bytes(T, K, proj, len(Ms)) // (256 * 256 * 4)
+
+
+@pytest.mark.parametrize("T,n_in,outs,way", [
+    (1500, 11008, (2048,), "forward"),               # rows that are no multiple of a tile
+    (1000, 16384, (960, 1088), "forward"),           # two jobs, ragged weight tiles
+    (700, 18944, (1088, 1088, 1088), "forward"),     # three
+    (1300, 2048, (11008, 11008), "backward"),        # input gradient: parts that span both projections
+    (1300, 1984, (11008, 11072), "backward"),        # and ragged weight tiles
 ])
-def test_long_products_of_few_tiles(artk_lib, gpu, T, n_in, outs):
+def test_long_products_of_few_tiles(artk_lib, gpu, T, n_in, outs, way):
     """Products whose K range is split over work-groups on 256 x 256 tiles, block by block (bf16 output rounding: 2e-3
-    relative; a part that is missing or added twice is a third of the block or more)."""
+    relative; a part that is missing or added twice is an eighth of the block or more)."""
+    K, Ms = (n_in, outs) if way == "forward" else (sum(outs), (n_in,))
+    tiles = sum((M + 255) // 256 for M in Ms) * ((T + 255) // 256)
+    units = partial_units(T, K, Ms)
+    assert units % tiles == 0 and 2 <= units // tiles <= 8, "the shape runs on other tiles now: choose another"
     print(f"long products T={T} in={n_in} outs={outs}", flush=True)
     g = torch.Generator().manual_seed(T)
     rand = lambda *s, std=1.0: (std * torch.randn(*s, generator=g)).to(torch.bfloat16).to(gpu)
