@@ -465,9 +465,10 @@ __global__ __launch_bounds__(256) void lora_split_reduce_kernel(LoraSmallParams 
 // reads whole cache lines), two of them in flight at a time.  Writes f32 [T,R] (unscaled) and bf16 [T,RP] (scaled, zero
 // padded to RP).
 // Where there are rows enough the factors are packed (e0 by R: two ranks of 8 are one block) and X is read once for
-// ranks that add up to 64; else every factor starts a block of its own (e0 by RP) and there are more work-groups.  us, a
-// work-group per 16 rows and factor / packed: [8192, 2048] and 2 ranks of 8 21 / 14, [4096, 2048] and 3 of 8 14 / 9,
-// [8192, 896] and 2 of 8 9 / 7, [1000, 3584] and 2 of 8 11 / 13.
+// ranks that add up to 64; else every 16 factor rows are a work-group's, every factor starts a block of its own (e0 by RP) and
+// there are more work-groups.  us, a work-group per 16 rows and factor / packed: [8192, 2048] and 2 ranks of 8 21 / 14,
+// [4096, 2048] and 3 of 8 14 / 9, [8192, 896] and 2 of 8 9 / 7, [1000, 3584] and 2 of 8 11 / 13; one factor: [8192, 2048] of 64
+// 37 / 23, [8192, 896] of 40 15 / 12, [4100, 3584] of 24 18 / 17.
 // (Eight waves and twice the pieces in flight: one factor of rank 8 over 8192 rows, K = 896 6.1 / 10.4, 1536 7.9 / 10.3,
 // 2048 11.8 / 9.4, 2560 10.5 / 14.8, 4096 15.3 / 15.5, 8192 31.7 / 30.3; two factors at 2048 11.6 / 12.4.  Not kept for one
 // width.)
@@ -756,7 +757,7 @@ static int32_t launch_rowdot_split(const void* X, const void* Mt, int64_t T, int
 
 // Fills m.e0 and launches.
 static int32_t launch_rowdot(const void* X, RowdotMulti& m, int64_t T, int64_t K, float scale, hipStream_t st) {
-  const bool pack = m.n > 1 && T >= 16 * num_cus();
+  const bool pack = T >= 16 * num_cus();
   int e = 0;
   for (int i = 0; i < m.n; ++i) {
     m.e0[i] = e;

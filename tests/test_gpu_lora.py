@@ -486,6 +486,7 @@ def test_skinny_passes_of_small_ranks(artk_lib, gpu, T, n_in, n_out, r):
     (4097, 64, (8, 24, 16, 40)),      # packed: blocks of 16 factor rows over several ranks, 6 of them
     (4100, 1600, (8, 8, 8)),          # packed, the last pieces of K short
     (5000, 192, (64, 64, 64, 64)),
+    (4100, 192, (24,)), (4097, 640, (40,)),  # one factor of several blocks, packed
     (37, 448, (8, 16)),               # few rows: every factor starts its own block
     (37, 8256, (16,)), (2000, 8192, (8,)),  # long K over few rows: split over the chunks of the one-pass kernel
 ])
