@@ -412,7 +412,10 @@ constexpr int SG_LDS_BYTES = 80 * 1024;           // two work-groups per CU
 template <int NQ> constexpr int sg_stages() { return NQ <= 2 ? 4 : 3; }
 
 // acc[i] += 32 weight rows of this wave x columns 32 i .. 32 i + 31 over nk K steps.  Every wave calls it together; LDS
-// may be reused when it returns.  ONCE: nobody reads the weights again, they pass the caches by (0.8 GB in 135 us instead of 150).
+// may be reused when it returns.  ONCE: nobody reads the weights again, they pass the caches by (0.8 GB in 135 us instead of
+// 150).  Whatever their size: a model's other layers come before they are read again.  Four products of a block, through / past
+// the caches, after 1 GiB of other writes: 8 experts (75 MB) 124 / 102 us, 16 151 / 101, 32 210 / 146; the same block again and
+// again, with nothing in between: 80 / 101, 107 / 101, 160 / 146.
 template <int NQ, bool ONCE>
 __device__ __forceinline__ void moe_stream_run(floatx16 (&acc)[NQ], char* smem, dma_rsrc_t prsrc, const int (&pv)[2],
                                                int pstep, dma_rsrc_t qrsrc, const int (&qv)[2 * NQ], int nk) {
