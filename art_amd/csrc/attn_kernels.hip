@@ -22,7 +22,7 @@
 // one's set-up and store behind the other's tiles, and a list is made for 128
 // queries instead of 256.  Against one work-group of 8 waves per CU with three
 // stages, 16384 positions of 8 prompts of 137 + 4 x 461, 28 / 4 heads of 128:
-// forward 205 -> 154 us, dQ 279 -> 244 us, dK/dV 433 -> 297 us.  On dense causal
+// forward 205 -> 154 us, dQ 279 -> 244 us, dK/dV 433 -> 297 us (and the second stage since).  On dense causal
 // rows, where every tile comes into LDS twice as often, forward + backward are
 // 15 % faster to 3 % slower (us, 8 waves / now):
 //   heads of 128, 28 / 4: 4096 positions 630 / 618, 8192 2248 / 2151, 16384 8268 / 8379
@@ -979,22 +979,21 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kern
         dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(T::row_frag(st + G::V_OFF, 32 * kt + n, s, h), dof[s],
                                                      dp, 0, 0, 0);
       }
+      if (partial) {  // one branch for all elements: tested inside the loop below it becomes one per element
 #pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const int kk = 32 * kt + 8 * g4 + 4 * h;
-        int kcv[4] = {0, 0, 0, 0};
-        if (partial) {
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const int kk = 32 * kt + 8 * g4 + 4 * h;
           const int4 kc = *(const int4*)(codes + kk);
-          kcv[0] = kc.x; kcv[1] = kc.y; kcv[2] = kc.z; kcv[3] = kc.w;
-        }
+          const int kcv[4] = {kc.x, kc.y, kc.z, kc.w};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int j = 4 * g4 + e;
-          float x = __builtin_fmaf(sc[j], p.scale_log2e, nlse2);
-          if (partial && !attn_visible(q, kb * ATT_BN + kk + e, gi, pi, kcv[e])) x = -INFINITY;
-          const float pr = __builtin_amdgcn_exp2f(x);
-          dsf[2 * kt + j / 8][j % 8] = (__bf16)(pr * (dp[j] - delta));
+          for (int e = 0; e < 4; ++e)
+            if (!attn_visible(q, kb * ATT_BN + kk + e, gi, pi, kcv[e])) sc[4 * g4 + e] = -INFINITY;
         }
+      }
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j], p.scale_log2e, nlse2));
+        dsf[2 * kt + j / 8][j % 8] = (__bf16)(pr * (dp[j] - delta));
       }
     }
     // dQ^T += K^T dS^T, K^T fragments by transposing reads of the K tile
@@ -1021,58 +1020,63 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kern
 // 4 wavefronts = 2 key groups of 32 x 2 halves of each 64-query tile; two work-groups per CU (D = 64:
 // three), so that the exp2 / convert work, the DMA latency and the set-up of one overlap the MFMAs of the
 // other.  The two waves of a key group keep separate accumulators, added through LDS at the end.
-// Bound: LDS.  A wave's step of 32 MFMAs reads 48 KiB of fragments and its share of the DMA writes 8, about 90 bytes per
-// clock and CU.  So the wave's K rows stay in registers for the whole kernel (40 KiB to read; the V rows, which do
-// not fit beside them, are re-read from LDS), with one register per fragment row instead of one per address to make
-// the room.  Dense causal rows, dK/dV in us before / after: 16384 positions, 28 / 4 heads of 128: 4225 / 4010; 8192,
-// 16 / 2: 665 / 633; the row of the header's figures: 314 / 297.  (The next tile's DMA issued in two halves, each as
-// soon as its tile is free, measured level.)
+// Bound: LDS reads, exp2 and the MFMAs, which two waves of a SIMD overlap in part.  The wave's K rows and the upper half of
+// its V rows (D = 128) stay in registers for the whole kernel: 36 KiB of fragments per step of 32 MFMAs instead of 48, and
+// room in LDS for a second stage, so that a query tile comes in during the step before instead of between two barriers of
+// its own.  The registers for that come from one per fragment row instead of one per address, and from P before dP (half
+// the fragments in flight).  One stage, V rows all in LDS / now, backward in us: dense causal rows of 16384 positions,
+// 28 / 4 heads of 128: 6640 / 6280; 8192, 16 / 2: 1000 / 976; 8192, 14 / 2 heads of 64: 518 / 465; the row of the header's
+// figures 570 / 525 (20 us of it, and of the short rows' 85 / 81, is the mask as one branch per step, here and in dQ, instead
+// of one per element).
 // A work-group that does not take all heads of its group writes fp32 partial sums, which
 // attn_kv_reduce_kernel adds in a fixed order.
-// LDS: Q tile, dO tile (64 queries), lse2 / delta / group / parent codes of those queries, and the block's K and V rows.
+// LDS: two stages of a Q tile, a dO tile (64 queries) and lse2 / delta / group / parent codes of those queries; then
+// columns 0 .. 63 of the block's V rows.  The K rows and what is left of the V rows pass through the second stage on
+// their way to registers.
 template <int D>
 struct AttnQStage {
   using T = AttnTile<D>;
+  using TV = AttnTile<64>;
   static constexpr int DO_OFF = T::BYTES;
   static constexpr int ROW_OFF = 2 * T::BYTES;
-  static constexpr int KV_OFF = ROW_OFF + 1024;          // K block, then V block
-  static constexpr int LDS = KV_OFF + 2 * T::BYTES;
+  static constexpr int STAGE = ROW_OFF + 1024;
+  static constexpr int V_OFF = 2 * STAGE;
+  static constexpr int LDS = V_OFF + TV::BYTES;
+  static constexpr int VR = D / 16 - 4;                  // 16-column steps of V in registers
 };
 
 // DMA of one query tile into a stage: this wave's share of the Q and dO tiles and
 // one of the four per-query arrays (wave 0: lse2, 1: delta, 2: group codes, 3: parent codes).
+// row_q, row_do, chunk: byte offset of this lane's row and chunk in instruction 0 (AttnTile::voff).  The instructions of a
+// wave begin a multiple of 4 (D = 64: 8) rows apart, so their swizzles differ by an XOR: three registers for both tiles
+// instead of one per instruction.
 template <int D>
 __device__ __forceinline__ void attn_issue_q(char* st, int hq, int q0, const uint16_t* q_row, const uint16_t* do_row,
-                                             dma_rsrc_t rsrc_row, const int* voff_q,
-                                             const int* voff_do, const AttnBwdParams& p, int wave,
+                                             dma_rsrc_t rsrc_row, int row_q, int row_do, int chunk, const AttnBwdParams& p, int wave,
                                              int lane) {
   using T = AttnTile<D>;
   using G = AttnQStage<D>;
   const dma_rsrc_t rsrc_q = attn_head_rsrc<D>(q_row + hq * p.q_hs, p.q_ss, p.S);
   const dma_rsrc_t rsrc_do = attn_head_rsrc<D>(do_row + hq * p.do_hs, p.do_ss, p.S);
-  const int so_q = (int)(q0 * p.q_ss * 2);
-  const int so_do = (int)(q0 * p.do_ss * 2);
 #pragma unroll
   for (int i = 0; i < T::N4; ++i) {
-    dma_load16(rsrc_q, voff_q[i], so_q, lds_addr_of(st + (wave * T::N4 + i) * 1024));
-    dma_load16(rsrc_do, voff_do[i], so_do, lds_addr_of(st + G::DO_OFF + (wave * T::N4 + i) * 1024));
+    const int r = (wave * T::N4 + i) * (64 / T::CHK);   // first row of the instruction
+    const int c = chunk ^ (T::swz(r) << 4);
+    dma_load16(rsrc_q, row_q + c, (int)((q0 + r) * p.q_ss * 2), lds_addr_of(st + (wave * T::N4 + i) * 1024));
+    dma_load16(rsrc_do, row_do + c, (int)((q0 + r) * p.do_ss * 2), lds_addr_of(st + G::DO_OFF + (wave * T::N4 + i) * 1024));
   }
   const int arr = wave;
   dma_load4(rsrc_row, lane * 4, (int)(((arr < 2 ? (int64_t)hq * p.Sp : 0) + q0) * 4), lds_addr_of(st + G::ROW_OFF + arr * 256));
 }
 
-// The block's K and V rows (64 each).
+// DMA of 64 rows from row0 on of one head into an LDS tile of D columns.
 template <int D>
-__device__ __forceinline__ void attn_issue_kv_block(char* dst, int key0, dma_rsrc_t rsrc_k,
-                                                    dma_rsrc_t rsrc_v, const int* voff_k,
-                                                    const int* voff_v, int64_t k_ss, int64_t v_ss,
-                                                    int wave) {
+__device__ __forceinline__ void attn_issue_block(char* dst, int row0, dma_rsrc_t rsrc, int64_t stride, int wave, int lane) {
   using T = AttnTile<D>;
 #pragma unroll
-  for (int i = 0; i < T::N4; ++i) {
-    dma_load16(rsrc_k, voff_k[i], (int)(key0 * k_ss * 2), lds_addr_of(dst + (wave * T::N4 + i) * 1024));
-    dma_load16(rsrc_v, voff_v[i], (int)(key0 * v_ss * 2), lds_addr_of(dst + T::BYTES + (wave * T::N4 + i) * 1024));
-  }
+  for (int i = 0; i < T::N4; ++i)
+    dma_load16(rsrc, T::voff(wave * T::N4 + i, lane, stride), (int)(row0 * stride * 2),
+               lds_addr_of(dst + (wave * T::N4 + i) * 1024));
 }
 
 template <int D>
@@ -1109,23 +1113,21 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
   const void* row_src = arr == 0 ? (const void*)(p.lse2 + stat_row) : arr == 1 ? (const void*)(p.delta + stat_row)
                         : arr == 2 ? (const void*)gc : (const void*)attn_row(p.pc, p.plan_stride, brow);
   const dma_rsrc_t rsrc_row = attn_rsrc(row_src);
-  int voff_q[T::N4], voff_do[T::N4];
+  int row_q = lane / T::CHK * (int)(p.q_ss * 2), row_do = lane / T::CHK * (int)(p.do_ss * 2);
+  int chunk = ((lane % T::CHK) ^ T::swz(lane / T::CHK)) << 4;
   {
-    int voff_k[T::N4], voff_v[T::N4];
-#pragma unroll
-    for (int i = 0; i < T::N4; ++i) {
-      voff_q[i] = T::voff(wave * T::N4 + i, lane, p.q_ss);
-      voff_do[i] = T::voff(wave * T::N4 + i, lane, p.do_ss);
-      voff_k[i] = T::voff(wave * T::N4 + i, lane, p.k_ss);
-      voff_v[i] = T::voff(wave * T::N4 + i, lane, p.v_ss);
-    }
-    attn_issue_kv_block<D>(smem + G::KV_OFF, kb * ATT_BK2, attn_head_rsrc<D>(p.K + brow * p.k_bs + (int64_t)hkv * p.k_hs, p.k_ss, p.S),
-                           attn_head_rsrc<D>(p.V + brow * p.v_bs + (int64_t)hkv * p.v_hs, p.v_ss, p.S), voff_k, voff_v, p.k_ss, p.v_ss, wave);
+    const uint16_t* const k_head = p.K + brow * p.k_bs + (int64_t)hkv * p.k_hs;
+    const uint16_t* const v_head = p.V + brow * p.v_bs + (int64_t)hkv * p.v_hs;
+    attn_issue_block<D>(smem + G::STAGE, kb * ATT_BK2, attn_head_rsrc<D>(k_head, p.k_ss, p.S), p.k_ss, wave, lane);
+    attn_issue_block<64>(smem + G::V_OFF, kb * ATT_BK2, attn_head_rsrc<64>(v_head, p.v_ss, p.S), p.v_ss, wave, lane);
+    if constexpr (D > 64)
+      attn_issue_block<D - 64>(smem + G::STAGE + T::BYTES, kb * ATT_BK2, attn_head_rsrc<D - 64>(v_head + 64, p.v_ss, p.S),
+                               p.v_ss, wave, lane);
   }
   const int total = cnt * nheads;
   if (total > 0)  // the first tile of the flattened (head, visible query tile) sequence
     attn_issue_q<D>(smem, hq, __builtin_amdgcn_readfirstlane(list[0] & 0x3fff) * ATT_BQ2, q_row, do_row, rsrc_row,
-                    voff_q, voff_do, p, wave, lane);
+                    row_q, row_do, chunk, p, wave, lane);
 
   floatx16 dk[D / 32], dv[D / 32];
 #pragma unroll
@@ -1136,69 +1138,99 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
   pin_loaded(gk);
   wait_vmcnt<0>();
   barrier_lds_only();  // the list, the block's K and V rows and the first tile are there
-  const char* const vblk = smem + G::KV_OFF + T::BYTES;
+  const char* const vblk = smem + G::V_OFF;
   const int krow = 32 * kg + n;  // this wave's keys inside the block
-  bf16x8 kf[D / 16];
+  bf16x8 kf[D / 16], vr[G::VR > 0 ? G::VR : 1];
 #pragma unroll
-  for (int s = 0; s < D / 16; ++s) kf[s] = T::row_frag(smem + G::KV_OFF, krow, s, h);
+  for (int s = 0; s < D / 16; ++s) kf[s] = T::row_frag(smem + G::STAGE, krow, s, h);
+#pragma unroll
+  for (int s = 0; s < G::VR; ++s) vr[s] = G::TV::row_frag(smem + G::STAGE + T::BYTES, krow, s, h);
 #pragma unroll
   for (int s = 0; s < D / 16; ++s) pin_loaded(kf[s]);
-  int bq = frag_base<D>(32 * qh + n, h), bv = frag_base<D>(krow, h);
+#pragma unroll
+  for (int s = 0; s < G::VR; ++s) pin_loaded(vr[s]);
+  int bq = frag_base<D>(32 * qh + n, h), bv = frag_base<64>(krow, h);
   TrBase bt = tr_base<D>(tr, 32 * qh);
   int ti = 0, head = hq;
   for (int it = 0; it < total; ++it) {
-    if (it > 0) {
-      barrier_lds_only();  // every wave is done with the tile before
-      attn_issue_q<D>(smem, head, __builtin_amdgcn_readfirstlane(s_list[ti] & 0x3fff) * ATT_BQ2, q_row, do_row, rsrc_row,
-                      voff_q, voff_do, p, wave, lane);
-      wait_vmcnt<0>();
-      barrier_lds_only();
-    }
+    wait_vmcnt<0>();
+    barrier_lds_only();  // this tile is there, and every wave is done with the one before (it = 0: with the K and V rows)
     const int entry = __builtin_amdgcn_readfirstlane(s_list[ti]);
     if (++ti == cnt) {
       ti = 0;
       ++head;
     }
+    pin_loaded(row_q);  // (or what follows from them is kept in registers of its own; so below)
+    pin_loaded(row_do);
+    pin_loaded(chunk);
+    if (it + 1 < total)
+      attn_issue_q<D>(smem + ((it + 1) & 1) * G::STAGE, head, __builtin_amdgcn_readfirstlane(s_list[ti] & 0x3fff) * ATT_BQ2,
+                      q_row, do_row, rsrc_row, row_q, row_do, chunk, p, wave, lane);
+    const char* const st = smem + (it & 1) * G::STAGE;
     const int q0 = (entry & 0x3fff) * ATT_BQ2;
     const bool active = (entry >> (16 + wave)) & 1;        // this wave's keys x query half
     const bool partial = !((entry >> (24 + wave)) & 1);
-    const char* dot = smem + G::DO_OFF;
-    const float* r_lse2 = (const float*)(smem + G::ROW_OFF);
+    const char* dot = st + G::DO_OFF;
+    const float* r_lse2 = (const float*)(st + G::ROW_OFF);
     const float* r_delta = r_lse2 + 64;
     const int* r_gc = (const int*)(r_lse2 + 128);
     const int* r_pc = r_gc + 64;
     if (!active) continue;
-    // (or the addresses of all reads are kept in registers of their own)
     pin_loaded(bq);
     pin_loaded(bv);
     pin_loaded(bt.lo);
     pin_loaded(bt.hi);
 
+    constexpr int NS = D / 16;
     floatx16 sc, dp;
 #pragma unroll
     for (int j = 0; j < 16; ++j) sc[j] = dp[j] = 0.f;
     {
-      // fragments two steps ahead of the MFMAs that use them (LDS latency; more would not fit the registers)
-      constexpr int NS = D / 16, PF = 2;
-      bf16x8 qf[NS], of[NS], vf[NS];
+      // fragments PF steps ahead of the MFMAs that use them (LDS latency; more would not fit the registers)
+      constexpr int PF = 3;
+      bf16x8 qf[NS];
+#pragma unroll
+      for (int s = 0; s < PF; ++s) qf[s] = frag_at(st, bq, s);
+      __builtin_amdgcn_sched_group_barrier(0x100, PF, 0);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        if (s + PF < NS) qf[s + PF] = frag_at(st, bq, s + PF);
+        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[s], kf[s], sc, 0, 0, 0);
+        if (s + PF < NS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      }
+    }
+    if (partial) {  // one branch for all elements: tested inside the loop below it becomes one per element
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const int qi = 32 * qh + 8 * g4 + 4 * h;
+        const int4 a4 = *(const int4*)(r_gc + qi);
+        const int4 b4 = *(const int4*)(r_pc + qi);
+        const int gq[4] = {a4.x, a4.y, a4.z, a4.w}, pq[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (!attn_visible(q0 + qi + e, key, gq[e], pq[e], gk)) sc[4 * g4 + e] = -INFINITY;
+      }
+    }
+    {
+      constexpr int PF = 2;
+      bf16x8 of[NS], vf[NS];
 #pragma unroll
       for (int s = 0; s < PF; ++s) {
-        qf[s] = frag_at(smem, bq, s);
         of[s] = frag_at(dot, bq, s);
         vf[s] = frag_at(vblk, bv, s);
       }
-      __builtin_amdgcn_sched_group_barrier(0x100, 3 * PF, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2 * PF, 1);
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
         if (s + PF < NS) {
-          qf[s + PF] = frag_at(smem, bq, s + PF);
           of[s + PF] = frag_at(dot, bq, s + PF);
-          vf[s + PF] = frag_at(vblk, bv, s + PF);
+          vf[s + PF] = s + PF < 4 ? frag_at(vblk, bv, s + PF) : vr[s + PF < 4 ? 0 : s + PF - 4];
         }
-        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[s], kf[s], sc, 0, 0, 0);
         dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(of[s], vf[s], dp, 0, 0, 0);
-        if (s + PF < NS) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        if (s + PF < 4) __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
+        else if (s + PF < NS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
       }
     }
     bf16x8 pf[2], dsf[2];
@@ -1207,19 +1239,10 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
       const int qi = 32 * qh + 8 * g4 + 4 * h;
       const floatx4 l4 = *(const floatx4*)(r_lse2 + qi);
       const floatx4 d4 = *(const floatx4*)(r_delta + qi);
-      int gq[4] = {0, 0, 0, 0}, pq[4] = {0, 0, 0, 0};
-      if (partial) {
-        const int4 a4 = *(const int4*)(r_gc + qi);
-        const int4 b4 = *(const int4*)(r_pc + qi);
-        gq[0] = a4.x; gq[1] = a4.y; gq[2] = a4.z; gq[3] = a4.w;
-        pq[0] = b4.x; pq[1] = b4.y; pq[2] = b4.z; pq[3] = b4.w;
-      }
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int j = 4 * g4 + e;
-        float x = __builtin_fmaf(sc[j], p.scale_log2e, -l4[e]);
-        if (partial && !attn_visible(q0 + qi + e, key, gq[e], pq[e], gk)) x = -INFINITY;
-        const float pr = __builtin_amdgcn_exp2f(x);
+        const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j], p.scale_log2e, -l4[e]));
         pf[j / 8][j % 8] = (__bf16)pr;
         dsf[j / 8][j % 8] = (__bf16)(pr * (dp[j] - d4[e]));
       }
@@ -1230,7 +1253,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
 #pragma unroll
       for (int dt = 0; dt < D / 32; ++dt) {
         dv[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_at<D>(dot, bt, u, dt), pf[u], dv[dt], 0, 0, 0);
-        dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_at<D>(smem, bt, u, dt), dsf[u], dk[dt], 0, 0, 0);
+        dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_at<D>(st, bt, u, dt), dsf[u], dk[dt], 0, 0, 0);
       }
     }
   }
