@@ -10,24 +10,26 @@
 // the attention kernels walk only the visible blocks and evaluate the rule per
 // element only in the partly visible ones.
 //
-// Forward work-group: 128 queries x one head, 4 wavefronts of 32 queries, key
-// tiles of 64, two work-groups per CU (three at a head dimension of 64).  Scores
+// Forward work-group: 128 queries x one head, 4 wavefronts of 32 queries, three
+// work-groups per CU.  Scores
 // are computed transposed (S^T = K Q^T, MFMA 32x32x16), so that a lane owns one
 // query: the row maximum and sum are in-lane reductions plus one exchange between
 // the two half-waves, the accumulator of S^T is already in the B-operand layout of
 // the second product O^T = V^T P^T, and the running rescale of O^T is a per-lane
 // scalar.  K and V tiles are brought into a 2-stage LDS ring by buffer_load ... lds.
-// Bound: MFMA plus the softmax's vector work, and for packed rows (lists of a few
-// tiles) the set-up of a work-group.  Two independent work-groups per CU hide the
-// one's set-up and store behind the other's tiles, and a list is made for 128
-// queries instead of 256.  Against one work-group of 8 waves per CU with three
-// stages, 16384 positions of 8 prompts of 137 + 4 x 461, 28 / 4 heads of 128:
-// forward 205 -> 154 us, dQ 279 -> 244 us, dK/dV 433 -> 297 us (and the second stage since).  On dense causal
-// rows, where every tile comes into LDS twice as often, forward + backward are
-// 15 % faster to 3 % slower (us, 8 waves / now):
-//   heads of 128, 28 / 4: 4096 positions 630 / 618, 8192 2248 / 2151, 16384 8268 / 8379
-//   16 / 2: 8192 1253 / 1284, 12288 2772 / 2731;  16 / 16: 8192 1232 / 1241
-//   heads of 64, 14 / 2: 2048 172 / 147, 8192 728 / 682, 16384 2671 / 2359
+// Bound: on long lists power (the clock falls to 1.7 GHz) with the MFMAs, the softmax's vector work and the LDS reads each
+// busy for more than half of the time; on packed rows (lists of a few tiles, a sixth of a work-group's time before its first
+// tile) latency.  Hence several independent work-groups of 4 waves per CU, one hiding the other's set-up and store, and
+// lists made for 128 queries.  Against one work-group of 8 waves per CU with three stages, two of 4 waves with tiles of 64
+// keys took 16384 positions of 8 prompts of 137 + 4 x 461, 28 / 4 heads of 128, from 205 to 154 us (dQ 279 -> 244, dK/dV
+// 433 -> 297); at up to 3 % more on dense rows of 16384 (16 / 2 heads of 128: 2772 -> 2895 us forward and backward at 12288).
+// Steps of 32 keys (AttnKeySteps) since, us before / after:
+//   forward, three work-groups per CU at a head dimension of 128 (64: three either way, tiles of 64 keys): the packed row
+//     157 / 136, the same with 16 / 2 heads 88 / 78, 8192 positions 80 / 70; dense 16384 1866 / 1840, 8192 with 16 / 2 heads
+//     270 / 268, 4096 127 / 129; a row of 2048 in two conversations 22 / 23
+//   backward with dK/dV's second stage: packed 563 / 522, 389 / 358, 329 / 302; dense 6735 / 6330, 1001 / 988, 468 / 461;
+//     heads of 64, 14 / 2: 16384 packed 190 / 168, 8192 dense 515 / 475; two conversations 86 / 83
+// A head dimension of 64 has too few MFMAs per key for steps of 32 in the forward (8192 dense: 138 -> 160 us).
 #include <stdlib.h>
 
 #include "common.hpp"
@@ -147,20 +149,20 @@ __device__ __forceinline__ bool attn_visible(int i, int j, int gi, int pi, int g
   return j <= i && (gj == gi || gj == pi);
 }
 
-// Visibility of one (owner block, tile) pair, per wavefront of the kernel that
-// will process it:
+// Visibility of one (owner block, tile) pair, by cells of 32 queries x 32 keys:
 //   bits 14-15  1 = some pairs visible, 2 = all
-//   bits 16-19  wave w has at least one visible pair in its part of the tile
-//   bits 24-27  every pair of wave w's part is visible (no per-element test needed)
+//   bits 16-23  cell c has at least one visible pair
+//   bits 24-31  every pair of cell c is visible (no per-element test needed)
 // 0 when nothing is visible.
-//   info  (forward, dQ): owner = 128 queries, tile = 64 keys, wave w (of 4) = queries 32w..32w+31.
-//   info2 (dK/dV):       owner = 64 keys, tile = 64 queries, wave w (of 4) = keys 32(w&1).. x
+//   info  (forward, dQ): owner = 128 queries, tile = 64 keys; wave w (of 4) = queries 32w..32w+31, its cells are
+//                        c = 2w (keys 0..31) and 2w + 1 (keys 32..63).
+//   info2 (dK/dV):       owner = 64 keys, tile = 64 queries; wave w (of 4) = cell w = keys 32(w&1).. x
 //                        queries 32(w>>1)..
 // One wavefront takes 128 queries x 64 keys = 8 cells of 32 x 32 and writes the entry of info and both
 // entries of info2.  A cell whose queries share their codes and whose keys share theirs is decided from
 // uni; only the others are evaluated pair by pair (64 lanes = 32 keys x 2 halves of the queries).
-__device__ __forceinline__ uint32_t attn_entry(uint32_t any, uint32_t all) {
-  return any ? ((all == 0xfu ? 2u : 1u) << 14) | (any << 16) | (all << 24) : 0u;
+__device__ __forceinline__ uint32_t attn_entry(uint32_t any, uint32_t all, uint32_t cells) {
+  return any ? ((all == cells ? 2u : 1u) << 14) | (any << 16) | (all << 24) : 0u;
 }
 // info_row: the query block's row of info.
 __device__ __forceinline__ void attn_classify_pair(const int* gc, const int* pc, const int2* uni, int nQb2, int owner, int kb, uint32_t* info_row, uint32_t* info2) {
@@ -188,15 +190,9 @@ __device__ __forceinline__ void attn_classify_pair(const int* gc, const int* pc,
     }
   }
   if (lane == 0) {
-    uint32_t a4 = 0, l4 = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      a4 |= (uint32_t)((any >> (2 * w) & 3u) != 0u) << w;
-      l4 |= (uint32_t)((all >> (2 * w) & 3u) == 3u) << w;
-    }
-    info_row[kb] = attn_entry(a4, l4);
-    info2[(int64_t)kb * nQb2 + 2 * owner] = attn_entry(any & 0xfu, all & 0xfu);
-    info2[(int64_t)kb * nQb2 + 2 * owner + 1] = attn_entry(any >> 4, all >> 4);
+    info_row[kb] = attn_entry(any, all, 0xffu);
+    info2[(int64_t)kb * nQb2 + 2 * owner] = attn_entry(any & 0xfu, all & 0xfu, 0xfu);
+    info2[(int64_t)kb * nQb2 + 2 * owner + 1] = attn_entry(any >> 4, all >> 4, 0xfu);
   }
 }
 __global__ __launch_bounds__(256) void attn_classify_kernel(const int* __restrict__ gc, const int* __restrict__ pc,
@@ -448,6 +444,13 @@ struct AttnTile {
     const int c = (lane % CHK) ^ swz(r);
     return (int)(r * stride * 2) + c * 16;
   }
+  // The same from three registers (row and chunk of instruction 0; the row's offset in the scalar offset of the
+  // instruction) instead of one per instruction: instructions begin a multiple of 4 (D = 64: 8) rows apart, so their
+  // swizzles differ by an XOR.
+  __device__ static __forceinline__ int row_of(int instr) { return instr * (64 / CHK); }
+  __device__ static __forceinline__ int lane_row(int lane, int64_t stride) { return lane / CHK * (int)(stride * 2); }
+  __device__ static __forceinline__ int lane_chunk(int lane) { return ((lane % CHK) ^ swz(lane / CHK)) << 4; }
+  __device__ static __forceinline__ int chunk_of(int chunk, int instr) { return chunk ^ (swz(row_of(instr)) << 4); }
   // row fragment: row `row`, d = 16 s + 8 h ..
   __device__ static __forceinline__ bf16x8 row_frag(const char* tile, int row, int s, int h) {
     return *(const bf16x8*)(tile + row * ROW + (((2 * s + h) ^ swz(row)) * 16));
@@ -472,25 +475,7 @@ struct TrLane {
   }
 };
 
-// Transposed fragment for the 16-row slab starting at row k0 and the 32 columns
-// starting at d0: lane (m, h) gets column d0 + m of rows k0 + 4h + {0..3} and
-// k0 + 8 + 4h + {0..3} -- the row order in which the accumulator of the score
-// tile, used as the other operand, holds a slab.
-template <int D>
-__device__ __forceinline__ bf16x8 tr_frag(const char* tile, const TrLane& t, int k0, int d0) {
-  using T = AttnTile<D>;
-  const int col = d0 + t.dcol;
-  const int r0 = k0 + t.row_off, r1 = r0 + 8;
-  const shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (lds_shortx4_ptr)(tile + r0 * T::ROW + (((col >> 3) ^ T::swz(r0)) * 16) + (col & 4) * 2));
-  const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (lds_shortx4_ptr)(tile + r1 * T::ROW + (((col >> 3) ^ T::swz(r1)) * 16) + (col & 4) * 2));
-  typedef __attribute__((__vector_size__(8 * sizeof(short)))) short shortx8;
-  const shortx8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-  return __builtin_bit_cast(bf16x8, v);
-}
-
-// The same reads from byte offsets that the caller prepares once.  A row is a power of two of bytes long, so the chunk
+// The reads of a tile, from byte offsets that the caller prepares once.  A row is a power of two of bytes long, so the chunk
 // of step s (row fragments) or of the 32 columns dt (transposed ones) can be XORed into the offset of chunk 0, and
 // rows 16 apart have the same swizzle.  One register per row instead of one per address: where those are short.
 template <int D>
@@ -500,6 +485,8 @@ __device__ __forceinline__ int frag_base(int row, int h) {
 __device__ __forceinline__ bf16x8 frag_at(const char* tile, int base, int s) {
   return *(const bf16x8*)(tile + (base ^ (s << 5)));
 }
+// Transposed fragment of a 16-row slab and 32 columns: lane (m, h) gets column m of rows 4h + {0..3} and
+// 8 + 4h + {0..3} -- the row order in which the accumulator of the score tile, used as the other operand, holds a slab.
 struct TrBase {
   int lo, hi;  // rows k0 + 4h + {0..3} and 8 below
 };
@@ -603,43 +590,106 @@ struct AttnFwdParams {
   float scale_log2e;
 };
 
-// LDS stage of the forward and dQ kernels: K tile, V tile, 64 key codes.
-template <int D>
-struct AttnKvStage {
+// The keys of a query block, KEYS at a time, in the forward and dQ kernels.  Step i is part i % STEPS of tile i / STEPS of
+// the list; steps that no wave sees are left out.  LDS stage of a step: its rows of K, of V and their codes.
+// KEYS = 32 takes half the LDS and a third fewer registers (so three work-groups of the forward fit a CU where two did), and
+// a wave computes 32 x 32 cells that it sees instead of 32 x 64: 13 % less on the packed row of the header, where 43 %
+// fewer elements are tested too.  It costs two barriers and two reductions of the maximum per 64 keys, so everything per
+// step is kept short: the offsets into LDS move with the stage, those of the DMA are precomputed, the next entry of the list
+// is read while the step is computed (without that: 1900 us instead of 1840 on the dense row).
+template <int D, int KT>
+struct AttnKeySteps {
   using T = AttnTile<D>;
-  static constexpr int V_OFF = T::BYTES;
-  static constexpr int CODE_OFF = 2 * T::BYTES;
+  static constexpr int KEYS = 32 * KT;
+  static constexpr int STEPS = ATT_BN / KEYS;           // of a tile of the list
+  static constexpr int V_OFF = KEYS * T::ROW;
+  static constexpr int CODE_OFF = 2 * V_OFF;
   static constexpr int STAGE = CODE_OFF + 1024;
+  static constexpr int DMAS = V_OFF / 4096;             // per operand and wave
+  static constexpr int LIST_OFF = ATT_STAGES * STAGE;
+  static constexpr int LDS = LIST_OFF + ATT_MAX_KB * 4 + 8;
+  dma_rsrc_t rsrc_k, rsrc_v, rsrc_c;
+  int voff_k[DMAS], voff_v[DMAS];
+  int64_t k_ss, v_ss;
+  int cur, nxt, n;           // this step, the next, their number
+  uint32_t entry, e_nxt;     // and their tiles' entries
+
+  __device__ static __forceinline__ bool seen(uint32_t e, int half) { return STEPS == 1 || (e >> (16 + half) & 0x55u) != 0; }
+  __device__ static __forceinline__ int key(uint32_t e, int i) {
+    return (int)(e & 0x3fff) * ATT_BN + (STEPS == 2 ? 32 * (i & 1) : 0);
+  }
+  __device__ __forceinline__ int key() const { return key(entry, cur); }
+  // Cells of `wave` in this step: bit kt of any: its 32 queries see part of keys 32 kt ..; of mixed: but not all of them.
+  __device__ __forceinline__ int any(int wave) const { return entry >> (16 + 2 * wave + (STEPS == 2 ? cur & 1 : 0)) & (2 * KT - 1); }
+  __device__ __forceinline__ int mixed(int wave) const { return ~entry >> (24 + 2 * wave + (STEPS == 2 ? cur & 1 : 0)) & (2 * KT - 1); }
+  // From the next step on; e1: the entry behind its tile's.
+  __device__ __forceinline__ void advance(uint32_t e1) {
+    if (STEPS == 2) {
+      const bool same = !(nxt & 1) && seen(e_nxt, 1);
+      nxt = same ? nxt + 1 : (nxt | 1) + (seen(e1, 0) ? 1 : 2);
+      e_nxt = same ? e_nxt : e1;
+    } else {
+      ++nxt;
+      e_nxt = e1;
+    }
+  }
+  // DMA of the keys from k0 on into the stage at st: this wave's share of the rows, and the codes (every wave writes the
+  // same bytes).
+  __device__ __forceinline__ void issue(char* st, int k0, int wave, int lane) const {
+    const int so_k = (int)(k0 * k_ss * 2), so_v = (int)(k0 * v_ss * 2);
+#pragma unroll
+    for (int i = 0; i < DMAS; ++i) {
+      dma_load16(rsrc_k, voff_k[i], so_k, lds_addr_of(st + (wave * DMAS + i) * 1024));
+      dma_load16(rsrc_v, voff_v[i], so_v, lds_addr_of(st + V_OFF + (wave * DMAS + i) * 1024));
+    }
+    dma_load4(rsrc_c, (lane & (KEYS - 1)) * 4, k0 * 4, lds_addr_of(st + CODE_OFF));
+  }
+  // The first two steps are on their way before anything else is read.  (A row of the plan has four entries or more.)
+  __device__ __forceinline__ void begin(char* smem, const uint16_t* k_head, int64_t k_stride, const uint16_t* v_head,
+                                        int64_t v_stride, int S, const int* codes, const uint32_t* list, int tiles, int wave,
+                                        int lane) {
+    rsrc_k = attn_head_rsrc<D>(k_head, k_stride, S);
+    rsrc_v = attn_head_rsrc<D>(v_head, v_stride, S);
+    rsrc_c = attn_rsrc(codes);
+    k_ss = k_stride;
+    v_ss = v_stride;
+#pragma unroll
+    for (int i = 0; i < DMAS; ++i) {
+      voff_k[i] = T::voff(wave * DMAS + i, lane, k_ss);
+      voff_v[i] = T::voff(wave * DMAS + i, lane, v_ss);
+    }
+    n = STEPS * tiles;
+    cur = nxt = 0;
+    entry = e_nxt = 0;
+    if (tiles > 0) {
+      entry = e_nxt = __builtin_amdgcn_readfirstlane(list[0]);
+      const uint32_t e1 = __builtin_amdgcn_readfirstlane(list[1]);
+      cur = nxt = seen(entry, 0) ? 0 : 1;
+      issue(smem, key(), wave, lane);
+      advance(e1);
+      if (nxt < n) issue(smem + STAGE, key(e_nxt, nxt), wave, lane);
+    }
+    for (int i = threadIdx.x; i < tiles; i += ATT_THREADS) ((uint32_t*)(smem + LIST_OFF))[i] = list[i];
+  }
+  // The entry that end() needs, read while the step is computed (past the end of the list: not used).
+  __device__ __forceinline__ uint32_t ahead(const char* smem) const { return ((const uint32_t*)(smem + LIST_OFF))[nxt / STEPS + 1]; }
+  // End of the step in `stage`.
+  __device__ __forceinline__ void end(char* smem, int stage, uint32_t e1, int wave, int lane) {
+    cur = nxt;
+    entry = e_nxt;
+    advance(__builtin_amdgcn_readfirstlane(e1));
+    wait_vmcnt<0>();
+    barrier_lds_only();  // the next step is there, and every wave is done with this one
+    if (nxt < n) issue(smem + stage * STAGE, key(e_nxt, nxt), wave, lane);
+  }
 };
 
-// DMA of key block kb into one stage: this wave's share of the K and V tiles,
-// plus the 64 key codes (every wave writes the same 256 bytes).
 template <int D>
-__device__ __forceinline__ void attn_issue_kv(char* st, int kb, dma_rsrc_t rsrc_k,
-                                              dma_rsrc_t rsrc_v,
-                                              dma_rsrc_t rsrc_c,
-                                              const int* voff_k,
-                                              const int* voff_v, int64_t k_ss,
-                                              int64_t v_ss, int wave, int lane) {
+__global__ __launch_bounds__(ATT_THREADS, 3) void attn_fwd_kernel(AttnFwdParams p) {
   using T = AttnTile<D>;
-  using G = AttnKvStage<D>;
-  const int k0 = kb * ATT_BN;
-#pragma unroll
-  for (int i = 0; i < T::N4; ++i)
-    dma_load16(rsrc_k, voff_k[i], (int)(k0 * k_ss * 2), lds_addr_of(st + (wave * T::N4 + i) * 1024));
-#pragma unroll
-  for (int i = 0; i < T::N4; ++i)
-    dma_load16(rsrc_v, voff_v[i], (int)(k0 * v_ss * 2), lds_addr_of(st + G::V_OFF + (wave * T::N4 + i) * 1024));
-  dma_load4(rsrc_c, lane * 4, k0 * 4, lds_addr_of(st + G::CODE_OFF));
-}
-
-template <int D>
-__global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_fwd_kernel(AttnFwdParams p) {
-  using T = AttnTile<D>;
-  using G = AttnKvStage<D>;
-  // one LDS object for the stages and the tile list (see attn_smem_note)
-  __shared__ __attribute__((aligned(1024))) char smem[ATT_STAGES * G::STAGE + ATT_MAX_KB * 4];
-  uint32_t* const s_list = (uint32_t*)(smem + ATT_STAGES * G::STAGE);
+  constexpr int KT = D == 64 ? 2 : 1;
+  using G = AttnKeySteps<D, KT>;
+  __shared__ __attribute__((aligned(1024))) char smem[G::LDS];  // one LDS object (see attn_smem_note)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5;
   const TrLane tr(lane);
@@ -651,23 +701,9 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_fwd_kernel(
   const int qc = q < p.S ? q : p.S - 1;  // queries past the end compute something that is not stored
   const int* const gc = attn_row(p.gc, p.plan_stride, row);
   const uint32_t* const list = attn_row(p.list, p.plan_stride, row) + (int64_t)qb * p.nKb;
-  const int cnt = attn_row(p.cnt, p.plan_stride, row)[qb];
-
-  const dma_rsrc_t rsrc_k = attn_head_rsrc<D>(p.K + row * p.k_bs + (int64_t)hkv * p.k_hs, p.k_ss, p.S);
-  const dma_rsrc_t rsrc_v = attn_head_rsrc<D>(p.V + row * p.v_bs + (int64_t)hkv * p.v_hs, p.v_ss, p.S);
-  const dma_rsrc_t rsrc_c = attn_rsrc(gc);
-  int voff_k[T::N4], voff_v[T::N4];
-#pragma unroll
-  for (int i = 0; i < T::N4; ++i) {
-    voff_k[i] = T::voff(wave * T::N4 + i, lane, p.k_ss);
-    voff_v[i] = T::voff(wave * T::N4 + i, lane, p.v_ss);
-  }
-#define ATTN_ISSUE(ENTRY, STG)                                                                        \
-  attn_issue_kv<D>(smem + (STG) * G::STAGE, __builtin_amdgcn_readfirstlane((ENTRY) & 0x3fff), rsrc_k,  \
-                   rsrc_v, rsrc_c, voff_k, voff_v, p.k_ss, p.v_ss, wave, lane)
-  // the first tile is on its way before anything else is read
-  if (cnt > 0) ATTN_ISSUE(list[0], 0);
-  for (int i = threadIdx.x; i < cnt; i += ATT_THREADS) s_list[i] = list[i];
+  G ks;
+  ks.begin(smem, p.K + row * p.k_bs + (int64_t)hkv * p.k_hs, p.k_ss, p.V + row * p.v_bs + (int64_t)hkv * p.v_hs, p.v_ss, p.S,
+           gc, list, attn_row(p.cnt, p.plan_stride, row)[qb], wave, lane);
 
   // this lane's query as B-operand fragments of S^T = K Q^T
   bf16x8 qf[D / 16];
@@ -689,109 +725,116 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_fwd_kernel(
   for (int s = 0; s < D / 16; ++s) pin_loaded(qf[s]);
   pin_loaded(gi);
   pin_loaded(pi);
-  for (int it = 0; it < cnt; ++it) {
-    wait_vmcnt<0>();
-    barrier_lds_only();
-    if (it + 1 < cnt) ATTN_ISSUE(s_list[it + 1], (it + 1) & 1);
-    const int entry = __builtin_amdgcn_readfirstlane(s_list[it]);
-    const int kb = entry & 0x3fff;
-    const bool active = (entry >> (16 + wave)) & 1;        // this wave's 32 queries see part of the tile
-    const bool partial = !((entry >> (24 + wave)) & 1);     // ... but not all of it
-    const char* st = smem + (it & 1) * G::STAGE;
-    if (!active) continue;  // nothing of this tile is visible to this wave's queries
-
-    // S^T tiles: keys 0..31 and 32..63 of the block x this wave's 32 queries
-    floatx16 sc[2];
+  int bk = frag_base<D>(n, h);     // of the stage at hand
+  TrBase bt = tr_base<D>(tr, 0);
+  bt.lo += G::V_OFF;
+  bt.hi += G::V_OFF;
+  int stage = 0;
+  wait_vmcnt<0>();
+  barrier_lds_only();
+  while (ks.cur < ks.n) {
+    const uint32_t ahead = ks.ahead(smem);
+    const int key0 = ks.key(), active = ks.any(wave), partial = ks.mixed(wave);
+    pin_loaded(bk);  // (or what follows from them is kept in registers of its own)
+    pin_loaded(bt.lo);
+    pin_loaded(bt.hi);
+    if (active) {
+      // S^T tiles: 32 keys each x this wave's 32 queries
+      floatx16 sc[KT];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) sc[0][j] = sc[1][j] = 0.f;
-    {
-      // K fragments three steps ahead of the MFMAs that use them (LDS latency)
-      constexpr int NS = D / 16, PF = 3;
-      bf16x8 kf[NS][2];
+      for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-      for (int s = 0; s < PF; ++s) {
-        kf[s][0] = T::row_frag(st, n, s, h);
-        kf[s][1] = T::row_frag(st, 32 + n, s, h);
-      }
-      __builtin_amdgcn_sched_group_barrier(0x100, 2 * PF, 0);
+        for (int j = 0; j < 16; ++j) sc[kt][j] = 0.f;
+      {
+        // K fragments PF steps ahead of the MFMAs that use them (LDS latency)
+        constexpr int NS = D / 16, PF = KT == 1 ? 4 : 3;
+        bf16x8 kf[NS][KT];
 #pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        if (s + PF < NS) {
-          kf[s + PF][0] = T::row_frag(st, n, s + PF, h);
-          kf[s + PF][1] = T::row_frag(st, 32 + n, s + PF, h);
+        for (int s = 0; s < PF; ++s)
+#pragma unroll
+          for (int kt = 0; kt < KT; ++kt) kf[s][kt] = frag_at(smem + 32 * kt * T::ROW, bk, s);
+        __builtin_amdgcn_sched_group_barrier(0x100, KT * PF, 0);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          if (s + PF < NS)
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) kf[s + PF][kt] = frag_at(smem + 32 * kt * T::ROW, bk, s + PF);
+#pragma unroll
+          for (int kt = 0; kt < KT; ++kt)
+            sc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s][kt], qf[s], sc[kt], 0, 0, 0);
+          if (s + PF < NS) __builtin_amdgcn_sched_group_barrier(0x100, KT, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, KT, 0);
         }
-        sc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s][0], qf[s], sc[0], 0, 0, 0);
-        sc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s][1], qf[s], sc[1], 0, 0, 0);
-        if (s + PF < NS) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
       }
-    }
 
-    // mask, running max (of the raw scores: the scale is positive and rides in the exponent's
-    // multiply-add below)
-    float mloc = -INFINITY;
-    if (partial) {
-      const int* codes = (const int*)(st + G::CODE_OFF);
+      // mask, running max (of the raw scores: the scale is positive and rides in the exponent's
+      // multiply-add below)
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+      for (int kt = 0; kt < KT; ++kt)
+        if (partial >> kt & 1) {
+          const int* codes = (const int*)(smem + stage * G::STAGE + G::CODE_OFF);
 #pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          const int kk = 32 * kt + 8 * g4 + 4 * h;
-          const int4 kc = *(const int4*)(codes + kk);
-          const int key = kb * ATT_BN + kk;
-          const int kcv[4] = {kc.x, kc.y, kc.z, kc.w};
+          for (int g4 = 0; g4 < 4; ++g4) {
+            const int kk = 32 * kt + 8 * g4 + 4 * h;
+            const int4 kc = *(const int4*)(codes + kk);
+            const int key = key0 + kk;
+            const int kcv[4] = {kc.x, kc.y, kc.z, kc.w};
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (!attn_visible(q, key + e, gi, pi, kcv[e])) sc[kt][4 * g4 + e] = -INFINITY;
+            for (int e = 0; e < 4; ++e)
+              if (!attn_visible(q, key + e, gi, pi, kcv[e])) sc[kt][4 * g4 + e] = -INFINITY;
+          }
         }
-    }
+      float mloc = -INFINITY;
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+      for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-      for (int j = 0; j < 16; ++j) mloc = fmaxf(mloc, sc[kt][j]);
-    {
-      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mloc), __float_as_uint(mloc), false, false);
-      mloc = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * p.scale_log2e;  // both halves of a query
-    }
-    // The reference of the exponentials follows the running maximum lazily: it moves only when
-    // some query of the wave has a score more than ATT_LAZY (in units of log2) above it, so the
-    // 64 output accumulators are rescaled on few tiles instead of on most early ones.  Until
-    // then exponentials are at most 2^ATT_LAZY, which fp32 sums and bf16 operands hold without
-    // loss; the final division by the sum is the same.
-    const bool move = __any(mloc > m_run + ATT_LAZY);
-    float lsum = 0.f;
-    bf16x8 pf[4];
-    if (move) {
-      const float m_new = fmaxf(m_run, mloc);
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-      m_run = m_new;
-      l_run *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) o[dt][j] *= alpha;
-    }
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kt][j], p.scale_log2e, -m_run));
-        lsum += e;
-        pf[2 * kt + j / 8][j % 8] = (__bf16)e;
+        for (int j = 0; j < 16; ++j) mloc = fmaxf(mloc, sc[kt][j]);
+      {
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mloc), __float_as_uint(mloc), false, false);
+        mloc = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * p.scale_log2e;  // both halves of a query
       }
-    l_run += lsum;
+      // The reference of the exponentials follows the running maximum lazily: it moves only when
+      // some query of the wave has a score more than ATT_LAZY (in units of log2) above it, so the
+      // 64 output accumulators are rescaled on few tiles instead of on most early ones.  Until
+      // then exponentials are at most 2^ATT_LAZY, which fp32 sums and bf16 operands hold without
+      // loss; the final division by the sum is the same.
+      if (__any(mloc > m_run + ATT_LAZY)) {
+        const float m_new = fmaxf(m_run, mloc);
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        m_run = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+          for (int j = 0; j < 16; ++j) o[dt][j] *= alpha;
+      }
+      float lsum = 0.f;
+      bf16x8 pf[2 * KT];
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kt][j], p.scale_log2e, -m_run));
+          lsum += e;
+          pf[2 * kt + j / 8][j % 8] = (__bf16)e;
+        }
+      l_run += lsum;
 
-    // O^T += V^T P^T, V^T fragments by transposing reads of the V tile
-    const char* vt = st + G::V_OFF;
+      // O^T += V^T P^T, V^T fragments by transposing reads of the V tile
 #pragma unroll
-    for (int s2 = 0; s2 < 4; ++s2) {
+      for (int s2 = 0; s2 < 2 * KT; ++s2) {
 #pragma unroll
-      for (int dt = 0; dt < D / 32; ++dt)
-        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag<D>(vt, tr, 16 * s2, 32 * dt), pf[s2], o[dt],
-                                                        0, 0, 0);
+        for (int dt = 0; dt < D / 32; ++dt)
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_at<D>(smem, bt, s2, dt), pf[s2], o[dt], 0, 0, 0);
+      }
     }
+    const int step = stage ? -G::STAGE : G::STAGE;
+    bk += step;
+    bt.lo += step;
+    bt.hi += step;
+    ks.end(smem, stage, ahead, wave, lane);
+    stage ^= 1;
   }
-#undef ATTN_ISSUE
 
   const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
@@ -882,10 +925,9 @@ struct AttnBwdParams {
 template <int D>
 __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kernel(AttnBwdParams p) {
   using T = AttnTile<D>;
-  using G = AttnKvStage<D>;
-  // one LDS object for the stages and the tile list (see attn_smem_note)
-  __shared__ __attribute__((aligned(1024))) char smem[ATT_STAGES * G::STAGE + ATT_MAX_KB * 4];
-  uint32_t* const s_list = (uint32_t*)(smem + ATT_STAGES * G::STAGE);
+  constexpr int KT = 1;
+  using G = AttnKeySteps<D, KT>;
+  __shared__ __attribute__((aligned(1024))) char smem[G::LDS];  // one LDS object (see attn_smem_note)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5;
   const TrLane tr(lane);
@@ -897,22 +939,9 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kern
   const int qc = q < p.S ? q : p.S - 1;  // queries past the end compute something that is not stored
   const int* const gc = attn_row(p.gc, p.plan_stride, row);
   const uint32_t* const list = attn_row(p.list, p.plan_stride, row) + (int64_t)qb * p.nKb;
-  const int cnt = attn_row(p.cnt, p.plan_stride, row)[qb];
-
-  const dma_rsrc_t rsrc_k = attn_head_rsrc<D>(p.K + row * p.k_bs + (int64_t)hkv * p.k_hs, p.k_ss, p.S);
-  const dma_rsrc_t rsrc_v = attn_head_rsrc<D>(p.V + row * p.v_bs + (int64_t)hkv * p.v_hs, p.v_ss, p.S);
-  const dma_rsrc_t rsrc_c = attn_rsrc(gc);
-  int voff_k[T::N4], voff_v[T::N4];
-#pragma unroll
-  for (int i = 0; i < T::N4; ++i) {
-    voff_k[i] = T::voff(wave * T::N4 + i, lane, p.k_ss);
-    voff_v[i] = T::voff(wave * T::N4 + i, lane, p.v_ss);
-  }
-#define ATTN_ISSUE(ENTRY, STG)                                                                        \
-  attn_issue_kv<D>(smem + (STG) * G::STAGE, __builtin_amdgcn_readfirstlane((ENTRY) & 0x3fff), rsrc_k,  \
-                   rsrc_v, rsrc_c, voff_k, voff_v, p.k_ss, p.v_ss, wave, lane)
-  if (cnt > 0) ATTN_ISSUE(list[0], 0);
-  for (int i = threadIdx.x; i < cnt; i += ATT_THREADS) s_list[i] = list[i];
+  G ks;
+  ks.begin(smem, p.K + row * p.k_bs + (int64_t)hkv * p.k_hs, p.k_ss, p.V + row * p.v_bs + (int64_t)hkv * p.v_hs, p.v_ss, p.S,
+           gc, list, attn_row(p.cnt, p.plan_stride, row)[qb], wave, lane);
 
   bf16x8 qf[D / 16], dof[D / 16];
   float delta = 0.f;
@@ -955,57 +984,63 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kern
   pin_loaded(pi);
   pin_loaded(nlse2);
   pin_loaded(delta);
-  for (int it = 0; it < cnt; ++it) {
-    wait_vmcnt<0>();
-    barrier_lds_only();
-    if (it + 1 < cnt) ATTN_ISSUE(s_list[it + 1], (it + 1) & 1);
-    const int entry = __builtin_amdgcn_readfirstlane(s_list[it]);
-    const int kb = entry & 0x3fff;
-    const bool active = (entry >> (16 + wave)) & 1;        // this wave's 32 queries see part of the tile
-    const bool partial = !((entry >> (24 + wave)) & 1);     // ... but not all of it
-    const char* st = smem + (it & 1) * G::STAGE;
-    const int* codes = (const int*)(st + G::CODE_OFF);
-    if (!active) continue;
-
-    bf16x8 dsf[4];
+  int bk = frag_base<D>(n, h);     // of the stage at hand
+  TrBase bt = tr_base<D>(tr, 0);
+  int stage = 0;
+  wait_vmcnt<0>();
+  barrier_lds_only();
+  while (ks.cur < ks.n) {
+    const uint32_t ahead = ks.ahead(smem);
+    const int key0 = ks.key(), active = ks.any(wave), partial = ks.mixed(wave);
+    const int* codes = (const int*)(smem + stage * G::STAGE + G::CODE_OFF);
+    pin_loaded(bk);  // (or what follows from them is kept in registers of its own)
+    pin_loaded(bt.lo);
+    pin_loaded(bt.hi);
+    if (active) {
+      bf16x8 dsf[2 * KT];
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      floatx16 sc, dp;
+      for (int kt = 0; kt < KT; ++kt) {
+        const char* const kh = smem + kt * 32 * T::ROW;
+        floatx16 sc, dp;
 #pragma unroll
-      for (int j = 0; j < 16; ++j) sc[j] = dp[j] = 0.f;
+        for (int j = 0; j < 16; ++j) sc[j] = dp[j] = 0.f;
 #pragma unroll
-      for (int s = 0; s < D / 16; ++s) {
-        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(T::row_frag(st, 32 * kt + n, s, h), qf[s], sc, 0, 0, 0);
-        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(T::row_frag(st + G::V_OFF, 32 * kt + n, s, h), dof[s],
-                                                     dp, 0, 0, 0);
-      }
-      if (partial) {  // one branch for all elements: tested inside the loop below it becomes one per element
+        for (int s = 0; s < D / 16; ++s) {
+          sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_at(kh, bk, s), qf[s], sc, 0, 0, 0);
+          dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_at(kh + G::V_OFF, bk, s), dof[s], dp, 0, 0, 0);
+        }
+        if (partial >> kt & 1) {  // one branch for all elements: tested inside the loop below it becomes one per element
 #pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          const int kk = 32 * kt + 8 * g4 + 4 * h;
-          const int4 kc = *(const int4*)(codes + kk);
-          const int kcv[4] = {kc.x, kc.y, kc.z, kc.w};
+          for (int g4 = 0; g4 < 4; ++g4) {
+            const int kk = 32 * kt + 8 * g4 + 4 * h;
+            const int4 kc = *(const int4*)(codes + kk);
+            const int kcv[4] = {kc.x, kc.y, kc.z, kc.w};
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (!attn_visible(q, kb * ATT_BN + kk + e, gi, pi, kcv[e])) sc[4 * g4 + e] = -INFINITY;
+            for (int e = 0; e < 4; ++e)
+              if (!attn_visible(q, key0 + kk + e, gi, pi, kcv[e])) sc[4 * g4 + e] = -INFINITY;
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j], p.scale_log2e, nlse2));
+          dsf[2 * kt + j / 8][j % 8] = (__bf16)(pr * (dp[j] - delta));
         }
       }
+      // dQ^T += K^T dS^T, K^T fragments by transposing reads of the K tile
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j], p.scale_log2e, nlse2));
-        dsf[2 * kt + j / 8][j % 8] = (__bf16)(pr * (dp[j] - delta));
+      for (int s2 = 0; s2 < 2 * KT; ++s2) {
+#pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt)
+          dq[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_at<D>(smem, bt, s2, dt), dsf[s2], dq[dt], 0, 0, 0);
       }
     }
-    // dQ^T += K^T dS^T, K^T fragments by transposing reads of the K tile
-#pragma unroll
-    for (int s2 = 0; s2 < 4; ++s2) {
-#pragma unroll
-      for (int dt = 0; dt < D / 32; ++dt)
-        dq[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag<D>(st, tr, 16 * s2, 32 * dt), dsf[s2], dq[dt],
-                                                         0, 0, 0);
-    }
+    const int step = stage ? -G::STAGE : G::STAGE;
+    bk += step;
+    bt.lo += step;
+    bt.hi += step;
+    ks.end(smem, stage, ahead, wave, lane);
+    stage ^= 1;
   }
-#undef ATTN_ISSUE
   if (q >= p.S) return;
   uint16_t* op = p.dQ + row * p.dq_bs + (int64_t)q * p.dq_ss + (int64_t)hq * p.dq_hs;
 #pragma unroll
@@ -1026,8 +1061,8 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kern
 // its own.  The registers for that come from one per fragment row instead of one per address, and from P before dP (half
 // the fragments in flight).  One stage, V rows all in LDS / now, backward in us: dense causal rows of 16384 positions,
 // 28 / 4 heads of 128: 6640 / 6280; 8192, 16 / 2: 1000 / 976; 8192, 14 / 2 heads of 64: 518 / 465; the row of the header's
-// figures 570 / 525 (20 us of it, and of the short rows' 85 / 81, is the mask as one branch per step, here and in dQ, instead
-// of one per element).
+// figures 570 / 525 (dQ and both masks as one branch per step instead of one per element included).  Offsets that move with
+// the stage instead of a sum per read: 6400 -> 6330 on the dense row.
 // A work-group that does not take all heads of its group writes fp32 partial sums, which
 // attn_kv_reduce_kernel adds in a fixed order.
 // LDS: two stages of a Q tile, a dO tile (64 queries) and lse2 / delta / group / parent codes of those queries; then
@@ -1047,9 +1082,7 @@ struct AttnQStage {
 
 // DMA of one query tile into a stage: this wave's share of the Q and dO tiles and
 // one of the four per-query arrays (wave 0: lse2, 1: delta, 2: group codes, 3: parent codes).
-// row_q, row_do, chunk: byte offset of this lane's row and chunk in instruction 0 (AttnTile::voff).  The instructions of a
-// wave begin a multiple of 4 (D = 64: 8) rows apart, so their swizzles differ by an XOR: three registers for both tiles
-// instead of one per instruction.
+// row_q, row_do, chunk: this lane's row and chunk in instruction 0, in bytes (AttnTile::row_of).
 template <int D>
 __device__ __forceinline__ void attn_issue_q(char* st, int hq, int q0, const uint16_t* q_row, const uint16_t* do_row,
                                              dma_rsrc_t rsrc_row, int row_q, int row_do, int chunk, const AttnBwdParams& p, int wave,
@@ -1060,8 +1093,7 @@ __device__ __forceinline__ void attn_issue_q(char* st, int hq, int q0, const uin
   const dma_rsrc_t rsrc_do = attn_head_rsrc<D>(do_row + hq * p.do_hs, p.do_ss, p.S);
 #pragma unroll
   for (int i = 0; i < T::N4; ++i) {
-    const int r = (wave * T::N4 + i) * (64 / T::CHK);   // first row of the instruction
-    const int c = chunk ^ (T::swz(r) << 4);
+    const int r = T::row_of(wave * T::N4 + i), c = T::chunk_of(chunk, wave * T::N4 + i);
     dma_load16(rsrc_q, row_q + c, (int)((q0 + r) * p.q_ss * 2), lds_addr_of(st + (wave * T::N4 + i) * 1024));
     dma_load16(rsrc_do, row_do + c, (int)((q0 + r) * p.do_ss * 2), lds_addr_of(st + G::DO_OFF + (wave * T::N4 + i) * 1024));
   }
@@ -1113,8 +1145,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
   const void* row_src = arr == 0 ? (const void*)(p.lse2 + stat_row) : arr == 1 ? (const void*)(p.delta + stat_row)
                         : arr == 2 ? (const void*)gc : (const void*)attn_row(p.pc, p.plan_stride, brow);
   const dma_rsrc_t rsrc_row = attn_rsrc(row_src);
-  int row_q = lane / T::CHK * (int)(p.q_ss * 2), row_do = lane / T::CHK * (int)(p.do_ss * 2);
-  int chunk = ((lane % T::CHK) ^ T::swz(lane / T::CHK)) << 4;
+  int row_q = T::lane_row(lane, p.q_ss), row_do = T::lane_row(lane, p.do_ss), chunk = T::lane_chunk(lane);
   {
     const uint16_t* const k_head = p.K + brow * p.k_bs + (int64_t)hkv * p.k_hs;
     const uint16_t* const v_head = p.V + brow * p.v_bs + (int64_t)hkv * p.v_hs;
@@ -1151,8 +1182,15 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
   for (int s = 0; s < G::VR; ++s) pin_loaded(vr[s]);
   int bq = frag_base<D>(32 * qh + n, h), bv = frag_base<64>(krow, h);
   TrBase bt = tr_base<D>(tr, 32 * qh);
+  bq += G::STAGE;
+  bt.lo += G::STAGE;
+  bt.hi += G::STAGE;
   int ti = 0, head = hq;
   for (int it = 0; it < total; ++it) {
+    const int step = it & 1 ? G::STAGE : -G::STAGE;
+    bq += step;
+    bt.lo += step;
+    bt.hi += step;
     wait_vmcnt<0>();
     barrier_lds_only();  // this tile is there, and every wave is done with the one before (it = 0: with the K and V rows)
     const int entry = __builtin_amdgcn_readfirstlane(s_list[ti]);
@@ -1170,7 +1208,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
     const int q0 = (entry & 0x3fff) * ATT_BQ2;
     const bool active = (entry >> (16 + wave)) & 1;        // this wave's keys x query half
     const bool partial = !((entry >> (24 + wave)) & 1);
-    const char* dot = st + G::DO_OFF;
+    const char* dot = smem + G::DO_OFF;  // (bq and bt move with the stage)
     const float* r_lse2 = (const float*)(st + G::ROW_OFF);
     const float* r_delta = r_lse2 + 64;
     const int* r_gc = (const int*)(r_lse2 + 128);
@@ -1190,11 +1228,11 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
       constexpr int PF = 3;
       bf16x8 qf[NS];
 #pragma unroll
-      for (int s = 0; s < PF; ++s) qf[s] = frag_at(st, bq, s);
+      for (int s = 0; s < PF; ++s) qf[s] = frag_at(smem, bq, s);
       __builtin_amdgcn_sched_group_barrier(0x100, PF, 0);
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
-        if (s + PF < NS) qf[s + PF] = frag_at(st, bq, s + PF);
+        if (s + PF < NS) qf[s + PF] = frag_at(smem, bq, s + PF);
         sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[s], kf[s], sc, 0, 0, 0);
         if (s + PF < NS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -1253,7 +1291,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
 #pragma unroll
       for (int dt = 0; dt < D / 32; ++dt) {
         dv[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_at<D>(dot, bt, u, dt), pf[u], dv[dt], 0, 0, 0);
-        dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_at<D>(st, bt, u, dt), dsf[u], dk[dt], 0, 0, 0);
+        dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_at<D>(smem, bt, u, dt), dsf[u], dk[dt], 0, 0, 0);
       }
     }
   }

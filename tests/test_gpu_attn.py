@@ -472,3 +472,24 @@ def test_plan_of_a_short_row_is_that_of_a_long_one(artk_lib, gpu, S, ids):
         assert n == int((b["heads"][:int(b["n_heads"])] < S).sum()) and torch.equal(a["heads"][:n], b["heads"][:n])
         whole = S // 32
         assert torch.equal(a["uni"][:whole], b["uni"][:whole])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("S", [31, 32, 33, 64, 96, 160, 480])
+def test_attn_steps_of_32_keys(artk_lib, gpu, S, D):
+    """Runs of 32 positions that belong to two groups by turns, and positions of the second that see the first one's: whole
+    halves of a 64-key tile are invisible to a work-group (first, last, alone in the list) or to some of its waves."""
+    from art_amd.attention import attention_plans, packed_attention
+    print("attention steps of 32 keys", S, D, flush=True)
+    Hq, Hkv = 4, 2
+    q, k, v = make_qkv(S + D, S, Hq, Hkv, D)
+    d_out = torch.randn(S, Hq, D, generator=torch.Generator().manual_seed(S)).to(torch.bfloat16)
+    run = torch.arange(S) // 32
+    for group, parent in ((run % 2, run % 2), (run % 2, (run % 3 == 2).long()), (run % 5, (run + 3) % 5), (run, run)):
+        ref_out, ref_dq, ref_dk, ref_dv = attn_oracle.attention_grads(q, k, v, group, parent, d_out)
+        plans = attention_plans(group.to(gpu), parent.to(gpu))
+        leaves = [t.to(gpu).requires_grad_(True) for t in (q, k, v)]
+        out = packed_attention(*leaves, plans)
+        got = [out.detach(), *torch.autograd.grad(out, leaves, d_out.to(gpu))]
+        for a, b in zip(got, (ref_out, ref_dq, ref_dk, ref_dv)):
+            assert rel_l2(a.float().cpu(), b) <= 1e-2
