@@ -86,6 +86,22 @@ __device__ __forceinline__ void unpack2(uint32_t w, float& lo, float& hi) {
   hi = __uint_as_float(w & 0xffff0000u);
 }
 
+// 8 x 8 bf16 in registers: out[c] = column c of in.
+__device__ __forceinline__ void transpose8x8(const uint4 (&in)[8], uint4 (&out)[8]) {
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    uint32_t o[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      auto word = [&](const uint4& v) { return c / 2 == 0 ? v.x : c / 2 == 1 ? v.y : c / 2 == 2 ? v.z : v.w; };
+      const uint32_t lo = (word(in[2 * k]) >> (16 * (c & 1))) & 0xffffu;
+      const uint32_t hi = (word(in[2 * k + 1]) >> (16 * (c & 1))) & 0xffffu;
+      o[k] = lo | (hi << 16);
+    }
+    out[c] = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+}
+
 // dst[c, r] = src[r, c] for n bf16 matrices [R, C] with R and C multiples of 8 (LoRA factors: one
 // dimension is the rank); blockIdx.y selects one of two jobs so that both transposes of a LoRA
 // backward share a launch.  A thread turns an 8 x 8 block in registers: eight 16-byte loads along
@@ -103,26 +119,12 @@ __device__ __forceinline__ void small_transpose_one(const SmallTranspose& t) {
   const int64_t rb = j / CB, cb = j - rb * CB;
   const uint16_t* src = t.src + m * t.R * t.C + rb * 8 * t.C + cb * 8;
   uint16_t* dst = t.dst + m * t.R * t.C + cb * 8 * t.R + rb * 8;
-  uint32_t in[8][4];  // in[r][k]: columns 2k, 2k + 1 of row r
+  uint4 in[8], out[8];
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    const uint4 v = *(const uint4*)(src + r * t.C);
-    in[r][0] = v.x;
-    in[r][1] = v.y;
-    in[r][2] = v.z;
-    in[r][3] = v.w;
-  }
+  for (int r = 0; r < 8; ++r) in[r] = *(const uint4*)(src + r * t.C);
+  transpose8x8(in, out);
 #pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    uint32_t o[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t lo = (in[2 * k][c >> 1] >> (16 * (c & 1))) & 0xffffu;
-      const uint32_t hi = (in[2 * k + 1][c >> 1] >> (16 * (c & 1))) & 0xffffu;
-      o[k] = lo | (hi << 16);
-    }
-    *(uint4*)(dst + c * t.R) = make_uint4(o[0], o[1], o[2], o[3]);
-  }
+  for (int c = 0; c < 8; ++c) *(uint4*)(dst + c * t.R) = out[c];
 }
 __global__ __launch_bounds__(256) static void small_transpose2_kernel(SmallTranspose a, SmallTranspose b) {
   small_transpose_one(blockIdx.y == 0 ? a : b);

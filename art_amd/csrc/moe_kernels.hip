@@ -20,18 +20,33 @@
 namespace artk {
 
 // ----------------------------------------------------------------------------
-// Routing: one wavefront per token.
+// Routing: one wavefront per token.  (The launch is moe_topk_pack_kernel.)
 // ----------------------------------------------------------------------------
 constexpr int MOE_NI = 2;  // 8 waves, 2 per SIMD (see gemm_nt.hpp)
 constexpr int MOE_MAX_E = 256;
 constexpr int MOE_MAX_K = 16;
 
-__global__ __launch_bounds__(256) void moe_topk_kernel(const float* __restrict__ logits, int64_t T,
-                                                       int E, int k, int* __restrict__ topk_idx,
-                                                       float* __restrict__ topk_w) {
+// Largest value of the wave, in every lane, by DPP (a shuffle goes through LDS and has its latency).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_max(float v) {
+  const int x = __float_as_int(v);  // (lanes without a source keep their own value)
+  return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(x, x, CTRL, ROWS, 0xf, false)));
+}
+__device__ __forceinline__ float wave_max_dpp(float v) {
+  v = dpp_max<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8: lane 15 of a row of 16 has the row's
+  v = dpp_max<0x112, 0xf>(v);
+  v = dpp_max<0x114, 0xf>(v);
+  v = dpp_max<0x118, 0xf>(v);
+  v = dpp_max<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v = dpp_max<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+// Token t of the routing, by one wave.  A round is a maximum over the experts that are left and a ballot for each 64 of them
+// (top-8 of 128 with an arg-max of shuffles: 8192 tokens 21 us, 203 tokens 9; now 12 and 5).
+__device__ __forceinline__ void moe_topk_token(const float* __restrict__ logits, int64_t t, int E, int k,
+                                               int* __restrict__ topk_idx, float* __restrict__ topk_w) {
   const int lane = threadIdx.x & 63;
-  const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= T) return;
   // NaN counts as -inf, so the order below is total: decreasing value, ties (also
   // among -inf) to the lower expert index; every round picks an index in [0, E).
   float x[4];
@@ -43,27 +58,21 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const float* __restrict__
     x[i] = v == v ? v : -INFINITY;
     if (e >= E) taken |= 1u << i;
   }
-  float m = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
-  m = wave_max(m);
+  float m = 0.f;
   float myp = 0.f;  // lane j keeps the probability mass of slot j
+  int mye = 0;      // ... and its expert
   float psum = 0.f;
   for (int j = 0; j < k; ++j) {
     float bv = -INFINITY;
-    int bi = 0x7fffffff;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (!(taken >> i & 1) && (bi == 0x7fffffff || x[i] > bv)) {
-        bv = x[i];
-        bi = lane + 64 * i;
-      }
+    for (int i = 0; i < 4; ++i) bv = fmaxf(bv, taken >> i & 1 ? -INFINITY : x[i]);
+    bv = wave_max_dpp(bv);
+    if (j == 0) m = bv;
+    int bi = -1;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int oi = __shfl_xor(bi, o, 64);
-      if (oi != 0x7fffffff && (bi == 0x7fffffff || ov > bv || (ov == bv && oi < bi))) {
-        bv = ov;
-        bi = oi;
-      }
+    for (int i = 0; i < 4; ++i) {
+      const unsigned long long at = __ballot(!(taken >> i & 1) && x[i] == bv);
+      if (bi < 0 && at != 0) bi = 64 * i + __builtin_ctzll(at);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -71,10 +80,15 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const float* __restrict__
     // exp(-inf - m) = 0; a row without any finite logit (m = -inf) has no mass at all
     const float pj = bv == -INFINITY ? 0.f : expf(bv - m);
     psum += pj;
-    if (lane == j) myp = pj;
-    if (lane == 0) topk_idx[t * k + j] = bi;
+    if (lane == j) {
+      myp = pj;
+      mye = bi;
+    }
   }
-  if (lane < k) topk_w[t * k + lane] = psum > 0.f ? myp / psum : 0.f;
+  if (lane < k) {
+    topk_idx[t * k + lane] = mye;
+    topk_w[t * k + lane] = psum > 0.f ? myp / psum : 0.f;
+  }
 }
 
 // ----------------------------------------------------------------------------
@@ -88,7 +102,7 @@ __global__ __launch_bounds__(PERM_CHUNK) void moe_hist_kernel(const int* __restr
   for (int i = threadIdx.x; i < E; i += PERM_CHUNK) hist[i] = 0;
   __syncthreads();
   const int f = blockIdx.x * PERM_CHUNK + threadIdx.x;
-  // keys come from moe_topk_kernel and lie in [0, E); anything else is ignored
+  // keys come from the top-k and lie in [0, E); anything else is ignored
   if (f < n && (unsigned)keys[f] < (unsigned)E) atomicAdd(&hist[keys[f]], 1);
   __syncthreads();
   for (int i = threadIdx.x; i < E; i += PERM_CHUNK) cnt[blockIdx.x * E + i] = hist[i];
@@ -116,37 +130,25 @@ __device__ __forceinline__ int moe_split_rows(const int* share, int n_rows) {
   }
   return 4 * 8 * most > 5 * all ? n_rows / 32 : 0x7fffffff;
 }
-__global__ __launch_bounds__(SCAN_PARTS * MOE_MAX_E) void moe_scan_kernel(const int* __restrict__ cnt, int nb, int E,
-                                                                          int* __restrict__ offsets,
-                                                                          int* __restrict__ base,
-                                                                          int* __restrict__ tile_prefix,
-                                                                          int* __restrict__ blk_prefix,
-                                                                          int* __restrict__ order) {
-  __shared__ int part[SCAN_PARTS][MOE_MAX_E];
-  __shared__ int wsum[3][MOE_MAX_E / 64];
-  __shared__ int off[MOE_MAX_E], rows[MOE_MAX_E], rank[MOE_MAX_E], share[8];
+struct MoeScanLds {
+  int part[SCAN_PARTS][MOE_MAX_E];  // rows of an expert in a quarter of the chunks
+  int wsum[3][MOE_MAX_E / 64];
+  int off[MOE_MAX_E], rows[MOE_MAX_E], rank[MOE_MAX_E], share[8];
+};
+struct MoeScanOut {
+  int *offsets, *tile_prefix, *blk_prefix, *order;
+};
+// The prefix sums over the experts, from l.part on (a barrier lies behind its last write); l.off and l.rows are there
+// when it returns.
+__device__ __forceinline__ void moe_scan_experts(MoeScanLds& l, int E, const MoeScanOut& o) {
   const int e = threadIdx.x % MOE_MAX_E, pt = threadIdx.x / MOE_MAX_E;
-  const int per = (nb + SCAN_PARTS - 1) / SCAN_PARTS;
-  const int b0 = pt * per, b1 = b0 + per < nb ? b0 + per : nb;
-  int s = 0;
-  if (e < E) {
-    for (int b = b0; b < b1; b += 8) {
-      int v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = b + u < b1 ? cnt[(b + u) * E + e] : 0;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) s += v[u];
-    }
-  }
-  part[pt][e] = s;
-  __syncthreads();
   // exclusive prefix sums over the experts (threads of part 0: one expert each)
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int tot = 0, run = 0, tp = 0, bp = 0;
   if (pt == 0) {
     if (e < E)
 #pragma unroll
-      for (int q = 0; q < SCAN_PARTS; ++q) tot += part[q][e];
+      for (int q = 0; q < SCAN_PARTS; ++q) tot += l.part[q][e];
     run = tot;
     tp = (tot + TILE - 1) / TILE;
     bp = (tot + 15) / 16;
@@ -160,38 +162,78 @@ __global__ __launch_bounds__(SCAN_PARTS * MOE_MAX_E) void moe_scan_kernel(const 
       }
     }
     if (lane == 63) {
-      wsum[0][wave] = run;
-      wsum[1][wave] = tp;
-      wsum[2][wave] = bp;
+      l.wsum[0][wave] = run;
+      l.wsum[1][wave] = tp;
+      l.wsum[2][wave] = bp;
     }
   }
   __syncthreads();
   if (pt == 0) {
     for (int w = 0; w < wave; ++w) {
-      run += wsum[0][w];
-      tp += wsum[1][w];
-      bp += wsum[2][w];
+      run += l.wsum[0][w];
+      tp += l.wsum[1][w];
+      bp += l.wsum[2][w];
     }
     // inclusive sums -> entry e + 1; entry 0 is zero
     if (e < E) {
-      offsets[e + 1] = run;
-      tile_prefix[e + 1] = tp;
-      blk_prefix[e + 1] = bp;
-      off[e] = run - tot;
-      rows[e] = tot;
-      rank[e] = 0;
+      o.offsets[e + 1] = run;
+      o.tile_prefix[e + 1] = tp;
+      o.blk_prefix[e + 1] = bp;
+      l.off[e] = run - tot;
+      l.rows[e] = tot;
+      l.rank[e] = 0;
     }
     if (e == 0) {
-      offsets[0] = 0;
-      tile_prefix[0] = 0;
-      blk_prefix[0] = 0;
+      o.offsets[0] = 0;
+      o.tile_prefix[0] = 0;
+      o.blk_prefix[0] = 0;
     }
-    if (e < 8) share[e] = 0;
+    if (e < 8) l.share[e] = 0;
   }
   __syncthreads();
+}
+__device__ __forceinline__ void moe_scan_order(MoeScanLds& l, int E, int* order) {
+  const int e = threadIdx.x % MOE_MAX_E, pt = threadIdx.x / MOE_MAX_E;
+  if (order == nullptr) return;
+  const int j0 = pt * (MOE_MAX_E / SCAN_PARTS), j1 = j0 + MOE_MAX_E / SCAN_PARTS;
   if (e < E) {
-    int pos = off[e];
-    for (int q = 0; q < pt; ++q) pos += part[q][e];
+    const int c = l.rows[e];
+    int before = 0;
+#pragma unroll 8
+    for (int j = j0; j < (j1 < E ? j1 : E); ++j) before += (l.rows[j] > c || (l.rows[j] == c && j < e)) ? 1 : 0;
+    atomicAdd(&l.rank[e], before);
+  }
+  __syncthreads();
+  if (pt == 0 && e < E) {
+    order[l.rank[e]] = e;
+    atomicAdd(&l.share[moe_dealt_to(l.rank[e])], (l.rows[e] + SG_COLS - 1) / SG_COLS);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) order[E] = moe_split_rows(l.share, l.off[E - 1] + l.rows[E - 1]);
+}
+
+__global__ __launch_bounds__(SCAN_PARTS * MOE_MAX_E) void moe_scan_kernel(const int* __restrict__ cnt, int nb, int E,
+                                                                          int* __restrict__ base, MoeScanOut o) {
+  __shared__ MoeScanLds l;
+  const int e = threadIdx.x % MOE_MAX_E, pt = threadIdx.x / MOE_MAX_E;
+  const int per = (nb + SCAN_PARTS - 1) / SCAN_PARTS;
+  const int b0 = pt * per, b1 = b0 + per < nb ? b0 + per : nb;
+  int s = 0;
+  if (e < E) {
+    for (int b = b0; b < b1; b += 8) {
+      int v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = b + u < b1 ? cnt[(b + u) * E + e] : 0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += v[u];
+    }
+  }
+  l.part[pt][e] = s;
+  __syncthreads();
+  moe_scan_experts(l, E, o);
+  if (e < E) {
+    int pos = l.off[e];
+    for (int q = 0; q < pt; ++q) pos += l.part[q][e];
     for (int b = b0; b < b1; b += 8) {
       int v[8];
 #pragma unroll
@@ -203,35 +245,85 @@ __global__ __launch_bounds__(SCAN_PARTS * MOE_MAX_E) void moe_scan_kernel(const 
       }
     }
   }
-  if (order != nullptr) {
-    const int j0 = pt * (MOE_MAX_E / SCAN_PARTS), j1 = j0 + MOE_MAX_E / SCAN_PARTS;
-    if (e < E) {
-      const int c = rows[e];
-      int before = 0;
-#pragma unroll 8
-      for (int j = j0; j < (j1 < E ? j1 : E); ++j) before += (rows[j] > c || (rows[j] == c && j < e)) ? 1 : 0;
-      atomicAdd(&rank[e], before);
-    }
-    __syncthreads();
-    if (pt == 0 && e < E) {
-      order[rank[e]] = e;
-      atomicAdd(&share[moe_dealt_to(rank[e])], (rows[e] + SG_COLS - 1) / SG_COLS);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) order[E] = moe_split_rows(share, off[E - 1] + rows[E - 1]);
+  moe_scan_order(l, E, o.order);
+}
+
+// Lanes of the wave whose key (0 .. 255) is this lane's; lanes with key < 0 match nobody.
+__device__ __forceinline__ unsigned long long moe_same_key(int key) {
+  unsigned long long same = __ballot(key >= 0);
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    const bool bit = key >> b & 1;
+    const unsigned long long with = __ballot(bit);
+    same &= bit ? with : ~with;
   }
+  return key >= 0 ? same : 0ull;
+}
+struct MoePerm {
+  int *perm, *inv_perm, *row_token;
+  __device__ __forceinline__ void place(int f, int pos, int k) const {
+    perm[pos] = f;
+    inv_perm[f] = pos;
+    row_token[pos] = f / k;
+  }
+};
+
+// The whole sort of a few chunks by one work-group: for 1624 keys histogram, scan and placement are 3 + 5 + 6 us as three
+// launches, and the gaps between them, and 7 as one.  (A launch per step is what many chunks need: their placement is spread.)
+constexpr int SORT_CHUNKS = 4;
+__global__ __launch_bounds__(PERM_CHUNK) void moe_sort_kernel(const int* __restrict__ keys, int n, int E, int k, MoeScanOut o,
+                                                              MoePerm out) {
+  static_assert(SORT_CHUNKS == SCAN_PARTS && PERM_CHUNK == SCAN_PARTS * MOE_MAX_E, "a part of the scan per chunk");
+  constexpr int NW = PERM_CHUNK / 64;
+  __shared__ MoeScanLds l;
+  __shared__ int hist[SORT_CHUNKS * NW][MOE_MAX_E];  // by chunk and wave: counts, then counts of the waves before in the chunk
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int key[SORT_CHUNKS], rank[SORT_CHUNKS];
+#pragma unroll
+  for (int c = 0; c < SORT_CHUNKS; ++c) {
+    const int f = c * PERM_CHUNK + threadIdx.x;
+    key[c] = f < n ? keys[f] : -1;
+    if ((unsigned)key[c] >= (unsigned)E) key[c] = -1;  // never produced by the top-k
+  }
+  for (int i = threadIdx.x; i < SORT_CHUNKS * NW * MOE_MAX_E; i += PERM_CHUNK) (&hist[0][0])[i] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < SORT_CHUNKS; ++c) {
+    const unsigned long long same = moe_same_key(key[c]);
+    rank[c] = __popcll(same & ((1ull << lane) - 1ull));
+    if (key[c] >= 0 && rank[c] == 0) hist[c * NW + wave][key[c]] = __popcll(same);
+  }
+  __syncthreads();
+  {
+    const int e = threadIdx.x % MOE_MAX_E, c = threadIdx.x / MOE_MAX_E;
+    int s = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const int v = hist[c * NW + w][e];
+      hist[c * NW + w][e] = s;
+      s += v;
+    }
+    l.part[c][e] = s;
+  }
+  __syncthreads();
+  moe_scan_experts(l, E, o);
+#pragma unroll
+  for (int c = 0; c < SORT_CHUNKS; ++c) {
+    if (key[c] < 0) continue;
+    int pos = l.off[key[c]] + hist[c * NW + wave][key[c]] + rank[c];
+#pragma unroll
+    for (int q = 0; q < c; ++q) pos += l.part[q][key[c]];
+    out.place(c * PERM_CHUNK + threadIdx.x, pos, k);
+  }
+  moe_scan_order(l, E, o.order);
 }
 
 // Stable placement of one chunk: position = base[chunk][key] + number of earlier
 // entries of the chunk with the same key.  That rank is the count in the earlier
 // waves (per-wave histograms in LDS) plus the count among the earlier lanes of the
-// own wave (64 shuffles), instead of a scan over the whole chunk per thread.
-__global__ __launch_bounds__(PERM_CHUNK) void moe_scatter_kernel(const int* __restrict__ keys, int n,
-                                                                 int E, int k,
-                                                                 const int* __restrict__ base,
-                                                                 int* __restrict__ perm,
-                                                                 int* __restrict__ inv_perm,
-                                                                 int* __restrict__ row_token) {
+// own wave.
+__global__ __launch_bounds__(PERM_CHUNK) void moe_scatter_kernel(const int* __restrict__ keys, int n, int E, int k,
+                                                                 const int* __restrict__ base, MoePerm out) {
   constexpr int NW = PERM_CHUNK / 64;
   __shared__ int hist[NW][256];  // E <= 256
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -239,20 +331,14 @@ __global__ __launch_bounds__(PERM_CHUNK) void moe_scatter_kernel(const int* __re
   __syncthreads();
   const int f = blockIdx.x * PERM_CHUNK + threadIdx.x;
   int key = f < n ? keys[f] : -1;
-  if ((unsigned)key >= (unsigned)E) key = -1;  // never produced by moe_topk_kernel
-  if (key >= 0) atomicAdd(&hist[wave][key], 1);
-  int rank = 0;
-  for (int j = 0; j < 64; ++j) {
-    const int kj = __shfl(key, j, 64);
-    rank += (j < lane && kj == key) ? 1 : 0;
-  }
+  if ((unsigned)key >= (unsigned)E) key = -1;  // never produced by the top-k
+  const unsigned long long same = moe_same_key(key);
+  int rank = __popcll(same & ((1ull << lane) - 1ull));
+  if (key >= 0 && rank == 0) hist[wave][key] = __popcll(same);
   __syncthreads();
   if (key >= 0) {
     for (int w = 0; w < wave; ++w) rank += hist[w][key];
-    const int pos = base[blockIdx.x * E + key] + rank;
-    perm[pos] = f;
-    inv_perm[f] = pos;
-    row_token[pos] = f / k;
+    out.place(f, base[blockIdx.x * E + key] + rank, k);
   }
 }
 
@@ -654,11 +740,14 @@ __global__ __launch_bounds__(256) void moe_rowdot16_kernel(
 // token gradient through the gather, and the weight multiplies the rank-r products and the gated gradient.
 // ----------------------------------------------------------------------------
 
-// bf16 adapters of one block from its six parameters (f32 or bf16): gate and up share their input, so their
-// A are stacked ([E, 2r, H]) and their B form a block-diagonal [E, 2I, 2r]; down's are copied.
+// bf16 adapters of one block from its six parameters (f32 or bf16), each as the forward reads it and transposed as the
+// backward does: gate and up share their input, so their A are stacked ([E, 2r, H]) and their B form a block-diagonal
+// [E, 2I, 2r]; down's are copied.  HBM-bound: 76 MB for 128 experts, hidden 2048, intermediate 768 and rank 8 take 17 us.  (A
+// copy alone took 11, and the transposes as a launch of the backward, which read the copies once more, 12 to 15.)
 struct MoePack {
   const void *gate_A, *gate_B, *up_A, *up_B, *down_A, *down_B;
   uint16_t *A_gu, *B_gu, *A_d, *B_d;
+  uint16_t *At_gu, *Bt_gu, *At_d, *Bt_d;  // [E,H,2r], [E,2r,2I], [E,I,r], [E,r,H]
   int64_t H, I;
   int E, r, bf16;
 };
@@ -669,35 +758,83 @@ __device__ __forceinline__ uint4 load8_bf16(const void* src, int64_t i, int is_b
   return make_uint4(pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w), pack_bf16x2(b.x, b.y), pack_bf16x2(b.z, b.w));
 }
 
-__global__ __launch_bounds__(256) void moe_pack_kernel(MoePack p) {
-  // every dimension is a multiple of 8: a thread writes 8 consecutive values of one output row
-  const int64_t nA = (int64_t)p.E * p.r * p.H / 8, nB = (int64_t)p.E * p.I * p.r / 8;   // per projection
-  const int64_t nAd = (int64_t)p.E * p.r * p.I / 8, nBd = (int64_t)p.E * p.H * p.r / 8;
-  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < 2 * nA) {
-    const int up = i >= nA;
-    i = (i - up * nA) * 8;
-    const int64_t per = (int64_t)p.r * p.H, e = i / per;
-    *(uint4*)(p.A_gu + (2 * e + up) * per + (i - e * per)) = load8_bf16(up ? p.up_A : p.gate_A, i, p.bf16);
+// Block `blk` of 256 threads.  Every dimension is a multiple of 8: a thread takes an 8 x 8 block of one matrix, of gate's and
+// of up's A, whose transposed rows lie side by side.
+__device__ __forceinline__ void moe_pack_block(const MoePack& p, int64_t blk) {
+  int64_t i = blk * 256 + threadIdx.x;
+  const int64_t nH = (int64_t)p.E * p.r * p.H / 64, nI = (int64_t)p.E * p.r * p.I / 64;
+  // 0: gate_A and up_A [E,r,H]; 1: gate_B, 2: up_B [E,I,r]; 3: down_A [E,r,I]; 4: down_B [E,H,r]
+  int m = 0;
+  for (; m < 5; ++m) {
+    const int64_t size = m == 0 || m == 4 ? nH : nI;
+    if (i < size) break;
+    i -= size;
+  }
+  if (m == 5) return;
+  const int64_t R = m == 0 || m == 3 ? p.r : m == 4 ? p.H : p.I, C = m == 0 ? p.H : m == 3 ? p.I : p.r;
+  const int64_t CB = C / 8, per = R / 8 * CB, e = i / per;
+  const int64_t r0 = (i - e * per) / CB * 8, c0 = (i - e * per) % CB * 8;
+  const int64_t src = (e * R + r0) * C + c0;
+  auto load = [&](const void* from, uint4 (&v)[8]) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = load8_bf16(from, src + q * C, p.bf16);
+  };
+  auto store = [&](uint16_t* to, int64_t ld, const uint4 (&v)[8]) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) *(uint4*)(to + q * ld) = v[q];
+  };
+  uint4 v[8], t[8];
+  if (m == 0) {
+    uint4 u[8], ut[8];
+    load(p.gate_A, v);
+    load(p.up_A, u);
+    transpose8x8(v, t);
+    transpose8x8(u, ut);
+    uint16_t* to = p.A_gu + (e * 2 * p.r + r0) * p.H + c0;
+    store(to, p.H, v);
+    store(to + p.r * p.H, p.H, u);
+    to = p.At_gu + (e * p.H + c0) * 2 * p.r + r0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      *(uint4*)(to + q * 2 * p.r) = t[q];
+      *(uint4*)(to + q * 2 * p.r + p.r) = ut[q];
+    }
     return;
   }
-  i -= 2 * nA;
-  if (i < 2 * nB) {
-    const int up = i >= nB;
-    i = (i - up * nB) * 8;
-    const int64_t row = i / p.r, c = i - row * p.r, e = row / p.I;   // row of [E, I]
-    uint16_t* dst = p.B_gu + ((2 * e + up) * p.I + (row - e * p.I)) * 2 * p.r + c;
-    *(uint4*)(dst + up * p.r) = load8_bf16(up ? p.up_B : p.gate_B, i, p.bf16);
-    *(uint4*)(dst + (1 - up) * p.r) = make_uint4(0, 0, 0, 0);
+  load(m == 1 ? p.gate_B : m == 2 ? p.up_B : m == 3 ? p.down_A : p.down_B, v);
+  transpose8x8(v, t);
+  if (m > 2) {
+    store((m == 3 ? p.A_d : p.B_d) + src, C, v);
+    store((m == 3 ? p.At_d : p.Bt_d) + (e * C + c0) * R + r0, R, t);
     return;
   }
-  i -= 2 * nB;
-  if (i < nAd) {
-    *(uint4*)(p.A_d + i * 8) = load8_bf16(p.down_A, i * 8, p.bf16);
+  // gate | up of B, and zeros beside them
+  const int up = m - 1;
+  uint16_t* to = p.B_gu + ((e * 2 + up) * p.I + r0) * 2 * p.r + c0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    *(uint4*)(to + q * 2 * p.r + up * p.r) = v[q];
+    *(uint4*)(to + q * 2 * p.r + (1 - up) * p.r) = make_uint4(0, 0, 0, 0);
+  }
+  to = p.Bt_gu + (e * 2 * p.r + c0) * 2 * p.I + r0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    *(uint4*)(to + (up * p.r + q) * 2 * p.I + up * p.I) = t[q];
+    *(uint4*)(to + (up * p.r + q) * 2 * p.I + (1 - up) * p.I) = make_uint4(0, 0, 0, 0);
+  }
+}
+
+// Routing of T tokens by the first blocks, the block's adapters by the rest (they have nothing to do with each other).
+__global__ __launch_bounds__(256) void moe_topk_pack_kernel(const float* __restrict__ logits, int64_t T, int E, int k,
+                                                            int* __restrict__ topk_idx, float* __restrict__ topk_w,
+                                                            MoePack p) {
+  const int64_t first = (T + 3) / 4;
+  if (blockIdx.x >= first) {
+    moe_pack_block(p, blockIdx.x - first);
     return;
   }
-  i -= nAd;
-  if (i < nBd) *(uint4*)(p.B_d + i * 8) = load8_bf16(p.down_B, i * 8, p.bf16);
+  const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t < T) moe_topk_token(logits, t, E, k, topk_idx, topk_w);
 }
 
 __device__ __forceinline__ void unpack8(const uint4& v, float (&f)[8]) {
@@ -897,6 +1034,8 @@ using namespace artk;
 
 extern "C" {
 
+static unsigned blocks256(int64_t n) { return (unsigned)((n + 255) / 256); }
+
 size_t artk_moe_route_workspace_bytes(int64_t T, int32_t E, int32_t k) {
   Workspace ws(nullptr, 0);
   const int64_t n = T * k;
@@ -909,7 +1048,7 @@ size_t artk_moe_route_workspace_bytes(int64_t T, int32_t E, int32_t k) {
 static int32_t moe_route(const float* router_logits, int64_t T, int32_t E, int32_t k, int32_t* topk_idx,
                          float* topk_w, int32_t* perm, int32_t* inv_perm, int32_t* row_token,
                          int32_t* expert_offsets, int32_t* tile_prefix, int32_t* blk_prefix, int32_t* order,
-                         void* workspace, size_t workspace_bytes, artk_stream_t stream) {
+                         const MoePack* pack, void* workspace, size_t workspace_bytes, artk_stream_t stream) {
   ARTK_CHECK_ARG(router_logits && topk_idx && topk_w && perm && inv_perm && row_token &&
                      expert_offsets && tile_prefix && blk_prefix,
                  "null pointer argument");
@@ -928,14 +1067,22 @@ static int32_t moe_route(const float* router_logits, int64_t T, int32_t E, int32
     return ARTK_ERR_WORKSPACE_TOO_SMALL;
   }
   hipStream_t st = (hipStream_t)stream;
-  moe_topk_kernel<<<(unsigned)((T + 3) / 4), 256, 0, st>>>(router_logits, T, E, k, topk_idx, topk_w);
+  const int64_t pack_blocks = pack ? blocks256((int64_t)pack->E * pack->r * (2 * pack->H + 3 * pack->I) / 64) : 0;
+  moe_topk_pack_kernel<<<(unsigned)((T + 3) / 4 + pack_blocks), 256, 0, st>>>(router_logits, T, E, k, topk_idx, topk_w,
+                                                                              pack ? *pack : MoePack{});
   ARTK_CHECK_LAUNCH();
+  const MoeScanOut scan{expert_offsets, tile_prefix, blk_prefix, order};
+  const MoePerm out{perm, inv_perm, row_token};
+  if (nb <= SORT_CHUNKS) {
+    moe_sort_kernel<<<1, PERM_CHUNK, 0, st>>>(topk_idx, n, E, k, scan, out);
+    ARTK_CHECK_LAUNCH();
+    return ARTK_OK;
+  }
   moe_hist_kernel<<<nb, PERM_CHUNK, 0, st>>>(topk_idx, n, E, cnt);
   ARTK_CHECK_LAUNCH();
-  moe_scan_kernel<<<1, SCAN_PARTS * MOE_MAX_E, 0, st>>>(cnt, nb, E, expert_offsets, base, tile_prefix, blk_prefix,
-                                                          order);
+  moe_scan_kernel<<<1, SCAN_PARTS * MOE_MAX_E, 0, st>>>(cnt, nb, E, base, scan);
   ARTK_CHECK_LAUNCH();
-  moe_scatter_kernel<<<nb, PERM_CHUNK, 0, st>>>(topk_idx, n, E, k, base, perm, inv_perm, row_token);
+  moe_scatter_kernel<<<nb, PERM_CHUNK, 0, st>>>(topk_idx, n, E, k, base, out);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }
@@ -945,7 +1092,7 @@ int32_t artk_moe_route(const float* router_logits, int64_t T, int32_t E, int32_t
                        int32_t* expert_offsets, int32_t* tile_prefix, int32_t* blk_prefix,
                        void* workspace, size_t workspace_bytes, artk_stream_t stream) {
   return moe_route(router_logits, T, E, k, topk_idx, topk_w, perm, inv_perm, row_token, expert_offsets, tile_prefix,
-                   blk_prefix, nullptr, workspace, workspace_bytes, stream);
+                   blk_prefix, nullptr, nullptr, workspace, workspace_bytes, stream);
 }
 
 size_t artk_moe_lora_grouped_fwd_workspace_bytes(int64_t n_rows, int64_t in, int64_t out, int32_t E,
@@ -1068,17 +1215,17 @@ int32_t artk_moe_lora_grouped_bwd(const void* g, const void* x, const int32_t* g
 // ---- the whole expert block ---------------------------------------------------------------------------
 // What the forward leaves for the backward, carved in the same order by the size query and both calls.
 struct MoeSaved {
-  uint16_t *A_gu, *B_gu, *A_d, *B_d;  // bf16 adapters [E,2r,H], [E,2I,2r], [E,r,I], [E,H,r]
+  uint16_t *Bt_gu, *At_gu, *Bt_d, *At_d;  // bf16 adapters, transposed: [E,2r,2I], [E,H,2r], [E,r,H], [E,I,r]
   float *xa_gu, *xaw_d;               // x A^T [n,2r]; routing weight times h A_d^T [n,r]
   uint16_t *gu, *h;                   // gate|up [n,2I], silu(gate) up [n,I]
   int* order;                         // [E+1] experts by falling number of rows, then moe_split_rows
 };
 static void carve_moe_saved(Workspace& ws, const artk_moe_experts_t& a, MoeSaved& c) {
   const size_t n = (size_t)(a.T * a.k), E = (size_t)a.E, r = (size_t)a.r, H = (size_t)a.H, I = (size_t)a.I;
-  c.A_gu = ws.take<uint16_t>(E * 2 * r * H);
-  c.B_gu = ws.take<uint16_t>(E * 2 * I * 2 * r);
-  c.A_d = ws.take<uint16_t>(E * r * I);
-  c.B_d = ws.take<uint16_t>(E * H * r);
+  c.Bt_gu = ws.take<uint16_t>(E * 2 * r * 2 * I);
+  c.At_gu = ws.take<uint16_t>(E * H * 2 * r);
+  c.Bt_d = ws.take<uint16_t>(E * r * H);
+  c.At_d = ws.take<uint16_t>(E * I * r);
   c.xa_gu = ws.take<float>(n * 2 * r);
   c.xaw_d = ws.take<float>(n * r);
   c.gu = ws.take<uint16_t>(n * 2 * I);
@@ -1088,10 +1235,15 @@ static void carve_moe_saved(Workspace& ws, const artk_moe_experts_t& a, MoeSaved
 struct MoeFwdScratch {
   char* route;
   size_t route_bytes;
+  uint16_t *A_gu, *B_gu, *A_d, *B_d;  // bf16 adapters [E,2r,H], [E,2I,2r], [E,r,I], [E,H,r]
   uint16_t *xa16_gu, *xa16_d, *down;
 };
 static void carve_moe_fwd(Workspace& ws, const artk_moe_experts_t& a, MoeFwdScratch& c) {
-  const size_t n = (size_t)(a.T * a.k);
+  const size_t n = (size_t)(a.T * a.k), E = (size_t)a.E, r = (size_t)a.r, H = (size_t)a.H, I = (size_t)a.I;
+  c.A_gu = ws.take<uint16_t>(E * 2 * r * H);
+  c.B_gu = ws.take<uint16_t>(E * 2 * I * 2 * r);
+  c.A_d = ws.take<uint16_t>(E * r * I);
+  c.B_d = ws.take<uint16_t>(E * H * r);
   c.route_bytes = artk_moe_route_workspace_bytes(a.T, a.E, a.k);
   c.route = ws.take<char>(c.route_bytes);
   c.xa16_gu = ws.take<uint16_t>(n * round16(2 * a.r));
@@ -1099,16 +1251,11 @@ static void carve_moe_fwd(Workspace& ws, const artk_moe_experts_t& a, MoeFwdScra
   c.down = ws.take<uint16_t>(n * a.H);
 }
 struct MoeBlockBwdScratch {
-  uint16_t *Bt_gu, *At_gu, *Bt_d, *At_d;  // [E,2r,2I], [E,H,2r], [E,r,H], [E,I,r]
   float *gb, *rowp, *dummy;
   uint16_t *gb16, *dhr, *g_gu, *dx_rows;
 };
 static void carve_moe_block_bwd(Workspace& ws, const artk_moe_experts_t& a, MoeBlockBwdScratch& c) {
-  const size_t n = (size_t)(a.T * a.k), E = (size_t)a.E, r = (size_t)a.r, H = (size_t)a.H, I = (size_t)a.I;
-  c.Bt_gu = ws.take<uint16_t>(E * 2 * r * 2 * I);
-  c.At_gu = ws.take<uint16_t>(E * H * 2 * r);
-  c.Bt_d = ws.take<uint16_t>(E * r * H);
-  c.At_d = ws.take<uint16_t>(E * I * r);
+  const size_t n = (size_t)(a.T * a.k), r = (size_t)a.r, H = (size_t)a.H, I = (size_t)a.I;
   const size_t p_d = (size_t)stats_grouped_chunks(a.T * a.k, a.H, a.r, a.E, true) * r;
   const size_t p_gu = (size_t)stats_grouped_chunks(a.T * a.k, 2 * a.I, 2 * a.r, a.E, true) * 2 * r;
   c.rowp = ws.take<float>((p_d > p_gu ? p_d : p_gu) * n);
@@ -1163,7 +1310,6 @@ size_t artk_moe_experts_bwd_workspace_bytes(const artk_moe_experts_t* a) {
   return ws.used + 256;
 }
 
-static unsigned blocks256(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 static int32_t launch_moe_combine(const uint16_t* rows, const artk_moe_experts_t* a, const float* w, void* out, hipStream_t st) {
   const int64_t n8 = a->T * a->H / 8;
@@ -1196,27 +1342,23 @@ int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_
   hipStream_t st = (hipStream_t)stream;
   const int64_t n = a->T * a->k, H = a->H, I = a->I;
   const int E = a->E, r = a->r;
+  const MoePack pack{a->gate_A, a->gate_B, a->up_A, a->up_B, a->down_A, a->down_B,
+                     c.A_gu, c.B_gu, c.A_d, c.B_d, s.At_gu, s.Bt_gu, s.At_d, s.Bt_d, H, I, E, r, a->adapters_bf16};
   if ((rc = moe_route(a->router_logits, a->T, E, a->k, a->topk_idx, a->topk_w, a->perm, a->inv_perm, a->row_token,
-                      a->offsets, a->tile_prefix, a->blk_prefix, s.order, c.route, c.route_bytes, stream)))
+                      a->offsets, a->tile_prefix, a->blk_prefix, s.order, &pack, c.route, c.route_bytes, stream)))
     return rc;
-  {
-    MoePack p{a->gate_A, a->gate_B, a->up_A, a->up_B, a->down_A, a->down_B, s.A_gu, s.B_gu, s.A_d, s.B_d,
-              H,         I,         E,       r,       a->adapters_bf16};
-    moe_pack_kernel<<<blocks256((int64_t)E * r * (3 * H + 3 * I) / 8), 256, 0, st>>>(p);
-    ARTK_CHECK_LAUNCH();
-  }
-  if ((rc = launch_moe_rowdot(a->x, a->row_token, s.A_gu, a->offsets, a->blk_prefix, n, E, H, 2 * r, round16(2 * r),
+  if ((rc = launch_moe_rowdot(a->x, a->row_token, c.A_gu, a->offsets, a->blk_prefix, n, E, H, 2 * r, round16(2 * r),
                               a->scale, s.xa_gu, c.xa16_gu, st)))
     return rc;
-  if ((rc = launch_moe_gemm(a->W_gu, a->x, a->row_token, s.B_gu, c.xa16_gu, s.gu, a->offsets, a->tile_prefix, n, 2 * I,
+  if ((rc = launch_moe_gemm(a->W_gu, a->x, a->row_token, c.B_gu, c.xa16_gu, s.gu, a->offsets, a->tile_prefix, n, 2 * I,
                             H, E, 2 * r, round16(2 * r), s.order, st)))
     return rc;
   moe_silu_mul_kernel<<<blocks256(n * I / 8), 256, 0, st>>>(s.gu, n * I / 8, (int)(I / 8), s.h);
   ARTK_CHECK_LAUNCH();
-  if ((rc = launch_moe_rowdot(s.h, nullptr, s.A_d, a->offsets, a->blk_prefix, n, E, I, r, round16(r), a->scale,
+  if ((rc = launch_moe_rowdot(s.h, nullptr, c.A_d, a->offsets, a->blk_prefix, n, E, I, r, round16(r), a->scale,
                               s.xaw_d, c.xa16_d, st, a->topk_w, a->perm)))
     return rc;
-  if ((rc = launch_moe_gemm(a->W_d, s.h, nullptr, s.B_d, c.xa16_d, c.down, a->offsets, a->tile_prefix, n, H, I, E, r,
+  if ((rc = launch_moe_gemm(a->W_d, s.h, nullptr, c.B_d, c.xa16_d, c.down, a->offsets, a->tile_prefix, n, H, I, E, r,
                             round16(r), s.order, st)))
     return rc;
   return launch_moe_combine(c.down, a, a->topk_w, a->y, st);
@@ -1247,18 +1389,9 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
   const int64_t n = a->T * a->k, H = a->H, I = a->I;
   const int E = a->E, r = a->r;
   const StatsBlock down{s.order}, gate_up_B{s.order, a->dup_B, r, I}, gate_up_A{s.order, a->dup_A, r, 0};
-  {
-    SmallTransposeMulti m;
-    m.n = 4;
-    m.t[0] = {s.B_gu, c.Bt_gu, E, 2 * I, 2 * r};
-    m.t[1] = {s.A_gu, c.At_gu, E, 2 * r, H};
-    m.t[2] = {s.B_d, c.Bt_d, E, H, r};
-    m.t[3] = {s.A_d, c.At_d, E, r, I};
-    if ((rc = launch_small_transpose_multi(m, st))) return rc;
-  }
   const StatsReduceJob none{nullptr, 0, 0, 0.f, nullptr, 0, nullptr, 0, 0.f};
   // down, on the unweighted rows g[token]: g B_d per row and dB_d = s g^T (w h A_d^T) in one pass
-  if ((rc = launch_stats_grouped(a->g, a->T, a->row_token, n, H, c.Bt_d, s.xaw_d, r, E, a->offsets, c.rowp, a->ddown_B,
+  if ((rc = launch_stats_grouped(a->g, a->T, a->row_token, n, H, s.Bt_d, s.xaw_d, r, E, a->offsets, c.rowp, a->ddown_B,
                                  a->scale, 0, c.dummy, st, &down)))
     return rc;
   {
@@ -1267,7 +1400,7 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
     ja.row_idx = a->perm;
     if ((rc = launch_stats_reduce(ja, none, r, st))) return rc;
   }
-  if ((rc = launch_moe_gemm(a->Wt_d, a->g, a->row_token, c.At_d, c.gb16, c.dhr, a->offsets, a->tile_prefix, n, I, H, E,
+  if ((rc = launch_moe_gemm(a->Wt_d, a->g, a->row_token, s.At_d, c.gb16, c.dhr, a->offsets, a->tile_prefix, n, I, H, E,
                             r, round16(r), s.order, st)))
     return rc;
   if ((rc = launch_stats_grouped(s.h, n, nullptr, n, I, nullptr, c.gb, r, E, a->offsets, nullptr, a->ddown_A, a->scale,
@@ -1277,7 +1410,7 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
                                                             c.g_gu);
   ARTK_CHECK_LAUNCH();
   // gate|up
-  if ((rc = launch_stats_grouped(c.g_gu, n, nullptr, n, 2 * I, c.Bt_gu, s.xa_gu, 2 * r, E, a->offsets, c.rowp,
+  if ((rc = launch_stats_grouped(c.g_gu, n, nullptr, n, 2 * I, s.Bt_gu, s.xa_gu, 2 * r, E, a->offsets, c.rowp,
                                  a->dgate_B, a->scale, 0, c.dummy, st, &gate_up_B)))
     return rc;
   {
@@ -1285,7 +1418,7 @@ int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_
                       a->scale};
     if ((rc = launch_stats_reduce(ja, none, 2 * r, st))) return rc;
   }
-  if ((rc = launch_moe_gemm(a->Wt_gu, c.g_gu, nullptr, c.At_gu, c.gb16, c.dx_rows, a->offsets, a->tile_prefix, n, H,
+  if ((rc = launch_moe_gemm(a->Wt_gu, c.g_gu, nullptr, s.At_gu, c.gb16, c.dx_rows, a->offsets, a->tile_prefix, n, H,
                             2 * I, E, 2 * r, round16(2 * r), s.order, st)))
     return rc;
   if ((rc = launch_stats_grouped(a->x, a->T, a->row_token, n, H, nullptr, c.gb, 2 * r, E, a->offsets, nullptr,

@@ -77,6 +77,18 @@ def test_route_nan_and_masked_logits(artk_lib, gpu):
     check_routing(logits, 5, gpu)
 
 
+@pytest.mark.parametrize("T,E,k", [(1, 1, 1), (1, 256, 16), (63, 65, 1), (1024, 64, 1), (1025, 64, 1), (1024, 256, 4),
+                                   (4097, 256, 1), (585, 130, 7)])
+def test_route_edges(artk_lib, gpu, T, E, k):
+    """Up to 4096 keys are sorted by one work-group, a chunk of 1024 after the other; logits of few values, so that most
+    choices are ties, with signed zeros among them."""
+    print(f"moe route edges T={T} E={E} k={k}", flush=True)
+    g = torch.Generator().manual_seed(T + E + k)
+    logits = torch.randint(-2, 3, (T, E), generator=g).float() * torch.where(torch.rand(T, E, generator=g) < 0.5, 1.0, -1.0)
+    check_routing(logits, k, gpu)
+    check_routing(torch.zeros(T, E), k, gpu)
+
+
 def make_experts(E, n_out, n_in, r, seed):
     g = torch.Generator().manual_seed(seed)
     W = (0.02 * torch.randn(E, n_out, n_in, generator=g)).to(torch.bfloat16)
