@@ -684,10 +684,10 @@ struct AttnKeySteps {
   }
 };
 
-template <int D>
-__global__ __launch_bounds__(ATT_THREADS, 3) void attn_fwd_kernel(AttnFwdParams p) {
+// KT: 32 keys of a step.
+template <int D, int KT>
+__global__ __launch_bounds__(ATT_THREADS, D == 128 && KT == 2 ? 2 : 3) void attn_fwd_kernel(AttnFwdParams p) {
   using T = AttnTile<D>;
-  constexpr int KT = D == 64 ? 2 : 1;
   using G = AttnKeySteps<D, KT>;
   __shared__ __attribute__((aligned(1024))) char smem[G::LDS];  // one LDS object (see attn_smem_note)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -861,19 +861,22 @@ __global__ __launch_bounds__(ATT_THREADS, 3) void attn_fwd_kernel(AttnFwdParams 
 // ----------------------------------------------------------------------------
 // How many heads of a group one dK/dV work-group takes for a key block with cnt query tiles.
 // A step is one (query tile, head); a work-group that takes all heads of a group writes dK and dV directly,
-// shares write fp32 partial sums.  So shares are as large as still lets the launch fill the GPU evenly: a
-// quarter of the steps that a resident work-group gets on average, two thirds where the key blocks alone
-// are at least two rounds of work-groups.  Backward in us by the divisor of that average (tenths):
-//   16384 positions, 8 prompts of 137 + 4 x 461, 28 / 4 heads of 128 (two rounds):  6: 629, 15: 595, 40: 623, 100: 707
-//   the same with 16 / 2 heads (one round):                                         15: 497, 30: 423, 40: 409, 100: 425
-//   8192 positions, 28 / 4 heads (one round):                                       15: 319, 30: 337, 40: 350, 100: 376
-//   16384 positions, one prompt of 900 + 2 x 7700, 16 / 2 heads (one round):        15: 2994, 30: 2483, 40: 2368, 100: 2273
+// shares write fp32 partial sums.  So shares are as large as still lets the launch fill the GPU evenly: 5/4 of the
+// steps that a resident work-group gets on average, two thirds where the key blocks alone are at least two rounds of
+// work-groups.  Forward and backward in us by the divisor of that average (tenths), one round, work-groups numbered share
+// by share (attn_kv_item):
+//   16384 positions, 8 prompts of 137 + 4 x 461, 16 / 2 heads of 128:  40: 419, 30: 414, 15: 402, 8: 376, 6: 410
+//   8192 positions, 28 / 4 heads:                                      40: 374, 30: 361, 15: 345, 8: 322, 6: 354
+//   12000 positions, 28 / 4 heads                                      40: 520, 12: 463, 8: 473, 6: 523
+//   16384 positions, 14 / 2 heads of 64:                               40: 217, 15: 207, 8: 202, 6: 205
+// two rounds, 16384 positions, 28 / 4 heads (numbered by head):  6: 629, 15: 595, 40: 623, 100: 707 (backward).
 // A share also costs evenness: its steps come in pieces that the dispatch order (longest list first) does not rank.
 // Where the lists are long on average the set-up is small against one head's steps, and every work-group takes one
-// head: from 16 tiles on where the key blocks are less than two rounds, from 100 on where they are more (there the
-// partial sums of all heads weigh more).  Backward and forward in us, shares / one head each, by the average list:
-//   one round:  8: 427 / 460 (8192 positions, 28 / 4 heads), 12: 315 / 316 (16384, 14 / 2 of 64), 19: 423 / 407 (4096,
-//     28 / 4), 24: 540 / 529 (16384, 14 / 2 of 64), 39: 1375 / 1342 (8192, 28 / 4), 64: 1326 / 1267 (8192, 16 / 2)
+// head: from 24 tiles on where the key blocks are one round (16 where they are less), from 100 on where they are two (there
+// the partial sums of all heads weigh more).  us, shares / one head each, by the average list:
+//   less than a round: 19: 423 / 407 (4096 positions, 28 / 4 heads), 20: 313 / 303 (4096, 16 / 2), 24: 540 / 529 (16384, 14 / 2
+//     of 64), 39: 1375 / 1342 (8192, 28 / 4), 64: 1326 / 1267 (8192, 16 / 2)
+//   a round: 20: 1079 / 1175 (12000, 28 / 4), 29: 1180 / 1201 (16384, 16 / 2), 32: 719 / 591 (4096, 28 / 4, backward and forward)
 //   two rounds (16384, 28 / 4): 19: 1416 / 1590, 30: 2055 / 2230, 72: 4700 / 4820, 128: 8207 / 8139
 struct AttnKvSplit {
   const int* total;  // steps of one head, from the plan
@@ -881,6 +884,10 @@ struct AttnKvSplit {
   int heads_all;     // query heads
   int div;           // steps of a share = total * heads_all / div
   int light_max;     // >= 0 (artk_attn_bwd_tuning): all heads where they make at most this many steps, else one
+  bool packed;       // work-groups are numbered share by share (attn_kv_item)
+  __device__ __forceinline__ bool one_head(int64_t stride, int row) const {  // every work-group of the row takes one head
+    return light_max < 0 && *attn_row(total, stride, row) >= long_total;
+  }
   __device__ __forceinline__ int heads(int cnt, int rep, int64_t stride, int row) const {
     if (light_max >= 0) return cnt * rep <= light_max ? rep : 1;
     const int all = *attn_row(total, stride, row);
@@ -892,6 +899,52 @@ struct AttnKvSplit {
     return (rep + groups - 1) / groups;   // even shares
   }
 };
+
+// (first query head, key block) of a work-group of the dK/dV kernel whose number on its XCD is `item`: the shares of its XCD's
+// units (as in attn_block) in their order, none left out.  A grid has room for a work-group per head; numbered by head,
+// those without a share lie between the others, and each holds its place on a CU for about 3 us (16384 positions of 8
+// prompts of 137 + 4 x 461, 28 / 4 heads: 5832 of 7168).  Numbered like this they come last.  The search costs a work-group
+// a microsecond, so it is for grids that do not fit the GPU at once.  `scratch`: 8 words of LDS.  False: no share left.
+__device__ __forceinline__ bool attn_kv_item(int Hq, int Hkv, int nKb, const int* order, const int* cnt, const AttnKvSplit& split,
+                                             int64_t stride, int row, int item, uint32_t* scratch, int& hq, int& kb) {
+  const int rep = Hq / Hkv, x = blockIdx.x & 7, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int units = (nKb * Hkv + 7) / 8;
+  int base = 0;
+  for (int u0 = 0; u0 < units; u0 += 256) {
+    const int unit = (u0 + (int)threadIdx.x) * 8 + x, rank = unit / Hkv;
+    int b = 0, per = 1, shares = 0;
+    if (rank < nKb) {
+      b = order[rank];
+      per = split.heads(cnt[b], rep, stride, row);
+      shares = (rep + per - 1) / per;
+    }
+    int end = shares;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(end, d, 64);
+      if (lane >= d) end += v;
+    }
+    __syncthreads();
+    if (lane == 63) scratch[wave] = (uint32_t)end;
+    __syncthreads();
+    const int total = (int)(scratch[0] + scratch[1] + scratch[2] + scratch[3]);
+    for (int w = 0; w < wave; ++w) end += (int)scratch[w];
+    const int at = item - base - (end - shares);
+    if (at >= 0 && at < shares) {
+      scratch[4] = (uint32_t)((unit % Hkv) * rep + at * per);
+      scratch[5] = (uint32_t)b;
+    }
+    __syncthreads();
+    if (item - base < total) {
+      hq = __builtin_amdgcn_readfirstlane((int)scratch[4]);
+      kb = __builtin_amdgcn_readfirstlane((int)scratch[5]);
+      __syncthreads();
+      return true;
+    }
+    base += total;
+  }
+  return false;
+}
 
 struct AttnBwdParams {
   const uint16_t *Q, *K, *V, *dO;
@@ -1123,13 +1176,20 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
   const int kg = wave & 1, qh = wave >> 1;
   const TrLane tr(lane);
   const int brow = p.row0 + blockIdx.y;
-  int hq, kb;
-  if (!attn_block(p.Hq, p.Hkv, p.nKb2, attn_row(p.orderT, p.plan_stride, brow), false, hq, kb)) return;
   const int rep = p.Hq / p.Hkv;
-  const int hkv = hq / rep, share = hq - hkv * rep;
+  const int* const order = attn_row(p.orderT, p.plan_stride, brow);
+  const int* const counts = attn_row(p.cntT, p.plan_stride, brow);
+  const bool packed = p.split.packed && !p.split.one_head(p.plan_stride, brow);
+  int hq, kb;
+  if (packed ? !attn_kv_item(p.Hq, p.Hkv, p.nKb2, order, counts, p.split, p.plan_stride, brow, blockIdx.x >> 3, s_list, hq, kb)
+             : !attn_block(p.Hq, p.Hkv, p.nKb2, order, false, hq, kb))
+    return;
+  const int hkv = hq / rep;
   const int key = kb * ATT_BK2 + kg * 32 + n;
-  const int cnt = attn_row(p.cntT, p.plan_stride, brow)[kb];
+  const int cnt = counts[kb];
   const int per = p.split.heads(cnt, rep, p.plan_stride, brow);
+  int share = hq - hkv * rep;
+  if (packed) share /= per;
   if (share * per >= rep) return;
   hq = hkv * rep + share * per;  // first head of this work-group's share
   const int nheads = rep - share * per < per ? rep - share * per : per;
@@ -1535,10 +1595,14 @@ int32_t artk_attn_fwd_rows(const void* q, const void* k, const void* v, const vo
   p.scale_log2e = scale * LOG2E;
   const dim3 grid(attn_grid(Hq, Hkv, pl.nQb), (unsigned)B);
   prof_begin(PROF_ATTN_FWD, st);
-  if (D == 128)
-    attn_fwd_kernel<128><<<grid, ATT_THREADS, 0, st>>>(p);
+  // Up to two work-groups per CU there is no third to make room for, and steps of 64 keys take less time (us, 32 / 64:
+  // 4096 positions in one conversation of 300 + 2 x 1800, 16 / 2 heads 78 / 71; 2048 in two, 28 / 4 heads 23 / 21).
+  if (D == 64)
+    attn_fwd_kernel<64, 2><<<grid, ATT_THREADS, 0, st>>>(p);
+  else if ((int64_t)grid.x * grid.y <= 2 * num_cus())
+    attn_fwd_kernel<128, 2><<<grid, ATT_THREADS, 0, st>>>(p);
   else
-    attn_fwd_kernel<64><<<grid, ATT_THREADS, 0, st>>>(p);
+    attn_fwd_kernel<128, 1><<<grid, ATT_THREADS, 0, st>>>(p);
   prof_end(PROF_ATTN_FWD, st);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
@@ -1665,14 +1729,16 @@ int32_t artk_attn_bwd_rows(const void* q, const void* k, const void* v, const vo
   for (int64_t row0 = 0; row0 < B; row0 += c.kv_rows) {
     const int64_t rows = B - row0 < c.kv_rows ? B - row0 : c.kv_rows;
     const int slots = num_cus() * (D == 64 ? 3 : 2);  // resident work-groups
-    const bool two_rounds = rows * pl.nKb2 * Hkv >= 2 * slots;
+    const int64_t units = rows * pl.nKb2 * Hkv;
+    const bool two_rounds = units >= 2 * slots;
     p.row0 = (int)row0;
     p.split.total = pl.total2;
-    p.split.long_total = (two_rounds ? 100 : 16) * pl.nKb2;
+    p.split.long_total = (two_rounds ? 100 : units >= slots ? 24 : 16) * pl.nKb2;
     p.split.heads_all = (int)(rows * Hq);   // (rows of a batch are taken to be alike)
-    p.split.div = two_rounds ? slots * 3 / 2 : slots * 4;
+    p.split.div = two_rounds ? slots * 3 / 2 : slots * 4 / 5;
     p.split.light_max = g_light_max_override;  // artk_attn_bwd_tuning
     const dim3 grid_kv(attn_grid(Hq, Hkv, pl.nKb2), (unsigned)rows);
+    p.split.packed = Hq != Hkv && !two_rounds && (int64_t)grid_kv.x * grid_kv.y > slots;
     prof_begin(PROF_ATTN_BWD_KV, st);
     if (D == 128)
       attn_bwd_kv_kernel<128><<<grid_kv, 256, 0, st>>>(p);

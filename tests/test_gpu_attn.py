@@ -493,3 +493,29 @@ def test_attn_steps_of_32_keys(artk_lib, gpu, S, D):
         got = [out.detach(), *torch.autograd.grad(out, leaves, d_out.to(gpu))]
         for a, b in zip(got, (ref_out, ref_dq, ref_dk, ref_dv)):
             assert rel_l2(a.float().cpu(), b) <= 1e-2
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,D,layout", [
+    (2560, 16, 2, 128, (4, 60, 4, 130)),    # more work-groups of dK/dV than the GPU holds, XCDs shared by two key/value heads
+    (2816, 15, 3, 128, (2, 90, 5, 250)),    # key/value heads that do not divide the XCDs
+    (3328, 16, 1, 64, (3, 500, 2, 250)),    # shares of 1 to 16 heads, all XCDs on one key/value head
+    (2816, 16, 16, 64, (4, 60, 4, 130)),    # nothing to share
+])
+def test_attn_bwd_numbers_work_groups_share_by_share(artk_lib, gpu, S, Hq, Hkv, D, layout):
+    print("attention shares", S, Hq, Hkv, D, flush=True)
+    q, k, v = make_qkv(S + Hq, S, Hq, Hkv, D)
+    d_out = torch.randn(S, Hq, D, generator=torch.Generator().manual_seed(S)).to(torch.bfloat16)
+    group, parent = synthetic.packed_row_ids(S, S, *layout)
+    ref = attn_oracle.attention_grads(q, k, v, group, parent, d_out)[1:]
+    plan = ops.attn_plan(group.to(gpu), parent.to(gpu))
+    qd, kd, vd, up = (t.to(gpu) for t in (q, k, v, d_out))
+    out, lse = ops.attn_fwd(qd, kd, vd, plan)
+    for knob in (-1, 8, 64):  # (the library's own shares, and two that mix whole groups with single heads)
+        artk_lib.artk_attn_bwd_tuning(knob)
+        try:
+            got, again = (ops.attn_bwd(qd, kd, vd, out, lse, up, plan) for _ in range(2))
+        finally:
+            artk_lib.artk_attn_bwd_tuning(-1)
+        for a, b, c in zip(got, ref, again):
+            assert rel_l2(a.float().cpu(), b) <= 1e-2
+            assert torch.equal(a, c)
