@@ -799,8 +799,14 @@ __global__ __launch_bounds__(nthreads<BWD_NI>()) void dhidden_gemm_kernel(BwdPar
 
   TileAcc<BWD_NI> acc;
   acc.zero();
-  gemm_tile_nt(acc, smem, p.Wt, p.V, (int64_t)ht * TILE, p.H, p.P, p.V, (int64_t)tt * TILE,
-               n_active, kb * BK, ke * BK, p.active_idx);
+  {
+    // rows past the last active one are neither fetched nor computed
+    TileLoaders<BWD_NI> L;
+    L.init(p.Wt, p.V, (int64_t)ht * TILE, p.H, p.P, p.V, (int64_t)tt * TILE, n_active, kb * BK, ke * BK, p.active_idx, true);
+    L.issue_first(smem);
+    const int left = n_active - tt * TILE;
+    gemm_tile_run_cols(acc, smem, L, left < TILE ? left : TILE);
+  }
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
