@@ -549,17 +549,6 @@ __device__ __forceinline__ void gemm_tile_run_pinned(TileAcc<4>& acc, char* smem
   __syncthreads();
 }
 
-template <int NI>
-__device__ __forceinline__ void gemm_tile_nt(TileAcc<NI>& acc, char* smem, const void* P, int64_t ldp,
-                                             int64_t prow0, int64_t prows, const void* Q,
-                                             int64_t ldq, int64_t qrow0, int64_t qrows, int k_begin,
-                                             int k_end, const int* qgather = nullptr) {
-  TileLoaders<NI> L;
-  L.init(P, ldp, prow0, prows, Q, ldq, qrow0, qrows, k_begin, k_end, qgather);
-  L.issue_first(smem);
-  gemm_tile_run(acc, smem, L);
-}
-
 // Map the hardware's round-robin block->XCD placement (block b runs on XCD
 // b % 8) onto contiguous ranges of logical tile ids, so that tiles sharing
 // operand panels run on the same XCD and hit in its private L2.
