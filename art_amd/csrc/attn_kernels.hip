@@ -732,6 +732,7 @@ __global__ __launch_bounds__(ATT_THREADS, D == 128 && KT == 2 ? 2 : 3) void attn
   int stage = 0;
   wait_vmcnt<0>();
   barrier_lds_only();
+  int fresh = 64;  // keys until the reference of the exponentials follows lazily
   while (ks.cur < ks.n) {
     const uint32_t ahead = ks.ahead(smem);
     const int key0 = ks.key(), active = ks.any(wave), partial = ks.mixed(wave);
@@ -798,7 +799,11 @@ __global__ __launch_bounds__(ATT_THREADS, D == 128 && KT == 2 ? 2 : 3) void attn
       // 64 output accumulators are rescaled on few tiles instead of on most early ones.  Until
       // then exponentials are at most 2^ATT_LAZY, which fp32 sums and bf16 operands hold without
       // loss; the final division by the sum is the same.
-      if (__any(mloc > m_run + ATT_LAZY)) {
+      // It follows at once over a wave's first 64 keys: the term at the reference is 1 and has no rounding error (out
+      // against 64 bits on dense rows 2.122e-3, and 2.137e-3 if it follows over the first 32 alone).
+      const bool move = __any(mloc > m_run + (fresh > 0 ? 0.f : ATT_LAZY));
+      fresh -= 32 * KT;
+      if (move) {
         const float m_new = fmaxf(m_run, mloc);
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
         m_run = m_new;
