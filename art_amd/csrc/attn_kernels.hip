@@ -41,7 +41,6 @@ constexpr int ATT_ROW = 256;   // row lengths are multiples of this
 constexpr int ATT_BM = 128;    // queries per work-group
 constexpr int ATT_BN = 64;     // keys per tile
 constexpr int ATT_STAGES = 2;
-constexpr float ATT_LAZY = 8.f;   // forward: how far a score may exceed the exponentials' reference (log2 units)
 constexpr int ATT_MAX_KB = 1024;  // key blocks per row the list in LDS can hold
 constexpr int ATT_BQ2 = 64;    // dK/dV kernel: queries per tile
 constexpr int ATT_BK2 = 64;    // dK/dV kernel: keys per work-group (2 key groups x 32)
@@ -689,6 +688,7 @@ template <int D, int KT>
 __global__ __launch_bounds__(ATT_THREADS, D == 128 && KT == 2 ? 2 : 3) void attn_fwd_kernel(AttnFwdParams p) {
   using T = AttnTile<D>;
   using G = AttnKeySteps<D, KT>;
+  constexpr float LAZY = KT == 1 ? 4.f : 8.f;
   __shared__ __attribute__((aligned(1024))) char smem[G::LDS];  // one LDS object (see attn_smem_note)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5;
@@ -795,13 +795,17 @@ __global__ __launch_bounds__(ATT_THREADS, D == 128 && KT == 2 ? 2 : 3) void attn
         mloc = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * p.scale_log2e;  // both halves of a query
       }
       // The reference of the exponentials follows the running maximum lazily: it moves only when
-      // some query of the wave has a score more than ATT_LAZY (in units of log2) above it, so the
+      // some query of the wave has a score more than LAZY (in units of log2) above it, so the
       // 64 output accumulators are rescaled on few tiles instead of on most early ones.  Until
-      // then exponentials are at most 2^ATT_LAZY, which fp32 sums and bf16 operands hold without
+      // then exponentials are at most 2^LAZY, which fp32 sums and bf16 operands hold without
       // loss; the final division by the sum is the same.
       // It follows at once over a wave's first 64 keys: the term at the reference is 1 and has no rounding error (out
       // against 64 bits on dense rows 2.122e-3, and 2.137e-3 if it follows over the first 32 alone).
-      const bool move = __any(mloc > m_run + (fresh > 0 ? 0.f : ATT_LAZY));
+      // For the same reason steps of 32 keys follow from 2^4 on: a move that the first half of 64 keys causes does not see the
+      // maximum of the second.  out against 64 bits in steps of 64 / of 32 with 2^8 / of 32 with 2^4, 16384 packed positions, 28 / 4
+      // heads: normal q and k 2.191e-3 / 2.141e-3 / 2.140e-3 (145 us / 145 us in steps of 32), q four times as large 2.028e-3 /
+      // 2.063e-3 / 1.837e-3 (144 / 146).
+      const bool move = __any(mloc > m_run + (fresh > 0 ? 0.f : LAZY));
       fresh -= 32 * KT;
       if (move) {
         const float m_new = fmaxf(m_run, mloc);

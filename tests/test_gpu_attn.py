@@ -519,3 +519,40 @@ def test_attn_bwd_numbers_work_groups_share_by_share(artk_lib, gpu, S, Hq, Hkv, 
         for a, b, c in zip(got, ref, again):
             assert rel_l2(a.float().cpu(), b) <= 1e-2
             assert torch.equal(a, c)
+
+
+def fwd_work_groups(S, Hq, Hkv):
+    """Work-groups of the forward for one row.  At a head dimension of 128 more than two per CU take steps of 32 keys."""
+    blocks = -(-S // 256) * 2
+    return -(-blocks * Hkv // 8) * 8 * (Hq // Hkv)
+
+
+def cus():
+    return torch.cuda.get_device_properties(0).multi_processor_count
+
+
+@pytest.mark.parametrize("std", [1.0, 2.0, 4.0, 8.0])
+def test_attn_steps_of_32_keys_are_as_exact(artk_lib, gpu, std):
+    """One row in steps of 32 keys (all heads in a call) and of 64 (a call per key/value head) against 64 bits: out is no
+    farther off, be the scores flat or peaked."""
+    S, Hq, Hkv, D = 2531, 28, 4, 128
+    assert fwd_work_groups(S, Hq, Hkv) > 2 * cus() >= fwd_work_groups(S, Hq // Hkv, 1)
+    print("attention against 64 bits", std, flush=True)
+    q, k, v = (t.to(gpu) for t in make_qkv(int(std), S, Hq, Hkv, D))
+    q = (q.float() * std).to(torch.bfloat16)
+    group, parent = (t.to(gpu) for t in synthetic.packed_row_ids(7, S, 2, 150, 4, 260))
+    plan = ops.attn_plan_rows(group[None], parent[None])
+    from art_amd.attention import packed_attention
+    rep = Hq // Hkv
+    with torch.no_grad():
+        whole = packed_attention(q, k, v, plan)
+        parts = torch.cat([packed_attention(q[:, h * rep:(h + 1) * rep], k[:, h:h + 1], v[:, h:h + 1], plan)
+                           for h in range(Hkv)], 1)
+    i = torch.arange(S, device=gpu)
+    hidden = (i[None] > i[:, None]) | ((group[:, None] != group[None]) & (parent[:, None] != group[None]))
+    err = torch.zeros(2, dtype=torch.float64, device=gpu)
+    for h in range(Hq):
+        s = q[:, h].double() @ k[:, h // rep].double().t().contiguous() * D ** -0.5
+        ref = torch.softmax(s.masked_fill_(hidden, float("-inf")), 1) @ v[:, h // rep].double()
+        err += torch.stack([(t[:, h].double() - ref).pow(2).sum() for t in (whole, parts)])
+    assert err[0] <= err[1], err.sqrt().tolist()
