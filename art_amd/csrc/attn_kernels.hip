@@ -1638,10 +1638,12 @@ int32_t artk_attn_fwd_rows(const void* q, const void* k, const void* v, const vo
   const dim3 grid(attn_grid(Hq, Hkv, pl.nQb), (unsigned)B);
   prof_begin(PROF_ATTN_FWD, st);
   // Up to two work-groups per CU there is no third to make room for, and steps of 64 keys take less time (us, 32 / 64:
-  // 4096 positions in one conversation of 300 + 2 x 1800, 16 / 2 heads 78 / 71; 2048 in two, 28 / 4 heads 23 / 21).
+  // 4096 positions in one conversation of 300 + 2 x 1800, 16 / 2 heads 78 / 71; 2048 in two, 28 / 4 heads 23 / 21).  The count is
+  // that of one row, so that its bits are the same in any batch.  That has a price in batches of short rows (2 of 1999
+  // positions, 28 / 4 heads 31 / 34; 8 of 1300, 16 / 2 41 / 50).
   if (D == 64)
     attn_fwd_kernel<64, 2><<<grid, ATT_THREADS, 0, st>>>(p);
-  else if ((int64_t)grid.x * grid.y <= 2 * num_cus())
+  else if ((int64_t)grid.x <= 2 * num_cus())
     attn_fwd_kernel<128, 2><<<grid, ATT_THREADS, 0, st>>>(p);
   else
     attn_fwd_kernel<128, 1><<<grid, ATT_THREADS, 0, st>>>(p);

@@ -556,3 +556,26 @@ def test_attn_steps_of_32_keys_are_as_exact(artk_lib, gpu, std):
         ref = torch.softmax(s.masked_fill_(hidden, float("-inf")), 1) @ v[:, h // rep].double()
         err += torch.stack([(t[:, h].double() - ref).pow(2).sum() for t in (whole, parts)])
     assert err[0] <= err[1], err.sqrt().tolist()
+
+
+def test_attn_row_is_the_same_in_any_batch(artk_lib, gpu):
+    """A row whose forward fills the GPU twice over only together with another: out and dQ (which reads lse) are those of the
+    row alone, bit for bit."""
+    from art_amd.attention import attention_plans, packed_attention
+    B, S, Hq, Hkv, D = 2, 2531, 16, 2, 128
+    assert fwd_work_groups(S, Hq, Hkv) <= 2 * cus() < B * fwd_work_groups(S, Hq, Hkv)
+    print("attention row in a batch", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(3)
+    data = [torch.randn(B, S, H, D, generator=g, device=gpu).to(torch.bfloat16) for H in (Hq, Hkv, Hkv, Hq)]
+    ids = [synthetic.packed_row_ids(80 + b, S, 2, 150, 4, 260) for b in range(B)]
+    group, parent = (torch.stack([i[j] for i in ids]).to(gpu) for j in (0, 1))
+
+    def call(rows):
+        leaves = [t[rows].detach().requires_grad_(True) for t in data[:3]]
+        out = packed_attention(*leaves, attention_plans(group[rows], parent[rows]))
+        return out.detach(), torch.autograd.grad(out, leaves, data[3][rows])[0]
+
+    batch = call(slice(None))
+    for b in range(B):
+        for got, want in zip(batch, call(slice(b, b + 1))):
+            assert torch.equal(got[b], want[0])
