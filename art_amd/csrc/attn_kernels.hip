@@ -1104,6 +1104,9 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kern
           sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_at(kh, bk, s), qf[s], sc, 0, 0, 0);
           dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_at(kh + G::V_OFF, bk, s), dof[s], dp, 0, 0, 0);
         }
+        // the mask comes behind the multiply-add: whatever a query's lse and the scale are, P is 0 where it sees nothing
+#pragma unroll
+        for (int j = 0; j < 16; ++j) sc[j] = __builtin_fmaf(sc[j], p.scale_log2e, nlse2);
         if (partial >> kt & 1) {  // one branch for all elements: tested inside the loop below it becomes one per element
 #pragma unroll
           for (int g4 = 0; g4 < 4; ++g4) {
@@ -1117,7 +1120,7 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kern
         }
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-          const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j], p.scale_log2e, nlse2));
+          const float pr = __builtin_amdgcn_exp2f(sc[j]);
           dsf[2 * kt + j / 8][j % 8] = (__bf16)(pr * (dp[j] - delta));
         }
       }
@@ -1340,6 +1343,13 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       }
     }
+    // the mask comes behind the multiply-add: whatever a query's lse and the scale are, P is 0 where it sees nothing
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      const floatx4 l4 = *(const floatx4*)(r_lse2 + 32 * qh + 8 * g4 + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sc[4 * g4 + e] = __builtin_fmaf(sc[4 * g4 + e], p.scale_log2e, -l4[e]);
+    }
     if (partial) {  // one branch for all elements: tested inside the loop below it becomes one per element
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4) {
@@ -1377,12 +1387,11 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_kv_kernel(AttnB
 #pragma unroll
     for (int g4 = 0; g4 < 4; ++g4) {
       const int qi = 32 * qh + 8 * g4 + 4 * h;
-      const floatx4 l4 = *(const floatx4*)(r_lse2 + qi);
       const floatx4 d4 = *(const floatx4*)(r_delta + qi);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int j = 4 * g4 + e;
-        const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j], p.scale_log2e, -l4[e]));
+        const float pr = __builtin_amdgcn_exp2f(sc[j]);
         pf[j / 8][j % 8] = (__bf16)pr;
         dsf[j / 8][j % 8] = (__bf16)(pr * (dp[j] - d4[e]));
       }

@@ -579,3 +579,33 @@ def test_attn_row_is_the_same_in_any_batch(artk_lib, gpu):
     for b in range(B):
         for got, want in zip(batch, call(slice(b, b + 1))):
             assert torch.equal(got[b], want[0])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_attn_bwd_mask_holds_for_any_lse_and_scale(artk_lib, gpu, D):
+    """P is 0 at a pair that is not visible, whatever the query's lse and the scale: dV of the keys that a poisoned query does
+    not see keeps its bits, and a scale that is not positive (the forward refuses it) gives the gradients of that scale."""
+    S, Hq, Hkv = 256, 4, 2
+    q, k, v = make_qkv(91 + D, S, Hq, Hkv, D)
+    d_out = torch.randn(S, Hq, D, generator=torch.Generator().manual_seed(5)).to(torch.bfloat16)
+    ids = (torch.arange(S) >= 48).long()   # the border of the two groups lies inside a cell of 32 x 32
+    plan = ops.attn_plan(ids.to(gpu), ids.to(gpu))
+    print("attention backward mask", D, flush=True)
+
+    def grads(q):
+        qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
+        out, lse = ops.attn_fwd(qd, kd, vd, plan)
+        return ops.attn_bwd(qd, kd, vd, out, lse, d_out.to(gpu), plan)
+
+    poisoned = q.clone()
+    poisoned[60] = float("nan")
+    (dq, _, dv), (dq_p, _, dv_p) = grads(q), grads(poisoned)
+    assert torch.equal(dv_p[:48], dv[:48]) and torch.equal(dq_p[:48], dq[:48])
+    for scale in (-0.05, 0.0):
+        out, lse = attn_oracle.attention(q, k, v, ids, ids, scale)
+        ref = attn_oracle.attention_grads(q, k, v, ids, ids, d_out, scale)[1:]
+        got = ops.attn_bwd(*(t.to(gpu) for t in (q, k, v, out.to(torch.bfloat16), lse, d_out)), plan, scale)
+        for a, b in zip(got, ref):
+            assert torch.isfinite(a).all()
+            if b.norm() > 0:
+                assert rel_l2(a.float().cpu(), b) <= 1e-2
