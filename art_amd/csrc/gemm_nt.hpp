@@ -402,8 +402,8 @@ __device__ __forceinline__ void gemm_tile_run_8(TileAcc<2>& acc, char* smem, con
 
 // gemm_tile_run for a tile whose column operand has only `ncols` (<= 256) rows that anybody
 // stores: a wave computes only those of its NI 32-column tiles that contain such a column
-// (wave-uniform choice; every variant executes the same barriers).  8-wave shape only.  Its caller
-// is the grouped GEMM, so the whole fill of a stage is requested right after the barrier.
+// (wave-uniform choice; every variant executes the same barriers).  8-wave shape only.  For partial tiles: with less to
+// compute the whole fill of a stage is requested right after the barrier.
 __device__ __forceinline__ void gemm_tile_run_cols(TileAcc<2>& acc, char* smem, const TileLoaders<2>& L,
                                                    int ncols) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -547,6 +547,17 @@ __device__ __forceinline__ void gemm_tile_run_pinned(TileAcc<4>& acc, char* smem
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   __syncthreads();
+}
+
+template <int NI>
+__device__ __forceinline__ void gemm_tile_nt(TileAcc<NI>& acc, char* smem, const void* P, int64_t ldp,
+                                             int64_t prow0, int64_t prows, const void* Q,
+                                             int64_t ldq, int64_t qrow0, int64_t qrows, int k_begin,
+                                             int k_end, const int* qgather = nullptr) {
+  TileLoaders<NI> L;
+  L.init(P, ldp, prow0, prows, Q, ldq, qrow0, qrows, k_begin, k_end, qgather);
+  L.issue_first(smem);
+  gemm_tile_run(acc, smem, L);
 }
 
 // Map the hardware's round-robin block->XCD placement (block b runs on XCD
