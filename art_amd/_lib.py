@@ -120,6 +120,8 @@ SIGNATURES.update({
     "artk_moe_experts_saved_bytes": (_sz, [C.POINTER(MoeExpertsStruct)]),
     "artk_moe_experts_fwd_workspace_bytes": (_sz, [C.POINTER(MoeExpertsStruct)]),
     "artk_moe_experts_fwd": (_i32, [C.POINTER(MoeExpertsStruct), _p, _sz, _p]),
+    "artk_moe_experts_eval_workspace_bytes": (_sz, [C.POINTER(MoeExpertsStruct)]),
+    "artk_moe_experts_eval": (_i32, [C.POINTER(MoeExpertsStruct), _p, _sz, _p]),
     "artk_moe_experts_bwd_workspace_bytes": (_sz, [C.POINTER(MoeExpertsStruct)]),
     "artk_moe_experts_bwd": (_i32, [C.POINTER(MoeExpertsStruct), _p, _sz, _p]),
     "artk_adamw8bit_step": (_i32, [_p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _f32, _f32, _f32, _f32, _f32, _i32,

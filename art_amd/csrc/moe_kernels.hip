@@ -743,11 +743,12 @@ __global__ __launch_bounds__(256) void moe_rowdot16_kernel(
 // bf16 adapters of one block from its six parameters (f32 or bf16), each as the forward reads it and transposed as the
 // backward does: gate and up share their input, so their A are stacked ([E, 2r, H]) and their B form a block-diagonal
 // [E, 2I, 2r]; down's are copied.  HBM-bound: 76 MB for 128 experts, hidden 2048, intermediate 768 and rank 8 take 17 us.  (A
-// copy alone took 11, and the transposes as a launch of the backward, which read the copies once more, 12 to 15.)
+// copy alone took 11, and the transposes as a launch of the backward, which read the copies once more, 12 to 15.)  A forward
+// that no backward follows leaves the transposes out (203 tokens 260 -> 257 us, rank 16 277 -> 264).
 struct MoePack {
   const void *gate_A, *gate_B, *up_A, *up_B, *down_A, *down_B;
   uint16_t *A_gu, *B_gu, *A_d, *B_d;
-  uint16_t *At_gu, *Bt_gu, *At_d, *Bt_d;  // [E,H,2r], [E,2r,2I], [E,I,r], [E,r,H]
+  uint16_t *At_gu, *Bt_gu, *At_d, *Bt_d;  // [E,H,2r], [E,2r,2I], [E,I,r], [E,r,H]; all null: no backward follows
   int64_t H, I;
   int E, r, bf16;
 };
@@ -783,16 +784,18 @@ __device__ __forceinline__ void moe_pack_block(const MoePack& p, int64_t blk) {
 #pragma unroll
     for (int q = 0; q < 8; ++q) *(uint4*)(to + q * ld) = v[q];
   };
+  const bool transposed = p.At_gu != nullptr;
   uint4 v[8], t[8];
   if (m == 0) {
     uint4 u[8], ut[8];
     load(p.gate_A, v);
     load(p.up_A, u);
-    transpose8x8(v, t);
-    transpose8x8(u, ut);
     uint16_t* to = p.A_gu + (e * 2 * p.r + r0) * p.H + c0;
     store(to, p.H, v);
     store(to + p.r * p.H, p.H, u);
+    if (!transposed) return;
+    transpose8x8(v, t);
+    transpose8x8(u, ut);
     to = p.At_gu + (e * p.H + c0) * 2 * p.r + r0;
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
@@ -802,9 +805,10 @@ __device__ __forceinline__ void moe_pack_block(const MoePack& p, int64_t blk) {
     return;
   }
   load(m == 1 ? p.gate_B : m == 2 ? p.up_B : m == 3 ? p.down_A : p.down_B, v);
-  transpose8x8(v, t);
   if (m > 2) {
     store((m == 3 ? p.A_d : p.B_d) + src, C, v);
+    if (!transposed) return;
+    transpose8x8(v, t);
     store((m == 3 ? p.At_d : p.Bt_d) + (e * C + c0) * R + r0, R, t);
     return;
   }
@@ -816,6 +820,8 @@ __device__ __forceinline__ void moe_pack_block(const MoePack& p, int64_t blk) {
     *(uint4*)(to + q * 2 * p.r + up * p.r) = v[q];
     *(uint4*)(to + q * 2 * p.r + (1 - up) * p.r) = make_uint4(0, 0, 0, 0);
   }
+  if (!transposed) return;
+  transpose8x8(v, t);
   to = p.Bt_gu + (e * 2 * p.r + c0) * 2 * p.I + r0;
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
@@ -1220,12 +1226,15 @@ struct MoeSaved {
   uint16_t *gu, *h;                   // gate|up [n,2I], silu(gate) up [n,I]
   int* order;                         // [E+1] experts by falling number of rows, then moe_split_rows
 };
-static void carve_moe_saved(Workspace& ws, const artk_moe_experts_t& a, MoeSaved& c) {
+static void carve_moe_saved(Workspace& ws, const artk_moe_experts_t& a, MoeSaved& c, bool backward = true) {
   const size_t n = (size_t)(a.T * a.k), E = (size_t)a.E, r = (size_t)a.r, H = (size_t)a.H, I = (size_t)a.I;
-  c.Bt_gu = ws.take<uint16_t>(E * 2 * r * 2 * I);
-  c.At_gu = ws.take<uint16_t>(E * H * 2 * r);
-  c.Bt_d = ws.take<uint16_t>(E * r * H);
-  c.At_d = ws.take<uint16_t>(E * I * r);
+  c.Bt_gu = c.At_gu = c.Bt_d = c.At_d = nullptr;
+  if (backward) {
+    c.Bt_gu = ws.take<uint16_t>(E * 2 * r * 2 * I);
+    c.At_gu = ws.take<uint16_t>(E * H * 2 * r);
+    c.Bt_d = ws.take<uint16_t>(E * r * H);
+    c.At_d = ws.take<uint16_t>(E * I * r);
+  }
   c.xa_gu = ws.take<float>(n * 2 * r);
   c.xaw_d = ws.take<float>(n * r);
   c.gu = ws.take<uint16_t>(n * 2 * I);
@@ -1267,7 +1276,7 @@ static void carve_moe_block_bwd(Workspace& ws, const artk_moe_experts_t& a, MoeB
   c.dx_rows = ws.take<uint16_t>(n * H);
 }
 
-static int32_t check_moe_experts(const artk_moe_experts_t* a, bool backward) {
+static int32_t check_moe_experts(const artk_moe_experts_t* a, bool backward, bool saved = true) {
   ARTK_CHECK_ARG(a != nullptr, "null argument");
   ARTK_CHECK_ARG(a->T > 0 && a->k > 0 && a->E > 0 && a->k <= a->E, "T, E, k must be positive and k <= E");
   if (a->E > MOE_MAX_E || a->k > MOE_MAX_K || a->T * a->k >= (1ll << 30)) {
@@ -1285,9 +1294,9 @@ static int32_t check_moe_experts(const artk_moe_experts_t* a, bool backward) {
     return ARTK_ERR_UNSUPPORTED_SHAPE;
   }
   ARTK_CHECK_ARG(a->x && a->topk_idx && a->topk_w && a->perm && a->inv_perm && a->row_token && a->offsets &&
-                     a->tile_prefix && a->blk_prefix && a->saved,
+                     a->tile_prefix && a->blk_prefix && (a->saved || !saved),
                  "null pointer argument");
-  ARTK_CHECK_ARG(aligned16(a->x) && aligned16(a->saved), "pointers must be 16-byte aligned");
+  ARTK_CHECK_ARG(aligned16(a->x) && (aligned16(a->saved) || !saved), "pointers must be 16-byte aligned");
   return ARTK_OK;
 }
 
@@ -1300,6 +1309,14 @@ size_t artk_moe_experts_saved_bytes(const artk_moe_experts_t* a) {
 size_t artk_moe_experts_fwd_workspace_bytes(const artk_moe_experts_t* a) {
   Workspace ws(nullptr, 0);
   MoeFwdScratch c;
+  carve_moe_fwd(ws, *a, c);
+  return ws.used + 256;
+}
+size_t artk_moe_experts_eval_workspace_bytes(const artk_moe_experts_t* a) {
+  Workspace ws(nullptr, 0);
+  MoeSaved s;
+  MoeFwdScratch c;
+  carve_moe_saved(ws, *a, s, false);
   carve_moe_fwd(ws, *a, c);
   return ws.used + 256;
 }
@@ -1318,9 +1335,10 @@ static int32_t launch_moe_combine(const uint16_t* rows, const artk_moe_experts_t
   return ARTK_OK;
 }
 
-int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,
-                             artk_stream_t stream) {
-  int32_t rc = check_moe_experts(a, false);
+// The forward pass; with `backward` the buffer a->saved keeps what one needs, else everything lies in the workspace.
+static int32_t moe_experts_forward(const artk_moe_experts_t* a, bool backward, void* workspace, size_t workspace_bytes,
+                                   artk_stream_t stream) {
+  int32_t rc = check_moe_experts(a, false, backward);
   if (rc) return rc;
   ARTK_CHECK_ARG(a->router_logits && a->W_gu && a->W_d && a->gate_A && a->gate_B && a->up_A && a->up_B && a->down_A &&
                      a->down_B && a->y,
@@ -1332,9 +1350,9 @@ int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_
   Workspace ws(workspace, workspace_bytes), sv(a->saved, a->saved_bytes);
   MoeFwdScratch c;
   MoeSaved s;
+  carve_moe_saved(backward ? sv : ws, *a, s, backward);
   carve_moe_fwd(ws, *a, c);
-  carve_moe_saved(sv, *a, s);
-  if (!ws.ok() || !sv.ok()) {
+  if (!ws.ok() || (backward && !sv.ok())) {
     set_error("workspace too small: need %zu and %zu bytes, got %zu and %zu", ws.used, sv.used, workspace_bytes,
               a->saved_bytes);
     return ARTK_ERR_WORKSPACE_TOO_SMALL;
@@ -1362,6 +1380,15 @@ int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_
                             round16(r), s.order, st)))
     return rc;
   return launch_moe_combine(c.down, a, a->topk_w, a->y, st);
+}
+
+int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,
+                             artk_stream_t stream) {
+  return moe_experts_forward(a, true, workspace, workspace_bytes, stream);
+}
+int32_t artk_moe_experts_eval(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,
+                              artk_stream_t stream) {
+  return moe_experts_forward(a, false, workspace, workspace_bytes, stream);
 }
 
 int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,

@@ -24,12 +24,12 @@ class _MoEExpertsFn(torch.autograd.Function):
     """The whole block (routing, three projections, gating, recombination) as one library call each way."""
 
     @staticmethod
-    def forward(ctx, x, logits, top_k, W_gu, W_d, Wt_gu, Wt_d, scale, *params):
+    def forward(ctx, x, logits, top_k, W_gu, W_d, Wt_gu, Wt_d, scale, backward, *params):
         dtype = params[0].dtype
         if dtype not in (torch.float32, torch.bfloat16) or any(p.dtype != dtype for p in params):
             dtype = torch.float32
         adapters = {n: _aligned(p.detach().to(dtype)) for n, p in zip(ops._MOE_PARAMS, params)}
-        y, routing, saved = ops.moe_experts_fwd(x, logits, top_k, W_gu, W_d, adapters, scale)
+        y, routing, saved = ops.moe_experts_fwd(x, logits, top_k, W_gu, W_d, adapters, scale, backward)
         ctx.save_for_backward(x, saved)
         # the module's transposed weights outlive the call: as saved tensors, hooks that move activations to the host
         # would copy them for every block
@@ -41,7 +41,7 @@ class _MoEExpertsFn(torch.autograd.Function):
     def backward(ctx, g, _g_routing):
         x, saved = ctx.saved_tensors
         dx, grads = ops.moe_experts_bwd(_aligned(g), x, ctx.routing, saved, *ctx.frozen, ctx.rank, ctx.scale)
-        return (dx,) + (None,) * 7 + tuple(grads[n].to(t) for n, t in zip(ops._MOE_PARAMS, ctx.dtypes))
+        return (dx,) + (None,) * 8 + tuple(grads[n].to(t) for n, t in zip(ops._MOE_PARAMS, ctx.dtypes))
 
 
 class MoELoRAExperts(nn.Module):
@@ -89,7 +89,9 @@ class MoELoRAExperts(nn.Module):
         """x bf16 [T,H], router_logits f32 [T,E] -> (y bf16 [T,H], routing)."""
         params = (self.gate_lora_A, self.gate_lora_B, self.up_lora_A, self.up_lora_B, self.down_lora_A,
                   self.down_lora_B)
+        # (inside the function grad mode is off either way)
+        backward = torch.is_grad_enabled() and any(t.requires_grad for t in (x, *params))
         return _MoEExpertsFn.apply(
             x.to(torch.bfloat16).contiguous(), router_logits.detach().float().contiguous(), self.top_k,
             self.gate_up_weight, self.down_weight, self._transposed("gate_up"), self._transposed("down"),
-            float(self.scaling), *params)
+            float(self.scaling), backward, *params)

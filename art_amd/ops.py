@@ -451,9 +451,10 @@ def _moe_experts_struct(x, routing: Routing, I: int, r: int, saved, scale: float
     return st, C.byref(st)
 
 
-def moe_experts_fwd(x, router_logits, k: int, W_gu, W_d, adapters: dict, scale: float):
+def moe_experts_fwd(x, router_logits, k: int, W_gu, W_d, adapters: dict, scale: float, backward: bool = True):
     """A block of gated-MLP experts (see artk_moe_experts_fwd): (y bf16 [T,H], routing, saved), where `saved`
-    is what moe_experts_bwd needs.  adapters: gate_A, gate_B, up_A, up_B, down_A, down_B, all f32 or all bf16."""
+    is what moe_experts_bwd needs (None with backward=False).  adapters: gate_A, gate_B, up_A, up_B, down_A, down_B,
+    all f32 or all bf16."""
     T, H = x.shape
     E, _, I = W_d.shape
     r = adapters["down_A"].shape[1]
@@ -477,15 +478,17 @@ def moe_experts_fwd(x, router_logits, k: int, W_gu, W_d, adapters: dict, scale: 
     rt.offsets, rt.tile_prefix, rt.blk_prefix = i32(E + 1), i32(E + 1), i32(E + 1)
     rt.n_rows, rt.n_experts, rt.k = n, E, k
     st, ref = _moe_experts_struct(x, rt, I, r, None, scale)
-    saved = _workspace(lib.artk_moe_experts_saved_bytes(ref), dev)
-    ws = _workspace(lib.artk_moe_experts_fwd_workspace_bytes(ref), dev)
+    kind = "fwd" if backward else "eval"
+    saved = _workspace(lib.artk_moe_experts_saved_bytes(ref), dev) if backward else None
+    ws = _workspace(getattr(lib, f"artk_moe_experts_{kind}_workspace_bytes")(ref), dev)
     y = torch.empty_like(x)
-    st.saved, st.saved_bytes = saved.data_ptr(), saved.numel()
+    if backward:
+        st.saved, st.saved_bytes = saved.data_ptr(), saved.numel()
     st.router_logits, st.W_gu, st.W_d, st.y = (t.data_ptr() for t in (router_logits, W_gu, W_d, y))
     for name in _MOE_PARAMS:
         setattr(st, name, adapters[name].data_ptr())
     st.adapters_bf16 = int(dtype == torch.bfloat16)
-    _lib.check(lib.artk_moe_experts_fwd(ref, ws.data_ptr(), ws.numel(), _stream(dev)))
+    _lib.check(getattr(lib, f"artk_moe_experts_{kind}")(ref, ws.data_ptr(), ws.numel(), _stream(dev)))
     return y, rt, saved
 
 

@@ -285,6 +285,11 @@ size_t artk_moe_experts_saved_bytes(const artk_moe_experts_t* a);
 size_t artk_moe_experts_fwd_workspace_bytes(const artk_moe_experts_t* a);
 int32_t artk_moe_experts_fwd(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,
                              artk_stream_t stream);
+/* The forward alone (evaluation, reference logprobs): the same y and routing; `saved` is not used, and the transposed
+ * adapters of the backward are not made. */
+size_t artk_moe_experts_eval_workspace_bytes(const artk_moe_experts_t* a);
+int32_t artk_moe_experts_eval(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,
+                              artk_stream_t stream);
 size_t artk_moe_experts_bwd_workspace_bytes(const artk_moe_experts_t* a);
 int32_t artk_moe_experts_bwd(const artk_moe_experts_t* a, void* workspace, size_t workspace_bytes,
                              artk_stream_t stream);

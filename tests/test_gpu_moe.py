@@ -528,3 +528,37 @@ def test_moe_block_hooks_see_no_frozen_weights(artk_lib, gpu):
     side.synchronize()
     assert all(torch.equal(a, b) for a, b in zip(got, want))
     assert (9, 128) in seen and not any(len(s) == 3 for s in seen)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_moe_block_without_a_backward(artk_lib, gpu, dtype):
+    """Under no_grad, and where nothing needs a gradient, the block gives the same bits and makes no transposed adapters: its
+    peak of memory is lower by at least their size (all else is allocated either way)."""
+    E, H, I, r, T = 16, 512, 256, 16, 24
+    torch.manual_seed(15)
+    mod = MoELoRAExperts(H, I, E, 2, r=r, lora_alpha=16, device=gpu)
+    params = [p for p in mod.parameters() if p.requires_grad]
+    with torch.no_grad():
+        for p in params:
+            p.data = p.normal_(std=0.05).to(dtype)
+    x, logits = torch.randn(T, H, device=gpu, dtype=torch.bfloat16), torch.randn(T, E, device=gpu)
+    print("moe block without a backward", dtype, flush=True)
+
+    def peak():
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        y, routing = mod(x, logits)
+        torch.cuda.synchronize()
+        assert y.requires_grad == (torch.is_grad_enabled() and params[0].requires_grad)
+        return torch.cuda.max_memory_allocated() - before, y.detach(), routing.topk_idx
+
+    peak()   # (the transposed frozen weights are made once)
+    with_grad, want, experts = peak()
+    transposed = 2 * E * (2 * r * 2 * I + H * 2 * r + r * H + I * r)
+    with torch.no_grad():
+        without, got, idx = peak()
+    assert torch.equal(got, want) and torch.equal(idx, experts) and without <= with_grad - transposed
+    for p in params:
+        p.requires_grad_(False)
+    assert peak()[0] == without
