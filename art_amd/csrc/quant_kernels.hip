@@ -65,8 +65,12 @@ __device__ __forceinline__ uint4 nf4_expand(const float* lut, uint32_t w, float 
 }
 
 // A thread turns 4 packed bytes into 8 elements, so a wave reads 256 contiguous bytes and writes 1 KiB contiguous, NF4_UNROLL
-// times with all reads on their way first: 2048 x 11008 elements in 10.0 us (one at a time 12.2; with quantised maxima 10.6 / 14.4).
-constexpr int NF4_UNROLL = 4;
+// times with all reads on their way first: 2048 x 11008 elements in 10.6 us (one at a time 11.8, 12.8 with a division per
+// element group; with quantised maxima 11.2 / 12.5 / 14.7).  Below NF4_FULL work-groups per CU of one read each there is
+// nothing left to fill the GPU with four: 896 x 896 3.3 us with one, 3.5 with four; 896 x 4864 4.5 / 4.6, 2048 x 2048 4.4 / 4.4,
+// 2048 x 3072 5.4 / 5.3.
+constexpr int NF4_FULL = 8;
+template <int NF4_UNROLL>
 __global__ __launch_bounds__(256) void nf4_dequant_kernel(Nf4Params p) {
   __shared__ float lut[16];
   if (threadIdx.x < 16) lut[threadIdx.x] = NF4_LEVELS[threadIdx.x];
@@ -91,7 +95,7 @@ __global__ __launch_bounds__(256) void nf4_dequant_kernel(Nf4Params p) {
 // Same values written transposed: the weight is [R, C] (C elements per row, quantisation blocks
 // run along a row), the output is bf16 [C, R].  A work-group takes 64 rows x 256 columns: a thread expands an 8 x 8 block and
 // transposes it in registers, and LDS gathers the 64 rows of a column, which are stored as one cache line.  (Two bytes at a
-// time through LDS: 2048 x 11008 elements 17.8 us, now 13.3; 3584 x 18944 45.4, now 33.1; 896 x 4864 5.0, now 5.2.)
+// time through LDS: 2048 x 11008 elements 18.2 us, now 14.1; 3584 x 18944 46.6, now 33.6.)
 __global__ __launch_bounds__(256) void nf4_dequant_t_kernel(Nf4Params p, int64_t R, int64_t C) {
   __shared__ float lut[16];
   __shared__ uint4 tile[256][8];  // [column][8 rows], chunk XORed by the column's group of 8
@@ -124,6 +128,40 @@ __global__ __launch_bounds__(256) void nf4_dequant_t_kernel(Nf4Params p, int64_t
   for (int i = 0; i < 8; ++i) {
     const int cc = i * 32 + (threadIdx.x >> 3), k = threadIdx.x & 7;
     if (c0 + cc < C && r0 + k * 8 < R) *(uint4*)(p.out + (c0 + cc) * R + r0 + k * 8) = tile[cc][k ^ ((cc >> 3) & 7)];
+  }
+}
+
+// The same for matrices of fewer than NF4_T_FULL such tiles per CU: 64 rows x 64 columns per work-group, a thread expands 8
+// columns of two rows and puts the pairs into LDS.  us, this / tiles of 64 x 256: 896 x 896 3.4 / 4.5, 896 x 4864 4.9 / 5.9,
+// 2048 x 2048 4.8 / 5.4, 2048 x 3072 6.2 / 6.5, 3584 x 3584 11.4 / 9.2.
+constexpr int NF4_T_FULL = 2;
+__global__ __launch_bounds__(256) void nf4_dequant_t_small_kernel(Nf4Params p, int64_t R, int64_t C) {
+  __shared__ float lut[16];
+  __shared__ uint4 tile[64][8];  // [column][8 rows], chunk XORed by the column's group of 8
+  if (threadIdx.x < 16) lut[threadIdx.x] = NF4_LEVELS[threadIdx.x];
+  __syncthreads();
+  const int64_t r0 = (int64_t)blockIdx.y * 64, c0 = (int64_t)blockIdx.x * 64;
+  const int cb = threadIdx.x & 7, rp = threadIdx.x >> 3;
+  const int64_t c = c0 + cb * 8, r = r0 + rp * 2;
+  if (r < R && c < C) {  // (R and C are multiples of 8)
+    const int shift = __builtin_ctz(p.blocksize);
+    const int64_t blk[2] = {(r * C + c) >> shift, (r * C + C + c) >> shift};
+    const uint32_t w0 = *(const uint32_t*)(p.packed + (r * C + c) / 2), w1 = *(const uint32_t*)(p.packed + (r * C + C + c) / 2);
+    float scale[2];
+    nf4_scales(p, blk, scale);
+    const uint4 a = nf4_expand(lut, w0, scale[0]), b = nf4_expand(lut, w1, scale[1]);
+    const uint32_t av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t lo = av[j / 2] >> (16 * (j & 1)) & 0xffffu, hi = bv[j / 2] >> (16 * (j & 1)) & 0xffffu;
+      ((uint32_t*)&tile[cb * 8 + j][(rp >> 2) ^ cb])[rp & 3] = lo | hi << 16;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int cc = i * 32 + (threadIdx.x >> 3), k = threadIdx.x & 7;
+    if (c0 + cc < C && r0 + k * 8 < R) *(uint4*)(p.out + (c0 + cc) * R + r0 + k * 8) = tile[cc][k ^ (cc >> 3)];
   }
 }
 
@@ -168,9 +206,12 @@ int32_t artk_nf4_dequant(const void* packed, const float* absmax, const void* ab
   int32_t rc = check_nf4(packed, absmax, absmax_q, code2, absmax2, n, blocksize, out_bf16);
   if (rc) return rc;
   Nf4Params p = nf4_params(packed, absmax, absmax_q, code2, absmax2, offset, n, blocksize, out_bf16);
-  const int64_t blocks = (n / 8 + 256 * NF4_UNROLL - 1) / (256 * NF4_UNROLL);
-  ARTK_CHECK_ARG(blocks < (1ll << 31), "too many elements");
-  nf4_dequant_kernel<<<(unsigned)blocks, 256, 0, (hipStream_t)stream>>>(p);
+  const int64_t reads = (n / 8 + 255) / 256;  // work-groups with a read per thread
+  ARTK_CHECK_ARG(reads < (1ll << 33), "too many elements");
+  if (reads >= NF4_FULL * num_cus())
+    nf4_dequant_kernel<4><<<(unsigned)((reads + 3) / 4), 256, 0, (hipStream_t)stream>>>(p);
+  else
+    nf4_dequant_kernel<1><<<(unsigned)reads, 256, 0, (hipStream_t)stream>>>(p);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }
@@ -183,8 +224,11 @@ int32_t artk_nf4_dequant_t(const void* packed, const float* absmax, const void* 
   int32_t rc = check_nf4(packed, absmax, absmax_q, code2, absmax2, rows * cols, blocksize, out_bf16);
   if (rc) return rc;
   Nf4Params p = nf4_params(packed, absmax, absmax_q, code2, absmax2, offset, rows * cols, blocksize, out_bf16);
-  dim3 grid((unsigned)((cols + 255) / 256), (unsigned)((rows + 63) / 64));
-  nf4_dequant_t_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(p, rows, cols);
+  const unsigned row_tiles = (unsigned)((rows + 63) / 64);
+  if ((cols + 255) / 256 * row_tiles >= NF4_T_FULL * num_cus())
+    nf4_dequant_t_kernel<<<dim3((unsigned)((cols + 255) / 256), row_tiles), 256, 0, (hipStream_t)stream>>>(p, rows, cols);
+  else
+    nf4_dequant_t_small_kernel<<<dim3((unsigned)((cols + 63) / 64), row_tiles), 256, 0, (hipStream_t)stream>>>(p, rows, cols);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;
 }

@@ -87,6 +87,20 @@ def test_dequant_transposed_bit_exact(artk_lib, gpu, rows, cols, blocksize, nest
     assert torch.equal(tr, plain.t().contiguous())
 
 
+@pytest.mark.parametrize("rows,cols", [(8, 8), (8, 520), (520, 8), (136, 72), (3592, 2312), (3640, 2048), (72, 130056)])
+def test_dequant_either_side_of_the_launch_rules(artk_lib, gpu, rows, cols):
+    """Both orders of both kernels (one read or four per thread; tiles of 64 x 64 or 64 x 256) at sizes with remainders:
+    the oracle's bits."""
+    g = np.random.default_rng(rows + cols)
+    n = rows * cols
+    packed, absmax = g.integers(0, 256, n // 2, dtype=np.uint8), g.random(n // 32, dtype=np.float32)
+    want = qo.to_bf16_bits(qo.dequantize(packed, absmax, 32)).reshape(rows, cols)
+    args = [torch.from_numpy(t).to(gpu) for t in (packed, absmax)]
+    print("nf4 launch rules", rows, cols, flush=True)
+    assert np.array_equal(bits(ops.nf4_dequant(*args, blocksize=32)).reshape(rows, cols), want)
+    assert np.array_equal(bits(ops.nf4_dequant_t(args[0], rows, cols, args[1], blocksize=32)).reshape(cols, rows), want.T)
+
+
 @pytest.mark.parametrize("n_out,n_in,T,r,with_bias", [(256, 128, 64, 8, False), (2048, 2048, 1024, 8, True),
                                                       (320, 192, 300, 16, True)])
 def test_lora_on_nf4_weight_without_resident_copies(artk_lib, gpu, n_out, n_in, T, r, with_bias):
