@@ -886,6 +886,8 @@ __global__ __launch_bounds__(ATT_THREADS, D == 128 && KT == 2 ? 2 : 3) void attn
 //   8192 positions, 28 / 4 heads:                                      40: 374, 30: 361, 15: 345, 8: 322, 6: 354
 //   12000 positions, 28 / 4 heads                                      40: 520, 12: 463, 8: 473, 6: 523
 //   16384 positions, 14 / 2 heads of 64:                               40: 217, 15: 207, 8: 202, 6: 205
+// A launch that fits the GPU at once (not numbered) hardly depends on it: 2 rows of 1009 positions, 16 / 2 heads, 40: 88, 15: 88, 8: 87,
+// 4: 86; 2700, 14 / 2 heads of 64, 118, 118, 117, 116.
 // two rounds, 16384 positions, 28 / 4 heads (numbered by head):  6: 629, 15: 595, 40: 623, 100: 707 (backward).
 // A share also costs evenness: its steps come in pieces that the dispatch order (longest list first) does not rank.
 // Where the lists are long on average the set-up is small against one head's steps, and every work-group takes one
@@ -921,46 +923,40 @@ struct AttnKvSplit {
 // units (as in attn_block) in their order, none left out.  A grid has room for a work-group per head; numbered by head,
 // those without a share lie between the others, and each holds its place on a CU for about 3 us (16384 positions of 8
 // prompts of 137 + 4 x 461, 28 / 4 heads: 5832 of 7168).  Numbered like this they come last.  The search costs a work-group
-// a microsecond, so it is for grids that do not fit the GPU at once.  `scratch`: 8 words of LDS.  False: no share left.
+// a microsecond, so it is for grids that do not fit the GPU at once.  It takes one unit per thread; fewer than two rounds of key
+// blocks are at most 192 units per XCD.  `scratch`: 8 words of LDS.  False: no share left.
+constexpr int ATT_KV_UNITS = 256;
 __device__ __forceinline__ bool attn_kv_item(int Hq, int Hkv, int nKb, const int* order, const int* cnt, const AttnKvSplit& split,
                                              int64_t stride, int row, int item, uint32_t* scratch, int& hq, int& kb) {
-  const int rep = Hq / Hkv, x = blockIdx.x & 7, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int units = (nKb * Hkv + 7) / 8;
-  int base = 0;
-  for (int u0 = 0; u0 < units; u0 += 256) {
-    const int unit = (u0 + (int)threadIdx.x) * 8 + x, rank = unit / Hkv;
-    int b = 0, per = 1, shares = 0;
-    if (rank < nKb) {
-      b = order[rank];
-      per = split.heads(cnt[b], rep, stride, row);
-      shares = (rep + per - 1) / per;
-    }
-    int end = shares;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int v = __shfl_up(end, d, 64);
-      if (lane >= d) end += v;
-    }
-    __syncthreads();
-    if (lane == 63) scratch[wave] = (uint32_t)end;
-    __syncthreads();
-    const int total = (int)(scratch[0] + scratch[1] + scratch[2] + scratch[3]);
-    for (int w = 0; w < wave; ++w) end += (int)scratch[w];
-    const int at = item - base - (end - shares);
-    if (at >= 0 && at < shares) {
-      scratch[4] = (uint32_t)((unit % Hkv) * rep + at * per);
-      scratch[5] = (uint32_t)b;
-    }
-    __syncthreads();
-    if (item - base < total) {
-      hq = __builtin_amdgcn_readfirstlane((int)scratch[4]);
-      kb = __builtin_amdgcn_readfirstlane((int)scratch[5]);
-      __syncthreads();
-      return true;
-    }
-    base += total;
+  const int rep = Hq / Hkv, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int unit = (int)threadIdx.x * 8 + (blockIdx.x & 7), rank = unit / Hkv;
+  int b = 0, per = 1, shares = 0;
+  if (rank < nKb) {
+    b = order[rank];
+    per = split.heads(cnt[b], rep, stride, row);
+    shares = (rep + per - 1) / per;
   }
-  return false;
+  int end = shares;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int v = __shfl_up(end, d, 64);
+    if (lane >= d) end += v;
+  }
+  if (lane == 63) scratch[wave] = (uint32_t)end;
+  __syncthreads();
+  const int total = (int)(scratch[0] + scratch[1] + scratch[2] + scratch[3]);
+  if (item >= total) return false;
+  for (int w = 0; w < wave; ++w) end += (int)scratch[w];
+  const int at = item - (end - shares);
+  if (at >= 0 && at < shares) {
+    scratch[4] = (uint32_t)((unit % Hkv) * rep + at * per);
+    scratch[5] = (uint32_t)b;
+  }
+  __syncthreads();
+  hq = __builtin_amdgcn_readfirstlane((int)scratch[4]);
+  kb = __builtin_amdgcn_readfirstlane((int)scratch[5]);
+  __syncthreads();
+  return true;
 }
 
 // 32 rows of a head as the operand fragments of one wave (lane (n, h): row n, 8 columns from 16 s + 8 h on).  Loaded row by
@@ -1799,7 +1795,8 @@ int32_t artk_attn_bwd_rows(const void* q, const void* k, const void* v, const vo
     p.split.div = two_rounds ? slots * 3 / 2 : slots * 4 / 5;
     p.split.light_max = g_light_max_override;  // artk_attn_bwd_tuning
     const dim3 grid_kv(attn_grid(Hq, Hkv, pl.nKb2), (unsigned)rows);
-    p.split.packed = Hq != Hkv && !two_rounds && (int64_t)grid_kv.x * grid_kv.y > slots;
+    p.split.packed = Hq != Hkv && !two_rounds && (int64_t)grid_kv.x * grid_kv.y > slots &&
+                     pl.nKb2 * (int64_t)Hkv <= 8 * ATT_KV_UNITS;
     prof_begin(PROF_ATTN_BWD_KV, st);
     if (D == 128)
       attn_bwd_kv_kernel<128><<<grid_kv, 256, 0, st>>>(p);
