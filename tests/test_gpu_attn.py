@@ -478,7 +478,8 @@ def test_plan_of_a_short_row_is_that_of_a_long_one(artk_lib, gpu, S, ids):
 @pytest.mark.parametrize("S", [31, 32, 33, 64, 96, 160, 480])
 def test_attn_steps_of_32_keys(artk_lib, gpu, S, D):
     """Runs of 32 positions that belong to two groups by turns, and positions of the second that see the first one's: whole
-    halves of a 64-key tile are invisible to a work-group (first, last, alone in the list) or to some of its waves."""
+    halves of a 64-key tile are invisible to a work-group (first, last, alone in the list) or to some of its waves.  dQ takes
+    steps of 32 at these sizes, the forward of 64 (test_attn_fwd_steps_of_32_keys has the heads that its steps of 32 need)."""
     from art_amd.attention import attention_plans, packed_attention
     print("attention steps of 32 keys", S, D, flush=True)
     Hq, Hkv = 4, 2
@@ -609,3 +610,55 @@ def test_attn_bwd_mask_holds_for_any_lse_and_scale(artk_lib, gpu, D):
             assert torch.isfinite(a).all()
             if b.norm() > 0:
                 assert rel_l2(a.float().cpu(), b) <= 1e-2
+
+
+@pytest.mark.parametrize("S", [31, 32, 33, 64, 96, 160, 255, 480])
+def test_attn_fwd_steps_of_32_keys(artk_lib, gpu, S):
+    """The ids of test_attn_steps_of_32_keys with so many heads of 128 that the forward takes steps of 32 keys too."""
+    from art_amd.attention import attention_plans, packed_attention
+    Hq, Hkv, D = (288, 16, 128) if S <= 256 else (144, 8, 128)
+    assert fwd_work_groups(S, Hq, Hkv) > 2 * cus()
+    print("attention forward in steps of 32 keys", S, flush=True)
+    q, k, v = make_qkv(S, S, Hq, Hkv, D)
+    run = torch.arange(S) // 32
+    for group, parent in ((run % 2, run % 2), (run % 2, (run % 3 == 2).long()), (run % 5, (run + 3) % 5), (run, run)):
+        plans = attention_plans(group.to(gpu), parent.to(gpu))
+        with torch.no_grad():
+            out = packed_attention(*(t.to(gpu) for t in (q, k, v)), plans)
+        assert rel_l2(out.float().cpu(), attn_oracle.attention(q, k, v, group, parent)[0]) <= 1e-2
+    # lse, by the gradients, which recompute P from it
+    d_out = torch.randn(S, Hq, D, generator=torch.Generator().manual_seed(S)).to(torch.bfloat16)
+    ref = attn_oracle.attention_grads(q, k, v, group, parent, d_out)[1:]
+    leaves = [t.to(gpu).requires_grad_(True) for t in (q, k, v)]
+    for a, b in zip(torch.autograd.grad(packed_attention(*leaves, plans), leaves, d_out.to(gpu)), ref):
+        assert rel_l2(a.float().cpu(), b) <= 1e-2
+
+
+@pytest.mark.parametrize("head_major", [False, True])
+@pytest.mark.parametrize("ids", ["dense", "scattered", "packed"])
+def test_attn_fwd_steps_of_32_keys_embedded_in_nan(artk_lib, gpu, ids, head_major):
+    """A row of 700 positions whose forward takes steps of 32 keys, inside larger tensors of NaN: one causal conversation,
+    ids without any order, and a packed row."""
+    from art_amd.attention import attention_plans, packed_attention
+    S, Hq, Hkv, D = 700, 88, 8, 128
+    assert fwd_work_groups(S, Hq, Hkv) > 2 * cus()
+    print("attention forward in steps of 32 keys", ids, head_major, flush=True)
+    g = torch.Generator().manual_seed(S)
+    data = [torch.randn(S, H, D, generator=g).to(torch.bfloat16) for H in (Hq, Hkv, Hkv, Hq)]
+    group, parent = {"dense": lambda: (torch.zeros(S, dtype=torch.int64),) * 2,
+                     "scattered": lambda: (torch.randint(0, 5, (S,), generator=g), torch.randint(0, 5, (S,), generator=g)),
+                     "packed": lambda: synthetic.packed_row_ids(3, S, 2, 41, 3, 97)}[ids]()
+
+    def embed(t):
+        s, h, d = t.shape
+        big = torch.full((h + 1, s + 9, d) if head_major else (s + 9, h + 1, d), float("nan"), dtype=torch.bfloat16, device=gpu)
+        view = big[:h, :s].transpose(0, 1) if head_major else big[:s, :h]
+        view.copy_(t)
+        return view
+
+    q, k, v, up = (embed(t) for t in data)
+    leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+    out = packed_attention(*leaves, attention_plans(group.to(gpu), parent.to(gpu)))
+    ref = attn_oracle.attention_grads(*data[:3], group, parent, data[3])
+    for got, want in zip((out.detach(), *torch.autograd.grad(out, leaves, up)), ref):
+        assert torch.isfinite(got).all() and rel_l2(got.float().cpu(), want) <= 1e-2
