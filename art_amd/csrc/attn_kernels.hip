@@ -412,7 +412,7 @@ __global__ __launch_bounds__(1024) void attn_plan_short_order_kernel(AttnPlan pl
 // ----------------------------------------------------------------------------
 // Tiles and fragments shared by the three kernels
 // ----------------------------------------------------------------------------
-// Every operand tile in LDS is 64 rows (keys or queries) x D elements, row-major
+// An operand tile in LDS is 64 or 32 rows (keys or queries) x D elements, row-major
 // as in HBM, its 16-byte chunks XOR-swizzled by row.  Two ways to read it:
 //   row fragments  (ds_read_b128): lane (m, h) gets 8 consecutive d of row m,
 //                   the A operand of a product that contracts over d;
@@ -1020,8 +1020,7 @@ struct AttnBwdParams {
 template <int D>
 __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kernel(AttnBwdParams p) {
   using T = AttnTile<D>;
-  constexpr int KT = 1;
-  using G = AttnKeySteps<D, KT>;
+  using G = AttnKeySteps<D, 1>;
   using R = AttnWaveRows<D>;
   constexpr int ROWS_OFF = (G::LDS + 1023) / 1024 * 1024;
   __shared__ __attribute__((aligned(1024))) char smem[ROWS_OFF + 4 * R::BYTES];  // one LDS object (see attn_smem_note)
@@ -1096,41 +1095,37 @@ __global__ __launch_bounds__(ATT_THREADS, D == 64 ? 3 : 2) void attn_bwd_dq_kern
     pin_loaded(bt.lo);
     pin_loaded(bt.hi);
     if (active) {
-      bf16x8 dsf[2 * KT];
+      floatx16 sc, dp;
 #pragma unroll
-      for (int kt = 0; kt < KT; ++kt) {
-        const char* const kh = smem + kt * 32 * T::ROW;
-        floatx16 sc, dp;
+      for (int j = 0; j < 16; ++j) sc[j] = dp[j] = 0.f;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) sc[j] = dp[j] = 0.f;
+      for (int s = 0; s < D / 16; ++s) {
+        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_at(smem, bk, s), qf[s], sc, 0, 0, 0);
+        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_at(smem + G::V_OFF, bk, s), dof[s], dp, 0, 0, 0);
+      }
+      // the mask comes behind the multiply-add: whatever a query's lse and the scale are, P is 0 where it sees nothing
 #pragma unroll
-        for (int s = 0; s < D / 16; ++s) {
-          sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_at(kh, bk, s), qf[s], sc, 0, 0, 0);
-          dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_at(kh + G::V_OFF, bk, s), dof[s], dp, 0, 0, 0);
+      for (int j = 0; j < 16; ++j) sc[j] = __builtin_fmaf(sc[j], p.scale_log2e, nlse2);
+      if (partial) {  // one branch for all elements: tested inside the loop below it becomes one per element
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const int kk = 8 * g4 + 4 * h;
+          const int4 kc = *(const int4*)(codes + kk);
+          const int kcv[4] = {kc.x, kc.y, kc.z, kc.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (!attn_visible(q, key0 + kk + e, gi, pi, kcv[e])) sc[4 * g4 + e] = -INFINITY;
         }
-        // the mask comes behind the multiply-add: whatever a query's lse and the scale are, P is 0 where it sees nothing
+      }
+      bf16x8 dsf[2];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) sc[j] = __builtin_fmaf(sc[j], p.scale_log2e, nlse2);
-        if (partial >> kt & 1) {  // one branch for all elements: tested inside the loop below it becomes one per element
-#pragma unroll
-          for (int g4 = 0; g4 < 4; ++g4) {
-            const int kk = 32 * kt + 8 * g4 + 4 * h;
-            const int4 kc = *(const int4*)(codes + kk);
-            const int kcv[4] = {kc.x, kc.y, kc.z, kc.w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (!attn_visible(q, key0 + kk + e, gi, pi, kcv[e])) sc[4 * g4 + e] = -INFINITY;
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const float pr = __builtin_amdgcn_exp2f(sc[j]);
-          dsf[2 * kt + j / 8][j % 8] = (__bf16)(pr * (dp[j] - delta));
-        }
+      for (int j = 0; j < 16; ++j) {
+        const float pr = __builtin_amdgcn_exp2f(sc[j]);
+        dsf[j / 8][j % 8] = (__bf16)(pr * (dp[j] - delta));
       }
       // dQ^T += K^T dS^T, K^T fragments by transposing reads of the K tile
 #pragma unroll
-      for (int s2 = 0; s2 < 2 * KT; ++s2) {
+      for (int s2 = 0; s2 < 2; ++s2) {
 #pragma unroll
         for (int dt = 0; dt < D / 32; ++dt)
           dq[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_at<D>(smem, bt, s2, dt), dsf[s2], dq[dt], 0, 0, 0);

@@ -94,6 +94,22 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
   return __builtin_bit_cast(uint16_t, h);
 }
 
+// 8 x 8 bf16 in registers: out[c] = column c of in.
+__device__ __forceinline__ void transpose8x8(const uint4 (&in)[8], uint4 (&out)[8]) {
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    uint32_t o[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      auto word = [&](const uint4& v) { return c / 2 == 0 ? v.x : c / 2 == 1 ? v.y : c / 2 == 2 ? v.z : v.w; };
+      const uint32_t lo = (word(in[2 * k]) >> (16 * (c & 1))) & 0xffffu;
+      const uint32_t hi = (word(in[2 * k + 1]) >> (16 * (c & 1))) & 0xffffu;
+      o[k] = lo | (hi << 16);
+    }
+    out[c] = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+}
+
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float LN2 = 0.6931471805599453f;
 

@@ -270,6 +270,8 @@ struct MoePerm {
 
 // The whole sort of a few chunks by one work-group: for 1624 keys histogram, scan and placement are 3 + 5 + 6 us as three
 // launches, and the gaps between them, and 7 as one.  (A launch per step is what many chunks need: their placement is spread.)
+// Routing of 128 experts in us, one launch / three: 1624 keys 11.3 / 12.4, 3072 12.6 / 12.7, 3584 13.1 / 13.0, 4096 13.6 / 12.8 in
+// the replay of a graph; a block's forward at 4096 keys, gaps included, 284.0 / 284.6.
 constexpr int SORT_CHUNKS = 4;
 __global__ __launch_bounds__(PERM_CHUNK) void moe_sort_kernel(const int* __restrict__ keys, int n, int E, int k, MoeScanOut o,
                                                               MoePerm out) {

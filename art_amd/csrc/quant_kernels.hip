@@ -10,7 +10,6 @@
 // 0.5 B (+ 0.06 B of scales) read and 2 B written per element, a few per cent
 // of the time of the GEMM that follows.
 #include "common.hpp"
-#include "lora_common.hpp"
 
 namespace artk {
 
