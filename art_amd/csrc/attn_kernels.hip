@@ -11,7 +11,7 @@
 // element only in the partly visible ones.
 //
 // Forward work-group: 128 queries x one head, 4 wavefronts of 32 queries, three
-// work-groups per CU.  Scores
+// work-groups per CU (two in launches of up to two at a head dimension of 128).  Scores
 // are computed transposed (S^T = K Q^T, MFMA 32x32x16), so that a lane owns one
 // query: the row maximum and sum are in-lane reductions plus one exchange between
 // the two half-waves, the accumulator of S^T is already in the B-operand layout of
@@ -23,12 +23,11 @@
 // lists made for 128 queries.  Against one work-group of 8 waves per CU with three stages, two of 4 waves with tiles of 64
 // keys took 16384 positions of 8 prompts of 137 + 4 x 461, 28 / 4 heads of 128, from 205 to 154 us (dQ 279 -> 244, dK/dV
 // 433 -> 297); at up to 3 % more on dense rows of 16384 (16 / 2 heads of 128: 2772 -> 2895 us forward and backward at 12288).
-// Steps of 32 keys (AttnKeySteps) since, us before / after:
-//   forward, three work-groups per CU at a head dimension of 128 (64: three either way, tiles of 64 keys): the packed row
-//     157 / 136, the same with 16 / 2 heads 88 / 78, 8192 positions 80 / 70; dense 16384 1866 / 1840, 8192 with 16 / 2 heads
-//     270 / 268, 4096 127 / 129; a row of 2048 in two conversations 22 / 23
-//   backward with dK/dV's second stage: packed 563 / 522, 389 / 358, 329 / 302; dense 6735 / 6330, 1001 / 988, 468 / 461;
-//     heads of 64, 14 / 2: 16384 packed 190 / 168, 8192 dense 515 / 475; two conversations 86 / 83
+// Steps of 32 keys (AttnKeySteps) since, us before (tiles of 64, one stage of query tiles in dK/dV) / now, heads of 128:
+//   forward, three work-groups per CU: the packed row 150 / 129, the same with 16 / 2 heads 88 / 76, 8192 positions of it 83 / 71;
+//     dense 16384 1766 / 1771, 4096 130 / 132, 8192 with 16 / 2 heads 274 / 273
+//   dQ: the packed row 248 / 214, 16 / 2 heads 142 / 119; dense 16384 2521 / 2447, 8192 660 / 643
+//   dK/dV: the packed row 303 / 262, 16 / 2 heads 219 / 154; dense 3832 / 3471, 945 / 896; heads of 64, 14 / 2: 8192 dense 296 / 270
 // A head dimension of 64 has too few MFMAs per key for steps of 32 in the forward (8192 dense: 138 -> 160 us).
 #include <stdlib.h>
 

@@ -800,8 +800,8 @@ __global__ __launch_bounds__(nthreads<BWD_NI>()) void dhidden_gemm_kernel(BwdPar
   TileAcc<BWD_NI> acc;
   acc.zero();
   // A full tile has its own loop: where some of its instructions may be left out, the DMA issues are branches that its
-  // schedule cannot cross.  d_hidden products of a step in us, one loop for all tiles / this: 16384 positions, 7B shape, 6267 /
-  // 5946; 8192 3290 / 3340; 8000 positions at a hidden size of 896 1306 / 1273.
+  // schedule cannot cross.  d_hidden products of a step in us, one loop for all tiles / this: 8000 positions at a hidden size of 896
+  // 1294 / 1256, 4000 at 2048 958 / 951, 7B shape: 16384 5945 / 5948 on one machine and 6267 / 5946 on another, 8192 3378 / 3406.
   const int left = n_active - tt * TILE;
   if (left >= TILE) {
     gemm_tile_nt(acc, smem, p.Wt, p.V, (int64_t)ht * TILE, p.H, p.P, p.V, (int64_t)tt * TILE, n_active, kb * BK, ke * BK,
