@@ -67,6 +67,28 @@ def test_argument_errors_have_codes_and_messages(artk_lib):
     assert rc == _lib.ERR_UNSUPPORTED_SHAPE and b"head dimension" in artk_lib.artk_last_error()
 
 
+def test_moe_forward_alone_needs_no_saved_buffer(artk_lib):
+    """artk_moe_experts_eval takes everything from its workspace, which is smaller than what a forward with a backward needs by
+    the transposed adapters; the same arguments are refused otherwise."""
+    from art_amd import _lib
+
+    buf = (C.c_char * 4096)()
+    p = (C.addressof(buf) + 15) // 16 * 16
+    st = _lib.MoeExpertsStruct()
+    for name, kind in st._fields_:
+        if kind is C.c_void_p and name != "saved":
+            setattr(st, name, p)
+    st.T, st.H, st.I, st.E, st.k, st.r, st.scale = 24, 512, 256, 16, 2, 16, 1.0
+    ref = C.byref(st)
+    assert artk_lib.artk_moe_experts_fwd(ref, p, 1 << 20, None) == _lib.ERR_INVALID_ARGUMENT   # no `saved`
+    assert artk_lib.artk_moe_experts_eval(ref, p, 4096, None) == _lib.ERR_WORKSPACE_TOO_SMALL
+    alone = artk_lib.artk_moe_experts_eval_workspace_bytes(ref)
+    both = artk_lib.artk_moe_experts_fwd_workspace_bytes(ref) + artk_lib.artk_moe_experts_saved_bytes(ref)
+    assert alone <= both - 2 * 16 * (32 * 512 + 512 * 32 + 16 * 512 + 256 * 16)
+    st.E = 300
+    assert artk_lib.artk_moe_experts_eval(ref, p, 1 << 20, None) == _lib.ERR_UNSUPPORTED_SHAPE
+
+
 def test_check_raises(artk_lib):
     import pytest
 
