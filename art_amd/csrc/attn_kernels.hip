@@ -11,7 +11,7 @@
 // element only in the partly visible ones.
 //
 // Forward work-group: 128 queries x one head, 4 wavefronts of 32 queries, three
-// work-groups per CU (two in launches of up to two at a head dimension of 128).  Scores
+// work-groups per CU.  Scores
 // are computed transposed (S^T = K Q^T, MFMA 32x32x16), so that a lane owns one
 // query: the row maximum and sum are in-lane reductions plus one exchange between
 // the two half-waves, the accumulator of S^T is already in the B-operand layout of
@@ -642,8 +642,7 @@ struct AttnKeySteps {
     }
     dma_load4(rsrc_c, (lane & (KEYS - 1)) * 4, k0 * 4, lds_addr_of(st + CODE_OFF));
   }
-  // The first two steps are on their way before anything else is read (of 64 keys: the first; the second would come before the
-  // queries: 2 % of a short row's forward).  (A row of the plan has four entries or more.)
+  // The first two steps are on their way before anything else is read.  (A row of the plan has four entries or more.)
   __device__ __forceinline__ void begin(char* smem, const uint16_t* k_head, int64_t k_stride, const uint16_t* v_head,
                                         int64_t v_stride, int S, const int* codes, const uint32_t* list, int tiles, int wave,
                                         int lane) {
@@ -666,12 +665,9 @@ struct AttnKeySteps {
       cur = nxt = seen(entry, 0) ? 0 : 1;
       issue(smem, key(), wave, lane);
       advance(e1);
-      if (STEPS == 2) second(smem, wave, lane);
+      if (nxt < n) issue(smem + STAGE, key(e_nxt, nxt), wave, lane);
     }
     for (int i = threadIdx.x; i < tiles; i += ATT_THREADS) ((uint32_t*)(smem + LIST_OFF))[i] = list[i];
-  }
-  __device__ __forceinline__ void second(char* smem, int wave, int lane) const {
-    if (nxt < n) issue(smem + STAGE, key(e_nxt, nxt), wave, lane);
   }
   // The entry that end() needs, read while the step is computed (past the end of the list: not used).
   __device__ __forceinline__ uint32_t ahead(const char* smem) const { return ((const uint32_t*)(smem + LIST_OFF))[nxt / STEPS + 1]; }
@@ -689,10 +685,13 @@ struct AttnKeySteps {
   }
 };
 
-// KT: 32 keys of a step.
-template <int D, int KT>
-__global__ __launch_bounds__(ATT_THREADS, D == 128 && KT == 2 ? 2 : 3) void attn_fwd_kernel(AttnFwdParams p) {
+template <int D>
+__global__ __launch_bounds__(ATT_THREADS, 3) void attn_fwd_kernel(AttnFwdParams p) {
   using T = AttnTile<D>;
+  // 32 keys of a step.  (The same for every launch of a head dimension: a row's bits do not depend on its batch.  Steps of 64, two
+  // work-groups per CU, in launches of up to two per CU at D = 128, us, 64 / 32: 1 x 4096 of 300 + 2 x 1800, 16 / 2 heads 73 / 69;
+  // 1 x 2048, 28 / 4 heads 26.5 / 25.2; 1 x 1009 13.9 / 13.9; 1 x 500 13.2 / 13.7; batches 2 x 1999 33 / 30, 8 x 1300, 16 / 2 48 / 39.)
+  constexpr int KT = D == 128 ? 1 : 2;
   using G = AttnKeySteps<D, KT>;
   constexpr float LAZY = KT == 1 ? 4.f : 8.f;
   __shared__ __attribute__((aligned(1024))) char smem[G::LDS];  // one LDS object (see attn_smem_note)
@@ -738,7 +737,6 @@ __global__ __launch_bounds__(ATT_THREADS, D == 128 && KT == 2 ? 2 : 3) void attn
   int stage = 0;
   wait_vmcnt<0>();
   barrier_lds_only();
-  if (KT == 2) ks.second(smem, wave, lane);
   int fresh = 64;  // keys until the reference of the exponentials follows lazily
   while (ks.cur < ks.n) {
     const uint32_t ahead = ks.ahead(smem);
@@ -1669,16 +1667,10 @@ int32_t artk_attn_fwd_rows(const void* q, const void* k, const void* v, const vo
   p.scale_log2e = scale * LOG2E;
   const dim3 grid(attn_grid(Hq, Hkv, pl.nQb), (unsigned)B);
   prof_begin(PROF_ATTN_FWD, st);
-  // Up to two work-groups per CU there is no third to make room for, and steps of 64 keys take less time (us, 32 / 64:
-  // 4096 positions in one conversation of 300 + 2 x 1800, 16 / 2 heads 78 / 71; 2048 in two, 28 / 4 heads 23 / 21).  The count is
-  // that of one row, so that its bits are the same in any batch.  That has a price in batches of short rows (2 of 1999
-  // positions, 28 / 4 heads 31 / 34; 8 of 1300, 16 / 2 41 / 50).
-  if (D == 64)
-    attn_fwd_kernel<64, 2><<<grid, ATT_THREADS, 0, st>>>(p);
-  else if ((int64_t)grid.x <= 2 * num_cus())
-    attn_fwd_kernel<128, 2><<<grid, ATT_THREADS, 0, st>>>(p);
+  if (D == 128)
+    attn_fwd_kernel<128><<<grid, ATT_THREADS, 0, st>>>(p);
   else
-    attn_fwd_kernel<128, 1><<<grid, ATT_THREADS, 0, st>>>(p);
+    attn_fwd_kernel<64><<<grid, ATT_THREADS, 0, st>>>(p);
   prof_end(PROF_ATTN_FWD, st);
   ARTK_CHECK_LAUNCH();
   return ARTK_OK;

@@ -478,8 +478,7 @@ def test_plan_of_a_short_row_is_that_of_a_long_one(artk_lib, gpu, S, ids):
 @pytest.mark.parametrize("S", [31, 32, 33, 64, 96, 160, 480])
 def test_attn_steps_of_32_keys(artk_lib, gpu, S, D):
     """Runs of 32 positions that belong to two groups by turns, and positions of the second that see the first one's: whole
-    halves of a 64-key tile are invisible to a work-group (first, last, alone in the list) or to some of its waves.  dQ takes
-    steps of 32 at these sizes, the forward of 64 (test_attn_fwd_steps_of_32_keys has the heads that its steps of 32 need)."""
+    halves of a 64-key tile are invisible to a work-group (first, last, alone in the list) or to some of its waves."""
     from art_amd.attention import attention_plans, packed_attention
     print("attention steps of 32 keys", S, D, flush=True)
     Hq, Hkv = 4, 2
@@ -522,64 +521,73 @@ def test_attn_bwd_numbers_work_groups_share_by_share(artk_lib, gpu, S, Hq, Hkv, 
             assert torch.equal(a, c)
 
 
-def fwd_work_groups(S, Hq, Hkv):
-    """Work-groups of the forward for one row.  At a head dimension of 128 more than two per CU take steps of 32 keys."""
-    blocks = -(-S // 256) * 2
-    return -(-blocks * Hkv // 8) * 8 * (Hq // Hkv)
-
-
-def cus():
-    return torch.cuda.get_device_properties(0).multi_processor_count
+def out_of_rounded_p(s, v, keys, lazy):
+    """[S, D] in 64 bits but for P, rounded to bf16 below a reference that waves of 32 queries move to their maximum over `keys` keys
+    where one of their scores is 2^lazy above it.  s: masked scores in units of log2."""
+    S, n = s.shape[0], -(-s.shape[0] // 64) * 64
+    w = torch.nn.functional.pad(s, (0, n - S, 0, n - S), value=float("-inf")).view(n // 32, 32, n)
+    v = torch.nn.functional.pad(v, (0, 0, 0, n - S))
+    m, total, o = w.new_full((n // 32, 32), -1e30), w.new_zeros(n // 32, 32), w.new_zeros(n // 32, 32, v.shape[1])
+    fresh = torch.ones(n // 32, dtype=torch.bool, device=s.device)   # the first keys that a wave sees move it at once
+    for k0 in range(0, n, keys):
+        x = w[:, :, k0:k0 + keys]
+        top = x.amax(2)
+        seen = torch.isfinite(top).any(1)
+        move = (top > m + torch.where(fresh, 0.0, lazy)[:, None]).any(1) & seen
+        new = torch.where(move[:, None], torch.maximum(m, top), m)
+        alpha = torch.exp2(m - new)
+        e = torch.exp2(x - new[..., None]).float()
+        o = o * alpha[..., None] + e.to(torch.bfloat16).double() @ v[k0:k0 + keys]
+        total, m, fresh = total * alpha + e.double().sum(2), new, fresh & ~seen
+    return (o / total[..., None]).view(n, -1)[:S]
 
 
 @pytest.mark.parametrize("std", [1.0, 2.0, 4.0, 8.0])
-def test_attn_steps_of_32_keys_are_as_exact(artk_lib, gpu, std):
-    """One row in steps of 32 keys (all heads in a call) and of 64 (a call per key/value head) against 64 bits: out is no
-    farther off, be the scores flat or peaked."""
+def test_attn_fwd_is_as_exact_as_steps_of_64_keys(artk_lib, gpu, std):
+    """out at a head dimension of 128 is no farther from 64 bits than one whose P is rounded below a reference that follows the
+    maximum of 64 keys from 2^8 on, be the scores flat or peaked."""
     S, Hq, Hkv, D = 2531, 28, 4, 128
-    assert fwd_work_groups(S, Hq, Hkv) > 2 * cus() >= fwd_work_groups(S, Hq // Hkv, 1)
     print("attention against 64 bits", std, flush=True)
     q, k, v = (t.to(gpu) for t in make_qkv(int(std), S, Hq, Hkv, D))
     q = (q.float() * std).to(torch.bfloat16)
     group, parent = (t.to(gpu) for t in synthetic.packed_row_ids(7, S, 2, 150, 4, 260))
-    plan = ops.attn_plan_rows(group[None], parent[None])
-    from art_amd.attention import packed_attention
-    rep = Hq // Hkv
+    from art_amd.attention import attention_plans, packed_attention
     with torch.no_grad():
-        whole = packed_attention(q, k, v, plan)
-        parts = torch.cat([packed_attention(q[:, h * rep:(h + 1) * rep], k[:, h:h + 1], v[:, h:h + 1], plan)
-                           for h in range(Hkv)], 1)
+        out = packed_attention(q, k, v, attention_plans(group, parent))
     i = torch.arange(S, device=gpu)
     hidden = (i[None] > i[:, None]) | ((group[:, None] != group[None]) & (parent[:, None] != group[None]))
     err = torch.zeros(2, dtype=torch.float64, device=gpu)
     for h in range(Hq):
-        s = q[:, h].double() @ k[:, h // rep].double().t().contiguous() * D ** -0.5
-        ref = torch.softmax(s.masked_fill_(hidden, float("-inf")), 1) @ v[:, h // rep].double()
-        err += torch.stack([(t[:, h].double() - ref).pow(2).sum() for t in (whole, parts)])
+        kh, vh = (t[:, h * Hkv // Hq].double() for t in (k, v))
+        s = (q[:, h].double() @ kh.t().contiguous() * D ** -0.5).masked_fill_(hidden, float("-inf"))
+        ref = torch.softmax(s, 1) @ vh
+        other = out_of_rounded_p(s * 1.4426950408889634, vh, 64, 8.0).to(torch.bfloat16)
+        err += torch.stack([(t.double() - ref).pow(2).sum() for t in (out[:, h], other)])
     assert err[0] <= err[1], err.sqrt().tolist()
 
 
 def test_attn_row_is_the_same_in_any_batch(artk_lib, gpu):
-    """A row whose forward fills the GPU twice over only together with another: out and dQ (which reads lse) are those of the
-    row alone, bit for bit."""
+    """A row that fills the GPU only together with another: out and dQ (which reads lse) are those of the row alone, bit for bit,
+    and of a call with some of its heads."""
     from art_amd.attention import attention_plans, packed_attention
     B, S, Hq, Hkv, D = 2, 2531, 16, 2, 128
-    assert fwd_work_groups(S, Hq, Hkv) <= 2 * cus() < B * fwd_work_groups(S, Hq, Hkv)
     print("attention row in a batch", flush=True)
     g = torch.Generator(device=gpu).manual_seed(3)
     data = [torch.randn(B, S, H, D, generator=g, device=gpu).to(torch.bfloat16) for H in (Hq, Hkv, Hkv, Hq)]
     ids = [synthetic.packed_row_ids(80 + b, S, 2, 150, 4, 260) for b in range(B)]
     group, parent = (torch.stack([i[j] for i in ids]).to(gpu) for j in (0, 1))
 
-    def call(rows):
-        leaves = [t[rows].detach().requires_grad_(True) for t in data[:3]]
+    def call(rows, heads=slice(None), kv_heads=slice(None)):
+        leaves = [t[rows, :, h].detach().requires_grad_(True) for t, h in zip(data, (heads, kv_heads, kv_heads))]
         out = packed_attention(*leaves, attention_plans(group[rows], parent[rows]))
-        return out.detach(), torch.autograd.grad(out, leaves, data[3][rows])[0]
+        return out.detach(), torch.autograd.grad(out, leaves, data[3][rows, :, heads])[0]
 
     batch = call(slice(None))
     for b in range(B):
         for got, want in zip(batch, call(slice(b, b + 1))):
             assert torch.equal(got[b], want[0])
+        for got, want in zip(batch, call(slice(b, b + 1), slice(0, Hq // Hkv), slice(0, 1))):
+            assert torch.equal(got[b, :, :Hq // Hkv], want[0])
 
 
 @pytest.mark.parametrize("D", [64, 128])
@@ -612,36 +620,13 @@ def test_attn_bwd_mask_holds_for_any_lse_and_scale(artk_lib, gpu, D):
                 assert rel_l2(a.float().cpu(), b) <= 1e-2
 
 
-@pytest.mark.parametrize("S", [31, 32, 33, 64, 96, 160, 255, 480])
-def test_attn_fwd_steps_of_32_keys(artk_lib, gpu, S):
-    """The ids of test_attn_steps_of_32_keys with so many heads of 128 that the forward takes steps of 32 keys too."""
-    from art_amd.attention import attention_plans, packed_attention
-    Hq, Hkv, D = (288, 16, 128) if S <= 256 else (144, 8, 128)
-    assert fwd_work_groups(S, Hq, Hkv) > 2 * cus()
-    print("attention forward in steps of 32 keys", S, flush=True)
-    q, k, v = make_qkv(S, S, Hq, Hkv, D)
-    run = torch.arange(S) // 32
-    for group, parent in ((run % 2, run % 2), (run % 2, (run % 3 == 2).long()), (run % 5, (run + 3) % 5), (run, run)):
-        plans = attention_plans(group.to(gpu), parent.to(gpu))
-        with torch.no_grad():
-            out = packed_attention(*(t.to(gpu) for t in (q, k, v)), plans)
-        assert rel_l2(out.float().cpu(), attn_oracle.attention(q, k, v, group, parent)[0]) <= 1e-2
-    # lse, by the gradients, which recompute P from it
-    d_out = torch.randn(S, Hq, D, generator=torch.Generator().manual_seed(S)).to(torch.bfloat16)
-    ref = attn_oracle.attention_grads(q, k, v, group, parent, d_out)[1:]
-    leaves = [t.to(gpu).requires_grad_(True) for t in (q, k, v)]
-    for a, b in zip(torch.autograd.grad(packed_attention(*leaves, plans), leaves, d_out.to(gpu)), ref):
-        assert rel_l2(a.float().cpu(), b) <= 1e-2
-
-
 @pytest.mark.parametrize("head_major", [False, True])
 @pytest.mark.parametrize("ids", ["dense", "scattered", "packed"])
 def test_attn_fwd_steps_of_32_keys_embedded_in_nan(artk_lib, gpu, ids, head_major):
-    """A row of 700 positions whose forward takes steps of 32 keys, inside larger tensors of NaN: one causal conversation,
-    ids without any order, and a packed row."""
+    """A row of 700 positions in more work-groups than two per CU, inside larger tensors of NaN: one causal conversation, ids
+    without any order, and a packed row."""
     from art_amd.attention import attention_plans, packed_attention
     S, Hq, Hkv, D = 700, 88, 8, 128
-    assert fwd_work_groups(S, Hq, Hkv) > 2 * cus()
     print("attention forward in steps of 32 keys", ids, head_major, flush=True)
     g = torch.Generator().manual_seed(S)
     data = [torch.randn(S, H, D, generator=g).to(torch.bfloat16) for H in (Hq, Hkv, Hkv, Hq)]
