@@ -299,8 +299,8 @@ __device__ __forceinline__ void gemm_tile_run_8(TileAcc<2>& acc, char* smem, con
 
   // DMA instructions per operand issued right after the barrier that frees their buffer, the rest at the
   // start of the next K-step.  All of them early (a full K-step of lead) pays where most row-operand
-  // panels miss in L2 (grouped GEMMs whose weights serve two or three tiles: +1-2 %); elsewhere the split
-  // is faster (lm_head forward at a hidden size of 896: 6 %, LoRA linear: 1.4 %).
+  // panels miss in L2 (grouped GEMMs whose weights serve two or three tiles: +1-2 %) and in part in d_hidden
+  // (dhidden_gemm_kernel); elsewhere the split is faster (lm_head forward at a hidden size of 896: 6 %, LoRA linear: 1.4 %).
   constexpr int EARLY = ALL_EARLY ? DI : NI;
   constexpr int TG = NQ + (ALL_EARLY ? 10 : 0);  // issue<> tag
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -402,8 +402,8 @@ __device__ __forceinline__ void gemm_tile_run_8(TileAcc<2>& acc, char* smem, con
 
 // gemm_tile_run for a tile whose column operand has only `ncols` (<= 256) rows that anybody
 // stores: a wave computes only those of its NI 32-column tiles that contain such a column
-// (wave-uniform choice; every variant executes the same barriers).  8-wave shape only.  For partial tiles: with less to
-// compute the whole fill of a stage is requested right after the barrier.
+// (wave-uniform choice; every variant executes the same barriers).  8-wave shape only.  Its callers
+// are the grouped GEMM and d_hidden, which measured faster with the whole fill of a stage requested right after the barrier.
 __device__ __forceinline__ void gemm_tile_run_cols(TileAcc<2>& acc, char* smem, const TileLoaders<2>& L,
                                                    int ncols) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

@@ -783,6 +783,10 @@ struct BwdParams {
 
 // The grid is sized for the worst case (every row active); the work-groups
 // beyond the device-side schedule exit at once.
+// OWN_LOOP: full tiles have a loop of their own, which pays below this hidden size.  (As a branch in one kernel the choice costs
+// half of what it gains.)
+constexpr int DHIDDEN_OWN_LOOP = 3072;
+template <bool OWN_LOOP>
 __global__ __launch_bounds__(nthreads<BWD_NI>()) void dhidden_gemm_kernel(BwdParams p) {
   __shared__ __attribute__((aligned(1024))) char smem[GEMM_LDS_BYTES];
   const int n_active = p.sched[0], TT = p.sched[1], nsplit = p.sched[2], n_work = p.sched[3];
@@ -799,19 +803,21 @@ __global__ __launch_bounds__(nthreads<BWD_NI>()) void dhidden_gemm_kernel(BwdPar
 
   TileAcc<BWD_NI> acc;
   acc.zero();
-  // A full tile has its own loop: where some of its instructions may be left out, the DMA issues are branches that its
-  // schedule cannot cross.  d_hidden products of a step in us, one loop for all tiles / this: 8000 positions at a hidden size of 896
-  // 1294 / 1256, 4000 at 2048 958 / 951, 7B shape: 16384 5945 / 5948 on one machine and 6267 / 5946 on another, 8192 3378 / 3406.
+  // Rows past the last active one are neither fetched nor computed (190 active rows: 94 -> 90 us).  The loop for that has a branch
+  // around every DMA instruction, which the schedule cannot cross, and asks for whole stages early; full tiles have the choice.
+  // Whole steps in us, that loop for all tiles / a loop of their own: 8000 positions at a hidden size of 896 3518 / 3493, 4000 at
+  // 2048 3031 / 3019, 3 x 4000 skipping at 2048 5264 / 5245; at 3584 1500 skipping 1467 / 1482, 5062 skipping 3932 / 3987, 8192
+  // 10260 / 10301, 16384 level (once 20566 / 20175).  (Own loop, whole stages early, no branches: d_hidden 1202 us instead of
+  // 1258 at 896, 986 instead of 951 at 2048.)
   const int left = n_active - tt * TILE;
-  if (left >= TILE) {
+  if (OWN_LOOP && left >= TILE) {
     gemm_tile_nt(acc, smem, p.Wt, p.V, (int64_t)ht * TILE, p.H, p.P, p.V, (int64_t)tt * TILE, n_active, kb * BK, ke * BK,
                  p.active_idx);
   } else {
-    // rows past the last active one are neither fetched nor computed (190 active rows: 94 -> 90 us)
     TileLoaders<BWD_NI> L;
     L.init(p.Wt, p.V, (int64_t)ht * TILE, p.H, p.P, p.V, (int64_t)tt * TILE, n_active, kb * BK, ke * BK, p.active_idx, true);
     L.issue_first(smem);
-    gemm_tile_run_cols(acc, smem, L, left);
+    gemm_tile_run_cols(acc, smem, L, left < TILE ? left : TILE);
   }
 
   const int lane = threadIdx.x & 63;
@@ -1197,7 +1203,10 @@ static int32_t launch_bwd_chunk(uint16_t* stash, const void* lm_head, const void
   const int64_t dense_cap = (int64_t)HT * TT * max_splits(HT, num_cus());
   const unsigned grid = (unsigned)(max_blocks < dense_cap ? max_blocks : dense_cap);
   prof_begin(PROF_DHIDDEN_GEMM, st);
-  dhidden_gemm_kernel<<<grid, nthreads<BWD_NI>(), 0, st>>>(b);
+  if (H < DHIDDEN_OWN_LOOP)
+    dhidden_gemm_kernel<true><<<grid, nthreads<BWD_NI>(), 0, st>>>(b);
+  else
+    dhidden_gemm_kernel<false><<<grid, nthreads<BWD_NI>(), 0, st>>>(b);
   prof_end(PROF_DHIDDEN_GEMM, st);
   ARTK_CHECK_LAUNCH();
   const int64_t n4 = Tc * H / 4;

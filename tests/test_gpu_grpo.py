@@ -112,6 +112,14 @@ def test_fused_matches_oracle(artk_lib, gpu, T, H, V, n_traj, chunk_tokens):
     assert hidden.grad[0][~m.to(gpu)].abs().max().item() == 0.0
 
 
+@pytest.mark.parametrize("H", [3008, 3072])
+@pytest.mark.parametrize("T", [1024, 1092])
+def test_fused_either_side_of_the_loops_of_d_hidden(artk_lib, gpu, T, H):
+    """Hidden sizes below and from 3072 on (full tiles of d_hidden in a loop of their own or in that of partial ones), with two full
+    tiles of active rows or a little more: as test_fused_matches_oracle."""
+    test_fused_matches_oracle(artk_lib, gpu, T, H, 2048, 4, 4096)
+
+
 def test_fused_wide_logit_range(artk_lib, gpu):
     """Peaked distributions: logits spread over +-35 nats, targets up to ~65 nats under their row's maximum.
     The backward works on exp(logit - target logit) in bf16, which has to hold over that range."""
